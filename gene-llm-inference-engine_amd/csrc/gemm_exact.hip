@@ -1,177 +1,418 @@
 // C[m, n] (=|+=) sum_k A[m, k] * W[n, k] in true 32-bit arithmetic.
 //
 // Both operands are row-major with k contiguous (activations [M, K], weights [N, K] as checkpoints
-// store them).  Every output element is one chain of fused multiply-adds over k = 0 .. K-1 in
-// ascending order, whatever M is and wherever the row lies in the batch: a row computed alone
-// has the same bits as the same row inside a large batch (the reference keeps the same rule,
-// src/gpu/device_kernels.inc:97-100).  Operands may be stored as bfloat16; they are widened
-// exactly.  This kernel is the 32-bit path of every matrix product, and the slow stand-in of the
-// bfloat16 path for shapes the matrix-core kernels refuse.
+// store them); operands may be stored as bfloat16 and are widened exactly.  This is the 32-bit path of
+// every matrix product, and the slow stand-in of the bfloat16 path for shapes the matrix-core kernels refuse.
+//
+// The order of a sum depends on K alone, never on M, the row's place in the batch or the kernel that serves it, so a row computed
+// alone has the same bits as the same row inside a large batch (the reference keeps the same rule, src/gpu/device_kernels.inc:97-100):
+//   * k is cut into 8 ranges of L = 32 * ceil(K / 256) (the last ones shorter or empty);
+//   * a range's sum is one chain of 16x16x4 32-bit matrix instructions from zero, 16 of k after 16 of k, the four instructions of
+//     such a block taking k0 + 4g + j (g = 0..3 inside the instruction) for j = 0, 1, 2, 3; what lies beyond K counts as zero;
+//   * the ranges' sums are added as a tree, ((s0 + s1) + (s2 + s3)) + ((s4 + s5) + (s6 + s7)); what C held is added last.
+// The tree is what lets a product of a few rows be shared out over the chip (a chain over all of K leaves one lane or wave per column
+// walking K alone) and what one with few tiles is cut along; its error is smaller than the single chain's.
 #include "common.h"
 
 namespace {
 
-constexpr int BM = 64, BN = 64, BK = 16, PAD = 4;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <typename TA, typename TW, typename TC, bool ACCUMULATE>
-__global__ __launch_bounds__(256) void gemm_exact_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N,
-                                                         int K, long lda, long ldw, long ldc) {
-    __shared__ float As[BK][BM + PAD];
-    __shared__ float Ws[BK][BN + PAD];
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < K; k0 += BK) {
+constexpr int RANGES = 8;
+__host__ __device__ constexpr int range_length(int K) { return 32 * ((K + 32 * RANGES - 1) / (32 * RANGES)); }
+
+__device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// four consecutive elements, widened
+__device__ __forceinline__ f32x4 load4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+__device__ __forceinline__ f32x4 load4(const bf16_t* p) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    return f32x4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u)};
+}
+
+// The sum of range q joins the tree: t[0..2] hold the finished left halves; what is finished so far comes back.
+template <int N>
+__device__ __forceinline__ void fold(int q, f32x4 (&acc)[N], f32x4 (&t)[3][N]) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int e = tid + 256 * r, row = e >> 4, kk = e & 15;
-            const int m = m0 + row, n = n0 + row, k = k0 + kk;
-            As[kk][row] = (m < M && k < K) ? load_f32(A, (size_t)m * lda + k) : 0.f;
-            Ws[kk][row] = (n < N && k < K) ? load_f32(W, (size_t)n * ldw + k) : 0.f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < BK; ++kk) {
-            float a[4], w[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                a[i] = As[kk][ty * 4 + i];
-                w[i] = Ws[kk][tx * 4 + i];
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
-        }
-        __syncthreads();
+    for (int i = 0; i < N; ++i) {
+        if (!(q & 1)) { t[0][i] = acc[i]; continue; }
+        acc[i] = t[0][i] + acc[i];
+        if (!(q & 2)) { t[1][i] = acc[i]; continue; }
+        acc[i] = t[1][i] + acc[i];
+        if (!(q & 4)) { t[2][i] = acc[i]; continue; }
+        acc[i] = t[2][i] + acc[i];
     }
+}
+
+template <typename TC, bool ACCUMULATE>
+__device__ __forceinline__ void put(TC* C, size_t o, float v) {
+    if constexpr (ACCUMULATE) store_f32(C, o, load_f32(C, o) + v);
+    else store_f32(C, o, v);
+}
+
+// ------------------------------------------------------------------------------------------ many rows
+// A workgroup of four waves makes a tile of BM rows x 64 columns, both operands staged through LDS 32 of k at a time (two stages,
+// the next one's loads in flight in registers meanwhile).  Bound by the matrix cores (256 flop a clock and compute unit in 32-bit,
+// a sixteenth of bfloat16's): a wave's tile of 32 x 32 (BM 64) needs 4 KB of LDS for 512 clocks of matrix instructions, so what
+// counts is enough workgroups a compute unit to cover the loads' latency and no compute unit left idle; hence small tiles and, where the
+// tiles are few, the eight ranges of k shared out over `splits` workgroups (each finishes its part of the tree and leaves it in
+// `part`, a second kernel adds the parts).  The ring kernel below reaches 110 TFLOP/s of the 154 that a bare loop of these instructions
+// makes (600 rows of 128,256 x 2,048; 64 x 128, 128 x 64 and 128 x 128 tiles reach no more); the kernel of single fused multiply-adds
+// that stood here before made 19 at 301 rows of the Llama-3.2-1B shape, where this one makes 75 (97 on the widest products).
+constexpr int BN = 64, BK = 32;
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+
+// LDS: rows of 32 floats; the eight 16-byte chunks of a row are permuted by the row so that 16 rows' reads of one chunk meet 16 different places
+__device__ __forceinline__ int chunk_at(int row, int c) { return row * BK + ((c ^ ((row >> 1) & 7)) << 2); }
+
+// a lane's four results of a tile of 16 x 16 are four neighbouring columns of one row
+template <int TM, int TN, typename TC, bool ACCUMULATE>
+__device__ __forceinline__ void store_tile(const f32x4 (&acc)[TN * TM], TC* C, float* part, int m_first, int n_first, int z, int M, int N, long ldc) {
+    const bool whole_rows = part ? (N & 3) == 0 : sizeof(TC) == 4 && (ldc & 3) == 0 && ((uintptr_t)C & 15) == 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty * 4 + i;
+    for (int i = 0; i < TM; ++i) {
+        const int m = m_first + i * 16;
         if (m >= M) continue;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx * 4 + j;
-            if (n >= N) continue;
-            const size_t o = (size_t)m * ldc + n;
-            if constexpr (ACCUMULATE) store_f32(C, o, load_f32(C, o) + acc[i][j]);
-            else store_f32(C, o, acc[i][j]);
+        for (int j = 0; j < TN; ++j) {
+            const int n = n_first + j * 16;
+            const f32x4 v = acc[j * TM + i];
+            if (whole_rows && n + 3 < N) {
+                f32x4* to = reinterpret_cast<f32x4*>(part ? part + ((size_t)z * M + m) * N + n : (float*)C + (size_t)m * ldc + n);
+                *to = ACCUMULATE && !part ? *to + v : v;
+                continue;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (n + e >= N) break;
+                if (part) part[((size_t)z * M + m) * N + n + e] = v[e];
+                else put<TC, ACCUMULATE>(C, (size_t)m * ldc + n + e, v[e]);
+            }
         }
     }
 }
 
-// The same product for at most FEW_ROWS rows of 32-bit activations (decoding): one lane per output column walks its
-// weight row alone, so that a product with a handful of rows is spread over N lanes instead of N / 64 workgroups.
-// Every output is the same chain of fused multiply-adds over ascending k as in the kernel above: the bits do not
-// depend on which of the two kernels a row met.  A lane reads 16 bytes of its own row at a time (the rows of a
-// wave's lanes are K elements apart, so a cache line a lane has touched serves its next loads); the activations
-// are the same for all lanes.
-constexpr int FEW_ROWS = 4;
-
-template <typename TW> struct Sixteen;                      // 16 bytes of a weight row, widened
-template <> struct Sixteen<float> {
-    static constexpr int N = 4;
-    static __device__ __forceinline__ void load(const float* p, float (&w)[4]) {
-        const float4 v = *reinterpret_cast<const float4*>(p);
-        w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
-    }
-};
-template <> struct Sixteen<bf16_t> {
-    static constexpr int N = 8;
-    static __device__ __forceinline__ void load(const bf16_t* p, float (&w)[8]) {
-        const uint4 v = *reinterpret_cast<const uint4*>(p);
-        const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+// VECTOR: K and the leading dimensions are multiples of 4 and the bases aligned to 4 elements
+template <bool VECTOR, typename T>
+__device__ __forceinline__ f32x4 fetch(const T* base, long ld, int row, int rows, int k, int K) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    const T* p = base + (size_t)min(row, rows - 1) * ld;
+    if constexpr (VECTOR) {
+        v = load4(p + min(k, K - 4));
+        if (k >= K) v = f32x4{0.f, 0.f, 0.f, 0.f};
+    } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            w[2 * i] = __uint_as_float(u[i] << 16);
-            w[2 * i + 1] = __uint_as_float(u[i] & 0xffff0000u);
+        for (int i = 0; i < 4; ++i) v[i] = k + i < K ? load_f32(p, (size_t)(k + i)) : 0.f;
+    }
+    return v;
+}
+
+template <int BM, bool VECTOR, typename TA, typename TW, typename TC, bool ACCUMULATE>
+__global__ __launch_bounds__(256) void gemm_exact_tiled_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, float* __restrict__ part,
+                                                               int M, int N, int K, long lda, long ldw, long ldc, int m_tiles, int n_tiles, int splits) {
+    constexpr int WAVES_M = BM / 32, WAVES_N = 4 / WAVES_M, TN = BN / WAVES_N / 16, TM = 2;        // a wave: 32 rows x 64 / WAVES_N columns
+    constexpr int LOADS_A = BM * BK / 4 / 256, LOADS_W = BN * BK / 4 / 256;
+    __shared__ float lds[2][(BM + BN) * BK];
+    // the tiles of one strip of weights follow each other on one die (workgroups go to the eight dies in turn), whose L2 then reads the strip once
+    const int total = m_tiles * n_tiles * splits, each = (total + 7) / 8, u = (blockIdx.x & 7) * each + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= each || u >= total) return;
+    const int m0 = (u % m_tiles) * BM, n0 = (u / m_tiles % n_tiles) * BN, z = u / (m_tiles * n_tiles);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
+    const int wm = (wave % WAVES_M) * 32, wn = (wave / WAVES_M) * (BN / WAVES_N);
+
+    const int stages_all = (K + BK - 1) / BK, per_range = range_length(K) / BK;
+    const int q0 = z * (RANGES / splits), q1 = q0 + RANGES / splits;
+    const int s_end = min(q1 * per_range, stages_all);
+    f32x4 next_a[LOADS_A], next_w[LOADS_W];
+    auto ask = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < LOADS_A; ++i) { const int e = tid + 256 * i; next_a[i] = fetch<VECTOR>(A, lda, m0 + (e >> 3), M, s * BK + (e & 7) * 4, K); }
+#pragma unroll
+        for (int i = 0; i < LOADS_W; ++i) { const int e = tid + 256 * i; next_w[i] = fetch<VECTOR>(W, ldw, n0 + (e >> 3), N, s * BK + (e & 7) * 4, K); }
+    };
+    auto lay = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < LOADS_A; ++i) { const int e = tid + 256 * i; *reinterpret_cast<f32x4*>(&lds[buf][chunk_at(e >> 3, e & 7)]) = next_a[i]; }
+#pragma unroll
+        for (int i = 0; i < LOADS_W; ++i) { const int e = tid + 256 * i; *reinterpret_cast<f32x4*>(&lds[buf][BM * BK + chunk_at(e >> 3, e & 7)]) = next_w[i]; }
+    };
+
+    f32x4 acc[TN * TM], t[3][TN * TM];
+    int s = q0 * per_range;
+    if (s < s_end) { ask(s); lay(s & 1); }
+    __syncthreads();
+    for (int q = q0; q < q1; ++q) {
+#pragma unroll
+        for (int i = 0; i < TN * TM; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int stop = min((q + 1) * per_range, s_end);
+        for (; s < stop; ++s) {
+            const bool more = s + 1 < s_end;
+            if (more) ask(s + 1);
+            const float *as = lds[s & 1], *ws = as + BM * BK;
+#pragma unroll
+            for (int b = 0; b < BK / 16; ++b) {
+                f32x4 a[TM], w[TN];
+#pragma unroll
+                for (int i = 0; i < TM; ++i) a[i] = *reinterpret_cast<const f32x4*>(&as[chunk_at(wm + i * 16 + r, b * 4 + g)]);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) w[j] = *reinterpret_cast<const f32x4*>(&ws[chunk_at(wn + j * 16 + r, b * 4 + g)]);
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+#pragma unroll
+                        for (int i = 0; i < TM; ++i) acc[j * TM + i] = mfma(w[j][kk], a[i][kk], acc[j * TM + i]);
+            }
+            if (more) lay((s + 1) & 1);
+            __syncthreads();
+        }
+        fold(q - q0, acc, t);              // (the workgroup's ranges are a whole branch of the tree)
+    }
+    store_tile<TM, TN, TC, ACCUMULATE>(acc, C, part, m0 + wm + r, n0 + wn + 4 * g, z, M, N, ldc);
+}
+
+// The same for 32-bit operands whose rows are whole blocks of 32 k: the operands go from memory straight into LDS, a ring of three
+// stages with two in flight while one is multiplied (asked for and waited for as the bfloat16 ring kernel does), so a stage costs a
+// wave four loads and a barrier beside its matrix instructions.
+template <int BM, bool ACCUMULATE>
+__global__ __launch_bounds__(256) void gemm_exact_ring_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, float* __restrict__ part,
+                                                             int M, int N, int K, long lda, long ldw, long ldc, int m_tiles, int n_tiles, int splits) {
+    constexpr int WAVES_M = BM / 32, WAVES_N = 4 / WAVES_M, TN = BN / WAVES_N / 16, TM = 2, STAGES = 3;
+    constexpr int ROWS = BM + BN, LOADS = ROWS / 32;                       // a wave's loads a stage, each 8 rows of 128 bytes
+    __shared__ __attribute__((aligned(16))) float ring[STAGES * ROWS * BK];
+    const int total = m_tiles * n_tiles * splits, each = (total + 7) / 8, u = (blockIdx.x & 7) * each + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= each || u >= total) return;
+    const int m0 = (u % m_tiles) * BM, n0 = (u / m_tiles % n_tiles) * BN, z = u / (m_tiles * n_tiles);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
+    const int wm = (wave % WAVES_M) * 32, wn = (wave / WAVES_M) * (BN / WAVES_N);
+    const int per_range = range_length(K) / BK, q0 = z * (RANGES / splits), q1 = q0 + RANGES / splits;
+    const int s_begin = q0 * per_range, s_end = max(s_begin, min(q1 * per_range, K / BK));
+
+    const float* src[LOADS];                       // this lane's 16 bytes of each of its wave's loads, at k = 0; LDS is filled in order, so the chunk is chosen here
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int row = (wave * LOADS + i) * 8 + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
+        src[i] = (row < BM ? A + (size_t)min(m0 + row, M - 1) * lda : W + (size_t)min(n0 + row - BM, N - 1) * ldw) + 4 * c;
+    }
+    const unsigned ring_base = (unsigned)(size_t)(lds_ptr_t)ring;
+    // (written as assembly so that the compiler does not wait for them; the counted wait and the barrier below order them against the reads)
+    auto issue = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const unsigned dst = __builtin_amdgcn_readfirstlane(ring_base + (((s - s_begin) % STAGES) * ROWS + (wave * LOADS + i) * 8) * BK * 4);
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src[i] + (size_t)s * BK) : "memory", "m0");
+        }
+    };
+    f32x4 acc[TN * TM], t[3][TN * TM];
+#pragma unroll
+    for (int i = 0; i < STAGES - 1; ++i)
+        if (s_begin + i < s_end) issue(s_begin + i);
+    int s = s_begin;
+    for (int q = q0; q < q1; ++q) {
+#pragma unroll
+        for (int i = 0; i < TN * TM; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int stop = min((q + 1) * per_range, s_end);
+        for (; s < stop; ++s) {
+            if (s + 1 < s_end) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");        // this wave's part of stage s has landed
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();                                                          // everyone's has, and everyone has read stage s - 1
+            asm volatile("" ::: "memory");
+            if (s + STAGES - 1 < s_end) issue(s + STAGES - 1);
+            const float *as = ring + ((s - s_begin) % STAGES) * ROWS * BK, *ws = as + BM * BK;
+            f32x4 a[2][TM], w[2][TN];
+            auto read = [&](int b) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) a[b][i] = *reinterpret_cast<const f32x4*>(&as[chunk_at(wm + i * 16 + r, b * 4 + g)]);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) w[b][j] = *reinterpret_cast<const f32x4*>(&ws[chunk_at(wn + j * 16 + r, b * 4 + g)]);
+            };
+            read(0);
+            read(1);
+            __builtin_amdgcn_sched_barrier(0);             // (the second half's operands arrive while the first half is multiplied)
+#pragma unroll
+            for (int b = 0; b < BK / 16; ++b)
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+#pragma unroll
+                        for (int i = 0; i < TM; ++i) acc[j * TM + i] = mfma(w[b][j][kk], a[b][i][kk], acc[j * TM + i]);
+        }
+        fold(q - q0, acc, t);
+    }
+    store_tile<TM, TN, float, ACCUMULATE>(acc, C, part, m0 + wm + r, n0 + wn + 4 * g, z, M, N, ldc);
+}
+
+// The parts of the tree that `splits` workgroups left, added up: splits is 2, 4 or 8, a part's neighbours in the tree its neighbours here.
+template <typename TC, bool ACCUMULATE>
+__global__ __launch_bounds__(256) void gemm_exact_add_parts_kernel(const float* __restrict__ part, TC* __restrict__ C, int M, int N, long ldc, int splits) {
+    const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x, plane = (size_t)M * N;
+    if (e >= plane) return;
+    float v[RANGES];
+#pragma unroll
+    for (int z = 0; z < RANGES; ++z) v[z] = z < splits ? part[z * plane + e] : 0.f;
+    for (int n = splits; n > 1; n >>= 1) {
+#pragma unroll
+        for (int z = 0; z < RANGES / 2; ++z)
+            if (z < n / 2) v[z] = v[2 * z] + v[2 * z + 1];
+    }
+    put<TC, ACCUMULATE>(C, (e / N) * ldc + e % N, v[0]);
+}
+
+// ------------------------------------------------------------------------------------------- few rows
+// Up to 16 rows (decoding): bound by reading the weights once.  A workgroup owns a strip of weight rows and all of k, a wave one
+// range of k (strips of 16 rows, 8 waves) or two (strips of 8 rows and at most 8 rows of activations, 4 waves: the idle half of
+// every matrix instruction takes the second range, weight rows 8..15 and activation rows 8..15 of the instruction standing for the
+// same rows at the other range's k; twice the workgroups for the same waves, which is what narrow outputs lack).  The operands go
+// from memory straight into the matrix instructions' registers, AHEAD blocks of 16 k asked for at once; the ranges' sums
+// meet in LDS and are added there.  At 3 rows: 16,384 x 2,048 in 27 us (5.0 TB/s), 2,048 x 8,192 in 16 (4.1), 128,256 x 2,048 in 181
+// (5.8); one lane per column, each walking all of k alone, took 290 us, 1.15 ms and 400 us.
+constexpr int FEW_ROWS = 16, AHEAD = 8;
+
+template <int STRIP, typename TA, typename TW, typename TC, bool ACCUMULATE>
+__global__ __launch_bounds__(STRIP == 16 ? 512 : 256) void gemm_exact_few_rows_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C,
+                                                                                      int M, int N, int K, long lda, long ldw, long ldc) {
+    __shared__ f32x4 sums[RANGES][STRIP == 16 ? 64 : 16];                 // per range: [group of 4 columns][row]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * STRIP, L = range_length(K);
+    const int q = STRIP == 16 ? wave : 2 * wave + (r >> 3), row = STRIP == 16 ? r : r & 7;
+    const int q_last = STRIP == 16 ? wave : 2 * wave + 1, q_first = STRIP == 16 ? wave : 2 * wave;       // of the wave
+    const int base = q * L + 4 * g;
+    const TW* w_row = W + (size_t)min(n0 + row, N - 1) * ldw;
+    const TA* a_row = A + (size_t)min(row, M - 1) * lda;
+    const int blocks = max(0, min(L, K - q_first * L) + 15) / 16;             // until both of the wave's ranges are through
+    const int whole = max(0, min(L, K - q_last * L)) / 16 / AHEAD * AHEAD;    // ... of them with nothing to guard, in groups
+    f32x4 acc[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
+    for (int b = 0; b < whole; b += AHEAD) {
+        f32x4 w[AHEAD], a[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) w[i] = load4(w_row + base + (b + i) * 16);
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) a[i] = load4(a_row + base + (b + i) * 16);
+        __builtin_amdgcn_sched_barrier(0);                     // all of them in flight before the first product
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i)
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) acc[0] = mfma(w[i][kk], a[i][kk], acc[0]);
+    }
+    for (int b = whole; b < blocks; ++b) {
+        const int k = base + b * 16, at = min(k, K - 4);
+        f32x4 w = load4(w_row + at), a = load4(a_row + at);
+        if (k >= K) w = a = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) acc[0] = mfma(w[kk], a[kk], acc[0]);
+    }
+    if constexpr (STRIP == 16) sums[q][g * 16 + r] = acc[0];
+    else if ((g >> 1) == (r >> 3)) sums[q][(g & 1) * 8 + (r & 7)] = acc[0];     // (the instruction's other two quarters mix the ranges)
+    __syncthreads();
+    const int e = threadIdx.x;
+    if (e >= STRIP * STRIP / 4) return;
+    const int m = e % STRIP, n = n0 + 4 * (e / STRIP);
+    if (m >= M) return;
+    f32x4 v[RANGES];
+#pragma unroll
+    for (int z = 0; z < RANGES; ++z) v[z] = sums[z][e];
+    const f32x4 sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (n + i < N) put<TC, ACCUMULATE>(C, (size_t)m * ldc + n + i, sum[i]);
+}
+
+// ------------------------------------------------------------------------------------------- dispatch
+// Which products of up to 16 rows the kernel without tiles serves.  With 9 to 16 rows a narrow output has only its strips of 16 columns for
+// workgroups, and each reads the activations for itself: 2,048 x 8,192 at 16 rows takes 32 us there and 21 with tiles and k shared out,
+// 2,048 x 2,048 takes 10 against 11, 3,072 x 2,048 10 against 13.
+bool few_rows(int M, int N, int K) { return M <= 8 || (M <= FEW_ROWS && (K <= 4096 || N >= 16 * gi_compute_units())); }
+
+struct Cut { int bm, m_tiles, n_tiles, splits; };
+
+// Tiles of 64 rows, or of 32 where those hold at least a tenth fewer rows beyond M.  The ranges of k go to 1, 2, 4 or 8 workgroups: what
+// counts is the compute unit with the most of them (they share its matrix cores, and reach about half, two thirds and 0.72 of its 0.6
+// TFLOP/s when there are one, two and three or more), against writing and reading the parts.  301 rows of 2,048 x 2,048 (160 tiles): 50
+// us with one workgroup a tile, 41 with four.
+Cut cut_for(int M, int N, int K) {
+    const int units = gi_compute_units();
+    Cut c;
+    const long rows64 = (M + 63) / 64 * 64, rows32 = (M + 31) / 32 * 32;
+    c.bm = rows32 * 10 <= rows64 * 9 ? 32 : 64;
+    c.m_tiles = (M + c.bm - 1) / c.bm;
+    c.n_tiles = (N + BN - 1) / BN;
+    double best = 0;
+    c.splits = 1;
+    for (int z = 1; z <= RANGES; z *= 2) {
+        const long a_unit = ((long)c.m_tiles * c.n_tiles * z + units - 1) / units;
+        const double reached = a_unit == 1 ? 0.48 : a_unit == 2 ? 0.64 : 0.72;
+        const double compute = (double)a_unit * 2.0 * c.bm * BN * ((double)K / z + 64) / 6.0e5 / reached;                               // us
+        const double parts = z == 1 ? 0.0 : 4.0 + (double)z * M * N * 8 / 4.0e6;                                                         // us: a launch, 4 TB/s
+        if (z == 1 || compute + parts < best) { best = compute + parts; c.splits = z; }
+    }
+    return c;
+}
+
+template <typename TA, typename TW, typename TC, bool ACC>
+int launch(const TA* A, const TW* W, TC* C, float* part, long part_floats, int M, int N, int K, long lda, long ldw, long ldc, hipStream_t stream) {
+    const auto by4 = [](const void* p, size_t elem) { return ((uintptr_t)p & (4 * elem - 1)) == 0; };
+    const bool vector = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && by4(A, sizeof(TA)) && by4(W, sizeof(TW));
+    if (vector && few_rows(M, N, K)) {
+        // strips of 8 where strips of 16 would give fewer than two workgroups a compute unit
+        if (M <= 8 && N < 32 * gi_compute_units())
+            gemm_exact_few_rows_kernel<8, TA, TW, TC, ACC><<<(N + 7) / 8, 256, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc);
+        else
+            gemm_exact_few_rows_kernel<16, TA, TW, TC, ACC><<<(N + 15) / 16, 512, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc);
+        return 0;
+    }
+    Cut c = cut_for(M, N, K);
+    if (c.splits > 1 && (part == nullptr || part_floats < (long)c.splits * M * N)) c.splits = 1;
+    const long total = (long)c.m_tiles * c.n_tiles * c.splits;
+    GI_REQUIRE(total < 2147483647L - 8, "gemm_exact: M %d, N %d have too many tiles", M, N);
+    const unsigned grid = (unsigned)((total + 7) / 8 * 8);
+    float* to = c.splits > 1 ? part : nullptr;
+    if constexpr (sizeof(TA) == 4 && sizeof(TW) == 4 && sizeof(TC) == 4) {
+        if (vector && K % BK == 0) {
+#define RING(BM) gemm_exact_ring_kernel<BM, ACC><<<grid, 256, 0, stream>>>(A, W, C, to, M, N, K, lda, ldw, ldc, c.m_tiles, c.n_tiles, c.splits)
+            if (c.bm == 64) RING(64);
+            else RING(32);
+#undef RING
+            if (to) gemm_exact_add_parts_kernel<TC, ACC><<<(unsigned)(((size_t)M * N + 255) / 256), 256, 0, stream>>>(part, C, M, N, ldc, c.splits);
+            return 0;
         }
     }
-};
-
-template <typename TW, bool ACCUMULATE, int MR>
-__global__ __launch_bounds__(64) void gemm_exact_few_rows_kernel(const float* __restrict__ A, const TW* __restrict__ W, float* __restrict__ C, int M,
-                                                                 int N, int K, long lda, long ldw, long ldc) {
-    constexpr int PIECE = Sixteen<TW>::N, AHEAD = 32;        // elements per load; loads in flight per lane (512 bytes: four cache lines of its row)
-    const int n = blockIdx.x * 64 + threadIdx.x;
-    const TW* wrow = W + (size_t)min(n, N - 1) * ldw;
-    float acc[MR];
-#pragma unroll
-    for (int m = 0; m < MR; ++m) acc[m] = 0.f;
-    const int k_whole = K - K % (PIECE * AHEAD);
-    for (int k0 = 0; k0 < k_whole; k0 += PIECE * AHEAD) {
-        float w[AHEAD][PIECE];
-#pragma unroll
-        for (int u = 0; u < AHEAD; ++u) Sixteen<TW>::load(wrow + k0 + u * PIECE, w[u]);
-#pragma unroll
-        for (int u = 0; u < AHEAD; ++u)
-#pragma unroll
-            for (int j = 0; j < PIECE; ++j)
-#pragma unroll
-                for (int m = 0; m < MR; ++m)
-                    if (m < M) acc[m] = fmaf(A[(size_t)m * lda + k0 + u * PIECE + j], w[u][j], acc[m]);
-    }
-    for (int k = k_whole; k < K; ++k) {
-        const float w = load_f32(wrow, (size_t)k);
-#pragma unroll
-        for (int m = 0; m < MR; ++m)
-            if (m < M) acc[m] = fmaf(A[(size_t)m * lda + k], w, acc[m]);
-    }
-    if (n >= N) return;
-#pragma unroll
-    for (int m = 0; m < MR; ++m) {
-        if (m >= M) break;
-        const size_t o = (size_t)m * ldc + n;
-        C[o] = ACCUMULATE ? C[o] + acc[m] : acc[m];
-    }
-}
-
-template <typename TW>
-int launch_few_rows(const void* A, const void* W, void* C, int accumulate, int M, int N, int K, long lda, long ldw, long ldc, hipStream_t stream) {
-    const unsigned blocks = (unsigned)((N + 63) / 64);
-#define FEW(ACC, MR) gemm_exact_few_rows_kernel<TW, ACC, MR><<<blocks, 64, 0, stream>>>((const float*)A, (const TW*)W, (float*)C, M, N, K, lda, ldw, ldc)
-    if (M == 1) { if (accumulate) FEW(true, 1); else FEW(false, 1); }
-    else if (M == 2) { if (accumulate) FEW(true, 2); else FEW(false, 2); }
-    else { if (accumulate) FEW(true, FEW_ROWS); else FEW(false, FEW_ROWS); }
-#undef FEW
-    return 0;
-}
-
-template <typename TA, typename TW>
-int launch(const void* A, const void* W, void* C, int c_dtype, int accumulate, int M, int N, int K, long lda, long ldw, long ldc,
-           hipStream_t stream) {
-    dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
-#define GO(TC, ACC) gemm_exact_kernel<TA, TW, TC, ACC><<<grid, 256, 0, stream>>>((const TA*)A, (const TW*)W, (TC*)C, M, N, K, lda, ldw, ldc)
-    if (c_dtype == GI_F32 && accumulate) GO(float, true);
-    else if (c_dtype == GI_F32) GO(float, false);
-    else if (c_dtype == GI_BF16 && !accumulate) GO(bf16_t, false);
-    else return gi_fail("gemm_exact: output dtype %d with accumulate %d is not supported", c_dtype, accumulate);
-#undef GO
+#define TILED(BM, VEC) gemm_exact_tiled_kernel<BM, VEC, TA, TW, TC, ACC><<<grid, 256, 0, stream>>>(A, W, C, to, M, N, K, lda, ldw, ldc, c.m_tiles, c.n_tiles, c.splits)
+    if (c.bm == 64) { if (vector) TILED(64, true); else TILED(64, false); }
+    else { if (vector) TILED(32, true); else TILED(32, false); }
+#undef TILED
+    if (to) gemm_exact_add_parts_kernel<TC, ACC><<<(unsigned)(((size_t)M * N + 255) / 256), 256, 0, stream>>>(part, C, M, N, ldc, c.splits);
     return 0;
 }
 
 }  // namespace
 
+// floats of scratch the product wants for the parts of its sums (0: none; it also runs, slower, without)
+GI_API long gi_gemm_exact_scratch_floats(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || few_rows(M, N, K)) return 0;
+    const Cut c = cut_for(M, N, K);
+    return c.splits > 1 ? (long)c.splits * M * N : 0;
+}
+
 GI_API int gi_gemm_exact(const void* A, int a_dtype, const void* W, int w_dtype, void* C, int c_dtype, int accumulate, int M, int N, int K,
-                         long lda, long ldw, long ldc, hipStream_t stream) {
+                         long lda, long ldw, long ldc, float* part, long part_floats, hipStream_t stream) {
     GI_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_exact: M %d, N %d, K %d must be positive", M, N, K);
     GI_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm_exact: leading dimensions (%ld, %ld, %ld) too small for K %d, N %d", lda, ldw, ldc, K, N);
-    GI_REQUIRE((M + BM - 1) / BM <= 65535, "gemm_exact: M %d is too large", M);
+    GI_REQUIRE(K <= 2147483647 - 256, "gemm_exact: K %d is too large", K);
     int rc;
-    // a few rows of 32-bit activations into a 32-bit result: a lane per output column (the loads need 16-byte pieces of the weight rows)
-    const long w_piece = w_dtype == GI_F32 ? 4 : 8;
-    if (M <= FEW_ROWS && a_dtype == GI_F32 && c_dtype == GI_F32 && (w_dtype == GI_F32 || w_dtype == GI_BF16) && ldw % w_piece == 0 &&
-        ((uintptr_t)W & 15) == 0) {
-        rc = w_dtype == GI_F32 ? launch_few_rows<float>(A, W, C, accumulate, M, N, K, lda, ldw, ldc, stream)
-                               : launch_few_rows<bf16_t>(A, W, C, accumulate, M, N, K, lda, ldw, ldc, stream);
-        GI_CHECK_LAUNCH("gemm_exact (few rows)");
-        return rc;
-    }
-    if (a_dtype == GI_F32 && w_dtype == GI_F32) rc = launch<float, float>(A, W, C, c_dtype, accumulate, M, N, K, lda, ldw, ldc, stream);
-    else if (a_dtype == GI_F32 && w_dtype == GI_BF16) rc = launch<float, bf16_t>(A, W, C, c_dtype, accumulate, M, N, K, lda, ldw, ldc, stream);
-    else if (a_dtype == GI_BF16 && w_dtype == GI_BF16) rc = launch<bf16_t, bf16_t>(A, W, C, c_dtype, accumulate, M, N, K, lda, ldw, ldc, stream);
-    else if (a_dtype == GI_BF16 && w_dtype == GI_F32) rc = launch<bf16_t, float>(A, W, C, c_dtype, accumulate, M, N, K, lda, ldw, ldc, stream);
+#define GO(TA, TW, TC, ACC) rc = launch<TA, TW, TC, ACC>((const TA*)A, (const TW*)W, (TC*)C, part, part_floats, M, N, K, lda, ldw, ldc, stream)
+#define BY_OUT(TA, TW)                                                  \
+    if (c_dtype == GI_F32 && accumulate) GO(TA, TW, float, true);       \
+    else if (c_dtype == GI_F32) GO(TA, TW, float, false);               \
+    else if (c_dtype == GI_BF16 && !accumulate) GO(TA, TW, bf16_t, false); \
+    else return gi_fail("gemm_exact: output dtype %d with accumulate %d is not supported", c_dtype, accumulate)
+    if (a_dtype == GI_F32 && w_dtype == GI_F32) { BY_OUT(float, float); }
+    else if (a_dtype == GI_F32 && w_dtype == GI_BF16) { BY_OUT(float, bf16_t); }
+    else if (a_dtype == GI_BF16 && w_dtype == GI_BF16) { BY_OUT(bf16_t, bf16_t); }
+    else if (a_dtype == GI_BF16 && w_dtype == GI_F32) { BY_OUT(bf16_t, float); }
     else return gi_fail("gemm_exact: unknown operand dtypes %d, %d", a_dtype, w_dtype);
+#undef BY_OUT
+#undef GO
     if (rc) return rc;
     GI_CHECK_LAUNCH("gemm_exact");
     return 0;

@@ -33,7 +33,7 @@ _SIGNATURES = {
     "gi_gather_rows": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
     "gi_scale_rows": [c_void_p, c_int, c_int, c_long, c_float, c_void_p],
     "gi_softcap_rows": [c_void_p, c_int, c_int, c_long, c_float, c_void_p],
-    "gi_gemm_exact": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p],
+    "gi_gemm_exact": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long, c_void_p],
     "gi_attention_exact": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_long, c_int,
                            c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_void_p, c_long, c_int, c_void_p],
     "gi_rmsnorm_add": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_float, c_long, c_long, c_void_p],
@@ -135,6 +135,8 @@ def lib():
         l.gi_attention_decode_workgroups_per_unit.restype = c_int
         l.gi_attention_bf16_supports.argtypes = [c_int, c_int, c_int]
         l.gi_attention_bf16_supports.restype = c_int
+        l.gi_gemm_exact_scratch_floats.argtypes = [c_int, c_int, c_int]
+        l.gi_gemm_exact_scratch_floats.restype = c_long
         l.gi_gemm_bf16_scratch_floats.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_bf16_scratch_floats.restype = c_long
         l.gi_gemm_bf16_norm_parts.argtypes = [c_int, c_int, c_int]
@@ -533,8 +535,10 @@ def gemm_exact(a, w, out, accumulate=False):
         raise KernelError("gemm: operands need unit inner stride")
     if _profile is not None:
         _profile.note = (f"{n}x{k}", n * k * w.element_size())
+    n_part = _exact_scratch_floats(m, n, k)
+    part = torch.empty(n_part, dtype=torch.float32, device=out.device) if n_part else None
     _call("gi_gemm_exact", a.data_ptr(), _code(a, "gemm: a"), w.data_ptr(), _code(w, "gemm: w"), out.data_ptr(), _code(out, "gemm: out"),
-          1 if accumulate else 0, m, n, k, a.stride(0), w.stride(0), out.stride(0), _stream())
+          1 if accumulate else 0, m, n, k, a.stride(0), w.stride(0), out.stride(0), _ptr(part), n_part, _stream())
     return out
 
 
@@ -1392,6 +1396,11 @@ def gemm_bf16_supports(a, w, out) -> bool:
 
 # What the library says about a shape does not change while the process lives, and a step asks it some hundred times: the answers
 # are kept (a question costs a call through ctypes, about a microsecond of the host's time each).
+@lru_cache(maxsize=None)
+def _exact_scratch_floats(m, n, k) -> int:
+    return lib().gi_gemm_exact_scratch_floats(m, n, k)
+
+
 @lru_cache(maxsize=None)
 def _scratch_floats(m, n, k) -> int:
     return lib().gi_gemm_bf16_scratch_floats(m, n, k)

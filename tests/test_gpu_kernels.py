@@ -58,6 +58,27 @@ def test_gemm_exact_rows_alone_have_the_same_bits(w_dtype, k):
         assert torch.equal(few, wide[:rows])                                # adding onto what is there, the same in both kernels
 
 
+@pytest.mark.parametrize("m,n,k", [(64, 256, 8192), (33, 130, 2080), (300, 160, 64), (129, 65, 4128), (16, 2048, 8192), (17, 90, 32), (70, 100, 1000), (40, 70, 203)])
+def test_gemm_exact_kernels_agree_in_bits(m, n, k):
+    """Whole blocks of 32 k go through LDS in a ring (tiles of 32 and 64 rows, k shared out over 1 to 8 workgroups where the tiles are few),
+    other aligned rows are staged through registers, unaligned ones element by element, a few rows need no tiles: one order of every sum."""
+    a, w = randn(m, k, seed=31), randn(n, k, seed=32)
+    full = torch.empty(m, n, device=DEV)
+    ops().gemm_exact(a, w, full)
+    assert rel(full, a.double() @ w.double().T) < 2e-6
+    shifted = torch.zeros(n, -(-k // 4) * 4 + 4, device=DEV)[:, 1:1 + k].copy_(w)              # the same weights where no 16-byte load may touch them
+    out = torch.empty_like(full)
+    ops().gemm_exact(a, shifted, out)
+    assert torch.equal(out, full)
+    for rows in {1, min(8, m), min(16, m), min(32, m)}:
+        few = torch.ones(rows, n, device=DEV)
+        ops().gemm_exact(a[m - rows:], w, few, accumulate=True)
+        assert torch.equal(few, 1.0 + full[m - rows:])
+    wide = torch.empty(m + 200, n, device=DEV)
+    ops().gemm_exact(torch.cat([a, a.new_ones(200, k)]), w, wide)
+    assert torch.equal(wide[:m], full)
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 16, 8), (1, 2048, 2048), (3, 100, 136), (8, 130, 264), (16, 64, 128), (17, 1000, 520),
                                    (33, 48, 72), (64, 515, 1032), (65, 128, 64), (100, 300, 200), (128, 128, 128), (200, 257, 96),
                                    (513, 384, 1024), (2048, 96, 160),
