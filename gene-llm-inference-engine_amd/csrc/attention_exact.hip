@@ -1,15 +1,13 @@
 // Causal attention of single rows over a paged key/value cache, in true 32-bit arithmetic.
 //
-// One wave per (row, query head).  Row t of the request in slot[t] at position pos[t] sees the
+// Row t of the request in slot[t] at position pos[t] sees the
 // keys at positions lo .. pos[t] of its own request, lo = max(0, pos - window + 1) with a window,
 // the start of the row's chunk, pos - pos % chunk, with a mask cut into chunks, and 0 without either;
 // query head h uses key/value head h / (n_heads / n_kv).  Scores are scaled by `scale` (the caller's,
-// 1/sqrt(hd) by default) after the dot product, softmax is taken with a running maximum over tiles of 64
-// keys, and the weighted sum of the values follows in position order
-// (src/model/transformer.cpp:228-255, src/gpu/device_kernels.inc:377-449).  The softmax's
-// denominator is a 64-bit sum, as the reference's (src/kernels/kernels.cpp:95-100): a 32-bit
+// 1/sqrt(hd) by default) after the dot product (src/model/transformer.cpp:228-255, src/gpu/device_kernels.inc:377-449).  The softmax's
+// denominator is a 64-bit sum over groups of keys, as the reference's (src/kernels/kernels.cpp:95-100): a 32-bit
 // running sum over tens of thousands of keys loses digits that every output of the head then lacks.
-// The order of every sum depends on (pos, window, hd) only, so a row's result has the same bits
+// The order of every sum depends on (pos, window, chunk, hd) only, so a row's result has the same bits
 // whatever else is in the batch and whichever pages hold its request.
 //
 // With `cap` > 0 a scaled score s becomes cap * tanh(s / cap) before the softmax.
@@ -20,11 +18,295 @@
 // Cache of one layer: per page the keys [kv_head][place][hd], then the values transposed
 // [kv_head][vd][place] (vd channels a value head, hd a key head); table[slot][i] is the page of
 // positions i*page_size .. (i+1)*page_size - 1.
+//
+// Two kernels.  Which one serves depends on the data types and on hd, vd and the page size alone, so one model meets one of them:
+//   tiles    32-bit throughout, hd and vd multiples of 16 up to 128, pages of a multiple of 4: both products on the 32-bit matrix
+//            instructions, four waves a workgroup, long contexts shared out over workgroups;
+//   rows     everything else: one wave per (row, query head), keys 64 at a time.
 #include "common.h"
 
 namespace {
 
 constexpr int MAX_HD = 640;
+
+// --------------------------------------------------------------------------------------------- tiles
+// A workgroup takes up to 16 (row, query head) pairs of one key/value head: the heads that share it, for one row (decoding) or for
+// several neighbouring rows of the batch.  Keys are taken in spans of 256 positions that start at multiples of 256, a block of 64 to each
+// of the four waves.  A block gives, for each pair, the largest score m, the sum l of exp(s - m) and O = sum of exp(s - m) v; the
+// span's four blocks meet in LDS (largest m first, then the scaled l and O in order), and spans are merged one behind the other in
+// order of position, either by the workgroup itself or, where the context is shared out (`part`), by the second kernel: the same
+// operations either way.
+// The scores of 16 keys come out of the matrix instruction in the very registers in which the second product wants the probabilities
+// (a lane has the keys 4g .. 4g+3 of pair r), and the cache's transposed values are 16-byte pieces along the keys: nothing is laid
+// out anew.  Bound by the latency of a span's loads (all of a wave's keys and values are asked for at once) until the contexts are
+// long; one wave per (row, head) that walked its keys 64 at a time, every lane a key of its own, took 169 us a layer for 3 rows at 600
+// positions of the Llama-3.2-1B shape and 215 for a prompt of 301.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+constexpr int BLOCK = 64, SPAN = 4 * BLOCK, PAIRS = 16;
+
+// A span joins what came before it (m, l, and every O with the two factors): nothing happens for a row that sees no key of the span.
+struct Join { float before, span; };
+__device__ __forceinline__ Join join(float& m, double& l, float m_span, double l_span) {
+    if (m_span == -INFINITY) return {1.f, 0.f};
+    const float top = fmaxf(m, m_span);
+    const Join f = {expf(m - top), expf(m_span - top)};       // (m = -inf at the first span without sinks: 0)
+    l = fma(l_span, (double)f.span, l * (double)f.before);
+    m = top;
+    return f;
+}
+__device__ __forceinline__ float joined(float o, float o_span, Join f) { return f.span == 0.f && f.before == 1.f ? o : fmaf(o_span, f.span, o * f.before); }
+
+__device__ __forceinline__ int first_key(int pos, int window, int chunk) {
+    int lo = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
+    return chunk > 0 ? max(lo, pos - pos % chunk) : lo;
+}
+
+// what becomes of a head's channel in the end
+__device__ __forceinline__ float finished(float o, double l, const float* gate, long gate_stride, int gate_channels, int t, int h, int d) {
+    float inv = 1.0f / (float)l;
+    if (gate && !gate_channels) inv *= 1.0f / (1.0f + expf(-gate[(size_t)t * gate_stride + h]));
+    o *= inv;
+    if (gate && gate_channels) o *= 1.0f / (1.0f + expf(-gate[(size_t)t * gate_stride + (size_t)h * gate_channels + d]));
+    return o;
+}
+
+// One (row, head, span) of `part`: vd sums, then l (64-bit), then m.
+__host__ __device__ constexpr int part_floats(int vd) { return vd + 4; }
+
+template <int D>
+__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_kernel(const float* __restrict__ q, const float* __restrict__ cache, float* __restrict__ out,
+                                                                   const int* __restrict__ pos, const int* __restrict__ slot, const int* __restrict__ table,
+                                                                   int table_stride, long page_stride, int page_size, int n_rows, int n_heads, int n_kv, int hd, int vd,
+                                                                   int window, int chunk, float scale, float cap, const float* __restrict__ sinks,
+                                                                   const float* __restrict__ gate, long gate_stride, int gate_channels, int rows_a_tile,
+                                                                   float* __restrict__ part, int n_spans) {
+    __shared__ float o_s[4][PAIRS][D + 4];
+    __shared__ float m_s[4][PAIRS], l_s[4][PAIRS], f_s[4][PAIRS];        // of the blocks; f: their factors
+    __shared__ float m_all[PAIRS];
+    __shared__ double l_all[PAIRS];
+    __shared__ Join join_s[PAIRS];
+    __shared__ int t_s[PAIRS], h_s[PAIRS], run_s[PAIRS], lo_s[PAIRS], pos_s[PAIRS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
+    const int group = n_heads / n_kv, head_tiles = (group + PAIRS - 1) / PAIRS;
+    const int tile = blockIdx.x / (n_kv * head_tiles), kv = blockIdx.x / head_tiles % n_kv, ht = blockIdx.x % head_tiles;
+    const int heads_here = min(PAIRS, group - ht * PAIRS);
+    const int place = r / heads_here, t = tile * rows_a_tile + place, h = kv * group + ht * PAIRS + r % heads_here;
+    const bool valid = place < rows_a_tile && t < n_rows;
+    const int my_pos = valid ? pos[t] : 0, my_slot = valid ? slot[t] : -1, my_lo = valid ? first_key(my_pos, window, chunk) : 0;
+    f32x4 qv[D / 16];
+#pragma unroll
+    for (int c = 0; c < D / 16; ++c)
+        qv[c] = valid && c * 16 < hd ? *reinterpret_cast<const f32x4*>(q + ((size_t)t * n_heads + h) * hd + c * 16 + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
+    const long v_plane = (long)n_kv * page_size * hd;   // from a page's keys to its values
+
+    // Rows of one request at a time (a tile at the edge of two requests' rows takes as many turns).
+    bool todo = valid;
+    while (__ballot(todo) != 0) {
+        const int run_slot = __shfl(my_slot, (int)__ffsll((unsigned long long)__ballot(todo)) - 1, 64);
+        const bool in_run = todo && my_slot == run_slot;
+        todo = todo && !in_run;
+        int lo_min = in_run ? my_lo : 2147483647, lo_max = in_run ? my_lo : 0, p_min = in_run ? my_pos : 2147483647, p_max = in_run ? my_pos : 0;
+#pragma unroll
+        for (int off = 1; off < PAIRS; off <<= 1) {
+            lo_min = min(lo_min, __shfl_xor(lo_min, off, 64));
+            lo_max = max(lo_max, __shfl_xor(lo_max, off, 64));
+            p_min = min(p_min, __shfl_xor(p_min, off, 64));
+            p_max = max(p_max, __shfl_xor(p_max, off, 64));
+        }
+        lo_min = __builtin_amdgcn_readfirstlane(lo_min);
+        p_max = __builtin_amdgcn_readfirstlane(p_max);
+        const int* tab = table + (size_t)run_slot * table_stride;
+        if (tid < PAIRS) {
+            m_all[tid] = sinks && valid ? sinks[h] : -INFINITY;
+            l_all[tid] = sinks ? 1.0 : 0.0;
+            t_s[tid] = t; h_s[tid] = h; run_s[tid] = in_run; lo_s[tid] = my_lo; pos_s[tid] = my_pos;
+        }
+        float o_all[PAIRS * D / 256];
+#pragma unroll
+        for (int e = 0; e < PAIRS * D / 256; ++e) o_all[e] = 0.f;
+
+        for (int s = lo_min / SPAN + blockIdx.y; s <= p_max / SPAN; s += gridDim.y) {
+            const int b0 = s * SPAN + wave * BLOCK;
+            float m = -INFINITY, l = 0.f;
+            if (b0 <= p_max && b0 + BLOCK > lo_min) {                     // (the same for the wave)
+                f32x4 kk[4][D / 16], vv[4][D / 16];
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt) {
+                    const int key = max(min(b0 + kt * 16 + r, p_max), lo_min);
+                    const float* from = cache + (size_t)tab[key / page_size] * page_stride + ((size_t)kv * page_size + key % page_size) * hd + 4 * g;
+#pragma unroll
+                    for (int c = 0; c < D / 16; ++c) kk[kt][c] = c * 16 < hd ? *reinterpret_cast<const f32x4*>(from + c * 16) : f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt) {
+                    const int first = b0 + kt * 16 + 4 * g, key = max(min(first, p_max), lo_min) & ~3;
+                    const float* from = cache + (size_t)tab[key / page_size] * page_stride + v_plane + ((size_t)kv * vd + r) * page_size + key % page_size;
+#pragma unroll
+                    for (int c = 0; c < D / 16; ++c) vv[kt][c] = c * 16 < vd ? *reinterpret_cast<const f32x4*>(from + (size_t)c * 16 * page_size) : f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+                f32x4 sc[4];
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt) {
+                    sc[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int c = 0; c < D / 16; ++c)
+                        if (c * 16 < hd) {
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) sc[kt] = mfma(kk[kt][c][j], qv[c][j], sc[kt]);
+                        }
+                }
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int key = b0 + kt * 16 + 4 * g + i;
+                        float x = sc[kt][i] * scale;
+                        if (cap > 0.f) x = cap * tanhf(x / cap);
+                        sc[kt][i] = in_run && key <= my_pos && key >= my_lo ? x : -INFINITY;
+                        m = fmaxf(m, sc[kt][i]);
+                    }
+                m = fmaxf(m, __shfl_xor(m, 16, 64));
+                m = fmaxf(m, __shfl_xor(m, 32, 64));
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        sc[kt][i] = sc[kt][i] == -INFINITY ? 0.f : expf(sc[kt][i] - m);
+                        l += sc[kt][i];
+                    }
+                l += __shfl_xor(l, 16, 64);
+                l += __shfl_xor(l, 32, 64);
+                // A probability of zero must not meet a value that is no number: places nobody has written, and, where some pair of the
+                // tile does not see all of the block, values a pair does not see (rare: then every row's own sum with those left out).
+                bool odd = false;
+                const bool all_seen = b0 >= lo_max && b0 + BLOCK - 1 <= p_min;
+                if (!all_seen) {
+#pragma unroll
+                    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int key = b0 + kt * 16 + 4 * g + i;
+#pragma unroll
+                            for (int c = 0; c < D / 16; ++c) {
+                                if (key > p_max || key < lo_min) vv[kt][c][i] = 0.f;
+                                odd = odd || !(fabsf(vv[kt][c][i]) < INFINITY);
+                            }
+                        }
+                }
+                f32x4 o[D / 16];
+#pragma unroll
+                for (int c = 0; c < D / 16; ++c) {
+                    o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    if (c * 16 >= vd) continue;
+#pragma unroll
+                    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) o[c] = mfma(vv[kt][c][j], sc[kt][j], o[c]);
+                }
+                if (__ballot(odd) != 0) {
+                    for (int row = 0; row < rows_a_tile; ++row) {
+                        const int row_pos = __shfl(my_pos, row * heads_here, 64), row_lo = __shfl(my_lo, row * heads_here, 64);
+#pragma unroll
+                        for (int c = 0; c < D / 16; ++c) {
+                            f32x4 own = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                            for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+                                for (int j = 0; j < 4; ++j) {
+                                    const int key = b0 + kt * 16 + 4 * g + j;
+                                    own = mfma(key > row_pos || key < row_lo ? 0.f : vv[kt][c][j], sc[kt][j], own);
+                                }
+                            if (place == row) o[c] = own;
+                        }
+                    }
+                }
+#pragma unroll
+                for (int c = 0; c < D / 16; ++c)
+                    if (c * 16 < vd) *reinterpret_cast<f32x4*>(&o_s[wave][r][c * 16 + 4 * g]) = o[c];
+            }
+            if (g == 0) { m_s[wave][r] = m; l_s[wave][r] = l; }
+            __syncthreads();
+            if (tid < PAIRS) {
+                float top = -INFINITY;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) top = fmaxf(top, m_s[b][tid]);
+                double sum = 0.0;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const float f = m_s[b][tid] == -INFINITY ? 0.f : expf(m_s[b][tid] - top);
+                    f_s[b][tid] = f;
+                    sum = fma((double)l_s[b][tid], (double)f, sum);
+                }
+                if (part) {
+                    const int at = s - lo_s[tid] / SPAN;
+                    if (run_s[tid] && at >= 0 && s <= pos_s[tid] / SPAN && at < n_spans) {
+                        float* p = part + (((size_t)t_s[tid] * n_heads + h_s[tid]) * n_spans + at) * part_floats(vd) + vd;
+                        *reinterpret_cast<double*>(p) = sum;
+                        p[2] = top;
+                    }
+                } else {
+                    float m_now = m_all[tid];
+                    double l_now = l_all[tid];
+                    join_s[tid] = join(m_now, l_now, top, sum);
+                    m_all[tid] = m_now;
+                    l_all[tid] = l_now;
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < PAIRS * D / 256; ++e) {
+                const int at = tid + 256 * e, pair = at / vd, d = at % vd;
+                if (pair >= PAIRS) break;
+                float o = 0.f;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const float f = f_s[b][pair];
+                    if (f != 0.f) o = fmaf(o_s[b][pair][d], f, o);         // (an empty block has left nothing there)
+                }
+                if (part) {
+                    const int span = s - lo_s[pair] / SPAN;
+                    if (run_s[pair] && span >= 0 && s <= pos_s[pair] / SPAN && span < n_spans)
+                        part[(((size_t)t_s[pair] * n_heads + h_s[pair]) * n_spans + span) * part_floats(vd) + d] = o;
+                } else {
+                    o_all[e] = joined(o_all[e], o, join_s[pair]);
+                }
+            }
+            __syncthreads();
+        }
+        if (!part) {
+#pragma unroll
+            for (int e = 0; e < PAIRS * D / 256; ++e) {
+                const int at = tid + 256 * e, pair = at / vd, d = at % vd;
+                if (pair >= PAIRS) break;
+                if (run_s[pair])
+                    out[((size_t)t_s[pair] * n_heads + h_s[pair]) * vd + d] = finished(o_all[e], l_all[pair], gate, gate_stride, gate_channels, t_s[pair], h_s[pair], d);
+            }
+        }
+        __syncthreads();                                  // the next turn writes the pairs' numbers anew
+    }
+}
+
+// The spans of a (row, head), left by several workgroups, joined in order.
+__global__ __launch_bounds__(128) void attention_exact_join_kernel(const float* __restrict__ part, float* __restrict__ out, const int* __restrict__ pos, int n_heads, int vd,
+                                                                  int window, int chunk, const float* __restrict__ sinks, const float* __restrict__ gate, long gate_stride,
+                                                                  int gate_channels, int n_spans) {
+    const int t = blockIdx.x / n_heads, h = blockIdx.x % n_heads, d = threadIdx.x, p = pos[t];
+    const int count = min(p / SPAN - first_key(p, window, chunk) / SPAN + 1, n_spans);
+    const float* from = part + (size_t)blockIdx.x * n_spans * part_floats(vd);
+    float m = sinks ? sinks[h] : -INFINITY, o = 0.f;
+    double l = sinks ? 1.0 : 0.0;
+    const int channel = min(d, vd - 1);
+    for (int s = 0; s < count; ++s, from += part_floats(vd)) {
+        const float o_span = from[channel];
+        const Join f = join(m, l, from[vd + 2], *reinterpret_cast<const double*>(from + vd));
+        o = joined(o, o_span, f);
+    }
+    if (d < vd) out[(size_t)blockIdx.x * vd + d] = finished(o, l, gate, gate_stride, gate_channels, t, h, d);
+}
+
+// ---------------------------------------------------------------------------------------------- rows
 
 template <typename TQ, typename TC, typename TO>
 __global__ __launch_bounds__(64) void attention_exact_kernel(const TQ* __restrict__ q, const TC* __restrict__ cache, TO* __restrict__ out,
@@ -39,8 +321,7 @@ __global__ __launch_bounds__(64) void attention_exact_kernel(const TQ* __restric
     const int t = blockIdx.x / n_heads, h = blockIdx.x % n_heads, g = h / (n_heads / n_kv);
     const int p_row = pos[t];
     const int* tab = table + (size_t)slot[t] * table_stride;
-    int lo = (window > 0 && p_row - window + 1 > 0) ? p_row - window + 1 : 0;
-    if (chunk > 0) lo = max(lo, p_row - p_row % chunk);
+    const int lo = first_key(p_row, window, chunk);
     for (int d = lane; d < hd; d += 64) q_s[d] = load_f32(q, (size_t)t * n_heads * hd + h * hd + d);
     __syncthreads();
 
@@ -84,16 +365,10 @@ __global__ __launch_bounds__(64) void attention_exact_kernel(const TQ* __restric
             }
         }
     }
-    float inv = 1.0f / (float)l;
-    if (gate && !gate_channels) inv *= 1.0f / (1.0f + expf(-gate[(size_t)t * gate_stride + h]));
 #pragma unroll
     for (int i = 0; i < MAX_HD / 64; ++i) {
         const int d = lane + 64 * i;
-        if (d < vd) {
-            float o = acc[i] * inv;
-            if (gate && gate_channels) o *= 1.0f / (1.0f + expf(-gate[(size_t)t * gate_stride + (size_t)h * gate_channels + d]));
-            store_f32(out, (size_t)t * n_heads * vd + h * vd + d, o);
-        }
+        if (d < vd) store_f32(out, (size_t)t * n_heads * vd + h * vd + d, finished(acc[i], l, gate, gate_stride, gate_channels, t, h, d));
     }
 }
 
@@ -101,10 +376,25 @@ __global__ __launch_bounds__(64) void attention_exact_kernel(const TQ* __restric
 
 GI_API int gi_attention_exact_max_head_size() { return MAX_HD; }
 
+// Whether the kernel with tiles serves these sizes (all operands 32-bit and aligned).
+static bool takes_tiles(int hd, int vd, int page_size) { return hd % 16 == 0 && vd % 16 == 0 && hd <= 128 && vd <= 128 && page_size % 4 == 0; }
+
+// How many spans of 256 keys the widest row of a step has at most, 0 where they are not shared out: `seen` positions at most are seen by a row.
+// They are shared out while the tiles alone give fewer than two workgroups a compute unit, and the parts stay under 64 MB.
+GI_API int gi_attention_exact_spans(int n_rows, int single_rows, int n_heads, int n_kv, int hd, int vd, int page_size, int seen) {
+    if (n_rows <= 0 || n_kv <= 0 || n_heads % n_kv != 0 || seen <= SPAN || !takes_tiles(hd, vd, page_size)) return 0;
+    const int group = n_heads / n_kv, a_tile = single_rows ? 1 : group < PAIRS ? PAIRS / group : 1;
+    const long tiles = (long)((n_rows + a_tile - 1) / a_tile) * n_kv * ((group + PAIRS - 1) / PAIRS);
+    const long spans = ((long)seen + SPAN - 1) / SPAN + 1;
+    if (tiles >= 2L * gi_compute_units() || spans * n_rows * n_heads * part_floats(vd) > (16L << 20)) return 0;
+    return (int)spans;
+}
+GI_API long gi_attention_exact_part_floats(int n_rows, int n_heads, int vd, int n_spans) { return (long)n_rows * n_heads * n_spans * part_floats(vd); }
+
 GI_API int gi_attention_exact(const void* q, int q_dtype, const void* cache, int cache_dtype, void* out, int out_dtype, const int* pos,
                               const int* slot, const int* table, int table_stride, long page_stride, int page_size, int n_rows,
                               int n_heads, int n_kv, int hd, int vd, int window, int chunk, float scale, float cap, const float* sinks, const float* gate,
-                              long gate_stride, int gate_channels, hipStream_t stream) {
+                              long gate_stride, int gate_channels, int single_rows, float* part, long part_size, int n_spans, hipStream_t stream) {
     GI_REQUIRE(n_rows > 0 && n_heads > 0 && n_kv > 0 && n_heads % n_kv == 0, "attention_exact: bad head counts (%d rows, %d heads, %d kv heads)",
                n_rows, n_heads, n_kv);
     GI_REQUIRE(hd > 0 && hd <= MAX_HD, "attention_exact: head size %d is outside 1..%d", hd, MAX_HD);
@@ -114,6 +404,26 @@ GI_API int gi_attention_exact(const void* q, int q_dtype, const void* cache, int
     GI_REQUIRE(page_size > 0 && page_stride >= (long)n_kv * page_size * (hd + vd), "attention_exact: page stride %ld too small", page_stride);
     GI_REQUIRE((long)n_rows * n_heads < 2147483647L, "attention_exact: too many (row, head) pairs");
     const unsigned grid = (unsigned)(n_rows * n_heads);
+    const auto aligned = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+    if (q_dtype == GI_F32 && cache_dtype == GI_F32 && out_dtype == GI_F32 && takes_tiles(hd, vd, page_size) && page_stride % 4 == 0 && aligned(q) && aligned(cache)) {
+        const int group = n_heads / n_kv, a_tile = single_rows ? 1 : group < PAIRS ? PAIRS / group : 1;      // (a lone new row a request: a tile of several would take a turn for each)
+        if (n_spans > 0) {
+            GI_REQUIRE(part != nullptr && aligned(part) && part_size >= gi_attention_exact_part_floats(n_rows, n_heads, vd, n_spans) && n_spans <= 65535,
+                       "attention_exact: sharing the keys out needs %ld floats", gi_attention_exact_part_floats(n_rows, n_heads, vd, n_spans));
+        } else {
+            part = nullptr;
+        }
+        const dim3 tiles((unsigned)((n_rows + a_tile - 1) / a_tile) * n_kv * ((group + PAIRS - 1) / PAIRS), part ? n_spans : 1);
+#define TILES(D)                                                                                                                           \
+    attention_exact_tiles_kernel<D><<<tiles, 256, 0, stream>>>((const float*)q, (const float*)cache, (float*)out, pos, slot, table, table_stride, page_stride, page_size, n_rows, \
+                                                               n_heads, n_kv, hd, vd, window, chunk, scale, cap, sinks, gate, gate_stride, gate_channels, a_tile, part, n_spans)
+        if (hd <= 64 && vd <= 64) TILES(64);
+        else TILES(128);
+#undef TILES
+        if (part) attention_exact_join_kernel<<<grid, 128, 0, stream>>>(part, (float*)out, pos, n_heads, vd, window, chunk, sinks, gate, gate_stride, gate_channels, n_spans);
+        GI_CHECK_LAUNCH("attention_exact (tiles)");
+        return 0;
+    }
 #define GO(TQ, TC, TO)                                                                                                          \
     attention_exact_kernel<TQ, TC, TO><<<grid, 64, 0, stream>>>((const TQ*)q, (const TC*)cache, (TO*)out, pos, slot, table, table_stride, \
                                                                 page_stride, page_size, n_heads, n_kv, hd, vd, window, chunk, scale, cap, sinks, gate, gate_stride, gate_channels)

@@ -35,7 +35,7 @@ _SIGNATURES = {
     "gi_softcap_rows": [c_void_p, c_int, c_int, c_long, c_float, c_void_p],
     "gi_gemm_exact": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long, c_void_p],
     "gi_attention_exact": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_long, c_int,
-                           c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_void_p, c_long, c_int, c_void_p],
+                           c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_void_p, c_long, c_int, c_int, c_void_p, c_long, c_int, c_void_p],
     "gi_rmsnorm_add": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_float, c_long, c_long, c_void_p],
     "gi_rmsnorm_add_norm": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_float, c_long, c_long, c_long, c_void_p],
     "gi_norm_rope_store": [c_void_p, c_void_p, c_void_p, c_long, c_long, c_long, c_void_p, c_void_p, c_int, c_float, c_void_p, c_void_p, c_int,
@@ -129,6 +129,10 @@ def lib():
         l.gi_argmax_chunks.restype = c_int
         l.gi_sample_filtered_histogram_bytes.argtypes = []
         l.gi_sample_filtered_histogram_bytes.restype = c_int
+        l.gi_attention_exact_spans.argtypes = [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int]
+        l.gi_attention_exact_spans.restype = c_int
+        l.gi_attention_exact_part_floats.argtypes = [c_int, c_int, c_int, c_int]
+        l.gi_attention_exact_part_floats.restype = c_long
         l.gi_attention_exact_max_head_size.argtypes = []
         l.gi_attention_exact_max_head_size.restype = c_int
         l.gi_attention_decode_workgroups_per_unit.argtypes = [c_int, c_int, c_int, c_int]
@@ -557,12 +561,14 @@ def _check_paged(cache, table, what):
 
 
 def attention_exact(q, cache, out, positions, slots, table, n_heads, n_kv, hd, window=None, scale=None, *, page_size=None, value_dim=None,
-                    chunk=None, sinks=None, gate=None, cap=None, channel_gate=None):
+                    chunk=None, sinks=None, gate=None, cap=None, channel_gate=None, single_rows=False, max_context=None):
     """Each row attends over its request's cached keys up to its own position, no further back than `window` positions and not
     beyond the start of its own chunk of `chunk` positions.  value_dim: channels of a value head (hd if not given); sinks:
     float32 [heads], a score per head that joins the softmax's denominator only; gate: float32 [n, >= heads] (unit inner
     stride), head h's output is multiplied by sigmoid(gate[t, h]); channel_gate: float32 [n, heads*value_dim], the output is
-    multiplied by its sigmoid element by element; cap: a scaled score s becomes cap * tanh(s / cap)."""
+    multiplied by its sigmoid element by element; cap: a scaled score s becomes cap * tanh(s / cap).  What the caller knows of the
+    step and the results do not depend on: single_rows (every row is its request's only one), max_context (no row lies beyond that
+    many positions; without it no row's keys are shared out over workgroups)."""
     _dev(q, cache, out, positions, slots, table, sinks, gate, channel_gate)
     if cap is not None and not cap > 0:
         raise KernelError("attention: the scores' cap must be positive")
@@ -580,11 +586,23 @@ def attention_exact(q, cache, out, positions, slots, table, n_heads, n_kv, hd, w
     gate, gate_stride, gate_channels = _gates(gate, channel_gate, n, n_heads, vd)
     _i32(positions, "attention: positions", n)
     _i32(slots, "attention: slots", n)
+    part, n_part, n_spans = None, 0, 0
+    if max_context is not None and q.dtype == torch.float32:
+        seen = min([int(max_context)] + ([int(window)] if window else []) + ([int(chunk)] if chunk else []))
+        n_spans = _exact_spans(n, 1 if single_rows else 0, n_heads, n_kv, hd, vd, page_size, -(-seen // 256) * 256)
+        if n_spans:
+            n_part = lib().gi_attention_exact_part_floats(n, n_heads, vd, n_spans)
+            part = torch.empty(n_part, dtype=torch.float32, device=out.device)
     _call("gi_attention_exact", q.data_ptr(), _code(q, "attention: q"), cache.data_ptr(), _code(cache, "attention: cache"), out.data_ptr(),
           _code(out, "attention: out"), positions.data_ptr(), slots.data_ptr(), table.data_ptr(), table.stride(0), cache.stride(0),
           page_size, n, n_heads, n_kv, hd, vd, int(window or 0), int(chunk or 0), float(scale if scale is not None else hd ** -0.5),
-          float(cap or 0.0), _ptr(sinks), _ptr(gate), gate_stride, gate_channels, _stream())
+          float(cap or 0.0), _ptr(sinks), _ptr(gate), gate_stride, gate_channels, 1 if single_rows else 0, _ptr(part), n_part, n_spans, _stream())
     return out
+
+
+@lru_cache(maxsize=1024)
+def _exact_spans(n, single_rows, n_heads, n_kv, hd, vd, page_size, seen) -> int:
+    return lib().gi_attention_exact_spans(n, single_rows, n_heads, n_kv, hd, vd, page_size, seen)
 
 
 def _gates(gate, channel_gate, n, n_heads, vd):
@@ -1344,7 +1362,16 @@ def attention(q, cache, out, ctx, table, n_heads, n_kv, hd, window=None):
         plan = _plan_of(ctx)
         if (not plan.n_tiles or attention_bf16_supports(hd, page_size, True)) and (not plan.n_decode or attention_bf16_supports(hd, page_size, False)):
             return attention_bf16(q, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window)
-    return attention_exact(q, cache, out, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window)
+    return attention_exact(q, cache, out, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, single_rows=ctx.max_seg_len == 1,
+                           max_context=_longest_context(ctx))
+
+
+def _longest_context(ctx) -> int:
+    """Positions of the longest context of the step, or of what a captured pass is made for."""
+    plan = ctx.memo.get("attention_plan")
+    if plan is not None:
+        return max(plan.max_decode_context, plan.max_tile_context)
+    return max(p + n for p, n in zip(ctx.seg_pos0, ctx.seg_len))
 
 
 def attention_general(q, cache, out, ctx, table, n_heads, n_kv, hd, *, page_size, value_dim=None, window=None, chunk=None, scale=None, sinks=None, gate=None,
@@ -1360,7 +1387,8 @@ def attention_general(q, cache, out, ctx, table, n_heads, n_kv, hd, *, page_size
             return attention_bf16(q, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, scale, chunk=chunk, sinks=sinks, gate=gate, cap=cap,
                                   channel_gate=channel_gate)
     return attention_exact(q, cache, out, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, scale, page_size=page_size,
-                           value_dim=value_dim, chunk=chunk, sinks=sinks, gate=gate, cap=cap, channel_gate=channel_gate)
+                           value_dim=value_dim, chunk=chunk, sinks=sinks, gate=gate, cap=cap, channel_gate=channel_gate, single_rows=ctx.max_seg_len == 1,
+                           max_context=_longest_context(ctx))
 
 
 # Up to so many rows the decode kernel rotates and writes the pages itself.  It saves the rotation kernel's launch wherever the

@@ -703,6 +703,41 @@ def test_prompt_attention_with_scores_that_climb_along_the_context(n_heads, n_kv
     assert worst_row < 3e-2, worst_row                                     # no row is off by a factor
 
 
+@pytest.mark.parametrize("n_heads,n_kv,hd,ps,window,chunk", [(4, 2, 64, 16, None, None), (6, 2, 128, 12, None, None), (40, 2, 32, 4, None, None), (3, 3, 96, 16, 300, None),
+                                                             (8, 1, 16, 20, None, 320), (32, 8, 64, 16, 256, None)])
+def test_attention_exact_has_one_order_of_sums(n_heads, n_kv, hd, ps, window, chunk):
+    """32-bit: tiles of several rows, of one row, contexts shared out over workgroups or not, rows alone: equal in bits; at contexts around
+    the blocks of 64 keys and spans of 256.  A value that is no number is met only by the rows that see its position."""
+    contexts = [1025, 256, 64, 513]
+    cache, table, dense = build_paged(contexts, n_kv, hd, ps, torch.float32, seed=hd + n_heads)
+    segs = [(0, 1018, 7), (1, 255, 1), (2, 0, 64), (3, 510, 3), (0, 766, 3)]
+    rows = [(slot, pos0 + i) for slot, pos0, n in segs for i in range(n)]
+    T = len(rows)
+    q = randn(T, n_heads * hd, seed=3)
+    pos = torch.tensor([p for _, p in rows], dtype=torch.int32, device=DEV)
+    slots = torch.tensor([s_ + 1 for s_, _ in rows], dtype=torch.int32, device=DEV)
+
+    def attend(pick=slice(None), **known):
+        out = torch.full((T, n_heads * hd), float("nan"), device=DEV)[pick]
+        return ops().attention_exact(q[pick].contiguous(), cache, out, pos[pick].contiguous(), slots[pick].contiguous(), table, n_heads, n_kv, hd, window, chunk=chunk, **known)
+
+    whole = attend()
+    lows = [max(0, p - window + 1) if window else p - p % chunk if chunk else 0 for _, p in rows]
+    want = torch.cat([plain_attention_rows(q[i:i + 1], {s_: (dense[s_][0][lo:], dense[s_][1][lo:])}, [(s_, p - lo)], n_heads, n_kv, hd, None)
+                      for i, ((s_, p), lo) in enumerate(zip(rows, lows))])
+    assert rel(whole, want) < 2e-6
+    assert torch.equal(attend(max_context=1025), whole) and torch.equal(attend(max_context=4096), whole)
+    assert torch.equal(attend(single_rows=True), whole) and torch.equal(attend(single_rows=True, max_context=1025), whole)
+    for i in (0, 6, 7, 40, T - 4, T - 1):
+        assert torch.equal(attend(slice(i, i + 1)), whole[i:i + 1]) and torch.equal(attend(slice(i, i + 1), max_context=2048), whole[i:i + 1])
+    place = 1022                                             # of request 0, whose rows 1018 .. 1024 share tiles
+    cache[int(table[1, place // ps]), 1].view(n_kv, hd, ps)[:, :, place % ps] = float("inf")
+    for known in (dict(), dict(max_context=1025), dict(single_rows=True)):
+        hurt = attend(**known)
+        sees = torch.tensor([s_ == 0 and p >= place and lo <= place for (s_, p), lo in zip(rows, lows)], device=DEV)
+        assert torch.equal(hurt[~sees], whole[~sees]) and not bool(torch.isfinite(hurt[sees]).any())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_finds_one_far_key(dtype):
     """Among 700 keys one is scaled so that its score stands out: the output must be its value."""
