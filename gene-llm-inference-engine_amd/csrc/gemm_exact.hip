@@ -56,9 +56,10 @@ __device__ __forceinline__ void put(TC* C, size_t o, float v) {
 // a sixteenth of bfloat16's): a wave's tile of 32 x 32 (BM 64) needs 4 KB of LDS for 512 clocks of matrix instructions, so what
 // counts is enough workgroups a compute unit to cover the loads' latency and no compute unit left idle; hence small tiles and, where the
 // tiles are few, the eight ranges of k shared out over `splits` workgroups (each finishes its part of the tree and leaves it in
-// `part`, a second kernel adds the parts).  The ring kernel below reaches 110 TFLOP/s of the 154 that a bare loop of these instructions
-// makes (600 rows of 128,256 x 2,048; 64 x 128, 128 x 64 and 128 x 128 tiles reach no more); the kernel of single fused multiply-adds
-// that stood here before made 19 at 301 rows of the Llama-3.2-1B shape, where this one makes 75 (97 on the widest products).
+// `part`, a second kernel adds the parts).  The ring kernel below reaches 123 TFLOP/s of the 154 that a bare loop of these instructions
+// makes (600 rows of 128,256 x 2,048; tiles of 64 x 128, 128 x 64 and 128 x 128 reach no more; 110 before a stage had almost no vector
+// instructions of its own); the kernel of single fused multiply-adds
+// that stood here before made 19 at 301 rows of the Llama-3.2-1B shape, where this one makes 70 to 120.
 constexpr int BN = 64, BK = 32;
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
@@ -183,31 +184,37 @@ __global__ __launch_bounds__(256) void gemm_exact_ring_kernel(const float* __res
     const int total = m_tiles * n_tiles * splits, each = (total + 7) / 8, u = (blockIdx.x & 7) * each + (blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= each || u >= total) return;
     const int m0 = (u % m_tiles) * BM, n0 = (u / m_tiles % n_tiles) * BN, z = u / (m_tiles * n_tiles);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
     const int wm = (wave % WAVES_M) * 32, wn = (wave / WAVES_M) * (BN / WAVES_N);
     const int per_range = range_length(K) / BK, q0 = z * (RANGES / splits), q1 = q0 + RANGES / splits;
     const int s_begin = q0 * per_range, s_end = max(s_begin, min(q1 * per_range, K / BK));
 
-    const float* src[LOADS];                       // this lane's 16 bytes of each of its wave's loads, at k = 0; LDS is filled in order, so the chunk is chosen here
+    // Vector instructions take the matrix instructions' place, so a stage has hardly any: a load's address is a scalar base (the tile's
+    // first row, advanced by the stage's k) plus an offset that stays, an LDS read's one of four registers plus a constant.
+    // LDS is filled in order, so a lane chooses the chunk that belongs at its place.
+    const float *a_tile = A + (size_t)m0 * lda, *w_tile = W + (size_t)n0 * ldw;
+    unsigned src[LOADS];
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
         const int row = (wave * LOADS + i) * 8 + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
-        src[i] = (row < BM ? A + (size_t)min(m0 + row, M - 1) * lda : W + (size_t)min(n0 + row - BM, N - 1) * ldw) + 4 * c;
+        src[i] = (unsigned)((row < BM ? min(row, M - 1 - m0) * lda : min(row - BM, N - 1 - n0) * ldw) + 4 * c) * 4;
     }
     const unsigned ring_base = (unsigned)(size_t)(lds_ptr_t)ring;
     // (written as assembly so that the compiler does not wait for them; the counted wait and the barrier below order them against the reads)
-    auto issue = [&](int s) {
+    auto issue = [&](int s, int slot) {
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
-            const unsigned dst = __builtin_amdgcn_readfirstlane(ring_base + (((s - s_begin) % STAGES) * ROWS + (wave * LOADS + i) * 8) * BK * 4);
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src[i] + (size_t)s * BK) : "memory", "m0");
+            const unsigned dst = ring_base + (slot * ROWS + (wave * LOADS + i) * 8) * BK * 4;
+            const float* base = ((wave * LOADS + i) * 8 < BM ? a_tile : w_tile) + s * BK;
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(src[i]), "s"(base) : "memory", "m0");
         }
     };
     f32x4 acc[TN * TM], t[3][TN * TM];
 #pragma unroll
     for (int i = 0; i < STAGES - 1; ++i)
-        if (s_begin + i < s_end) issue(s_begin + i);
-    int s = s_begin;
+        if (s_begin + i < s_end) issue(s_begin + i, i);
+    const int a_at[2] = {chunk_at(wm + r, g), chunk_at(wm + r, 4 + g)}, w_at[2] = {BM * BK + chunk_at(wn + r, g), BM * BK + chunk_at(wn + r, 4 + g)};
+    int s = s_begin, slot = 0;
     for (int q = q0; q < q1; ++q) {
 #pragma unroll
         for (int i = 0; i < TN * TM; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -217,17 +224,18 @@ __global__ __launch_bounds__(256) void gemm_exact_ring_kernel(const float* __res
             else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();                                                          // everyone's has, and everyone has read stage s - 1
             asm volatile("" ::: "memory");
-            if (s + STAGES - 1 < s_end) issue(s + STAGES - 1);
-            const float *as = ring + ((s - s_begin) % STAGES) * ROWS * BK, *ws = as + BM * BK;
+            if (s + STAGES - 1 < s_end) issue(s + STAGES - 1, slot == 0 ? STAGES - 1 : slot - 1);      // into the place of stage s - 1
+            const float* stage = ring + slot * ROWS * BK;
+            slot = slot + 1 == STAGES ? 0 : slot + 1;
             f32x4 a[2][TM], w[2][TN];
-            auto read = [&](int b) {
+            // (rows 16 apart have the same permutation of chunks)
 #pragma unroll
-                for (int i = 0; i < TM; ++i) a[b][i] = *reinterpret_cast<const f32x4*>(&as[chunk_at(wm + i * 16 + r, b * 4 + g)]);
+            for (int b = 0; b < BK / 16; ++b) {
 #pragma unroll
-                for (int j = 0; j < TN; ++j) w[b][j] = *reinterpret_cast<const f32x4*>(&ws[chunk_at(wn + j * 16 + r, b * 4 + g)]);
-            };
-            read(0);
-            read(1);
+                for (int i = 0; i < TM; ++i) a[b][i] = *reinterpret_cast<const f32x4*>(stage + a_at[b] + i * 16 * BK);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) w[b][j] = *reinterpret_cast<const f32x4*>(stage + w_at[b] + j * 16 * BK);
+            }
             __builtin_amdgcn_sched_barrier(0);             // (the second half's operands arrive while the first half is multiplied)
 #pragma unroll
             for (int b = 0; b < BK / 16; ++b)
@@ -368,7 +376,7 @@ int launch(const TA* A, const TW* W, TC* C, float* part, long part_floats, int M
     const unsigned grid = (unsigned)((total + 7) / 8 * 8);
     float* to = c.splits > 1 ? part : nullptr;
     if constexpr (sizeof(TA) == 4 && sizeof(TW) == 4 && sizeof(TC) == 4) {
-        if (vector && K % BK == 0) {
+        if (vector && K % BK == 0 && lda < (1L << 22) && ldw < (1L << 22)) {           // (a tile's rows within 32-bit offsets)
 #define RING(BM) gemm_exact_ring_kernel<BM, ACC><<<grid, 256, 0, stream>>>(A, W, C, to, M, N, K, lda, ldw, ldc, c.m_tiles, c.n_tiles, c.splits)
             if (c.bm == 64) RING(64);
             else RING(32);
