@@ -344,6 +344,42 @@ __global__ __launch_bounds__(256) void gemm_bf16_tiled_kernel(const bf16_t* __re
             }
 }
 
+// A tile of 128 x 128 sums, row-major in LDS, goes onto 32-bit rows, 32 threads a row with four columns each.  `old`: what the sums are
+// added onto, all of a thread's rows (a row beyond M is clamped, and not written).
+template <int NT>
+struct TileOld { float4 v[128 / (NT / 32)]; };
+template <int NT>
+__device__ __forceinline__ void tile_old(TileOld<NT>& old, const float* C, long ldc, int m0, int n0, int M) {
+#pragma unroll
+    for (int it = 0; it < 128 / (NT / 32); ++it)
+        old.v[it] = *reinterpret_cast<const float4*>(C + (size_t)min(m0 + (int)(threadIdx.x >> 5) + it * (NT / 32), M - 1) * ldc + n0 + (threadIdx.x & 31) * 4);
+}
+// ... with a norm handed on: the rows' new values, the same times the norm's weights in bfloat16, and the tile's piece of every row's
+// sum of squares (N is a multiple of 128).
+template <int NT>
+__device__ __forceinline__ void tile_add_handing_norm(const float* tile, const TileOld<NT>& old, float* C, long ldc, int m0, int n0, int M, const NormOut& norm_out,
+                                                      int piece, int pieces) {
+    const int tid = threadIdx.x, c4 = (tid & 31) * 4;
+    const float4 g = *reinterpret_cast<const float4*>(norm_out.g + n0 + c4);
+#pragma unroll
+    for (int it = 0; it < 128 / (NT / 32); ++it) {
+        const int row = (tid >> 5) + it * (NT / 32), m = m0 + row;
+        float square = 0.f;
+        if (m < M) {
+            const float4 t = *reinterpret_cast<const float4*>(tile + row * 128 + c4);
+            float4 x = old.v[it];
+            x.x += t.x; x.y += t.y; x.z += t.z; x.w += t.w;
+            *reinterpret_cast<float4*>(C + (size_t)m * ldc + n0 + c4) = x;
+            *reinterpret_cast<uint2*>(norm_out.scaled + (size_t)m * norm_out.ld + n0 + c4) =
+                uint2{f32x2_to_bf16x2(g.x * x.x, g.y * x.y), f32x2_to_bf16x2(g.z * x.z, g.w * x.w)};
+            square = x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
+        }
+#pragma unroll
+        for (int off = 16; off > 0; off >>= 1) square += __shfl_xor(square, off, 64);
+        if ((tid & 31) == 0 && m < M) norm_out.squares[(size_t)m * pieces + piece] = square;
+    }
+}
+
 // ------------------------------------------------------------------------------------------ piped
 // The same product for large shapes, with the operands going from global memory straight into LDS
 // (global_load_lds_dwordx4: no registers in between) through a ring of blocks of 64 k, so that
@@ -466,15 +502,11 @@ __device__ __forceinline__ void piped_tile(const bf16_t* __restrict__ A, const b
             // The sums go onto 32-bit rows whose next reader is a norm: the tile is laid into LDS (the ring is free once everyone
             // has read the last block) and leaves row by row, 32 threads a row with four columns each: the rows' new values, the
             // same times the norm's weights in bfloat16, and the tile's piece of every row's sum of squares (N is a multiple of 128).
-            constexpr int NT = 64 * WAVES_M * WAVES_N, PASSES = 128 / (NT / 32);
             // What the sums are added onto is asked for first, all of a thread's rows at once (a row beyond M is clamped and not
             // written): read row by row behind the tile, it was a round trip to memory a row, eight in a row at the end of the kernel.
-            const int c4 = (tid & 31) * 4;
-            const float4 g = *reinterpret_cast<const float4*>(norm_out.g + n0 + c4);
-            float4 old[PASSES];
-#pragma unroll
-            for (int it = 0; it < PASSES; ++it)
-                old[it] = *reinterpret_cast<const float4*>((const float*)C + (size_t)min(m0 + (tid >> 5) + it * (NT / 32), M - 1) * ldc + n0 + c4);
+            constexpr int NT = 64 * WAVES_M * WAVES_N;
+            TileOld<NT> old;
+            tile_old<NT>(old, (const float*)C, ldc, m0, n0, M);
             __syncthreads();
             float* tile = reinterpret_cast<float*>(ring);
 #pragma unroll
@@ -485,24 +517,7 @@ __device__ __forceinline__ void piped_tile(const bf16_t* __restrict__ A, const b
                     for (int v = 0; v < 16; ++v)
                         tile[(wm + i * 32 + 8 * (v / 4) + 4 * (lane >> 5) + (v & 3)) * 128 + wn + j * 32 + (lane & 31)] = acc[i][j][v];
             __syncthreads();
-#pragma unroll
-            for (int it = 0; it < PASSES; ++it) {
-                const int row = (tid >> 5) + it * (NT / 32), m = m0 + row;
-                float square = 0.f;
-                if (m < M) {
-                    const float4 t = *reinterpret_cast<const float4*>(tile + row * 128 + c4);
-                    float4* at = reinterpret_cast<float4*>((float*)C + (size_t)m * ldc + n0 + c4);
-                    float4 x = old[it];
-                    x.x += t.x; x.y += t.y; x.z += t.z; x.w += t.w;
-                    *at = x;
-                    *reinterpret_cast<uint2*>(norm_out.scaled + (size_t)m * norm_out.ld + n0 + c4) =
-                        uint2{f32x2_to_bf16x2(g.x * x.x, g.y * x.y), f32x2_to_bf16x2(g.z * x.z, g.w * x.w)};
-                    square = x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
-                }
-#pragma unroll
-                for (int off = 16; off > 0; off >>= 1) square += __shfl_xor(square, off, 64);
-                if ((tid & 31) == 0 && m < M) norm_out.squares[(size_t)m * gridDim.x + blockIdx.x] = square;
-            }
+            tile_add_handing_norm<NT>(tile, old, (float*)C, ldc, m0, n0, M, norm_out, blockIdx.x, gridDim.x);
             return;
         }
     }
@@ -795,6 +810,194 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
                 }
             }
         }
+    }
+}
+
+// ------------------------------------------------------------------------------------------- tall
+// The ping-pong kernel's order of work on tiles of 256 x 128, for products that have no 256 x 256 tile for every compute unit and more
+// than one of 128 x 128.  What bounds both kernels is the rate at which loads reach LDS (about 25 bytes a clock and compute unit,
+// whatever the tiles' order over the dies and however many bytes are read from LDS): a block of 64 k takes a tile of 128 x 128 1,300 to 1,500
+// clocks (32 KB), one of 256 x 128 TALL_CLOCKS (48 KB), so where the 128 x 128 tiles need a second round on some compute units
+// one round of tall tiles is the shorter.  2,048 rows: TALL_NUMBERS
+// A wave owns 64 x 64; group 0 (waves 0 .. 3) the first 128 rows of A, group 1 the last.  The ring has three blocks: in its R(b) a wave
+// sends for its six loads (8 rows each) of block b + 2, whose place held block b - 1, last read by group 1 in the interval before group 0's
+// R(b).  Block b + 1, sent for in R(b - 1), is read from group 0's R(b + 1) on: by the barrier before it group 0 has waited for its loads
+// behind M(b) and group 1 behind R(b), each with the six of block b + 2 still in flight (with two blocks and one of them ahead, weights
+// that came from memory and not from a cache arrived too late).  The sums of an element are
+// taken in the order of the kernel with tiles of 128 x 128, whose epilogues serve, one group's 128 rows at a time.
+// Which tile a workgroup makes.  Workgroups go to the eight dies in turn, each with an L2 of its own, and a die's tiles walk k together:
+// what a die fetches from beyond its L2 is a strip of rows for every different row and column of tiles it holds.  So a die gets a run of
+// neighbouring tiles in panels of `panel` columns, about as many bytes high as wide (2,048 x 8,192 at 3,000 and 4,096 rows: 121 -> 113 and
+// 158 -> 149 us against columns dealt out in turn; nothing at short k).
+struct TileOrder {
+    int m_tiles, n_tiles, each, panel;         // each: tiles a die
+    struct Tile { int m, n; };
+    __device__ __forceinline__ Tile tile(int id) const {
+        const int u = (id & 7) * each + (id >> 3);
+        if ((id >> 3) >= each || u >= m_tiles * n_tiles) return {-1, 0};
+        const int in_panel = panel * m_tiles, p = u / in_panel, rest = u - p * in_panel, width = min(panel, n_tiles - p * panel);
+        return {rest / width, p * panel + rest % width};
+    }
+};
+template <int EPI>
+__global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ C, int M, int N, int K,
+                                                            long lda, long ldw, long ldc, NormIn norm_in, RopeStore rope, NormOut norm_out, TileOrder order) {
+    const TileOrder::Tile at_tile = order.tile(blockIdx.x);
+    if (at_tile.m < 0) return;
+    constexpr int BM = 256, BN = 128, NT = 512, TM = 2, TN = 2, ROWS = BM + BN, STAGE_BYTES = ROWS * 128, LOADS = 6;
+    extern __shared__ __attribute__((aligned(16))) unsigned char ring[];               // 3 * STAGE_BYTES
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), group = wave >> 2, turn = wave & 3;
+    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+    const int m0 = at_tile.m * BM, n0 = at_tile.n * BN;
+    const bf16_t* a_tile = A + (size_t)m0 * lda;
+    const bf16_t* w_tile = W + (size_t)n0 * ldw;
+    auto source = [&](int row) -> unsigned {                                            // as in the ping-pong kernel
+        const int c = (lane & 7) ^ ((row >> 1) & 7);
+        return row < BM ? (unsigned)(((size_t)min(row, M - 1 - m0) * lda + 8 * c) * 2) : (unsigned)(((size_t)min(row - BM, N - 1 - n0) * ldw + 8 * c) * 2);
+    };
+    const unsigned ring_base = (unsigned)(size_t)(lds_ptr_t)ring;
+    unsigned src[LOADS];                                                                // this wave's loads: rows (wave * 6 + i) * 8 .. + 7 of every block
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) src[i] = source((wave * LOADS + i) * 8 + (lane >> 3));
+    auto load_block = [&](int block, int slot) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const int first_row = (wave * LOADS + i) * 8;
+            const unsigned dst = ring_base + slot * STAGE_BYTES + first_row * 128;
+            const bf16_t* base = (first_row < BM ? a_tile : w_tile) + block * PK;
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(src[i]), "s"(base) : "memory", "m0");
+        }
+    };
+    const int n_k = K / PK;
+    auto phase_barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    floatx16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = floatx16{};
+    load_block(0, 0);
+    if (n_k > 1) {
+        load_block(1, 1);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+    } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    phase_barrier();
+    if (group == 1) phase_barrier();            // group 1 runs one barrier behind group 0's phases
+    const int r = lane & 31, swz = (r >> 1) & 7;
+    const unsigned char* a_rows = ring + (wm + r) * 128;
+    const unsigned char* b_rows = ring + (BM + wn + r) * 128;
+    int slot = 0;
+    for (int block = 0; block < n_k; ++block) {
+        const int stage_off = slot * STAGE_BYTES, ahead = slot == 0 ? 2 : slot - 1;      // ahead: the place of blocks b - 1 and b + 2
+        slot = slot == 2 ? 0 : slot + 1;
+        const bool more = block + 2 < n_k;
+        bf16x8 a[PK / 16][TM], b[PK / 16][TN];
+        if ((turn & 1) && more) load_block(block + 2, ahead);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int step = 0; step < PK / 16; ++step) {
+            const int chunk = ((2 * step + (lane >> 5)) ^ swz) * 16;
+#pragma unroll
+            for (int i = 0; i < TM; ++i) a[step][i] = as_bf16x8(*reinterpret_cast<const uint4*>(a_rows + stage_off + i * 32 * 128 + chunk));
+#pragma unroll
+            for (int j = 0; j < TN; ++j) b[step][j] = as_bf16x8(*reinterpret_cast<const uint4*>(b_rows + stage_off + j * 32 * 128 + chunk));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (!(turn & 1) && more) load_block(block + 2, ahead);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                          // the reads are done before anyone may refill the stage
+        // what this wave sent for a block ago has landed: group 1 sees to it here, group 0 behind its products, one barrier before group 0 reads it
+        auto landed = [&]() {
+            if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        };
+        if (group == 1) landed();
+        phase_barrier();
+#pragma unroll
+        for (int step = 0; step < PK / 16; ++step)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[step][i], b[step][j], acc[i][j], 0, 0, 0);
+        if (group == 0) landed();
+        phase_barrier();
+    }
+    if (group == 0) phase_barrier();
+    // Element v of a lane's 32x32 result: row 8*(v/4) + 4*(lane/32) + v%4, column lane%32.  The sums leave through LDS (the ring is free:
+    // every wave has passed the barrier behind its last read), a group's 128 rows at a time.
+    __shared__ float row_scale[EPI == EPI_QKV_ROPE ? BM : 1];
+    __shared__ TilePlaces places[EPI == EPI_QKV_ROPE ? 2 : 1];
+    const bool scaled_rows = EPI == EPI_QKV_ROPE && norm_in.squares != nullptr;
+    TileOld<NT> old[2];
+    if constexpr (EPI == EPI_QKV_ROPE) {
+        if (scaled_rows) tile_row_scales<NT>(row_scale, norm_in, m0, BM, M);
+        if (n0 + BN > rope.n_heads * rope.hd) {                                          // (a tile of queries alone needs no pages)
+            tile_places(places[0], m0, M, rope);
+            tile_places(places[1], m0 + 128, M, rope);
+        }
+        __syncthreads();
+    }
+    if constexpr (EPI == EPI_ADD_F32) {
+        if (norm_out.scaled != nullptr) {
+            tile_old<NT>(old[0], (const float*)C, ldc, m0, n0, M);
+            tile_old<NT>(old[1], (const float*)C, ldc, m0 + 128, n0, M);
+        }
+    }
+    float* tile = reinterpret_cast<float*>(ring);
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        const int first = m0 + half * 128;
+        if (first >= M) break;
+        if (group == half) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        const int row = wm - half * 128 + i * 32 + 8 * (v / 4) + 4 * (lane >> 5) + (v & 3);
+                        tile[row * 128 + wn + j * 32 + (lane & 31)] = scaled_rows ? acc[i][j][v] * row_scale[half * 128 + row] : acc[i][j][v];
+                    }
+        }
+        __syncthreads();
+        if constexpr (EPI == EPI_QKV_ROPE) {
+            qkv_tile_rope_store<NT>(tile, places[half], first, n0, M, N, rope);
+        } else if (EPI == EPI_ADD_F32 && norm_out.scaled != nullptr) {
+            tile_add_handing_norm<NT>(tile, old[half], (float*)C, ldc, first, n0, M, norm_out, at_tile.n, order.n_tiles);
+        } else {
+            constexpr int ELEM = EPI == EPI_STORE_BF16 ? 2 : 4;
+            const int c = n0 + (tid & 31) * 4;
+            const bool whole = c + 3 < N && (ldc & 3) == 0 && ((uintptr_t)C & (4 * ELEM - 1)) == 0;
+#pragma unroll
+            for (int it = 0; it < 8; ++it) {
+                const int row = (tid >> 5) + it * 16, m = first + row;
+                if (m >= M) continue;
+                float4 v = *reinterpret_cast<const float4*>(tile + row * 128 + (tid & 31) * 4);
+                const size_t at = (size_t)m * ldc + c;
+                if (whole) {
+                    if constexpr (EPI == EPI_STORE_BF16) {
+                        *reinterpret_cast<uint2*>((bf16_t*)C + at) = uint2{f32x2_to_bf16x2(v.x, v.y), f32x2_to_bf16x2(v.z, v.w)};
+                    } else {
+                        if constexpr (EPI == EPI_ADD_F32) {
+                            const float4 o = *reinterpret_cast<const float4*>((const float*)C + at);
+                            v.x += o.x; v.y += o.y; v.z += o.z; v.w += o.w;
+                        }
+                        *reinterpret_cast<float4*>((float*)C + at) = v;
+                    }
+                } else {
+                    const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                    for (int x = 0; x < 4; ++x)
+                        if (c + x < N) write_out<EPI == EPI_QKV_ROPE ? EPI_STORE_F32 : EPI>(C, at + x, e[x]);
+                }
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -1508,6 +1711,13 @@ static int consumer_max_parts(int M) { return M <= 16 ? slim_max_parts(M) : M <=
 // 47.4 against 52.8.)
 static bool takes_pingpong(int M, int N) { return (long)((M + 255) / 256) * ((N + 255) / 256) >= gi_compute_units() * 3 / 4; }
 
+// Whether a product of more than 128 rows that neither shares k out nor takes the ping-pong kernel takes tiles of 256 x 128: one round of those
+// on the compute units takes about 1.45 times as long as one of 128 x 128 (see the kernel), so where they need fewer rounds by more.
+static bool takes_tall(int M, int N) {
+    const long units = gi_compute_units(), small = (long)((M + 127) / 128) * ((N + 127) / 128), tall = (long)((M + 255) / 256) * ((N + 127) / 128);
+    return small > units && 29 * ((tall + units - 1) / units) < 20 * ((small + units - 1) / units);
+}
+
 static const NormIn NO_NORM_IN = {nullptr, 0, 0.f, 1, 0.f};
 static const NormOut NO_NORM_OUT = {nullptr, nullptr, 0, nullptr};
 
@@ -1706,6 +1916,16 @@ static int launch_skinny(const void* A, const void* W, void* C, int epi, int M, 
     return reduce_partials(scratch, C, epi, M, N, splits, ldc, stream, norm_in, norm_out);
 }
 
+static TileOrder tall_order(int M, int N) {
+    TileOrder o = {(M + 255) / 256, (N + 127) / 128, 0, 1};
+    o.each = (o.m_tiles * o.n_tiles + 7) / 8;
+    const int run = o.each < gi_compute_units() / 8 ? o.each : gi_compute_units() / 8;       // of a die at a time
+    while ((o.panel + 1) * (o.panel + 1) <= 2 * run) ++o.panel;
+    if (o.panel * o.m_tiles < run) o.panel = (run + o.m_tiles - 1) / o.m_tiles;
+    if (o.panel > o.n_tiles) o.panel = o.n_tiles;
+    return o;
+}
+
 static const RopeStore NO_ROPE = {nullptr, nullptr, nullptr, nullptr, nullptr, 0, nullptr, nullptr, 0, 0, 0, 0, 0};
 
 // The pieces per row that a product of more than 128 rows writes when it hands a norm on, 0 if it cannot: one per tile of 128 columns
@@ -1784,6 +2004,26 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
         else if (epi == EPI_STORE_BF16) PINGPONG(EPI_STORE_BF16); else if (epi == EPI_GATED_BF16) PINGPONG(EPI_GATED_BF16); else if (epi == EPI_GATED_GELU_BF16) PINGPONG(EPI_GATED_GELU_BF16); else PINGPONG(EPI_GATED_CLAMP_BF16);
 #undef PINGPONG
         GI_CHECK_LAUNCH("gemm_bf16 (pingpong)");
+        return 0;
+    }
+    if (takes_tall(M, N) && (rope != nullptr || !is_gated(epi)) && lda < (1L << 22) && ldw < (1L << 22)) {
+#define TALL(EPI_)                                                                                                                      \
+    do {                                                                                                                                \
+        constexpr int bytes = 3 * 384 * 128;                                                                                            \
+        static bool raised = false;                                                                                                     \
+        if (!raised) {                                                                                                                  \
+            if (hipFuncSetAttribute((const void*)gemm_bf16_tall_kernel<EPI_>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) \
+                return gi_fail("gemm_bf16: cannot reserve %d bytes of LDS", bytes);                                                     \
+            raised = true;                                                                                                              \
+        }                                                                                                                               \
+        const TileOrder order = tall_order(M, N);                                                                                       \
+        dim3 grid(8 * order.each);                                                                                                      \
+        gemm_bf16_tall_kernel<EPI_><<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldw, ldc, norm_in, \
+                                                                  rope != nullptr ? *rope : NO_ROPE, norm_out, order);                  \
+    } while (0)
+        if (rope != nullptr) TALL(EPI_QKV_ROPE); else if (epi == EPI_STORE_F32) TALL(EPI_STORE_F32); else if (epi == EPI_ADD_F32) TALL(EPI_ADD_F32); else TALL(EPI_STORE_BF16);
+#undef TALL
+        GI_CHECK_LAUNCH("gemm_bf16 (tall)");
         return 0;
     }
     if (tiles128 > gi_compute_units()) PIPED_EPI(128, 128, 2, 2, 2);
