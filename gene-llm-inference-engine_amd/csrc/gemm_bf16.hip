@@ -1,11 +1,12 @@
 // C[m, n] (=|+=) sum_k A[m, k] * W[n, k] with bfloat16 operands on the matrix cores, 32-bit sums.
 //
 // Both operands are row-major with k contiguous, so each lane's operand of a matrix instruction is
-// one 16-byte load of 8 consecutive k.  Five kernels:
+// one 16-byte load of 8 consecutive k.  Six kernels:
 //
 //   pingpong  large prompt-sized products (256 x 256 tiles for most of the compute units): operands loaded
 //           from global memory straight into two LDS stages; the workgroup's eight waves form two
 //           groups that take turns at reading LDS and at the matrix instructions.
+//   tall    those in between: the same on tiles of 256 x 128 and three LDS stages.
 //   piped   the other products of 128 rows or more (K a multiple of 64): tiles of 128 x 128,
 //           operands loaded from global memory straight into a ring of LDS stages, several
 //           blocks of k in flight; v_mfma_f32_32x32x16_bf16.
@@ -813,17 +814,18 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
     }
 }
 
-// ------------------------------------------------------------------------------------------- tall
-// The ping-pong kernel's order of work on tiles of 256 x 128, for products that have no 256 x 256 tile for every compute unit and more
-// than one of 128 x 128.  What bounds both kernels is the rate at which loads reach LDS (about 25 bytes a clock and compute unit,
-// whatever the tiles' order over the dies and however many bytes are read from LDS): a block of 64 k takes a tile of 128 x 128 1,300 to 1,500
-// clocks (32 KB), one of 256 x 128 TALL_CLOCKS (48 KB), so where the 128 x 128 tiles need a second round on some compute units
-// one round of tall tiles is the shorter.  2,048 rows: TALL_NUMBERS
-// A wave owns 64 x 64; group 0 (waves 0 .. 3) the first 128 rows of A, group 1 the last.  The ring has three blocks: in its R(b) a wave
+// ------------------------------------------------------------------------------------------ tall
+// The ping-pong kernel's order of work on tiles of 256 x 128 (group 0 makes the tile's first 128 rows, group 1 its last; a wave 64 x 64), for
+// products that have more than one 128 x 128 tile a compute unit and no round number of 256 x 256 tiles.
+// The ring has three blocks of 48 KB: in its R(b) a wave
 // sends for its six loads (8 rows each) of block b + 2, whose place held block b - 1, last read by group 1 in the interval before group 0's
 // R(b).  Block b + 1, sent for in R(b - 1), is read from group 0's R(b + 1) on: by the barrier before it group 0 has waited for its loads
-// behind M(b) and group 1 behind R(b), each with the six of block b + 2 still in flight (with two blocks and one of them ahead, weights
-// that came from memory and not from a cache arrived too late).  The sums of an element are
+// behind M(b) and group 1 behind R(b), each with the six of block b + 2 still in flight.
+// Bound by the loads into LDS and by how far ahead they are sent: a block takes 1,720 clocks, of which its matrix instructions are 1,024; with
+// two blocks in the ring and one ahead (which is all that 256 x 256 tiles leave room for) it took 2,100 to 2,600.  2,048 rows of
+// 3,072 x 2,048 take 36.0 us, of 3,072 x 3,072 45, 3,072 x 8,192 104, 5,120 x 3,072 87; with two or three rounds of 128 x 128 tiles 52.5, 64,
+// 137 and 115.  With several rounds a compute unit the 13 us that a tile takes to begin and to end count as much: 2,048 rows of 16,384 x 2,048
+// gated take 152 us here and 120 in the ping-pong kernel, 8,192 of 28,672 x 4,096 1,660 and 1,550.  The sums of an element are
 // taken in the order of the kernel with tiles of 128 x 128, whose epilogues serve, one group's 128 rows at a time.
 // Which tile a workgroup makes.  Workgroups go to the eight dies in turn, each with an L2 of its own, and a die's tiles walk k together:
 // what a die fetches from beyond its L2 is a strip of rows for every different row and column of tiles it holds.  So a die gets a run of
@@ -852,7 +854,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
     const int m0 = at_tile.m * BM, n0 = at_tile.n * BN;
     const bf16_t* a_tile = A + (size_t)m0 * lda;
     const bf16_t* w_tile = W + (size_t)n0 * ldw;
-    auto source = [&](int row) -> unsigned {                                            // as in the ping-pong kernel
+    auto source = [&](int row) -> unsigned {                                            // where this lane's 16 bytes of a stage's row lie, in bytes from the tile's first row of A or of W at k = 0
         const int c = (lane & 7) ^ ((row >> 1) & 7);
         return row < BM ? (unsigned)(((size_t)min(row, M - 1 - m0) * lda + 8 * c) * 2) : (unsigned)(((size_t)min(row - BM, N - 1 - n0) * ldw + 8 * c) * 2);
     };
@@ -881,12 +883,28 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = floatx16{};
     load_block(0, 0);
-    if (n_k > 1) {
-        load_block(1, 1);
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
-    } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (n_k > 1) load_block(1, 1);
+    // With a norm handed on (the rows of A are g * x, and the results lack the rows' rsqrt(mean square + eps)),
+    // the tile's 256 rows' factors are worked out once, a thread a row (16-byte reads of the row's pieces where they allow it: a lane
+    // that asked for its rows' pieces one by one cost 18 us at 16 pieces), and wait in LDS for the epilogue (asked for behind the first
+    // blocks' loads; the barriers of the loop lie between this write and the epilogue's reads).
+    __shared__ float row_scale[EPI == EPI_QKV_ROPE || is_gated(EPI) ? BM : 1];
+    const bool scaled_rows = (EPI == EPI_QKV_ROPE || is_gated(EPI)) && norm_in.squares != nullptr;
+    if (scaled_rows && tid < BM) {
+        const float* pieces = norm_in.squares + (size_t)min(m0 + tid, M - 1) * norm_in.parts;
+        float sum = 0.f;
+        if ((norm_in.parts & 3) == 0 && ((uintptr_t)norm_in.squares & 15) == 0) {
+            for (int p = 0; p < norm_in.parts; p += 4) {
+                const float4 v = *reinterpret_cast<const float4*>(pieces + p);
+                sum += v.x; sum += v.y; sum += v.z; sum += v.w;
+            }
+        } else {
+            for (int p = 0; p < norm_in.parts; ++p) sum += pieces[p];
+        }
+        row_scale[tid] = 1.0f / sqrtf(sum / (float)norm_in.dim + norm_in.eps);
     }
+    if (n_k > 1 && !scaled_rows) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     phase_barrier();
     if (group == 1) phase_barrier();            // group 1 runs one barrier behind group 0's phases
     const int r = lane & 31, swz = (r >> 1) & 7;
@@ -930,12 +948,9 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
     if (group == 0) phase_barrier();
     // Element v of a lane's 32x32 result: row 8*(v/4) + 4*(lane/32) + v%4, column lane%32.  The sums leave through LDS (the ring is free:
     // every wave has passed the barrier behind its last read), a group's 128 rows at a time.
-    __shared__ float row_scale[EPI == EPI_QKV_ROPE ? BM : 1];
     __shared__ TilePlaces places[EPI == EPI_QKV_ROPE ? 2 : 1];
-    const bool scaled_rows = EPI == EPI_QKV_ROPE && norm_in.squares != nullptr;
     TileOld<NT> old[2];
     if constexpr (EPI == EPI_QKV_ROPE) {
-        if (scaled_rows) tile_row_scales<NT>(row_scale, norm_in, m0, BM, M);
         if (n0 + BN > rope.n_heads * rope.hd) {                                          // (a tile of queries alone needs no pages)
             tile_places(places[0], m0, M, rope);
             tile_places(places[1], m0 + 128, M, rope);
@@ -969,6 +984,24 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
             qkv_tile_rope_store<NT>(tile, places[half], first, n0, M, N, rope);
         } else if (EPI == EPI_ADD_F32 && norm_out.scaled != nullptr) {
             tile_add_handing_norm<NT>(tile, old[half], (float*)C, ldc, first, n0, M, norm_out, at_tile.n, order.n_tiles);
+        } else if constexpr (is_gated(EPI)) {
+            // columns 32b .. 32b+15 are gates, 32b+16 .. 32b+31 the ups of outputs 16b .. 16b+15; a thread makes two neighbouring outputs
+            const int o = (tid & 31) * 2, c = n0 / 2 + o;
+#pragma unroll
+            for (int it = 0; it < 8; ++it) {
+                const int row = (tid >> 5) + it * 16, m = first + row;
+                if (m >= M || c >= N / 2) continue;
+                const float* from = tile + row * 128 + (o >> 4) * 32 + (o & 15);
+                const float2 g = *reinterpret_cast<const float2*>(from), u = *reinterpret_cast<const float2*>(from + 16);
+                const uint32_t both = f32x2_to_bf16x2(gate_fast_of<EPI>(g.x, u.x, norm_in.limit), gate_fast_of<EPI>(g.y, u.y, norm_in.limit));
+                bf16_t* to = (bf16_t*)C + (size_t)m * ldc + c;
+                if ((ldc & 1) == 0 && ((uintptr_t)C & 3) == 0) {                          // (N / 2 is a multiple of 16: both exist)
+                    *reinterpret_cast<uint32_t*>(to) = both;
+                } else {
+                    to[0] = (bf16_t)(both & 0xffffu);
+                    to[1] = (bf16_t)(both >> 16);
+                }
+            }
         } else {
             constexpr int ELEM = EPI == EPI_STORE_BF16 ? 2 : 4;
             const int c = n0 + (tid & 31) * 4;
@@ -993,7 +1026,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
                     const float e[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
                     for (int x = 0; x < 4; ++x)
-                        if (c + x < N) write_out<EPI == EPI_QKV_ROPE ? EPI_STORE_F32 : EPI>(C, at + x, e[x]);
+                        if (c + x < N) write_out<EPI == EPI_QKV_ROPE || is_gated(EPI) ? EPI_STORE_F32 : EPI>(C, at + x, e[x]);
                 }
             }
         }
@@ -1702,20 +1735,28 @@ GI_API long gi_gemm_bf16_scratch_floats(int M, int N, int K) {
 // The most pieces a reader of M rows takes: what a writer of as many rows makes.
 static int consumer_max_parts(int M) { return M <= 16 ? slim_max_parts(M) : M <= 32 ? TILES_MAX_PARTS : REDUCE_MAX_PARTS; }
 
-// Whether a product of more than 128 rows takes the ping-pong kernel: 256 x 256 tiles for three quarters of the compute units or
-// more.  (Measured on whole prompts, gate/up being the one product wide enough: with 192 tiles on 256 units 640 and 768 rows of
-// the Llama-3.2-1B shape take 2.94 and 3.51 ms against 3.27 and 3.81 with tiles of 128 x 128, the 3B shape 7.4 and 7.6 against 8.1
-// and 8.3, 320 to 512 rows of the 8B shape, 224 tiles, 10.7 to 11.0 against 12.1 to 12.5; with 128 tiles, half of the units, 512
-// rows take 2.82 ms against 2.73.  Long prompts whose narrower products reach that many tiles gain as much although this kernel
-// hands no norm on and the norm's own kernel runs again: 4,096 rows of the 3B shape 28.3 against 31.0 ms, 3,072 of the 8B shape
-// 47.4 against 52.8.)
-static bool takes_pingpong(int M, int N) { return (long)((M + 255) / 256) * ((N + 255) / 256) >= gi_compute_units() * 3 / 4; }
+// Whether a product of more than 128 rows is one of a long prompt or a wide output: 256 x 256 results for three quarters of the compute units or
+// more.  Such a gated product finishes a norm handed on; such a product onto the residual hands none on, and such a q/k/v product takes
+// none: the norm's own kernel runs there.
+static bool many_tiles(int M, int N) { return (long)((M + 255) / 256) * ((N + 255) / 256) >= gi_compute_units() * 3 / 4; }
 
-// Whether a product of more than 128 rows that neither shares k out nor takes the ping-pong kernel takes tiles of 256 x 128: one round of those
-// on the compute units takes about 1.45 times as long as one of 128 x 128 (see the kernel), so where they need fewer rounds by more.
-static bool takes_tall(int M, int N) {
-    const long units = gi_compute_units(), small = (long)((M + 127) / 128) * ((N + 127) / 128), tall = (long)((M + 255) / 256) * ((N + 127) / 128);
-    return small > units && 29 * ((tall + units - 1) / units) < 20 * ((small + units - 1) / units);
+// Which kernel takes a product of more than 128 rows that does not share k out: what counts are the rounds of tiles on the compute units,
+// each with what a tile takes to begin and to end.  Microseconds, fitted to measurements at K = 1,024 to 8,192 (2,048 rows of 3,072 x 2,048:
+// 51.5 with 128 x 128 tiles in two rounds, 35.0 with 256 x 128 in one; 300 rows of 16,384 x 2,048 gated 42.5 and 36.2; 3,000 rows of 3,072 x 2,048
+// 88 and 66; 2,048 rows of 16,384 x 2,048 gated 152 with 256 x 128 in four rounds, 120 with 256 x 256 in two).  Only the two larger tiles finish a
+// norm handed on to a gated product; the q/k/v product's epilogue rotates tiles 128 columns wide.
+enum Large { PIPED_128, TALL_256, PINGPONG_256 };
+static Large large_kernel(int M, int N, int K, bool rope, bool gated, bool scaled_rows) {
+    const long units = gi_compute_units(), m128 = (M + 127) / 128, m256 = (M + 255) / 256, n128 = (N + 127) / 128, n256 = (N + 255) / 256;
+    const auto rounds = [&](long tiles) { return (double)((tiles + units - 1) / units); };
+    const double blocks = K / PK, small = rounds(m128 * n128);
+    double piped = small > 1 ? small * (blocks * 0.45 + (gated ? 6 : 10)) : blocks * 0.55 + 12;      // (several: two workgroups a unit)
+    if (small > 2) piped *= 1.15;
+    if (scaled_rows && !rope) piped = 1e30;
+    const double tall = rounds(m256 * n128) * (blocks * 0.715 + 13);
+    const double pingpong = many_tiles(M, N) && !rope ? rounds(m256 * n256) * (blocks * 1.5 + 14) : 1e30;
+    if (pingpong < piped && 0.95 * pingpong <= tall) return PINGPONG_256;
+    return tall < piped ? TALL_256 : PIPED_128;
 }
 
 static const NormIn NO_NORM_IN = {nullptr, 0, 0.f, 1, 0.f};
@@ -1930,9 +1971,9 @@ static const RopeStore NO_ROPE = {nullptr, nullptr, nullptr, nullptr, nullptr, 0
 
 // The pieces per row that a product of more than 128 rows writes when it hands a norm on, 0 if it cannot: one per tile of 128 columns
 // from the epilogue of the kernel with tiles of 128 x 128, one per 1024 columns where k is shared out and a second kernel adds the
-// shares; not from the ping-pong kernel.
+// shares; none from a product with many tiles.
 static int large_norm_parts(int M, int N, int K) {
-    if (K % PK != 0 || N < 128 || takes_pingpong(M, N)) return 0;
+    if (K % PK != 0 || N < 128 || many_tiles(M, N)) return 0;
     if (gi_gemm_bf16_piped_splits(M, N, K) > 1) return N % REDUCE_COLUMNS == 0 && N / REDUCE_COLUMNS <= REDUCE_MAX_PARTS ? N / REDUCE_COLUMNS : 0;
     return N % 128 == 0 && N / 128 <= PIPED_MAX_PARTS ? N / 128 : 0;
 }
@@ -1979,14 +2020,13 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
         }
         return reduce_partials(scratch, C, epi, M, N, splits, ldc, stream, norm_in, norm_out);
     }
-    // Measured at 2,048 rows (K = 2048 and 8192): where 256 x 256 tiles give three quarters of the compute units one or more, they halve
-    // the traffic into LDS and run the two groups of waves out of step (the ping-pong kernel); otherwise 128 x 128, two
-    // workgroups per unit with two stages each when there are enough tiles, else one workgroup of eight waves with four stages.
     const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-    GI_REQUIRE(norm_out.scaled == nullptr || (!takes_pingpong(M, N) && large_norm_parts(M, N, K) > 0), "gemm_bf16: a product of M %d, N %d, K %d hands no norm on", M, N, K);
-    GI_REQUIRE(norm_in.squares == nullptr || rope != nullptr || (is_gated(epi) && takes_pingpong(M, N) && norm_in.parts <= PIPED_MAX_PARTS),
+    GI_REQUIRE(norm_out.scaled == nullptr || (!many_tiles(M, N) && large_norm_parts(M, N, K) > 0), "gemm_bf16: a product of M %d, N %d, K %d hands no norm on", M, N, K);
+    GI_REQUIRE(norm_in.squares == nullptr || rope != nullptr || (is_gated(epi) && many_tiles(M, N) && norm_in.parts <= PIPED_MAX_PARTS),
                "gemm_bf16: a product of M %d, N %d, K %d takes no norm handed on in %d pieces", M, N, K, norm_in.parts);
-    if (takes_pingpong(M, N) && rope == nullptr) {     // 256 x 256 tiles for most of the compute units: the ping-pong kernel
+    GI_REQUIRE(!many_tiles(M, N) || (lda < (1L << 22) && ldw < (1L << 22)), "gemm_bf16: row strides %ld, %ld are too large for the tile-relative addressing", lda, ldw);
+    const Large which = lda < (1L << 22) && ldw < (1L << 22) ? large_kernel(M, N, K, rope != nullptr, rope == nullptr && is_gated(epi), norm_in.squares != nullptr) : PIPED_128;
+    if (which == PINGPONG_256) {
 #define PINGPONG(EPI_)                                                                                                                  \
     do {                                                                                                                                \
         constexpr int bytes = 2 * 512 * 128;                                                                                            \
@@ -1999,14 +2039,13 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
         dim3 grid((N + 255) / 256, (M + 255) / 256);                                                                                    \
         gemm_bf16_pingpong_kernel<256, EPI_><<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldw, ldc, norm_in); \
     } while (0)
-        GI_REQUIRE(lda < (1L << 22) && ldw < (1L << 22), "gemm_bf16: row strides %ld, %ld are too large for the tile-relative addressing", lda, ldw);
         if (epi == EPI_STORE_F32) PINGPONG(EPI_STORE_F32); else if (epi == EPI_ADD_F32) PINGPONG(EPI_ADD_F32);
         else if (epi == EPI_STORE_BF16) PINGPONG(EPI_STORE_BF16); else if (epi == EPI_GATED_BF16) PINGPONG(EPI_GATED_BF16); else if (epi == EPI_GATED_GELU_BF16) PINGPONG(EPI_GATED_GELU_BF16); else PINGPONG(EPI_GATED_CLAMP_BF16);
 #undef PINGPONG
         GI_CHECK_LAUNCH("gemm_bf16 (pingpong)");
         return 0;
     }
-    if (takes_tall(M, N) && (rope != nullptr || !is_gated(epi)) && lda < (1L << 22) && ldw < (1L << 22)) {
+    if (which == TALL_256) {
 #define TALL(EPI_)                                                                                                                      \
     do {                                                                                                                                \
         constexpr int bytes = 3 * 384 * 128;                                                                                            \
@@ -2021,11 +2060,13 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
         gemm_bf16_tall_kernel<EPI_><<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldw, ldc, norm_in, \
                                                                   rope != nullptr ? *rope : NO_ROPE, norm_out, order);                  \
     } while (0)
-        if (rope != nullptr) TALL(EPI_QKV_ROPE); else if (epi == EPI_STORE_F32) TALL(EPI_STORE_F32); else if (epi == EPI_ADD_F32) TALL(EPI_ADD_F32); else TALL(EPI_STORE_BF16);
+        if (rope != nullptr) TALL(EPI_QKV_ROPE); else if (epi == EPI_STORE_F32) TALL(EPI_STORE_F32); else if (epi == EPI_ADD_F32) TALL(EPI_ADD_F32);
+        else if (epi == EPI_STORE_BF16) TALL(EPI_STORE_BF16); else if (epi == EPI_GATED_BF16) TALL(EPI_GATED_BF16); else if (epi == EPI_GATED_GELU_BF16) TALL(EPI_GATED_GELU_BF16); else TALL(EPI_GATED_CLAMP_BF16);
 #undef TALL
         GI_CHECK_LAUNCH("gemm_bf16 (tall)");
         return 0;
     }
+    // tiles of 128 x 128: two workgroups per unit with two stages each when there are enough tiles, else one of eight waves with four stages
     if (tiles128 > gi_compute_units()) PIPED_EPI(128, 128, 2, 2, 2);
     else PIPED_EPI(128, 128, 2, 4, 4);
 #undef PIPED_EPI
@@ -2056,8 +2097,8 @@ GI_API int gi_gemm_bf16_norm_parts(int M, int N, int K) {
 // of as many rows.
 GI_API int gi_gemm_bf16_takes_norm(int M, int N, int K, int gated) {
     if (takes_slim(M, N, K) || takes_slim_tiles(M, N, K, gated ? EPI_GATED_BF16 : EPI_STORE_F32)) return 1;
-    if (M > SKINNY_MAX_ROWS)                      // the rows of prompts: the gated product on the ping-pong kernel scales in its epilogue
-        return gated && K % PK == 0 && N >= 128 && takes_pingpong(M, N) ? 1 : 0;
+    if (M > SKINNY_MAX_ROWS)                      // the rows of prompts: the gated product with many tiles scales in its epilogue
+        return gated && K % PK == 0 && N >= 128 && many_tiles(M, N) ? 1 : 0;
     if (gi_gemm_bf16_skinny_splits(N, K) == 0) return 1;      // the weight-streaming kernel finishes its columns and scales them
     return M > 32 && !gated ? 1 : 0;                          // the kernel that adds the shares of k scales: with a few pieces only
 }
@@ -2106,18 +2147,18 @@ GI_API int gi_gemm_bf16_handing(const void* A, const void* W, void* C, int c_dty
 // Whether gi_gemm_bf16_qkv_rope_store takes a q/k/v product of these sizes with heads of hd channels.  17 or 33 to 128 rows: the
 // shapes whose k is shared out over workgroups, whose sums a second kernel adds up anyway.  More rows: the kernels with tiles of
 // 128 x 128, whose epilogue lays the tile into LDS and sends it off rotated (whole heads must lie inside a tile), or, where they
-// share k out, that second kernel again; not where the ping-pong kernel with its larger tiles is the faster product.
+// share k out, that second kernel again.
 GI_API int gi_gemm_bf16_qkv_rope_store_takes(int M, int N, int K, int hd) {
     if (hd < 8 || hd > 256 || (hd & (hd - 1)) != 0) return 0;
     if (M <= SKINNY_MAX_ROWS)
         return !takes_slim(M, N, K) && !takes_slim_tiles(M, N, K, EPI_STORE_F32) && gi_gemm_bf16_skinny_splits(N, K) > 0 && N % 256 == 0 ? 1 : 0;
-    if (K % PK != 0 || N < 128 || takes_pingpong(M, N)) return 0;
+    if (K % PK != 0 || N < 128) return 0;
     return gi_gemm_bf16_piped_splits(M, N, K) > 1 ? N % 256 == 0 : hd <= 128;
 }
 
 // The most pieces of a row's sum of squares that gi_gemm_bf16_qkv_rope_store reads for a product of M rows.
 GI_API int gi_gemm_bf16_qkv_rope_store_max_parts(int M, int N, int K) {
-    return M <= SKINNY_MAX_ROWS || gi_gemm_bf16_piped_splits(M, N, K) > 1 ? REDUCE_MAX_PARTS : PIPED_MAX_PARTS;
+    return M <= SKINNY_MAX_ROWS || gi_gemm_bf16_piped_splits(M, N, K) > 1 ? REDUCE_MAX_PARTS : many_tiles(M, N) ? 0 : PIPED_MAX_PARTS;
 }
 
 // The q/k/v product of an attention layer, A [M, K] x W [N, K]^T with N = (n_heads + 2 n_kv) * hd, whose results do not come back:

@@ -210,7 +210,8 @@ class Attention(Mixer):
             return True
         # the rows of prompts: the q/k/v product that rotates and fills the pages itself finishes the norm, where it serves
         half_split = self.position is None or getattr(type(self.position), "half_split_tables", None) is not PositionEncoding.half_split_tables
-        return half_split and ops.gemm_bf16_qkv_rope_store_takes(n_rows, self.w_qkv.shape[0], self.w_qkv.shape[1], self.spec.head_dim)
+        n, k = self.w_qkv.shape
+        return half_split and ops.gemm_bf16_qkv_rope_store_takes(n_rows, n, k, self.spec.head_dim) and ops.gemm_bf16_qkv_rope_store_max_parts(n_rows, n, k) > 0
 
     def _attend_general(self, h, ctx, cache, projected=None):
         """The heads' outputs [rows, heads * value_dim] by the general path."""
