@@ -562,7 +562,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_grouped_kernel(const bf16_t* __
 }
 
 // --------------------------------------------------------------------------------------- pingpong
-// A 256 x 256 tile and two LDS stages of 64 k, filled straight from global memory like the piped kernel's, with another
+// A 256 x 256 tile and LDS stages of 64 k, two of A and three of W, filled straight from global memory like the piped kernel's, with another
 // order of work inside the workgroup.  Its eight waves form two groups of four, and a compute unit's four SIMDs hold
 // one wave of each group.  A group alternates between a phase R in which it reads the operands of a block's 64 k from
 // LDS into registers (and issues loads that refill the stages) and a phase M in which it does nothing but matrix
@@ -577,15 +577,17 @@ __global__ __launch_bounds__(256) void gemm_bf16_grouped_kernel(const bf16_t* __
 // Every wave passes the same number of barriers: group 1's one ahead is matched by one more of group 0 at the end.
 // Who loads which rows of which block when is said where the loads are set up, below.  Measured (cycle stamps per
 // phase): M takes 1,080 clocks for its 32 matrix instructions, R 500 for its 24 reads plus what its 8 loads take to
-// issue, which is what bounds the interval between two barriers (1,700 clocks); a load costs the wave that issues it
-// 23 clocks when nothing else runs and 70 to 140 here, wherever in the two phases it is put.
+// issue, which is what bounds the interval between two barriers; a load costs the wave that issues it
+// 23 clocks when nothing else runs and 70 to 140 here, wherever in the two phases it is put.  How far ahead the loads are sent
+// counts as well (all of LDS is taken for it): with two stages of W, sent for one block ahead, 8,192 rows of 28,672 x 4,096 gated took 1,558 us,
+// of 4,096 x 14,336 831, of 6,144 x 4,096 368; with three 1,470, 740 and 332 (K = 2,048, 32 blocks a tile: no difference).
 template <int BN, int EPI>
 __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ C,
                                                                 int M, int N, int K, long lda, long ldw, long ldc, NormIn norm_in) {
     static_assert(BN == 256, "the sharing of the loads below is written for 256 x 256 tiles");
     constexpr int BM = 256, WAVES = 8, WM = 64, WN = BN / 2, TM = WM / 32, TN = WN / 32;
-    constexpr int ROWS = BM + BN, STAGE_BYTES = ROWS * 128, LOADS = ROWS / 8 / WAVES;      // a wave-wide load fills 8 rows of 128 bytes
-    extern __shared__ __attribute__((aligned(16))) unsigned char ring[];               // 2 * STAGE_BYTES
+    constexpr int ROWS = BM + BN, A_BYTES = BM * 128, W_BYTES = BN * 128, LOADS = ROWS / 8 / WAVES;      // a wave-wide load fills 8 rows of 128 bytes
+    extern __shared__ __attribute__((aligned(16))) unsigned char ring[];               // two blocks of A, three of W
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), group = wave >> 2;
     const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
@@ -602,8 +604,8 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
         return row < BM ? (unsigned)(((size_t)min(row, M - 1 - m0) * lda + 8 * c) * 2) : (unsigned)(((size_t)min(row - BM, N - 1 - n0) * ldw + 8 * c) * 2);
     };
     const unsigned ring_base = (unsigned)(size_t)(lds_ptr_t)ring;
-    auto load_rows = [&](unsigned from, int first_row, int block) {                  // 8 rows from `first_row` (the same for the wave) of block `block`
-        const unsigned dst = ring_base + (block & 1) * STAGE_BYTES + first_row * 128;
+    auto load_rows = [&](unsigned from, int first_row, int block, int w_slot) {      // 8 rows from `first_row` (the same for the wave) of block `block`
+        const unsigned dst = ring_base + (first_row < BM ? (block & 1) * A_BYTES + first_row * 128 : 2 * A_BYTES + w_slot * W_BYTES + (first_row - BM) * 128);
         const bf16_t* base = (first_row < BM ? a_tile : w_tile) + block * PK;
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(from), "s"(base) : "memory", "m0");
     };
@@ -611,21 +613,29 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
     // three quarters of the time the block's matrix instructions take; and a wave that issues one is held for as long as the loads
     // of its workgroup that are ahead of it take, with its next instructions behind it.  So the loads are issued by the group that
     // reads, behind its reads of LDS (while it would wait for those and then for the other group's matrix instructions anyway), and
-    // they are spread evenly over the block's two barrier intervals.  Which rows can be loaded when follows from who reads them:
+    // they are spread evenly over the block's two barrier intervals.  They are sent for as far ahead as LDS has room: A has two places, W, which
+    // comes from memory where A was just written, three.  Which rows can be loaded when follows from who reads them:
     //   group 0 reads the first 128 rows of A and all of W, in the first interval of a block; group 1 the last 128 rows of A and all of W, in the second.
-    //   group 0, R(b):  the rows of W of block b + 1           (their stage fell free at the barrier before, when group 1 had read block b - 1)
-    //   group 1, R(b):  the first 128 rows of A of block b + 2 (group 0 has just read those of block b) and the last 128 of block b + 1
-    // Every wave waits for its own loads at the end of its M phase; the rows are read two barriers later or more.
+    //   group 0, R(b):  the last 128 rows of A of block b + 1 (group 1 read those of block b - 1 in the interval before) and half of W of block b + 2
+    //   group 1, R(b):  the first 128 rows of A of block b + 2 (group 0 has just read those of block b) and the other half of W of block b + 2
+    // and who has waited for them when: group 0 for its rows of A (the older of its loads) behind R(b + 1), a barrier before group 1 reads
+    // them, and for its half of W behind M(b + 1); group 1 for both behind R(b + 1): in both cases a barrier before group 0's R(b + 2).
     const int turn = wave & 3;
-    const int first_row = group == 0 ? BM + turn * 64 : turn * 32;                     // of the wave's load 0; group 1's loads 4 .. 7 lie 128 rows further
-    auto row_of = [&](int i) { return first_row + (group == 0 ? 8 * i : 8 * (i & 3) + 128 * (i >> 2)); };
+    auto row_of = [&](int i) { return i < 4 ? (1 - group) * 128 + turn * 32 + 8 * i : BM + group * 128 + turn * 32 + 8 * (i - 4); };      // of the wave's load i
     unsigned src[LOADS];
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) src[i] = source(row_of(i) + (lane >> 3));
     const int n_k = K / PK;
-    auto load_one = [&](int i, int block) {                                         // this wave's load i during R(block)
-        const int of_block = group == 0 ? block + 1 : (i < 4 ? block + 2 : block + 1);
-        if (of_block < n_k) load_rows(src[i], row_of(i), of_block);
+    auto load_ahead = [&](int block, int w_slot) {                                  // this wave's loads during R(block); w_slot: where W of block + 2 goes
+        const int a_block = block + 1 + group;
+        if (a_block < n_k) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) load_rows(src[i], row_of(i), a_block, 0);
+        }
+        if (block + 2 < n_k) {
+#pragma unroll
+            for (int i = 4; i < LOADS; ++i) load_rows(src[i], row_of(i), block + 2, w_slot);
+        }
     };
     auto phase_barrier = [&]() {
         __builtin_amdgcn_sched_barrier(0);
@@ -639,18 +649,21 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = floatx16{};
 
-    // to begin with: all of block 0, and the first 128 rows of A of block 1 (which the R phase before block 0 would have sent for)
+    // to begin with: all of block 0, and of block 1 the first 128 rows of A and all of W
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) load_rows(source((wave * LOADS + i) * 8 + (lane >> 3)), (wave * LOADS + i) * 8, 0);
+    for (int i = 0; i < LOADS; ++i) load_rows(source((wave * LOADS + i) * 8 + (lane >> 3)), (wave * LOADS + i) * 8, 0, 0);
     if (n_k > 1) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) load_rows(source((wave * 2 + i) * 8 + (lane >> 3)), (wave * 2 + i) * 8, 1);
+        for (int i = 0; i < 6; ++i) {
+            const int first_row = (wave * 6 + i) * 8 + (wave * 6 + i >= 16 ? 128 : 0);
+            load_rows(source(first_row + (lane >> 3)), first_row, 1, 1);
+        }
     }
     // With a norm handed on (the gated product: the rows of A are g * x, and the results lack the rows' rsqrt(mean square + eps)),
     // the tile's 256 rows' factors are worked out once, a thread a row (16-byte reads of the row's pieces where they allow it: a lane
     // that asked for its rows' pieces one by one cost the kernel 18 us at 16 pieces), and wait in LDS for the epilogue (asked for behind the first block's loads; the
-    // barriers of the loop lie between this write and the epilogue's reads).
-    __shared__ float row_scale[is_gated(EPI) ? BM : 1];
+    // ring has no room for them before the loop is through).
+    float my_row_scale = 1.0f;
     if constexpr (is_gated(EPI)) {
         if (norm_in.squares != nullptr) {
             if (tid < BM) {
@@ -664,42 +677,50 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
                 } else {
                     for (int p = 0; p < norm_in.parts; ++p) sum += pieces[p];
                 }
-                row_scale[tid] = 1.0f / sqrtf(sum / (float)norm_in.dim + norm_in.eps);
+                my_row_scale = 1.0f / sqrtf(sum / (float)norm_in.dim + norm_in.eps);
             }
         }
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (n_k > 1 && !(is_gated(EPI) && norm_in.squares != nullptr)) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     phase_barrier();
     if (group == 1) phase_barrier();            // group 1 runs one barrier behind group 0's phases
 
     const int r = lane & 31, swz = (r >> 1) & 7;
     const unsigned char* a_rows = ring + (wm + r) * 128;
-    const unsigned char* b_rows = ring + (BM + wn + r) * 128;
+    const unsigned char* b_rows = ring + 2 * A_BYTES + (wn + r) * 128;
+    int w_slot = 0;
     for (int block = 0; block < n_k; ++block) {
-        const int stage_off = (block & 1) * STAGE_BYTES;
+        const int a_off = (block & 1) * A_BYTES, b_off = w_slot * W_BYTES, w_ahead = w_slot == 0 ? 2 : w_slot - 1;       // w_ahead: the place of blocks b - 1 and b + 2
+        w_slot = w_slot == 2 ? 0 : w_slot + 1;
+        const bool more = block + 2 < n_k;
         // ---- R: the operands of the block's 64 k into registers, and behind the reads this wave's loads
         // (two of the group's waves send their loads first and read then, two the other way round: the memory pipeline is at work
         // from the start of the interval, and nobody's reads wait behind everybody's loads)
         bf16x8 a[PK / 16][TM], b[PK / 16][TN];
-        if (turn & 1) {
-#pragma unroll
-            for (int i = 0; i < LOADS; ++i) load_one(i, block);
-        }
+        if (turn & 1) load_ahead(block, w_ahead);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int step = 0; step < PK / 16; ++step) {
             const int chunk = ((2 * step + (lane >> 5)) ^ swz) * 16;
 #pragma unroll
-            for (int i = 0; i < TM; ++i) a[step][i] = as_bf16x8(*reinterpret_cast<const uint4*>(a_rows + stage_off + i * 32 * 128 + chunk));
+            for (int i = 0; i < TM; ++i) a[step][i] = as_bf16x8(*reinterpret_cast<const uint4*>(a_rows + a_off + i * 32 * 128 + chunk));
 #pragma unroll
-            for (int j = 0; j < TN; ++j) b[step][j] = as_bf16x8(*reinterpret_cast<const uint4*>(b_rows + stage_off + j * 32 * 128 + chunk));
+            for (int j = 0; j < TN; ++j) b[step][j] = as_bf16x8(*reinterpret_cast<const uint4*>(b_rows + b_off + j * 32 * 128 + chunk));
         }
         __builtin_amdgcn_sched_barrier(0);
-        if (!(turn & 1)) {
-#pragma unroll
-            for (int i = 0; i < LOADS; ++i) load_one(i, block);
-        }
+        if (!(turn & 1)) load_ahead(block, w_ahead);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                          // the reads are done before anyone may refill the stage
+        // (in the last block but one group 0 sends for its rows of A alone and group 1 for nothing, in the last nobody for anything)
+        const bool last_rows = block + 2 == n_k;
+        if (group == 0) {                                                           // the rows of A sent for a block ago have landed
+            if (more) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+            else if (last_rows) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        } else {                                                                    // what was sent for a block ago has
+            if (more) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
         phase_barrier();
         // ---- M: nothing but matrix instructions
 #pragma unroll
@@ -708,10 +729,21 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[step][j], a[step][i], acc[i][j], 0, 0, 0);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                            // what this wave sent for during R has landed
+        if (group == 0) {                                                           // the half of W sent for a block ago has landed
+            if (more) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+            else if (last_rows) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
         phase_barrier();
     }
     if (group == 0) phase_barrier();
+    float* row_scale = reinterpret_cast<float*>(ring + 2 * A_BYTES + W_BYTES);      // (behind what the waves' results pass through)
+    if constexpr (is_gated(EPI)) {
+        if (norm_in.squares != nullptr) {
+            if (tid < BM) row_scale[tid] = my_row_scale;
+            __syncthreads();
+        }
+    }
     // The weights were the first operand: a lane's 32x32 result holds row (of A) m = lane%32 and, as element v, column
     // (row of W) n = 8*(v/4) + 4*(lane/32) + v%4, four neighbouring columns at a time.  The results leave through LDS
     // (the ring is free now: every wave has passed the barrier behind its last read), 128 bytes of 64 rows at a time
@@ -825,7 +857,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
 // two blocks in the ring and one ahead (which is all that 256 x 256 tiles leave room for) it took 2,100 to 2,600.  2,048 rows of
 // 3,072 x 2,048 take 36.0 us, of 3,072 x 3,072 45, 3,072 x 8,192 104, 5,120 x 3,072 87; with two or three rounds of 128 x 128 tiles 52.5, 64,
 // 137 and 115.  With several rounds a compute unit the 13 us that a tile takes to begin and to end count as much: 2,048 rows of 16,384 x 2,048
-// gated take 152 us here and 120 in the ping-pong kernel, 8,192 of 28,672 x 4,096 1,660 and 1,550.  The sums of an element are
+// gated take 152 us here and 120 in the ping-pong kernel, 8,192 of 28,672 x 4,096 1,660 and 1,470.  The sums of an element are
 // taken in the order of the kernel with tiles of 128 x 128, whose epilogues serve, one group's 128 rows at a time.
 // Which tile a workgroup makes.  Workgroups go to the eight dies in turn, each with an L2 of its own, and a die's tiles walk k together:
 // what a die fetches from beyond its L2 is a strip of rows for every different row and column of tiles it holds.  So a die gets a run of
@@ -1754,7 +1786,7 @@ static Large large_kernel(int M, int N, int K, bool rope, bool gated, bool scale
     if (small > 2) piped *= 1.15;
     if (scaled_rows && !rope) piped = 1e30;
     const double tall = rounds(m256 * n128) * (blocks * 0.715 + 13);
-    const double pingpong = many_tiles(M, N) && !rope ? rounds(m256 * n256) * (blocks * 1.5 + 14) : 1e30;
+    const double pingpong = many_tiles(M, N) && !rope ? rounds(m256 * n256) * (blocks * 1.45 + 14) : 1e30;
     if (pingpong < piped && 0.95 * pingpong <= tall) return PINGPONG_256;
     return tall < piped ? TALL_256 : PIPED_128;
 }
@@ -2029,7 +2061,7 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
     if (which == PINGPONG_256) {
 #define PINGPONG(EPI_)                                                                                                                  \
     do {                                                                                                                                \
-        constexpr int bytes = 2 * 512 * 128;                                                                                            \
+        constexpr int bytes = (2 * 256 + 3 * 256) * 128;                                                                                            \
         static bool raised = false;                                                                                                     \
         if (!raised) {                                                                                                                  \
             if (hipFuncSetAttribute((const void*)gemm_bf16_pingpong_kernel<256, EPI_>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) \
