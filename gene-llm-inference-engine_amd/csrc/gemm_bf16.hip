@@ -158,8 +158,9 @@ __device__ __forceinline__ float row_scale_from(const NormIn& n, int row, const 
 }
 __device__ __forceinline__ float row_scale_of(const NormIn& n, int row) { return row_scale_from(n, row, row_pieces(n, row)); }
 
-// Where the rows of a tile of 128 go in the cache: per row the page's offset and the place in the page, and per group of
-// eight rows whether they are eight consecutive positions of one request that begin at a multiple of eight (rows of a prompt).
+// Where the rows of a tile of 128 go in the cache: per row the page's offset and the place in the page, and per window of
+// eight rows the one in it (or -1) from which on eight rows are eight consecutive positions of one request that begin at a multiple of eight
+// (rows of a prompt, wherever its first row lies in the tile).
 struct TilePlaces {
     long page[128];              // page * page_stride
     int place[128];
@@ -174,19 +175,22 @@ __device__ __forceinline__ void tile_places(TilePlaces& t, int m0, int M, const 
     const int m = min(m0 + row, M - 1), p = rs.pos[m], slot = rs.slot[m];
     t.page[row] = (long)rs.table[(size_t)slot * rs.table_stride + p / rs.page_size] * rs.page_stride;
     t.place[row] = p % rs.page_size;
-    // the eight lanes of a group agree on the first row's slot and position
-    const int first = row & ~7, p0 = __shfl(p, first & 63, 64), slot0 = __shfl(slot, first & 63, 64);
-    const bool fits = m0 + row < M && slot == slot0 && p == p0 + (row & 7);
-    const unsigned long long all = __ballot(fits);
-    if ((row & 7) == 0) t.run[row >> 3] = ((all >> (row & 63)) & 0xffull) == 0xffull && p % 8 == 0 && rs.page_size % 8 == 0;
+    bool begins = p % 8 == 0 && rs.page_size % 8 == 0 && row + 7 < 128 && m0 + row + 7 < M;
+    if (begins) {
+#pragma unroll
+        for (int i = 1; i < 8; ++i) begins = begins & (rs.pos[m + i] == p + i) & (rs.slot[m + i] == slot);
+    }
+    const unsigned here = (unsigned)(__ballot(begins) >> (row & 56)) & 0xffu;         // (two such rows are eight apart or more)
+    if ((row & 7) == 0) t.run[row >> 3] = here ? row + __ffs(here) - 1 : -1;
 }
 
 // A tile of 128 x 128 sums of a q/k/v product, row-major in LDS, goes where `RopeStore` says.  Whole heads lie inside the
 // tile (hd divides 128, the tile starts at a multiple of 128 columns), so the other half of every pair is in LDS too.  Queries
 // and keys: a thread takes four pairs of a row at a time, whose two halves leave as 8-byte pieces of contiguous rows; the
 // cosines and sines of four such items are asked for at once.  Values are stored transposed in their pages ([hd][place]),
-// so they are taken column by column, eight rows at a time: where those are a run of eight positions (`TilePlaces`), they
-// leave as one 16-byte piece, otherwise one by one.
+// so they are taken column by column: runs of eight positions (`TilePlaces`) leave as 16-byte pieces, the rows that belong to none
+// one by one (a step's portions begin anywhere: with runs looked for at every eighth row of the tile only, the product of a mixed step of 2,048
+// rows of 5,120 x 3,072 took 125 us, 99 now).
 template <int NT>
 __device__ __forceinline__ void qkv_tile_rope_store(const float* tile, const TilePlaces& at, int m0, int n0, int M, int N, const RopeStore& rs) {
     const int a_dim = rs.n_heads * rs.hd, kv_dim = rs.n_kv * rs.hd, half = rs.hd / 2;
@@ -238,19 +242,20 @@ __device__ __forceinline__ void qkv_tile_rope_store(const float* tile, const Til
         const size_t v_plane = (size_t)rs.n_kv * rs.page_size * rs.hd;           // from a page's keys to its values
         const bool aligned = ((uintptr_t)rs.cache & 15) == 0 && rs.page_stride % 8 == 0;
         for (int e = threadIdx.x; e < 16 * 128; e += NT) {
-            const int rows = (e >> 7) * 8, c1 = e & 127, m = m0 + rows, col = n0 + c1;
-            if (m >= M || col >= N || col < a_dim + kv_dim) continue;
-            const size_t c = (size_t)(col - a_dim - kv_dim) * rs.page_size;     // (h * hd + kk) * page_size
-            float v[8];
+            const int window = e >> 7, c1 = e & 127, col = n0 + c1, run = at.run[window], before = window ? at.run[window - 1] : -1;
+            if (col >= N || col < a_dim + kv_dim) continue;
+            const size_t c = v_plane + (size_t)(col - a_dim - kv_dim) * rs.page_size;     // (h * hd + kk) * page_size
+            const bool whole = aligned && run >= 0;
+            if (whole) {
+                float v[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = tile[(rows + i) * 128 + c1];
-            if (aligned && at.run[e >> 7]) {
+                for (int i = 0; i < 8; ++i) v[i] = tile[(run + i) * 128 + c1];
                 const uint4 packed = {f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]), f32x2_to_bf16x2(v[4], v[5]), f32x2_to_bf16x2(v[6], v[7])};
-                *reinterpret_cast<uint4*>(rs.cache + at.page[rows] + v_plane + c + at.place[rows]) = packed;
-            } else {
-                const int last = min(7, M - 1 - m);
-                for (int i = 0; i <= last; ++i) rs.cache[at.page[rows + i] + v_plane + c + at.place[rows + i]] = f32_to_bf16(v[i]);
+                *reinterpret_cast<uint4*>(rs.cache + at.page[run] + c + at.place[run]) = packed;
             }
+            // the window's rows that neither its run nor the one that reaches in from the window before covers
+            const int from = max(window * 8, aligned && before >= 0 ? before + 8 : 0), to = min(whole ? run : window * 8 + 8, M - m0);
+            for (int row = from; row < to; ++row) rs.cache[at.page[row] + c + at.place[row]] = f32_to_bf16(tile[row * 128 + c1]);
         }
     }
 }
@@ -935,7 +940,17 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
         }
         row_scale[tid] = 1.0f / sqrtf(sum / (float)norm_in.dim + norm_in.eps);
     }
-    if (n_k > 1 && !scaled_rows) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+    // Likewise where the rows' keys and values go (two loads that depend on each other).
+    __shared__ TilePlaces places[EPI == EPI_QKV_ROPE ? 2 : 1];
+    bool asked = scaled_rows;
+    if constexpr (EPI == EPI_QKV_ROPE) {
+        if (n0 + BN > rope.n_heads * rope.hd) {                                          // (a tile of queries alone needs no pages)
+            tile_places(places[0], m0, M, rope);
+            tile_places(places[1], m0 + 128, M, rope);
+            asked = true;
+        }
+    }
+    if (n_k > 1 && !asked) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     phase_barrier();
     if (group == 1) phase_barrier();            // group 1 runs one barrier behind group 0's phases
@@ -980,15 +995,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
     if (group == 0) phase_barrier();
     // Element v of a lane's 32x32 result: row 8*(v/4) + 4*(lane/32) + v%4, column lane%32.  The sums leave through LDS (the ring is free:
     // every wave has passed the barrier behind its last read), a group's 128 rows at a time.
-    __shared__ TilePlaces places[EPI == EPI_QKV_ROPE ? 2 : 1];
     TileOld<NT> old[2];
-    if constexpr (EPI == EPI_QKV_ROPE) {
-        if (n0 + BN > rope.n_heads * rope.hd) {                                          // (a tile of queries alone needs no pages)
-            tile_places(places[0], m0, M, rope);
-            tile_places(places[1], m0 + 128, M, rope);
-        }
-        __syncthreads();
-    }
     if constexpr (EPI == EPI_ADD_F32) {
         if (norm_out.scaled != nullptr) {
             tile_old<NT>(old[0], (const float*)C, ldc, m0, n0, M);

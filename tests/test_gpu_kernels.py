@@ -361,6 +361,35 @@ def test_qkv_product_that_rotates_and_fills_the_pages(m, hidden, n_heads, n_kv, 
     assert float((got_q.float() != want_q.float()).float().mean()) < 0.01 and float((got_cache.float() != want_cache.float()).float().mean()) < 0.01
 
 
+@pytest.mark.parametrize("m,page_size,portions", [(2048, 16, [(0, 24, 0), (24, 1300, 701), (1324, 724, 3)]),      # single rows, then portions that begin anywhere
+                                                  (1500, 16, [(0, 3, 0), (3, 9, 5), (12, 8, 16), (20, 1, 7), (21, 1479, 1000)]),
+                                                  (2048, 12, [(0, 1000, 5), (1000, 1048, 0)]), (1410, 24, [(0, 1410, 23)])])
+def test_qkv_product_fills_the_pages_of_portions(m, page_size, portions):
+    """The epilogue of tiles of a prompt's rows: values of eight consecutive positions leave their pages' way as one piece wherever in the
+    tile their rows lie, those around them one by one: what the kernel that rotates and stores writes, at every place."""
+    o = ops()
+    hidden, n_heads, n_kv, hd = 192, 24, 8, 128
+    n = (n_heads + 2 * n_kv) * hd
+    assert o.gemm_bf16_qkv_rope_store_takes(m, n, hidden, hd)
+    a, w = randn(m, hidden, dtype=torch.bfloat16, seed=41), randn(n, hidden, dtype=torch.bfloat16, seed=42, scale=0.05)
+    slots, positions = torch.empty(m, dtype=torch.int32), torch.empty(m, dtype=torch.int32)
+    for slot, (first, rows, pos0) in enumerate(portions):
+        slots[first:first + rows] = slot
+        positions[first:first + rows] = pos0 + torch.arange(rows, dtype=torch.int32)
+    slots[:portions[0][1]] = torch.where(torch.tensor(portions[0][1] <= 24), len(portions) + torch.arange(portions[0][1]), torch.zeros(portions[0][1])).int()      # (few rows: a request each)
+    n_slots, pages = len(portions) + 25, -(-2600 // page_size)
+    table = torch.randperm(n_slots * pages, generator=torch.Generator().manual_seed(3)).view(n_slots, pages).to(torch.int32).to(DEV)
+    slots, positions = slots.to(DEV), positions.to(DEV)
+    want_cache, got_cache = (torch.full((n_slots * pages, 2, n_kv, page_size, hd), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    want_q, got_q = (torch.full((m, n_heads * hd), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    qkv = torch.empty(m, n, device=DEV)
+    o.gemm_bf16(a, w, qkv)
+    a_dim, kv_dim = n_heads * hd, n_kv * hd
+    o.rope_store(qkv[:, :a_dim], qkv[:, a_dim:a_dim + kv_dim], qkv[:, a_dim + kv_dim:], None, None, positions, slots, table, want_q, want_cache, n_heads, n_kv, hd)
+    o.gemm_bf16_qkv_rope_store(a, w, None, None, positions, slots, table, got_q, got_cache, n_heads, n_kv, hd)
+    assert torch.equal(got_q, want_q) and torch.equal(got_cache, want_cache)             # (nothing is rotated: the same sums, rounded once)
+
+
 # -------------------------------------------------------------------------------------- sampling
 def test_argmax_lowest_index_on_ties():
     rows = [[1, 5, 5, 2], [3, 3, 3, 3], [-7, -8, -9, -10], [0, -1, 9, 9]]          # tests/verify_sampler.py:173-178
