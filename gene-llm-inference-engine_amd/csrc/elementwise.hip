@@ -721,18 +721,14 @@ GI_API int gi_act_mul(const float* gate_up, void* h, int h_dtype, int n_rows, in
 }
 
 // ------------------------------------------------------------------------- feed-forward without a gate
-// h[t, i] = act(x[t, i]) for the two-parameter activation "xielu": with a = softplus(params[0]) and b = 1/2 + softplus(params[1]),
-//   z > 0:  a z^2 + z / 2          z <= 0:  b (exp(z) - 1 - z) + z / 2
-// (quadratic on the right, bounded below on the left, slope 1/2 on both sides of 0).  params: two float32 numbers on the device.
-__device__ __forceinline__ float softplus_f32(float z) { return z > 20.f ? z : log1pf(expf(z)); }
-
+// h[t, i] = xielu(x[t, i]).  params: its two float32 numbers on the device.
 template <typename TO>
 __global__ __launch_bounds__(256) void xielu_kernel(const float* __restrict__ x, long ldx, TO* __restrict__ h, long ldh, int inter, const float* __restrict__ params) {
     // one row a workgroup (blockIdx.x) and 1,024 columns of it (blockIdx.y): four neighbouring columns a thread where the row allows
     const float a = softplus_f32(params[0]), b = 0.5f + softplus_f32(params[1]);
     const float* xr = x + (size_t)blockIdx.x * ldx;
     TO* hr = h + (size_t)blockIdx.x * ldh;
-    auto act = [&](float z) { return z > 0.f ? fmaf(a * z, z, 0.5f * z) : fmaf(b, expm1f(z) - z, 0.5f * z); };
+    auto act = [&](float z) { return xielu(z, a, b); };
     const int c0 = blockIdx.y * 1024 + threadIdx.x * 4;
     if (c0 + 3 < inter && (ldx & 3) == 0 && (((uintptr_t)x) & 15) == 0) {
         const float4 z = *reinterpret_cast<const float4*>(xr + c0);

@@ -35,7 +35,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-enum Epilogue : int { EPI_STORE_F32 = 0, EPI_ADD_F32 = 1, EPI_STORE_BF16 = 2, EPI_GATED_BF16 = 3, EPI_QKV_ROPE = 4, EPI_GATED_GELU_BF16 = 5, EPI_GATED_CLAMP_BF16 = 6 };
+enum Epilogue : int { EPI_STORE_F32 = 0, EPI_ADD_F32 = 1, EPI_STORE_BF16 = 2, EPI_GATED_BF16 = 3, EPI_QKV_ROPE = 4, EPI_GATED_GELU_BF16 = 5, EPI_GATED_CLAMP_BF16 = 6, EPI_XIELU = 7 };
 // The gated epilogues differ in the activation alone: SiLU (EPI_GATED_BF16), the tanh form of GELU, or the clamped form
 // g sigmoid(1.702 g) (u + 1) with g <- min(g, limit), u <- clamp(u, -limit, limit) (EPI_GATED_CLAMP_BF16; `limit` comes with `NormIn`).
 __host__ __device__ constexpr bool is_gated(int epi) { return epi == EPI_GATED_BF16 || epi == EPI_GATED_GELU_BF16 || epi == EPI_GATED_CLAMP_BF16; }
@@ -100,8 +100,14 @@ struct NormIn {                  // for a product whose rows A are g * x without
     int parts;
     float eps;
     int dim;                     // r = rsqrt(sum / dim + eps)
-    float limit;                 // of the clamped gated epilogue (nothing of the norm's: it travels here because every kernel takes this struct)
+    union {                      // (nothing of the norm's: it travels here because every kernel takes this struct)
+        float limit;             // of the clamped gated epilogue
+        int first;               // of the epilogue with xielu: the first column that goes through it
+    };
 };
+// The epilogue with xielu (a feed-forward without a gate) takes no further arguments either, as longer ones made every launch of a decoded
+// row slower (818 -> 831 us a step of 1B parameters with 32 bytes more): the two parameters are NormOut::g - for the kernel that takes none,
+// NormIn::squares, its rows being ready-made - and the few rows' activated columns NormOut::scaled, of leading dimension NormOut::ld.
 
 // Where an attention layer wants the sums of its q/k/v product (columns: n_heads * hd queries, n_kv * hd keys, n_kv * hd values):
 // queries rotated into q_out, keys rotated and values as they are into the page table[slot][pos / page_size] at place
@@ -527,6 +533,8 @@ __device__ __forceinline__ void piped_tile(const bf16_t* __restrict__ A, const b
             return;
         }
     }
+    float act_a = 0.f, act_b = 0.f;
+    if constexpr (EPI == EPI_XIELU) { act_a = softplus_f32(norm_out.g[0]); act_b = 0.5f + softplus_f32(norm_out.g[1]); }
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -540,7 +548,9 @@ __device__ __forceinline__ void piped_tile(const bf16_t* __restrict__ A, const b
                     if ((lane & 16) == 0 && m < M && n < N)
                         ((bf16_t*)C)[(size_t)m * ldc + (n >> 5) * 16 + (lane & 15)] = f32_to_bf16(gate_of<EPI>(acc[i][j][v], up, norm_in.limit));
                 } else if constexpr (EPI != EPI_QKV_ROPE) {
-                    if (m < M && n < N) write_out<EPI>(C, (size_t)m * ldc + n, acc[i][j][v]);
+                    float sum = acc[i][j][v];
+                    if constexpr (EPI == EPI_XIELU) sum = xielu_fast(sum, act_a, act_b);
+                    if (m < M && n < N) write_out<EPI>(C, (size_t)m * ldc + n, sum);
                 }
             }
 }
@@ -791,7 +801,16 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
                 }
             }
         }
-    } else if constexpr (EPI == EPI_STORE_BF16) {
+    } else if constexpr (EPI == EPI_STORE_BF16 || EPI == EPI_XIELU) {
+        if constexpr (EPI == EPI_XIELU) {
+            const float act_a = softplus_f32(norm_in.squares[0]), act_b = 0.5f + softplus_f32(norm_in.squares[1]);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[i][j][v] = xielu_fast(acc[i][j][v], act_a, act_b);
+        }
 #pragma unroll
         for (int part = 0; part < TN / 2; ++part) {                                // 64 columns = 128 bytes a row at a time
 #pragma unroll
@@ -1042,7 +1061,9 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
                 }
             }
         } else {
-            constexpr int ELEM = EPI == EPI_STORE_BF16 ? 2 : 4;
+            constexpr int ELEM = EPI == EPI_STORE_BF16 || EPI == EPI_XIELU ? 2 : 4;
+            float act_a = 0.f, act_b = 0.f;
+            if constexpr (EPI == EPI_XIELU) { act_a = softplus_f32(norm_out.g[0]); act_b = 0.5f + softplus_f32(norm_out.g[1]); }
             const int c = n0 + (tid & 31) * 4;
             const bool whole = c + 3 < N && (ldc & 3) == 0 && ((uintptr_t)C & (4 * ELEM - 1)) == 0;
 #pragma unroll
@@ -1050,9 +1071,10 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
                 const int row = (tid >> 5) + it * 16, m = first + row;
                 if (m >= M) continue;
                 float4 v = *reinterpret_cast<const float4*>(tile + row * 128 + (tid & 31) * 4);
+                if constexpr (EPI == EPI_XIELU) v = float4{xielu_fast(v.x, act_a, act_b), xielu_fast(v.y, act_a, act_b), xielu_fast(v.z, act_a, act_b), xielu_fast(v.w, act_a, act_b)};
                 const size_t at = (size_t)m * ldc + c;
                 if (whole) {
-                    if constexpr (EPI == EPI_STORE_BF16) {
+                    if constexpr (ELEM == 2) {
                         *reinterpret_cast<uint2*>((bf16_t*)C + at) = uint2{f32x2_to_bf16x2(v.x, v.y), f32x2_to_bf16x2(v.z, v.w)};
                     } else {
                         if constexpr (EPI == EPI_ADD_F32) {
@@ -1456,6 +1478,8 @@ __global__ __launch_bounds__(256) void skinny_reduce_rope_store_kernel(const flo
 template <int STRIPS, int ROWS, int EPI, bool HAND, int FOLD = 0>
 __global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ C,
                                                             int M, int N, int K, long lda, long ldw, long ldc, NormIn norm_in, NormOut norm_out) {
+    float act_p = 0.f, act_q = 0.f;
+    if constexpr (EPI == EPI_XIELU) { act_p = norm_out.g[0]; act_q = norm_out.g[1]; }
     static_assert(FOLD == 0 || ROWS == 8, "folding k into the idle rows needs strips of 8 weight rows");
     constexpr int BLOCK = FOLD ? 2 * SK : SK, SPAN = BLOCK / 4;       // k of a block, and of one of its four products
     constexpr int XT = FOLD == 2 ? 2 : 1;                             // groups of rows of A
@@ -1607,6 +1631,9 @@ __global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __
                                 square = x * x;
                             }
                         }
+                    } else if constexpr (EPI == EPI_XIELU) {
+                        if (col < norm_in.first) ((float*)C)[(size_t)m * ldc + col] = sum;
+                        else norm_out.scaled[(size_t)m * norm_out.ld + col - norm_in.first] = f32_to_bf16(xielu(sum, softplus_f32(act_p), 0.5f + softplus_f32(act_q)));
                     } else {
                         write_out<EPI>(C, (size_t)m * ldc + col, sum);
                     }
@@ -1874,7 +1901,7 @@ static int slim_parts(int M, int N) {
 
 static int launch_slim(const void* A, const void* W, void* C, int epi, int M, int N, int K, long lda, long ldw, long ldc, NormIn norm_in,
                        NormOut norm_out, hipStream_t stream) {
-    const bool hand = norm_in.squares != nullptr || norm_out.scaled != nullptr;
+    const bool hand = norm_in.squares != nullptr || (norm_out.scaled != nullptr && epi != EPI_XIELU);
 #define SLIM(STRIPS_, ROWS_, EPI_)                                                                                                                     \
     do {                                                                                                                                               \
         if (hand) gemm_bf16_slim_kernel<STRIPS_, ROWS_, EPI_, true><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldw, ldc, norm_in, norm_out); \
@@ -1885,13 +1912,13 @@ static int launch_slim(const void* A, const void* W, void* C, int epi, int M, in
         if (epi == EPI_GATED_BF16) SLIM(2, 16, EPI_GATED_BF16); else if (epi == EPI_GATED_GELU_BF16) SLIM(2, 16, EPI_GATED_GELU_BF16); else SLIM(2, 16, EPI_GATED_CLAMP_BF16);
     } else if (slim_strip_rows(M, N, epi) == 16) {
         dim3 grid((N + 15) / 16);
-        if (epi == EPI_STORE_F32) SLIM(1, 16, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM(1, 16, EPI_ADD_F32); else SLIM(1, 16, EPI_STORE_BF16);
+        if (epi == EPI_STORE_F32) SLIM(1, 16, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM(1, 16, EPI_ADD_F32); else if (epi == EPI_XIELU) SLIM(1, 16, EPI_XIELU); else SLIM(1, 16, EPI_STORE_BF16);
     } else if (slim_strip_rows(M, N, epi) == 12) {     // (the last 4 of a product's 16 weight rows are the strip's last row again; their results are dropped)
         dim3 grid((N + 11) / 12);
-        if (epi == EPI_STORE_F32) SLIM(1, 12, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM(1, 12, EPI_ADD_F32); else SLIM(1, 12, EPI_STORE_BF16);
+        if (epi == EPI_STORE_F32) SLIM(1, 12, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM(1, 12, EPI_ADD_F32); else if (epi == EPI_XIELU) SLIM(1, 12, EPI_XIELU); else SLIM(1, 12, EPI_STORE_BF16);
     } else if (slim_strip_rows(M, N, epi) == 10) {
         dim3 grid((N + 9) / 10);
-        if (epi == EPI_STORE_F32) SLIM(1, 10, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM(1, 10, EPI_ADD_F32); else SLIM(1, 10, EPI_STORE_BF16);
+        if (epi == EPI_STORE_F32) SLIM(1, 10, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM(1, 10, EPI_ADD_F32); else if (epi == EPI_XIELU) SLIM(1, 10, EPI_XIELU); else SLIM(1, 10, EPI_STORE_BF16);
     } else {                                   // a narrow output: strips of 8 rows, twice the workgroups
         dim3 grid((N + 7) / 8);
 #define SLIM_FOLD(EPI_, FOLD_)                                                                                                                         \
@@ -1901,9 +1928,9 @@ static int launch_slim(const void* A, const void* W, void* C, int epi, int M, in
     } while (0)
         // the idle halves of the products take a further 32 of k: for up to 8 rows of A on both sides, for more on the weights' side
         if (M <= 8) {
-            if (epi == EPI_STORE_F32) SLIM_FOLD(EPI_STORE_F32, 1); else if (epi == EPI_ADD_F32) SLIM_FOLD(EPI_ADD_F32, 1); else SLIM_FOLD(EPI_STORE_BF16, 1);
+            if (epi == EPI_STORE_F32) SLIM_FOLD(EPI_STORE_F32, 1); else if (epi == EPI_ADD_F32) SLIM_FOLD(EPI_ADD_F32, 1); else if (epi == EPI_XIELU) SLIM_FOLD(EPI_XIELU, 1); else SLIM_FOLD(EPI_STORE_BF16, 1);
         } else {
-            if (epi == EPI_STORE_F32) SLIM_FOLD(EPI_STORE_F32, 2); else if (epi == EPI_ADD_F32) SLIM_FOLD(EPI_ADD_F32, 2); else SLIM_FOLD(EPI_STORE_BF16, 2);
+            if (epi == EPI_STORE_F32) SLIM_FOLD(EPI_STORE_F32, 2); else if (epi == EPI_ADD_F32) SLIM_FOLD(EPI_ADD_F32, 2); else if (epi == EPI_XIELU) SLIM_FOLD(EPI_XIELU, 2); else SLIM_FOLD(EPI_STORE_BF16, 2);
         }
 #undef SLIM_FOLD
     }
@@ -2041,6 +2068,7 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
         else if (epi == EPI_STORE_F32) PIPED(BM_, BN_, WM_, WN_, ST_, EPI_STORE_F32, C, ldc, 1, K, 0L, NO_NORM_IN, NO_ROPE);            \
         else if (epi == EPI_ADD_F32) PIPED(BM_, BN_, WM_, WN_, ST_, EPI_ADD_F32, C, ldc, 1, K, 0L, NO_NORM_IN, NO_ROPE);                \
         else if (epi == EPI_STORE_BF16) PIPED(BM_, BN_, WM_, WN_, ST_, EPI_STORE_BF16, C, ldc, 1, K, 0L, NO_NORM_IN, NO_ROPE);          \
+        else if (epi == EPI_XIELU) PIPED(BM_, BN_, WM_, WN_, ST_, EPI_XIELU, C, ldc, 1, K, 0L, NO_NORM_IN, NO_ROPE);                    \
         else if (epi == EPI_GATED_BF16) PIPED(BM_, BN_, WM_, WN_, ST_, EPI_GATED_BF16, C, ldc, 1, K, 0L, NO_NORM_IN, NO_ROPE);          \
         else if (epi == EPI_GATED_GELU_BF16) PIPED(BM_, BN_, WM_, WN_, ST_, EPI_GATED_GELU_BF16, C, ldc, 1, K, 0L, NO_NORM_IN, NO_ROPE); \
         else PIPED(BM_, BN_, WM_, WN_, ST_, EPI_GATED_CLAMP_BF16, C, ldc, 1, K, 0L, limit_in, NO_ROPE);                                 \
@@ -2079,6 +2107,7 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
         gemm_bf16_pingpong_kernel<256, EPI_><<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldw, ldc, norm_in); \
     } while (0)
         if (epi == EPI_STORE_F32) PINGPONG(EPI_STORE_F32); else if (epi == EPI_ADD_F32) PINGPONG(EPI_ADD_F32);
+        else if (epi == EPI_XIELU) { norm_in.squares = norm_out.g; PINGPONG(EPI_XIELU); }
         else if (epi == EPI_STORE_BF16) PINGPONG(EPI_STORE_BF16); else if (epi == EPI_GATED_BF16) PINGPONG(EPI_GATED_BF16); else if (epi == EPI_GATED_GELU_BF16) PINGPONG(EPI_GATED_GELU_BF16); else PINGPONG(EPI_GATED_CLAMP_BF16);
 #undef PINGPONG
         GI_CHECK_LAUNCH("gemm_bf16 (pingpong)");
@@ -2100,6 +2129,7 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
                                                                   rope != nullptr ? *rope : NO_ROPE, norm_out, order);                  \
     } while (0)
         if (rope != nullptr) TALL(EPI_QKV_ROPE); else if (epi == EPI_STORE_F32) TALL(EPI_STORE_F32); else if (epi == EPI_ADD_F32) TALL(EPI_ADD_F32);
+        else if (epi == EPI_XIELU) TALL(EPI_XIELU);
         else if (epi == EPI_STORE_BF16) TALL(EPI_STORE_BF16); else if (epi == EPI_GATED_BF16) TALL(EPI_GATED_BF16); else if (epi == EPI_GATED_GELU_BF16) TALL(EPI_GATED_GELU_BF16); else TALL(EPI_GATED_CLAMP_BF16);
 #undef TALL
         GI_CHECK_LAUNCH("gemm_bf16 (tall)");
@@ -2225,6 +2255,32 @@ GI_API int gi_gemm_bf16_qkv_rope_store(const void* A, const void* W, int M, int 
         return launch_large(A, W, nullptr, EPI_STORE_F32, M, N, K, lda, ldw, (long)N, scratch, scratch_floats, NormIn{squares_in, parts_in, eps, K}, &rope, stream);
     return launch_skinny(A, W, nullptr, EPI_STORE_F32, M, N, K, lda, ldw, (long)N, scratch, scratch_floats, NormIn{squares_in, parts_in, eps, K}, NO_NORM_OUT,
                          stream, &rope);
+}
+
+// Whether gi_gemm_bf16_xielu takes a product of these sizes: up to 16 rows where the kernel for those serves; the rows of prompts
+// where all of a tile's k is one workgroup's, with all columns through the activation.
+GI_API int gi_gemm_bf16_xielu_takes(int M, int N, int K, int first) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 8 != 0 || first < 0 || first >= N) return 0;
+    if (takes_slim(M, N, K)) return 1;
+    return M > SKINNY_MAX_ROWS && first == 0 && K % PK == 0 && N >= 128 && gi_gemm_bf16_piped_splits(M, N, K) == 1;
+}
+
+// A product whose columns from `first` on are a feed-forward's that has no gate: they leave through the activation xielu (params: its two
+// numbers) as act_out [M, ld_act] in bfloat16, the columns before as 32-bit C [M, ldc] (null where first is 0).  squares_in, parts_in, eps: a
+// norm handed on, as for gi_gemm_bf16_handing (null: none; up to 16 rows only).
+GI_API int gi_gemm_bf16_xielu(const void* A, const void* W, void* C, int M, int N, int K, long lda, long ldw, long ldc, int first, const float* params, void* act_out,
+                              long ld_act, const float* squares_in, int parts_in, float eps, hipStream_t stream) {
+    GI_REQUIRE((M + 63) / 64 <= 65535, "gemm_bf16: M %d is too large", M);
+    GI_REQUIRE(gi_gemm_bf16_xielu_takes(M, N, K, first), "gemm_bf16 (xielu): sizes M %d, N %d, K %d with %d columns as they are are not taken", M, N, K, first);
+    GI_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && lda >= K && ldw >= K && ((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0,
+               "gemm_bf16 (xielu): rows must be 16-byte aligned (strides %ld, %ld)", lda, ldw);
+    GI_REQUIRE(params != nullptr && act_out != nullptr && ld_act >= N - first && (first == 0 || (C != nullptr && ldc >= first)), "gemm_bf16 (xielu): outputs or parameters are missing");
+    const bool slim = takes_slim(M, N, K);
+    GI_REQUIRE(squares_in == nullptr || (slim && parts_in > 0 && parts_in <= slim_max_parts(M)), "gemm_bf16 (xielu): %d pieces of a sum of squares are not taken", parts_in);
+    NormIn in = {squares_in, parts_in, eps, K, 0.f};
+    in.first = first;
+    if (slim) return launch_slim(A, W, C, EPI_XIELU, M, N, K, lda, ldw, ldc, in, NormOut{params, (bf16_t*)act_out, ld_act, nullptr}, stream);
+    return launch_large(A, W, act_out, EPI_XIELU, M, N, K, lda, ldw, ld_act, nullptr, 0, NO_NORM_IN, nullptr, stream, NormOut{params, nullptr, 0, nullptr});
 }
 
 // `gated` != 0: W is [gate; up] interleaved in groups of 16 rows (N rows in all, a multiple of 32)

@@ -66,6 +66,8 @@ _SIGNATURES = {
                          c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "gi_gemm_bf16_grouped": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long, c_void_p],
     "gi_experts_down": [c_void_p, c_int, c_long, c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_long, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_long, c_int, c_void_p],
+    "gi_gemm_bf16_xielu": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_int, c_void_p, c_void_p, c_long, c_void_p, c_int, c_float,
+                           c_void_p],
     "gi_xielu": [c_void_p, c_long, c_void_p, c_int, c_long, c_int, c_int, c_void_p, c_void_p],
     "gi_delta_prepare": [c_void_p, c_long, c_int, c_void_p, c_long, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p,
                          c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p],
@@ -145,6 +147,8 @@ def lib():
         l.gi_gemm_bf16_scratch_floats.restype = c_long
         l.gi_gemm_bf16_norm_parts.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_bf16_norm_parts.restype = c_int
+        l.gi_gemm_bf16_xielu_takes.argtypes = [c_int, c_int, c_int, c_int]
+        l.gi_gemm_bf16_xielu_takes.restype = c_int
         l.gi_gemm_bf16_takes_norm.argtypes = [c_int, c_int, c_int, c_int]
         l.gi_gemm_bf16_takes_norm.restype = c_int
         l.gi_gemm_bf16_qkv_rope_store_takes.argtypes = [c_int, c_int, c_int, c_int]
@@ -188,7 +192,7 @@ def _call(name, *args):
         raise KernelError(lib().gi_last_error().decode())
 
 
-_PROFILE_LABEL = {"gi_gemm_bf16_handing": "gemm_bf16", "gi_gemm_bf16_qkv_rope_store": "gemm_bf16"}        # the same products, with a norm's share on top
+_PROFILE_LABEL = {"gi_gemm_bf16_handing": "gemm_bf16", "gi_gemm_bf16_xielu": "gemm_bf16", "gi_gemm_bf16_qkv_rope_store": "gemm_bf16"}        # the same products, with a norm's share on top
 
 
 class KernelProfile:
@@ -1494,6 +1498,34 @@ def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=N
     _call("gi_gemm_bf16", a.data_ptr(), w.data_ptr(), out.data_ptr(), _code(out, "gemm: out"), 1 if accumulate else 0, gate_code, float(gate_limit),
           m, n, k, a.stride(0), w.stride(0), out.stride(0), _ptr(scratch), n_scratch, _stream())
     return out
+
+
+@lru_cache(maxsize=None)
+def gemm_bf16_xielu_takes(m, n, k, first=0) -> bool:
+    """Whether `gemm_bf16_xielu` takes a product of these sizes, `first` of whose columns stay as they are."""
+    return bool(lib().gi_gemm_bf16_xielu_takes(m, n, k, first))
+
+
+def gemm_bf16_xielu(a, w, params, mid, out=None, norm_in=None):
+    """a @ w.T whose last mid.shape[1] columns leave through the activation `xielu` (params as there) as mid, bfloat16 [m, columns]; the columns
+    before them, if there are any, go to the first columns of out, float32 [m, >= columns].  norm_in as for `gemm_bf16`."""
+    _dev(a, w, params, mid, out)
+    m, k = a.shape
+    n = w.shape[0]
+    first = n - mid.shape[1]
+    if not (w.shape == (n, k) and a.dtype == w.dtype == mid.dtype == torch.bfloat16 and a.stride(1) == 1 and w.stride(1) == 1 and mid.shape[0] == m and mid.stride(1) == 1
+            and params.dtype == torch.float32 and params.is_contiguous() and params.numel() == 2):
+        raise KernelError("gemm (xielu): bfloat16 operands and results [m, columns] with unit inner stride and two float32 parameters are needed")
+    if first and not (out is not None and out.dtype == torch.float32 and out.dim() == 2 and out.shape[0] == m and out.shape[1] >= first and out.stride(1) == 1):
+        raise KernelError(f"gemm (xielu): float32 [m, {first}] is needed for the columns that stay as they are")
+    squares_in, eps = norm_in if norm_in is not None else (None, 0.0)
+    if squares_in is not None and not (squares_in.dtype == torch.float32 and squares_in.is_contiguous() and squares_in.dim() == 2 and squares_in.shape[0] == m):
+        raise KernelError("gemm: the pieces of the sums of squares must be float32 [m, pieces]")
+    if _profile is not None:
+        _profile.note = (f"{n}x{k} xielu", n * k * w.element_size())
+    _call("gi_gemm_bf16_xielu", a.data_ptr(), w.data_ptr(), _ptr(out), m, n, k, a.stride(0), w.stride(0), out.stride(0) if out is not None else 0, first, params.data_ptr(),
+          mid.data_ptr(), mid.stride(0), _ptr(squares_in), squares_in.shape[1] if squares_in is not None else 0, float(eps), _stream())
+    return mid
 
 
 @lru_cache(maxsize=None)

@@ -14,7 +14,7 @@ import torch
 
 from ..kernels import ops
 from .base import feed_forward_class, mixer_class, norm_class, register_block
-from .linear import linear, takes_handed_norm
+from .linear import linear, linear_xielu, takes_handed_norm
 from .norm import NormedRows, ReadyRows, norm_to_apply, norm_to_hand_on
 
 
@@ -272,8 +272,12 @@ class ParallelBlock:
         w_first = self._stacked(ctx.n_rows)
         if w_first is not None:
             both = torch.empty((ctx.n_rows, w_first.shape[0]), dtype=torch.float32, device=x.device)
-            linear(rows(self.mixer), w_first, both)
-            own[0]["projected"], own[1]["projected"] = both[:, :self._split], both[:, self._split:]
+            activated = self.feed_forward.activated(ctx.n_rows, x.device) if hasattr(self.feed_forward, "activated") else None
+            if activated is not None and linear_xielu(rows(self.mixer), w_first, activated[1], activated[0], both):
+                own[0]["projected"], own[1]["activated"] = both[:, :self._split], activated[0]
+            else:
+                linear(rows(self.mixer), w_first, both)
+                own[0]["projected"], own[1]["projected"] = both[:, :self._split], both[:, self._split:]
         if then is not None:
             own[0 if last is self.mixer else 1]["then"] = then
         out = self.mixer.forward(rows(self.mixer), x, ctx, cache, **own[0])

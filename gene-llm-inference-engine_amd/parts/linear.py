@@ -33,6 +33,26 @@ def linear(a, weight: torch.Tensor, out: torch.Tensor, accumulate: bool = False,
     return ops.gemm_exact(a, weight, out, accumulate)
 
 
+def linear_xielu(a, weight: torch.Tensor, params: torch.Tensor, mid: torch.Tensor, out: torch.Tensor = None) -> bool:
+    """The product of `linear` with the activation of a feed-forward that has no gate in its epilogue, where a kernel does both
+    (`ops.gemm_bf16_xielu`): its last mid.shape[1] columns go to mid, the ones before to out.  False, and nothing done, where none does."""
+    n, k = weight.shape
+    rows = mid.shape[0]
+    if not (weight.dtype == torch.bfloat16 and mid.dtype == torch.bfloat16 and ops.gemm_bf16_xielu_takes(rows, n, k, n - mid.shape[1])):
+        return False
+    if isinstance(a, HandedRows) and rows <= 16 and takes_handed_norm(weight, rows) and ops.gemm_bf16_supports(a.scaled, weight, mid):
+        ops.gemm_bf16_xielu(a.scaled, weight, params, mid, out, norm_in=(a.squares, a.eps))
+        return True
+    if isinstance(a, HandedRows) or not (torch.is_tensor(a) or isinstance(a, NormedRows)):
+        return False
+    if isinstance(a, NormedRows):
+        a = a.materialize()
+    if not ops.gemm_bf16_supports(a, weight, mid):
+        return False
+    ops.gemm_bf16_xielu(a, weight, params, mid, out)
+    return True
+
+
 def linear_onto(a: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor, then=None):
     """residual += a @ weight.T.  `then`: the norm that reads `residual` next, if it and its reader can take it half applied
     (see `HandedRows`); the product then also does the norm's share and the `HandedRows` are returned, None otherwise."""

@@ -96,6 +96,38 @@ def test_activation_of_the_plain_feed_forward():
         assert torch.equal(half.cpu(), out.cpu().to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("rows, n, k, first", [(1, 416, 128, 320), (16, 320, 136, 3), (9, 1100, 2048, 0), (300, 8192, 256, 0), (131, 16400, 192, 0), (700, 8192, 512, 0), (1777, 8200, 320, 0),
+                                               (2048, 6000, 1024, 0)])
+def test_product_with_the_activation_of_the_plain_feed_forward(rows, n, k, first):
+    """Against the product and the activation one after the other: the sums are the same, the activation's own error is below 2^-20 of the
+    numbers it is made of (measured 2e-7 against 64 bits), so the results are the same up to one rounding to bfloat16."""
+    from geneinfer_amd.kernels import ops
+    assert ops.gemm_bf16_xielu_takes(rows, n, k, first)
+    g = torch.Generator(device=DEV).manual_seed(rows + n)
+    a = torch.randn(rows, k, device=DEV, generator=g).bfloat16()
+    w = (torch.randn(n, k, device=DEV, generator=g) * 1.5 / k ** 0.5).bfloat16()
+    a[0, :] = 0                                                          # (a row of zeros; one that leaves the range of exp; one of infinities)
+    if rows > 2:
+        a[1, :] *= 300
+        a[2, 0] = float("inf")
+    params = torch.tensor([0.3, -0.7], device=DEV)
+    both = torch.empty(rows, n, device=DEV)
+    ops.gemm_bf16(a, w, both)
+    want = torch.empty(rows, n - first, dtype=torch.bfloat16, device=DEV)
+    ops.xielu(both[:, first:], want, params)
+    out = torch.full((rows, n), 7.0, device=DEV) if first else None
+    mid = torch.full((rows + 1, n - first + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.gemm_bf16_xielu(a, w, params, mid[:rows, :n - first], out)
+    assert (mid[rows] == 7).all() and (mid[:, n - first:] == 7).all()
+    if first:
+        assert torch.equal(out[:, :first].nan_to_num(nan=9.0), both[:, :first].nan_to_num(nan=9.0)) and (out[:, first:] == 7).all()
+    got, want, z = mid[:rows, :n - first].float(), want.float(), both[:, first:]
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    fine = want.isfinite()
+    assert ((got - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -20 * z.abs())[fine].all()
+    assert ((got != want) & fine).float().mean() < 1e-3
+
+
 @pytest.mark.parametrize("heads, kv, dk, dv, taps", [(4, 2, 16, 24, 4), (3, 3, 64, 64, 2), (2, 1, 130, 10, 5), (1, 1, 7, 201, 1), (5, 5, 3, 5, 3), (2, 2, 300, 6, 8), (1, 1, 20, 9, 13)])
 def test_gated_delta_rule_kernels(heads, kv, dk, dv, taps):
     """Two requests of unequal length in one step; then the longer one again from a fresh slot in steps down to one and two rows:
