@@ -1821,7 +1821,9 @@ static Large large_kernel(int M, int N, int K, bool rope, bool gated, bool scale
     if (scaled_rows && !rope) piped = 1e30;
     const double tall = rounds(m256 * n128) * (blocks * 0.715 + 13);
     const double pingpong = many_tiles(M, N) && !rope ? rounds(m256 * n256) * (blocks * 1.45 + 14) : 1e30;
-    if (pingpong < piped && 0.95 * pingpong <= tall) return PINGPONG_256;
+    // (gating 256 x 128 sums at a time costs the tall kernel 3 us a round more: 1,500 rows by 16,384 of 2,048, three rounds of it against one and a
+    // half of the ping-pong kernel: 114 us against 103)
+    if (pingpong < piped && 0.95 * pingpong <= tall + (gated ? 3 * rounds(m256 * n128) : 0)) return PINGPONG_256;
     return tall < piped ? TALL_256 : PIPED_128;
 }
 
