@@ -4,7 +4,7 @@
 // one 16-byte load of 8 consecutive k.  Six kernels:
 //
 //   pingpong  large prompt-sized products (256 x 256 tiles for most of the compute units): operands loaded
-//           from global memory straight into two LDS stages; the workgroup's eight waves form two
+//           from global memory straight into LDS, two stages of A and three of W; the workgroup's eight waves form two
 //           groups that take turns at reading LDS and at the matrix instructions.
 //   tall    those in between: the same on tiles of 256 x 128 and three LDS stages.
 //   piped   the other products of 128 rows or more (K a multiple of 64): tiles of 128 x 128,
