@@ -46,17 +46,20 @@ __device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) { return __buil
 
 constexpr int BLOCK = 64, SPAN = 4 * BLOCK, PAIRS = 16;
 
-// A span joins what came before it (m, l, and every O with the two factors): nothing happens for a row that sees no key of the span.
-struct Join { float before, span; };
-__device__ __forceinline__ Join join(float& m, double& l, float m_span, double l_span) {
-    if (m_span == -INFINITY) return {1.f, 0.f};
+// A span joins what came before it (m, l, and every O with the two factors): nothing happens for a row that sees no key of the span, which its
+// positions tell and not the scores (a score that is no number does not show in the largest one: the row's sums must hand it on, and so must
+// a value that is none, whatever factor it meets).
+struct Join { float before, span; };             // span < 0: the row sees none of it
+__device__ __forceinline__ Join join(float& m, double& l, bool sees, float m_span, double l_span) {
+    if (!sees) return {1.f, -1.f};
     const float top = fmaxf(m, m_span);
-    const Join f = {expf(m - top), expf(m_span - top)};       // (m = -inf at the first span without sinks: 0)
+    // (m = -inf at the first span without sinks: 0; both -inf: sums of zeros, or ones that are no numbers)
+    const Join f = top == -INFINITY ? Join{1.f, 1.f} : Join{expf(m - top), expf(m_span - top)};
     l = fma(l_span, (double)f.span, l * (double)f.before);
     m = top;
     return f;
 }
-__device__ __forceinline__ float joined(float o, float o_span, Join f) { return f.span == 0.f && f.before == 1.f ? o : fmaf(o_span, f.span, o * f.before); }
+__device__ __forceinline__ float joined(float o, float o_span, Join f) { return f.span < 0.f ? o : fmaf(o_span, f.span, o * f.before); }
 
 __device__ __forceinline__ int first_key(int pos, int window, int chunk) {
     int lo = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
@@ -83,7 +86,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
                                                                    const float* __restrict__ gate, long gate_stride, int gate_channels, int rows_a_tile,
                                                                    float* __restrict__ part, int n_spans) {
     __shared__ float o_s[4][PAIRS][D + 4];
-    __shared__ float m_s[4][PAIRS], l_s[4][PAIRS], f_s[4][PAIRS];        // of the blocks; f: their factors
+    __shared__ float m_s[4][PAIRS], l_s[4][PAIRS], f_s[4][PAIRS];        // of the blocks; f: their factors, negative where the pair sees none of the block's keys
     __shared__ float m_all[PAIRS];
     __shared__ double l_all[PAIRS];
     __shared__ Join join_s[PAIRS];
@@ -235,9 +238,10 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
                 double sum = 0.0;
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
+                    const bool sees = run_s[tid] && s * SPAN + b * BLOCK <= pos_s[tid] && s * SPAN + (b + 1) * BLOCK > lo_s[tid];
                     const float f = m_s[b][tid] == -INFINITY ? 0.f : expf(m_s[b][tid] - top);
-                    f_s[b][tid] = f;
-                    sum = fma((double)l_s[b][tid], (double)f, sum);
+                    f_s[b][tid] = sees ? f : -1.f;
+                    if (sees) sum = fma((double)l_s[b][tid], (double)f, sum);
                 }
                 if (part) {
                     const int at = s - lo_s[tid] / SPAN;
@@ -249,7 +253,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
                 } else {
                     float m_now = m_all[tid];
                     double l_now = l_all[tid];
-                    join_s[tid] = join(m_now, l_now, top, sum);
+                    join_s[tid] = join(m_now, l_now, run_s[tid] && s * SPAN <= pos_s[tid] && (s + 1) * SPAN > lo_s[tid], top, sum);
                     m_all[tid] = m_now;
                     l_all[tid] = l_now;
                 }
@@ -263,7 +267,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
                     const float f = f_s[b][pair];
-                    if (f != 0.f) o = fmaf(o_s[b][pair][d], f, o);         // (an empty block has left nothing there)
+                    if (!(f < 0.f)) o = fmaf(o_s[b][pair][d], f, o);       // (a block the pair sees nothing of may have left nothing there)
                 }
                 if (part) {
                     const int span = s - lo_s[pair] / SPAN;
@@ -300,7 +304,7 @@ __global__ __launch_bounds__(128) void attention_exact_join_kernel(const float* 
     const int channel = min(d, vd - 1);
     for (int s = 0; s < count; ++s, from += part_floats(vd)) {
         const float o_span = from[channel];
-        const Join f = join(m, l, from[vd + 2], *reinterpret_cast<const double*>(from + vd));
+        const Join f = join(m, l, true, from[vd + 2], *reinterpret_cast<const double*>(from + vd));
         o = joined(o, o_span, f);
     }
     if (d < vd) out[(size_t)blockIdx.x * vd + d] = finished(o, l, gate, gate_stride, gate_channels, t, h, d);

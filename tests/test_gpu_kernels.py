@@ -767,6 +767,101 @@ def test_attention_exact_has_one_order_of_sums(n_heads, n_kv, hd, ps, window, ch
         assert torch.equal(hurt[~sees], whole[~sees]) and not bool(torch.isfinite(hurt[sees]).any())
 
 
+@pytest.mark.parametrize("sinks", [False, True])
+@pytest.mark.parametrize("n_heads,n_kv,hd,ps,window", [(4, 2, 64, 16, None), (6, 1, 128, 4, None), (2, 2, 32, 16, 400)])
+@pytest.mark.parametrize("known", [dict(), dict(max_context=770), dict(single_rows=True), dict(single_rows=True, max_context=770)], ids=["whole", "shared", "single", "single-shared"])
+def test_attention_exact_hands_on_what_is_no_number(n_heads, n_kv, hd, ps, window, sinks, known):
+    """32-bit: a query, a key or a value that is no number shows in every row that sees it and in no other, also where it is all that a row
+    sees of a span of 256 keys (positions 256, 512, 768), with sinks that keep the denominator finite, and where its block's factor is zero."""
+    contexts = [770, 300]
+    cache, table, _ = build_paged(contexts, n_kv, hd, ps, torch.float32, seed=5)
+    rows = [(0, p) for p in (0, 2, 3, 255, 256, 257, 300, 511, 512, 513, 767, 768, 769)] + [(1, p) for p in (256, 299)]
+    pos = torch.tensor([p for _, p in rows], dtype=torch.int32, device=DEV)
+    slots = torch.tensor([r + 1 for r, _ in rows], dtype=torch.int32, device=DEV)
+    one = randn(hd, seed=7)
+    q = one.repeat(len(rows), n_heads).contiguous()
+    s = randn(n_heads, seed=8) if sinks else None
+
+    def attend():
+        out = torch.full_like(q, 7.0)
+        return ops().attention_exact(q, cache, out, pos, slots, table, n_heads, n_kv, hd, window, sinks=s, **known)
+
+    def sees(request, place):
+        return torch.tensor([r == request and p >= place and (window is None or p - window < place) for r, p in rows], device=DEV)
+
+    def keys(place):
+        return cache[int(table[1, place // ps]), 0][:, place % ps]
+
+    clean = attend()
+    assert bool(torch.isfinite(clean).all())
+    for place in (256, 512, 768, 300):
+        kept = keys(place).clone()
+        for bad in (float("nan"), float("inf")):                              # (infinite keys: scores of +inf, -inf or none, by the query's signs)
+            keys(place)[:] = bad
+            hurt, hit = attend(), sees(0, place)
+            assert torch.equal(hurt[~hit], clean[~hit]) and (bad == float("inf") or bool(torch.isnan(hurt[hit]).all()))
+        keys(place)[:] = kept
+    kept, q[4] = q[4].clone(), float("nan")                                    # position 256
+    hurt = attend()
+    assert bool(torch.isnan(hurt[4]).all()) and torch.equal(hurt[:4], clean[:4]) and torch.equal(hurt[5:], clean[5:])
+    q[4] = kept
+    keys(300)[:] = 30 * one                                                   # all others' shares are zero in 32 bits wherever this key is seen
+    cache[int(table[1, 3 // ps]), 1].view(n_kv, hd, ps)[:, :, 3 % ps] = float("inf")
+    hurt, hit, moved = attend(), sees(0, 3), sees(0, 300)
+    assert not bool(torch.isfinite(hurt[hit]).any())
+    assert torch.equal(hurt[~hit & ~moved], clean[~hit & ~moved]) and bool(torch.isfinite(hurt[~hit]).all())
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd,vd,cap,sinks,gate,chunk", [(6, 2, 64, 128, None, True, None, None), (4, 1, 128, 48, 5.0, False, "head", None), (8, 8, 32, 16, None, True, "channel", None),
+                                                                    (20, 1, 64, 64, 3.0, True, "head", 600), (3, 3, 16, 96, None, False, "channel", 320)])
+def test_attention_exact_shares_contexts_out_with_all_it_takes(n_heads, n_kv, hd, vd, cap, sinks, gate, chunk):
+    """32-bit: value heads of another size, capped scores, sinks, gates: a context shared out over workgroups gives the bits of one that is not,
+    and both are the plain statement's in 64 bits."""
+    ps, contexts = 8, [1030, 257]
+    g = torch.Generator().manual_seed(hd + vd)
+    pages = [-(-n // ps) for n in contexts]
+    order = torch.randperm(sum(pages), generator=g)
+    table = torch.full((2, max(pages)), -1, dtype=torch.int32)
+    cache = torch.full((sum(pages), n_kv * ps * (hd + vd)), float("nan"))
+    dense, at = [], 0
+    for r, n in enumerate(contexts):
+        k, v = torch.randn(pages[r] * ps, n_kv, hd, generator=g), torch.randn(pages[r] * ps, n_kv, vd, generator=g)
+        dense.append((k[:n].double(), v[:n].double()))
+        for i in range(pages[r]):
+            page = int(order[at])
+            table[r, i], at = page, at + 1
+            cache[page, :n_kv * ps * hd] = k[i * ps:(i + 1) * ps].permute(1, 0, 2).reshape(-1)
+            cache[page, n_kv * ps * hd:] = v[i * ps:(i + 1) * ps].permute(1, 2, 0).reshape(-1)
+    rows = [(0, p) for p in (1020, 1021, 1022, 1023, 1024, 1025, 63, 64, 600)] + [(1, p) for p in (256, 255, 0)]
+    pos = torch.tensor([p for _, p in rows], dtype=torch.int32)
+    slots = torch.tensor([r for r, _ in rows], dtype=torch.int32)
+    T = len(rows)
+    q = torch.randn(T, n_heads * hd, generator=g)
+    s = torch.randn(n_heads, generator=g) if sinks else None
+    gates = torch.randn(T, n_heads if gate == "head" else n_heads * vd, generator=g) if gate else None
+    want = torch.empty(T, n_heads, vd, dtype=torch.float64)
+    for i, (r, p) in enumerate(rows):
+        lo = p - p % chunk if chunk else 0
+        for h in range(n_heads):
+            kv = h // (n_heads // n_kv)
+            sc = dense[r][0][lo:p + 1, kv] @ q[i].view(n_heads, hd)[h].double() / math.sqrt(hd)
+            sc = cap * torch.tanh(sc / cap) if cap else sc
+            e = torch.exp(sc - sc.max())
+            o = e @ dense[r][1][lo:p + 1, kv] / (e.sum() + (torch.exp(s[h].double() - sc.max()) if sinks else 0))
+            want[i, h] = o * (torch.sigmoid(gates[i, h] if gate == "head" else gates[i].view(n_heads, vd)[h]).double() if gate else 1)
+    device = dict(sinks=s.to(DEV) if sinks else None, gate=gates.to(DEV) if gate == "head" else None, channel_gate=gates.to(DEV) if gate == "channel" else None)
+    q, cache, pos, slots, table = (x.to(DEV) for x in (q, cache, pos, slots, table))
+
+    def attend(**known):
+        out = torch.full((T, n_heads * vd), float("nan"), device=DEV)
+        return ops().attention_exact(q, cache, out, pos, slots, table, n_heads, n_kv, hd, page_size=ps, value_dim=vd, cap=cap, chunk=chunk, **device, **known)
+
+    whole = attend()
+    assert rel(whole, want.view(T, -1)) < 2e-6                                 # (as the test of one order of sums)
+    for known in (dict(max_context=1030), dict(max_context=4096), dict(single_rows=True), dict(single_rows=True, max_context=1030)):
+        assert torch.equal(attend(**known), whole), known
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_finds_one_far_key(dtype):
     """Among 700 keys one is scaled so that its score stands out: the output must be its value."""
