@@ -899,7 +899,7 @@ struct TileOrder {
 };
 template <int EPI>
 __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ C, int M, int N, int K,
-                                                            long lda, long ldw, long ldc, NormIn norm_in, RopeStore rope, NormOut norm_out, TileOrder order) {
+                                                            long lda, long ldw, long ldc, NormIn norm_in, RopeStore rope, NormOut norm_out, TileOrder order, bool quick_gate) {
     const TileOrder::Tile at_tile = order.tile(blockIdx.x);
     if (at_tile.m < 0) return;
     constexpr int BM = 256, BN = 128, NT = 512, TM = 2, TN = 2, ROWS = BM + BN, STAGE_BYTES = ROWS * 128, LOADS = 6;
@@ -1043,7 +1043,9 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
         } else if (EPI == EPI_ADD_F32 && norm_out.scaled != nullptr) {
             tile_add_handing_norm<NT>(tile, old[half], (float*)C, ldc, first, n0, M, norm_out, at_tile.n, order.n_tiles);
         } else if constexpr (is_gated(EPI)) {
-            // columns 32b .. 32b+15 are gates, 32b+16 .. 32b+31 the ups of outputs 16b .. 16b+15; a thread makes two neighbouring outputs
+            // Columns 32b .. 32b+15 are gates, 32b+16 .. 32b+31 the ups of outputs 16b .. 16b+15; a thread makes two neighbouring outputs.
+            // The quick gate is the ping-pong kernel's, whose products with many tiles these may be; the others have the gate of the
+            // kernel with tiles of 128 x 128, in bits (at 300 rows of 16,384 x 2,048 it costs 2.5 us of 39).
             const int o = (tid & 31) * 2, c = n0 / 2 + o;
 #pragma unroll
             for (int it = 0; it < 8; ++it) {
@@ -1051,7 +1053,8 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
                 if (m >= M || c >= N / 2) continue;
                 const float* from = tile + row * 128 + (o >> 4) * 32 + (o & 15);
                 const float2 g = *reinterpret_cast<const float2*>(from), u = *reinterpret_cast<const float2*>(from + 16);
-                const uint32_t both = f32x2_to_bf16x2(gate_fast_of<EPI>(g.x, u.x, norm_in.limit), gate_fast_of<EPI>(g.y, u.y, norm_in.limit));
+                const uint32_t both = quick_gate ? f32x2_to_bf16x2(gate_fast_of<EPI>(g.x, u.x, norm_in.limit), gate_fast_of<EPI>(g.y, u.y, norm_in.limit))
+                                                 : f32x2_to_bf16x2(gate_of<EPI>(g.x, u.x, norm_in.limit), gate_of<EPI>(g.y, u.y, norm_in.limit));
                 bf16_t* to = (bf16_t*)C + (size_t)m * ldc + c;
                 if ((ldc & 1) == 0 && ((uintptr_t)C & 3) == 0) {                          // (N / 2 is a multiple of 16: both exist)
                     *reinterpret_cast<uint32_t*>(to) = both;
@@ -1808,7 +1811,7 @@ static bool many_tiles(int M, int N) { return (long)((M + 255) / 256) * ((N + 25
 
 // Which kernel takes a product of more than 128 rows that does not share k out: what counts are the rounds of tiles on the compute units,
 // each with what a tile takes to begin and to end.  Microseconds, fitted to measurements at K = 1,024 to 8,192 (2,048 rows of 3,072 x 2,048:
-// 51.5 with 128 x 128 tiles in two rounds, 35.0 with 256 x 128 in one; 300 rows of 16,384 x 2,048 gated 42.5 and 36.2; 3,000 rows of 3,072 x 2,048
+// 51.5 with 128 x 128 tiles in two rounds, 35.0 with 256 x 128 in one; 300 rows of 16,384 x 2,048 gated 42 and 39; 3,000 rows of 3,072 x 2,048
 // 88 and 66; 2,048 rows of 16,384 x 2,048 gated 152 with 256 x 128 in four rounds, 120 with 256 x 256 in two).  Only the two larger tiles finish a
 // norm handed on to a gated product; the q/k/v product's epilogue rotates tiles 128 columns wide.
 enum Large { PIPED_128, TALL_256, PINGPONG_256 };
@@ -2128,7 +2131,7 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
         const TileOrder order = tall_order(M, N);                                                                                       \
         dim3 grid(8 * order.each);                                                                                                      \
         gemm_bf16_tall_kernel<EPI_><<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldw, ldc, norm_in, \
-                                                                  rope != nullptr ? *rope : NO_ROPE, norm_out, order);                  \
+                                                                  rope != nullptr ? *rope : NO_ROPE, norm_out, order, many_tiles(M, N)); \
     } while (0)
         if (rope != nullptr) TALL(EPI_QKV_ROPE); else if (epi == EPI_STORE_F32) TALL(EPI_STORE_F32); else if (epi == EPI_ADD_F32) TALL(EPI_ADD_F32);
         else if (epi == EPI_XIELU) TALL(EPI_XIELU);

@@ -135,6 +135,19 @@ def test_gemm_bf16_gated(m, inter, k):
     assert torch.all(out[:, inter:] == 3.0)
 
 
+@pytest.mark.parametrize("gated,limit", [(True, 0.0), ("gelu_tanh", 0.0), ("swish_clamped", 1.5)])
+@pytest.mark.parametrize("m,inter,k,few,columns,stride", [(300, 8192, 2048, 256, 8192, 8192), (500, 8192, 512, 131, 8192, 8195), (200, 14336, 512, 200, 8192, 14336), (257, 8176, 512, 256, 8176, 8178)])
+def test_gated_products_have_one_gate(m, inter, k, few, columns, stride, gated, limit):
+    """The tiles of 256 x 128 gate as those of 128 x 128 do, which fewer rows or fewer columns take: the same sums, the same results in bits."""
+    a = randn(m, k, dtype=torch.bfloat16, seed=15)
+    w = randn(2 * inter, k, dtype=torch.bfloat16, seed=16, scale=2.0 / k ** 0.5)
+    out = torch.full((m, stride), 3.0, dtype=torch.bfloat16, device=DEV)
+    ops().gemm_bf16(a, w, out[:, :inter], gated=gated, gate_limit=limit)
+    alone = torch.empty(few, columns, dtype=torch.bfloat16, device=DEV)
+    ops().gemm_bf16(a[:few], w[:2 * columns], alone, gated=gated, gate_limit=limit)
+    assert torch.equal(out[:few, :columns], alone) and bool((out[:, inter:] == 3.0).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(4109, 4120, 192), (4096, 4096, 448)])
 def test_gemm_bf16_ping_pong_with_whole_lines(m, n, k):
     """Outputs whose rows are 16-byte aligned leave the ping-pong kernel in whole cache lines: every epilogue, with edge tiles."""
