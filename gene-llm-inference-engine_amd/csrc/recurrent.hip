@@ -361,200 +361,238 @@ __global__ __launch_bounds__(256) void delta_tail_kernel(const float* __restrict
     }
 }
 
-// The rule itself: one wave per (request of the step, head, two columns of M).  lane = column * 32 + group of rows; a lane keeps
-// ROWS neighbouring rows of its column.  State of a request slot: [head][tile]{[dk][4]}, tiles of four columns.
-// With M the memory before the token, e = s (v - d M^T k), M' = d M + k e^T after it and y = M'^T q.  A token's chain is one pass over
-// the rows, one sum over 32 lanes and the update; a token's read-out y is summed beside the next token's M^T k (both read the memory
-// that the token left).  Every sum over the
-// key's rows is the lanes' own shares in a fixed order, then the 32 groups by lane moves: the bits do not depend on the cut.
-// CHANNEL: the decay is a number per key channel and scales the memory's rows first: e = s (v - (D M)^T k), M' = D M + k e^T.
-// Bound by that chain and by the seven clocks or so that each instruction of a wave alone on its SIMD takes, token after token (two waves a
-// compute unit at 8 heads of 64 x 128): a token's numbers come from memory
-// into the lanes' registers TB tokens and more ahead, and nothing but its own 22 instructions stands in the way.  1,777 tokens of 8 such heads
-// take 191 us; 201 with four columns a wave (38 instructions a token), 281 with keys and queries staged in LDS, each token's reads
-// waited for in its turn, and k . q as a third sum (y = d M^T q + e (k . q)).
+// The rule itself: one wave per (request of the step, head, four columns of M).  lane = column * 16 + group of rows; a lane keeps
+// the rows 16 apart of its column.  State of a request slot: [head][tile]{[dk][4]}.
+// With M the memory before the token, M' = d M + k e^T after it and e = s (v - d M^T k), the read-out is
+//     y = M'^T q = d M^T q + e (k . q):
+// both sums over the old memory's rows (M^T k and M^T q) are taken in one pass and reduced side by side, the memory is
+// updated behind them, and a token's chain of dependent steps is one pass and one reduction, not two of each.  Every sum over the
+// key's rows is the lanes' own shares in a fixed order, then the 16 groups by lane moves: the bits do not depend on the cut.
+// CHANNEL: the decay is a number per key channel, so the sums are taken over D M, whose rows the decays have scaled already:
+//     e = s (v - (D M)^T k),   y = (D M)^T q + e (k . q).
+// Bound by the seven clocks or so that each instruction of a wave alone on its SIMD takes, token after token (one wave a compute unit at 8
+// heads of 64 x 128), so nothing stands in a token that can stand elsewhere: a block's keys and queries are asked for a block ahead, four
+// channels a load, and wait in LDS; a token's numbers leave LDS while the token before is worked on; k . q, in which nothing of the memory
+// is, is summed for four tokens at once before the block.  Microseconds for 1,777 tokens of 8 such heads, five requests of 200, 1,024
+// tokens of 32 heads of 128 x 128 with decays per channel: 207, 38, 270; each token's reads waited for in its turn and k . q summed in it: 279, 51,
+// 317; two columns a wave (rows of a lane neighbours, another order of the sums), a token's numbers loaded straight into registers: 192, 69,
+// 246, but 115 for 64 single rows of 32 heads of 128 x 128 that take 57 with four columns.
+// A token's numbers for a lane's rows of a column: {k, q} of every row, the rows' decays where there is one per channel, and own = {decay, step, v, k . q}.
 template <int ROWS, bool CHANNEL>
-struct DeltaItem {
-    float k[ROWS], q[ROWS], d[CHANNEL ? ROWS : 1];
-    float v, decay, step;
+struct DeltaToken {
+    float2 kq[ROWS];
+    float d[CHANNEL ? ROWS : 1];
+    float4 own;
 };
 
-// The sums of x and of y over the 32 lanes of a column, taken side by side: rows of 16 lanes trade places so that one addition leaves
-// x's sixteen pairs in the column's first row and y's in its second, and four moves within a row finish both.
-struct PairSum { float x, y; };                  // x in every lane; y in the column's second row
-__device__ __forceinline__ PairSum pair_sum(float x, float y) {
-    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);      // {x of row 0, y of row 0}, {x of row 1, y of row 1}
-    const float both = group_sum<16>(__uint_as_float(rows[0]) + __uint_as_float(rows[1]));
-    // row_bcast:15, rows 1 and 3: the last lane of the row before
-    return {__int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(both), __float_as_int(both), 0x142, 0xA, 0xF, false)), both};
+// A lane's share of k . q (the form with decays per channel rounds every product).
+template <int ROWS, bool CHANNEL>
+__device__ __forceinline__ float delta_key_query(const float2 (&x)[ROWS]) {
+#pragma clang fp contract(off)
+    float kq = 0.f;
+#pragma unroll
+    for (int rr = 0; rr < ROWS; ++rr) kq = CHANNEL ? kq + x[rr].x * x[rr].y : fmaf(x[rr].x, x[rr].y, kq);
+    return kq;
 }
 
-// The sums over a column's rows that a token and the read-out before it need: one pass over the memory as the last token left it.
+// One token for one lane's rows of a column: the memory moves on, the column's read-out comes back (in every lane of the column).
 template <int ROWS, bool CHANNEL>
-__device__ __forceinline__ PairSum delta_sums(float (&S)[ROWS], const float (&q)[ROWS], const DeltaItem<ROWS, CHANNEL>& x) {
+__device__ __forceinline__ float delta_token(float (&S)[ROWS], const DeltaToken<ROWS, CHANNEL>& x) {
+    const float decay = x.own.x, step = x.own.y, v = x.own.z, kq = x.own.w;
     float sk = 0.f, sq = 0.f;
 #pragma unroll
     for (int rr = 0; rr < ROWS; ++rr) {
-        sq = fmaf(S[rr], q[rr], sq);
         if constexpr (CHANNEL) S[rr] *= x.d[rr];
-        sk = fmaf(S[rr], x.k[rr], sk);
+        sk = fmaf(S[rr], x.kq[rr].x, sk);
+        sq = fmaf(S[rr], x.kq[rr].y, sq);
     }
-    return pair_sum(sk, sq);
-}
-
-// ... and the token's write.
-template <int ROWS, bool CHANNEL>
-__device__ __forceinline__ void delta_write(float (&S)[ROWS], const DeltaItem<ROWS, CHANNEL>& x, float seen) {
-    const float w = CHANNEL ? x.step * (x.v - seen) : x.step * (x.v - x.decay * seen);
+    sk = group_sum<16>(sk);
+    sq = group_sum<16>(sq);
+    if constexpr (CHANNEL) {
+        const float w = step * (v - sk);
 #pragma unroll
-    for (int rr = 0; rr < ROWS; ++rr) S[rr] = CHANNEL ? fmaf(x.k[rr], w, S[rr]) : fmaf(x.k[rr], w, x.decay * S[rr]);
-}
-
-// The read-out alone (behind the last token).
-template <int ROWS>
-__device__ __forceinline__ float delta_read(const float (&S)[ROWS], const float (&q)[ROWS]) {
-    float sq = 0.f;
-#pragma unroll
-    for (int rr = 0; rr < ROWS; ++rr) sq = fmaf(S[rr], q[rr], sq);
-    return pair_sum(0.f, sq).y;
-}
-
-// A lane's ROWS numbers from row `first` of a key on.  How they lie: anyhow (keys that end within a lane's rows or leave lanes without any
-// read their last row there), four at a time (dk a multiple of 4, every token's numbers at multiples of 16 bytes), and so with rows for every lane.
-enum DeltaRows { ANYHOW, BY_FOUR, EVERY_LANE };
-template <int ROWS, int HOW>
-__device__ __forceinline__ void delta_rows(float (&x)[ROWS], const float* __restrict__ row, int first, int dk) {
-    if constexpr (HOW != ANYHOW && ROWS == 2) {
-        const float2 v = *reinterpret_cast<const float2*>(row + min(first, dk - 2));
-        x[0] = v.x, x[1] = v.y;
-    } else if constexpr (HOW != ANYHOW) {
-#pragma unroll
-        for (int rr = 0; rr < ROWS; rr += 4) {
-            const float4 v = *reinterpret_cast<const float4*>(row + min(first + rr, dk - 4));
-            x[rr] = v.x, x[rr + 1] = v.y, x[rr + 2] = v.z, x[rr + 3] = v.w;
-        }
+        for (int rr = 0; rr < ROWS; ++rr) S[rr] = fmaf(x.kq[rr].x, w, S[rr]);
+        return fmaf(w, kq, sq);
     } else {
+        const float w = step * (v - decay * sk);               // s (v - d M^T k)
 #pragma unroll
-        for (int rr = 0; rr < ROWS; ++rr) x[rr] = row[min(first + rr, dk - 1)];
+        for (int rr = 0; rr < ROWS; ++rr) S[rr] = fmaf(decay, S[rr], x.kq[rr].x * w);
+        return fmaf(decay, sq, w * kq);
     }
 }
 
-// (Rows beyond dk: the memory's are zero and must stay so, whatever the token's numbers read there.)
-template <int ROWS, int HOW>
-__device__ __forceinline__ void delta_cut(float (&x)[ROWS], int first, int dk) {
-    if constexpr (HOW == EVERY_LANE) return;
-#pragma unroll
-    for (int rr = 0; rr < ROWS; ++rr)
-        if (first + rr >= dk) x[rr] = 0.f;
-}
+// A lane keeps a block's keys and queries as they come until they are laid into LDS.
+template <int N>
+struct DeltaBlock {
+    float k[N], q[N], d[N];
+    float v, decay, step;
+};
 
-template <int ROWS, bool CHANNEL, int HOW>
+// EVERY: keys of 16 ROWS channels and every token's numbers at multiples of 16 bytes, so that they come four at a time and nothing is masked.
+template <int ROWS, bool CHANNEL, bool EVERY>
 __global__ __launch_bounds__(64) void delta_scan_kernel(const float* __restrict__ qkv, long ld, const float* __restrict__ gates,
                                                        const int* __restrict__ seg_start, const int* __restrict__ seg_len,
                                                        const int* __restrict__ row_slot, float* __restrict__ state, long state_stride,
                                                        float* __restrict__ out, long ldo, int n_heads, int n_kv, int dk, int dv) {
-    constexpr int C = 4, TB = ROWS <= 2 ? 16 : ROWS <= 4 ? 8 : ROWS <= 8 ? 4 : 2;        // columns a tile of the state; tokens a block, two blocks in registers
-    typedef DeltaItem<ROWS, CHANNEL> item_t;
-    const int seg = blockIdx.x, h = blockIdx.y, vt = blockIdx.z / 2, n_tiles = gridDim.z / 2;
-    const int lane = threadIdx.x, c = (blockIdx.z & 1) * 2 + lane / 32, rg = lane % 32, first = rg * ROWS;
+    constexpr int C = 4, RG = 16, KQ = RG * ROWS;
+    constexpr int TB = (1024 / KQ) < 16 ? (1024 / KQ) : 16;      // tokens staged at a time
+    constexpr int PER = TB * KQ / 64, WIDE = EVERY ? 4 : 1;      // (k, q) pairs a lane brings per block, and at a time
+    static_assert(TB >= 2 && TB * C <= 64, "a block of 2 to 16 tokens; a lane brings one token's numbers of one column");
+    __shared__ __attribute__((aligned(16))) float2 kq_s[2][TB][KQ];
+    __shared__ __attribute__((aligned(16))) float d_s[2][TB][CHANNEL ? KQ : 4];
+    __shared__ float4 own_s[2][TB][C];                           // per token and column {decay, step, v, k . q}
+    const int seg = blockIdx.x, h = blockIdx.y, vt = blockIdx.z, n_tiles = gridDim.z;
+    const int lane = threadIdx.x, c = lane / RG, rg = lane % RG;
     const int n = seg_len[seg];
     if (n <= 0) return;
     const int t0 = seg_start[seg];
     const int col = vt * C + c, kvh = h / (n_heads / n_kv);
     const bool live = col < dv;
     float* st = state + (size_t)row_slot[t0] * state_stride + ((size_t)h * n_tiles + vt) * ((size_t)dk * C);
-    const int q_at = kvh * dk, k_at = (n_kv + kvh) * dk, v_at = 2 * n_kv * dk + h * dv + min(col, dv - 1);
-    const int dn = CHANNEL ? dk : 1;             // decays a head
-    const size_t ldg = (size_t)n_heads * (dn + 1);
+    const int q_at = kvh * dk, k_at = (n_kv + kvh) * dk, v_at = 2 * n_kv * dk + h * dv;
 
     float S[ROWS];
 #pragma unroll
     for (int rr = 0; rr < ROWS; ++rr) {
-        const float s = st[(size_t)min(first + rr, dk - 1) * C + c];
-        S[rr] = first + rr < dk ? s : 0.f;
+        const int i = rr * RG + rg;
+        S[rr] = EVERY || i < dk ? st[(size_t)i * C + c] : 0.f;
     }
-    // The tokens from `at` on (those beyond the request's last are read as its last, and never used): always as many loads, none skipped, so
-    // that the wait for a block's numbers is for that block alone.  The gates, the same for all lanes, come lane by token.
-    struct Gates { float decay, step; };
-    auto fetch = [&](item_t (&x)[TB], Gates& gb, int at) {
-#pragma unroll
-        for (int u = 0; u < TB; ++u) {
-            const size_t t = (size_t)t0 + min(at + u, n - 1);
-            const float *row = qkv + t * ld, *g = gates + t * ldg;
-            delta_rows<ROWS, HOW>(x[u].k, row + k_at, first, dk);
-            delta_rows<ROWS, HOW>(x[u].q, row + q_at, first, dk);
-            if constexpr (CHANNEL) delta_rows<ROWS, HOW>(x[u].d, g + (size_t)h * dk, first, dk);
-            x[u].v = row[v_at];
-        }
-        const float* g = gates + ((size_t)t0 + min(at + lane % TB, n - 1)) * ldg;
-        gb.decay = CHANNEL ? 0.f : g[h];
-        gb.step = g[(size_t)n_heads * dn + h];
-        __builtin_amdgcn_sched_barrier(0);
+    // A block of TB tokens from `first` on (rows beyond the request's last are read as its last: finite, and never used).
+    const int dn = CHANNEL ? dk : 1;             // decays a head
+    const size_t ldg = (size_t)n_heads * (dn + 1);
+    // The numbers stay as they come until they are laid into LDS: a condition or a product here would make the wave wait for each.
+    DeltaBlock<PER> r;
+    const auto four = [](float* to, const void* from) {
+        const float4 x = *reinterpret_cast<const float4*>(from);
+        to[0] = x.x, to[1] = x.y, to[2] = x.z, to[3] = x.w;
     };
-    float q_last[ROWS];                          // the query whose read-out is due with the next token's sums
+    // Keys of up to 256 channels: a lane brings the same channels of several tokens, from one token's row to the next a scalar step.
+    constexpr bool STEPS = EVERY && KQ <= 256;
+    const char* from_row = (const char*)(qkv + (size_t)(t0 + lane * 4 / KQ) * ld + q_at + lane * 4 % KQ);
+    const char* from_gates = (const char*)(gates + (size_t)(t0 + lane * 4 / KQ) * ldg + (size_t)h * dk + lane * 4 % KQ);
+    const size_t row_step = (size_t)ld * (4 * 256 / KQ), gates_step = ldg * (4 * 256 / KQ), to_keys = (size_t)n_kv * dk * 4;
+    auto fetch = [&](int first) {
+        if (STEPS && first + TB <= n) {
+            const size_t row = (size_t)first * ld * 4, row_gates = (size_t)first * ldg * 4;
 #pragma unroll
-    for (int rr = 0; rr < ROWS; ++rr) q_last[rr] = 0.f;
-    auto token = [&](item_t& x, const Gates& gb, int u) {                     // gives the read-out of the token before, in the column's second row
-        delta_cut<ROWS, HOW>(x.k, first, dk);
-        delta_cut<ROWS, HOW>(x.q, first, dk);
-        x.decay = lane_value(gb.decay, u);
-        x.step = lane_value(gb.step, u);
-        const PairSum s = delta_sums<ROWS, CHANNEL>(S, q_last, x);
-        delta_write<ROWS, CHANNEL>(S, x, s.x);
+            for (int e = 0; e < PER; e += WIDE) {
+                four(&r.q[e], from_row + (row + e / 4 * row_step));
+                four(&r.k[e], from_row + (row + e / 4 * row_step + to_keys));
+                if constexpr (CHANNEL) four(&r.d[e], from_gates + (row_gates + e / 4 * gates_step));
+            }
+        } else {
 #pragma unroll
-        for (int rr = 0; rr < ROWS; ++rr) q_last[rr] = x.q[rr];
-        return s.y;
-    };
-    // (a column's second row holds equal results: its lane u keeps the one that token u of the block brought, and a block leaves in one store)
-    auto block = [&](item_t (&x)[TB], const Gates& gb, int at) {
-        float mine = 0.f;
-#pragma unroll
-        for (int u = 0; u < TB; ++u) {
-            const float y = token(x[u], gb, u);
-            mine = rg == 16 + u ? y : mine;
-        }
-        const int t = at + rg - 17;
-        if (rg >= 16 && rg < 16 + TB && t >= 0 && live) out[(size_t)(t0 + t) * ldo + h * dv + col] = mine;
-    };
-    auto part_of_block = [&](item_t (&x)[TB], const Gates& gb, int at, int here) {
-#pragma unroll
-        for (int u = 0; u < TB; ++u) {
-            if (u < here) {
-                const float y = token(x[u], gb, u);
-                if (rg == 16 && at + u > 0 && live) out[(size_t)(t0 + at + u - 1) * ldo + h * dv + col] = y;
+            for (int e = 0; e < PER; e += WIDE) {
+                const int idx = lane * WIDE + 64 * e, u = idx / KQ, i = idx % KQ;
+                const size_t t = t0 + min(first + u, n - 1);
+                const float *row = qkv + t * ld, *decays = gates + t * ldg + h * dk;
+                if constexpr (EVERY) {
+                    four(&r.k[e], row + k_at + i);
+                    four(&r.q[e], row + q_at + i);
+                    if constexpr (CHANNEL) four(&r.d[e], decays + i);
+                } else {
+                    const int ic = min(i, dk - 1);
+                    r.k[e] = row[k_at + ic], r.q[e] = row[q_at + ic];
+                    if constexpr (CHANNEL) r.d[e] = decays[ic];
+                }
             }
         }
+        const size_t t = t0 + min(first + min(lane / C, TB - 1), n - 1);
+        r.v = qkv[t * ld + v_at + min(vt * C + lane % C, dv - 1)];
+        const float* g = gates + t * ldg;
+        r.decay = CHANNEL ? 0.f : g[h], r.step = g[n_heads * dn + h];
     };
-    item_t even[TB], odd[TB];
-    Gates even_gates, odd_gates;
-    fetch(even, even_gates, 0);
-    int at = 0;
-    for (; at + 2 * TB <= n; at += 2 * TB) {
-        fetch(odd, odd_gates, at + TB);
-        block(even, even_gates, at);
-        fetch(even, even_gates, at + 2 * TB);
-        block(odd, odd_gates, at + TB);
-    }
-    fetch(odd, odd_gates, at + TB);
-    part_of_block(even, even_gates, at, n - at);
-    part_of_block(odd, odd_gates, at + TB, n - at - TB);
-    const float y_last = delta_read<ROWS>(S, q_last);
-    if (rg == 16 && live) out[(size_t)(t0 + n - 1) * ldo + h * dv + col] = y_last;
+    auto stash = [&](int buf) {
 #pragma unroll
-    for (int rr = 0; rr < ROWS; ++rr)
-        if (first + rr < dk) st[(size_t)(first + rr) * C + c] = S[rr];
+        for (int e = 0; e < PER; e += WIDE) {
+            const int idx = lane * WIDE + 64 * e, i = idx % KQ;
+            const int u = idx / KQ;
+            if constexpr (EVERY) {
+                float4* to = reinterpret_cast<float4*>(&kq_s[buf][u][i]);
+                to[0] = float4{r.k[e], r.q[e], r.k[e + 1], r.q[e + 1]};
+                to[1] = float4{r.k[e + 2], r.q[e + 2], r.k[e + 3], r.q[e + 3]};
+                if constexpr (CHANNEL) *reinterpret_cast<float4*>(&d_s[buf][u][i]) = float4{r.d[e], r.d[e + 1], r.d[e + 2], r.d[e + 3]};
+            } else {
+                const int keep = i < dk ? -1 : 0;                     // (zeros beyond the key, without a branch)
+                const auto kept = [&](float x) { return __int_as_float(__float_as_int(x) & keep); };
+                kq_s[buf][u][i] = float2{kept(r.k[e]), kept(r.q[e])};
+                if constexpr (CHANNEL) d_s[buf][u][i] = kept(r.d[e]);
+            }
+        }
+        if (lane < TB * C) own_s[buf][lane / C][lane % C] = float4{r.decay, r.step, r.v, 0.f};
+    };
+    // k . q of a block's tokens, a token per column of lanes at a time: nothing of the memory is in it, so it does not stand in the tokens' way.
+    auto key_queries = [&](int buf) {
+#pragma unroll
+        for (int j = 0; j < TB; j += C) {
+            const int u = min(j + c, TB - 1);
+            float2 x[ROWS];
+#pragma unroll
+            for (int rr = 0; rr < ROWS; ++rr) x[rr] = kq_s[buf][u][rr * RG + rg];
+            const float kq = group_sum<16>(delta_key_query<ROWS, CHANNEL>(x));
+            if (rg < C) own_s[buf][u][rg].w = kq;
+        }
+    };
+    fetch(0);
+    stash(0);
+    barrier_lds();
+    int buf = 0;
+    for (int b0 = 0; b0 < n; b0 += TB, buf ^= 1) {
+        const int here = min(TB, n - b0);
+        const bool more = b0 + TB < n;
+        if (more) fetch(b0 + TB);
+        key_queries(buf);
+        barrier_lds();
+        auto read = [&](int u, DeltaToken<ROWS, CHANNEL>& x) {
+#pragma unroll
+            for (int rr = 0; rr < ROWS; ++rr) x.kq[rr] = kq_s[buf][u][rr * RG + rg];
+            if constexpr (CHANNEL) {
+#pragma unroll
+                for (int rr = 0; rr < ROWS; ++rr) x.d[rr] = d_s[buf][u][rr * RG + rg];
+            }
+            x.own = own_s[buf][u][c];
+        };
+        if (ROWS <= 8 && here == TB) {           // a whole block: straight code, a token's numbers leave LDS while the one before is worked on, the results one store
+            float mine = 0.f;                    // (the lanes of a column hold equal results: lane u of it keeps token u's)
+            DeltaToken<ROWS, CHANNEL> x[2];
+            read(0, x[0]);
+#pragma unroll
+            for (int u = 0; u < TB; ++u) {
+                if (u + 1 < TB) read(u + 1, x[(u + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+                const float y = delta_token<ROWS, CHANNEL>(S, x[u & 1]);
+                mine = rg == u ? y : mine;
+            }
+            asm volatile("" : "+v"(mine));       // (else the read-outs' last steps move behind the branch, three instructions a token for one)
+            if (rg < TB && live) out[(size_t)(t0 + b0 + rg) * ldo + h * dv + col] = mine;
+        } else {
+            for (int u = 0; u < here; ++u) {
+                DeltaToken<ROWS, CHANNEL> x;
+                read(u, x);
+                const float y = delta_token<ROWS, CHANNEL>(S, x);
+                if (rg == 0 && live) out[(size_t)(t0 + b0 + u) * ldo + h * dv + col] = y;
+            }
+        }
+        if (more) stash(buf ^ 1);                // (the buffer the block before this one was read from)
+        barrier_lds();
+    }
+#pragma unroll
+    for (int rr = 0; rr < ROWS; ++rr) {
+        const int i = rr * RG + rg;
+        if (EVERY || i < dk) st[(size_t)i * C + c] = S[rr];
+    }
 }
 
 // The same for steps in which every request brings one row: nothing is staged, a wave takes its row's numbers as they lie, and a
 // workgroup is four waves (tiles).  Every sum in the scan's order: the same bits.
-template <int ROWS, bool CHANNEL, int HOW>
+template <int ROWS, bool CHANNEL>
 __global__ __launch_bounds__(256) void delta_single_kernel(const float* __restrict__ qkv, long ld, const float* __restrict__ gates,
                                                           const int* __restrict__ seg_start, const int* __restrict__ seg_len,
                                                           const int* __restrict__ row_slot, float* __restrict__ state, long state_stride,
                                                           float* __restrict__ out, long ldo, int n_heads, int n_kv, int dk, int dv) {
-    constexpr int C = 4;
-    const int half = blockIdx.z * 4 + (threadIdx.x >> 6), seg = blockIdx.x, h = blockIdx.y, vt = half / 2, n_tiles = (dv + C - 1) / C;
-    const int lane = threadIdx.x & 63, c = (half & 1) * 2 + lane / 32, rg = lane % 32, first = rg * ROWS;
+    constexpr int C = 4, RG = 16;
+    const int seg = blockIdx.x, h = blockIdx.y, vt = blockIdx.z * 4 + (threadIdx.x >> 6), n_tiles = (dv + C - 1) / C;
+    const int lane = threadIdx.x & 63, c = lane / RG, rg = lane % RG;
     if (vt >= n_tiles || seg_len[seg] <= 0) return;
     const size_t t = seg_start[seg];
     const int col = vt * C + c, kvh = h / (n_heads / n_kv), dn = CHANNEL ? dk : 1;
@@ -562,25 +600,24 @@ __global__ __launch_bounds__(256) void delta_single_kernel(const float* __restri
     const float* row = qkv + t * ld;
     const float* g = gates + t * n_heads * (dn + 1);
     float S[ROWS];
-    DeltaItem<ROWS, CHANNEL> x;
+    DeltaToken<ROWS, CHANNEL> x;
 #pragma unroll
     for (int rr = 0; rr < ROWS; ++rr) {
-        const float s = st[(size_t)min(first + rr, dk - 1) * C + c];
-        S[rr] = first + rr < dk ? s : 0.f;
+        const int i = rr * RG + rg, ic = min(i, dk - 1);
+        const float s = st[(size_t)ic * C + c], k = row[(n_kv + kvh) * dk + ic], q = row[kvh * dk + ic], d = CHANNEL ? g[h * dk + ic] : 0.f;
+        S[rr] = i < dk ? s : 0.f;
+        x.kq[rr] = i < dk ? float2{k, q} : float2{0.f, 0.f};
+        if constexpr (CHANNEL) x.d[rr] = i < dk ? d : 0.f;
     }
-    delta_rows<ROWS, HOW>(x.k, row + (size_t)(n_kv + kvh) * dk, first, dk);
-    delta_rows<ROWS, HOW>(x.q, row + (size_t)kvh * dk, first, dk);
-    if constexpr (CHANNEL) delta_rows<ROWS, HOW>(x.d, g + (size_t)h * dk, first, dk);
-    x.v = row[2 * n_kv * dk + h * dv + min(col, dv - 1)], x.decay = CHANNEL ? 0.f : g[h], x.step = g[(size_t)n_heads * dn + h];
-    delta_cut<ROWS, HOW>(x.k, first, dk);
-    delta_cut<ROWS, HOW>(x.q, first, dk);
-    float q_before[ROWS] = {};
-    delta_write<ROWS, CHANNEL>(S, x, delta_sums<ROWS, CHANNEL>(S, q_before, x).x);
-    const float y = delta_read<ROWS>(S, x.q);
-    if (rg == 16 && col < dv) out[t * ldo + h * dv + col] = y;
+    const float v = row[2 * n_kv * dk + h * dv + min(col, dv - 1)];
+    x.own = float4{CHANNEL ? 0.f : g[h], g[n_heads * dn + h], v, group_sum<16>(delta_key_query<ROWS, CHANNEL>(x.kq))};
+    const float y = delta_token<ROWS, CHANNEL>(S, x);
+    if (rg == 0 && col < dv) out[t * ldo + h * dv + col] = y;
 #pragma unroll
-    for (int rr = 0; rr < ROWS; ++rr)
-        if (first + rr < dk) st[(size_t)(first + rr) * C + c] = S[rr];
+    for (int rr = 0; rr < ROWS; ++rr) {
+        const int i = rr * RG + rg;
+        if (i < dk) st[(size_t)i * C + c] = S[rr];
+    }
 }
 
 }  // namespace
@@ -670,23 +707,18 @@ GI_API int gi_delta_scan(const float* qkv, long ld, const float* gates, const in
                n_segs, n_heads, n_kv, dk, dv);
     GI_REQUIRE(ld >= 2L * n_kv * dk + (long)n_heads * dv && ldo >= (long)n_heads * dv && state_stride >= gi_delta_memory_floats(n_heads, dk, dv), "delta_scan: row or state strides too small");
     const int tiles = (dv + 3) / 4;
-    GI_REQUIRE(n_heads <= 65535 && tiles <= 32767, "delta_scan: too many heads or value channels");
-    dim3 grid(n_segs, n_heads, 2 * tiles);
+    GI_REQUIRE(n_heads <= 65535 && tiles <= 65535, "delta_scan: too many heads or value channels");
+    dim3 grid(n_segs, n_heads, tiles);
 #define ARGS qkv, ld, gates, seg_start, seg_len, row_slot, state, state_stride, out, ldo, n_heads, n_kv, dk, dv
-    // two or four rows of a key at a time where every token's numbers start at multiples of 16 bytes
-    const bool vector = dk % 4 == 0 && ld % 4 == 0 && ((uintptr_t)qkv & 15) == 0 && (!channel || (((long)n_heads * (dk + 1)) % 4 == 0 && ((uintptr_t)gates & 15) == 0));
-#define KIND(R, CH, HOW)                                                                                                            \
-    do {                                                                                                                            \
-        if (single) delta_single_kernel<R, CH, HOW><<<dim3(n_segs, n_heads, (2 * tiles + 3) / 4), 256, 0, stream>>>(ARGS);              \
-        else delta_scan_kernel<R, CH, HOW><<<grid, 64, 0, stream>>>(ARGS);                                                          \
+    const bool aligned = ld % 4 == 0 && ((uintptr_t)qkv & 15) == 0 && (!channel || (((long)n_heads * (dk + 1)) % 4 == 0 && ((uintptr_t)gates & 15) == 0));
+#define KIND(R, CH)                                                                                                             \
+    do {                                                                                                                        \
+        if (single) delta_single_kernel<R, CH><<<dim3(n_segs, n_heads, (tiles + 3) / 4), 256, 0, stream>>>(ARGS);               \
+        else if (aligned && dk == 16 * R) delta_scan_kernel<R, CH, true><<<grid, 64, 0, stream>>>(ARGS);                        \
+        else delta_scan_kernel<R, CH, false><<<grid, 64, 0, stream>>>(ARGS);                                                    \
     } while (0)
-#define GO(R)                                                                                                                       \
-    do {                                                                                                                            \
-        constexpr int FOUR = R >= 2 ? BY_FOUR : ANYHOW, EVERY = R >= 2 ? EVERY_LANE : ANYHOW;                                       \
-        if (channel) { if (vector && dk == 32 * R) KIND(R, true, EVERY); else if (vector) KIND(R, true, FOUR); else KIND(R, true, ANYHOW); } \
-        else { if (vector && dk == 32 * R) KIND(R, false, EVERY); else if (vector) KIND(R, false, FOUR); else KIND(R, false, ANYHOW); } \
-    } while (0)
-    if (dk <= 32) GO(1); else if (dk <= 64) GO(2); else if (dk <= 128) GO(4); else if (dk <= 256) GO(8); else GO(16);
+#define GO(R) do { if (channel) KIND(R, true); else KIND(R, false); } while (0)
+    if (dk <= 32) GO(2); else if (dk <= 64) GO(4); else if (dk <= 128) GO(8); else if (dk <= 256) GO(16); else GO(32);
 #undef GO
 #undef KIND
 #undef ARGS

@@ -4,6 +4,7 @@ scheduler.  In float32 the engine's logits must not depend on the cutting at all
 to the exact model as rounding alone explains."""
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -182,6 +183,95 @@ def test_gated_delta_rule_kernels(heads, kv, dk, dv, taps):
     both = run(torch.cat([more[:4], more[4:]]), [4, 7], [1, 3], [lens[0], lens[1]])
     alone = torch.cat([run(more[:4], [4], [2], [lens[0]]), run(more[4:], [7], [4], [lens[1]])])
     assert torch.equal(both, alone)
+
+
+def _rule_in_its_order(qkv, gates, M, heads, kv, dk, dv, channel):
+    """The rule over one run of rows in 32 bits, every sum in the kernel's order: of a key's rows those 16 apart are one chain of fused
+    multiply-adds, the 16 chains meet as a tree (place i and its mirror image, in 16, then in 8, then two apart, then neighbours).
+    M [heads, dk, dv] is moved on; the read-outs come back.  A fused multiply-add: 64 bits of mantissa, rounded once to 32-bit."""
+    f = np.float32
+    fma = lambda a, b, c: (a.astype(np.longdouble) * b.astype(np.longdouble) + np.asarray(c).astype(np.longdouble)).astype(f)
+
+    def chains(x, y, rounded=False):                                      # [..., dk, columns] -> [..., columns]
+        rows = -(-dk // 16)
+        acc = np.zeros(x.shape[:-2] + (16, x.shape[-1]), f)
+        for r in range(rows):
+            n = min(16, dk - 16 * r)
+            a, b = x[..., 16 * r:16 * r + n, :], y[..., 16 * r:16 * r + n, :]
+            acc[..., :n, :] = acc[..., :n, :] + a * b if rounded else fma(a, b, acc[..., :n, :])
+        i = np.arange(16)
+        for other in (15 - i, i ^ 7, i ^ 2, i ^ 1):
+            acc = acc + acc[..., other, :]
+        return acc[..., 0, :]
+
+    n, per = qkv.shape[0], heads // kv
+    q, k = (np.repeat(qkv[:, at:at + kv * dk].reshape(n, kv, dk), per, 1)[..., None] for at in (0, kv * dk))
+    v = qkv[:, 2 * kv * dk:2 * kv * dk + heads * dv].reshape(n, heads, dv)
+    decay, step = gates[:, :-heads].reshape(n, heads, -1, 1), gates[:, -heads:, None]
+    out = np.empty((n, heads, dv), f)
+    for t in range(n):
+        kt, qt = np.broadcast_to(k[t], M.shape), np.broadcast_to(q[t], M.shape)
+        kq = chains(k[t], q[t], rounded=channel)
+        if channel:
+            M[:] = M * decay[t]
+            sk, sq = chains(M, kt), chains(M, qt)
+            w = step[t] * (v[t] - sk)
+            M[:] = fma(kt, w[:, None], M)
+            out[t] = fma(w, np.broadcast_to(kq, w.shape), sq)
+        else:
+            sk, sq, d = chains(M, kt), chains(M, qt), np.broadcast_to(decay[t][:, 0], v[t].shape)
+            w = step[t] * fma(-d, sk, v[t])
+            M[:] = fma(np.broadcast_to(decay[t], M.shape), M, kt * w[:, None])
+            out[t] = fma(d, sq, w * kq)
+    return out.reshape(n, -1)
+
+
+@pytest.mark.parametrize("channel", [False, True])
+@pytest.mark.parametrize("heads, kv, dk, dv, spare", [(2, 1, 64, 9, 3), (2, 2, 64, 8, 1), (2, 1, 32, 4, 0), (1, 1, 128, 6, 2), (1, 1, 100, 5, 3), (2, 2, 256, 4, 0), (1, 1, 512, 3, 1), (1, 1, 300, 3, 0)])
+def test_delta_rule_sums_in_one_order(heads, kv, dk, dv, spare, channel):
+    """The rule's results in bits: whole keys that are loaded four channels at a time (32, 64, 128, 256, 512 at aligned rows) and others, whole
+    blocks of tokens and their ends, one row alone."""
+    from geneinfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(dk)
+    width = 2 * kv * dk + heads * dv
+    lens = [21, 1, 34]
+    n = sum(lens)
+    wide = torch.randn(n, width + spare, generator=g)
+    unit = wide[:, :2 * kv * dk].view(n, 2 * kv, dk)
+    unit /= unit.norm(dim=2, keepdim=True)
+    gates = torch.cat([torch.exp(-0.5 * torch.rand(n, heads * (dk if channel else 1), generator=g)), torch.rand(n, heads, generator=g)], 1)
+    start = torch.tensor([0, 21, 22], dtype=torch.int32, device=DEV)
+    length = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    slot = torch.tensor([2] * 21 + [0] + [1] * 34, dtype=torch.int32, device=DEV)
+    tiles = -(-dv // 4)
+    first = torch.randn(3, heads, tiles, dk, 4, generator=g)
+    state, out = first.clone().view(3, -1).to(DEV), torch.full((n, heads * dv), 7.0, device=DEV)
+    ops.delta_scan(wide.to(DEV), gates.to(DEV), start, length, slot, state, out, heads, kv, dk, dv, channel=channel)
+    one_state, one = first.clone().view(3, -1).to(DEV), torch.full((1, heads * dv), 7.0, device=DEV)
+    ops.delta_scan(wide[21:22].to(DEV), gates[21:22].to(DEV), start[:1], length[1:2], slot[21:22], one_state, one, heads, kv, dk, dv, channel=channel, single_rows=True)
+    at = 0
+    for m, s in zip(lens, (2, 0, 1)):
+        M = first[s].permute(0, 2, 1, 3).reshape(heads, dk, 4 * tiles)[:, :, :dv].numpy().copy()
+        want = _rule_in_its_order(wide[at:at + m, :width].numpy(), gates[at:at + m].numpy(), M, heads, kv, dk, dv, channel)
+        assert torch.equal(out[at:at + m].cpu(), torch.from_numpy(want))
+        held = state[s].view(heads, tiles, dk, 4).permute(0, 2, 1, 3).reshape(heads, dk, 4 * tiles)[:, :, :dv].cpu()
+        assert torch.equal(held, torch.from_numpy(M))
+        at += m
+    assert torch.equal(one, out[21:22]) and torch.equal(one_state[0], state[0])
+
+
+def test_delta_rule_takes_very_wide_values():
+    """More tiles of four value channels than half of what a launch's third dimension holds."""
+    from geneinfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(4)
+    n, dk, dv = 3, 8, 4 * 32768 + 3
+    qkv = torch.randn(n, 2 * dk + dv, generator=g)
+    gates = torch.rand(n, 2, generator=g)
+    ints = lambda *x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    state, out = torch.zeros(1, ops.delta_memory_floats(1, dk, dv), device=DEV), torch.empty(n, dv, device=DEV)
+    ops.delta_scan(qkv.to(DEV), gates.to(DEV), ints(0), ints(n), ints(0, 0, 0), state, out, 1, 1, dk, dv)
+    x = qkv.double()
+    assert relative_error(out, P.delta_rule(x[:, :dk], x[:, dk:2 * dk], x[:, 2 * dk:], gates[:, 1].double(), gates[:, 0].double())) < 1e-5
 
 
 def test_head_norm_with_shared_weights_and_a_silu_gate():
