@@ -67,22 +67,6 @@ __device__ __forceinline__ float gated_act(float g, float u, int act, float limi
 // (quadratic on the right, bounded below on the left, slope 1/2 on both sides of 0).
 __device__ __forceinline__ float softplus_f32(float z) { return z > 20.f ? z : log1pf(expf(z)); }
 __device__ __forceinline__ float xielu(float z, float a, float b) { return z > 0.f ? fmaf(a * z, z, 0.5f * z) : fmaf(b, expm1f(z) - z, 0.5f * z); }
-// The same where a tile of sums is activated at once, as bfloat16: exp(z) - 1 - z by its Taylor series to z^10 from -1 on (the rest is below
-// 2.6e-8), further left, where nothing cancels, by the hardware's exp2.  About half of expm1f's instructions; over normal rows of a spread
-// of 0.1 to 3 its error against 64 bits was 0.3 to 1.7e-7 of the rows before the rounding (with expm1f 0.8 to 1.8e-7), after it the same.
-__device__ __forceinline__ float xielu_fast(float z, float a, float b) {
-    float s = 2.7557319e-7f;
-    s = fmaf(s, z, 2.7557319e-6f);
-    s = fmaf(s, z, 2.4801587e-5f);
-    s = fmaf(s, z, 1.9841270e-4f);
-    s = fmaf(s, z, 1.3888889e-3f);
-    s = fmaf(s, z, 8.3333333e-3f);
-    s = fmaf(s, z, 4.1666667e-2f);
-    s = fmaf(s, z, 1.6666667e-1f);
-    s = fmaf(s, z, 0.5f);
-    const float below = z > -1.f ? z * z * s : __builtin_amdgcn_exp2f(z * 1.4426950408889634f) - 1.0f - z;
-    return z > 0.f ? fmaf(a * z, z, 0.5f * z) : fmaf(b, below, 0.5f * z);
-}
 
 // A workgroup barrier that waits for this wave's LDS traffic only.  __syncthreads() also waits for every load
 // from global memory the wave has in flight, which undoes a prefetch into registers; use this one where the

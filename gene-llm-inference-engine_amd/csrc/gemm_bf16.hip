@@ -549,7 +549,7 @@ __device__ __forceinline__ void piped_tile(const bf16_t* __restrict__ A, const b
                         ((bf16_t*)C)[(size_t)m * ldc + (n >> 5) * 16 + (lane & 15)] = f32_to_bf16(gate_of<EPI>(acc[i][j][v], up, norm_in.limit));
                 } else if constexpr (EPI != EPI_QKV_ROPE) {
                     float sum = acc[i][j][v];
-                    if constexpr (EPI == EPI_XIELU) sum = xielu_fast(sum, act_a, act_b);
+                    if constexpr (EPI == EPI_XIELU) sum = xielu(sum, act_a, act_b);
                     if (m < M && n < N) write_out<EPI>(C, (size_t)m * ldc + n, sum);
                 }
             }
@@ -809,7 +809,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) acc[i][j][v] = xielu_fast(acc[i][j][v], act_a, act_b);
+                    for (int v = 0; v < 16; ++v) acc[i][j][v] = xielu(acc[i][j][v], act_a, act_b);
         }
 #pragma unroll
         for (int part = 0; part < TN / 2; ++part) {                                // 64 columns = 128 bytes a row at a time
@@ -1074,7 +1074,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
                 const int row = (tid >> 5) + it * 16, m = first + row;
                 if (m >= M) continue;
                 float4 v = *reinterpret_cast<const float4*>(tile + row * 128 + (tid & 31) * 4);
-                if constexpr (EPI == EPI_XIELU) v = float4{xielu_fast(v.x, act_a, act_b), xielu_fast(v.y, act_a, act_b), xielu_fast(v.z, act_a, act_b), xielu_fast(v.w, act_a, act_b)};
+                if constexpr (EPI == EPI_XIELU) v = float4{xielu(v.x, act_a, act_b), xielu(v.y, act_a, act_b), xielu(v.z, act_a, act_b), xielu(v.w, act_a, act_b)};
                 const size_t at = (size_t)m * ldc + c;
                 if (whole) {
                     if constexpr (ELEM == 2) {

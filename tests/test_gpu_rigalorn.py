@@ -100,8 +100,7 @@ def test_activation_of_the_plain_feed_forward():
 @pytest.mark.parametrize("rows, n, k, first", [(1, 416, 128, 320), (16, 320, 136, 3), (9, 1100, 2048, 0), (300, 8192, 256, 0), (131, 16400, 192, 0), (700, 8192, 512, 0), (1777, 8200, 320, 0),
                                                (2048, 6000, 1024, 0)])
 def test_product_with_the_activation_of_the_plain_feed_forward(rows, n, k, first):
-    """Against the product and the activation one after the other: the sums are the same, the activation's own error is below 2^-20 of the
-    numbers it is made of (measured 2e-7 against 64 bits), so the results are the same up to one rounding to bfloat16."""
+    """Against the product and the activation one after the other: the same sums and the same activation, so the same bits."""
     from geneinfer_amd.kernels import ops
     assert ops.gemm_bf16_xielu_takes(rows, n, k, first)
     g = torch.Generator(device=DEV).manual_seed(rows + n)
@@ -122,11 +121,9 @@ def test_product_with_the_activation_of_the_plain_feed_forward(rows, n, k, first
     assert (mid[rows] == 7).all() and (mid[:, n - first:] == 7).all()
     if first:
         assert torch.equal(out[:, :first].nan_to_num(nan=9.0), both[:, :first].nan_to_num(nan=9.0)) and (out[:, first:] == 7).all()
-    got, want, z = mid[:rows, :n - first].float(), want.float(), both[:, first:]
-    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
-    fine = want.isfinite()
-    assert ((got - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -20 * z.abs())[fine].all()
-    assert ((got != want) & fine).float().mean() < 1e-3
+    got, want = mid[:rows, :n - first].float(), want.float()
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.nan_to_num(nan=9.0), want.nan_to_num(nan=9.0))
 
 
 @pytest.mark.parametrize("heads, kv, dk, dv, taps", [(4, 2, 16, 24, 4), (3, 3, 64, 64, 2), (2, 1, 130, 10, 5), (1, 1, 7, 201, 1), (5, 5, 3, 5, 3), (2, 2, 300, 6, 8), (1, 1, 20, 9, 13)])
