@@ -83,7 +83,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
                                                                    const int* __restrict__ pos, const int* __restrict__ slot, const int* __restrict__ table,
                                                                    int table_stride, long page_stride, int page_size, int n_rows, int n_heads, int n_kv, int hd, int vd,
                                                                    int window, int chunk, float scale, float cap, const float* __restrict__ sinks,
-                                                                   const float* __restrict__ gate, long gate_stride, int gate_channels, int rows_a_tile,
+                                                                   const float* __restrict__ gate, long gate_stride, int gate_channels, int n_single, int rows_a_tile,
                                                                    float* __restrict__ part, int n_spans) {
     __shared__ float o_s[4][PAIRS][D + 4];
     __shared__ float m_s[4][PAIRS], l_s[4][PAIRS], f_s[4][PAIRS];        // of the blocks; f: their factors, negative where the pair sees none of the block's keys
@@ -95,8 +95,9 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
     const int group = n_heads / n_kv, head_tiles = (group + PAIRS - 1) / PAIRS;
     const int tile = blockIdx.x / (n_kv * head_tiles), kv = blockIdx.x / head_tiles % n_kv, ht = blockIdx.x % head_tiles;
     const int heads_here = min(PAIRS, group - ht * PAIRS);
-    const int place = r / heads_here, t = tile * rows_a_tile + place, h = kv * group + ht * PAIRS + r % heads_here;
-    const bool valid = place < rows_a_tile && t < n_rows;
+    const int rows_here = tile < n_single ? 1 : rows_a_tile, t_first = tile < n_single ? tile : n_single + (tile - n_single) * rows_a_tile;
+    const int place = r / heads_here, t = t_first + place, h = kv * group + ht * PAIRS + r % heads_here;
+    const bool valid = place < rows_here && t < n_rows;
     const int my_pos = valid ? pos[t] : 0, my_slot = valid ? slot[t] : -1, my_lo = valid ? first_key(my_pos, window, chunk) : 0;
     f32x4 qv[D / 16];
 #pragma unroll
@@ -104,12 +105,16 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
         qv[c] = valid && c * 16 < hd ? *reinterpret_cast<const f32x4*>(q + ((size_t)t * n_heads + h) * hd + c * 16 + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
     const long v_plane = (long)n_kv * page_size * hd;   // from a page's keys to its values
 
-    // Rows of one request at a time (a tile at the edge of two requests' rows takes as many turns).
+    // Rows of one request at a time: a tile with rows of several requests takes as many turns, shared out over gridDim.z workgroups.  (One after the
+    // other, with single rows in such tiles too, they took 237 us where a wave per (row, head) takes 39: 16 requests of one row at 100 positions and a
+    // prompt of 48 rows, 16 heads of 128 with keys of their own; 37 now.)
     bool todo = valid;
+    unsigned turn = 0;
     while (__ballot(todo) != 0) {
         const int run_slot = __shfl(my_slot, (int)__ffsll((unsigned long long)__ballot(todo)) - 1, 64);
         const bool in_run = todo && my_slot == run_slot;
         todo = todo && !in_run;
+        if (turn++ % gridDim.z != blockIdx.z) continue;
         int lo_min = in_run ? my_lo : 2147483647, lo_max = in_run ? my_lo : 0, p_min = in_run ? my_pos : 2147483647, p_max = in_run ? my_pos : 0;
 #pragma unroll
         for (int off = 1; off < PAIRS; off <<= 1) {
@@ -209,7 +214,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
                         for (int j = 0; j < 4; ++j) o[c] = mfma(vv[kt][c][j], sc[kt][j], o[c]);
                 }
                 if (__ballot(odd) != 0) {
-                    for (int row = 0; row < rows_a_tile; ++row) {
+                    for (int row = 0; row < rows_here; ++row) {
                         const int row_pos = __shfl(my_pos, row * heads_here, 64), row_lo = __shfl(my_lo, row * heads_here, 64);
 #pragma unroll
                         for (int c = 0; c < D / 16; ++c) {
@@ -238,7 +243,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
                 double sum = 0.0;
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
-                    const bool sees = run_s[tid] && s * SPAN + b * BLOCK <= pos_s[tid] && s * SPAN + (b + 1) * BLOCK > lo_s[tid];
+                    const bool sees = in_run && s * SPAN + b * BLOCK <= my_pos && s * SPAN + (b + 1) * BLOCK > my_lo;      // (lane `tid` has pair `tid`)
                     const float f = m_s[b][tid] == -INFINITY ? 0.f : expf(m_s[b][tid] - top);
                     f_s[b][tid] = sees ? f : -1.f;
                     if (sees) sum = fma((double)l_s[b][tid], (double)f, sum);
@@ -253,7 +258,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
                 } else {
                     float m_now = m_all[tid];
                     double l_now = l_all[tid];
-                    join_s[tid] = join(m_now, l_now, run_s[tid] && s * SPAN <= pos_s[tid] && (s + 1) * SPAN > lo_s[tid], top, sum);
+                    join_s[tid] = join(m_now, l_now, in_run && s * SPAN <= my_pos && (s + 1) * SPAN > my_lo, top, sum);
                     m_all[tid] = m_now;
                     l_all[tid] = l_now;
                 }
@@ -383,12 +388,18 @@ GI_API int gi_attention_exact_max_head_size() { return MAX_HD; }
 // Whether the kernel with tiles serves these sizes (all operands 32-bit and aligned).
 static bool takes_tiles(int hd, int vd, int page_size) { return hd % 16 == 0 && vd % 16 == 0 && hd <= 128 && vd <= 128 && page_size % 4 == 0; }
 
+// Rows of a tile: what its 16 pairs have room for.  The first `n_single` rows of a step, its requests' only ones (decoded rows), have tiles of their own.
+static int rows_a_tile(int group) { return group < PAIRS ? PAIRS / group : 1; }
+static long count_tiles(int n_rows, int n_single, int n_kv, int group) {
+    const int a_tile = rows_a_tile(group);
+    return (long)(n_single + (n_rows - n_single + a_tile - 1) / a_tile) * n_kv * ((group + PAIRS - 1) / PAIRS);
+}
+
 // How many spans of 256 keys the widest row of a step has at most, 0 where they are not shared out: `seen` positions at most are seen by a row.
 // They are shared out while the tiles alone give fewer than two workgroups a compute unit, and the parts stay under 64 MB.
-GI_API int gi_attention_exact_spans(int n_rows, int single_rows, int n_heads, int n_kv, int hd, int vd, int page_size, int seen) {
-    if (n_rows <= 0 || n_kv <= 0 || n_heads % n_kv != 0 || seen <= SPAN || !takes_tiles(hd, vd, page_size)) return 0;
-    const int group = n_heads / n_kv, a_tile = single_rows ? 1 : group < PAIRS ? PAIRS / group : 1;
-    const long tiles = (long)((n_rows + a_tile - 1) / a_tile) * n_kv * ((group + PAIRS - 1) / PAIRS);
+GI_API int gi_attention_exact_spans(int n_rows, int n_single, int n_heads, int n_kv, int hd, int vd, int page_size, int seen) {
+    if (n_rows <= 0 || n_single < 0 || n_single > n_rows || n_kv <= 0 || n_heads % n_kv != 0 || seen <= SPAN || !takes_tiles(hd, vd, page_size)) return 0;
+    const long tiles = count_tiles(n_rows, n_single, n_kv, n_heads / n_kv);
     const long spans = ((long)seen + SPAN - 1) / SPAN + 1;
     if (tiles >= 2L * gi_compute_units() || spans * n_rows * n_heads * part_floats(vd) > (16L << 20)) return 0;
     return (int)spans;
@@ -398,7 +409,7 @@ GI_API long gi_attention_exact_part_floats(int n_rows, int n_heads, int vd, int 
 GI_API int gi_attention_exact(const void* q, int q_dtype, const void* cache, int cache_dtype, void* out, int out_dtype, const int* pos,
                               const int* slot, const int* table, int table_stride, long page_stride, int page_size, int n_rows,
                               int n_heads, int n_kv, int hd, int vd, int window, int chunk, float scale, float cap, const float* sinks, const float* gate,
-                              long gate_stride, int gate_channels, int single_rows, float* part, long part_size, int n_spans, hipStream_t stream) {
+                              long gate_stride, int gate_channels, int n_single, int n_requests, float* part, long part_size, int n_spans, hipStream_t stream) {
     GI_REQUIRE(n_rows > 0 && n_heads > 0 && n_kv > 0 && n_heads % n_kv == 0, "attention_exact: bad head counts (%d rows, %d heads, %d kv heads)",
                n_rows, n_heads, n_kv);
     GI_REQUIRE(hd > 0 && hd <= MAX_HD, "attention_exact: head size %d is outside 1..%d", hd, MAX_HD);
@@ -410,17 +421,18 @@ GI_API int gi_attention_exact(const void* q, int q_dtype, const void* cache, int
     const unsigned grid = (unsigned)(n_rows * n_heads);
     const auto aligned = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
     if (q_dtype == GI_F32 && cache_dtype == GI_F32 && out_dtype == GI_F32 && takes_tiles(hd, vd, page_size) && page_stride % 4 == 0 && aligned(q) && aligned(cache)) {
-        const int group = n_heads / n_kv, a_tile = single_rows ? 1 : group < PAIRS ? PAIRS / group : 1;      // (a lone new row a request: a tile of several would take a turn for each)
+        GI_REQUIRE(n_single >= 0 && n_single <= n_rows, "attention_exact: %d single rows of %d", n_single, n_rows);
+        const int a_tile = rows_a_tile(n_heads / n_kv), turns = n_single == n_rows ? 1 : n_requests > 0 && n_requests < a_tile ? n_requests : a_tile;
         if (n_spans > 0) {
             GI_REQUIRE(part != nullptr && aligned(part) && part_size >= gi_attention_exact_part_floats(n_rows, n_heads, vd, n_spans) && n_spans <= 65535,
                        "attention_exact: sharing the keys out needs %ld floats", gi_attention_exact_part_floats(n_rows, n_heads, vd, n_spans));
         } else {
             part = nullptr;
         }
-        const dim3 tiles((unsigned)((n_rows + a_tile - 1) / a_tile) * n_kv * ((group + PAIRS - 1) / PAIRS), part ? n_spans : 1);
+        const dim3 tiles((unsigned)count_tiles(n_rows, n_single, n_kv, n_heads / n_kv), part ? n_spans : 1, turns);
 #define TILES(D)                                                                                                                           \
     attention_exact_tiles_kernel<D><<<tiles, 256, 0, stream>>>((const float*)q, (const float*)cache, (float*)out, pos, slot, table, table_stride, page_stride, page_size, n_rows, \
-                                                               n_heads, n_kv, hd, vd, window, chunk, scale, cap, sinks, gate, gate_stride, gate_channels, a_tile, part, n_spans)
+                                                               n_heads, n_kv, hd, vd, window, chunk, scale, cap, sinks, gate, gate_stride, gate_channels, n_single, a_tile, part, n_spans)
         if (hd <= 64 && vd <= 64) TILES(64);
         else TILES(128);
 #undef TILES

@@ -35,7 +35,7 @@ _SIGNATURES = {
     "gi_softcap_rows": [c_void_p, c_int, c_int, c_long, c_float, c_void_p],
     "gi_gemm_exact": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long, c_void_p],
     "gi_attention_exact": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_long, c_int,
-                           c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_void_p, c_long, c_int, c_int, c_void_p, c_long, c_int, c_void_p],
+                           c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_void_p, c_long, c_int, c_void_p],
     "gi_rmsnorm_add": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_float, c_long, c_long, c_void_p],
     "gi_rmsnorm_add_norm": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_float, c_long, c_long, c_long, c_void_p],
     "gi_norm_rope_store": [c_void_p, c_void_p, c_void_p, c_long, c_long, c_long, c_void_p, c_void_p, c_int, c_float, c_void_p, c_void_p, c_int,
@@ -565,14 +565,15 @@ def _check_paged(cache, table, what):
 
 
 def attention_exact(q, cache, out, positions, slots, table, n_heads, n_kv, hd, window=None, scale=None, *, page_size=None, value_dim=None,
-                    chunk=None, sinks=None, gate=None, cap=None, channel_gate=None, single_rows=False, max_context=None):
+                    chunk=None, sinks=None, gate=None, cap=None, channel_gate=None, single_rows=False, max_context=None, n_requests=None):
     """Each row attends over its request's cached keys up to its own position, no further back than `window` positions and not
     beyond the start of its own chunk of `chunk` positions.  value_dim: channels of a value head (hd if not given); sinks:
     float32 [heads], a score per head that joins the softmax's denominator only; gate: float32 [n, >= heads] (unit inner
     stride), head h's output is multiplied by sigmoid(gate[t, h]); channel_gate: float32 [n, heads*value_dim], the output is
     multiplied by its sigmoid element by element; cap: a scaled score s becomes cap * tanh(s / cap).  What the caller knows of the
-    step and the results do not depend on: single_rows (every row is its request's only one), max_context (no row lies beyond that
-    many positions; without it no row's keys are shared out over workgroups)."""
+    step and the results do not depend on: single_rows (every row is its request's only one; a number: the first so many are), max_context
+    (no row lies beyond that many positions; without it no row's keys are shared out over workgroups), n_requests (so many requests
+    have the rows behind those)."""
     _dev(q, cache, out, positions, slots, table, sinks, gate, channel_gate)
     if cap is not None and not cap > 0:
         raise KernelError("attention: the scores' cap must be positive")
@@ -590,23 +591,24 @@ def attention_exact(q, cache, out, positions, slots, table, n_heads, n_kv, hd, w
     gate, gate_stride, gate_channels = _gates(gate, channel_gate, n, n_heads, vd)
     _i32(positions, "attention: positions", n)
     _i32(slots, "attention: slots", n)
+    n_single = n if single_rows is True else min(int(single_rows), n)
     part, n_part, n_spans = None, 0, 0
     if max_context is not None and q.dtype == torch.float32:
         seen = min([int(max_context)] + ([int(window)] if window else []) + ([int(chunk)] if chunk else []))
-        n_spans = _exact_spans(n, 1 if single_rows else 0, n_heads, n_kv, hd, vd, page_size, -(-seen // 256) * 256)
+        n_spans = _exact_spans(n, n_single, n_heads, n_kv, hd, vd, page_size, -(-seen // 256) * 256)
         if n_spans:
             n_part = lib().gi_attention_exact_part_floats(n, n_heads, vd, n_spans)
             part = torch.empty(n_part, dtype=torch.float32, device=out.device)
     _call("gi_attention_exact", q.data_ptr(), _code(q, "attention: q"), cache.data_ptr(), _code(cache, "attention: cache"), out.data_ptr(),
           _code(out, "attention: out"), positions.data_ptr(), slots.data_ptr(), table.data_ptr(), table.stride(0), cache.stride(0),
           page_size, n, n_heads, n_kv, hd, vd, int(window or 0), int(chunk or 0), float(scale if scale is not None else hd ** -0.5),
-          float(cap or 0.0), _ptr(sinks), _ptr(gate), gate_stride, gate_channels, 1 if single_rows else 0, _ptr(part), n_part, n_spans, _stream())
+          float(cap or 0.0), _ptr(sinks), _ptr(gate), gate_stride, gate_channels, n_single, int(n_requests or 0), _ptr(part), n_part, n_spans, _stream())
     return out
 
 
 @lru_cache(maxsize=1024)
-def _exact_spans(n, single_rows, n_heads, n_kv, hd, vd, page_size, seen) -> int:
-    return lib().gi_attention_exact_spans(n, single_rows, n_heads, n_kv, hd, vd, page_size, seen)
+def _exact_spans(n, n_single, n_heads, n_kv, hd, vd, page_size, seen) -> int:
+    return lib().gi_attention_exact_spans(n, n_single, n_heads, n_kv, hd, vd, page_size, seen)
 
 
 def _gates(gate, channel_gate, n, n_heads, vd):
@@ -1366,8 +1368,13 @@ def attention(q, cache, out, ctx, table, n_heads, n_kv, hd, window=None):
         plan = _plan_of(ctx)
         if (not plan.n_tiles or attention_bf16_supports(hd, page_size, True)) and (not plan.n_decode or attention_bf16_supports(hd, page_size, False)):
             return attention_bf16(q, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window)
-    return attention_exact(q, cache, out, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, single_rows=ctx.max_seg_len == 1,
-                           max_context=_longest_context(ctx))
+    return attention_exact(q, cache, out, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, **_known_of(ctx))
+
+
+def _known_of(ctx) -> dict:
+    """What `attention_exact` may know of a step: its shape, which a captured pass shares with its replays."""
+    single = next((i for i, n in enumerate(ctx.seg_len) if n > 1), len(ctx.seg_len))
+    return dict(single_rows=single, max_context=_longest_context(ctx), n_requests=len(ctx.seg_len) - single)
 
 
 def _longest_context(ctx) -> int:
@@ -1391,8 +1398,7 @@ def attention_general(q, cache, out, ctx, table, n_heads, n_kv, hd, *, page_size
             return attention_bf16(q, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, scale, chunk=chunk, sinks=sinks, gate=gate, cap=cap,
                                   channel_gate=channel_gate)
     return attention_exact(q, cache, out, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, scale, page_size=page_size,
-                           value_dim=value_dim, chunk=chunk, sinks=sinks, gate=gate, cap=cap, channel_gate=channel_gate, single_rows=ctx.max_seg_len == 1,
-                           max_context=_longest_context(ctx))
+                           value_dim=value_dim, chunk=chunk, sinks=sinks, gate=gate, cap=cap, channel_gate=channel_gate, **_known_of(ctx))
 
 
 # Up to so many rows the decode kernel rotates and writes the pages itself.  It saves the rotation kernel's launch wherever the

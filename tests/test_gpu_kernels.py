@@ -770,6 +770,8 @@ def test_attention_exact_has_one_order_of_sums(n_heads, n_kv, hd, ps, window, ch
     assert rel(whole, want) < 2e-6
     assert torch.equal(attend(max_context=1025), whole) and torch.equal(attend(max_context=4096), whole)
     assert torch.equal(attend(single_rows=True), whole) and torch.equal(attend(single_rows=True, max_context=1025), whole)
+    for known in (dict(single_rows=5), dict(single_rows=8, n_requests=1), dict(single_rows=T - 1, n_requests=1, max_context=1025), dict(n_requests=2), dict(n_requests=5, max_context=1025)):
+        assert torch.equal(attend(**known), whole), known
     for i in (0, 6, 7, 40, T - 4, T - 1):
         assert torch.equal(attend(slice(i, i + 1)), whole[i:i + 1]) and torch.equal(attend(slice(i, i + 1), max_context=2048), whole[i:i + 1])
     place = 1022                                             # of request 0, whose rows 1018 .. 1024 share tiles
