@@ -1810,20 +1810,29 @@ static int consumer_max_parts(int M) { return M <= 16 ? slim_max_parts(M) : M <=
 static bool many_tiles(int M, int N) { return (long)((M + 255) / 256) * ((N + 255) / 256) >= gi_compute_units() * 3 / 4; }
 
 // Which kernel takes a product of more than 128 rows that does not share k out: what counts are the rounds of tiles on the compute units,
-// each with what a tile takes to begin and to end.  Microseconds, fitted to measurements at K = 1,024 to 8,192 (2,048 rows of 3,072 x 2,048:
-// 51.5 with 128 x 128 tiles in two rounds, 35.0 with 256 x 128 in one; 300 rows of 16,384 x 2,048 gated 42 and 39; 3,000 rows of 3,072 x 2,048
-// 88 and 66; 2,048 rows of 16,384 x 2,048 gated 152 with 256 x 128 in four rounds, 120 with 256 x 256 in two).  Only the two larger tiles finish a
+// each with what a tile takes to begin and to end.  Microseconds, fitted to measurements at K = 128 to 8,192 (2,048 rows of 3,072 x 2,048 added onto
+// what is there: 51.5 with 128 x 128 tiles in two rounds, 35.0 with 256 x 128 in one; 300 rows of 16,384 x 2,048 gated 42 and 39; 3,000 rows of
+// 3,072 x 2,048 88 and 66; 2,048 rows of 16,384 x 2,048 gated 152 with 256 x 128 in four rounds, 120 with 256 x 256 in two).  A tile of 128 x 128 ends
+// soonest where its sums leave as they are or through LDS (stored, rotated, added with a norm handed on) and latest where they are added one by
+// one: at short k several rounds of those are the faster ones (2,600 rows of 4,096 x 512 stored: 21 us in three, 25.5 with 256 x 128 in two; of
+// 4,096 x 1,536 the same either way; 2,048 rows of 5,120 x 1,024 rotated 36 and 42).  Only the two larger tiles finish a
 // norm handed on to a gated product; the q/k/v product's epilogue rotates tiles 128 columns wide.
 enum Large { PIPED_128, TALL_256, PINGPONG_256 };
-static Large large_kernel(int M, int N, int K, bool rope, bool gated, bool scaled_rows) {
+static Large large_kernel(int M, int N, int K, int epi, bool rope, bool hands_norm, bool scaled_rows) {
     const long units = gi_compute_units(), m128 = (M + 127) / 128, m256 = (M + 255) / 256, n128 = (N + 127) / 128, n256 = (N + 255) / 256;
     const auto rounds = [&](long tiles) { return (double)((tiles + units - 1) / units); };
+    const bool many = many_tiles(M, N), gated = !rope && is_gated(epi);
+    // what a round of 128 x 128 tiles takes to end, and what of the last round's others need not wait for
+    struct { double each, less; } ends = {10, 0};                                            // added one by one (and stores with many tiles)
+    if (gated) ends = {6, 0};
+    else if (rope) ends = {7.4, 5};
+    else if (hands_norm || (!many && epi == EPI_STORE_BF16)) ends = {8, 4};
+    else if (!many && epi == EPI_STORE_F32) ends = {9, 8.4};
     const double blocks = K / PK, small = rounds(m128 * n128);
-    double piped = small > 1 ? small * (blocks * 0.45 + (gated ? 6 : 10)) : blocks * 0.55 + 12;      // (several: two workgroups a unit)
-    if (small > 2) piped *= 1.15;
+    double piped = small > 1 ? small * (blocks * 0.45 + ends.each) * (small > 2 ? 1.15 : 1) - ends.less : blocks * 0.55 + 12;      // (several: two workgroups a unit)
     if (scaled_rows && !rope) piped = 1e30;
     const double tall = rounds(m256 * n128) * (blocks * 0.715 + 13);
-    const double pingpong = many_tiles(M, N) && !rope ? rounds(m256 * n256) * (blocks * 1.45 + 14) : 1e30;
+    const double pingpong = many && !rope ? rounds(m256 * n256) * (blocks * 1.45 + 14) : 1e30;
     // (gating 256 x 128 sums at a time costs the tall kernel 3 us a round more: 1,500 rows by 16,384 of 2,048, three rounds of it against one and a
     // half of the ping-pong kernel: 114 us against 103)
     if (pingpong < piped && 0.95 * pingpong <= tall + (gated ? 3 * rounds(m256 * n128) : 0)) return PINGPONG_256;
@@ -2097,7 +2106,7 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
     GI_REQUIRE(norm_in.squares == nullptr || rope != nullptr || (is_gated(epi) && many_tiles(M, N) && norm_in.parts <= PIPED_MAX_PARTS),
                "gemm_bf16: a product of M %d, N %d, K %d takes no norm handed on in %d pieces", M, N, K, norm_in.parts);
     GI_REQUIRE(!many_tiles(M, N) || (lda < (1L << 22) && ldw < (1L << 22)), "gemm_bf16: row strides %ld, %ld are too large for the tile-relative addressing", lda, ldw);
-    const Large which = lda < (1L << 22) && ldw < (1L << 22) ? large_kernel(M, N, K, rope != nullptr, rope == nullptr && is_gated(epi), norm_in.squares != nullptr) : PIPED_128;
+    const Large which = lda < (1L << 22) && ldw < (1L << 22) ? large_kernel(M, N, K, epi, rope != nullptr, norm_out.scaled != nullptr, norm_in.squares != nullptr) : PIPED_128;
     if (which == PINGPONG_256) {
 #define PINGPONG(EPI_)                                                                                                                  \
     do {                                                                                                                                \
@@ -2260,6 +2269,16 @@ GI_API int gi_gemm_bf16_qkv_rope_store(const void* A, const void* W, int M, int 
         return launch_large(A, W, nullptr, EPI_STORE_F32, M, N, K, lda, ldw, (long)N, scratch, scratch_floats, NormIn{squares_in, parts_in, eps, K}, &rope, stream);
     return launch_skinny(A, W, nullptr, EPI_STORE_F32, M, N, K, lda, ldw, (long)N, scratch, scratch_floats, NormIn{squares_in, parts_in, eps, K}, NO_NORM_OUT,
                          stream, &rope);
+}
+
+// Which kernel makes a product of more than 128 rows whose rows lie whole in memory: 0 the tiles of 128 x 128, 1 those of 256 x 128, 2 those of 256 x 256,
+// 3 the first with k shared out over workgroups; -1 for sizes that none of these takes.  kind: 0 stored, 1 added, 2 added with a norm handed on, 3 gated,
+// 4 gated with a norm taken, 5 rotated into the pages, 6 through xielu.
+GI_API int gi_gemm_bf16_large_kernel(int M, int N, int K, int kind) {
+    if (M <= SKINNY_MAX_ROWS || K % PK != 0 || N < 128 || kind < 0 || kind > 6) return -1;
+    if (gi_gemm_bf16_piped_splits(M, N, K) > 1) return 3;
+    const int epi = kind == 0 ? EPI_STORE_F32 : kind <= 2 ? EPI_ADD_F32 : kind == 6 ? EPI_XIELU : EPI_GATED_BF16;
+    return large_kernel(M, N, K, epi, kind == 5, kind == 2, kind == 4);
 }
 
 // Whether gi_gemm_bf16_xielu takes a product of these sizes: up to 16 rows where the kernel for those serves; the rows of prompts

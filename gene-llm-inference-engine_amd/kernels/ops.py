@@ -147,6 +147,8 @@ def lib():
         l.gi_gemm_bf16_scratch_floats.restype = c_long
         l.gi_gemm_bf16_norm_parts.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_bf16_norm_parts.restype = c_int
+        l.gi_gemm_bf16_large_kernel.argtypes = [c_int, c_int, c_int, c_int]
+        l.gi_gemm_bf16_large_kernel.restype = c_int
         l.gi_gemm_bf16_xielu_takes.argtypes = [c_int, c_int, c_int, c_int]
         l.gi_gemm_bf16_xielu_takes.restype = c_int
         l.gi_gemm_bf16_takes_norm.argtypes = [c_int, c_int, c_int, c_int]
@@ -1504,6 +1506,14 @@ def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=N
     _call("gi_gemm_bf16", a.data_ptr(), w.data_ptr(), out.data_ptr(), _code(out, "gemm: out"), 1 if accumulate else 0, gate_code, float(gate_limit),
           m, n, k, a.stride(0), w.stride(0), out.stride(0), _ptr(scratch), n_scratch, _stream())
     return out
+
+
+def gemm_bf16_large_kernel(m, n, k, kind):
+    """Which kernel makes a product of more than 128 rows (None: none of these): "128x128", "256x128", "256x256" or "128x128 shared" (k shared out over
+    workgroups).  kind: "stored", "added", "added handing a norm on", "gated", "gated with a norm", "rotated" or "xielu"."""
+    kinds = ("stored", "added", "added handing a norm on", "gated", "gated with a norm", "rotated", "xielu")
+    which = lib().gi_gemm_bf16_large_kernel(m, n, k, kinds.index(kind))
+    return None if which < 0 else ("128x128", "256x128", "256x256", "128x128 shared")[which]
 
 
 @lru_cache(maxsize=None)

@@ -1,0 +1,24 @@
+"""Which kernel makes a product of a prompt's rows: the library's rule at sizes on both sides of its lines, on 256 compute units (which it
+assumes where there is no GPU)."""
+import pytest
+
+from geneinfer_amd.kernels import ops
+
+# m, n, k, what becomes of the sums -> the kernel that was the faster one there, by more than 4 %
+MEASURED = [
+    (2600, 4096, 128, "stored", "128x128"), (2600, 4096, 512, "stored", "128x128"), (2048, 4096, 768, "stored", "128x128"), (1777, 5120, 3072, "stored", "256x128"),
+    (1300, 6144, 256, "stored", "128x128"), (2048, 3072, 2048, "stored", "256x128"),
+    (2048, 3072, 512, "added", "256x128"), (2048, 3072, 2048, "added", "256x128"), (2600, 2048, 256, "added", "256x128"), (3000, 3072, 8192, "added", "256x128"),
+    (3000, 3072, 256, "added handing a norm on", "128x128"), (2600, 4096, 256, "added handing a norm on", "128x128"), (2048, 3072, 2048, "added handing a norm on", "256x128"),
+    (3000, 3072, 8192, "added handing a norm on", "256x128"),
+    (3000, 3072, 256, "rotated", "128x128"), (2048, 5120, 1024, "rotated", "128x128"), (1777, 6144, 1024, "rotated", "128x128"), (2048, 3072, 2048, "rotated", "256x128"),
+    (777, 5120, 3072, "rotated", "256x128"),
+    (300, 16384, 2048, "gated", "256x128"), (256, 16384, 2048, "gated", "128x128"), (2048, 16384, 2048, "gated", "256x256"), (1500, 16384, 2048, "gated with a norm", "256x256"),
+    (8192, 28672, 4096, "gated with a norm", "256x256"), (1777, 8192, 2048, "xielu", "256x256"), (2048, 2048, 2048, "added", "128x128"), (300, 2048, 2048, "added", "128x128 shared"),
+    (128, 4096, 4096, "stored", None), (200, 4096, 100, "stored", None),
+]
+
+
+@pytest.mark.parametrize("m,n,k,kind,kernel", MEASURED)
+def test_the_faster_kernel_is_chosen(m, n, k, kind, kernel):
+    assert ops.gemm_bf16_large_kernel(m, n, k, kind) == kernel
