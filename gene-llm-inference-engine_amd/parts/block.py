@@ -10,6 +10,8 @@
 The residual stream x is float32 [T, hidden] and is changed in place."""
 from __future__ import annotations
 
+import inspect
+
 import torch
 
 from ..kernels import ops
@@ -229,6 +231,8 @@ class ParallelBlock:
                 self.w_first = torch.cat(first, dim=0).contiguous()
                 self.mixer.use_input_weight(self.w_first[:self._split])
                 self.feed_forward.use_input_weight(self.w_first[self._split:])
+        # (a feed-forward built on one that takes activated columns may have a `forward` of its own that does not)
+        self._activates = hasattr(self.feed_forward, "input_activation") and "activated" in inspect.signature(self.feed_forward.forward).parameters
         self._readers = _Readers(self._parts()[1:], self._stacked)
 
     def _parts(self):
@@ -272,12 +276,11 @@ class ParallelBlock:
         w_first = self._stacked(ctx.n_rows)
         if w_first is not None:
             both = torch.empty((ctx.n_rows, w_first.shape[0]), dtype=torch.float32, device=x.device)
-            activated = self.feed_forward.activated(ctx.n_rows, x.device) if hasattr(self.feed_forward, "activated") else None
-            if activated is not None and linear_xielu(rows(self.mixer), w_first, activated[1], activated[0], both):
-                own[0]["projected"], own[1]["activated"] = both[:, :self._split], activated[0]
-            else:
+            activated = linear_xielu(rows(self.mixer), w_first, *self.feed_forward.input_activation(), both) if self._activates else None
+            if activated is None:
                 linear(rows(self.mixer), w_first, both)
-                own[0]["projected"], own[1]["projected"] = both[:, :self._split], both[:, self._split:]
+            own[0]["projected"] = both[:, :self._split]
+            own[1].update(activated=activated) if activated is not None else own[1].update(projected=both[:, self._split:])
         if then is not None:
             own[0 if last is self.mixer else 1]["then"] = then
         out = self.mixer.forward(rows(self.mixer), x, ctx, cache, **own[0])

@@ -33,24 +33,25 @@ def linear(a, weight: torch.Tensor, out: torch.Tensor, accumulate: bool = False,
     return ops.gemm_exact(a, weight, out, accumulate)
 
 
-def linear_xielu(a, weight: torch.Tensor, params: torch.Tensor, mid: torch.Tensor, out: torch.Tensor = None) -> bool:
+def linear_xielu(a, weight: torch.Tensor, params: torch.Tensor, columns: int, dtype: torch.dtype, out: torch.Tensor = None):
     """The product of `linear` with the activation of a feed-forward that has no gate in its epilogue, where a kernel does both
-    (`ops.gemm_bf16_xielu`): its last mid.shape[1] columns go to mid, the ones before to out.  False, and nothing done, where none does."""
+    (`ops.gemm_bf16_xielu`): its last `columns` columns come back activated, as `dtype`, the ones before go to out.  None where no
+    kernel does, and out is as it was."""
     n, k = weight.shape
-    rows = mid.shape[0]
-    if not (weight.dtype == torch.bfloat16 and mid.dtype == torch.bfloat16 and ops.gemm_bf16_xielu_takes(rows, n, k, n - mid.shape[1])):
-        return False
-    if isinstance(a, HandedRows) and rows <= 16 and takes_handed_norm(weight, rows) and ops.gemm_bf16_supports(a.scaled, weight, mid):
-        ops.gemm_bf16_xielu(a.scaled, weight, params, mid, out, norm_in=(a.squares, a.eps))
-        return True
-    if isinstance(a, HandedRows) or not (torch.is_tensor(a) or isinstance(a, NormedRows)):
-        return False
-    if isinstance(a, NormedRows):
-        a = a.materialize()
-    if not ops.gemm_bf16_supports(a, weight, mid):
-        return False
-    ops.gemm_bf16_xielu(a, weight, params, mid, out)
-    return True
+    rows = a.n_rows if isinstance(a, NormedRows) else a.shape[0]
+    if not (weight.dtype == dtype == torch.bfloat16 and ops.gemm_bf16_xielu_takes(rows, n, k, n - columns)):
+        return None
+    norm_in = None
+    if isinstance(a, HandedRows):
+        if not (rows <= 16 and takes_handed_norm(weight, rows)):
+            return None
+        a, norm_in = a.scaled, (a.squares, a.eps)
+    elif isinstance(a, NormedRows):
+        a = a.materialize()                      # (kept by `a` for whoever asks next)
+    if not ops.gemm_bf16_supports(a, weight, weight):
+        return None
+    mid = torch.empty((rows, columns), dtype=dtype, device=weight.device)
+    return ops.gemm_bf16_xielu(a, weight, params, mid, out, norm_in)
 
 
 def linear_onto(a: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor, then=None):

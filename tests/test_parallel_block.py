@@ -1,0 +1,79 @@
+"""A layer whose two halves' first products are one: what its feed-forward is told, on the CPU with stand-ins for the products."""
+from types import SimpleNamespace as Spec
+
+import pytest
+import torch
+
+from geneinfer_amd.parts import base, block
+from geneinfer_amd.parts.mlp import DenseMlp
+
+D, MIX, INTER = 16, 24, 32
+
+
+class Norm(base.Part):
+    def __init__(self, spec, tensors, dtype, device):
+        pass
+
+    def __call__(self, x, out_dtype):
+        return x.to(out_dtype)
+
+
+class Mixer(base.Part):
+    in_dtype = torch.bfloat16
+
+    def __init__(self, spec, tensors, dtype, device):
+        self.w = tensors["mix"]
+
+    def input_weight(self):
+        return self.w
+
+    def use_input_weight(self, view):
+        self.w = view
+
+    def forward(self, h, residual, ctx, cache, projected=None):
+        self.told = projected
+
+
+class Recording(DenseMlp):
+    def forward(self, h, residual, ctx, then=None, overwrite=False, projected=None, activated=None):
+        self.told = dict(projected=projected, activated=activated)
+
+
+class OfItsOwn(DenseMlp):
+    """Built on the feed-forward without a gate, with a `forward` that knows nothing of activated columns."""
+
+    def forward(self, h, residual, ctx, then=None, overwrite=False, projected=None):
+        self.told = dict(projected=projected)
+
+
+@pytest.fixture(scope="module", autouse=True)
+def kinds():
+    for register, kind, cls in ((base.register_norm, "stand_in", Norm), (base.register_mixer, "stand_in", Mixer), (base.register_feed_forward, "recording", Recording),
+                                (base.register_feed_forward, "of_its_own", OfItsOwn)):
+        register(kind, cls)
+
+
+@pytest.mark.parametrize("kind, taken", [("recording", True), ("recording", False), ("of_its_own", True)])
+def test_a_feed_forward_gets_its_columns_as_it_takes_them(kind, taken, monkeypatch):
+    up = torch.randn(INTER, D).bfloat16()
+    tensors = dict(mix=torch.randn(MIX, D).bfloat16(), up=up, down=torch.randn(D, INTER).bfloat16(), act=torch.tensor([0.3, 0.1]))
+    ff = Spec(kind=kind, activation="xielu", activation_params="act", up_proj="up", down_proj="down", intermediate_size=INTER, hidden_size=D)
+    spec = Spec(feed_forward_norm=None, mixer_post_norm=None, feed_forward_post_norm=None, mixer_norm=Spec(kind="stand_in"), mixer=Spec(kind="stand_in"), feed_forward=ff)
+    b = block.ParallelBlock(spec, tensors, torch.bfloat16, "cpu")
+    x = torch.randn(3, D)
+    ready = torch.randn(3, INTER).bfloat16()
+
+    def both_at_once(a, weight, params, columns, dtype, out):
+        if taken:
+            out[:, :MIX] = a.float() @ weight[:MIX].float().T
+            return ready
+
+    monkeypatch.setattr(block, "linear_xielu", both_at_once)
+    monkeypatch.setattr(block, "linear", lambda a, weight, out: out.copy_(a.float() @ weight.float().T))
+    b.forward(x, Spec(n_rows=3, dtype=torch.bfloat16, trace=None), None)
+    assert torch.equal(b.mixer.told, x.bfloat16().float() @ tensors["mix"].float().T)
+    told = b.feed_forward.told
+    if kind == "recording" and taken:
+        assert told["activated"] is ready and told["projected"] is None
+    else:
+        assert torch.equal(told["projected"], x.bfloat16().float() @ up.float().T) and told.get("activated") is None
