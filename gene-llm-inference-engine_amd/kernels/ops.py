@@ -1435,25 +1435,26 @@ def gemm_bf16_supports(a, w, out) -> bool:
 
 
 # What the library says about a shape does not change while the process lives, and a step asks it some hundred times: the answers
-# are kept (a question costs a call through ctypes, about a microsecond of the host's time each).
-@lru_cache(maxsize=None)
+# are kept (a question costs a call through ctypes, about a microsecond of the host's time each), a bounded number of them: prompts
+# come in any number of rows.
+@lru_cache(maxsize=8192)
 def _exact_scratch_floats(m, n, k) -> int:
     return lib().gi_gemm_exact_scratch_floats(m, n, k)
 
 
-@lru_cache(maxsize=None)
+@lru_cache(maxsize=8192)
 def _scratch_floats(m, n, k) -> int:
     return lib().gi_gemm_bf16_scratch_floats(m, n, k)
 
 
-@lru_cache(maxsize=None)
+@lru_cache(maxsize=8192)
 def gemm_bf16_norm_parts(m, n, k) -> int:
     """The pieces per row in which a product [m, k] x [n, k] that adds onto rows writes their sums of squares when it hands
     the next norm on (`gemm_bf16(..., norm_out=...)`); 0 if a product of these sizes cannot."""
     return lib().gi_gemm_bf16_norm_parts(m, n, k)
 
 
-@lru_cache(maxsize=None)
+@lru_cache(maxsize=8192)
 def gemm_bf16_takes_norm(m, n, k, gated=False) -> bool:
     """Whether a product of these sizes can read rows whose norm was handed on (`gemm_bf16(..., norm_in=...)`) by a product
     of as many rows."""
@@ -1516,7 +1517,7 @@ def gemm_bf16_large_kernel(m, n, k, kind):
     return None if which < 0 else ("128x128", "256x128", "256x256", "128x128 shared")[which]
 
 
-@lru_cache(maxsize=None)
+@lru_cache(maxsize=8192)
 def gemm_bf16_xielu_takes(m, n, k, first=0) -> bool:
     """Whether `gemm_bf16_xielu` takes a product of these sizes, `first` of whose columns stay as they are."""
     return bool(lib().gi_gemm_bf16_xielu_takes(m, n, k, first))
@@ -1544,13 +1545,13 @@ def gemm_bf16_xielu(a, w, params, mid, out=None, norm_in=None):
     return mid
 
 
-@lru_cache(maxsize=None)
+@lru_cache(maxsize=8192)
 def gemm_bf16_qkv_rope_store_takes(m, n, k, hd) -> bool:
     """Whether `gemm_bf16_qkv_rope_store` takes a q/k/v product of m rows, n = (heads + 2 kv heads) * hd columns and k."""
     return bool(lib().gi_gemm_bf16_qkv_rope_store_takes(m, n, k, hd))
 
 
-@lru_cache(maxsize=None)
+@lru_cache(maxsize=8192)
 def gemm_bf16_qkv_rope_store_max_parts(m, n, k) -> int:
     """The most pieces of a row's sum of squares (`norm_in`) that `gemm_bf16_qkv_rope_store` reads for these sizes."""
     return lib().gi_gemm_bf16_qkv_rope_store_max_parts(m, n, k)
