@@ -43,8 +43,8 @@ def test_gemm_exact(m, n, k, dtypes):
 
 @pytest.mark.parametrize("w_dtype,k", [(torch.float32, 200), (torch.float32, 203), (torch.bfloat16, 264), (torch.bfloat16, 520)])
 def test_gemm_exact_rows_alone_have_the_same_bits(w_dtype, k):
-    """One to four rows take the kernel with a lane per output column, more rows the tiled one; k = 203 leaves a tail
-    beside the 16-byte loads, 264 and 520 pieces of 8 beside whole groups of 64."""
+    """Few rows take the kernel without tiles where their rows lie aligned, more rows (and k = 203, which no 16-byte load may step through)
+    one with tiles; k = 200, 264 and 520 end within a range of k, or within a block of it."""
     a, w = randn(37, k, seed=3), randn(90, -(-k // 8) * 8, dtype=w_dtype, seed=4)[:, :k]      # the row stride stays a multiple of the 16-byte piece
     full = torch.empty(37, 90, device=DEV)
     ops().gemm_exact(a, w, full)
@@ -82,7 +82,7 @@ def test_gemm_exact_kernels_agree_in_bits(m, n, k):
 @pytest.mark.parametrize("m,n,k", [(1, 16, 8), (1, 2048, 2048), (3, 100, 136), (8, 130, 264), (16, 64, 128), (17, 1000, 520),
                                    (33, 48, 72), (64, 515, 1032), (65, 128, 64), (100, 300, 200), (128, 128, 128), (200, 257, 96),
                                    (513, 384, 1024), (2048, 96, 160),
-                                   # the LDS-ring kernel: one block of k, edge tiles, each of its three tile choices
+                                   # the kernels for more than 128 rows: one block of k, edge tiles (which kernel is whose: the next test)
                                    (256, 160, 64), (130, 129, 192), (2100, 2200, 192), (4000, 8200, 128),
                                    # the ping-pong kernel (256 x 256 tiles for every compute unit or more): one block of k, an odd number of them, edges
                                    (4100, 4104, 64), (4096, 4100, 320),
@@ -114,6 +114,63 @@ def test_gemm_bf16(m, n, k, out_dtype, accumulate):
     assert torch.equal(out[:, n:], base[:, n:])
 
 
+@pytest.mark.parametrize("kernel,kind,m,n,k", [
+    # two workgroups of four waves a unit; one of eight
+    ("128x128", "stored", 2600, 3072, 2048), ("128x128", "added", 2600, 3072, 2048), ("128x128", "added handing a norm on", 2600, 3072, 1024), ("128x128", "gated", 2600, 3072, 192),
+    ("128x128", "xielu", 2600, 3072, 192), ("128x128", "stored", 2590, 3070, 64), ("128x128", "added", 2590, 3070, 128), ("128x128", "gated", 2590, 3040, 64),
+    ("128x128", "stored", 300, 3000, 320), ("128x128", "added", 300, 3000, 64), ("128x128", "added handing a norm on", 1300, 1024, 256), ("128x128", "gated", 300, 3040, 128), ("128x128", "xielu", 300, 3000, 320),
+    # one block of k, two (where the loop's first and last waits meet), more; edge tiles
+    ("256x128", "added", 2048, 3072, 64), ("256x128", "added", 2048, 3072, 128), ("256x128", "added", 2047, 3050, 192), ("256x128", "stored", 2030, 3050, 1536), ("256x128", "stored", 2048, 3072, 2048),
+    ("256x128", "added handing a norm on", 2048, 3072, 1024), ("256x128", "added handing a norm on", 1700, 3072, 2048), ("256x128", "gated", 300, 16384, 512), ("256x128", "gated", 390, 16352, 384),
+    ("256x128", "xielu", 2048, 3072, 64), ("256x128", "xielu", 2030, 3050, 128),
+    ("256x256", "stored", 4100, 4104, 64), ("256x256", "added", 4100, 4104, 128), ("256x256", "gated", 2048, 16384, 192), ("256x256", "xielu", 2048, 8192, 64)])
+def test_products_of_prompts_in_each_kernel(kernel, kind, m, n, k):
+    """Every kernel for more than 128 rows with every end of a product it may be given, at sizes the library's rule sends to it, against 64 bits.
+    (Rotated into the pages: `test_qkv_product_that_rotates_and_fills_the_pages`.)"""
+    o = ops()
+    assert o.gemm_bf16_large_kernel(m, n, k, kind) == kernel
+    a, w = randn(m, k, dtype=torch.bfloat16, seed=11), randn(n, k, dtype=torch.bfloat16, seed=12, scale=1.5 / k ** 0.5)
+    want = a.double() @ w.double().T
+    if kind == "stored":
+        out, half = torch.full((m, n + 3), 7.0, device=DEV), torch.full((m, n + 4), 7.0, dtype=torch.bfloat16, device=DEV)
+        o.gemm_bf16(a, w, out[:, :n])
+        o.gemm_bf16(a, w, half[:, :n])
+        assert rel(out[:, :n], want) < 1e-5 and torch.equal(half[:, :n], out[:, :n].to(torch.bfloat16))
+        assert bool((out[:, n:] == 7).all()) and bool((half[:, n:] == 7).all())
+    elif kind == "added":
+        base = randn(m, n + 1, seed=13)
+        out = base.clone()
+        o.gemm_bf16(a, w, out[:, :n], accumulate=True)
+        assert rel(out[:, :n], want + base[:, :n].double()) < 1e-5 and torch.equal(out[:, n:], base[:, n:])
+    elif kind == "added handing a norm on":
+        parts = o.gemm_bf16_norm_parts(m, n, k)
+        assert parts == n // 128
+        base, g = randn(m, n, seed=13), (1 + 0.1 * randn(n, seed=14)).float()
+        plain, x = base.clone(), base.clone()
+        o.gemm_bf16(a, w, plain, accumulate=True)
+        scaled, squares = torch.empty(m, n, dtype=torch.bfloat16, device=DEV), torch.empty(m, parts, device=DEV)
+        o.gemm_bf16(a, w, x, accumulate=True, norm_out=(g, scaled, squares))
+        assert rel(x, want + base.double()) < 1e-5 and torch.equal(x, plain) and torch.equal(scaled, (g * x).to(torch.bfloat16))
+        assert rel(squares.double(), (x.double() ** 2).view(m, parts, 128).sum(2)) < 1e-6
+    elif kind == "gated":
+        v = want.view(m, n // 32, 2, 16)
+        gate, up = v[:, :, 0].reshape(m, -1), v[:, :, 1].reshape(m, -1)
+        ends = dict(silu=torch.nn.functional.silu(gate) * up, gelu_tanh=torch.nn.functional.gelu(gate, approximate="tanh") * up)
+        low = gate.clamp(max=1.5)
+        ends["swish_clamped"] = low * torch.sigmoid(1.702 * low) * (up.clamp(-1.5, 1.5) + 1)
+        for name, right in ends.items():
+            out = torch.full((m, n // 2 + 1), 7.0, dtype=torch.bfloat16, device=DEV)
+            o.gemm_bf16(a, w, out[:, :n // 2], gated=name, gate_limit=1.5)
+            assert rel(out[:, :n // 2], right) < 4e-3 and bool((out[:, n // 2:] == 7).all()), name        # (one rounding to bfloat16: 2^-8 of the largest at most)
+    else:
+        params = torch.tensor([0.3, -0.7], device=DEV)
+        pa, pb = torch.nn.functional.softplus(params.double())
+        right = torch.where(want > 0, pa * want * want + 0.5 * want, (0.5 + pb) * (torch.expm1(want) - want) + 0.5 * want)
+        out = torch.full((m, n + 5), 7.0, dtype=torch.bfloat16, device=DEV)
+        o.gemm_bf16_xielu(a, w, params, out[:, :n])
+        assert rel(out[:, :n], right) < 4e-3 and bool((out[:, n:] == 7).all())
+
+
 @pytest.mark.parametrize("m,inter,k", [(1, 16, 8), (5, 48, 136), (16, 160, 96), (17, 176, 64), (64, 32, 264), (70, 192, 128), (300, 8192 // 16, 2048 // 8),
                                        (72, 8192, 2048), (128, 6144, 264), (100, 288, 136),
                                        (40, 6144, 264), (13, 6160, 72), (64, 8192, 512), (2048, 1024, 192), (600, 288, 64), (200, 512, 1024),
@@ -142,6 +199,7 @@ def test_gated_products_have_one_gate(m, inter, k, few, columns, stride, gated, 
     a = randn(m, k, dtype=torch.bfloat16, seed=15)
     w = randn(2 * inter, k, dtype=torch.bfloat16, seed=16, scale=2.0 / k ** 0.5)
     out = torch.full((m, stride), 3.0, dtype=torch.bfloat16, device=DEV)
+    assert ops().gemm_bf16_large_kernel(m, 2 * inter, k, "gated") == "256x128" and ops().gemm_bf16_large_kernel(few, 2 * columns, k, "gated") == "128x128"
     ops().gemm_bf16(a, w, out[:, :inter], gated=gated, gate_limit=limit)
     alone = torch.empty(few, columns, dtype=torch.bfloat16, device=DEV)
     ops().gemm_bf16(a[:few], w[:2 * columns], alone, gated=gated, gate_limit=limit)
@@ -320,9 +378,11 @@ def test_norm_handed_on_by_a_product_of_many_rows(m, d, k1):
 @pytest.mark.parametrize("m,hidden,n_heads,n_kv,hd,page_size,rotate,handed", [(64, 2048, 32, 8, 64, 16, True, True), (40, 2048, 32, 8, 64, 16, True, False),
                                                                               (128, 3072, 24, 8, 128, 16, True, True), (33, 512, 6, 1, 32, 8, False, False),
                                                                               (17, 4096, 32, 8, 128, 32, True, False), (100, 1024, 2, 1, 256, 16, True, True),
-                                                                              # rows of prompts: tiles of 128 x 128 whose epilogue rotates and stores (two workgroups
-                                                                              # of four waves a unit; one of eight), and shapes whose k is shared out over workgroups
-                                                                              (2048, 2048, 32, 8, 64, 16, True, False), (1100, 256, 20, 2, 128, 16, True, True),
+                                                                              # rows of prompts: tiles of 256 x 128 and of 128 x 128 whose epilogue rotates and stores (the
+                                                                              # smaller ones with two workgroups of four waves a unit, and with one of eight), and shapes
+                                                                              # whose k is shared out over workgroups
+                                                                              (2048, 2048, 32, 8, 64, 16, True, False), (2048, 2048, 32, 8, 64, 16, True, True), (777, 2048, 24, 8, 128, 12, False, True),
+                                                                              (2600, 2048, 32, 8, 64, 16, True, False), (2600, 1024, 32, 8, 64, 16, True, True), (1100, 256, 20, 2, 128, 16, True, True),
                                                                               (1100, 256, 80, 8, 32, 8, False, True), (300, 3072, 24, 8, 128, 16, True, True),
                                                                               (520, 512, 28, 2, 64, 16, True, False), (129, 2048, 32, 8, 64, 16, True, True)])
 def test_qkv_product_that_rotates_and_fills_the_pages(m, hidden, n_heads, n_kv, hd, page_size, rotate, handed):
@@ -333,6 +393,8 @@ def test_qkv_product_that_rotates_and_fills_the_pages(m, hidden, n_heads, n_kv, 
     o = ops()
     n = (n_heads + 2 * n_kv) * hd
     assert o.gemm_bf16_qkv_rope_store_takes(m, n, hidden, hd)
+    if m in (777, 2048, 2600):
+        assert o.gemm_bf16_large_kernel(m, n, hidden, "rotated") == ("128x128" if m == 2600 else "256x128")
     a = randn(m, hidden, dtype=torch.bfloat16, seed=1)
     w = randn(n, hidden, dtype=torch.bfloat16, seed=2, scale=0.05)
     g = torch.Generator().manual_seed(9)
