@@ -44,7 +44,7 @@ constexpr int MAX_HD = 640;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
-constexpr int BLOCK = 64, SPAN = 4 * BLOCK, PAIRS = 16;
+constexpr int BLOCK = 64, SPAN = 4 * BLOCK, PAIRS = 16, MAX_SPANS = 65535;
 
 // A span joins what came before it (m, l, and every O with the two factors): nothing happens for a row that sees no key of the span, which its
 // positions tell and not the scores (a score that is no number does not show in the largest one: the row's sums must hand it on, and so must
@@ -396,12 +396,13 @@ static long count_tiles(int n_rows, int n_single, int n_kv, int group) {
 }
 
 // How many spans of 256 keys the widest row of a step has at most, 0 where they are not shared out: `seen` positions at most are seen by a row.
-// They are shared out while the tiles alone give fewer than two workgroups a compute unit, and the parts stay under 64 MB.
+// They are shared out while the tiles alone give fewer than two workgroups a compute unit, and the parts stay under 64 MB and in number
+// under what a grid's second dimension holds.
 GI_API int gi_attention_exact_spans(int n_rows, int n_single, int n_heads, int n_kv, int hd, int vd, int page_size, int seen) {
     if (n_rows <= 0 || n_single < 0 || n_single > n_rows || n_kv <= 0 || n_heads % n_kv != 0 || seen <= SPAN || !takes_tiles(hd, vd, page_size)) return 0;
     const long tiles = count_tiles(n_rows, n_single, n_kv, n_heads / n_kv);
     const long spans = ((long)seen + SPAN - 1) / SPAN + 1;
-    if (tiles >= 2L * gi_compute_units() || spans * n_rows * n_heads * part_floats(vd) > (16L << 20)) return 0;
+    if (tiles >= 2L * gi_compute_units() || spans > MAX_SPANS || spans * n_rows * n_heads * part_floats(vd) > (16L << 20)) return 0;
     return (int)spans;
 }
 GI_API long gi_attention_exact_part_floats(int n_rows, int n_heads, int vd, int n_spans) { return (long)n_rows * n_heads * n_spans * part_floats(vd); }
@@ -424,7 +425,7 @@ GI_API int gi_attention_exact(const void* q, int q_dtype, const void* cache, int
         GI_REQUIRE(n_single >= 0 && n_single <= n_rows, "attention_exact: %d single rows of %d", n_single, n_rows);
         const int a_tile = rows_a_tile(n_heads / n_kv), turns = n_single == n_rows ? 1 : n_requests > 0 && n_requests < a_tile ? n_requests : a_tile;
         if (n_spans > 0) {
-            GI_REQUIRE(part != nullptr && aligned(part) && part_size >= gi_attention_exact_part_floats(n_rows, n_heads, vd, n_spans) && n_spans <= 65535,
+            GI_REQUIRE(part != nullptr && aligned(part) && part_size >= gi_attention_exact_part_floats(n_rows, n_heads, vd, n_spans) && n_spans <= MAX_SPANS,
                        "attention_exact: sharing the keys out needs %ld floats", gi_attention_exact_part_floats(n_rows, n_heads, vd, n_spans));
         } else {
             part = nullptr;

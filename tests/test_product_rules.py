@@ -1,5 +1,5 @@
-"""Which kernel makes a product of a prompt's rows: the library's rule at sizes on both sides of its lines, on 256 compute units (which it
-assumes where there is no GPU)."""
+"""The library's own rules at sizes on both sides of their lines, on 256 compute units (which it assumes where there is no GPU): which kernel
+makes a product of a prompt's rows, and which contexts the 32-bit attention shares out."""
 import pytest
 
 from geneinfer_amd.kernels import ops
@@ -22,3 +22,9 @@ MEASURED = [
 @pytest.mark.parametrize("m,n,k,kind,kernel", MEASURED)
 def test_the_faster_kernel_is_chosen(m, n, k, kind, kernel):
     assert ops.gemm_bf16_large_kernel(m, n, k, kind) == kernel
+
+
+@pytest.mark.parametrize("rows,seen,spans", [(1, 256, 0), (1, 257, 3), (3, 4096, 17), (1, 65534 * 256, 65535), (1, 65534 * 256 + 1, 0), (1, 1 << 30, 0)])
+def test_a_context_is_shared_out_over_so_many_spans_as_a_grid_takes(rows, seen, spans):
+    """One head of 16 channels, whose parts are small: longer contexts stay whole (0), they are not refused."""
+    assert ops.lib().gi_attention_exact_spans(rows, rows, 1, 1, 16, 16, 16, seen) == spans
