@@ -595,7 +595,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_grouped_kernel(const bf16_t* __
 // issue, which is what bounds the interval between two barriers; a load costs the wave that issues it
 // 23 clocks when nothing else runs and 70 to 140 here, wherever in the two phases it is put.  How far ahead the loads are sent
 // counts as well (all of LDS is taken for it): with two stages of W, sent for one block ahead, 8,192 rows of 28,672 x 4,096 gated took 1,558 us,
-// of 4,096 x 14,336 831, of 6,144 x 4,096 368; with three 1,470, 740 and 332 (K = 2,048, 32 blocks a tile: no difference).
+// of 4,096 x 14,336 831, of 6,144 x 4,096 368; with three 1,470, 740 and 332.  At K = 2,048, 32 blocks a tile, it is 0 to 2 %: 1,500 rows
+// of 16,384 gated 104.8 and 102.6 us, 2,048 rows 118.4 and 118.0, 3,000 rows 174.8 and 174.1, 8,192 rows 460 and 451.
 template <int BN, int EPI>
 __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ C,
                                                                 int M, int N, int K, long lda, long ldw, long ldc, NormIn norm_in) {
@@ -2235,7 +2236,7 @@ GI_API int gi_gemm_bf16_handing(const void* A, const void* W, void* C, int c_dty
 
 // Whether gi_gemm_bf16_qkv_rope_store takes a q/k/v product of these sizes with heads of hd channels.  17 or 33 to 128 rows: the
 // shapes whose k is shared out over workgroups, whose sums a second kernel adds up anyway.  More rows: the kernels with tiles of
-// 128 x 128, whose epilogue lays the tile into LDS and sends it off rotated (whole heads must lie inside a tile), or, where they
+// 128 x 128 and 256 x 128, whose epilogues lay 128 rows of the tile into LDS and send them off rotated (whole heads must lie inside a tile), or, where they
 // share k out, that second kernel again.
 GI_API int gi_gemm_bf16_qkv_rope_store_takes(int M, int N, int K, int hd) {
     if (hd < 8 || hd > 256 || (hd & (hd - 1)) != 0) return 0;
