@@ -44,6 +44,17 @@ __device__ __forceinline__ void fold(int q, f32x4 (&acc)[N], f32x4 (&t)[3][N]) {
     }
 }
 
+// ... where the ranges behind the first n have nothing of k in them: the tree's open branches are closed (their other halves are zeros).
+template <int N>
+__device__ __forceinline__ void close(int n, f32x4 (&acc)[N], const f32x4 (&t)[3][N]) {
+#pragma unroll
+    for (int b = 1; b < 3; ++b) {
+        if (!(n >> b & 1) || (n & ((1 << b) - 1)) == 0) continue;
+#pragma unroll
+        for (int i = 0; i < N; ++i) acc[i] = t[b][i] + acc[i];
+    }
+}
+
 template <typename TC, bool ACCUMULATE>
 __device__ __forceinline__ void put(TC* C, size_t o, float v) {
     if constexpr (ACCUMULATE) store_f32(C, o, load_f32(C, o) + v);
@@ -102,8 +113,11 @@ __device__ __forceinline__ f32x4 fetch(const T* base, long ld, int row, int rows
         v = load4(p + min(k, K - 4));
         if (k >= K) v = f32x4{0.f, 0.f, 0.f, 0.f};
     } else {
+        // (asked for by every lane, wherever K ends: a load under a condition is waited for before the next)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = k + i < K ? load_f32(p, (size_t)(k + i)) : 0.f;
+        for (int i = 0; i < 4; ++i) v[i] = load_f32(p, (size_t)min(k + i, K - 1));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = k + i < K ? v[i] : 0.f;
     }
     return v;
 }
@@ -142,7 +156,10 @@ __global__ __launch_bounds__(256) void gemm_exact_tiled_kernel(const TA* __restr
     int s = q0 * per_range;
     if (s < s_end) { ask(s); lay(s & 1); }
     __syncthreads();
-    for (int q = q0; q < q1; ++q) {
+    const int q_end = max(q0, min(q1, (s_end + per_range - 1) / per_range));              // (short k leaves ranges empty)
+#pragma unroll
+    for (int i = 0; i < TN * TM; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int q = q0; q < q_end; ++q) {
 #pragma unroll
         for (int i = 0; i < TN * TM; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
         const int stop = min((q + 1) * per_range, s_end);
@@ -169,6 +186,7 @@ __global__ __launch_bounds__(256) void gemm_exact_tiled_kernel(const TA* __restr
         }
         fold(q - q0, acc, t);              // (the workgroup's ranges are a whole branch of the tree)
     }
+    close(q_end - q0, acc, t);
     store_tile<TM, TN, TC, ACCUMULATE>(acc, C, part, m0 + wm + r, n0 + wn + 4 * g, z, M, N, ldc);
 }
 
@@ -215,7 +233,10 @@ __global__ __launch_bounds__(256) void gemm_exact_ring_kernel(const float* __res
         if (s_begin + i < s_end) issue(s_begin + i, i);
     const int a_at[2] = {chunk_at(wm + r, g), chunk_at(wm + r, 4 + g)}, w_at[2] = {BM * BK + chunk_at(wn + r, g), BM * BK + chunk_at(wn + r, 4 + g)};
     int s = s_begin, slot = 0;
-    for (int q = q0; q < q1; ++q) {
+    const int q_end = max(q0, min(q1, (s_end + per_range - 1) / per_range));              // (short k leaves ranges empty)
+#pragma unroll
+    for (int i = 0; i < TN * TM; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int q = q0; q < q_end; ++q) {
 #pragma unroll
         for (int i = 0; i < TN * TM; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
         const int stop = min((q + 1) * per_range, s_end);
@@ -248,6 +269,7 @@ __global__ __launch_bounds__(256) void gemm_exact_ring_kernel(const float* __res
         }
         fold(q - q0, acc, t);
     }
+    close(q_end - q0, acc, t);
     store_tile<TM, TN, float, ACCUMULATE>(acc, C, part, m0 + wm + r, n0 + wn + 4 * g, z, M, N, ldc);
 }
 

@@ -58,7 +58,9 @@ def test_gemm_exact_rows_alone_have_the_same_bits(w_dtype, k):
         assert torch.equal(few, wide[:rows])                                # adding onto what is there, the same in both kernels
 
 
-@pytest.mark.parametrize("m,n,k", [(64, 256, 8192), (33, 130, 2080), (300, 160, 64), (129, 65, 4128), (16, 2048, 8192), (17, 90, 32), (70, 100, 1000), (40, 70, 203)])
+@pytest.mark.parametrize("m,n,k", [(64, 256, 8192), (33, 130, 2080), (300, 160, 64), (129, 65, 4128), (16, 2048, 8192), (17, 90, 32), (70, 100, 1000), (40, 70, 203),
+                                   # three, five, six and seven ranges of k that are not empty, the last ones whole or not
+                                   (40, 70, 96), (300, 160, 160), (33, 90, 192), (70, 100, 224), (40, 70, 75), (70, 90, 141), (40, 70, 201)])
 def test_gemm_exact_kernels_agree_in_bits(m, n, k):
     """Whole blocks of 32 k go through LDS in a ring (tiles of 32 and 64 rows, k shared out over 1 to 8 workgroups where the tiles are few),
     other aligned rows are staged through registers, unaligned ones element by element, a few rows need no tiles: one order of every sum."""
