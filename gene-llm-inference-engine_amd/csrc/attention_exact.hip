@@ -19,9 +19,9 @@
 // [kv_head][vd][place] (vd channels a value head, hd a key head); table[slot][i] is the page of
 // positions i*page_size .. (i+1)*page_size - 1.
 //
-// Two kernels.  Which one serves depends on the data types and on hd, vd and the page size alone, so one model meets one of them:
-//   tiles    32-bit throughout, hd and vd multiples of 16 up to 128, pages of a multiple of 4: both products on the 32-bit matrix
-//            instructions, four waves a workgroup, long contexts shared out over workgroups;
+// Two kernels.  Which one serves depends on the data types and on hd, vd, the page size, the window and the chunk alone, so one layer meets one of them:
+//   tiles    32-bit throughout, hd and vd multiples of 16 up to 128, pages of a multiple of 4, rows that may see more than 16 keys: both products
+//            on the 32-bit matrix instructions, four waves a workgroup, long contexts shared out over workgroups;
 //   rows     everything else: one wave per (row, query head), keys 64 at a time.
 #include "common.h"
 
@@ -78,10 +78,14 @@ __device__ __forceinline__ float finished(float o, double l, const float* gate, 
 // One (row, head, span) of `part`: vd sums, then l (64-bit), then m.
 __host__ __device__ constexpr int part_floats(int vd) { return vd + 4; }
 
+// n / size for n >= 0, without the division (magic = floor(2^32 (2^shift - size) / size) + 1, shift = ceil(log2(size)))
+struct Divisor { int size; unsigned magic; int shift; };
+__device__ __forceinline__ int quotient(int n, const Divisor& by) { return (int)((__umulhi(by.magic, (unsigned)n) + (unsigned)n) >> by.shift); }
+
 template <int D>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_kernel(const float* __restrict__ q, const float* __restrict__ cache, float* __restrict__ out,
                                                                    const int* __restrict__ pos, const int* __restrict__ slot, const int* __restrict__ table,
-                                                                   int table_stride, long page_stride, int page_size, int n_rows, int n_heads, int n_kv, int hd, int vd,
+                                                                   int table_stride, long page_stride, Divisor pages, int n_rows, int n_heads, int n_kv, int hd, int vd,
                                                                    int window, int chunk, float scale, float cap, const float* __restrict__ sinks,
                                                                    const float* __restrict__ gate, long gate_stride, int gate_channels, int n_single, int rows_a_tile,
                                                                    float* __restrict__ part, int n_spans) {
@@ -103,6 +107,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
 #pragma unroll
     for (int c = 0; c < D / 16; ++c)
         qv[c] = valid && c * 16 < hd ? *reinterpret_cast<const f32x4*>(q + ((size_t)t * n_heads + h) * hd + c * 16 + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
+    const int page_size = pages.size;
     const long v_plane = (long)n_kv * page_size * hd;   // from a page's keys to its values
 
     // Rows of one request at a time: a tile with rows of several requests takes as many turns, shared out over gridDim.z workgroups.  (One after the
@@ -139,18 +144,25 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
             const int b0 = s * SPAN + wave * BLOCK;
             float m = -INFINITY, l = 0.f;
             if (b0 <= p_max && b0 + BLOCK > lo_min) {                     // (the same for the wave)
+                // Groups of 16 keys that no row of the tile sees are loaded (from a place that one does see) and left out.  A wave alone on its SIMD
+                // takes seven clocks or so an instruction, and at short contexts and windows a span is little else.
+                bool live[4];
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt) live[kt] = b0 + kt * 16 <= p_max && b0 + kt * 16 + 16 > lo_min;
                 f32x4 kk[4][D / 16], vv[4][D / 16];
 #pragma unroll
                 for (int kt = 0; kt < 4; ++kt) {
                     const int key = max(min(b0 + kt * 16 + r, p_max), lo_min);
-                    const float* from = cache + (size_t)tab[key / page_size] * page_stride + ((size_t)kv * page_size + key % page_size) * hd + 4 * g;
+                    const int page = quotient(key, pages);
+                    const float* from = cache + (size_t)tab[page] * page_stride + ((size_t)kv * page_size + key - page * page_size) * hd + 4 * g;
 #pragma unroll
                     for (int c = 0; c < D / 16; ++c) kk[kt][c] = c * 16 < hd ? *reinterpret_cast<const f32x4*>(from + c * 16) : f32x4{0.f, 0.f, 0.f, 0.f};
                 }
 #pragma unroll
                 for (int kt = 0; kt < 4; ++kt) {
                     const int first = b0 + kt * 16 + 4 * g, key = max(min(first, p_max), lo_min) & ~3;
-                    const float* from = cache + (size_t)tab[key / page_size] * page_stride + v_plane + ((size_t)kv * vd + r) * page_size + key % page_size;
+                    const int page = quotient(key, pages);
+                    const float* from = cache + (size_t)tab[page] * page_stride + v_plane + ((size_t)kv * vd + r) * page_size + key - page * page_size;
 #pragma unroll
                     for (int c = 0; c < D / 16; ++c) vv[kt][c] = c * 16 < vd ? *reinterpret_cast<const f32x4*>(from + (size_t)c * 16 * page_size) : f32x4{0.f, 0.f, 0.f, 0.f};
                 }
@@ -158,6 +170,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
 #pragma unroll
                 for (int kt = 0; kt < 4; ++kt) {
                     sc[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    if (!live[kt]) continue;
 #pragma unroll
                     for (int c = 0; c < D / 16; ++c)
                         if (c * 16 < hd) {
@@ -166,7 +179,8 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
                         }
                 }
 #pragma unroll
-                for (int kt = 0; kt < 4; ++kt)
+                for (int kt = 0; kt < 4; ++kt) {
+                    if (!live[kt]) continue;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const int key = b0 + kt * 16 + 4 * g + i;
@@ -175,15 +189,18 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
                         sc[kt][i] = in_run && key <= my_pos && key >= my_lo ? x : -INFINITY;
                         m = fmaxf(m, sc[kt][i]);
                     }
+                }
                 m = fmaxf(m, __shfl_xor(m, 16, 64));
                 m = fmaxf(m, __shfl_xor(m, 32, 64));
 #pragma unroll
-                for (int kt = 0; kt < 4; ++kt)
+                for (int kt = 0; kt < 4; ++kt) {
+                    if (!live[kt]) continue;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         sc[kt][i] = sc[kt][i] == -INFINITY ? 0.f : expf(sc[kt][i] - m);
                         l += sc[kt][i];
                     }
+                }
                 l += __shfl_xor(l, 16, 64);
                 l += __shfl_xor(l, 32, 64);
                 // A probability of zero must not meet a value that is no number: places nobody has written, and, where some pair of the
@@ -192,7 +209,8 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
                 const bool all_seen = b0 >= lo_max && b0 + BLOCK - 1 <= p_min;
                 if (!all_seen) {
 #pragma unroll
-                    for (int kt = 0; kt < 4; ++kt)
+                    for (int kt = 0; kt < 4; ++kt) {
+                        if (!live[kt]) continue;
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
                             const int key = b0 + kt * 16 + 4 * g + i;
@@ -202,16 +220,20 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
                                 odd = odd || !(fabsf(vv[kt][c][i]) < INFINITY);
                             }
                         }
+                    }
                 }
                 f32x4 o[D / 16];
 #pragma unroll
-                for (int c = 0; c < D / 16; ++c) {
-                    o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-                    if (c * 16 >= vd) continue;
+                for (int c = 0; c < D / 16; ++c) o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int kt = 0; kt < 4; ++kt)
+                for (int kt = 0; kt < 4; ++kt) {
+                    if (!live[kt]) continue;
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) o[c] = mfma(vv[kt][c][j], sc[kt][j], o[c]);
+                    for (int c = 0; c < D / 16; ++c)
+                        if (c * 16 < vd) {
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) o[c] = mfma(vv[kt][c][j], sc[kt][j], o[c]);
+                        }
                 }
                 if (__ballot(odd) != 0) {
                     for (int row = 0; row < rows_here; ++row) {
@@ -220,12 +242,14 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
                         for (int c = 0; c < D / 16; ++c) {
                             f32x4 own = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                            for (int kt = 0; kt < 4; ++kt)
+                            for (int kt = 0; kt < 4; ++kt) {
+                                if (!live[kt]) continue;
 #pragma unroll
                                 for (int j = 0; j < 4; ++j) {
                                     const int key = b0 + kt * 16 + 4 * g + j;
                                     own = mfma(key > row_pos || key < row_lo ? 0.f : vv[kt][c][j], sc[kt][j], own);
                                 }
+                            }
                             if (place == row) o[c] = own;
                         }
                     }
@@ -266,8 +290,8 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
             __syncthreads();
 #pragma unroll
             for (int e = 0; e < PAIRS * D / 256; ++e) {
-                const int at = tid + 256 * e, pair = at / vd, d = at % vd;
-                if (pair >= PAIRS) break;
+                const int pair = (tid + 256 * e) / D, d = (tid + 256 * e) % D;
+                if (d >= vd) continue;
                 float o = 0.f;
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
@@ -287,9 +311,8 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
         if (!part) {
 #pragma unroll
             for (int e = 0; e < PAIRS * D / 256; ++e) {
-                const int at = tid + 256 * e, pair = at / vd, d = at % vd;
-                if (pair >= PAIRS) break;
-                if (run_s[pair])
+                const int pair = (tid + 256 * e) / D, d = (tid + 256 * e) % D;
+                if (d < vd && run_s[pair])
                     out[((size_t)t_s[pair] * n_heads + h_s[pair]) * vd + d] = finished(o_all[e], l_all[pair], gate, gate_stride, gate_channels, t_s[pair], h_s[pair], d);
             }
         }
@@ -385,8 +408,14 @@ __global__ __launch_bounds__(64) void attention_exact_kernel(const TQ* __restric
 
 GI_API int gi_attention_exact_max_head_size() { return MAX_HD; }
 
-// Whether the kernel with tiles serves these sizes (all operands 32-bit and aligned).
-static bool takes_tiles(int hd, int vd, int page_size) { return hd % 16 == 0 && vd % 16 == 0 && hd <= 128 && vd <= 128 && page_size % 4 == 0; }
+// Whether the kernel with tiles serves these sizes (all operands 32-bit and aligned).  Not where a window or a chunk leaves a row 16 keys at most: a block
+// of 64 keys costs a tile much the same however few it sees of them.  Microseconds of rows and tiles, 16 single rows at 400 positions and more and a prompt of 300, 32/8 heads of 64:
+// windows of 8 keys 6 and 13, 18 and 22; of 16 8 and 13, 28 and 23; of 32 11 and 14, 46 and 24; of 64 19 and 16, 82 and 28; of 256 74 and 22, 204 and 32.  (The
+// tiles took 19 and 31 at all of the first three while they divided by the page size and worked on keys that nobody sees.)
+static bool takes_tiles(int hd, int vd, int page_size, int window, int chunk) {
+    if ((window > 0 && window <= 16) || (chunk > 0 && chunk <= 16)) return false;
+    return hd % 16 == 0 && vd % 16 == 0 && hd <= 128 && vd <= 128 && page_size % 4 == 0;
+}
 
 // Rows of a tile: what its 16 pairs have room for.  The first `n_single` rows of a step, its requests' only ones (decoded rows), have tiles of their own.
 static int rows_a_tile(int group) { return group < PAIRS ? PAIRS / group : 1; }
@@ -399,7 +428,7 @@ static long count_tiles(int n_rows, int n_single, int n_kv, int group) {
 // They are shared out while the tiles alone give fewer than two workgroups a compute unit, and the parts stay under 64 MB and in number
 // under what a grid's second dimension holds.
 GI_API int gi_attention_exact_spans(int n_rows, int n_single, int n_heads, int n_kv, int hd, int vd, int page_size, int seen) {
-    if (n_rows <= 0 || n_single < 0 || n_single > n_rows || n_kv <= 0 || n_heads % n_kv != 0 || seen <= SPAN || !takes_tiles(hd, vd, page_size)) return 0;
+    if (n_rows <= 0 || n_single < 0 || n_single > n_rows || n_kv <= 0 || n_heads % n_kv != 0 || seen <= SPAN || !takes_tiles(hd, vd, page_size, 0, 0)) return 0;
     const long tiles = count_tiles(n_rows, n_single, n_kv, n_heads / n_kv);
     const long spans = ((long)seen + SPAN - 1) / SPAN + 1;
     if (tiles >= 2L * gi_compute_units() || spans > MAX_SPANS || spans * n_rows * n_heads * part_floats(vd) > (16L << 20)) return 0;
@@ -421,7 +450,7 @@ GI_API int gi_attention_exact(const void* q, int q_dtype, const void* cache, int
     GI_REQUIRE((long)n_rows * n_heads < 2147483647L, "attention_exact: too many (row, head) pairs");
     const unsigned grid = (unsigned)(n_rows * n_heads);
     const auto aligned = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
-    if (q_dtype == GI_F32 && cache_dtype == GI_F32 && out_dtype == GI_F32 && takes_tiles(hd, vd, page_size) && page_stride % 4 == 0 && aligned(q) && aligned(cache)) {
+    if (q_dtype == GI_F32 && cache_dtype == GI_F32 && out_dtype == GI_F32 && takes_tiles(hd, vd, page_size, window, chunk) && page_stride % 4 == 0 && aligned(q) && aligned(cache)) {
         GI_REQUIRE(n_single >= 0 && n_single <= n_rows, "attention_exact: %d single rows of %d", n_single, n_rows);
         const int a_tile = rows_a_tile(n_heads / n_kv), turns = n_single == n_rows ? 1 : n_requests > 0 && n_requests < a_tile ? n_requests : a_tile;
         if (n_spans > 0) {
@@ -430,9 +459,12 @@ GI_API int gi_attention_exact(const void* q, int q_dtype, const void* cache, int
         } else {
             part = nullptr;
         }
+        Divisor pages = {page_size, 0, 0};
+        while ((1LL << pages.shift) < page_size) ++pages.shift;
+        pages.magic = (unsigned)((((1ULL << pages.shift) - page_size) << 32) / page_size + 1);
         const dim3 tiles((unsigned)count_tiles(n_rows, n_single, n_kv, n_heads / n_kv), part ? n_spans : 1, turns);
 #define TILES(D)                                                                                                                           \
-    attention_exact_tiles_kernel<D><<<tiles, 256, 0, stream>>>((const float*)q, (const float*)cache, (float*)out, pos, slot, table, table_stride, page_stride, page_size, n_rows, \
+    attention_exact_tiles_kernel<D><<<tiles, 256, 0, stream>>>((const float*)q, (const float*)cache, (float*)out, pos, slot, table, table_stride, page_stride, pages, n_rows, \
                                                                n_heads, n_kv, hd, vd, window, chunk, scale, cap, sinks, gate, gate_stride, gate_channels, n_single, a_tile, part, n_spans)
         if (hd <= 64 && vd <= 64) TILES(64);
         else TILES(128);

@@ -846,6 +846,33 @@ def test_attention_exact_has_one_order_of_sums(n_heads, n_kv, hd, ps, window, ch
         assert torch.equal(hurt[~sees], whole[~sees]) and not bool(torch.isfinite(hurt[sees]).any())
 
 
+@pytest.mark.parametrize("window,chunk", [(1, None), (16, None), (17, None), (40, None), (None, 1), (None, 16), (None, 17), (None, 48)])
+@pytest.mark.parametrize("n_heads,n_kv,hd,ps", [(4, 2, 64, 16), (3, 1, 128, 12)])
+def test_attention_exact_with_few_keys(n_heads, n_kv, hd, ps, window, chunk):
+    """32-bit: short contexts, and windows and chunks on both sides of the line between the two kernels: groups of 16 keys that no row of a tile sees, at
+    all ends of blocks of 64 and spans of 256; the same bits whatever is known of the step, and alone."""
+    contexts = [600, 70, 18, 1]
+    cache, table, dense = build_paged(contexts, n_kv, hd, ps, torch.float32, seed=hd + n_heads)
+    rows = [(3, 0)] + [(0, p) for p in (0, 14, 15, 16, 17, 47, 48, 63, 64, 65, 79, 255, 256, 257, 271, 272, 300, 511, 512, 599)] + [(1, p) for p in range(50, 70)] + [(2, p) for p in range(18)]
+    pos = torch.tensor([p for _, p in rows], dtype=torch.int32, device=DEV)
+    slots = torch.tensor([s_ + 1 for s_, _ in rows], dtype=torch.int32, device=DEV)
+    q = randn(len(rows), n_heads * hd, seed=3)
+
+    def attend(pick=slice(None), **known):
+        out = torch.full_like(q, float("nan"))[pick]
+        return ops().attention_exact(q[pick].contiguous(), cache, out, pos[pick].contiguous(), slots[pick].contiguous(), table, n_heads, n_kv, hd, window, chunk=chunk, **known)
+
+    lows = [max(0, p - window + 1) if window else p - p % chunk for _, p in rows]
+    want = torch.cat([plain_attention_rows(q[i:i + 1], {s_: (dense[s_][0][lo:], dense[s_][1][lo:])}, [(s_, p - lo)], n_heads, n_kv, hd, None)
+                      for i, ((s_, p), lo) in enumerate(zip(rows, lows))])
+    whole = attend()
+    assert rel(whole, want) < 2e-6
+    for known in (dict(single_rows=21), dict(single_rows=True, max_context=600), dict(n_requests=4, max_context=600)):
+        assert torch.equal(attend(**known), whole), known
+    for i in (0, 4, 12, 20, 25, len(rows) - 1):
+        assert torch.equal(attend(slice(i, i + 1)), whole[i:i + 1])
+
+
 @pytest.mark.parametrize("sinks", [False, True])
 @pytest.mark.parametrize("n_heads,n_kv,hd,ps,window", [(4, 2, 64, 16, None), (6, 1, 128, 4, None), (2, 2, 32, 16, 400)])
 @pytest.mark.parametrize("known", [dict(), dict(max_context=770), dict(single_rows=True), dict(single_rows=True, max_context=770)], ids=["whole", "shared", "single", "single-shared"])
