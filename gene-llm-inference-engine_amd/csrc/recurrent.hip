@@ -433,7 +433,7 @@ template <int ROWS, bool CHANNEL, bool EVERY>
 __global__ __launch_bounds__(64) void delta_scan_kernel(const float* __restrict__ qkv, long ld, const float* __restrict__ gates,
                                                        const int* __restrict__ seg_start, const int* __restrict__ seg_len,
                                                        const int* __restrict__ row_slot, float* __restrict__ state, long state_stride,
-                                                       float* __restrict__ out, long ldo, int n_heads, int n_kv, int dk, int dv) {
+                                                       float* __restrict__ out, long ldo, int n_heads, int n_kv, int dk, int dv, int below) {
     constexpr int C = 4, RG = 16, KQ = RG * ROWS;
     constexpr int TB = (1024 / KQ) < 16 ? (1024 / KQ) : 16;      // tokens staged at a time
     constexpr int PER = TB * KQ / 64, WIDE = EVERY ? 4 : 1;      // (k, q) pairs a lane brings per block, and at a time
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(64) void delta_scan_kernel(const float* __restrict_
     const int seg = blockIdx.x, h = blockIdx.y, vt = blockIdx.z, n_tiles = gridDim.z;
     const int lane = threadIdx.x, c = lane / RG, rg = lane % RG;
     const int n = seg_len[seg];
-    if (n <= 0) return;
+    if (n <= 0 || (below && n >= below)) return;
     const int t0 = seg_start[seg];
     const int col = vt * C + c, kvh = h / (n_heads / n_kv);
     const bool live = col < dv;
@@ -620,6 +620,375 @@ __global__ __launch_bounds__(256) void delta_single_kernel(const float* __restri
     }
 }
 
+// ------------------------------------------------------------------------------------- gated delta rule, a prompt's rows in blocks
+// The same rule for requests that bring many rows (keys of 64 channels, one decay a head).  With d_t the decays, R_ti = d_{i+1} .. d_t and
+// g_t = d_0 .. d_t inside a block of 64 rows, S_0 the memory before it, the rule's updates w_t = s_t (v_t - d_t S_{t-1}^T k_t) are the
+// solution of (1 + A) W = s (V - g K S_0), A_ti = s_t R_ti (k_t . k_i) below the diagonal.  So with U = (1 + A)^-1 s V and P = (1 + A)^-1 s g K,
+// which need no memory,
+//     S_64 = g_63 S_0 + (N - M S_0),     M = K'^T P,  N = K'^T U   (K' the keys times R_63,i)
+//     O    = Q' S_0 + B U,  Q' = g Q - B P,  B_ti = R_ti (q_t . k_i) up to the diagonal
+// and only the first line goes from block to block.  Three kernels: every block's M, N, Q' and B U, all blocks at once; the blocks' memories, one
+// product of 64 x 64 a block; Q' S_0 onto B U, all blocks at once.  What is kept is 32-bit, the products are on the matrix instructions of 16 x 16 x 4.  The places
+// of k in a matrix instruction are chosen so that a lane's four are neighbours (lane group g takes 4 g + v in instruction v): operands leave LDS and
+// memory 16 bytes at a time, and a result as it lies is an operand of the next product.
+// Distance to 64 bits: products of decays, k . k, q . k and the keys' products with U and P are summed in 64 bits (the decays' products alone brought the
+// memories from 1.2 to 2.5 times the scan's distance down to 0.9), the other sums in parts of 8 or 16 terms that meet in a tree, and what a block
+// forgets of a memory is taken off its product with g_63, not multiplied in with it.  1,777 rows: read-outs 1.1e-7 (scan 1.3e-7), memories 0.9e-7 (1.2e-7).
+// A product with a block of zeros would spread a number that is no number to rows before its own: blocks with such an input, and all behind
+// them, go token by token, as does all of a memory that holds one.
+// Bound by the chain of blocks in the second kernel (0.7 us a block) and by a workgroup's matrix instructions and barriers in the first, where it has a compute
+// unit to itself.  1,777 rows of 8 heads of 64 x 128: 28, 25 and 10 us, the scan 203; the rule of choice is `ops.delta_chunks_pay`.
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+constexpr int CHUNK = 64, CHUNK_DK = 64, CHUNK_LD = 68;               // rows of LDS 68 numbers apart: 16 rows' pieces of 16 bytes lie in different banks
+constexpr int CHUNK_WAVES = 12;
+
+// (first row, number of rows) of block `index` among the runs of at least `from` rows; rows 0: there are no so many blocks.
+struct ChunkPlace { int row, rows; };
+__device__ __forceinline__ ChunkPlace chunk_place(const int* __restrict__ seg_start, const int* __restrict__ seg_len, int n_segs, int from, int index) {
+    const int lane = threadIdx.x & 63;
+    for (int s0 = 0; s0 < n_segs; s0 += 64) {
+        const bool there = s0 + lane < n_segs;
+        const int n = there ? seg_len[s0 + lane] : 0, start = there ? seg_start[s0 + lane] : 0, mine = n >= from ? (n + CHUNK - 1) / CHUNK : 0;
+        int sum = mine;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int other = __shfl_up(sum, off, 64);
+            if (lane >= off) sum += other;
+        }
+        const unsigned long long past = __ballot(sum > index);
+        if (past) {
+            const int l = __ffsll(past) - 1, block = index - __shfl(sum - mine, l, 64);
+            return {__shfl(start, l, 64) + block * CHUNK, min(CHUNK, __shfl(n, l, 64) - block * CHUNK)};
+        }
+        index -= __shfl(sum, 63, 64);
+    }
+    return {0, 0};
+}
+// The blocks of the runs before `run`.
+__device__ __forceinline__ int chunks_before(const int* __restrict__ seg_len, int run, int from) {
+    const int lane = threadIdx.x & 63;
+    int sum = 0;
+    for (int s = lane; s < run; s += 64) sum += seg_len[s] >= from ? (seg_len[s] + CHUNK - 1) / CHUNK : 0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+    return sum;
+}
+__device__ __forceinline__ bool no_number(float x) { return !(fabsf(x) <= 3.402823466e38f); }
+__device__ __forceinline__ floatx4 four_of(const float* p) { return *reinterpret_cast<const floatx4*>(p); }
+__device__ __forceinline__ void mfma_four(floatx4 a, floatx4 b, floatx4& acc) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[v], b[v], acc, 0, 0, 0);
+}
+
+// The same in 64 bits.  Result v of a lane is row 4 v + g of the instruction's there: `spread` names the row to give place c, so that it is row 4 g + v as above.
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ int spread(int c) { return 4 * (c & 3) + (c >> 2); }
+__device__ __forceinline__ void mfma_four(floatx4 a, floatx4 b, doublex4& acc) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[v], (double)b[v], acc, 0, 0, 0);
+}
+__device__ __forceinline__ floatx4 mfma_part(floatx4 a, floatx4 b) {
+    floatx4 acc = floatx4{};
+    mfma_four(a, b, acc);
+    return acc;
+}
+
+// Numbers a block and head leave for the kernels behind: M [64][64], N^T [dv][64], Q' [64][64], S_0^T [dv][64], then g_63, whether the
+// block goes token by token (0 or 1), and two unused.
+__host__ __device__ constexpr long chunk_floats(int dv) { return 2L * CHUNK_DK * (CHUNK + dv) + 4; }
+
+// One workgroup per (block, head): a wave takes columns of [V | K], 16 at a time, from the solution to everything made of it.
+__global__ __launch_bounds__(64 * CHUNK_WAVES) void delta_chunk_prepare_kernel(const float* __restrict__ qkv, long ld, const float* __restrict__ gates, const int* __restrict__ seg_start,
+                                                                               const int* __restrict__ seg_len, int n_segs, int from, float* __restrict__ scratch,
+                                                                               float* __restrict__ out, long ldo, int n_heads, int n_kv, int dv) {
+    __shared__ __attribute__((aligned(16))) float Ks[CHUNK][CHUNK_LD], Qs[CHUNK][CHUNK_LD], KT[CHUNK_DK][CHUNK_LD], As[CHUNK][CHUNK_LD], Bs[CHUNK][CHUNK_LD];
+    __shared__ float step_s[CHUNK], since_s[CHUNK], last_s[CHUNK];     // s, g and R_63
+    const int h = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4, n_waves = blockDim.x >> 6;
+    const ChunkPlace at = chunk_place(seg_start, seg_len, n_segs, from, blockIdx.x);
+    if (at.rows <= 0) return;
+    const int n = at.rows, kvh = h / (n_heads / n_kv), v_tiles = dv / 16;
+    const size_t t0 = at.row;
+    const float *q_rows = qkv + t0 * ld + kvh * CHUNK_DK, *k_rows = q_rows + n_kv * CHUNK_DK, *v_rows = qkv + t0 * ld + 2 * n_kv * CHUNK_DK + h * dv;
+    float* mine = scratch + ((size_t)blockIdx.x * n_heads + h) * chunk_floats(dv);
+    float *M = mine, *NT = M + CHUNK_DK * CHUNK_DK, *Qp = NT + (size_t)dv * CHUNK_DK;
+
+    bool bad = false;
+    for (int i = tid; i < CHUNK * CHUNK_DK / 4; i += blockDim.x) {                      // rows behind the run's last: zeros, and decays of 1
+        const int t = i / (CHUNK_DK / 4), d = i % (CHUNK_DK / 4) * 4;
+        floatx4 k = floatx4{}, q = floatx4{};
+        if (t < n) k = four_of(k_rows + (size_t)t * ld + d), q = four_of(q_rows + (size_t)t * ld + d);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) bad |= no_number(k[v]) || no_number(q[v]);
+        *reinterpret_cast<floatx4*>(&Ks[t][d]) = k;
+        *reinterpret_cast<floatx4*>(&Qs[t][d]) = q;
+    }
+    floatx4 x[4];                                                                       // x[I][v]: row 16 I + 4 g + v, column 16 tile + c
+    const auto fetch_values = [&](int tile) {
+#pragma unroll
+        for (int I = 0; I < 4; ++I)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) x[I][v] = v_rows[(size_t)min(16 * I + 4 * g + v, n - 1) * ld + 16 * tile + c];
+    };
+    for (int tile = wave + n_waves; tile < v_tiles; tile += n_waves) {
+        fetch_values(tile);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) bad |= no_number(x[e / 4][e % 4]);
+    }
+    fetch_values(min(wave, v_tiles - 1));                                               // (the wave's first columns stay)
+    if (wave == n_waves - 1) {
+        const float* at_t = gates + (t0 + min(lane, n - 1)) * 2 * n_heads;
+        const float d = lane < n ? at_t[h] : 1.f, s = lane < n ? at_t[n_heads + h] : 0.f;
+        bad |= no_number(d) || no_number(s);
+        // R's column `lane` into B's place, and g: products of up to 64 decays, in 64 bits (their error is that of everything that is kept)
+        double r = 0., since = 1., mine_since = 0.;
+#pragma unroll
+        for (int t = 0; t < CHUNK; ++t) {
+            const double dt = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(d), t));
+            r = t == lane ? 1. : r * dt;
+            since *= dt;
+            mine_since = t == lane ? since : mine_since;
+            Bs[t][lane] = (float)r;
+        }
+        step_s[lane] = s, since_s[lane] = (float)mine_since, last_s[lane] = (float)r;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) bad |= no_number(x[e / 4][e % 4]);
+    bad = __syncthreads_or(bad);
+    if (tid == 0) *reinterpret_cast<float2*>(mine + 2L * CHUNK_DK * (CHUNK + dv)) = float2{since_s[CHUNK - 1], bad ? 1.f : 0.f};
+    if (bad) return;
+    // A and B, 16 x 16 at a time, on and below the diagonal; the keys' transpose
+    for (int block = wave; block < 10; block += n_waves) {
+        const int I = block < 1 ? 0 : block < 3 ? 1 : block < 6 ? 2 : 3, J = block - I * (I + 1) / 2;
+        const auto sums = [&](const float (*rows)[CHUNK_LD]) {
+            doublex4 sum = {};
+#pragma unroll
+            for (int m = 0; m < 4; ++m) mfma_four(four_of(&rows[16 * I + spread(c)][16 * m + 4 * g]), four_of(&Ks[16 * J + c][16 * m + 4 * g]), sum);
+            return floatx4{(float)sum[0], (float)sum[1], (float)sum[2], (float)sum[3]};
+        };
+        const floatx4 k_sum = sums(Ks);
+        __builtin_amdgcn_sched_barrier(0);                                              // (else both sums' parts want registers at once; likewise below)
+        const floatx4 q_sum = sums(Qs);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int t = 16 * I + 4 * g + v, i = 16 * J + c;
+            const float r = Bs[t][i];
+            As[t][i] = t > i ? -(step_s[t] * (r * k_sum[v])) : 0.f;
+            Bs[t][i] = t >= i ? r * q_sum[v] : 0.f;
+        }
+    }
+    for (int i = tid; i < CHUNK * CHUNK_DK; i += blockDim.x) {
+        const int t = i % CHUNK, d = i / CHUNK;
+        KT[d][t] = Ks[t][d] * last_s[t];
+    }
+    __syncthreads();
+    // the inverses of the diagonal's blocks, a column a lane, in place
+    if (wave < 4) {
+        floatx4 row[4];                                                                 // a lane holds row c
+#pragma unroll
+        for (int m = 0; m < 4; ++m) row[m] = four_of(&As[16 * wave + c][16 * wave + 4 * m]);
+        float y[16];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            float sum = t == c ? 1.f : 0.f;
+#pragma unroll
+            for (int i = 0; i < t; ++i) sum = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(row[i / 4][i % 4]), t)), y[i], sum);
+            y[t] = sum;
+        }
+        if (g == 0) {
+#pragma unroll
+            for (int t = 0; t < 16; ++t) As[16 * wave + t][16 * wave + c] = y[t];
+        }
+    }
+    __syncthreads();
+    for (int tile = wave; tile < v_tiles + CHUNK_DK / 16; tile += n_waves) {
+        const bool values = tile < v_tiles;
+        const int col0 = 16 * (values ? tile : tile - v_tiles);
+        if (values && tile != wave) fetch_values(tile);
+#pragma unroll
+        for (int I = 0; I < 4; ++I)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {                                               // (step sizes behind the run's last row are 0)
+                const int t = 16 * I + 4 * g + v;
+                x[I][v] = values ? step_s[t] * x[I][v] : (step_s[t] * since_s[t]) * Ks[t][col0 + c];
+            }
+#pragma unroll
+        for (int I = 0; I < 4; ++I) {
+            floatx4 part = floatx4{};
+#pragma unroll
+            for (int J = 0; J < I; ++J) part += mfma_part(four_of(&As[16 * I + c][16 * J + 4 * g]), x[J]);
+            x[I] = mfma_part(four_of(&As[16 * I + c][16 * I + 4 * g]), x[I] + part);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int r = 0; r < CHUNK_DK / 16; ++r) {
+            doublex4 sum = {};
+            // values: [v] is key channel 16 r + 4 g + v, column col0 + c; keys: column col0 + 4 v + g, key channel 16 r + c
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                const floatx4 k = four_of(&KT[16 * r + (values ? spread(c) : c)][16 * m + 4 * g]);
+                if (values) mfma_four(k, x[m], sum);
+                else mfma_four(x[m], k, sum);
+            }
+            if (values) *reinterpret_cast<floatx4*>(NT + (size_t)(col0 + c) * CHUNK_DK + 16 * r + 4 * g) = floatx4{(float)sum[0], (float)sum[1], (float)sum[2], (float)sum[3]};
+            else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) M[(size_t)(16 * r + c) * CHUNK_DK + col0 + 4 * v + g] = (float)sum[v];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int I = 0; I < 4; ++I) {
+            floatx4 acc = floatx4{};                                                    // acc[v]: column col0 + 4 g + v, row 16 I + c
+#pragma unroll
+            for (int m = 0; m <= I; ++m) acc += mfma_part(x[m], four_of(&Bs[16 * I + c][16 * m + 4 * g]));
+            const int t = 16 * I + c;
+            if (!values) {
+                const floatx4 q = four_of(&Qs[t][col0 + 4 * g]);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[v] = since_s[t] * q[v] - acc[v];
+                *reinterpret_cast<floatx4*>(Qp + (size_t)t * CHUNK_DK + col0 + 4 * g) = acc;
+            } else if (t < n) {
+                *reinterpret_cast<floatx4*>(out + (t0 + t) * ldo + h * dv + col0 + 4 * g) = acc;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
+// The memories from block to block: one workgroup of four waves per (run, head, 16 columns), 16 rows a wave; the blocks' M and N come
+// CHUNK_AHEAD blocks ahead (they were just written by other compute dies and come from beyond the L2: two ahead 1.1 us a block).
+constexpr int CHUNK_AHEAD = 6;
+__global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __restrict__ qkv, long ld, const float* __restrict__ gates, const int* __restrict__ seg_start,
+                                                               const int* __restrict__ seg_len, int from, const int* __restrict__ row_slot, float* __restrict__ state, long state_stride,
+                                                               float* __restrict__ scratch, int* __restrict__ by_token, float* __restrict__ out, long ldo,
+                                                               int n_heads, int n_kv, int dv) {
+    __shared__ __attribute__((aligned(16))) float St[2][16][CHUNK_LD];                  // [column][key channel]
+    const int run = blockIdx.x, h = blockIdx.y, tile = blockIdx.z, n_tiles = gridDim.z;
+    const int n = seg_len[run];
+    if (n < from) return;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
+    const int before = chunks_before(seg_len, run, from), n_chunks = (n + CHUNK - 1) / CHUNK;
+    const size_t t0 = seg_start[run], per = chunk_floats(dv);
+    float* st = state + (size_t)row_slot[t0] * state_stride + ((size_t)h * (dv / 4) + tile * 4) * (CHUNK_DK * 4);       // [four columns][key channel][4]
+    const size_t step = (size_t)n_heads * per;
+    float* base = scratch + ((size_t)before * n_heads + h) * per;
+    const float *M = base + (size_t)(16 * wave + c) * CHUNK_DK + 4 * g;
+    const size_t in_tile = (size_t)(16 * tile + c) * CHUNK_DK + 16 * wave + 4 * g;
+    const float* NT = base + CHUNK_DK * CHUNK_DK + in_tile;
+    float* S0 = base + CHUNK_DK * (2 * CHUNK_DK + (size_t)dv) + in_tile;
+    const float* word = base + 2L * CHUNK_DK * (CHUNK + dv);
+    struct Ahead { floatx4 m[4], n; float since; } ahead[CHUNK_AHEAD];
+    int by_lane = 0;                                       // (a vector load: scalar ones come back in any order, so each would be waited for with the newest)
+    asm volatile("" : "+v"(by_lane));
+    auto fetch = [&](int b, Ahead& x) {
+        const size_t off = min(b, n_chunks - 1) * step;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x.m[i] = four_of(M + off + 16 * i);
+        x.n = four_of(NT + off);
+        x.since = word[off + by_lane];
+    };
+#pragma unroll
+    for (int b = 0; b < CHUNK_AHEAD; ++b) fetch(b, ahead[b]);
+    floatx4 own;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) own[v] = st[((size_t)(c / 4) * CHUNK_DK + 16 * wave + 4 * g + v) * 4 + c % 4];
+    *reinterpret_cast<floatx4*>(&St[0][c][16 * wave + 4 * g]) = own;
+    // the blocks up to the first that goes token by token (found beforehand: with a choice in it the loop would wait for every load in flight)
+    int n_fast = 0;
+    for (bool all = true; all && n_fast < n_chunks;) {
+        const unsigned long long slow = __ballot(n_fast + lane < n_chunks && word[(size_t)min(n_fast + lane, n_chunks - 1) * step + 1] != 0.f);
+        n_fast = min(n_chunks, n_fast + (slow ? __ffsll(slow) - 1 : 64));
+        all = !slow;
+    }
+    if (__syncthreads_or(no_number(own[0]) || no_number(own[1]) || no_number(own[2]) || no_number(own[3]))) n_fast = 0;
+    n_fast = __builtin_amdgcn_readfirstlane(n_fast);
+    for (int b = tid; b < n_chunks; b += 256) by_token[((size_t)(before + b) * n_heads + h) * n_tiles + tile] = b >= n_fast;
+    auto block = [&](int b, Ahead& x) {
+        const int buf = b & 1;
+        *reinterpret_cast<floatx4*>(S0 + b * step) = own;
+        floatx4 part[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part[i] = mfma_part(x.m[i], four_of(&St[buf][c][16 * i + 4 * g]));
+        const floatx4 put = x.n - ((part[0] + part[1]) + (part[2] + part[3]));
+#pragma unroll
+        for (int v = 0; v < 4; ++v) own[v] = fmaf(x.since, own[v], put[v]);
+        *reinterpret_cast<floatx4*>(&St[buf ^ 1][c][16 * wave + 4 * g]) = own;
+        fetch(b + CHUNK_AHEAD, x);
+        barrier_lds();
+    };
+    for (int b = 0;; b += CHUNK_AHEAD) {
+#pragma unroll
+        for (int i = 0; i < CHUNK_AHEAD; ++i) {
+            if (b + i >= n_fast) goto walked;
+            block(b + i, ahead[i]);
+        }
+    }
+walked:
+    if (n_fast < n_chunks) {
+        const int col = tid >> 4, rg = tid & 15, kvh = h / (n_heads / n_kv);
+        float S[4];
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) S[rr] = St[n_fast & 1][col][16 * rr + rg];
+        for (size_t t = t0 + n_fast * CHUNK; t < t0 + n; ++t) {
+            const float* row = qkv + t * ld;
+            DeltaToken<4, false> x;
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) x.kq[rr] = float2{row[(n_kv + kvh) * CHUNK_DK + 16 * rr + rg], row[kvh * CHUNK_DK + 16 * rr + rg]};
+            x.own = float4{gates[t * 2 * n_heads + h], gates[t * 2 * n_heads + n_heads + h], row[2 * n_kv * CHUNK_DK + h * dv + tile * 16 + col],
+                           group_sum<16>(delta_key_query<4, false>(x.kq))};
+            const float y = delta_token<4, false>(S, x);
+            if (rg == 0) out[t * ldo + h * dv + tile * 16 + col] = y;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) St[0][col][16 * rr + rg] = S[rr];
+        __syncthreads();
+        own = four_of(&St[0][c][16 * wave + 4 * g]);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) st[((size_t)(c / 4) * CHUNK_DK + 16 * wave + 4 * g + v) * 4 + c % 4] = own[v];
+}
+
+// Q' S_0 onto the blocks' read-outs: one workgroup per (block, head), a wave per 16 columns.
+__global__ __launch_bounds__(512) void delta_chunk_read_kernel(const int* __restrict__ seg_start, const int* __restrict__ seg_len, int n_segs, int from, const float* __restrict__ scratch,
+                                                               const int* __restrict__ by_token, float* __restrict__ out, long ldo, int n_heads, int dv) {
+    const int h = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4, n_tiles = dv / 16, n_waves = blockDim.x >> 6;
+    const float* mine = scratch + ((size_t)blockIdx.x * n_heads + h) * chunk_floats(dv);
+    const float *Qp = mine + CHUNK_DK * (CHUNK_DK + (size_t)dv), *S0 = Qp + CHUNK * CHUNK_DK;
+    floatx4 s[4], q[4][4];                                 // (asked for before the block's rows are known)
+    const auto fetch = [&](int tile) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m) s[m] = four_of(S0 + (size_t)(16 * tile + c) * CHUNK_DK + 16 * m + 4 * g);
+    };
+    fetch(wave);
+#pragma unroll
+    for (int I = 0; I < 4; ++I)
+#pragma unroll
+        for (int m = 0; m < 4; ++m) q[I][m] = four_of(Qp + (size_t)(16 * I + c) * CHUNK_DK + 16 * m + 4 * g);
+    const ChunkPlace at = chunk_place(seg_start, seg_len, n_segs, from, blockIdx.x);
+    for (int tile = wave; tile < n_tiles && at.rows > 0; tile += n_waves) {
+        if (tile != wave) fetch(tile);
+        const int slow = by_token[((size_t)blockIdx.x * n_heads + h) * n_tiles + tile];
+        floatx4 block[4];
+        float* to[4];
+#pragma unroll
+        for (int I = 0; I < 4; ++I) {
+            to[I] = out + ((size_t)at.row + min(16 * I + c, at.rows - 1)) * ldo + h * dv + 16 * tile + 4 * g;
+            block[I] = four_of(to[I]);
+        }
+#pragma unroll
+        for (int I = 0; I < 4; ++I) {
+            floatx4 part[8] = {};
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) part[2 * m + v / 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[m][v], q[I][m][v], part[2 * m + v / 2], 0, 0, 0);
+            const floatx4 sum = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+            if (16 * I + c < at.rows && !slow) *reinterpret_cast<floatx4*>(to[I]) = sum + block[I];
+        }
+    }
+}
+
 }  // namespace
 
 GI_API int gi_segments(const int* slot, const int* pos, int n_rows, int* seg_start, int* seg_len, int n_segs, hipStream_t stream) {
@@ -700,9 +1069,9 @@ GI_API int gi_delta_tail(const float* proj, long ld, int conv_off, int n_taps, c
 
 // qkv: float32 [n_rows, ld], a row's unit queries [n_kv][dk], unit keys [n_kv][dk], values [n_heads][dv]; gates: float32 [n_rows, 2 n_heads],
 // or [n_rows, n_heads dk + n_heads] with a decay per head and key channel (channel != 0);
-// out: float32 [n_rows, ldo] gets the heads' read-outs [n_heads][dv].
+// out: float32 [n_rows, ldo] gets the heads' read-outs [n_heads][dv].  below > 0: only the runs of fewer rows than that (not with `single`).
 GI_API int gi_delta_scan(const float* qkv, long ld, const float* gates, const int* seg_start, const int* seg_len, int n_segs, const int* row_slot,
-                         float* state, long state_stride, float* out, long ldo, int n_heads, int n_kv, int dk, int dv, int channel, int single, hipStream_t stream) {
+                         float* state, long state_stride, float* out, long ldo, int n_heads, int n_kv, int dk, int dv, int channel, int single, int below, hipStream_t stream) {
     GI_REQUIRE(n_segs > 0 && n_heads > 0 && n_kv > 0 && n_heads % n_kv == 0 && dk > 0 && dk <= 512 && dv > 0, "delta_scan: bad sizes (runs %d, heads %d, kv heads %d, dk %d, dv %d; dk at most 512)",
                n_segs, n_heads, n_kv, dk, dv);
     GI_REQUIRE(ld >= 2L * n_kv * dk + (long)n_heads * dv && ldo >= (long)n_heads * dv && state_stride >= gi_delta_memory_floats(n_heads, dk, dv), "delta_scan: row or state strides too small");
@@ -714,8 +1083,8 @@ GI_API int gi_delta_scan(const float* qkv, long ld, const float* gates, const in
 #define KIND(R, CH)                                                                                                             \
     do {                                                                                                                        \
         if (single) delta_single_kernel<R, CH><<<dim3(n_segs, n_heads, (tiles + 3) / 4), 256, 0, stream>>>(ARGS);               \
-        else if (aligned && dk == 16 * R) delta_scan_kernel<R, CH, true><<<grid, 64, 0, stream>>>(ARGS);                        \
-        else delta_scan_kernel<R, CH, false><<<grid, 64, 0, stream>>>(ARGS);                                                    \
+        else if (aligned && dk == 16 * R) delta_scan_kernel<R, CH, true><<<grid, 64, 0, stream>>>(ARGS, below);                        \
+        else delta_scan_kernel<R, CH, false><<<grid, 64, 0, stream>>>(ARGS, below);                                                    \
     } while (0)
 #define GO(R) do { if (channel) KIND(R, true); else KIND(R, false); } while (0)
     if (dk <= 32) GO(2); else if (dk <= 64) GO(4); else if (dk <= 128) GO(8); else if (dk <= 256) GO(16); else GO(32);
@@ -723,6 +1092,30 @@ GI_API int gi_delta_scan(const float* qkv, long ld, const float* gates, const in
 #undef KIND
 #undef ARGS
     GI_CHECK_LAUNCH("delta_scan");
+    return 0;
+}
+
+// The runs of at least `from` rows, in blocks of 64 (delta_chunk_prepare_kernel); n_chunks: their blocks together.  Keys of 64 channels, one decay a head,
+// values of a multiple of 16 channels, rows of qkv and out at multiples of 16 bytes.  scratch: float32, gi_delta_chunk_floats(n_chunks, n_heads, dv) numbers,
+// at a multiple of 16 bytes.
+GI_API long gi_delta_chunk_floats(int n_chunks, int n_heads, int dv) { return (long)n_chunks * n_heads * (chunk_floats(dv) + dv / 16); }
+GI_API int gi_delta_chunks(const float* qkv, long ld, const float* gates, const int* seg_start, const int* seg_len, int n_segs, int from, int n_chunks, const int* row_slot,
+                           float* state, long state_stride, float* scratch, float* out, long ldo, int n_heads, int n_kv, int dv, hipStream_t stream) {
+    GI_REQUIRE(n_segs > 0 && n_heads > 0 && n_kv > 0 && n_heads % n_kv == 0 && dv > 0 && dv % 16 == 0 && from > 0 && n_chunks > 0,
+               "delta_chunks: bad sizes (runs %d, heads %d, kv heads %d, dv %d, from %d rows, %d blocks)", n_segs, n_heads, n_kv, dv, from, n_chunks);
+    GI_REQUIRE(ld >= 2L * n_kv * CHUNK_DK + (long)n_heads * dv && ldo >= (long)n_heads * dv && state_stride >= gi_delta_memory_floats(n_heads, CHUNK_DK, dv),
+               "delta_chunks: row or state strides too small");
+    GI_REQUIRE(ld % 4 == 0 && ldo % 4 == 0 && (((uintptr_t)qkv | (uintptr_t)out | (uintptr_t)scratch) & 15) == 0, "delta_chunks: rows must lie at multiples of 16 bytes");
+    GI_REQUIRE(n_heads <= 65535 && dv / 16 <= 65535, "delta_chunks: too many heads or value channels");
+    int* by_token = (int*)(scratch + (long)n_chunks * n_heads * chunk_floats(dv));
+    const int tiles = dv / 16, waves = tiles + CHUNK_DK / 16 < CHUNK_WAVES ? tiles + CHUNK_DK / 16 : CHUNK_WAVES;
+    delta_chunk_prepare_kernel<<<dim3(n_chunks, n_heads), 64 * waves, 0, stream>>>(qkv, ld, gates, seg_start, seg_len, n_segs, from, scratch, out, ldo, n_heads, n_kv, dv);
+    GI_CHECK_LAUNCH("delta_chunks");
+    delta_chunk_scan_kernel<<<dim3(n_segs, n_heads, tiles), 256, 0, stream>>>(qkv, ld, gates, seg_start, seg_len, from, row_slot, state, state_stride, scratch, by_token, out, ldo,
+                                                                              n_heads, n_kv, dv);
+    GI_CHECK_LAUNCH("delta_chunks");
+    delta_chunk_read_kernel<<<dim3(n_chunks, n_heads), 64 * (tiles < 8 ? tiles : 8), 0, stream>>>(seg_start, seg_len, n_segs, from, scratch, by_token, out, ldo, n_heads, dv);
+    GI_CHECK_LAUNCH("delta_chunks");
     return 0;
 }
 

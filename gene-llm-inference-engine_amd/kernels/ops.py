@@ -72,7 +72,8 @@ _SIGNATURES = {
     "gi_delta_prepare": [c_void_p, c_long, c_int, c_void_p, c_long, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p,
                          c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p],
     "gi_delta_tail": [c_void_p, c_long, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_int, c_void_p],
-    "gi_delta_scan": [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_long, c_void_p, c_long, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+    "gi_delta_scan": [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_long, c_void_p, c_long, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+    "gi_delta_chunks": [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_void_p],
     "gi_latent_prepare": [c_void_p, c_long, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_float, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                           c_void_p, c_int, c_long, c_void_p, c_int, c_long, c_int, c_int, c_int, c_void_p],
     "gi_heads_product": [c_void_p, c_long, c_void_p, c_void_p, c_int, c_long, c_long, c_int, c_int, c_int, c_int, c_void_p, c_long, c_void_p],
@@ -161,6 +162,8 @@ def lib():
         l.gi_gemm_bf16_qkv_rope_store_max_parts.restype = c_int
         l.gi_mlstm_state_floats.argtypes = [c_int, c_int, c_int]
         l.gi_mlstm_state_floats.restype = c_long
+        l.gi_delta_chunk_floats.argtypes = [c_int, c_int, c_int]
+        l.gi_delta_chunk_floats.restype = c_long
         l.gi_mlstm_max_key_dim.argtypes = []
         l.gi_mlstm_max_key_dim.restype = c_int
         l.gi_latent_attention_supports.argtypes = [c_int, c_int, c_int]
@@ -1003,13 +1006,15 @@ def delta_tail(proj, conv_off, n_taps, seg_start, seg_len, row_slot, state, n_he
           state.data_ptr(), state.stride(0), n_heads, n_kv, dk, dv, _stream())
 
 
-def delta_scan(qkv, gates, seg_start, seg_len, row_slot, state, out, n_heads, n_kv, dk, dv, channel=False, single_rows=False):
+def delta_scan(qkv, gates, seg_start, seg_len, row_slot, state, out, n_heads, n_kv, dk, dv, channel=False, single_rows=False, below=0):
     """The gated delta rule over every request's rows of the step, in order (csrc/recurrent.hip states it): qkv and gates as
     `delta_prepare` leaves them, out float32 [n, heads*dv] gets the read-outs M^T q; the memories come from the request's state
     slot and go back into it.  channel: the decays are one per head and key channel.  single_rows: every request of the step has one row
-    (a kernel without staging; the same bits)."""
+    (a kernel without staging; the same bits).  below: only requests of fewer rows than that (0: all; `delta_chunks` serves the others)."""
     _dev(qkv, gates, seg_start, seg_len, row_slot, state, out)
     n = qkv.shape[0]
+    if single_rows and below:
+        raise KernelError("delta_scan: single rows are not parted by their number")
     if not (qkv.dtype == torch.float32 and qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.shape[1] >= 2 * n_kv * dk + n_heads * dv and gates.dtype == torch.float32
             and gates.shape == (n, n_heads * (dk + 1 if channel else 2)) and gates.is_contiguous() and out.dtype == torch.float32 and out.shape == (n, n_heads * dv)
             and out.stride(1) == 1):
@@ -1023,7 +1028,53 @@ def delta_scan(qkv, gates, seg_start, seg_len, row_slot, state, out, n_heads, n_
     _i32(seg_len, "delta_scan: seg_len", n_segs)
     _i32(row_slot, "delta_scan: slots", n)
     _call("gi_delta_scan", qkv.data_ptr(), qkv.stride(0), gates.data_ptr(), seg_start.data_ptr(), seg_len.data_ptr(), n_segs, row_slot.data_ptr(), state.data_ptr(),
-          state.stride(0), out.data_ptr(), out.stride(0), n_heads, n_kv, dk, dv, 1 if channel else 0, 1 if single_rows else 0, _stream())
+          state.stride(0), out.data_ptr(), out.stride(0), n_heads, n_kv, dk, dv, 1 if channel else 0, 1 if single_rows else 0, int(below), _stream())
+    return out
+
+
+DELTA_CHUNK = 64
+
+
+def delta_chunks_serve(dk, dv, channel) -> bool:
+    """Whether `delta_chunks` takes memories of these sizes."""
+    return dk == 64 and dv % 16 == 0 and not channel
+
+
+def delta_chunks_pay(rows_per_request, least, n_heads) -> bool:
+    """Whether a step's long requests go faster in blocks.  The scan takes 3 us and 0.115 us a row of the longest request, the blocks 38 us, 0.014 us a row
+    and 32 us for every round of workgroups (one per block and head, one to a compute unit) behind the first.  Microseconds, scan / blocks, heads of 64 x 128: 8
+    heads and one request of 256, 384, 512, 2,048 rows 32 / 42, 46 / 44, 61 / 46, 237 / 66; 32 heads, 512 and 2,048 rows 69 / 51, 251 / 161, two of 1,000
+    168 / 164, eight of 200 143 / 191."""
+    longest = max(rows_per_request)
+    if longest < 350:
+        return False
+    blocks = sum(-(-m // DELTA_CHUNK) for m in rows_per_request if m >= least)
+    return 0.1 * longest > 35 + 32 * (-(-blocks * n_heads // lib().gi_compute_units()) - 1)
+
+
+def delta_chunks(qkv, gates, seg_start, seg_len, rows_per_request, least, row_slot, state, out, n_heads, n_kv, dk, dv):
+    """`delta_scan` for the requests of at least `least` rows, 64 rows at a time on the 32-bit matrix instructions (csrc/recurrent.hip states it; sums in
+    another order than the scan's, no further from 64 bits).  rows_per_request: the numbers in seg_len, on the host."""
+    _dev(qkv, gates, seg_start, seg_len, row_slot, state, out)
+    n, n_segs = qkv.shape[0], seg_start.numel()
+    if not (qkv.dtype == torch.float32 and qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.shape[1] >= 2 * n_kv * dk + n_heads * dv and gates.dtype == torch.float32
+            and gates.shape == (n, n_heads * 2) and gates.is_contiguous() and out.dtype == torch.float32 and out.shape == (n, n_heads * dv) and out.stride(1) == 1):
+        raise KernelError("delta_chunks: qkv must be float32 [n, channels], gates float32 [n, 2 heads], out float32 [n, heads*dv]")
+    if not (state.dtype == torch.float32 and state.dim() == 2 and state.stride(1) == 1 and state.shape[1] >= delta_memory_floats(n_heads, dk, dv)):
+        raise KernelError("delta_chunks: state must be float32 [slots, at least delta_memory_floats]")
+    if not (delta_chunks_serve(dk, dv, False) and n_heads % n_kv == 0):
+        raise KernelError("delta_chunks: keys of 64 channels, values of a multiple of 16 and heads in whole groups are served")
+    if len(rows_per_request) != n_segs or least < 1:
+        raise KernelError("delta_chunks: one number of rows per request, and at least one row")
+    _i32(seg_start, "delta_chunks: seg_start", n_segs)
+    _i32(seg_len, "delta_chunks: seg_len", n_segs)
+    _i32(row_slot, "delta_chunks: slots", n)
+    blocks = sum(-(-m // DELTA_CHUNK) for m in rows_per_request if m >= least)
+    if blocks == 0:
+        return out
+    scratch = torch.empty(lib().gi_delta_chunk_floats(blocks, n_heads, dv), dtype=torch.float32, device=out.device)
+    _call("gi_delta_chunks", qkv.data_ptr(), qkv.stride(0), gates.data_ptr(), seg_start.data_ptr(), seg_len.data_ptr(), n_segs, int(least), blocks, row_slot.data_ptr(),
+          state.data_ptr(), state.stride(0), scratch.data_ptr(), out.data_ptr(), out.stride(0), n_heads, n_kv, dv, _stream())
     return out
 
 

@@ -4,7 +4,7 @@ One product with the stacked matrix [q; k; v; output gate; a; b] gives the 32-bi
 makes of them what the rule reads: q, k and v through their short convolutions (a request's rows before this step come from
 its state) and SiLU, q and k as unit vectors, the decays and step sizes.  One kernel keeps every request's last rows for the
 next step's convolutions (in a step of single rows the kernel before it does that on its way).  One kernel steps the memories over every request's rows, in order, from the request's state slot
-and back into it.  One kernel divides every head's read-out by its root mean square, multiplies by the norm's weights and by
+and back into it (in bfloat16 a long prompt's rows in blocks of 64, three kernels).  One kernel divides every head's read-out by its root mean square, multiplies by the norm's weights and by
 SiLU of the output gate, and stores the rows as the output product reads them.  Everything between the projections and the
 output product is 32-bit, whatever the compute dtype.
 
@@ -33,6 +33,8 @@ class GatedDelta(Mixer):
     hands_norm_on = True              # `forward` takes `then`, the norm that reads the residual next
     can_overwrite = True
     FEW_ROWS = 16                     # up to so many rows (bfloat16) the products behind the narrow middles are made inside the kernels that need them
+
+    ROWS_IN_BLOCKS = 65               # requests of so many rows go through the rule in blocks where a step's long requests make that the faster way
 
     def takes_handed_norm(self, n_rows: int) -> bool:
         return self.in_dtype == torch.bfloat16 and takes_handed_norm(self.w_in, n_rows)
@@ -84,6 +86,7 @@ class GatedDelta(Mixer):
         self.w_o = tensors[s.o_proj]
         self.in_dtype = activation_dtype_for(self.w_in, dtype)
         self.mid_dtype = activation_dtype_for(self.w_o, dtype)
+        self.in_blocks = dtype == torch.bfloat16 and ops.delta_chunks_serve(s.key_dim, s.value_dim, s.channel_decay)    # (32-bit: bits that do not depend on the cut)
 
     def weights_read_per_step(self):
         return [self.w_in, self.taps, self.a_log, self.dt_bias, self.out_norm, self.w_o] + ([w for w in (self.w_a_up, self.w_g_up) if w is not None] if self.w_low is not None else [])
@@ -143,7 +146,11 @@ class GatedDelta(Mixer):
         if not single_rows:
             ops.delta_tail(proj, o["conv"], s.conv_taps, seg_start, seg_len, ctx.row_slot, cache.state, H, G, dk, dv)
         read = torch.empty((T, vv), dtype=torch.float32, device=dev)
-        ops.delta_scan(qkv, gates, seg_start, seg_len, ctx.row_slot, cache.state, read, H, G, dk, dv, s.channel_decay, single_rows)
+        chunked = self.in_blocks and ops.delta_chunks_pay(ctx.seg_len, self.ROWS_IN_BLOCKS, H)
+        if chunked:
+            ops.delta_chunks(qkv, gates, seg_start, seg_len, ctx.seg_len, self.ROWS_IN_BLOCKS, ctx.row_slot, cache.state, read, H, G, dk, dv)
+        if not chunked or min(ctx.seg_len) < self.ROWS_IN_BLOCKS:
+            ops.delta_scan(qkv, gates, seg_start, seg_len, ctx.row_slot, cache.state, read, H, G, dk, dv, s.channel_decay, single_rows, self.ROWS_IN_BLOCKS if chunked else 0)
         mid = torch.empty((T, vv), dtype=self.mid_dtype, device=dev)
         ops.head_norm_gate(read, gate, self.out_norm, s.norm_eps, mid, H, dv, gate_activation=s.gate_activation, gate_up=gate_up)
         if overwrite:

@@ -257,6 +257,92 @@ def test_delta_rule_sums_in_one_order(heads, kv, dk, dv, spare, channel):
     assert torch.equal(one, out[21:22]) and torch.equal(one_state[0], state[0])
 
 
+def _delta_inputs(lens, heads, kv, dv, seed, steps=None, spare=0):
+    """Rows as `delta_prepare` leaves them: unit keys, queries of length 1/8, decays as at initialisation, and where given one step size for all."""
+    g = torch.Generator().manual_seed(seed)
+    n, dk = sum(lens), 64
+    qkv = torch.nn.functional.silu(0.5 * torch.randn(n, 2 * kv * dk + heads * dv + spare, generator=g))
+    unit = qkv[:, :2 * kv * dk].view(n, 2 * kv, dk)
+    unit /= unit.norm(dim=2, keepdim=True)
+    qkv[:, :kv * dk] *= dk ** -0.5
+    size = torch.exp(torch.rand(heads, generator=g) * 4.6 - 6.9)
+    decay = torch.exp(-(1 + 15 * torch.rand(heads, generator=g)) * torch.nn.functional.softplus(torch.log(torch.expm1(size)) + 0.5 * torch.randn(n, heads, generator=g)))
+    step = torch.sigmoid(torch.randn(n, heads, generator=g)) if steps is None else torch.full((n, heads), steps)
+    return qkv, torch.cat([decay, step], 1)
+
+
+@pytest.mark.parametrize("lens, least, heads, kv, dv, spare, steps", [([1777], 65, 8, 4, 128, 0, None), ([200, 3, 64, 65, 129], 65, 4, 2, 128, 4, None), ([128, 1], 64, 3, 1, 16, 0, None),
+                                                                      ([66] * 70, 1, 2, 2, 48, 0, None), ([1, 63, 64, 2], 1, 2, 1, 208, 12, None), ([500], 65, 2, 1, 64, 0, 1.0)])
+def test_delta_rule_in_blocks(lens, least, heads, kv, dv, spare, steps):
+    """Blocks of 64 rows against the rule in 64 bits and against the scan, whose distance to it the blocks may not exceed by more than rounding's own
+    spread; runs below `least` are left alone."""
+    from geneinfer_amd.kernels import ops
+    dk, n, tiles = 64, sum(lens), dv // 4
+    qkv, gates = _delta_inputs(lens, heads, kv, dv, dv + n, steps, spare)
+    starts = [sum(lens[:i]) for i in range(len(lens))]
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    slots = list(range(len(lens)))[::-1]
+    rows = (qkv.to(DEV), gates.to(DEV), ints(starts), ints(lens))
+    slot = ints([s for s, m in zip(slots, lens) for _ in range(m)])
+    first = 0.2 * torch.randn(len(lens), heads, tiles, dk, 4, generator=torch.Generator().manual_seed(n))
+    state, out = first.clone().view(len(lens), -1).to(DEV), torch.full((n, heads * dv), 7.0, device=DEV)
+    ops.delta_chunks(*rows, lens, least, slot, state, out, heads, kv, dk, dv)
+    scan_state, scan = first.clone().view(len(lens), -1).to(DEV), torch.full((n, heads * dv), 7.0, device=DEV)
+    ops.delta_scan(*rows, slot, scan_state, scan, heads, kv, dk, dv)
+    below_state, below = first.clone().view(len(lens), -1).to(DEV), torch.full((n, heads * dv), 7.0, device=DEV)
+    ops.delta_scan(*rows, slot, below_state, below, heads, kv, dk, dv, below=least)
+    far = lambda x, y, want: (float((x.double() - want).norm() / want.norm()), float((y.double() - want).norm() / want.norm()))
+    for at, m, s in zip(starts, lens, slots):
+        if m < least:
+            assert torch.all(out[at:at + m] == 7.0) and torch.equal(state[s].cpu(), first[s].view(-1))
+            assert torch.equal(below[at:at + m], scan[at:at + m]) and torch.equal(below_state[s], scan_state[s])
+            continue
+        assert torch.all(below[at:at + m] == 7.0) and torch.equal(below_state[s].cpu(), first[s].view(-1))
+        M = first[s].permute(0, 2, 1, 3).reshape(heads, dk, dv).double()
+        x, e = qkv[at:at + m].double(), gates[at:at + m].double()
+        q, k = (x[:, i * kv * dk:(i + 1) * kv * dk].view(m, kv, dk).repeat_interleave(heads // kv, 1) for i in (0, 1))
+        v, want = x[:, 2 * kv * dk:2 * kv * dk + heads * dv].view(m, heads, dv), torch.empty(m, heads, dv, dtype=torch.float64)
+        for t in range(m):
+            M = M * e[t, :heads, None, None]
+            M = M + k[t][:, :, None] * (e[t, heads:, None] * (v[t] - torch.matmul(k[t][:, None], M)[:, 0]))[:, None]
+            want[t] = torch.matmul(q[t][:, None], M)[:, 0]
+        ours, scans = far(out[at:at + m].cpu(), scan[at:at + m].cpu(), want.view(m, -1))
+        held, scan_held = far(*(y[s].view(heads, tiles, dk, 4).permute(0, 2, 1, 3).reshape(heads, dk, dv).cpu() for y in (state, scan_state)), M)
+        print(f"{m} rows, {heads} heads, dv {dv}: read-outs {ours:.2e} (scan {scans:.2e}), memories {held:.2e} (scan {scan_held:.2e})", flush=True)
+        # (2e-8: a third of a rounding, what two orders of the same sums differ by in their distance over one or two rows)
+        assert ours < 1.2 * scans + 2e-8 and held < 1.2 * scan_held + 2e-8
+
+
+@pytest.mark.parametrize("what, value", [("k", float("nan")), ("v", float("inf")), ("decay", float("nan")), ("q", float("-inf")), ("memory", float("nan"))])
+def test_delta_rule_in_blocks_with_no_numbers(what, value):
+    """A number that is none reaches what it reaches in the scan: its own row and the rows behind it, of its own head and columns."""
+    from geneinfer_amd.kernels import ops
+    lens, heads, kv, dk, dv = [300, 130], 4, 2, 64, 32
+    qkv, gates = _delta_inputs(lens, heads, kv, dv, 5)
+    state = torch.zeros(2, ops.delta_memory_floats(heads, dk, dv))
+    if what == "memory":
+        state[0, 70] = value
+    elif what == "decay":
+        gates[100, 1] = value
+    else:
+        qkv[100, {"q": 5, "k": kv * dk + 5, "v": 2 * kv * dk + dv + 3}[what]] = value
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    slot = ints([0] * 300 + [1] * 130)
+    got = []
+    for blocks in (True, False):
+        st, out = state.clone().to(DEV), torch.empty(sum(lens), heads * dv, device=DEV)
+        if blocks:
+            ops.delta_chunks(qkv.to(DEV), gates.to(DEV), ints([0, 300]), ints(lens), lens, 65, slot, st, out, heads, kv, dk, dv)
+        else:
+            ops.delta_scan(qkv.to(DEV), gates.to(DEV), ints([0, 300]), ints(lens), slot, st, out, heads, kv, dk, dv)
+        got.append((out.cpu(), st.cpu()[:, :state.shape[1]]))
+    assert not bool(torch.isfinite(got[1][0]).all())
+    for ours, scans in zip(*got):
+        assert torch.equal(torch.isfinite(ours), torch.isfinite(scans)) and torch.equal(ours.isnan(), scans.isnan())
+        keep = torch.isfinite(scans)
+        assert relative_error(ours[keep].double(), scans[keep].double()) < 2e-6
+
+
 def test_delta_rule_takes_very_wide_values():
     """More tiles of four value channels than half of what a launch's third dimension holds."""
     from geneinfer_amd.kernels import ops
