@@ -704,17 +704,43 @@ __device__ __forceinline__ uint4 rotated8(const Pairs8& p, const Angles8& u) {
     return uint4{w[0], w[1], w[2], w[3]};
 }
 
+// Which (place in the list of rows, group of heads, split) a workgroup takes.  units > 0: the list holds the longest contexts first, and workgroups, which
+// go to the `units` compute units in turn, take its items there and back: the unit that has one of the longest in one round has one of the shortest in the next.
+struct DecodeItem { int row, heads, split; };
+__device__ __forceinline__ DecodeItem decode_item(int units) {
+    if (units <= 0) return {(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z};
+    const unsigned each = gridDim.y * gridDim.z, total = gridDim.x * each, at = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    const unsigned round = at / units, first = round * units, behind = min(first + units, total);
+    const unsigned item = round & 1 ? behind - 1 - (at - first) : at, rest = item % each;
+    return {(int)(item / each), (int)(rest % gridDim.y), (int)(rest / gridDim.y)};
+}
+
+// The rows (`rows`, or 0 .. n - 1) with the longest contexts first; equal ones in their order.  One workgroup, a row a thread.
+constexpr int ORDER_MAX_ROWS = 1024;
+__global__ __launch_bounds__(ORDER_MAX_ROWS) void decode_order_kernel(const int* __restrict__ pos, const int* __restrict__ rows, int n, int* __restrict__ order) {
+    __shared__ int length[ORDER_MAX_ROWS];
+    const int i = threadIdx.x, row = i < n ? (rows ? rows[i] : i) : 0, mine = i < n ? pos[row] : 0;
+    length[i] = mine;
+    __syncthreads();
+    if (i >= n) return;
+    int before = 0;
+#pragma unroll 8
+    for (int j = 0; j < n; ++j) before += length[j] > mine || (length[j] == mine && j < i);
+    order[before] = row;
+}
+
 template <int HD, bool FUSED, bool CAP>
 __global__ __launch_bounds__(64 * DecodeShape<HD>::MAX_WAVES) void attention_decode_kernel(
     const bf16_t* __restrict__ q, const float* __restrict__ qf, const float* __restrict__ kf, const float* __restrict__ vf, long ldq, long ldk,
     long ldv, const float* __restrict__ cos_t, const float* __restrict__ sin_t, bf16_t* __restrict__ cache, float* __restrict__ part,
     bf16_t* __restrict__ out, const int* __restrict__ rows, const int* __restrict__ pos, const int* __restrict__ slots,
     const int* __restrict__ table, int table_stride, long page_stride, int page_size, int n_heads, int n_kv, int window, float scale,
-    int n_splits, int gh, Extras extra) {
+    int n_splits, int gh, int units, Extras extra) {
     constexpr int KSTEPS = HD / 32, DT = HD / 16;
     extern __shared__ float merged[];                        // [wave][gh][HD + 2]
     const int group = n_heads / n_kv, hg_per_kv = (group + 15) / 16;
-    const int row = rows ? rows[blockIdx.x] : blockIdx.x, g = blockIdx.y / hg_per_kv, hg = blockIdx.y % hg_per_kv, split = blockIdx.z;
+    const DecodeItem item = decode_item(units);
+    const int row = rows ? rows[item.row] : item.row, g = item.heads / hg_per_kv, hg = item.heads % hg_per_kv, split = item.split;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n_waves = blockDim.x >> 6;
     const int r = lane & 15, q4 = lane >> 4;
     const int head_in_group = hg * 16 + r;
@@ -979,7 +1005,7 @@ __global__ __launch_bounds__(64 * DecodeShape<HD>::MAX_WAVES) void attention_dec
         if (n_splits == 1) {
             out[((size_t)row * n_heads + out_head) * HD + d] = f32_to_bf16(acc / denom * gate_of(extra, (size_t)row, out_head) * channel_gate_of(extra, (size_t)row, out_head, d));
         } else {                                             // part[row_index][head][split] = {m, l, O[HD]}
-            float* dst = part + (((size_t)blockIdx.x * n_heads + out_head) * n_splits + split) * (HD + 2);
+            float* dst = part + (((size_t)item.row * n_heads + out_head) * n_splits + split) * (HD + 2);
             if (d == 0) {
                 dst[0] = big;
                 dst[1] = denom;
@@ -1181,12 +1207,13 @@ GI_API int gi_attention_decode_workgroups_per_unit(int hd, int fused, int n_wave
 // `kf`, `vf` hold the unrotated 32-bit products, `cos_t`/`sin_t` the rotation (or null for none),
 // and the kernel rotates, attends and writes the new keys and values to the cache itself (`kf`
 // null: the pages belong to another layer and hold them already).  `n_waves` pieces per workgroup,
-// `n_splits` workgroups per row and head group; `part` is needed for n_splits > 1.
+// `n_splits` workgroups per row and head group; `part` is needed for n_splits > 1.  ordered: `rows` has the longest contexts first (gi_decode_order),
+// and the workgroups share them out evenly over the compute units.
 GI_API int gi_attention_decode_bf16(const void* q, const float* qf, const float* kf, const float* vf, long ldq, long ldk, long ldv,
                                     const float* cos_t, const float* sin_t, void* cache, void* out, float* part, long part_floats,
                                     const int* rows, int n_rows, const int* pos, const int* slots, const int* table, int table_stride,
                                     long page_stride, int page_size, int n_heads, int n_kv, int hd, int window, float scale, int n_splits,
-                                    int n_waves, int chunk, const float* sinks, const float* gate, long gate_stride, int gate_channels, float cap,
+                                    int n_waves, int ordered, int chunk, const float* sinks, const float* gate, long gate_stride, int gate_channels, float cap,
                                     hipStream_t stream) {
     GI_REQUIRE(chunk >= 0 && cap >= 0.f && (gate_channels == 0 || gate_channels == hd) && (gate == nullptr || gate_stride >= (long)n_heads * (gate_channels ? hd : 1)) &&
                    (gate == nullptr || gate_channels == 0 || (gate_stride % 4 == 0 && ((uintptr_t)gate & 15) == 0)),
@@ -1219,11 +1246,13 @@ GI_API int gi_attention_decode_bf16(const void* q, const float* qf, const float*
     GI_REQUIRE(lds <= 64 * 1024, "attention_decode: %d heads of size %d per key/value head do not fit", gh, hd);
     lds = decode_lds_bytes(hd, n_waves, gh);
     dim3 grid(n_rows, n_kv * hg, n_splits);
+    GI_REQUIRE(!ordered || (rows != nullptr && (long)n_rows * n_kv * hg * n_splits < 2147483647L), "attention_decode: an order needs its rows, and fewer workgroups");
+    const int units = ordered ? gi_compute_units() : 0;
 #define GO2(HD, FUSED_, CAP_)                                                                                                              \
     attention_decode_kernel<HD, FUSED_, CAP_><<<grid, 64 * n_waves, lds, stream>>>((const bf16_t*)q, qf, kf, vf, ldq, ldk, ldv, cos_t, sin_t, \
                                                                                    (bf16_t*)cache, part, (bf16_t*)out, rows, pos, slots, table, \
                                                                                    table_stride, page_stride, page_size, n_heads, n_kv, window, \
-                                                                                   scale, n_splits, gh, extra)
+                                                                                   scale, n_splits, gh, units, extra)
     GI_REQUIRE(!(qf && extra.cap > 0.f), "attention_decode: capped scores are not served from unrotated products");
 #define GO(HD)                                         \
     do {                                               \
@@ -1240,5 +1269,13 @@ GI_API int gi_attention_decode_bf16(const void* q, const float* qf, const float*
         attention_decode_combine_kernel<<<cgrid, 64, 0, stream>>>(part, (bf16_t*)out, rows, n_heads, hd, n_splits, extra);
         GI_CHECK_LAUNCH("attention_decode (combine)");
     }
+    return 0;
+}
+
+// order [n] gets the rows (`rows`, or 0 .. n - 1) with the longest contexts first, for gi_attention_decode_bf16.
+GI_API int gi_decode_order(const int* pos, const int* rows, int n, int* order, hipStream_t stream) {
+    GI_REQUIRE(n > 0 && n <= ORDER_MAX_ROWS && order != nullptr && order != rows, "decode_order: %d rows (at most %d), into a list of its own", n, ORDER_MAX_ROWS);
+    decode_order_kernel<<<1, (n + 63) / 64 * 64, 0, stream>>>(pos, rows, n, order);
+    GI_CHECK_LAUNCH("decode_order");
     return 0;
 }

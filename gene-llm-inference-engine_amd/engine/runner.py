@@ -527,7 +527,7 @@ class _StepGraph:
         if plan.n_tiles:
             plan.max_tile_context = self.bracket
         if plan.n_decode:
-            plan.max_decode_context = self.bracket
+            plan.max_decode_context, plan.decode_positions = self.bracket, None
         m = self.model
         meta_dev = self._view(0).view(3, self.n_rows)
         ctx = StepContext(n_rows=self.n_rows, dtype=m.dtype, device=m.device, tokens=meta_dev[0], row_pos=meta_dev[1], row_slot=meta_dev[2],

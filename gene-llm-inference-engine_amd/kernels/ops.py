@@ -104,7 +104,8 @@ _SIGNATURES = {
                                  c_float, c_int, c_void_p, c_void_p, c_int, c_void_p, c_long, c_int, c_void_p, c_void_p, c_long, c_int, c_float, c_void_p],
     "gi_attention_decode_bf16": [c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_long, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                  c_long, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int,
-                                 c_float, c_int, c_int, c_int, c_void_p, c_void_p, c_long, c_int, c_float, c_void_p],
+                                 c_float, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_long, c_int, c_float, c_void_p],
+    "gi_decode_order": [c_void_p, c_void_p, c_int, c_void_p, c_void_p],
     "gi_random_normal": [c_void_p, c_int, c_long, ctypes.c_ulonglong, ctypes.c_double, ctypes.c_double, c_void_p],
     "gi_probe_stream": [c_void_p, c_void_p, c_long, c_void_p, c_int, c_int, c_void_p],
     "gi_probe_mfma": [c_int, c_void_p, c_int, c_void_p],
@@ -1167,12 +1168,14 @@ class AttentionPlan:
         plan = cls.__new__(cls)
         plan.n_decode, plan.n_tiles, plan.max_decode_context, plan.single_rows = n_rows, 0, max_context, True
         plan.decode_rows = None                                  # rows 0 .. n_rows-1
+        plan.decode_positions = None
         plan.tiles = torch.empty(0, dtype=torch.int32, device=device)
         plan.n_tile_rows, plan.max_tile_context, plan.tile_first, plan.tile_rows, plan.paired, plan.tile = 0, 0, None, None, False, 128
         return plan
 
     def __init__(self, seg_start, seg_len, seg_pos0, seg_slot, device, to_device=None):
         dec, tiles, portions, self.max_decode_context = [], [], [], 0
+        self.decode_positions = 0            # positions that the single rows see together; None: of a step still to come
         short_rows = sum(n for n in seg_len if 1 < n <= self.SHORT)
         row_by_row = self.SHORT if short_rows <= self.SHORT_TOTAL else 1
         self.single_rows = all(n == 1 for n in seg_len)          # every row is a request's only new row
@@ -1181,6 +1184,7 @@ class AttentionPlan:
             if n <= row_by_row:
                 dec.extend(range(start, start + n))
                 self.max_decode_context = max(self.max_decode_context, pos0 + n)
+                self.decode_positions += n * pos0 + n * (n + 1) // 2
             else:
                 portions.append([(start + off, min(self.tile, n - off), pos0 + off, slot) for off in range(0, n, self.tile)])
         # Tile i of a portion sees the keys of the tiles before it: the last tile goes with the first, the last but
@@ -1275,6 +1279,23 @@ def _decode_single_split(groups, span, hd, max_waves):
     return (1, min(n_waves, max_waves))
 
 
+def _decode_ragged_split(groups, longest, mean, hd, n_waves):
+    """(splits, waves) for contexts whose lengths are known, where the plain rule cuts none: one workgroup per (row, group of heads) takes the time of the
+    longest context; cut in two or more and dealt out there and back (`_decode_order`), the compute units share the bytes more evenly, for the merge.  24
+    rows of 8 groups of 128 channels at 380 to 3,000 positions beside a prompt's portions: 44.6 -> 35.3 us a layer and 5 for the merge (expected: 49.5 and
+    34; so it has to promise a fifth)."""
+    units, row_mb = lib().gi_compute_units(), hd * 4 / 1e6
+    even_us = max(groups * mean * row_mb / units / _DECODE_SHARED_UNIT_MB_PER_S, groups * mean * row_mb / _DECODE_CHIP_MB_PER_S) * 1e6
+    best, best_us = (1, n_waves), 0.8 * max(even_us, longest * row_mb / _DECODE_UNIT_MB_PER_S * 1e6)
+    for splits in (2, 3, 4):
+        if longest / splits < 256:
+            break
+        us = max(even_us, longest / splits * row_mb / _DECODE_UNIT_MB_PER_S * 1e6) + _DECODE_MERGE_US
+        if us < best_us:
+            best, best_us = (splits, min(4, n_waves)), us          # (several workgroups to a compute unit)
+    return best
+
+
 @lru_cache(maxsize=None)
 def decode_attention_shape(n_decode, n_heads, n_kv, hd, span, target_waves=4096, fused=False):
     """(splits, waves per workgroup) of the decode kernel: about `target_waves` waves in all and pieces of
@@ -1341,8 +1362,8 @@ def decode_attention_shape(n_decode, n_heads, n_kv, hd, span, target_waves=4096,
 
 
 def attention_bf16(q, cache, out, plan: AttentionPlan, positions, slots, table, n_heads, n_kv, hd, window=None, scale=None,
-                   target_waves: int = 4096, products=None, chunk=None, sinks=None, gate=None, cap=None, channel_gate=None):
-    """Attention of a step's rows with the matrix-core kernels (bfloat16 cache and out).
+                   target_waves: int = 4096, products=None, chunk=None, sinks=None, gate=None, cap=None, channel_gate=None, memo=None):
+    """Attention of a step's rows with the matrix-core kernels (bfloat16 cache and out).  memo: what the pass keeps for its layers (the order of its rows).
 
     `q` holds the rotated queries in bfloat16 and the cache the rows' keys and values; or, for a step
     of single decoded rows only, `q` is None and `products = (q, k, v, cos, sin)` holds the unrotated
@@ -1399,13 +1420,31 @@ def attention_bf16(q, cache, out, plan: AttentionPlan, positions, slots, table, 
     if plan.n_decode:
         span = seen(plan.max_decode_context, 31)
         n_splits, n_waves = decode_attention_shape(plan.n_decode, n_heads, n_kv, hd, span, target_waves, products is not None)
+        groups = plan.n_decode * n_kv * ((n_heads // n_kv + 15) // 16)
+        if plan.decode_positions is not None and n_splits == 1 and products is None and span == plan.max_decode_context:
+            n_splits, n_waves = _decode_ragged_split(groups, span, plan.decode_positions / plan.n_decode, hd, n_waves)
+        rows = plan.decode_rows
+        ordered = memo is not None and 16 < plan.n_decode <= 1024 and groups * n_splits > lib().gi_compute_units()
+        if ordered:
+            rows = _decode_order(memo, plan, positions)
         n_part = plan.n_decode * n_heads * n_splits * (hd + 2) if n_splits > 1 else 0
         part = torch.empty(n_part, dtype=torch.float32, device=out.device) if n_part else None
         _call("gi_attention_decode_bf16", _ptr(q), _ptr(qf), _ptr(kf), _ptr(vf), qf.stride(0) if qf is not None else 0,
               kf.stride(0) if kf is not None else 0, vf.stride(0) if vf is not None else 0, _ptr(cos), _ptr(sin), cache.data_ptr(),
-              out.data_ptr(), _ptr(part), n_part, _ptr(plan.decode_rows), plan.n_decode, positions.data_ptr(), slots.data_ptr(),
-              table.data_ptr(), table.stride(0), cache.stride(0), page_size, n_heads, n_kv, hd, window, scale, n_splits, n_waves, *extras, _stream())
+              out.data_ptr(), _ptr(part), n_part, _ptr(rows), plan.n_decode, positions.data_ptr(), slots.data_ptr(),
+              table.data_ptr(), table.stride(0), cache.stride(0), page_size, n_heads, n_kv, hd, window, scale, n_splits, n_waves, 1 if ordered else 0, *extras, _stream())
     return out
+
+
+def _decode_order(memo, plan, positions):
+    """The step's single rows with the longest contexts first, made once per pass (on the device: a captured pass makes it anew in every replay), 4 us.
+    Dealt out in the rows' own order, a compute unit had the same row's heads in every round, the longest contexts' units twice and four times: 64 rows of 8
+    groups of 64 channels at 512 to 2,048 positions took 37.4 us a layer, there and back 32.4."""
+    if "decode_order" not in memo:
+        order = torch.empty(plan.n_decode, dtype=torch.int32, device=positions.device)
+        _call("gi_decode_order", positions.data_ptr(), _ptr(plan.decode_rows), plan.n_decode, order.data_ptr(), _stream())
+        memo["decode_order"] = order
+    return memo["decode_order"]
 
 
 def _plan_of(ctx):
@@ -1420,7 +1459,7 @@ def attention(q, cache, out, ctx, table, n_heads, n_kv, hd, window=None):
     if q.dtype == torch.bfloat16 and cache.dtype == torch.bfloat16 and out.dtype == torch.bfloat16:
         plan = _plan_of(ctx)
         if (not plan.n_tiles or attention_bf16_supports(hd, page_size, True)) and (not plan.n_decode or attention_bf16_supports(hd, page_size, False)):
-            return attention_bf16(q, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window)
+            return attention_bf16(q, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, memo=ctx.memo)
     return attention_exact(q, cache, out, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, **_known_of(ctx))
 
 
@@ -1449,7 +1488,7 @@ def attention_general(q, cache, out, ctx, table, n_heads, n_kv, hd, *, page_size
         plan = _plan_of(ctx)
         if (not plan.n_tiles or attention_bf16_supports(hd, page_size, True)) and (not plan.n_decode or attention_bf16_supports(hd, page_size, False)):
             return attention_bf16(q, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, scale, chunk=chunk, sinks=sinks, gate=gate, cap=cap,
-                                  channel_gate=channel_gate)
+                                  channel_gate=channel_gate, memo=ctx.memo)
     return attention_exact(q, cache, out, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, scale, page_size=page_size,
                            value_dim=value_dim, chunk=chunk, sinks=sinks, gate=gate, cap=cap, channel_gate=channel_gate, **_known_of(ctx))
 
@@ -1473,7 +1512,7 @@ def attention_from_products(q, k, v, cos, sin, cache, out, ctx, table, n_heads, 
         return False
     if q.stride(0) % 4 or q.data_ptr() % 16 or (k is not None and (k.stride(0) % 4 or k.data_ptr() % 16)):
         return False
-    attention_bf16(None, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, products=(q, k, v, cos, sin))
+    attention_bf16(None, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, products=(q, k, v, cos, sin), memo=ctx.memo)
     return True
 
 

@@ -735,6 +735,45 @@ def test_few_prompt_tiles_over_a_long_context_share_their_keys_out(n_heads, n_kv
     assert rel(out, want) < 8e-3, rel(out, want)
 
 
+@pytest.mark.parametrize("n_single, portion, n_heads, n_kv, hd, window", [(40, 0, 16, 8, 64, None), (65, 0, 8, 4, 128, 100), (33, 90, 32, 8, 128, None), (200, 80, 4, 2, 64, None), (17, 0, 64, 16, 64, None)])
+def test_decoded_rows_of_unequal_contexts_dealt_out_over_the_chip(n_single, portion, n_heads, n_kv, hd, window):
+    """More workgroups than compute units: the single rows are taken longest context first, there and back.  Each row's result is what it is in the step's own
+    order (where neither cuts a context), and the right one; a prompt's portion in the middle makes the single rows a list."""
+    from geneinfer_amd.parts import StepContext
+    g = torch.Generator().manual_seed(n_single)
+    contexts = [int(c) for c in torch.randint(1, 700, (n_single,), generator=g)]
+    contexts[3] = contexts[7] = 700
+    if portion:
+        contexts.insert(n_single // 2, 200 + portion)
+    cache, table, dense = build_paged(contexts, n_kv, hd, 16, torch.bfloat16, seed=5)
+    rows, seg_start, seg_len, seg_pos0, seg_slot = [], [], [], [], []
+    for slot, c in enumerate(contexts):
+        n = portion if portion and slot == n_single // 2 else 1
+        seg_start.append(len(rows)); seg_len.append(n); seg_pos0.append(c - n); seg_slot.append(slot + 1)
+        rows += [(slot, c - n + i) for i in range(n)]
+    T = len(rows)
+    q = randn(T, n_heads * hd, dtype=torch.bfloat16, seed=3)
+    pos = torch.tensor([p for _, p in rows], dtype=torch.int32, device=DEV)
+    slots = torch.tensor([s_ + 1 for s_, _ in rows], dtype=torch.int32, device=DEV)
+    ctx = StepContext(n_rows=T, dtype=torch.bfloat16, device=torch.device(DEV), tokens=pos, row_pos=pos, row_slot=slots, seg_slot=seg_slot,
+                      seg_start=seg_start, seg_len=seg_len, seg_pos0=seg_pos0)
+    out = torch.full((T, n_heads * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops().attention(q, cache, out, ctx, table, n_heads, n_kv, hd, window)
+    want = plain_attention_rows(q, dense, rows, n_heads, n_kv, hd, window)
+    assert rel(out, want) < 8e-3, rel(out, want)
+    order = ctx.memo["decode_order"].tolist()
+    single = [i for i, (slot, _) in enumerate(rows) if not (portion and slot == n_single // 2)]
+    assert order == sorted(single, key=lambda i: (-rows[i][1], i))
+    plan = ops().AttentionPlan(seg_start, seg_len, seg_pos0, seg_slot, DEV)
+    assert plan.decode_positions == sum(rows[i][1] + 1 for i in single)
+    plan.decode_positions = None
+    both = []
+    for memo in ({}, None):
+        both.append(torch.full_like(out, float("nan")))
+        ops().attention_bf16(q, cache, both[-1], plan, pos, slots, table, n_heads, n_kv, hd, window, memo=memo)
+    assert torch.equal(*both)
+
+
 @pytest.mark.parametrize("window", [None, 200])
 def test_many_prompt_tiles_of_many_heads(window):
     """More workgroups than compute units at head size 64 (5 pairs of tiles x 64 heads): the step takes the kernel with a
