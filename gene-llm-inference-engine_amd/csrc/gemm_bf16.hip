@@ -1370,6 +1370,65 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
     }
 }
 
+// The same sums onto 32-bit rows, whole rows at a time (a workgroup a row of up to 4096 columns), and the norm that reads the rows next beside them:
+// out = bfloat16(g * (x * rsqrt(mean(x^2) + eps))), as the norm's own kernel makes it, in bits.  131 rows of 2,048 out of eight shares: 5.0 us, as the
+// kernel without the norm, whose kernel behind it took 5.1.
+struct WholeNorm {
+    const float* g;
+    bf16_t* out;
+    long ld;
+    float eps;
+};
+constexpr int WHOLE_NORM_COLUMNS = 4096;
+template <int EACH>
+__global__ __launch_bounds__(256) void skinny_reduce_norm_kernel(const float* __restrict__ P, float* __restrict__ C, int M, int N, int splits, long ldc, WholeNorm norm) {
+    __shared__ float red[4];
+    const size_t row = blockIdx.x, slab = (size_t)M * N;
+    float4 x[EACH], sum[EACH], g[EACH];
+#pragma unroll
+    for (int e = 0; e < EACH; ++e) {
+        const int c = 4 * (threadIdx.x + 256 * e);
+        x[e] = sum[e] = g[e] = float4{0.f, 0.f, 0.f, 0.f};
+        if (c < N) {
+            x[e] = *reinterpret_cast<const float4*>(C + row * ldc + c);
+            g[e] = *reinterpret_cast<const float4*>(norm.g + c);
+        }
+    }
+    for (int sp0 = 0; sp0 < splits; sp0 += 4) {
+        float4 part[4][EACH];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int e = 0; e < EACH; ++e)
+                part[u][e] = *reinterpret_cast<const float4*>(P + (size_t)min(sp0 + u, splits - 1) * slab + row * N + min(4 * (int)(threadIdx.x + 256 * e), N - 4));
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (sp0 + u < splits) {
+#pragma unroll
+                for (int e = 0; e < EACH; ++e) { sum[e].x += part[u][e].x; sum[e].y += part[u][e].y; sum[e].z += part[u][e].z; sum[e].w += part[u][e].w; }
+            }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < EACH; ++e) {
+        const int c = 4 * (threadIdx.x + 256 * e);
+        if (c < N) {
+            x[e].x += sum[e].x; x[e].y += sum[e].y; x[e].z += sum[e].z; x[e].w += sum[e].w;
+            *reinterpret_cast<float4*>(C + row * ldc + c) = x[e];
+            ss = fmaf(x[e].x, x[e].x, ss); ss = fmaf(x[e].y, x[e].y, ss); ss = fmaf(x[e].z, x[e].z, ss); ss = fmaf(x[e].w, x[e].w, ss);
+        }
+    }
+    ss = block_sum<256>(ss, red);
+    const float scale = 1.0f / sqrtf(ss / (float)N + norm.eps);
+#pragma unroll
+    for (int e = 0; e < EACH; ++e) {
+        const int c = 4 * (threadIdx.x + 256 * e);
+        if (c < N)
+            *reinterpret_cast<uint2*>(norm.out + row * norm.ld + c) =
+                uint2{f32x2_to_bf16x2(g[e].x * (scale * x[e].x), g[e].y * (scale * x[e].y)), f32x2_to_bf16x2(g[e].z * (scale * x[e].z), g[e].w * (scale * x[e].w))};
+    }
+}
+
 // The same for the gated product: columns 32b .. 32b+15 of the partial sums are gates, 32b+16 .. 32b+31 the ups of
 // outputs 16b .. 16b+15; the output [M, N/2] is silu(gate) * up in bfloat16.
 __global__ void skinny_reduce_gated_kernel(const float* __restrict__ P, bf16_t* __restrict__ C, int M, int N, int splits, long ldc, int epi, float limit) {
@@ -1850,8 +1909,12 @@ static const NormIn NO_NORM_IN = {nullptr, 0, 0.f, 1, 0.f};
 static const NormOut NO_NORM_OUT = {nullptr, nullptr, 0, nullptr};
 
 static int reduce_partials(const float* scratch, void* C, int epi, int M, int N, int splits, long ldc, hipStream_t stream, NormIn norm_in = NO_NORM_IN,
-                           NormOut norm_out = NO_NORM_OUT) {
-    if (is_gated(epi)) {
+                           NormOut norm_out = NO_NORM_OUT, const WholeNorm* whole = nullptr) {
+    if (whole != nullptr) {
+#define WHOLE(EACH_) skinny_reduce_norm_kernel<EACH_><<<M, 256, 0, stream>>>(scratch, (float*)C, M, N, splits, ldc, *whole)
+        if (N <= 1024) WHOLE(1); else if (N <= 2048) WHOLE(2); else if (N <= 3072) WHOLE(3); else WHOLE(4);
+#undef WHOLE
+    } else if (is_gated(epi)) {
         GI_REQUIRE(norm_in.squares == nullptr, "gemm_bf16: a gated product whose k is shared out cannot finish a norm handed on");
         skinny_reduce_gated_kernel<<<(unsigned)(((size_t)M * (N / 2) + 255) / 256), 256, 0, stream>>>(scratch, (bf16_t*)C, M, N, splits, ldc, epi, norm_in.limit);
     } else {
@@ -2004,7 +2067,7 @@ static int launch_slim_tiles(const void* A, const void* W, void* C, int epi, int
 // Up to 128 rows the weights are the traffic and every workgroup streams its share of them once (measured on the decode step of
 // the Llama-3.2-1B shape: 72 rows took 2.69 ms through the tiles of 128 rows of the kernels for more rows, against 2.11 ms at 64 rows).
 static int launch_skinny(const void* A, const void* W, void* C, int epi, int M, int N, int K, long lda, long ldw, long ldc, float* scratch,
-                         long scratch_floats, NormIn norm_in, NormOut norm_out, hipStream_t stream, const RopeStore* rope = nullptr) {
+                         long scratch_floats, NormIn norm_in, NormOut norm_out, hipStream_t stream, const RopeStore* rope = nullptr, const WholeNorm* whole = nullptr) {
     const int splits = gi_gemm_bf16_skinny_splits(N, K), mt = (M + 15) / 16;
 #define SKINNY_MT(EPI_, PARTIAL_)                                                                                                   \
     do {                                                                                                                            \
@@ -2041,7 +2104,7 @@ static int launch_skinny(const void* A, const void* W, void* C, int epi, int M, 
         GI_CHECK_LAUNCH("gemm_bf16 (reduce, rotate, store)");
         return 0;
     }
-    return reduce_partials(scratch, C, epi, M, N, splits, ldc, stream, norm_in, norm_out);
+    return reduce_partials(scratch, C, epi, M, N, splits, ldc, stream, norm_in, norm_out, whole);
 }
 
 static TileOrder tall_order(int M, int N) {
@@ -2068,7 +2131,7 @@ static int large_norm_parts(int M, int N, int K) {
 // More than 128 rows, K a multiple of 64, 128 columns or more: the kernels that load their operands straight into LDS.
 // `rope` != null: the sums are those of an attention layer's q/k/v product and go where it says (`epi` is then not looked at).
 static int launch_large(const void* A, const void* W, void* C, int epi, int M, int N, int K, long lda, long ldw, long ldc, float* scratch,
-                        long scratch_floats, NormIn norm_in, const RopeStore* rope, hipStream_t stream, NormOut norm_out = NO_NORM_OUT) {
+                        long scratch_floats, NormIn norm_in, const RopeStore* rope, hipStream_t stream, NormOut norm_out = NO_NORM_OUT, const WholeNorm* whole = nullptr) {
     const NormIn limit_in = {nullptr, 0, 0.f, 1, norm_in.limit};          // no norm to finish, the clamped gate's limit alone
 #define PIPED(BM_, BN_, WM_, WN_, ST_, EPI_, OUT_, LDC_, SPLITS_, KPS_, SLAB_, NORM_, ROPE_)                                            \
     do {                                                                                                                                \
@@ -2106,7 +2169,7 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
             GI_CHECK_LAUNCH("gemm_bf16 (reduce, rotate, store)");
             return 0;
         }
-        return reduce_partials(scratch, C, epi, M, N, splits, ldc, stream, norm_in, norm_out);
+        return reduce_partials(scratch, C, epi, M, N, splits, ldc, stream, norm_in, norm_out, whole);
     }
     const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
     GI_REQUIRE(norm_out.scaled == nullptr || (!many_tiles(M, N) && large_norm_parts(M, N, K) > 0), "gemm_bf16: a product of M %d, N %d, K %d hands no norm on", M, N, K);
@@ -2232,6 +2295,28 @@ GI_API int gi_gemm_bf16_handing(const void* A, const void* W, void* C, int c_dty
         return launch_large(A, W, C, epi, M, N, K, lda, ldw, ldc, scratch, scratch_floats, norm_in, nullptr, stream, norm_out);
     }
     return launch_skinny(A, W, C, epi, M, N, K, lda, ldw, ldc, scratch, scratch_floats, norm_in, norm_out, stream);
+}
+
+// Whether a product of these sizes can make the whole norm of the rows it adds onto (gi_gemm_bf16_onto_norm): where k is shared out over workgroups, the kernel
+// that adds the shares up sees whole rows.
+GI_API int gi_gemm_bf16_onto_norm_takes(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || N % 4 != 0 || N > WHOLE_NORM_COLUMNS || K <= 0 || K % 8 != 0) return 0;
+    if (M <= SKINNY_MAX_ROWS) return !takes_slim(M, N, K) && !takes_slim_tiles(M, N, K, EPI_ADD_F32) && gi_gemm_bf16_skinny_splits(N, K) > 0;
+    return K % PK == 0 && N >= 128 && gi_gemm_bf16_piped_splits(M, N, K) > 1;
+}
+
+// C += A W^T onto 32-bit rows C [M, ldc], and normed [M, ld_normed] = bfloat16(g * (C * rsqrt(mean(C^2) + eps))), the norm that reads the rows next.
+GI_API int gi_gemm_bf16_onto_norm(const void* A, const void* W, float* C, int M, int N, int K, long lda, long ldw, long ldc, float* scratch, long scratch_floats, const float* g,
+                                  float eps, void* normed, long ld_normed, hipStream_t stream) {
+    GI_REQUIRE(gi_gemm_bf16_onto_norm_takes(M, N, K), "gemm_bf16 (norm): sizes M %d, N %d, K %d are not taken", M, N, K);
+    GI_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && lda >= K && ldw >= K && ((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0,
+               "gemm_bf16 (norm): rows must be 16-byte aligned (strides %ld, %ld)", lda, ldw);
+    GI_REQUIRE(C != nullptr && g != nullptr && normed != nullptr && ldc >= N && ldc % 4 == 0 && ld_normed >= N && ld_normed % 4 == 0 &&
+                   (((uintptr_t)C | (uintptr_t)g | (uintptr_t)scratch) & 15) == 0 && ((uintptr_t)normed & 7) == 0,
+               "gemm_bf16 (norm): outputs or weights are missing or not aligned (strides %ld, %ld)", ldc, ld_normed);
+    const WholeNorm whole = {g, (bf16_t*)normed, ld_normed, eps};
+    if (M <= SKINNY_MAX_ROWS) return launch_skinny(A, W, C, EPI_ADD_F32, M, N, K, lda, ldw, ldc, scratch, scratch_floats, NO_NORM_IN, NO_NORM_OUT, stream, nullptr, &whole);
+    return launch_large(A, W, C, EPI_ADD_F32, M, N, K, lda, ldw, ldc, scratch, scratch_floats, NO_NORM_IN, nullptr, stream, NO_NORM_OUT, &whole);
 }
 
 // Whether gi_gemm_bf16_qkv_rope_store takes a q/k/v product of these sizes with heads of hd channels.  17 or 33 to 128 rows: the

@@ -109,6 +109,7 @@ _SIGNATURES = {
     "gi_random_normal": [c_void_p, c_int, c_long, ctypes.c_ulonglong, ctypes.c_double, ctypes.c_double, c_void_p],
     "gi_probe_stream": [c_void_p, c_void_p, c_long, c_void_p, c_int, c_int, c_void_p],
     "gi_probe_mfma": [c_int, c_void_p, c_int, c_void_p],
+    "gi_gemm_bf16_onto_norm": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long, c_void_p, c_float, c_void_p, c_long, c_void_p],
     "gi_gemm_bf16_handing": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long,
                              c_void_p, c_int, c_float, c_void_p, c_void_p, c_long, c_void_p, c_void_p],
     "gi_gemm_bf16_qkv_rope_store": [c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_void_p, c_long, c_void_p, c_int, c_float, c_void_p, c_void_p,
@@ -151,6 +152,8 @@ def lib():
         l.gi_gemm_bf16_norm_parts.restype = c_int
         l.gi_gemm_bf16_large_kernel.argtypes = [c_int, c_int, c_int, c_int]
         l.gi_gemm_bf16_large_kernel.restype = c_int
+        l.gi_gemm_bf16_onto_norm_takes.argtypes = [c_int, c_int, c_int]
+        l.gi_gemm_bf16_onto_norm_takes.restype = c_int
         l.gi_gemm_bf16_xielu_takes.argtypes = [c_int, c_int, c_int, c_int]
         l.gi_gemm_bf16_xielu_takes.restype = c_int
         l.gi_gemm_bf16_takes_norm.argtypes = [c_int, c_int, c_int, c_int]
@@ -198,7 +201,7 @@ def _call(name, *args):
         raise KernelError(lib().gi_last_error().decode())
 
 
-_PROFILE_LABEL = {"gi_gemm_bf16_handing": "gemm_bf16", "gi_gemm_bf16_xielu": "gemm_bf16", "gi_gemm_bf16_qkv_rope_store": "gemm_bf16"}        # the same products, with a norm's share on top
+_PROFILE_LABEL = {"gi_gemm_bf16_handing": "gemm_bf16", "gi_gemm_bf16_onto_norm": "gemm_bf16", "gi_gemm_bf16_xielu": "gemm_bf16", "gi_gemm_bf16_qkv_rope_store": "gemm_bf16"}        # the same products, with a norm's share on top
 
 
 class KernelProfile:
@@ -1597,6 +1600,30 @@ def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=N
     _call("gi_gemm_bf16", a.data_ptr(), w.data_ptr(), out.data_ptr(), _code(out, "gemm: out"), 1 if accumulate else 0, gate_code, float(gate_limit),
           m, n, k, a.stride(0), w.stride(0), out.stride(0), _ptr(scratch), n_scratch, _stream())
     return out
+
+
+@lru_cache(maxsize=8192)
+def gemm_bf16_onto_norm_takes(m, n, k) -> bool:
+    """Whether `gemm_bf16_onto_norm` takes a product of these sizes."""
+    return bool(lib().gi_gemm_bf16_onto_norm_takes(m, n, k))
+
+
+def gemm_bf16_onto_norm(a, w, x, g, eps, normed):
+    """x += a @ w.T onto float32 rows, and normed = bfloat16(g * (x * rsqrt(mean(x^2) + eps))), as `rmsnorm` makes it of the new rows, in the kernel that adds
+    the shares of k up."""
+    _dev(a, w, x, g, normed)
+    m, k = a.shape
+    n = w.shape[0]
+    if not (w.shape == (n, k) and x.shape == (m, n) and gemm_bf16_supports(a, w, x) and x.dtype == torch.float32 and gemm_bf16_onto_norm_takes(m, n, k)
+            and g.dtype == torch.float32 and g.shape == (n,) and g.is_contiguous() and normed.dtype == torch.bfloat16 and normed.shape == (m, n) and normed.stride(1) == 1):
+        raise KernelError("gemm_bf16_onto_norm: bfloat16 operands, float32 rows [m, n] and weights [n], bfloat16 [m, n] for the normed rows, and sizes that are taken")
+    n_scratch = _scratch_floats(m, n, k)
+    scratch = torch.empty(n_scratch, dtype=torch.float32, device=a.device)
+    if _profile is not None:
+        _profile.note = (f"{n}x{k}", n * k * w.element_size())
+    _call("gi_gemm_bf16_onto_norm", a.data_ptr(), w.data_ptr(), x.data_ptr(), m, n, k, a.stride(0), w.stride(0), x.stride(0), scratch.data_ptr(), n_scratch, g.data_ptr(),
+          float(eps), normed.data_ptr(), normed.stride(0), _stream())
+    return normed
 
 
 def gemm_bf16_large_kernel(m, n, k, kind):

@@ -92,6 +92,7 @@ class Attention(Mixer):
     stores, and the attention kernel that knows all of these."""
     accepts_deferred_norm = True      # its input goes into `linear` only
     hands_norm_on = True              # `forward` takes `then`, the norm that reads the residual next
+    hands_whole_norms = True          # ... also as a `NormToMake`
     can_overwrite = True              # `forward(..., overwrite=True)` stores its result in `residual` instead of adding onto it
 
     def __init__(self, spec, tensors, dtype, device):

@@ -17,7 +17,7 @@ import torch
 from ..kernels import ops
 from .base import feed_forward_class, mixer_class, norm_class, register_block
 from .linear import linear, linear_xielu, takes_handed_norm
-from .norm import NormedRows, ReadyRows, norm_to_apply, norm_to_hand_on
+from .norm import NormedRows, ReadyRows, norm_to_apply, norm_to_hand_on, norm_to_make
 
 
 class PreNormBlock:
@@ -61,7 +61,9 @@ class PreNormBlock:
 
     @staticmethod
     def _then(part, reader, n_rows):
-        return norm_to_hand_on(reader, n_rows) if getattr(part, "hands_norm_on", False) else None
+        """The norm that reads next, as the part's `then`: to be half applied, else to be made whole; None where the part does neither."""
+        then = norm_to_hand_on(reader, n_rows) if getattr(part, "hands_norm_on", False) else None
+        return norm_to_make(reader, part) if then is None else then
 
     def forward(self, x, ctx, cache, handed=None, next_reader=None):
         """handed: this block's first norm as whoever wrote x last left it, or None.  next_reader: `first_reader()` of whatever

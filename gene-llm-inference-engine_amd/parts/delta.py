@@ -31,6 +31,7 @@ class GatedDelta(Mixer):
     graph_safe = True
     accepts_deferred_norm = True      # its input goes into `linear` only
     hands_norm_on = True              # `forward` takes `then`, the norm that reads the residual next
+    hands_whole_norms = True          # ... also as a `NormToMake`
     can_overwrite = True
     FEW_ROWS = 16                     # up to so many rows (bfloat16) the products behind the narrow middles are made inside the kernels that need them
 

@@ -52,6 +52,7 @@ def heads_product(a, w, out, n_heads, out_head_stride=None, channel_gate=None):
 class LatentAttention(Mixer):
     accepts_deferred_norm = True      # its input goes into `linear` only
     hands_norm_on = True              # `forward` takes `then`, the norm that reads the residual next
+    hands_whole_norms = True          # ... also as a `NormToMake`
     can_overwrite = True
 
     def takes_handed_norm(self, n_rows: int) -> bool:

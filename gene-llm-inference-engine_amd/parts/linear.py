@@ -14,7 +14,7 @@ from __future__ import annotations
 import torch
 
 from ..kernels import ops
-from .norm import HandedRows, NormedRows
+from .norm import HandedRows, NormedRows, NormToMake, ReadyRows
 
 
 def linear(a, weight: torch.Tensor, out: torch.Tensor, accumulate: bool = False, gated: bool = False, gate_limit: float = 0.0) -> torch.Tensor:
@@ -56,7 +56,15 @@ def linear_xielu(a, weight: torch.Tensor, params: torch.Tensor, columns: int, dt
 
 def linear_onto(a: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor, then=None):
     """residual += a @ weight.T.  `then`: the norm that reads `residual` next, if it and its reader can take it half applied
-    (see `HandedRows`); the product then also does the norm's share and the `HandedRows` are returned, None otherwise."""
+    (see `HandedRows`); the product then also does the norm's share and the `HandedRows` are returned, None otherwise.  Or that norm as a
+    `NormToMake`, for a reader that takes no other than a whole one: the rows come back normed where the product's kernel can."""
+    if isinstance(then, NormToMake):
+        norm, n, k = then.norm, weight.shape[0], weight.shape[1]
+        if (a.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and residual.dtype == torch.float32 and residual.stride(0) % 4 == 0 and residual.data_ptr() % 16 == 0
+                and norm.handed_weight().data_ptr() % 16 == 0 and ops.gemm_bf16_supports(a, weight, residual) and ops.gemm_bf16_onto_norm_takes(residual.shape[0], n, k)):
+            normed = torch.empty(residual.shape, dtype=torch.bfloat16, device=residual.device)
+            return ReadyRows(norm, residual, ops.gemm_bf16_onto_norm(a, weight, residual, norm.handed_weight(), norm.eps, normed))
+        then = None
     if (then is not None and a.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and residual.dtype == torch.float32
             and residual.is_contiguous() and ops.gemm_bf16_supports(a, weight, residual)):
         rows, width = residual.shape

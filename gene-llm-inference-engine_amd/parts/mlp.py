@@ -15,6 +15,7 @@ class SwiGlu(FeedForward):
     graph_safe = True
     accepts_deferred_norm = True      # its input goes into `linear` only
     hands_norm_on = True              # `forward` takes `then`, the norm that reads the residual next
+    hands_whole_norms = True          # ... also as a `NormToMake`
     can_overwrite = True              # `forward(..., overwrite=True)` stores its result in `residual` instead of adding onto it
 
     def __init__(self, spec, tensors, dtype, device):
@@ -65,6 +66,7 @@ class DenseMlp(FeedForward):
     graph_safe = True
     accepts_deferred_norm = True      # its input goes into `linear` only
     hands_norm_on = True              # `forward` takes `then`, the norm that reads the residual next
+    hands_whole_norms = True          # ... also as a `NormToMake`
     can_overwrite = True
 
     def takes_handed_norm(self, n_rows: int) -> bool:

@@ -62,6 +62,23 @@ def norm_to_hand_on(reader, n_rows: int):
     return norm
 
 
+class NormToMake:
+    """A norm that whoever writes its rows may make whole on the way (`ReadyRows`), as a part's `then`: the parts whose `then` goes to `linear_onto` alone
+    (`hands_whole_norms`) take it."""
+
+    def __init__(self, norm: "RmsNorm"):
+        self.norm = norm
+
+
+def norm_to_make(reader, part):
+    """reader: as above.  The norm as `part`'s `then`, if the part may make it whole and its reader takes it so in bfloat16; None otherwise."""
+    norm, reads = reader if reader is not None else (None, None)
+    if (not getattr(part, "hands_whole_norms", False) or not hasattr(norm, "handed_weight") or not getattr(reads, "accepts_deferred_norm", False)
+            or getattr(reads, "in_dtype", None) != torch.bfloat16):
+        return None
+    return NormToMake(norm)
+
+
 def norm_to_apply(reader, part):
     """reader: as above.  The norm, if `part`, which writes the rows it reads, can make the normed rows on the way (`makes_next_norm(norm)`)
     for a reader that takes them ready in bfloat16; None otherwise."""

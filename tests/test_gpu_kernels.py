@@ -1154,3 +1154,19 @@ def test_rope_store_writes_the_right_places():
         touched[page, 0, :, place, :] = True
         touched[page, 1].view(n_kv, hd, ps)[:, :, place] = True
     assert torch.all(cache[~touched] == -777.25), "rope_store wrote outside its places"
+
+
+@pytest.mark.parametrize("m, n, k", [(131, 2048, 2048), (129, 2048, 8192), (300, 1028, 1024), (500, 3072, 512), (257, 4096, 512), (64, 2048, 2048), (40, 3072, 1024), (128, 132, 512)])
+def test_product_onto_rows_that_makes_the_whole_norm(m, n, k):
+    """Shares of k added up, onto the rows, and the rows' norm: what the product and the norm's kernel make one after the other, in bits."""
+    assert ops().gemm_bf16_onto_norm_takes(m, n, k)
+    a, w = randn(m, k, dtype=torch.bfloat16, seed=1), randn(n, k, dtype=torch.bfloat16, seed=2)
+    x = randn(m, n, dtype=torch.float32, seed=3)
+    g = (1 + 0.1 * randn(n, dtype=torch.float32, seed=4)).to(torch.bfloat16)
+    want_x = x.clone()
+    ops().gemm_bf16(a, w, want_x, accumulate=True)
+    want = ops().rmsnorm(want_x, g, 1e-5, torch.empty(m, n, dtype=torch.bfloat16, device=DEV))
+    got = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops().gemm_bf16_onto_norm(a, w, x, g.float(), 1e-5, got)
+    assert torch.equal(x, want_x) and torch.equal(got, want)
+    assert rel(x, randn(m, n, dtype=torch.float32, seed=3).double() + a.double() @ w.double().t()) < 1e-5
