@@ -474,6 +474,155 @@ __global__ __launch_bounds__(512) void latent_attention_tiles_kernel(const bf16_
         }
 }
 
+// The rows of prompts where the heads come in whole groups of 32: a wave takes one row's 32 heads (the columns of the 32x32x16 matrix instruction), a workgroup up
+// to eight (row, group) pairs of consecutive rows, all on the same tiles of 32 positions.  What bounds the kernel above is LDS (a wave reads a whole tile for 16
+// columns, twice the time of its products) and a tile's round trip through registers; here a tile serves 32 columns a wave and goes from memory
+// into LDS directly, into the one of two places that the waves are not reading, while they multiply.  Layout of a tile in LDS: keys [32 positions][pieces
+// of 16 bytes], then values [channels][4 pieces], a row's pieces in fours exchanged by (row / 4) % 4, so that 16 rows' reads of a piece fall into different
+// banks.  A lane reads the key rows in the order that makes its 16 scores the positions 8 h + 0 .. 7 and 16 + 8 h + 0 .. 7 (h: which half of the
+// wave): as they lie, packed, they are the second operand of O^T = V^T P^T, and its first operand is one piece.  A column's maximum follows its scores
+// only when it lags by more than LATENT_SLACK (in units of log2 e; any reference gives the same O / l), which takes the rescaling of the sums off most tiles.
+// 1,777 rows of 32 heads, keys of 288 and values of 256 channels, a window of 1,024: 84 us, 223 in the kernel above.
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+constexpr float LATENT_SLACK = 8.f;
+template <int KS, int VT>          // keys of up to 32 KS channels, values of up to 32 VT
+__global__ __launch_bounds__(512) void latent_attention_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache, bf16_t* __restrict__ out,
+                                                                   const int4* __restrict__ tiles, int pieces_per_tile, int TR, int HG,
+                                                                   const int* __restrict__ table, int table_stride, long page_stride, int page_size,
+                                                                   int n_heads, int kd, int vd, int window, float scale2, const float* __restrict__ sinks) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    constexpr int KPIECES = 4 * KS, K_BYTES = 32 * KPIECES * 16, V_BYTES = VT * 32 * 64, STAGE = K_BYTES + V_BYTES, PARTS = STAGE / 1024, MOST = (PARTS + 7) / 8;
+    static_assert(K_BYTES % 1024 == 0 && V_BYTES % 1024 == 0, "a wave-wide load fills 1 KB");
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, half = lane >> 5;
+    const int4 tile = tiles[blockIdx.x / pieces_per_tile];
+    const int piece = blockIdx.x % pieces_per_tile;
+    const int row0 = tile.x + piece * TR, n_tok = min(TR, tile.x + tile.y - row0);
+    if (n_tok <= 0) return;                              // (the whole workgroup, before any barrier)
+    const int p_first = tile.z + piece * TR, p_last = p_first + n_tok - 1;
+    const int lo_all = (window > 0 && p_first - window + 1 > 0) ? p_first - window + 1 : 0;
+    const int* tab = table + (size_t)tile.w * table_stride;
+    const bool works = wave < n_tok * HG;                // (every wave loads; one without a row multiplies nothing)
+    const int ti = min(wave / HG, n_tok - 1), head = (wave % HG) * 32 + r;
+    const int t = row0 + ti, p = p_first + ti;
+    const int lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
+
+    // This wave's loads of a tile: 1 KB each, parts wave, wave + 8, ..  Where a lane's 16 bytes lie: bytes behind its block's first key, or behind its block's
+    // first place of channel 0; the highest bit says which of the tile's two blocks of 16 positions (each within one page).
+    unsigned from[MOST];
+#pragma unroll
+    for (int i = 0; i < MOST; ++i) {
+        const int part = wave + i * 8, slot = part * 64 + lane;
+        if (part * 1024 < K_BYTES) {
+            const int row = slot / KPIECES, c = (slot % KPIECES) ^ ((row >> 2) & 3);
+            from[i] = (unsigned)((row & 15) * kd * 2 + min(c, (kd >> 3) - 1) * 16) | (row >= 16 ? 0x80000000u : 0u);       // (beyond the key: any piece that is numbers; the query has zeros there)
+        } else {
+            const int s = slot - K_BYTES / 16, e = (s & 3) ^ ((s >> 4) & 3);
+            from[i] = (unsigned)(min(s >> 2, vd - 1) * page_size * 2 + (e & 1) * 16) | (e >= 2 ? 0x80000000u : 0u);
+        }
+    }
+    const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) void*)lds;
+    auto load_tile = [&](int tk, int place) {
+        const char *keys[2], *values[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {                    // a block that nobody sees is read from one that somebody does
+            const int j0 = __builtin_amdgcn_readfirstlane(min(max((tk << 5) + 16 * b, lo_all & ~15), p_last & ~15)), at = j0 % page_size;
+            const bf16_t* page = cache + (long)tab[j0 / page_size] * page_stride;
+            keys[b] = (const char*)(page + (long)at * kd);
+            values[b] = (const char*)(page + (long)page_size * kd + at);
+        }
+#pragma unroll
+        for (int i = 0; i < MOST; ++i) {
+            const int part = wave + i * 8;
+            if (part < PARTS) {
+                const bool is_key = part * 1024 < K_BYTES, second = (int)from[i] < 0;
+                const char* src = (is_key ? (second ? keys[1] : keys[0]) : (second ? values[1] : values[0])) + (from[i] & 0x7fffffffu);
+                const unsigned dst = __builtin_amdgcn_readfirstlane(lds_base + place * STAGE + part * 1024);
+                // (as assembly, so that the compiler does not wait for them before every read of LDS: the wait and the barrier below order them)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src) : "memory", "m0");
+            }
+        }
+    };
+    int tk = lo_all >> 5;
+    const int tk_last = p_last >> 5;
+    load_tile(tk, 0);
+    bf16x8 qreg[2 * KS];
+#pragma unroll
+    for (int s = 0; s < 2 * KS; ++s) {
+        const int c = 16 * s + 8 * half;
+        uint4 v = *reinterpret_cast<const uint4*>(q + ((size_t)t * n_heads + head) * kd + (c < kd ? c : 0));
+        if (c >= kd) v = uint4{0, 0, 0, 0};
+        qreg[s] = as_bf16x8(v);
+    }
+    floatx16 o[VT];
+#pragma unroll
+    for (int i = 0; i < VT; ++i) o[i] = floatx16{};
+    float m = -INFINITY, l = 0.f;                        // (l: this lane's share of its column's sum)
+    if (sinks) m = sinks[head] * LOG2E, l = half == 0 ? 1.f : 0.f;
+    const int key = 16 * (r >> 4) + 8 * ((r >> 2) & 1) + 4 * ((r >> 3) & 1) + (r & 3), k_swz = (key >> 2) & 3, v_swz = (r >> 2) & 3;
+    const unsigned char* k_row = lds + key * (KPIECES * 16);
+    const unsigned char* v_row = lds + K_BYTES + r * 64;
+    const int k_off[2] = {(half ^ k_swz) * 16, ((2 + half) ^ k_swz) * 16}, v_off[2] = {(half ^ v_swz) * 16, ((2 + half) ^ v_swz) * 16};
+
+    for (int place = 0; tk <= tk_last; ++tk, place ^= 1) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                               // this wave's loads of the tile have landed
+        __builtin_amdgcn_s_barrier();                                                  // everyone's have, and nobody reads the other place any more
+        asm volatile("" ::: "memory");
+        if (tk < tk_last) load_tile(tk + 1, place ^ 1);
+        const int kv0 = tk << 5;
+        if (!works || kv0 + 31 < lo || kv0 > p) continue;
+        const unsigned char *kr = k_row + place * STAGE, *vr = v_row + place * STAGE;
+        floatx16 s = floatx16{};
+#pragma unroll
+        for (int ks = 0; ks < 2 * KS; ++ks)
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(*reinterpret_cast<const uint4*>(kr + (ks >> 1) * 64 + k_off[ks & 1])), qreg[ks], s, 0, 0, 0);
+        // element v: position kv0 + 16 (v / 8) + 8 half + v % 8, head `head`
+#pragma unroll
+        for (int v = 0; v < 16; ++v) s[v] *= scale2;
+        if (kv0 < lo || kv0 + 31 > p) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int j = kv0 + 16 * (v >> 3) + 8 * half + (v & 7);
+                s[v] = j >= lo && j <= p ? s[v] : -INFINITY;
+            }
+        }
+        float mx = s[0];
+#pragma unroll
+        for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const bool follow = mx > m + LATENT_SLACK;
+        if (__any(follow)) {
+            const float m_new = follow ? mx : m, corr = follow ? exp2_fast(m - m_new) : 1.f;
+            m = m_new;
+            l *= corr;
+#pragma unroll
+            for (int i = 0; i < VT; ++i)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) o[i][v] *= corr;
+        }
+        const float m_use = m == -INFINITY ? 0.f : m;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) s[v] = exp2_fast(s[v] - m_use);
+        l += (((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]))) + (((s[8] + s[9]) + (s[10] + s[11])) + ((s[12] + s[13]) + (s[14] + s[15])));
+        const bf16x8 pb[2] = {as_bf16x8(uint4{f32x2_to_bf16x2(s[0], s[1]), f32x2_to_bf16x2(s[2], s[3]), f32x2_to_bf16x2(s[4], s[5]), f32x2_to_bf16x2(s[6], s[7])}),
+                              as_bf16x8(uint4{f32x2_to_bf16x2(s[8], s[9]), f32x2_to_bf16x2(s[10], s[11]), f32x2_to_bf16x2(s[12], s[13]), f32x2_to_bf16x2(s[14], s[15])})};
+#pragma unroll
+        for (int i = 0; i < VT; ++i)
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+                o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(*reinterpret_cast<const uint4*>(vr + i * 2048 + v_off[ks])), pb[ks], o[i], 0, 0, 0);
+    }
+    if (!works) return;
+    l += __shfl_xor(l, 32, 64);
+    const float inv = 1.0f / l;                          // (a row always sees itself)
+    bf16_t* to = out + ((size_t)t * n_heads + head) * vd;
+#pragma unroll
+    for (int i = 0; i < VT; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; v += 4) {
+            const int c = 32 * i + 2 * v + 4 * half;      // element v: channel 32 i + 8 (v / 4) + 4 half + v % 4
+            if (c < vd) *reinterpret_cast<uint2*>(to + c) = uint2{f32x2_to_bf16x2(o[i][v] * inv, o[i][v + 1] * inv), f32x2_to_bf16x2(o[i][v + 2] * inv, o[i][v + 3] * inv)};
+        }
+}
 
 }  // namespace
 
@@ -624,9 +773,24 @@ static int allow_latent_tiles_lds() {
     return 0;
 }
 
+template <int KS, int VT>
+static int allow_latent_wide_lds() {
+    static bool allowed = false;
+    if (!allowed) {
+        const int lds_bytes = 2 * (KS * 2048 + VT * 2048);
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_attention_wide_kernel<KS, VT>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
+            return gi_fail("latent_attention: %d bytes of LDS are not granted", lds_bytes);
+        allowed = true;
+    }
+    return 0;
+}
+
 // Asks for the kernels' LDS once, outside any captured pass (a part calls it when it is built).
 GI_API int gi_latent_attention_tiles_prepare() {
-    int rc = allow_latent_tiles_lds<3, 4>();
+    int rc = allow_latent_wide_lds<3, 2>();
+    if (!rc) rc = allow_latent_wide_lds<5, 4>();
+    if (!rc) rc = allow_latent_wide_lds<9, 8>();
+    if (!rc) rc = allow_latent_tiles_lds<3, 4>();
     if (!rc) rc = allow_latent_tiles_lds<5, 8>();
     if (!rc) rc = allow_latent_tiles_lds<9, 16>();
     if (!rc) rc = allow_latent_tiles_lds<18, 32>();
@@ -646,6 +810,16 @@ static int launch_latent_tiles(const void* q, const void* cache, void* out, cons
     return 0;
 }
 
+template <int KS, int VT>
+static int launch_latent_wide(const void* q, const void* cache, void* out, const void* tiles, int n_tiles, int tile_rows, const int* table, int table_stride,
+                              long page_stride, int page_size, int n_heads, int kd, int vd, int window, float scale2, const float* sinks, hipStream_t stream) {
+    const int HG = n_heads / 32, TR = 8 / HG, pieces = (tile_rows + TR - 1) / TR;
+    if (int rc = allow_latent_wide_lds<KS, VT>()) return rc;
+    latent_attention_wide_kernel<KS, VT><<<(unsigned)(n_tiles * pieces), 512, 2 * (KS * 2048 + VT * 2048), stream>>>(
+        (const bf16_t*)q, (const bf16_t*)cache, (bf16_t*)out, (const int4*)tiles, pieces, TR, HG, table, table_stride, page_stride, page_size, n_heads, kd, vd, window, scale2, sinks);
+    return 0;
+}
+
 GI_API int gi_latent_attention_tiles_bf16(const void* q, const void* cache, void* out, const void* tiles, int n_tiles, int tile_rows, const int* table, int table_stride,
                                           long page_stride, int page_size, int n_heads, int kd, int vd, int window, float scale, const float* sinks, hipStream_t stream) {
     GI_REQUIRE(n_tiles > 0 && tile_rows > 0 && n_heads > 0 && gi_latent_attention_tiles_supports(n_heads, kd, vd, page_size),
@@ -656,10 +830,14 @@ GI_API int gi_latent_attention_tiles_bf16(const void* q, const void* cache, void
     const float scale2 = scale * 1.4426950408889634f;
     int rc;
 #define GO(KS, DT) rc = launch_latent_tiles<KS, DT>(q, cache, out, tiles, n_tiles, tile_rows, table, table_stride, page_stride, page_size, n_heads, kd, vd, window, scale2, sinks, stream)
-    if (kd <= 96 && vd <= 64) GO(3, 4);
-    else if (kd <= 160 && vd <= 128) GO(5, 8);
-    else if (kd <= 288 && vd <= 256) GO(9, 16);
+#define WIDE(KS, VT) rc = launch_latent_wide<KS, VT>(q, cache, out, tiles, n_tiles, tile_rows, table, table_stride, page_stride, page_size, n_heads, kd, vd, window, scale2, sinks, stream)
+    // whole groups of 32 heads whose sums fit in registers: 32 columns a wave (other numbers of heads would leave columns idle)
+    const bool wide = n_heads % 32 == 0 && n_heads <= 256 && kd <= 288 && vd <= 256 && vd % 8 == 0 && ((uintptr_t)out & 7) == 0 && (long)vd * page_size < (1L << 29);
+    if (kd <= 96 && vd <= 64) { if (wide) WIDE(3, 2); else GO(3, 4); }
+    else if (kd <= 160 && vd <= 128) { if (wide) WIDE(5, 4); else GO(5, 8); }
+    else if (kd <= 288 && vd <= 256) { if (wide) WIDE(9, 8); else GO(9, 16); }
     else GO(18, 32);
+#undef WIDE
 #undef GO
     if (rc) return rc;
     GI_CHECK_LAUNCH("latent_attention (tiles)");

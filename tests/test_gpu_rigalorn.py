@@ -522,6 +522,52 @@ def test_matrix_core_attention_over_latent_pages(H, kd, vd, window, lens, pos0):
     assert relative_error(exact, want) < 6e-3 and relative_error(out, exact.double()) < 1.5e-2
 
 
+@pytest.mark.parametrize("H, kd, vd, window, lens, pos0", [(32, 288, 256, 1000, [270], [900]), (64, 88, 56, None, [140, 33], [0, 40]), (96, 160, 128, 33, [65], [7]), (256, 24, 16, 20, [70], [3]),
+                                                          (32, 256, 248, 31, [100, 1], [31, 9]), (160, 96, 64, None, [66], [0])])
+def test_matrix_core_attention_over_latent_pages_with_heads_in_groups_of_32(H, kd, vd, window, lens, pos0):
+    """A wave per row and 32 heads: one to eight groups, numbers of groups that leave waves without a row, keys and values shorter than the kernel's."""
+    test_matrix_core_attention_over_latent_pages(H, kd, vd, window, lens, pos0)
+
+
+@pytest.mark.parametrize("page, window", [(16, None), (48, 130), (64, None)])
+def test_latent_attention_with_scores_that_climb_along_the_context_and_sinks(page, window):
+    """Scores grow along the context by 0 to 12 units a tile of 32 positions, up to 60 and more: a column's maximum moves in every tile, by less and by more than what
+    it may lag behind, and a maximum applied wrongly once is a factor.  Some heads' sinks are larger than every score."""
+    from geneinfer_amd.kernels import ops
+    from geneinfer_amd.parts import StepContext
+    H, kd, vd, T, p0, scale = 32, 288, 256, 150, 203, 0.1
+    g = torch.Generator().manual_seed(page)
+    total = p0 + T
+    n_pages = -(-total // page)
+    order = torch.randperm(n_pages + 2, generator=g).tolist()
+    table = torch.full((1, n_pages + 1), -1, dtype=torch.int32)
+    cache = torch.zeros(n_pages + 2, page * (kd + vd), dtype=torch.bfloat16)
+    direction = torch.nn.functional.normalize(torch.randn(kd, generator=g), dim=0)
+    height = torch.cumsum(torch.where(torch.arange(total) < 120, 0.02, torch.where(torch.arange(total) < 280, 0.35, -0.2)), 0)
+    k = (0.3 * torch.randn(total, kd, generator=g) + height[:, None] / scale / 8 * direction).to(torch.bfloat16)
+    for i in range(n_pages):
+        block = k[i * page:(i + 1) * page]
+        table[0, i] = pg = order.pop()
+        cache[pg, :block.shape[0] * kd] = block.reshape(-1)
+        values = torch.zeros(vd, page, dtype=torch.bfloat16)
+        values[:, :block.shape[0]] = block[:, :vd].T
+        cache[pg, page * kd:] = values.reshape(-1)
+    q = (8 * direction + 0.3 * torch.randn(T, H, kd, generator=g)).to(torch.bfloat16)
+    sinks = torch.where(torch.arange(H) % 5 == 0, 70.0, torch.randn(H, generator=g))
+    scores = torch.einsum("thd,sd->hts", q.double(), k.double()) * scale
+    i_, j_ = torch.arange(p0, total)[:, None], torch.arange(total)[None, :]
+    seen = (j_ <= i_) & ((i_ - j_ < window) if window else True)
+    scores = torch.cat([scores.masked_fill(~seen[None], float("-inf")), sinks.double()[:, None, None].expand(H, T, 1)], -1)
+    assert float(scores[1].max()) > 50
+    want = torch.einsum("hts,sd->thd", torch.softmax(scores, -1)[..., :-1], k[:, :vd].double()).reshape(T, H * vd)
+    pos = torch.arange(p0, total, dtype=torch.int32, device=DEV)
+    slots = torch.zeros(T, dtype=torch.int32, device=DEV)
+    ctx = StepContext(n_rows=T, dtype=torch.bfloat16, device=torch.device(DEV), tokens=slots, row_pos=pos, row_slot=slots, seg_slot=[0], seg_start=[0], seg_len=[T], seg_pos0=[p0])
+    out = torch.empty(T, H * vd, dtype=torch.bfloat16, device=DEV)
+    ops.latent_attention_bf16(q.view(T, -1).to(DEV), cache.to(DEV), out, ctx, table.to(DEV), H, kd, vd, page, window, scale, sinks.to(DEV))
+    assert relative_error(out, want) < 1.5e-2                                   # (probabilities and outputs are kept in bfloat16)
+
+
 @pytest.mark.parametrize("rows, H, k, n", [(1, 8, 32, 128), (37, 3, 72, 40), (300, 32, 64, 256), (16, 2, 256, 64), (5, 1, 8, 7)])
 def test_every_head_s_product_in_one_launch(rows, H, k, n):
     from geneinfer_amd.kernels import ops
