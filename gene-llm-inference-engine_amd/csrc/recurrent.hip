@@ -336,8 +336,117 @@ __global__ __launch_bounds__(64) void delta_prepare_kernel(const float* __restri
     for (int d = lane; d < width; d += 64) qkv[(size_t)t * n_conv + first + d] *= r;
 }
 
+// The same for the rows of prompts (up to four taps, a decay a head, query and key heads of up to 64 channels): a wave takes PREPARE_ROWS rows of an item, whose inputs it
+// asks for at once, each once, with the taps and the rows' places in their runs, and four items' waves are a workgroup (1,777 rows of 17 items as waves of
+// their own, each with its chain of places, inputs and taps: 23.2 us, so 14.7).  Every number is made as above: the same bits.
+constexpr int PREPARE_ROWS = 8, PREPARE_TAPS = 4;
+__global__ __launch_bounds__(256) void delta_prepare_rows_kernel(const float* __restrict__ proj, long ld, int conv_off, const float* __restrict__ pre_a, long lda, int b_off,
+                                                                const float* __restrict__ taps, int n_taps, const float* __restrict__ tail, long tail_stride,
+                                                                const float* __restrict__ a_log, const float* __restrict__ dt_bias, const int* __restrict__ slot,
+                                                                const int* __restrict__ pos, float* __restrict__ qkv, float* __restrict__ gates, int n_rows, int n_heads, int n_kv,
+                                                                int dk, int dv, float q_scale) {
+    const int t0 = blockIdx.x * PREPARE_ROWS, item = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int n = min(PREPARE_ROWS, n_rows - t0);
+    if (item > 2 * n_kv + n_heads) return;
+    if (item == 2 * n_kv + n_heads) {
+        for (int i = lane; i < n * n_heads; i += 64) {
+            const size_t t = t0 + i / n_heads;
+            const int h = i % n_heads;
+            gates[t * 2 * n_heads + h] = expf(-expf(a_log[h]) * softplus_f(pre_a[t * lda + h] + dt_bias[h]));
+            gates[t * 2 * n_heads + n_heads + h] = 1.0f / (1.0f + expf(-proj[t * ld + b_off + h]));
+        }
+        return;
+    }
+    // bit l of `follows`: row t0 - 2 + l belongs to the run of the row before it
+    const int mine = t0 - (PREPARE_TAPS - 2) + lane;
+    const bool there = lane < PREPARE_ROWS + PREPARE_TAPS - 2 && mine > 0 && mine < n_rows;
+    const int at = there ? mine : 0, at_before = there ? mine - 1 : 0;
+    const bool same = slot[at_before] == slot[at] && pos[at_before] == pos[at] - 1;
+    const unsigned follows = (unsigned)__ballot(there && same);
+    const int n_conv = 2 * n_kv * dk + n_heads * dv;
+    const bool unit = item < 2 * n_kv;
+    const int first = unit ? item * dk : 2 * n_kv * dk + (item - 2 * n_kv) * dv, width = unit ? dk : dv;
+    for (int d0 = 0; d0 < width; d0 += 64) {                                            // (a query or key head: once)
+        const bool live = d0 + lane < width;
+        const int c = first + min(d0 + lane, width - 1);
+        float x[PREPARE_ROWS + PREPARE_TAPS - 1], w[PREPARE_TAPS];                      // w[b]: of the row b before
+#pragma unroll
+        for (int i = 0; i < PREPARE_ROWS + PREPARE_TAPS - 1; ++i) x[i] = proj[(size_t)min(max(t0 - (PREPARE_TAPS - 1) + i, 0), n_rows - 1) * ld + conv_off + c];
+#pragma unroll
+        for (int b = 0; b < PREPARE_TAPS; ++b) w[b] = taps[(size_t)c * n_taps + max(n_taps - 1 - b, 0)];
+#pragma unroll
+        for (int i = 0; i < PREPARE_ROWS; ++i) {
+            if (i >= n) break;
+            const unsigned run = follows >> i;                                          // bits 2, 1, 0: the row, the one before it, the one before that
+            const int before = run & 4 ? (run & 2 ? (run & 1 ? 3 : 2) : 1) : 0;
+            float y = 0.f;
+#pragma unroll
+            for (int b = PREPARE_TAPS - 1; b >= 0; --b) {
+                if (b >= n_taps) continue;
+                float from = x[i + PREPARE_TAPS - 1 - b];
+                if (b > before) from = tail[(size_t)slot[t0 + i] * tail_stride + (size_t)(n_taps - 1 - (b - before)) * n_conv + c];      // (the request's rows before this step)
+                y = fmaf(w[b], from, y);
+            }
+            y = y / (1.0f + expf(-y));
+            float r = 1.0f;
+            if (unit) r = (item < n_kv ? q_scale : 1.0f) / sqrtf(wave_sum(live ? fmaf(y, y, 0.f) : 0.f) + 1e-6f);
+            if (live) qkv[(size_t)(t0 + i) * n_conv + c] = unit ? y * r : y;
+        }
+    }
+}
+
+// And for steps of single rows (two to four taps, heads of up to 64 and 128 channels): no row has one of its request's before it, and a channel's tail, input and taps
+// are asked for at once (one after the other, with the tail's places moved on in between, 5 rows took 6.9 us, so 4.6).
+__global__ __launch_bounds__(64) void delta_prepare_single_kernel(const float* __restrict__ proj, long ld, int conv_off, const float* __restrict__ pre_a, long lda, int b_off,
+                                                                 const float* __restrict__ taps, int n_taps, float* __restrict__ tail, long tail_stride,
+                                                                 const float* __restrict__ a_log, const float* __restrict__ dt_bias, const int* __restrict__ slot,
+                                                                 float* __restrict__ qkv, float* __restrict__ gates, int n_heads, int n_kv, int dk, int dv, float q_scale) {
+    const int item = blockIdx.y, lane = threadIdx.x;
+    const size_t t = blockIdx.x;
+    if (item == 2 * n_kv + n_heads) {
+        for (int h = lane; h < n_heads; h += 64) {
+            gates[t * 2 * n_heads + h] = expf(-expf(a_log[h]) * softplus_f(pre_a[t * lda + h] + dt_bias[h]));
+            gates[t * 2 * n_heads + n_heads + h] = 1.0f / (1.0f + expf(-proj[t * ld + b_off + h]));
+        }
+        return;
+    }
+    const int n_conv = 2 * n_kv * dk + n_heads * dv;
+    const bool unit = item < 2 * n_kv;
+    const int first = unit ? item * dk : 2 * n_kv * dk + (item - 2 * n_kv) * dv, width = unit ? dk : dv;
+    float* old = tail + (size_t)slot[t] * tail_stride;
+    float x[2][PREPARE_TAPS], w[2][PREPARE_TAPS];                                       // x[.][0] the row's own input, x[.][b] the one b before; w likewise
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const int c = first + min(lane + 64 * e, width - 1);
+        x[e][0] = proj[t * ld + conv_off + c];
+#pragma unroll
+        for (int b = 0; b < PREPARE_TAPS; ++b) w[e][b] = taps[(size_t)c * n_taps + max(n_taps - 1 - b, 0)];
+#pragma unroll
+        for (int b = 1; b < PREPARE_TAPS; ++b) x[e][b] = old[(size_t)max(n_taps - 1 - b, 0) * n_conv + c];
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        if (64 * e >= width) break;
+        const bool live = lane + 64 * e < width;
+        const int c = first + min(lane + 64 * e, width - 1);
+        float y = 0.f;
+#pragma unroll
+        for (int b = PREPARE_TAPS - 1; b >= 0; --b)
+            if (b < n_taps) y = fmaf(w[e][b], x[e][b], y);
+        y = y / (1.0f + expf(-y));
+        float r = 1.0f;
+        if (unit) r = (item < n_kv ? q_scale : 1.0f) / sqrtf(wave_sum(live ? fmaf(y, y, 0.f) : 0.f) + 1e-6f);
+        if (!live) continue;
+        qkv[t * n_conv + c] = unit ? y * r : y;
+#pragma unroll
+        for (int b = 0; b < PREPARE_TAPS - 1; ++b)
+            if (b < n_taps - 1) old[(size_t)(n_taps - 2 - b) * n_conv + c] = x[e][b];
+    }
+}
+
 // After a step's rows the request's tail is its last n_taps - 1 inputs: of this step's rows, and of the old tail where the step
-// brought fewer.  One workgroup per request of the step; a thread reads all it needs of a channel before it writes.
+// brought fewer.  A thread reads all it needs of a channel before it writes; a request's channels lie over the grid's second dimension
+// (one workgroup a request that went through 1,536 channels 256 at a time took 7.5 us).
 __global__ __launch_bounds__(256) void delta_tail_kernel(const float* __restrict__ proj, long ld, int conv_off, int n_conv, int n_taps,
                                                         const int* __restrict__ seg_start, const int* __restrict__ seg_len,
                                                         const int* __restrict__ slot, float* __restrict__ tail, long tail_stride) {
@@ -345,7 +454,7 @@ __global__ __launch_bounds__(256) void delta_tail_kernel(const float* __restrict
     if (n <= 0) return;
     const int t0 = seg_start[blockIdx.x], keep = n_taps - 1;
     float* mine = tail + (size_t)slot[t0] * tail_stride;
-    for (int c = threadIdx.x; c < n_conv; c += 256) {
+    for (int c = blockIdx.y * 256 + threadIdx.x; c < n_conv; c += 256 * gridDim.y) {
         float held[DELTA_MAX_TAPS];
 #pragma unroll
         for (int s = 0; s < DELTA_MAX_TAPS; ++s) {
@@ -1050,7 +1159,21 @@ GI_API int gi_delta_prepare(const float* proj, long ld, int conv_off, const floa
     GI_REQUIRE(low != nullptr ? (rank > 0 && w_up != nullptr) : (pre_a != nullptr && lda >= (long)n_heads * dn), "delta_prepare: the decays' inputs are missing or too short");
     GI_REQUIRE(state_stride >= gi_delta_state_floats(n_heads, n_kv, dk, dv, n_taps) && 2 * n_kv + 2 * n_heads <= 65535, "delta_prepare: state stride %ld too small, or too many heads", state_stride);
     dim3 grid(n_rows, 2 * n_kv + n_heads + (dn > 1 ? n_heads : 1));
-    delta_prepare_kernel<<<grid, 64, 0, stream>>>(proj, ld, conv_off, pre_a, lda, b_off, taps, n_taps, state + gi_delta_memory_floats(n_heads, dk, dv), state_stride, move_tail,
+    float* tail = state + gi_delta_memory_floats(n_heads, dk, dv);
+    const bool common = dn == 1 && low == nullptr && n_taps <= PREPARE_TAPS && dk <= 64;
+    if (common && move_tail && n_taps >= 2 && dv <= 128) {
+        delta_prepare_single_kernel<<<grid, 64, 0, stream>>>(proj, ld, conv_off, pre_a, lda, b_off, taps, n_taps, tail, state_stride, a_log, dt_bias, slot, qkv, gates, n_heads, n_kv, dk,
+                                                             dv, q_scale);
+        GI_CHECK_LAUNCH("delta_prepare (single rows)");
+        return 0;
+    }
+    if (common && !move_tail && n_rows >= 64) {
+        delta_prepare_rows_kernel<<<dim3((n_rows + PREPARE_ROWS - 1) / PREPARE_ROWS, (2 * n_kv + n_heads + 1 + 3) / 4), 256, 0, stream>>>(
+            proj, ld, conv_off, pre_a, lda, b_off, taps, n_taps, tail, state_stride, a_log, dt_bias, slot, pos, qkv, gates, n_rows, n_heads, n_kv, dk, dv, q_scale);
+        GI_CHECK_LAUNCH("delta_prepare (rows)");
+        return 0;
+    }
+    delta_prepare_kernel<<<grid, 64, 0, stream>>>(proj, ld, conv_off, pre_a, lda, b_off, taps, n_taps, tail, state_stride, move_tail,
                                                   a_log, dt_bias, slot, pos, qkv, gates, n_heads, n_kv, dk, dv, q_scale, dn, low, rank, (const bf16_t*)w_up);
     GI_CHECK_LAUNCH("delta_prepare");
     return 0;
@@ -1062,7 +1185,7 @@ GI_API int gi_delta_tail(const float* proj, long ld, int conv_off, int n_taps, c
     const long n_conv = 2L * n_kv * dk + (long)n_heads * dv;
     GI_REQUIRE(conv_off >= 0 && ld >= conv_off + n_conv && state_stride >= gi_delta_state_floats(n_heads, n_kv, dk, dv, n_taps), "delta_tail: columns outside the rows, or state stride too small");
     if (n_taps == 1) return 0;
-    delta_tail_kernel<<<n_segs, 256, 0, stream>>>(proj, ld, conv_off, (int)n_conv, n_taps, seg_start, seg_len, slot, state + gi_delta_memory_floats(n_heads, dk, dv), state_stride);
+    delta_tail_kernel<<<dim3(n_segs, n_conv < 256L * 64 ? (unsigned)((n_conv + 255) / 256) : 64), 256, 0, stream>>>(proj, ld, conv_off, (int)n_conv, n_taps, seg_start, seg_len, slot, state + gi_delta_memory_floats(n_heads, dk, dv), state_stride);
     GI_CHECK_LAUNCH("delta_tail");
     return 0;
 }

@@ -182,6 +182,40 @@ def test_gated_delta_rule_kernels(heads, kv, dk, dv, taps):
     assert torch.equal(both, alone)
 
 
+@pytest.mark.parametrize("heads, kv, dk, dv, taps", [(8, 4, 64, 128, 4), (3, 3, 20, 65, 2), (2, 1, 64, 64, 3), (2, 2, 33, 130, 4), (2, 1, 16, 24, 5), (2, 1, 16, 24, 1)])
+def test_what_the_delta_rule_reads_of_single_rows_and_of_prompts(heads, kv, dk, dv, taps):
+    """A step of single rows, each with a tail before it, in the kernel that moves the tails on, and a long step of several requests (one goes on, one begins, one of a
+    single row, more rows than a wave takes at the end): row by row in steps of their own, in bits."""
+    from geneinfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(dk + taps)
+    n_conv = 2 * kv * dk + heads * dv
+    cols, lens = n_conv + 2 * heads + 1, [5, 60, 1, 9]
+    n = sum(lens)
+    proj = torch.randn(n, cols, generator=g).to(DEV)
+    w_taps, a_log, dt_bias = (x.to(DEV) for x in (0.6 * torch.randn(n_conv, taps, generator=g), 0.3 * torch.randn(heads, generator=g), 0.5 * torch.randn(heads, generator=g)))
+    first = torch.randn(6, ops.delta_state_floats(heads, kv, dk, dv, taps) + 3, generator=g).to(DEV)
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+
+    def step(rows, slots, positions, state, single):
+        qkv, gates = torch.full((len(rows), n_conv), float("nan"), device=DEV), torch.full((len(rows), 2 * heads), float("nan"), device=DEV)
+        ops.delta_prepare(rows, 1, 1 + n_conv, 1 + n_conv - heads, w_taps, a_log, dt_bias, ints(slots), ints(positions), state, qkv, gates, heads, kv, dk, dv, dk ** -0.5, single)
+        return qkv, gates
+
+    slots = [s for s, m in zip((4, 0, 5, 2), lens) for _ in range(m)]
+    positions = [p + i for p, m in zip((7, 0, 3, 11), lens) for i in range(m)]
+    together = step(proj, slots, positions, first.clone(), False)
+    state = first.clone()
+    for t in range(n):                                           # one row at a time through the general kernels
+        one = step(proj[t:t + 1], slots[t:t + 1], positions[t:t + 1], state, False)
+        ops.delta_tail(proj[t:t + 1], 1, taps, ints([0]), ints([1]), ints(slots[t:t + 1]), state, heads, kv, dk, dv)
+        assert torch.equal(together[0][t], one[0][0]) and torch.equal(together[1][t], one[1][0]), t
+    at, moved, kept = [0, 3, 70, 74], first.clone(), first.clone()
+    rows = proj[at].contiguous()
+    single, general = step(rows, [3, 1, 0, 5], [9, 2, 4, 1], moved, True), step(rows, [3, 1, 0, 5], [9, 2, 4, 1], kept, False)
+    ops.delta_tail(rows, 1, taps, ints([0, 1, 2, 3]), ints([1] * 4), ints([3, 1, 0, 5]), kept, heads, kv, dk, dv)
+    assert torch.equal(single[0], general[0]) and torch.equal(single[1], general[1]) and torch.equal(moved, kept)
+
+
 def _rule_in_its_order(qkv, gates, M, heads, kv, dk, dv, channel):
     """The rule over one run of rows in 32 bits, every sum in the kernel's order: of a key's rows those 16 apart are one chain of fused
     multiply-adds, the 16 chains meet as a tree (place i and its mirror image, in 16, then in 8, then two apart, then neighbours).
