@@ -37,22 +37,50 @@ __device__ __forceinline__ void turn_pairs(const float* __restrict__ src, const 
     }
 }
 
+// A latent's numbers, a lane those 64 apart: up to 64 LATENT_HELD of them stay in registers, all asked for at once (read twice, 5 rows
+// of 768 and 256 + 32 numbers took 9.4 us, so 5.3); longer ones are read a second time.
+constexpr int LATENT_HELD = 16;
+template <typename TW, typename STORE>
+__device__ __forceinline__ void norm_latent(const float* __restrict__ src, const TW* __restrict__ w, int n, float eps, int lane, STORE store) {
+    float ss = 0.f;
+    if (n <= 64 * LATENT_HELD) {
+        float x[LATENT_HELD], g[LATENT_HELD];
+#pragma unroll
+        for (int i = 0; i < LATENT_HELD; ++i) {
+            if (64 * i >= n) break;
+            const int d = min(lane + 64 * i, n - 1);
+            x[i] = src[d], g[i] = load_f32(w, d);
+        }
+#pragma unroll
+        for (int i = 0; i < LATENT_HELD; ++i) {
+            if (64 * i >= n) break;
+            if (lane + 64 * i < n) ss = fmaf(x[i], x[i], ss);
+        }
+        const float r = 1.0f / sqrtf(wave_sum(ss) / (float)n + eps);
+#pragma unroll
+        for (int i = 0; i < LATENT_HELD; ++i) {
+            if (64 * i >= n) break;
+            if (lane + 64 * i < n) store(lane + 64 * i, g[i] * (r * x[i]));
+        }
+        return;
+    }
+    for (int d = lane; d < n; d += 64) ss = fmaf(src[d], src[d], ss);
+    const float r = 1.0f / sqrtf(wave_sum(ss) / (float)n + eps);
+    for (int d = lane; d < n; d += 64) store(d, load_f32(w, d) * (r * src[d]));
+}
+
 // The key/value latent at src normed, and the rotated part behind it turned, to the row's place of its page: one wave.
 template <typename TW, typename TC>
 __device__ __forceinline__ void store_latent(const float* __restrict__ src, size_t t, int kv_rank, int rot, int half_split, const TW* __restrict__ w, float eps,
                                              const float* __restrict__ cos_t, const float* __restrict__ sin_t, int p, long page, TC* __restrict__ cache, long page_stride,
                                              int page_size, int lane) {
-    float ss = 0.f;
-    for (int d = lane; d < kv_rank; d += 64) ss = fmaf(src[d], src[d], ss);
-    const float r = 1.0f / sqrtf(wave_sum(ss) / (float)kv_rank + eps);
     TC* dst = cache + page * page_stride + (size_t)(p % page_size) * (kv_rank + rot);
     TC* as_value = cache + page * page_stride + (size_t)page_size * (kv_rank + rot) + p % page_size;      // [kv_rank][place]
-    for (int d = lane; d < kv_rank; d += 64) {
-        const float c = load_f32(w, d) * (r * src[d]);
+    turn_pairs(src + kv_rank, cos_t, sin_t, t, rot, half_split, lane, dst + kv_rank);
+    norm_latent(src, w, kv_rank, eps, lane, [&](int d, float c) {
         store_f32(dst, d, c);
         store_f32(as_value, (size_t)d * page_size, c);
-    }
-    turn_pairs(src + kv_rank, cos_t, sin_t, t, rot, half_split, lane, dst + kv_rank);
+    });
 }
 
 // A head's query at src parted: its unrotated channels to `plain`, the turned ones to `turned`: one wave.
@@ -73,22 +101,21 @@ __global__ __launch_bounds__(64) void latent_prepare_kernel(const float* __restr
     const int t = blockIdx.x, lane = threadIdx.x;
     const float* src = proj + (size_t)t * ld;
     if (blockIdx.y == 0) {
-        float ss = 0.f;
-        for (int d = lane; d < q_rank; d += 64) ss = fmaf(src[d], src[d], ss);
-        const float r = 1.0f / sqrtf(wave_sum(ss) / (float)q_rank + eps);
-        for (int d = lane; d < q_rank; d += 64) store_f32(cq, (size_t)t * ldcq + d, load_f32(q_norm, d) * (r * src[d]));
+        norm_latent(src, q_norm, q_rank, eps, lane, [&](int d, float c) { store_f32(cq, (size_t)t * ldcq + d, c); });
         return;
     }
     const int p = pos[t];
     store_latent(src + q_rank, t, kv_rank, rot, half_split, kv_norm, eps, cos_t, sin_t, p, (long)table[(size_t)slot[t] * table_stride + p / page_size], cache, page_stride, page_size, lane);
 }
 
+// (Four heads' waves to a workgroup: 57,000 workgroups of a wave took 14.7 us, most of it to start them.)
 template <typename TA, typename TC>
-__global__ __launch_bounds__(64) void latent_queries_kernel(const float* __restrict__ q, long ldq, const float* __restrict__ cos_t,
+__global__ __launch_bounds__(256) void latent_queries_kernel(const float* __restrict__ q, long ldq, const float* __restrict__ cos_t,
                                                            const float* __restrict__ sin_t, TA* __restrict__ plain, long ld_plain,
-                                                           TC* __restrict__ folded, long ld_folded, int dim, int rot, int kv_rank, int half_split) {
-    const size_t t = blockIdx.x, h = blockIdx.y;
-    part_query(q + t * ldq + h * (dim + rot), t, dim, rot, half_split, cos_t, sin_t, threadIdx.x, plain + t * ld_plain + h * dim, folded + t * ld_folded + h * (kv_rank + rot) + kv_rank);
+                                                           TC* __restrict__ folded, long ld_folded, int n_heads, int dim, int rot, int kv_rank, int half_split) {
+    const size_t t = blockIdx.x, h = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (h >= (size_t)n_heads) return;
+    part_query(q + t * ldq + h * (dim + rot), t, dim, rot, half_split, cos_t, sin_t, threadIdx.x & 63, plain + t * ld_plain + h * dim, folded + t * ld_folded + h * (kv_rank + rot) + kv_rank);
 }
 
 // item 0: the row's key/value latent into its page; items 1 ..: the heads' queries.
@@ -115,43 +142,81 @@ __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) { return __builtin_bit_cast
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 constexpr float LOG2E = 1.4426950408889634f;
 
-// out[t, h*n_out + n] = sum_k a[t, h*k_dim + k] * w[h][n][k], bfloat16 operands, 32-bit sums.  One wave per (16 rows, head, 64
-// columns): the operands of the 16x16x32 matrix instruction are 16-byte pieces of a's and w's rows as they lie in memory.  With `gate`
-// (float32 [n_rows, ldg], head h's channels from h*n_out on) every result is multiplied by sigmoid(gate).
-template <typename TO>
+// out[t, h*n_out + n] = sum_k a[t, h*k_dim + k] * w[h][n][k], bfloat16 operands, 32-bit sums.  One wave per (16 RT rows, head, 16 J
+// columns): the operands of the 16x16x32 matrix instruction are 16-byte pieces of a's and w's rows as they lie in memory; w's rows come in the order that
+// leaves a lane 4 J neighbouring columns of its row, stored 16 bytes at a time.  With `gate` (float32 [n_rows, ldg], head h's channels from h*n_out on) every
+// result is multiplied by sigmoid(gate).
+// A few rows are bound by a round trip to memory (16 columns a wave, all of k asked for at once), the rows of prompts by how often w is read (64 rows a
+// wave) and by the stores: 1,777 rows of 32 heads, 64 -> 256 and 256 -> 64 channels together 45.0 us with 16 rows a wave and stores of 2 bytes, so 29.4;
+// 5 rows 11.8 with 64 columns a wave, so 7.5.
+template <typename TO, int RT, int J>
 __global__ __launch_bounds__(64) void heads_product_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restrict__ w, TO* __restrict__ out, long ldo,
                                                           long out_head_stride, int n_rows, int k_dim, int n_out, const float* __restrict__ gate, long ldg) {
     const int lane = threadIdx.x, r = lane & 15, q4 = lane >> 4;
-    const int row0 = blockIdx.x * 16, h = blockIdx.y, col0 = blockIdx.z * 64;
-    const int row = min(row0 + r, n_rows - 1);
-    const bf16_t* arow = a + (size_t)row * lda + (size_t)h * k_dim;
-    const bf16_t* wh = w + (size_t)h * n_out * k_dim;
-    floatx4 acc[4] = {floatx4{}, floatx4{}, floatx4{}, floatx4{}};
-#pragma unroll 4
+    const int row0 = blockIdx.x * (16 * RT), h = blockIdx.y, col0 = blockIdx.z * (16 * J);
+    const bf16_t* arow[RT];
+    const bf16_t* wrow[J];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) arow[i] = a + (size_t)min(row0 + 16 * i + r, n_rows - 1) * lda + (size_t)h * k_dim;
+#pragma unroll
+    for (int j = 0; j < J; ++j) wrow[j] = w + ((size_t)h * n_out + min(col0 + 4 * J * (r >> 2) + 4 * j + (r & 3), n_out - 1)) * k_dim;
+    floatx4 acc[RT][J];
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < J; ++j) acc[i][j] = floatx4{};
+#pragma unroll (RT == 1 ? 8 : 2)
     for (int k0 = 0; k0 < k_dim; k0 += 32) {
         const int k = k0 + 8 * q4;
         const bool in = k < k_dim;                       // (k_dim is a multiple of 8: a piece is inside or outside as a whole)
-        uint4 av = *reinterpret_cast<const uint4*>(arow + (in ? k : 0));
-        if (!in) av = uint4{0, 0, 0, 0};
+        uint4 av[RT], wv[J];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int col = min(col0 + 16 * j + r, n_out - 1);
-            uint4 wv = *reinterpret_cast<const uint4*>(wh + (size_t)col * k_dim + (in ? k : 0));
-            if (!in) wv = uint4{0, 0, 0, 0};
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(av), as_bf16x8(wv), acc[j], 0, 0, 0);
+        for (int i = 0; i < RT; ++i) av[i] = *reinterpret_cast<const uint4*>(arow[i] + (in ? k : 0));
+#pragma unroll
+        for (int j = 0; j < J; ++j) wv[j] = *reinterpret_cast<const uint4*>(wrow[j] + (in ? k : 0));
+        if (!in) {
+#pragma unroll
+            for (int i = 0; i < RT; ++i) av[i] = uint4{0, 0, 0, 0};
+#pragma unroll
+            for (int j = 0; j < J; ++j) wv[j] = uint4{0, 0, 0, 0};
         }
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int j = 0; j < J; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wv[j]), as_bf16x8(av[i]), acc[i][j], 0, 0, 0);
     }
-    // element v of acc[j]: row row0 + 4*q4 + v, column col0 + 16*j + r
+    // element v of acc[i][j]: row row0 + 16 i + r, column col0 + 4 J q4 + 4 j + v
+    const int col = col0 + 4 * J * q4;
+    const bool whole = col + 4 * J <= n_out && (((uintptr_t)out | (size_t)ldo * sizeof(TO) | (size_t)out_head_stride * sizeof(TO)) & (J == 1 && sizeof(TO) == 2 ? 7 : 15)) == 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int col = col0 + 16 * j + r;
+    for (int i = 0; i < RT; ++i) {
+        const int t = row0 + 16 * i + r;
+        if (t >= n_rows) break;
+        if (gate) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int t = row0 + 4 * q4 + v;
-            if (t < n_rows && col < n_out) {
-                const float y = gate ? acc[j][v] / (1.0f + expf(-gate[(size_t)t * ldg + (size_t)h * n_out + col])) : acc[j][v];
-                store_f32(out, (size_t)t * ldo + (size_t)h * out_head_stride + col, y);
+            for (int j = 0; j < J; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[i][j][v] = acc[i][j][v] / (1.0f + expf(-gate[(size_t)t * ldg + (size_t)h * n_out + min(col + 4 * j + v, n_out - 1)]));
+        }
+        TO* to = out + (size_t)t * ldo + (size_t)h * out_head_stride + col;
+        if (whole) {
+            if constexpr (sizeof(TO) == 4) {
+#pragma unroll
+                for (int j = 0; j < J; ++j) *reinterpret_cast<floatx4*>(to + 4 * j) = acc[i][j];
+            } else if constexpr (J == 1) {
+                *reinterpret_cast<uint2*>(to) = uint2{f32x2_to_bf16x2(acc[i][0][0], acc[i][0][1]), f32x2_to_bf16x2(acc[i][0][2], acc[i][0][3])};
+            } else {
+#pragma unroll
+                for (int j = 0; j < J; j += 2)
+                    *reinterpret_cast<uint4*>(to + 4 * j) = uint4{f32x2_to_bf16x2(acc[i][j][0], acc[i][j][1]), f32x2_to_bf16x2(acc[i][j][2], acc[i][j][3]),
+                                                                  f32x2_to_bf16x2(acc[i][j + 1][0], acc[i][j + 1][1]), f32x2_to_bf16x2(acc[i][j + 1][2], acc[i][j + 1][3])};
             }
+        } else {
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (col + 4 * j + v < n_out) store_f32(to, 4 * j + v, acc[i][j][v]);
         }
     }
 }
@@ -206,17 +271,40 @@ __global__ __launch_bounds__(64) void latent_attention_kernel(const bf16_t* __re
             page[b] = cache + (long)tab[j0 / page_size] * page_stride;
             place[b] = j0 % page_size;
         }
+        // The values are asked for with the keys (up to keys of 288 channels: registers): behind the scores they were a second round trip to memory, most of
+        // the time of a share of one tile (5 rows of 32 heads at 212 positions: 13.4 us, so 8.7).
+        constexpr bool EARLY = KS <= 9;
+        uint4 k_early[2][EARLY ? KS : 1];
+        uint2 v_early[2][EARLY ? DT : 1];
+        const auto value = [&](int b, int i) {
+            const int c = 16 * i + r;
+            return *reinterpret_cast<const uint2*>(page[b] + v_plane + (size_t)(c < vd ? c : 0) * page_size + place[b] + 4 * q4);
+        };
+        const auto key = [&](int b, int ks) {
+            return *reinterpret_cast<const uint4*>(page[b] + (size_t)(place[b] + r) * kd + (32 * ks + 8 * q4 < kd ? 32 * ks + 8 * q4 : 0));
+        };
+        if constexpr (EARLY) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) k_early[b][ks] = key(b, ks);
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int i = 0; i < DT; ++i) v_early[b][i] = value(b, i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         floatx4 s[2];
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             s[b] = floatx4{};
-            const bf16_t* krow = page[b] + (size_t)(place[b] + r) * kd;
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
-                const int c = 32 * ks + 8 * q4;
-                uint4 kv = *reinterpret_cast<const uint4*>(krow + (c < kd ? c : 0));
-                if (c >= kd) kv = uint4{0, 0, 0, 0};
-                s[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kv), qreg[ks], s[b], 0, 0, 0);
+                uint4 k;
+                if constexpr (EARLY) k = k_early[b][ks];
+                else k = key(b, ks);
+                if (32 * ks + 8 * q4 >= kd) k = uint4{0, 0, 0, 0};
+                s[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k), qreg[ks], s[b], 0, 0, 0);
             }
         }
         // element v of s[b]: position kv0 + 16*b + 4*q4 + v, head r
@@ -250,11 +338,10 @@ __global__ __launch_bounds__(64) void latent_attention_kernel(const bf16_t* __re
         // a block whose positions are all masked was read from another block's place: its probabilities are zeros, which is all that matters
 #pragma unroll
         for (int i = 0; i < DT; ++i) {
-            const int c = 16 * i + r;
-            const size_t ch = (size_t)(c < vd ? c : 0) * page_size;
-            uint2 v0 = *reinterpret_cast<const uint2*>(page[0] + v_plane + ch + place[0] + 4 * q4);
-            uint2 v1 = *reinterpret_cast<const uint2*>(page[1] + v_plane + ch + place[1] + 4 * q4);
-            if (c >= vd) v0 = v1 = uint2{0, 0};
+            uint2 v0, v1;
+            if constexpr (EARLY) v0 = v_early[0][i], v1 = v_early[1][i];
+            else v0 = value(0, i), v1 = value(1, i);
+            if (16 * i + r >= vd) v0 = v1 = uint2{0, 0};
 #pragma unroll
             for (int v = 0; v < 4; ++v) o[i][v] *= corr;
             o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(uint4{v0.x, v0.y, v1.x, v1.y}), as_bf16x8(pb), o[i], 0, 0, 0);
@@ -660,8 +747,8 @@ GI_API int gi_latent_queries(const float* q, long ldq, const float* cos_t, const
                n_rows, n_heads, dim, rot);
     GI_REQUIRE(ldq >= (long)n_heads * (dim + rot) && ld_plain >= (long)n_heads * dim && ld_folded >= (long)n_heads * (kv_rank + rot), "latent_queries: rows too short");
     GI_REQUIRE(rot == 0 || (cos_t != nullptr && sin_t != nullptr), "latent_queries: a rotation needs its cosines and sines");
-    dim3 grid(n_rows, n_heads);
-#define GO(TA, TC) latent_queries_kernel<TA, TC><<<grid, 64, 0, stream>>>(q, ldq, cos_t, sin_t, (TA*)plain, ld_plain, (TC*)folded, ld_folded, dim, rot, kv_rank, half_split)
+    dim3 grid(n_rows, (n_heads + 3) / 4);
+#define GO(TA, TC) latent_queries_kernel<TA, TC><<<grid, 256, 0, stream>>>(q, ldq, cos_t, sin_t, (TA*)plain, ld_plain, (TC*)folded, ld_folded, n_heads, dim, rot, kv_rank, half_split)
     if (plain_dtype == GI_F32 && folded_dtype == GI_F32) GO(float, float);
     else if (plain_dtype == GI_BF16 && folded_dtype == GI_BF16) GO(bf16_t, bf16_t);
     else if (plain_dtype == GI_F32 && folded_dtype == GI_BF16) GO(float, bf16_t);
@@ -708,11 +795,21 @@ GI_API int gi_heads_product(const void* a, long lda, const void* w, void* out, i
                n_rows, n_heads, k_dim, n_out);
     GI_REQUIRE(lda % 8 == 0 && lda >= (long)n_heads * k_dim && ((uintptr_t)a & 15) == 0 && ((uintptr_t)w & 15) == 0 && out_head_stride >= n_out &&
                ldo >= (long)(n_heads - 1) * out_head_stride + n_out, "heads_product: operands must be 16-byte aligned with row strides that are multiples of 8, and rows long enough");
-    GI_REQUIRE((n_out + 63) / 64 <= 65535, "heads_product: too many columns");
-    dim3 grid((n_rows + 15) / 16, n_heads, (n_out + 63) / 64);
-    if (out_dtype == GI_F32) heads_product_kernel<float><<<grid, 64, 0, stream>>>((const bf16_t*)a, lda, (const bf16_t*)w, (float*)out, ldo, out_head_stride, n_rows, k_dim, n_out, gate, ldg);
-    else if (out_dtype == GI_BF16) heads_product_kernel<bf16_t><<<grid, 64, 0, stream>>>((const bf16_t*)a, lda, (const bf16_t*)w, (bf16_t*)out, ldo, out_head_stride, n_rows, k_dim, n_out, gate, ldg);
+    GI_REQUIRE((n_out + 15) / 16 <= 65535, "heads_product: too many columns");
+#define GO_AS(TO, RT, J)                                                                                                                            \
+    heads_product_kernel<TO, RT, J><<<dim3((n_rows + 16 * RT - 1) / (16 * RT), n_heads, (n_out + 16 * J - 1) / (16 * J)), 64, 0, stream>>>(           \
+        (const bf16_t*)a, lda, (const bf16_t*)w, (TO*)out, ldo, out_head_stride, n_rows, k_dim, n_out, gate, ldg)
+#define GO(TO)                                  \
+    do {                                        \
+        if (n_rows <= 16) GO_AS(TO, 1, 1);      \
+        else if (n_rows <= 256) GO_AS(TO, 1, 4); \
+        else GO_AS(TO, 4, 4);                   \
+    } while (0)
+    if (out_dtype == GI_F32) GO(float);
+    else if (out_dtype == GI_BF16) GO(bf16_t);
     else return gi_fail("heads_product: unknown output dtype %d", out_dtype);
+#undef GO
+#undef GO_AS
     GI_CHECK_LAUNCH("heads_product");
     return 0;
 }
