@@ -891,26 +891,54 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
 struct TileOrder {
     int m_tiles, n_tiles, each, panel;         // each: tiles a die
     struct Tile { int m, n; };
-    __device__ __forceinline__ Tile tile(int id) const {
-        const int u = (id & 7) * each + (id >> 3);
-        if ((id >> 3) >= each || u >= m_tiles * n_tiles) return {-1, 0};
+    __device__ __forceinline__ Tile at(int u) const {
         const int in_panel = panel * m_tiles, p = u / in_panel, rest = u - p * in_panel, width = min(panel, n_tiles - p * panel);
         return {rest / width, p * panel + rest % width};
     }
 };
+// The tiles of the last, incomplete round share their k out: with at most half as many left as there are compute units, each is made by
+// `shares` workgroups, every one of which sums a part of k.  The one that comes last to its end adds the others' sums to its own, in the order of k whoever it
+// is, and goes on to the epilogue.  An earlier one leaves its sums in its place and ends.  A tile's two counters are drawn from when a workgroup has its sums
+// and raised when these are in memory: the last waits, but only for workgroups that have drawn, whose way to the second counter holds no wait of their own.
+// The sums go past the L2s, which belong to one die each (stores and loads of device scope): no fence, whose write-back of a whole L2 costs more than
+// all of this.
+struct TileShares {
+    int whole, rest, shares;                   // tiles made by one workgroup; those shared out; by how many (1: none)
+    float* sums;                               // [rest][shares][32,768], each in the order of the lanes' registers
+    unsigned* counters;                        // [rest][2 halves][2], 0 at the start and at the end
+};
+__global__ void clear_counters_kernel(unsigned* counters, int n) {
+    for (int i = threadIdx.x; i < n; i += blockDim.x) counters[i] = 0;
+}
+constexpr int TALL_MAX_SHARES = 4;
+typedef unsigned gi_uint4 __attribute__((ext_vector_type(4)));
+constexpr int DEVICE_SCOPE = 16;               // sc1 in a buffer access's cache policy
 template <int EPI>
 __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ C, int M, int N, int K,
-                                                            long lda, long ldw, long ldc, NormIn norm_in, RopeStore rope, NormOut norm_out, TileOrder order, bool quick_gate) {
-    const TileOrder::Tile at_tile = order.tile(blockIdx.x);
-    if (at_tile.m < 0) return;
+                                                            long lda, long ldw, long ldc, NormIn norm_in, RopeStore rope, NormOut norm_out, TileOrder order, TileShares shared, bool quick_gate) {
+    int u, share = 0;
+    bool part = false;
+    if ((int)blockIdx.x < 8 * order.each) {
+        u = (blockIdx.x & 7) * order.each + (blockIdx.x >> 3);
+        if (u >= shared.whole) return;
+    } else {                                                                            // (a die's shares are of neighbouring tiles and mostly of one part of k)
+        const int id = blockIdx.x - 8 * order.each, pieces = shared.rest * shared.shares, each = (pieces + 7) / 8, piece = (id & 7) * each + (id >> 3);
+        if ((id >> 3) >= each || piece >= pieces) return;
+        share = piece / shared.rest;
+        u = shared.whole + piece - share * shared.rest;
+        part = true;
+    }
+    const TileOrder::Tile at_tile = order.at(u);
     constexpr int BM = 256, BN = 128, NT = 512, TM = 2, TN = 2, ROWS = BM + BN, STAGE_BYTES = ROWS * 128, LOADS = 6;
     extern __shared__ __attribute__((aligned(16))) unsigned char ring[];               // 3 * STAGE_BYTES
-    const int tid = threadIdx.x, lane = tid & 63;
+    int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), group = wave >> 2, turn = wave & 3;
     const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
     const int m0 = at_tile.m * BM, n0 = at_tile.n * BN;
-    const bf16_t* a_tile = A + (size_t)m0 * lda;
-    const bf16_t* w_tile = W + (size_t)n0 * ldw;
+    const int all_blocks = K / PK, first_block = part ? all_blocks * share / shared.shares : 0;
+    const int n_k = (part ? all_blocks * (share + 1) / shared.shares : all_blocks) - first_block;
+    const bf16_t* a_tile = A + (size_t)m0 * lda + (size_t)first_block * PK;
+    const bf16_t* w_tile = W + (size_t)n0 * ldw + (size_t)first_block * PK;
     auto source = [&](int row) -> unsigned {                                            // where this lane's 16 bytes of a stage's row lie, in bytes from the tile's first row of A or of W at k = 0
         const int c = (lane & 7) ^ ((row >> 1) & 7);
         return row < BM ? (unsigned)(((size_t)min(row, M - 1 - m0) * lda + 8 * c) * 2) : (unsigned)(((size_t)min(row - BM, N - 1 - n0) * ldw + 8 * c) * 2);
@@ -928,7 +956,6 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(src[i]), "s"(base) : "memory", "m0");
         }
     };
-    const int n_k = K / PK;
     auto phase_barrier = [&]() {
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
@@ -1015,34 +1042,21 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
     if (group == 0) phase_barrier();
     // Element v of a lane's 32x32 result: row 8*(v/4) + 4*(lane/32) + v%4, column lane%32.  The sums leave through LDS (the ring is free:
     // every wave has passed the barrier behind its last read), a group's 128 rows at a time.
-    TileOld<NT> old[2];
-    if constexpr (EPI == EPI_ADD_F32) {
-        if (norm_out.scaled != nullptr) {
-            tile_old<NT>(old[0], (const float*)C, ldc, m0, n0, M);
-            tile_old<NT>(old[1], (const float*)C, ldc, m0 + 128, n0, M);
-        }
-    }
     float* tile = reinterpret_cast<float*>(ring);
+    auto lay_out = [&](int half, int i, int j, const floatx16& sums) {
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        const int first = m0 + half * 128;
-        if (first >= M) break;
-        if (group == half) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const int row = wm - half * 128 + i * 32 + 8 * (v / 4) + 4 * (lane >> 5) + (v & 3);
-                        tile[row * 128 + wn + j * 32 + (lane & 31)] = scaled_rows ? acc[i][j][v] * row_scale[half * 128 + row] : acc[i][j][v];
-                    }
+        for (int v = 0; v < 16; ++v) {
+            const int row = wm - half * 128 + i * 32 + 8 * (v / 4) + 4 * (lane >> 5) + (v & 3);
+            tile[row * 128 + wn + j * 32 + (lane & 31)] = scaled_rows ? sums[v] * row_scale[half * 128 + row] : sums[v];
         }
+    };
+    auto leave = [&](int half, const TileOld<NT>& old) {                                 // (all of the half's rows are laid out)
+        const int first = m0 + half * 128;
         __syncthreads();
         if constexpr (EPI == EPI_QKV_ROPE) {
             qkv_tile_rope_store<NT>(tile, places[half], first, n0, M, N, rope);
         } else if (EPI == EPI_ADD_F32 && norm_out.scaled != nullptr) {
-            tile_add_handing_norm<NT>(tile, old[half], (float*)C, ldc, first, n0, M, norm_out, at_tile.n, order.n_tiles);
+            tile_add_handing_norm<NT>(tile, old, (float*)C, ldc, first, n0, M, norm_out, at_tile.n, order.n_tiles);
         } else if constexpr (is_gated(EPI)) {
             // Columns 32b .. 32b+15 are gates, 32b+16 .. 32b+31 the ups of outputs 16b .. 16b+15; a thread makes two neighbouring outputs.
             // The quick gate is the ping-pong kernel's, whose products with many tiles these may be; the others have the gate of the
@@ -1096,6 +1110,90 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
             }
         }
         __syncthreads();
+    };
+    const bool hands_norm = EPI == EPI_ADD_F32 && norm_out.scaled != nullptr;
+    if (!part) {
+        TileOld<NT> old[2];
+        if (hands_norm) {
+            tile_old<NT>(old[0], (const float*)C, ldc, m0, n0, M);
+            tile_old<NT>(old[1], (const float*)C, ldc, m0 + 128, n0, M);
+        }
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            if (m0 + half * 128 >= M) break;
+            if (group == half) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) lay_out(half, i, j, acc[i][j]);
+            }
+            leave(half, old[half]);
+        }
+        return;
+    }
+    // A half at a time: first the one that another share would rather finish.
+    __shared__ unsigned drawn[2];
+    unsigned* const counters = shared.counters + (u - shared.whole) * 4;
+    float* const places_of_tile = shared.sums + (size_t)(u - shared.whole) * shared.shares * (BM * BN);
+    auto place = [&](int of) { return __builtin_amdgcn_make_buffer_rsrc(places_of_tile + (size_t)of * (BM * BN), 0, BM * BN * 4, 0x00027000); };
+    const int at = (wave * TM * TN * 4 * 64 + lane) * 16;                                // four registers a lane and store: a wave's are 1 KB together
+#pragma unroll 1
+    for (int turn_of = 0; turn_of < 2; ++turn_of) {
+        int half = (share & 1) ^ 1 ^ turn_of;
+        asm volatile("" : "+s"(half), "+v"(tid), "+v"(lane));                            // (the compiler would keep what both turns share in registers that the sums need)
+        if (m0 + half * 128 >= M) continue;                                             // (nobody has rows there)
+        unsigned* const counter = counters + 2 * half;
+        if (tid == 0) drawn[turn_of] = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if ((int)drawn[turn_of] + 1 < shared.shares) {
+            if (group == half) {
+                const auto mine = place(share);
+#pragma unroll
+                for (int f = 0; f < TM * TN * 4; ++f) {
+                    const floatx16& from = acc[f >> 3][(f >> 2) & 1];
+                    const int v = (f & 3) * 4;
+                    __builtin_amdgcn_raw_buffer_store_b128(gi_uint4{__float_as_uint(from[v]), __float_as_uint(from[v + 1]), __float_as_uint(from[v + 2]), __float_as_uint(from[v + 3])},
+                                                           mine, at, f * 1024, DEVICE_SCOPE);
+                }
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                         // this wave's sums are in memory
+            }
+            __syncthreads();
+            if (tid == 0) __hip_atomic_fetch_add(counter + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            continue;
+        }
+        TileOld<NT> old;
+        if (hands_norm) tile_old<NT>(old, (const float*)C, ldc, m0 + half * 128, n0, M);
+        if (tid == 0)
+            while ((int)__hip_atomic_load(counter + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 < shared.shares) __builtin_amdgcn_s_sleep(1);
+        __syncthreads();
+        if (tid < 2) __hip_atomic_store(counter + tid, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // as the next product of the step wants them
+        if (group == half) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                floatx16 total[TN];
+#pragma unroll
+                for (int j = 0; j < TN; ++j) total[j] = floatx16{};
+#pragma unroll 1
+                for (int of = 0; of < shared.shares; ++of) {
+                    if (of == share) {
+#pragma unroll
+                        for (int j = 0; j < TN; ++j) total[j] += acc[i][j];
+                        continue;
+                    }
+                    const auto theirs = place(of);
+                    gi_uint4 sums[TN * 4];
+#pragma unroll
+                    for (int f = 0; f < TN * 4; ++f) sums[f] = __builtin_amdgcn_raw_buffer_load_b128(theirs, at, (i * TN * 4 + f) * 1024, DEVICE_SCOPE);
+#pragma unroll
+                    for (int f = 0; f < TN * 4; ++f)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) total[f >> 2][(f & 3) * 4 + e] += __uint_as_float(sums[f][e]);
+                }
+#pragma unroll
+                for (int j = 0; j < TN; ++j) lay_out(half, i, j, total[j]);
+            }
+        }
+        leave(half, old);
     }
 }
 
@@ -1860,13 +1958,6 @@ GI_API int gi_gemm_bf16_piped_splits(int M, int N, int K) {
     return splits;
 }
 
-// Floats of scratch a product of these sizes needs (partial sums of k-splits), 0 if none.
-GI_API long gi_gemm_bf16_scratch_floats(int M, int N, int K) {
-    if (M <= SKINNY_MAX_ROWS) return (long)gi_gemm_bf16_skinny_splits(N, K) * M * N;
-    const int splits = gi_gemm_bf16_piped_splits(M, N, K);
-    return splits > 1 ? (long)splits * M * N : 0;
-}
-
 // The most pieces a reader of M rows takes: what a writer of as many rows makes.
 static int consumer_max_parts(int M) { return M <= 16 ? slim_max_parts(M) : M <= 32 ? TILES_MAX_PARTS : REDUCE_MAX_PARTS; }
 
@@ -1884,7 +1975,30 @@ static bool many_tiles(int M, int N) { return (long)((M + 255) / 256) * ((N + 25
 // 4,096 x 1,536 the same either way; 2,048 rows of 5,120 x 1,024 rotated 36 and 42).  Only the two larger tiles finish a
 // norm handed on to a gated product; the q/k/v product's epilogue rotates tiles 128 columns wide.
 enum Large { PIPED_128, TALL_256, PINGPONG_256 };
-static Large large_kernel(int M, int N, int K, int epi, bool rope, bool hands_norm, bool scaled_rows) {
+
+// How the tall kernel's tiles are made (`TileShares`): a last round of at most half as many tiles as there are compute units in shares of k, where
+// that is the faster way.  `us`: what all of it takes.  A block of k takes longer with the whole chip at work on different parts of k (0.85 us), a tile ends
+// some 5 us later for the exchange, and 2 for every share.  Alone, 2,048 rows of 2,048 x 8,192 take 76 us in two shares (95 as 128 x 128 tiles, one a unit),
+// of 2,048 x 4,096 47 (58), of 2,048 x 2,048 33 (31: not taken); 3,000 rows of 3,072 x 8,192, one round and 32 tiles, 163 in four shares and 180 in two
+// (203 in two rounds), of 3,072 x 3,072 83 (96); 2,048 rows of 5,120 x 3,072 76 in four (78).  Fewer than 8 blocks a share are not worth the exchange.
+struct TallCut { int whole, rest, shares; double us; };
+static TallCut tall_cut(int M, int N, int K, bool may_share) {
+    const int units = gi_compute_units(), tiles = ((M + 255) / 256) * ((N + 127) / 128), rest = tiles % units;
+    const double blocks = K / PK, each = blocks * 0.715 + 13;
+    TallCut cut = {tiles, 0, 1, (tiles + units - 1) / units * each};
+    if (!may_share || rest == 0 || 2 * rest > units) return cut;
+    const double before = tiles / units * each, whole = cut.us;
+    for (int shares = 2; shares * rest <= units && shares <= TALL_MAX_SHARES && blocks >= 8 * shares; ++shares) {
+        const double us = before + ((int)blocks + shares - 1) / shares * 0.85 + 16 + 2 * shares;
+        if (us < 0.95 * whole && us < cut.us) cut = {tiles - rest, rest, shares, us};
+    }
+    return cut;
+}
+// Floats of scratch for it: the counters, then the sums.
+static long tall_counter_floats(const TallCut& cut) { return (4L * cut.rest + 63) / 64 * 64; }
+static long tall_scratch_floats(const TallCut& cut) { return cut.shares > 1 ? tall_counter_floats(cut) + (long)cut.rest * cut.shares * 256 * 128 : 0; }
+
+static Large large_kernel(int M, int N, int K, int epi, bool rope, bool hands_norm, bool scaled_rows, bool may_share) {
     const long units = gi_compute_units(), m128 = (M + 127) / 128, m256 = (M + 255) / 256, n128 = (N + 127) / 128, n256 = (N + 255) / 256;
     const auto rounds = [&](long tiles) { return (double)((tiles + units - 1) / units); };
     const bool many = many_tiles(M, N), gated = !rope && is_gated(epi);
@@ -1895,14 +2009,31 @@ static Large large_kernel(int M, int N, int K, int epi, bool rope, bool hands_no
     else if (hands_norm || (!many && epi == EPI_STORE_BF16)) ends = {8, 4};
     else if (!many && epi == EPI_STORE_F32) ends = {9, 8.4};
     const double blocks = K / PK, small = rounds(m128 * n128);
-    double piped = small > 1 ? small * (blocks * 0.45 + ends.each) * (small > 2 ? 1.15 : 1) - ends.less : blocks * 0.55 + 12;      // (several: two workgroups a unit)
+    // (one: measured 31 us at 32 blocks, 50 to 58 at 64, 95 at 128)
+    double piped = small > 1 ? small * (blocks * 0.45 + ends.each) * (small > 2 ? 1.15 : 1) - ends.less : blocks * 0.65 + 10.5;      // (several: two workgroups a unit)
     if (scaled_rows && !rope) piped = 1e30;
-    const double tall = rounds(m256 * n128) * (blocks * 0.715 + 13);
+    const double tall = tall_cut(M, N, K, may_share).us;
     const double pingpong = many && !rope ? rounds(m256 * n256) * (blocks * 1.45 + 14) : 1e30;
     // (gating 256 x 128 sums at a time costs the tall kernel 3 us a round more: 1,500 rows by 16,384 of 2,048, three rounds of it against one and a
     // half of the ping-pong kernel: 114 us against 103)
     if (pingpong < piped && 0.95 * pingpong <= tall + (gated ? 3 * rounds(m256 * n128) : 0)) return PINGPONG_256;
     return tall < piped ? TALL_256 : PIPED_128;
+}
+static Large large_kernel_of_kind(int M, int N, int K, int kind) {               // kinds as for gi_gemm_bf16_large_kernel
+    const int epi = kind == 0 ? EPI_STORE_F32 : kind <= 2 ? EPI_ADD_F32 : kind == 6 ? EPI_XIELU : EPI_GATED_BF16;
+    return large_kernel(M, N, K, epi, kind == 5, kind == 2, kind == 4, kind != 6);
+}
+
+// Floats of scratch a product of these sizes needs (partial sums where k is shared out), 0 if none.
+GI_API long gi_gemm_bf16_scratch_floats(int M, int N, int K) {
+    if (M <= SKINNY_MAX_ROWS) return (long)gi_gemm_bf16_skinny_splits(N, K) * M * N;
+    const int splits = gi_gemm_bf16_piped_splits(M, N, K);
+    if (splits > 1) return (long)splits * M * N;
+    if (K % PK != 0 || N < 128) return 0;
+    const long shared = tall_scratch_floats(tall_cut(M, N, K, true));
+    for (int kind = 0; shared > 0 && kind < 6; ++kind)
+        if (large_kernel_of_kind(M, N, K, kind) == TALL_256) return shared;
+    return 0;
 }
 
 static const NormIn NO_NORM_IN = {nullptr, 0, 0.f, 1, 0.f};
@@ -2107,10 +2238,10 @@ static int launch_skinny(const void* A, const void* W, void* C, int epi, int M, 
     return reduce_partials(scratch, C, epi, M, N, splits, ldc, stream, norm_in, norm_out, whole);
 }
 
-static TileOrder tall_order(int M, int N) {
+static TileOrder tall_order(int M, int N, int whole) {
     TileOrder o = {(M + 255) / 256, (N + 127) / 128, 0, 1};
-    o.each = (o.m_tiles * o.n_tiles + 7) / 8;
-    const int run = o.each < gi_compute_units() / 8 ? o.each : gi_compute_units() / 8;       // of a die at a time
+    o.each = (whole + 7) / 8;
+    const int all = (o.m_tiles * o.n_tiles + 7) / 8, run = all < gi_compute_units() / 8 ? all : gi_compute_units() / 8;       // of a die at a time
     while ((o.panel + 1) * (o.panel + 1) <= 2 * run) ++o.panel;
     if (o.panel * o.m_tiles < run) o.panel = (run + o.m_tiles - 1) / o.m_tiles;
     if (o.panel > o.n_tiles) o.panel = o.n_tiles;
@@ -2131,7 +2262,8 @@ static int large_norm_parts(int M, int N, int K) {
 // More than 128 rows, K a multiple of 64, 128 columns or more: the kernels that load their operands straight into LDS.
 // `rope` != null: the sums are those of an attention layer's q/k/v product and go where it says (`epi` is then not looked at).
 static int launch_large(const void* A, const void* W, void* C, int epi, int M, int N, int K, long lda, long ldw, long ldc, float* scratch,
-                        long scratch_floats, NormIn norm_in, const RopeStore* rope, hipStream_t stream, NormOut norm_out = NO_NORM_OUT, const WholeNorm* whole = nullptr) {
+                        long scratch_floats, NormIn norm_in, const RopeStore* rope, hipStream_t stream, NormOut norm_out = NO_NORM_OUT, const WholeNorm* whole = nullptr,
+                        unsigned* counters = nullptr) {
     const NormIn limit_in = {nullptr, 0, 0.f, 1, norm_in.limit};          // no norm to finish, the clamped gate's limit alone
 #define PIPED(BM_, BN_, WM_, WN_, ST_, EPI_, OUT_, LDC_, SPLITS_, KPS_, SLAB_, NORM_, ROPE_)                                            \
     do {                                                                                                                                \
@@ -2176,7 +2308,10 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
     GI_REQUIRE(norm_in.squares == nullptr || rope != nullptr || (is_gated(epi) && many_tiles(M, N) && norm_in.parts <= PIPED_MAX_PARTS),
                "gemm_bf16: a product of M %d, N %d, K %d takes no norm handed on in %d pieces", M, N, K, norm_in.parts);
     GI_REQUIRE(!many_tiles(M, N) || (lda < (1L << 22) && ldw < (1L << 22)), "gemm_bf16: row strides %ld, %ld are too large for the tile-relative addressing", lda, ldw);
-    const Large which = lda < (1L << 22) && ldw < (1L << 22) ? large_kernel(M, N, K, epi, rope != nullptr, norm_out.scaled != nullptr, norm_in.squares != nullptr) : PIPED_128;
+    const long sharing = tall_scratch_floats(tall_cut(M, N, K, true));
+    const bool may_share = sharing > 0 && scratch != nullptr && scratch_floats >= sharing && ((uintptr_t)scratch & 15) == 0;
+    const Large which = lda < (1L << 22) && ldw < (1L << 22)
+                            ? large_kernel(M, N, K, epi, rope != nullptr, norm_out.scaled != nullptr, norm_in.squares != nullptr, may_share) : PIPED_128;
     if (which == PINGPONG_256) {
 #define PINGPONG(EPI_)                                                                                                                  \
     do {                                                                                                                                \
@@ -2198,6 +2333,13 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
         return 0;
     }
     if (which == TALL_256) {
+        const TallCut cut = tall_cut(M, N, K, may_share);
+        const TileOrder order = tall_order(M, N, cut.whole);
+        const TileShares shared = {cut.whole, cut.rest, cut.shares, cut.shares > 1 ? scratch + tall_counter_floats(cut) : nullptr, counters != nullptr ? counters : (unsigned*)scratch};
+        if (cut.shares > 1 && counters == nullptr) {                                     // (5.5 us)
+            clear_counters_kernel<<<1, 256, 0, stream>>>(shared.counters, 4 * cut.rest);
+            GI_CHECK_LAUNCH("gemm_bf16 (counters)");
+        }
 #define TALL(EPI_)                                                                                                                      \
     do {                                                                                                                                \
         constexpr int bytes = 3 * 384 * 128;                                                                                            \
@@ -2207,10 +2349,9 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
                 return gi_fail("gemm_bf16: cannot reserve %d bytes of LDS", bytes);                                                     \
             raised = true;                                                                                                              \
         }                                                                                                                               \
-        const TileOrder order = tall_order(M, N);                                                                                       \
-        dim3 grid(8 * order.each);                                                                                                      \
+        dim3 grid(8 * order.each + (cut.shares > 1 ? (cut.rest * cut.shares + 7) / 8 * 8 : 0));                                          \
         gemm_bf16_tall_kernel<EPI_><<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldw, ldc, norm_in, \
-                                                                  rope != nullptr ? *rope : NO_ROPE, norm_out, order, many_tiles(M, N)); \
+                                                                  rope != nullptr ? *rope : NO_ROPE, norm_out, order, shared, many_tiles(M, N)); \
     } while (0)
         if (rope != nullptr) TALL(EPI_QKV_ROPE); else if (epi == EPI_STORE_F32) TALL(EPI_STORE_F32); else if (epi == EPI_ADD_F32) TALL(EPI_ADD_F32);
         else if (epi == EPI_XIELU) TALL(EPI_XIELU);
@@ -2263,7 +2404,7 @@ GI_API int gi_gemm_bf16_takes_norm(int M, int N, int K, int gated) {
 // pieces of the rows' sums of C^2, for the next product.  Where the two queries above say no, it fails.
 GI_API int gi_gemm_bf16_handing(const void* A, const void* W, void* C, int c_dtype, int accumulate, int gated, float gate_limit, int M, int N, int K, long lda,
                                 long ldw, long ldc, float* scratch, long scratch_floats, const float* squares_in, int parts_in, float eps,
-                                const float* g, void* scaled_out, long ld_scaled, float* squares_out, hipStream_t stream) {
+                                const float* g, void* scaled_out, long ld_scaled, float* squares_out, unsigned* counters, hipStream_t stream) {
     GI_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_bf16: M %d, N %d, K %d must be positive", M, N, K);
     GI_REQUIRE(K % 8 == 0 && lda % 8 == 0 && ldw % 8 == 0, "gemm_bf16: K %d and the row strides (%ld, %ld) must be multiples of 8", K, lda, ldw);
     GI_REQUIRE(((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0, "gemm_bf16: operands must be 16-byte aligned");
@@ -2292,7 +2433,7 @@ GI_API int gi_gemm_bf16_handing(const void* A, const void* W, void* C, int c_dty
     if (M > SKINNY_MAX_ROWS) {                   // the rows of prompts: a norm is handed on (to a q/k/v product that takes it), none is taken
         GI_REQUIRE(scaled_out == nullptr || (ldc % 4 == 0 && ld_scaled % 4 == 0 && ((uintptr_t)C & 15) == 0 && ((uintptr_t)scaled_out & 7) == 0 && ((uintptr_t)g & 15) == 0),
                    "gemm_bf16: handing a norm on from %d rows needs aligned operands", M);
-        return launch_large(A, W, C, epi, M, N, K, lda, ldw, ldc, scratch, scratch_floats, norm_in, nullptr, stream, norm_out);
+        return launch_large(A, W, C, epi, M, N, K, lda, ldw, ldc, scratch, scratch_floats, norm_in, nullptr, stream, norm_out, nullptr, counters);
     }
     return launch_skinny(A, W, C, epi, M, N, K, lda, ldw, ldc, scratch, scratch_floats, norm_in, norm_out, stream);
 }
@@ -2343,7 +2484,7 @@ GI_API int gi_gemm_bf16_qkv_rope_store_max_parts(int M, int N, int K) {
 GI_API int gi_gemm_bf16_qkv_rope_store(const void* A, const void* W, int M, int N, int K, long lda, long ldw, float* scratch, long scratch_floats,
                                        const float* squares_in, int parts_in, float eps, const float* cos_t, const float* sin_t, const int* pos,
                                        const int* slot, const int* table, int table_stride, void* q_out, void* cache, long page_stride, int page_size,
-                                       int n_heads, int n_kv, int hd, hipStream_t stream) {
+                                       int n_heads, int n_kv, int hd, unsigned* counters, hipStream_t stream) {
     GI_REQUIRE(M > 0 && N > 0 && K > 0 && n_heads > 0 && n_kv > 0 && hd > 0 && N == (n_heads + 2 * n_kv) * hd,
                "gemm_bf16 (q/k/v): M %d, N %d, K %d, %d heads, %d key/value heads of %d do not fit together", M, N, K, n_heads, n_kv, hd);
     GI_REQUIRE(K % 8 == 0 && lda % 8 == 0 && ldw % 8 == 0 && lda >= K && ldw >= K, "gemm_bf16: K %d and the row strides (%ld, %ld) must be multiples of 8", K, lda, ldw);
@@ -2358,7 +2499,8 @@ GI_API int gi_gemm_bf16_qkv_rope_store(const void* A, const void* W, int M, int 
                "gemm_bf16 (q/k/v): %d pieces of a sum of squares, at most %d", parts_in, gi_gemm_bf16_qkv_rope_store_max_parts(M, N, K));
     const RopeStore rope = {cos_t, sin_t, pos, slot, table, table_stride, (bf16_t*)q_out, (bf16_t*)cache, page_stride, page_size, n_heads, n_kv, hd};
     if (M > SKINNY_MAX_ROWS)
-        return launch_large(A, W, nullptr, EPI_STORE_F32, M, N, K, lda, ldw, (long)N, scratch, scratch_floats, NormIn{squares_in, parts_in, eps, K}, &rope, stream);
+        return launch_large(A, W, nullptr, EPI_STORE_F32, M, N, K, lda, ldw, (long)N, scratch, scratch_floats, NormIn{squares_in, parts_in, eps, K}, &rope, stream, NO_NORM_OUT, nullptr,
+                            counters);
     return launch_skinny(A, W, nullptr, EPI_STORE_F32, M, N, K, lda, ldw, (long)N, scratch, scratch_floats, NormIn{squares_in, parts_in, eps, K}, NO_NORM_OUT,
                          stream, &rope);
 }
@@ -2369,9 +2511,17 @@ GI_API int gi_gemm_bf16_qkv_rope_store(const void* A, const void* W, int M, int 
 GI_API int gi_gemm_bf16_large_kernel(int M, int N, int K, int kind) {
     if (M <= SKINNY_MAX_ROWS || K % PK != 0 || N < 128 || kind < 0 || kind > 6) return -1;
     if (gi_gemm_bf16_piped_splits(M, N, K) > 1) return 3;
-    const int epi = kind == 0 ? EPI_STORE_F32 : kind <= 2 ? EPI_ADD_F32 : kind == 6 ? EPI_XIELU : EPI_GATED_BF16;
-    return large_kernel(M, N, K, epi, kind == 5, kind == 2, kind == 4);
+    return large_kernel_of_kind(M, N, K, kind);
 }
+
+// By how many workgroups each tile of the last round is made where the tiles of 256 x 128 make such a product with all the scratch it asks for (1: one).
+GI_API int gi_gemm_bf16_tall_shares(int M, int N, int K) {
+    return M <= SKINNY_MAX_ROWS || K % PK != 0 || N < 128 || gi_gemm_bf16_piped_splits(M, N, K) > 1 ? 1 : tall_cut(M, N, K, true).shares;
+}
+
+// So many 32-bit counters, all 0, are what a product may be given as `counters`; it leaves them 0 again.  Without (null) it makes its own with a launch.  Products
+// that may run at the same time must not be given the same.
+GI_API int gi_gemm_bf16_counters() { return 2 * gi_compute_units(); }
 
 // Whether gi_gemm_bf16_xielu takes a product of these sizes: up to 16 rows where the kernel for those serves; the rows of prompts
 // where all of a tile's k is one workgroup's, with all columns through the activation.
@@ -2402,7 +2552,7 @@ GI_API int gi_gemm_bf16_xielu(const void* A, const void* W, void* C, int M, int 
 // `gated` != 0: W is [gate; up] interleaved in groups of 16 rows (N rows in all, a multiple of 32)
 // and C is bfloat16 [M, N/2] = silu(gate) * up.
 GI_API int gi_gemm_bf16(const void* A, const void* W, void* C, int c_dtype, int accumulate, int gated, float gate_limit, int M, int N, int K, long lda,
-                        long ldw, long ldc, float* scratch, long scratch_floats, hipStream_t stream) {
+                        long ldw, long ldc, float* scratch, long scratch_floats, unsigned* counters, hipStream_t stream) {
     GI_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_bf16: M %d, N %d, K %d must be positive", M, N, K);
     GI_REQUIRE(K % 8 == 0 && lda % 8 == 0 && ldw % 8 == 0, "gemm_bf16: K %d and the row strides (%ld, %ld) must be multiples of 8", K, lda, ldw);
     GI_REQUIRE(((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0, "gemm_bf16: operands must be 16-byte aligned");
@@ -2421,7 +2571,7 @@ GI_API int gi_gemm_bf16(const void* A, const void* W, void* C, int c_dtype, int 
     if (M <= SKINNY_MAX_ROWS) return launch_skinny(A, W, C, epi, M, N, K, lda, ldw, ldc, scratch, scratch_floats, plain_in, NO_NORM_OUT, stream);
 
     GI_REQUIRE((M + 63) / 64 <= 65535, "gemm_bf16: M %d is too large", M);
-    if (K % PK == 0 && N >= 128) return launch_large(A, W, C, epi, M, N, K, lda, ldw, ldc, scratch, scratch_floats, plain_in, nullptr, stream);
+    if (K % PK == 0 && N >= 128) return launch_large(A, W, C, epi, M, N, K, lda, ldw, ldc, scratch, scratch_floats, plain_in, nullptr, stream, NO_NORM_OUT, nullptr, counters);
 #define TILED(BM_, EPI_) gemm_bf16_tiled_kernel<BM_, EPI_><<<grid, 256, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldw, ldc, gate_limit)
     if ((long)((M + 127) / 128) * ((N + BN - 1) / BN) < 512) {   // few tiles: smaller ones fill more of the chip
         dim3 grid((N + BN - 1) / BN, (M + 63) / 64);

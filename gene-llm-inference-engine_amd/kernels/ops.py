@@ -99,7 +99,7 @@ _SIGNATURES = {
     "gi_mlstm_scan": [c_void_p, c_long, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float, c_float, c_void_p, c_void_p, c_int, c_void_p,
                       c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_int, c_int, c_void_p],
     "gi_head_norm_gate": [c_void_p, c_long, c_void_p, c_void_p, c_long, c_void_p, c_int, c_void_p, c_int, c_long, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p],
-    "gi_gemm_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long, c_void_p],
+    "gi_gemm_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long, c_void_p, c_void_p],
     "gi_attention_prompt_bf16": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int,
                                  c_float, c_int, c_void_p, c_void_p, c_int, c_void_p, c_long, c_int, c_void_p, c_void_p, c_long, c_int, c_float, c_void_p],
     "gi_attention_decode_bf16": [c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_long, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
@@ -111,9 +111,9 @@ _SIGNATURES = {
     "gi_probe_mfma": [c_int, c_void_p, c_int, c_void_p],
     "gi_gemm_bf16_onto_norm": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long, c_void_p, c_float, c_void_p, c_long, c_void_p],
     "gi_gemm_bf16_handing": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long,
-                             c_void_p, c_int, c_float, c_void_p, c_void_p, c_long, c_void_p, c_void_p],
+                             c_void_p, c_int, c_float, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_void_p],
     "gi_gemm_bf16_qkv_rope_store": [c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_void_p, c_long, c_void_p, c_int, c_float, c_void_p, c_void_p,
-                                    c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_int, c_void_p],
+                                    c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_int, c_void_p, c_void_p],
     "gi_argmax": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_long, c_void_p],
     "gi_sample_temperature": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_long, c_void_p],
     "gi_sample_filtered": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_long, c_void_p],
@@ -150,6 +150,10 @@ def lib():
         l.gi_gemm_bf16_scratch_floats.restype = c_long
         l.gi_gemm_bf16_norm_parts.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_bf16_norm_parts.restype = c_int
+        l.gi_gemm_bf16_tall_shares.argtypes = [c_int, c_int, c_int]
+        l.gi_gemm_bf16_tall_shares.restype = c_int
+        l.gi_gemm_bf16_counters.argtypes = []
+        l.gi_gemm_bf16_counters.restype = c_int
         l.gi_gemm_bf16_large_kernel.argtypes = [c_int, c_int, c_int, c_int]
         l.gi_gemm_bf16_large_kernel.restype = c_int
         l.gi_gemm_bf16_onto_norm_takes.argtypes = [c_int, c_int, c_int]
@@ -1541,6 +1545,28 @@ def _scratch_floats(m, n, k) -> int:
 
 
 @lru_cache(maxsize=8192)
+def gemm_bf16_tall_shares(m, n, k) -> int:
+    """By how many workgroups the last tiles of a product of these sizes are made, where the tiles of 256 x 128 make it (1: one)."""
+    return lib().gi_gemm_bf16_tall_shares(m, n, k)
+
+
+def step_counters(ctx, m, n, k):
+    """`counters` for a product of these sizes in the step `ctx`: the step's own, filled once and left as they were by every product (a step's products run one
+    after the other); None for a product that has no use for them."""
+    if ctx is None or gemm_bf16_tall_shares(m, n, k) == 1:
+        return None
+    counters = ctx.memo.get("product_counters")
+    if counters is None:
+        counters = ctx.memo["product_counters"] = torch.zeros(lib().gi_gemm_bf16_counters(), dtype=torch.int32, device=ctx.device)
+    return counters
+
+
+def _check_counters(counters):
+    if counters is not None and not (counters.dtype == torch.int32 and counters.is_contiguous() and counters.numel() >= lib().gi_gemm_bf16_counters()):
+        raise KernelError("gemm: the counters must be int32, as many as gi_gemm_bf16_counters says, contiguous")
+
+
+@lru_cache(maxsize=8192)
 def gemm_bf16_norm_parts(m, n, k) -> int:
     """The pieces per row in which a product [m, k] x [n, k] that adds onto rows writes their sums of squares when it hands
     the next norm on (`gemm_bf16(..., norm_out=...)`); 0 if a product of these sizes cannot."""
@@ -1554,7 +1580,7 @@ def gemm_bf16_takes_norm(m, n, k, gated=False) -> bool:
     return bool(lib().gi_gemm_bf16_takes_norm(m, n, k, 1 if gated else 0))
 
 
-def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=None, norm_out=None, gate_limit=0.0):
+def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=None, norm_out=None, gate_limit=0.0, counters=None):
     """out (=|+=) a @ w.T with bfloat16 operands on the matrix cores, float32 sums.
     gated: w is [gate; up] interleaved in groups of 16 rows and out = act(a @ gate.T) * (a @ up.T), bfloat16 [m, n/2]; act is
     SiLU (gated = True or "silu"), the tanh form of GELU (gated = "gelu_tanh") or the clamped form (gated = "swish_clamped", with
@@ -1563,8 +1589,10 @@ def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=N
     An RMS norm between two products of a few rows, without a kernel of its own:
     norm_out = (g, scaled, squares), with accumulate: beside out += a @ w.T, scaled = bfloat16(g * out) and squares
     [m, gemm_bf16_norm_parts(m, n, k)] = the pieces of the rows' sums of out^2;
-    norm_in = (squares, eps): a is such a `scaled`, and the results are multiplied by rsqrt(sum of the row's pieces / k + eps)."""
-    _dev(a, w, out)
+    norm_in = (squares, eps): a is such a `scaled`, and the results are multiplied by rsqrt(sum of the row's pieces / k + eps).
+    counters: see `step_counters`; the product clears its own where it needs them and has none."""
+    _dev(a, w, out, counters)
+    _check_counters(counters)
     m, k = a.shape
     n = w.shape[0]
     if not (w.shape == (n, k)):
@@ -1595,10 +1623,10 @@ def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=N
             _dev(g, scaled, squares_out)
         _call("gi_gemm_bf16_handing", a.data_ptr(), w.data_ptr(), out.data_ptr(), _code(out, "gemm: out"), 1 if accumulate else 0, gate_code, float(gate_limit),
               m, n, k, a.stride(0), w.stride(0), out.stride(0), _ptr(scratch), n_scratch, _ptr(squares_in), squares_in.shape[1] if squares_in is not None else 0, float(eps),
-              _ptr(g), _ptr(scaled), scaled.stride(0) if scaled is not None else 0, _ptr(squares_out), _stream())
+              _ptr(g), _ptr(scaled), scaled.stride(0) if scaled is not None else 0, _ptr(squares_out), _ptr(counters), _stream())
         return out
     _call("gi_gemm_bf16", a.data_ptr(), w.data_ptr(), out.data_ptr(), _code(out, "gemm: out"), 1 if accumulate else 0, gate_code, float(gate_limit),
-          m, n, k, a.stride(0), w.stride(0), out.stride(0), _ptr(scratch), n_scratch, _stream())
+          m, n, k, a.stride(0), w.stride(0), out.stride(0), _ptr(scratch), n_scratch, _ptr(counters), _stream())
     return out
 
 
@@ -1674,11 +1702,12 @@ def gemm_bf16_qkv_rope_store_max_parts(m, n, k) -> int:
     return lib().gi_gemm_bf16_qkv_rope_store_max_parts(m, n, k)
 
 
-def gemm_bf16_qkv_rope_store(a, w, cos, sin, positions, slots, table, q_out, cache, n_heads, n_kv, hd, norm_in=None):
+def gemm_bf16_qkv_rope_store(a, w, cos, sin, positions, slots, table, q_out, cache, n_heads, n_kv, hd, norm_in=None, counters=None):
     """The q/k/v product a @ w.T of an attention layer whose results do not come back: the queries go, rotated, into q_out
     (bfloat16 [m, heads*hd]), the keys (rotated) and the values into the cache's pages, as `rope_store` puts them.
     cos, sin: float32 [m, hd/2] or None; norm_in as for `gemm_bf16`."""
-    _dev(a, w, cos, sin, positions, slots, table, q_out, cache)
+    _dev(a, w, cos, sin, positions, slots, table, q_out, cache, counters)
+    _check_counters(counters)
     m, k = a.shape
     n = w.shape[0]
     if not (gemm_bf16_supports(a, w, q_out) and w.shape == (n, k) and n == (n_heads + 2 * n_kv) * hd and gemm_bf16_qkv_rope_store_takes(m, n, k, hd)):
@@ -1702,7 +1731,7 @@ def gemm_bf16_qkv_rope_store(a, w, cos, sin, positions, slots, table, q_out, cac
         _profile.note = (f"{n}x{k}", n * k * w.element_size())
     _call("gi_gemm_bf16_qkv_rope_store", a.data_ptr(), w.data_ptr(), m, n, k, a.stride(0), w.stride(0), _ptr(scratch), n_scratch,
           _ptr(squares_in), squares_in.shape[1] if squares_in is not None else 0, float(eps), _ptr(cos), _ptr(sin), positions.data_ptr(),
-          slots.data_ptr(), table.data_ptr(), table.stride(0), q_out.data_ptr(), cache.data_ptr(), cache.stride(0), page_size, n_heads, n_kv, hd, _stream())
+          slots.data_ptr(), table.data_ptr(), table.stride(0), q_out.data_ptr(), cache.data_ptr(), cache.stride(0), page_size, n_heads, n_kv, hd, _ptr(counters), _stream())
     return q_out
 
 

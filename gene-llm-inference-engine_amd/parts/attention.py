@@ -54,13 +54,13 @@ def qkv_rotate_store_attend(h, w_qkv, ctx, cache, *, n_heads, n_kv_heads, head_d
         if ops.gemm_bf16_supports(rows, w_qkv, att):
             q_rot = torch.empty((T, a_dim), dtype=torch.bfloat16, device=ctx.device)
             ops.gemm_bf16_qkv_rope_store(rows, w_qkv, cos, sin, ctx.row_pos, ctx.row_slot, cache.table, q_rot, cache.kv, n_heads, n_kv_heads,
-                                         head_dim, norm_in)
+                                         head_dim, norm_in, ops.step_counters(ctx, T, *w_qkv.shape))
             return ops.attention(q_rot, cache.kv, att, ctx, cache.table, n_heads, n_kv_heads, head_dim, window)
         if norm_in is None:
             h = rows                  # (whole rows: what `linear` below would make of h)
     if cache.writes:
         qkv = torch.empty((T, a_dim + 2 * kv_dim), dtype=torch.float32, device=ctx.device)
-        linear(h, w_qkv, qkv)
+        linear(h, w_qkv, qkv, ctx=ctx)
         q, k, v = qkv[:, :a_dim], qkv[:, a_dim:a_dim + kv_dim], qkv[:, a_dim + kv_dim:]
     else:                       # the pages are another layer's: only the queries are made
         q, k, v = torch.empty((T, a_dim), dtype=torch.float32, device=ctx.device), None, None
@@ -220,7 +220,7 @@ class Attention(Mixer):
         proj = projected
         if proj is None:
             proj = torch.empty((T, self.w_qkv.shape[0]), dtype=torch.float32, device=ctx.device)
-            linear(h, self.w_qkv, proj)
+            linear(h, self.w_qkv, proj, ctx=ctx)
         q, k, v = proj[:, :self.a_dim], None, None
         if s.k_proj is not None and cache.writes:
             k = proj[:, self.a_dim:self.a_dim + self.kv_dim]
@@ -284,14 +284,14 @@ class Attention(Mixer):
             if overwrite:
                 linear(att, self.w_o, residual)
                 return None
-            return linear_onto(att, self.w_o, residual, then)
+            return linear_onto(att, self.w_o, residual, then, ctx)
         if overwrite:
             residual.zero_()
         att = qkv_rotate_store_attend(h, self.w_qkv, ctx, cache, n_heads=s.n_heads, n_kv_heads=s.n_kv_heads, head_dim=s.head_dim,
                                       position=self.position, window=s.window, in_dtype=self.in_dtype)
         if att.dtype != self.att_dtype:
             att = att.to(self.att_dtype)
-        return linear_onto(att, self.w_o, residual, then)
+        return linear_onto(att, self.w_o, residual, then, ctx)
 
 
 register_mixer("attention", Attention)

@@ -122,7 +122,7 @@ class GatedDelta(Mixer):
         proj = projected
         if proj is None:
             proj = torch.empty((T, self.w_in.shape[0]), dtype=torch.float32, device=dev)
-            linear(h, self.w_in, proj)
+            linear(h, self.w_in, proj, ctx=ctx)
         seg_start, seg_len = ops.segments(ctx)
         qkv = torch.empty((T, 2 * G * dk + vv), dtype=torch.float32, device=dev)
         gates = torch.empty((T, self.n_decays + H), dtype=torch.float32, device=dev)
@@ -157,7 +157,7 @@ class GatedDelta(Mixer):
         if overwrite:
             linear(mid, self.w_o, residual)
             return None
-        return linear_onto(mid, self.w_o, residual, then)
+        return linear_onto(mid, self.w_o, residual, then, ctx)
 
 
 register_mixer("gated_delta", GatedDelta)

@@ -162,7 +162,7 @@ class LatentAttention(Mixer):
         if overwrite:
             linear(att, self.w_o, residual)
             return None
-        return linear_onto(att, self.w_o, residual, then)
+        return linear_onto(att, self.w_o, residual, then, ctx)
 
 
 register_mixer("latent_attention", LatentAttention)

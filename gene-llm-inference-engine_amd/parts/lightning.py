@@ -67,7 +67,7 @@ class Lightning(Mixer):
         proj = projected
         if proj is None:
             proj = torch.empty((T, self.w_in.shape[0]), dtype=torch.float32, device=ctx.device)
-            linear(h, self.w_in, proj)
+            linear(h, self.w_in, proj, ctx=ctx)
         seg_start, seg_len = ops.segments(ctx)
         out = torch.empty((T, vv), dtype=torch.float32, device=ctx.device)
         ops.lightning_scan(proj, (self.q_at, self.k_at, self.v_at), self.powers, seg_start, seg_len, ctx.row_slot, cache.state, out, s.n_heads, s.key_dim, s.value_dim,
@@ -77,7 +77,7 @@ class Lightning(Mixer):
         if overwrite:
             linear(mid, self.w_o, residual)
             return None
-        return linear_onto(mid, self.w_o, residual, then)
+        return linear_onto(mid, self.w_o, residual, then, ctx)
 
 
 register_mixer("lightning", Lightning)

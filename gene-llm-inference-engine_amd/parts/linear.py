@@ -17,17 +17,20 @@ from ..kernels import ops
 from .norm import HandedRows, NormedRows, NormToMake, ReadyRows
 
 
-def linear(a, weight: torch.Tensor, out: torch.Tensor, accumulate: bool = False, gated: bool = False, gate_limit: float = 0.0) -> torch.Tensor:
+def linear(a, weight: torch.Tensor, out: torch.Tensor, accumulate: bool = False, gated: bool = False, gate_limit: float = 0.0,
+           ctx=None) -> torch.Tensor:
     """gated: weight is [gate; up] interleaved by `ops.interleave_gate_up` and out = act(gate) * up (bfloat16 only); True or "silu"
-    for SiLU, "gelu_tanh" for the tanh form of GELU, "swish_clamped" (with `gate_limit`) for the clamped form."""
+    for SiLU, "gelu_tanh" for the tanh form of GELU, "swish_clamped" (with `gate_limit`) for the clamped form.  ctx: the step the product is one
+    of, whose counters (`ops.step_counters`) save it a launch where it has a use for them."""
     if isinstance(a, HandedRows):
         if (weight.dtype == torch.bfloat16 and ops.gemm_bf16_supports(a.scaled, weight, out)
                 and ops.gemm_bf16_takes_norm(a.scaled.shape[0], weight.shape[0], weight.shape[1], gated)):
-            return ops.gemm_bf16(a.scaled, weight, out, accumulate, gated, checked=True, norm_in=(a.squares, a.eps), gate_limit=gate_limit)
+            return ops.gemm_bf16(a.scaled, weight, out, accumulate, gated, checked=True, norm_in=(a.squares, a.eps), gate_limit=gate_limit,
+                                 counters=ops.step_counters(ctx, a.scaled.shape[0], *weight.shape))
     if isinstance(a, NormedRows):
         a = a.materialize()
     if a.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and ops.gemm_bf16_supports(a, weight, out):
-        return ops.gemm_bf16(a, weight, out, accumulate, gated, checked=True, gate_limit=gate_limit)
+        return ops.gemm_bf16(a, weight, out, accumulate, gated, checked=True, gate_limit=gate_limit, counters=ops.step_counters(ctx, a.shape[0], *weight.shape))
     if gated:
         raise ops.KernelError("the gated product exists for bfloat16 operands only")
     return ops.gemm_exact(a, weight, out, accumulate)
@@ -54,7 +57,7 @@ def linear_xielu(a, weight: torch.Tensor, params: torch.Tensor, columns: int, dt
     return ops.gemm_bf16_xielu(a, weight, params, mid, out, norm_in)
 
 
-def linear_onto(a: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor, then=None):
+def linear_onto(a: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor, then=None, ctx=None):
     """residual += a @ weight.T.  `then`: the norm that reads `residual` next, if it and its reader can take it half applied
     (see `HandedRows`); the product then also does the norm's share and the `HandedRows` are returned, None otherwise.  Or that norm as a
     `NormToMake`, for a reader that takes no other than a whole one: the rows come back normed where the product's kernel can."""
@@ -72,9 +75,10 @@ def linear_onto(a: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor, t
         if parts:
             scaled = torch.empty((rows, width), dtype=torch.bfloat16, device=residual.device)
             squares = torch.empty((rows, parts), dtype=torch.float32, device=residual.device)
-            ops.gemm_bf16(a, weight, residual, accumulate=True, checked=True, norm_out=(then.handed_weight(), scaled, squares))
+            ops.gemm_bf16(a, weight, residual, accumulate=True, checked=True, norm_out=(then.handed_weight(), scaled, squares),
+                          counters=ops.step_counters(ctx, rows, *weight.shape))
             return HandedRows(then, residual, scaled, squares)
-    linear(a, weight, residual, accumulate=True)
+    linear(a, weight, residual, accumulate=True, ctx=ctx)
     return None
 
 

@@ -45,7 +45,7 @@ class SwiGlu(FeedForward):
         T, inter = ctx.n_rows, self.spec.intermediate_size
         if self.fused:
             mid = torch.empty((T, inter), dtype=torch.bfloat16, device=ctx.device)
-            linear(h, self.w_gate_up, mid, gated=self.activation, gate_limit=self.limit)
+            linear(h, self.w_gate_up, mid, gated=self.activation, gate_limit=self.limit, ctx=ctx)
         else:
             gate_up = torch.empty((T, 2 * inter), dtype=torch.float32, device=ctx.device)
             linear(h, self.w_gate_up, gate_up)
@@ -54,7 +54,7 @@ class SwiGlu(FeedForward):
         if overwrite:
             linear(mid, self.w_down, residual)
             return None
-        return linear_onto(mid, self.w_down, residual, then)
+        return linear_onto(mid, self.w_down, residual, then, ctx)
 
 
 register_feed_forward("swiglu", SwiGlu)
@@ -114,7 +114,7 @@ class DenseMlp(FeedForward):
         if overwrite:
             linear(mid, self.w_down, residual)
             return None
-        return linear_onto(mid, self.w_down, residual, then)
+        return linear_onto(mid, self.w_down, residual, then, ctx)
 
 
 register_feed_forward("dense_mlp", DenseMlp)

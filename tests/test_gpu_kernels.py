@@ -173,6 +173,47 @@ def test_products_of_prompts_in_each_kernel(kernel, kind, m, n, k):
         assert rel(out[:, :n], right) < 4e-3 and bool((out[:, n:] == 7).all())
 
 
+@pytest.mark.parametrize("kind,m,n,k,shares", [
+    # no whole round: two shares of equal and of unequal parts of k, ragged tiles; one whole round and a few tiles in four, three and two shares
+    ("added", 2048, 2048, 8192, 2), ("added", 1777, 2050, 8256, 2), ("handing", 2048, 2048, 8192, 2), ("stored", 1777, 2050, 8256, 2), ("bfloat16", 1777, 2050, 8256, 2),
+    ("rotated", 2048, 5120, 3072, 4), ("added", 2047, 5130, 3072, 3), ("gated", 2600, 4064, 4160, 2)])
+def test_products_whose_last_tiles_share_k_out(kind, m, n, k, shares):
+    """The tiles of 256 x 128 of an incomplete round, each made by several workgroups: against 64 bits, and every time the same bits, whoever came last; counters that are
+    given come back as they were."""
+    o = ops()
+    asked = {"handing": "added handing a norm on", "bfloat16": "stored"}.get(kind, kind)
+    assert o.gemm_bf16_large_kernel(m, n, k, asked) == "256x128" and o.lib().gi_gemm_bf16_tall_shares(m, n, k) == shares
+    a, w = randn(m, k, dtype=torch.bfloat16, seed=11), randn(n, k, dtype=torch.bfloat16, seed=12, scale=1.5 / k ** 0.5)
+    want = a.double() @ w.double().T
+    seen, counters = [], torch.zeros(o.lib().gi_gemm_bf16_counters(), dtype=torch.int32, device=DEV)
+    for given in (None, counters, counters, None):
+        if kind == "rotated":
+            heads, hd, page = n // 128 - 16, 128, 16
+            q, cache = torch.zeros(m, heads * hd, dtype=torch.bfloat16, device=DEV), torch.zeros(m // page, 2, 8, page, hd, dtype=torch.bfloat16, device=DEV)
+            positions, slots = torch.arange(m, dtype=torch.int32, device=DEV), torch.zeros(m, dtype=torch.int32, device=DEV)
+            o.gemm_bf16_qkv_rope_store(a, w, None, None, positions, slots, torch.arange(m // page, dtype=torch.int32, device=DEV).view(1, -1), q, cache, heads, 8, hd,
+                                       counters=given)
+            keys, values = cache[:, 0].permute(0, 2, 1, 3).reshape(m, -1), cache[:, 1].reshape(-1, 8, hd, page).permute(0, 3, 1, 2).reshape(m, -1)
+            got, right, tol = torch.cat([q, keys, values], dim=1), want, 4e-3
+        elif kind == "gated":
+            got = torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV)
+            o.gemm_bf16(a, w, got, gated=True, counters=given)
+            v = want.view(m, n // 32, 2, 16)
+            right, tol = torch.nn.functional.silu(v[:, :, 0].reshape(m, -1)) * v[:, :, 1].reshape(m, -1), 4e-3
+        else:
+            got = torch.full((m, n), 0.5, dtype=torch.bfloat16 if kind == "bfloat16" else torch.float32, device=DEV)
+            norm_out = None
+            if kind == "handing":
+                norm_out = (torch.ones(n, device=DEV), torch.empty(m, n, dtype=torch.bfloat16, device=DEV), torch.empty(m, o.gemm_bf16_norm_parts(m, n, k), device=DEV))
+            o.gemm_bf16(a, w, got, accumulate=kind in ("added", "handing"), norm_out=norm_out, counters=given)
+            right, tol = want + (0.5 if kind in ("added", "handing") else 0.0), 4e-3 if kind == "bfloat16" else 1e-5
+            if kind == "handing":
+                assert torch.equal(norm_out[1], got.to(torch.bfloat16))
+        assert rel(got, right) < tol
+        seen.append(got)
+    assert all(torch.equal(seen[0], s) for s in seen[1:]) and not bool(counters.any())
+
+
 @pytest.mark.parametrize("m,inter,k", [(1, 16, 8), (5, 48, 136), (16, 160, 96), (17, 176, 64), (64, 32, 264), (70, 192, 128), (300, 8192 // 16, 2048 // 8),
                                        (72, 8192, 2048), (128, 6144, 264), (100, 288, 136),
                                        (40, 6144, 264), (13, 6160, 72), (64, 8192, 512), (2048, 1024, 192), (600, 288, 64), (200, 512, 1024),
