@@ -414,13 +414,28 @@ __global__ __launch_bounds__(128 * NW * PAIR) void attention_prompt_kernel(const
 // The rows of a key tile are taken in another order by the score product: row i of the matrix instruction reads key
 // pi(i) = 16 (i / 16) + 8 ((i / 4) % 2) + 4 ((i / 8) % 2) + i % 4 of its 32, so that the 8 scores a lane holds for the
 // next product's k index are 8 consecutive keys, and the value operand is one 16-byte read (8 positions of a channel).
+//
+// A walk that is much longer than the others' share of the chip is cut into shares of keys, up to WideShares::most of them by its own length, whose workgroups meet
+// in the kernel: the one that comes last merges the others' {m, l, O} with its own, in the order of the keys whoever it is, and writes the rows; the
+// others leave theirs in the order of their registers and end.  Who has come is counted, and the sums go past the L2s of the dies, as in the products'
+// kernel for the last tiles of a round (`TileShares` in gemm_bf16.hip): the last waits only for workgroups that have nothing left to wait for.
+// 24 heads of 128 over a portion of 1,350 rows behind 1,000 positions and one of 674 (264 workgroups that walk up to 37 tiles of keys beside 144 short ones).
+struct WideShares {
+    int most, keys;                            // shares at most (1: none), and keys a share should have
+    unsigned* counters;                        // [tile][head][2], 0 at the start and at the end
+    unsigned char* sums;                       // [tile][head][share][wave][(16 or 32 channels' worth of) registers / 4 + 1][64 lanes][16 bytes]
+};
+constexpr int WIDE_MAX_SHARES = 4;
+typedef unsigned gi_uint4 __attribute__((ext_vector_type(4)));
+constexpr int DEVICE_SCOPE = 16;               // sc1 in a buffer access's cache policy
+template <int HD> constexpr int wide_share_bytes(int nw) { return nw * (HD / 32 * 4 + 1) * 1024; }
 template <int HD, int NW, bool CAP>
 __global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache,
                                                                        bf16_t* __restrict__ out, const int4* __restrict__ tiles,
                                                                        const int* __restrict__ table, int table_stride, long page_stride,
                                                                        int page_size, int n_heads, int n_kv, int window, float scale,
                                                                        int n_splits, const int* __restrict__ tile_first, float* __restrict__ part,
-                                                                       int list_order, Extras extra) {
+                                                                       int list_order, Extras extra, WideShares shares) {
     static_assert(HD == 128 || HD == 64, "the chunk swizzle is made for key rows of 256 or 128 bytes");
     constexpr int QSTEPS = HD / 16, DT = HD / 32;
     constexpr int K_BYTES = KV_TILE * HD * 2, V_BYTES = HD * KV_TILE * 2, STAGE = K_BYTES + V_BYTES;
@@ -434,12 +449,18 @@ __global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_w
     // short ones fill the end.  A plain list runs from early tiles to late ones and is taken backwards; a list of pairs names a
     // late tile, an early one, the next later one, the next earlier one, ...: first its late tiles in their order, then its early
     // ones backwards.
-    const int n_groups = gridDim.y / n_splits, turn = blockIdx.y / n_splits, split = blockIdx.y % n_splits;
+    const int places = shares.most > 1 ? shares.most : n_splits;
+    const int n_groups = gridDim.y / places, turn = blockIdx.y / places, split = blockIdx.y % places;
     const int group = !list_order ? n_groups - 1 - turn : turn < n_groups / 2 ? 2 * turn : 2 * (n_groups - 1 - turn) + 1;
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int4 tile = tiles[group];
     const int row0 = tile.x, n_rows = tile.y, pos0 = tile.z, slot = tile.w;
     if (n_rows == 0) return;                                  // (a tile that only fills a pair)
+    if (shares.most > 1) {
+        const int walk = pos0 + n_rows - (lowest_seen(pos0, window, extra.chunk) & ~(KV_TILE - 1));
+        n_splits = min(shares.most, (walk + shares.keys - 1) / shares.keys);
+        if (split >= n_splits) return;
+    }
     const int head = blockIdx.x, g = head / (n_heads / n_kv);
     const int col = lane & 31, hf = lane >> 5;
     const int* tab = table + (size_t)slot * table_stride;
@@ -616,9 +637,80 @@ __global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_w
         landed_barrier();
     }
     l += __shfl_xor(l, 32, 64);
-    if (!row_ok) return;
-    if (extra.sinks != nullptr && split == 0) add_sink(extra.sinks[head], m, l);
-    if (n_splits > 1) {                                       // part[row of the split tiles][head][split] = {m, l, O[HD]}
+    if (shares.most > 1 && n_splits > 1) {
+        if (extra.sinks != nullptr && split == 0) add_sink(extra.sinks[head], m, l);
+        constexpr int PIECES = DT * 4 + 1;                    // 16 bytes a lane each; the last holds m and l
+        unsigned& drawn = *reinterpret_cast<unsigned*>(lds);   // (everybody is past the last tile)
+        const size_t walk = (size_t)group * n_heads + head;
+        unsigned* const counter = shares.counters + 2 * walk;
+        const int at = (wv * PIECES * 64 + lane) * 16;
+        auto place = [&](int of) {
+            return __builtin_amdgcn_make_buffer_rsrc(shares.sums + (walk * shares.most + of) * wide_share_bytes<HD>(NW), 0, wide_share_bytes<HD>(NW), 0x00027000);
+        };
+        if (tid == 0) drawn = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if ((int)drawn + 1 < n_splits) {
+            const auto mine = place(split);
+#pragma unroll
+            for (int f = 0; f < DT * 4; ++f) {
+                const int v = (f & 3) * 4;
+                __builtin_amdgcn_raw_buffer_store_b128(gi_uint4{__float_as_uint(o[f >> 2][v]), __float_as_uint(o[f >> 2][v + 1]), __float_as_uint(o[f >> 2][v + 2]),
+                                                                __float_as_uint(o[f >> 2][v + 3])}, mine, at, f * 1024, DEVICE_SCOPE);
+            }
+            __builtin_amdgcn_raw_buffer_store_b128(gi_uint4{__float_as_uint(m), __float_as_uint(l), 0u, 0u}, mine, at, DT * 4 * 1024, DEVICE_SCOPE);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's sums are in memory
+            __syncthreads();
+            if (tid == 0) __hip_atomic_fetch_add(counter + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return;
+        }
+        if (tid == 0)
+            while ((int)__hip_atomic_load(counter + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 < n_splits) __builtin_amdgcn_s_sleep(1);
+        __syncthreads();
+        if (tid < 2) __hip_atomic_store(counter + tid, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        float weight[WIDE_MAX_SHARES], share_l[WIDE_MAX_SHARES], big = -INFINITY;
+#pragma unroll
+        for (int of = 0; of < WIDE_MAX_SHARES; ++of) {
+            weight[of] = of == split ? m : -INFINITY;
+            share_l[of] = of == split ? l : 0.f;
+            if (of < n_splits && of != split) {
+                const gi_uint4 v = __builtin_amdgcn_raw_buffer_load_b128(place(of), at, DT * 4 * 1024, DEVICE_SCOPE);
+                weight[of] = __uint_as_float(v[0]);
+                share_l[of] = __uint_as_float(v[1]);
+            }
+        }
+#pragma unroll
+        for (int of = 0; of < WIDE_MAX_SHARES; ++of) big = fmaxf(big, weight[of]);
+        l = 0.f;
+#pragma unroll
+        for (int of = 0; of < WIDE_MAX_SHARES; ++of) {
+            weight[of] = weight[of] == -INFINITY ? 0.f : exp2_fast(weight[of] - big);
+            if (of < n_splits) l = fmaf(weight[of], share_l[of], l);
+        }
+#pragma unroll
+        for (int i = 0; i < DT; ++i) {
+            floatx16 total = floatx16{};
+#pragma unroll
+            for (int of = 0; of < WIDE_MAX_SHARES; ++of) {
+                if (of == split) {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) total[v] = fmaf(weight[of], o[i][v], total[v]);
+                } else if (of < n_splits) {
+                    const auto theirs = place(of);
+                    gi_uint4 sums[4];
+#pragma unroll
+                    for (int f = 0; f < 4; ++f) sums[f] = __builtin_amdgcn_raw_buffer_load_b128(theirs, at, (i * 4 + f) * 1024, DEVICE_SCOPE);
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) total[v] = fmaf(weight[of], __uint_as_float(sums[v >> 2][v & 3]), total[v]);
+                }
+            }
+            o[i] = total;
+        }
+        if (!row_ok) return;
+    } else {
+        if (!row_ok) return;
+        if (extra.sinks != nullptr && split == 0) add_sink(extra.sinks[head], m, l);
+    }
+    if (shares.most <= 1 && n_splits > 1) {                   // part[row of the split tiles][head][split] = {m, l, O[HD]}
         float* dst = part + (((size_t)(tile_first[group] + my_row) * n_heads + head) * n_splits + split) * (HD + 2);
         if (hf == 0) {
             dst[0] = m;
@@ -1083,6 +1175,18 @@ GI_API int gi_attention_bf16_supports(int hd, int page_size, int prompt) {
     return hd == 32 || hd == 64 || hd == 96 || hd == 128 || hd == 256;
 }
 
+static bool takes_wide(int n_tiles, int n_heads, int hd, int n_splits, int paired) {
+    const bool one_round = (long)(paired ? n_tiles / 2 : n_tiles) * n_heads <= gi_compute_units();
+    return hd == 128 || (hd == 64 && n_splits == 1 && !one_round);
+}
+// Floats of scratch for gi_attention_prompt_bf16 with `most_shares` shares; 0 where the kernel that takes these sizes shares no keys out.  The counters it
+// wants are 2 * n_tiles * n_heads of 32 bits, all 0, and are left so.
+GI_API long gi_attention_prompt_share_floats(int n_tiles, int rows_per_tile, int n_heads, int hd, int n_splits, int paired, int most_shares) {
+    if (n_splits != 1 || most_shares < 2 || most_shares > WIDE_MAX_SHARES || (long)n_tiles * most_shares > 65535 || !takes_wide(n_tiles, n_heads, hd, n_splits, paired)) return 0;
+    const int waves = hd == 64 && rows_per_tile == 64 ? 2 : 4;
+    return (long)n_tiles * n_heads * most_shares * (hd == 128 ? wide_share_bytes<128>(waves) : wide_share_bytes<64>(waves)) / 4;
+}
+
 // tiles hold at most `rows_per_tile` rows each (64 or 128).  `paired` != 0: tiles 2w and 2w + 1 belong to one request
 // and share workgroup w (a late tile of a prompt beside an early one; a tile of 0 rows fills a pair).  n_splits > 1:
 // the keys of a workgroup's tiles are shared out over that many workgroups; `tile_first[i]` is the number of rows in
@@ -1092,7 +1196,7 @@ GI_API int gi_attention_prompt_bf16(const void* q, const void* cache, void* out,
                                     const int* table, int table_stride, long page_stride, int page_size, int n_heads, int n_kv, int hd,
                                     int window, float scale, int n_splits, const int* tile_first, const int* rows, int n_rows, float* part,
                                     long part_floats, int chunk, const float* sinks, const float* gate, long gate_stride, int gate_channels, float cap,
-                                    hipStream_t stream) {
+                                    int share_keys, int most_shares, unsigned* counters, hipStream_t stream) {
     GI_REQUIRE(chunk >= 0 && cap >= 0.f && (gate_channels == 0 || gate_channels == hd) && (gate == nullptr || gate_stride >= (long)n_heads * (gate_channels ? hd : 1)) &&
                    (gate == nullptr || gate_channels == 0 || (gate_stride % 4 == 0 && ((uintptr_t)gate & 15) == 0)),
                "attention_prompt: bad chunk, cap or gate stride, or a channels' gate whose rows do not start at multiples of 16 bytes");
@@ -1113,20 +1217,26 @@ GI_API int gi_attention_prompt_bf16(const void* q, const void* cache, void* out,
     // first kernel's pairs of tiles are the better balance while they fit the chip in one round (a workgroup of 16 waves a compute
     // unit: 2,048 rows of 32 heads take 56 against 61 us) and where few tiles share their keys out; beyond one round its time
     // doubles at once and the wide kernel's many small workgroups win (2,560 rows: 68 against 100 us; 8,192: 360 against 572).
-    const bool one_round = (long)(paired ? n_tiles / 2 : n_tiles) * n_heads <= gi_compute_units();
-    if (hd == 128 || (hd == 64 && n_splits == 1 && !one_round)) {
-        GI_REQUIRE((long)n_tiles * n_splits <= 65535, "attention_prompt: %d tiles in %d splits are too many for one launch", n_tiles, n_splits);
-        dim3 wgrid(n_heads, n_tiles * n_splits);
+    if (takes_wide(n_tiles, n_heads, hd, n_splits, paired)) {
+        GI_REQUIRE((long)n_tiles * n_splits * (most_shares > 1 ? most_shares : 1) <= 65535, "attention_prompt: %d tiles in %d splits are too many for one launch", n_tiles, n_splits);
+        WideShares shares = {1, 0, nullptr, nullptr};
+        if (most_shares > 1) {
+            GI_REQUIRE(gi_attention_prompt_share_floats(n_tiles, rows_per_tile, n_heads, hd, n_splits, paired, most_shares) > 0 && share_keys > 0 && counters != nullptr && part != nullptr &&
+                           ((uintptr_t)part & 15) == 0 && part_floats >= gi_attention_prompt_share_floats(n_tiles, rows_per_tile, n_heads, hd, n_splits, paired, most_shares),
+                       "attention_prompt: %d shares of %d keys need counters and scratch that were not given, or sizes that are not shared out", most_shares, share_keys);
+            shares = {most_shares, share_keys, counters, (unsigned char*)part};
+        }
+        dim3 wgrid(n_heads, n_tiles * n_splits * shares.most);
 #define WIDE(HD, NW)                                                                                                                    \
     do {                                                                                                                                \
         if (extra.cap > 0.f)                                                                                                            \
             attention_prompt_wide_kernel<HD, NW, true><<<wgrid, 64 * NW, 0, stream>>>((const bf16_t*)q, (const bf16_t*)cache, (bf16_t*)out, (const int4*)tiles, table, \
                                                                                      table_stride, page_stride, page_size, n_heads, n_kv, window, scale, n_splits, \
-                                                                                     tile_first, part, paired ? 1 : 0, extra);            \
+                                                                                     tile_first, part, paired ? 1 : 0, extra, shares);            \
         else                                                                                                                            \
             attention_prompt_wide_kernel<HD, NW, false><<<wgrid, 64 * NW, 0, stream>>>((const bf16_t*)q, (const bf16_t*)cache, (bf16_t*)out, (const int4*)tiles, table, \
                                                                                       table_stride, page_stride, page_size, n_heads, n_kv, window, scale, n_splits, \
-                                                                                      tile_first, part, paired ? 1 : 0, extra);           \
+                                                                                      tile_first, part, paired ? 1 : 0, extra, shares);           \
     } while (0)
         if (hd == 64) { if (rows_per_tile == 64) WIDE(64, 2); else WIDE(64, 4); }
         else WIDE(128, 4);      // (tiles of 64 rows too: two of its waves then only load; a workgroup of two waves would need 16 loads a wave and more registers than two to a SIMD leave)
@@ -1139,6 +1249,7 @@ GI_API int gi_attention_prompt_bf16(const void* q, const void* cache, void* out,
         }
         return 0;
     }
+    GI_REQUIRE(most_shares <= 1, "attention_prompt: this kernel's workgroups do not meet");
     const bool pairs = paired && hd <= 64;
     dim3 grid((pairs ? n_tiles / 2 : n_tiles) * n_splits, n_heads);
 #define GO_(HD, NW, PAIR)                                                                                                               \

@@ -525,7 +525,7 @@ class _StepGraph:
             flat[offset:offset + size] = a
         self.block[:total].copy_(staged, non_blocking=True)
         if plan.n_tiles:
-            plan.max_tile_context = self.bracket
+            plan.max_tile_context, plan.tile_contexts = self.bracket, None
         if plan.n_decode:
             plan.max_decode_context, plan.decode_positions = self.bracket, None
         m = self.model

@@ -101,7 +101,7 @@ _SIGNATURES = {
     "gi_head_norm_gate": [c_void_p, c_long, c_void_p, c_void_p, c_long, c_void_p, c_int, c_void_p, c_int, c_long, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p],
     "gi_gemm_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long, c_void_p, c_void_p],
     "gi_attention_prompt_bf16": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int,
-                                 c_float, c_int, c_void_p, c_void_p, c_int, c_void_p, c_long, c_int, c_void_p, c_void_p, c_long, c_int, c_float, c_void_p],
+                                 c_float, c_int, c_void_p, c_void_p, c_int, c_void_p, c_long, c_int, c_void_p, c_void_p, c_long, c_int, c_float, c_int, c_int, c_void_p, c_void_p],
     "gi_attention_decode_bf16": [c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_long, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                  c_long, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int,
                                  c_float, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_long, c_int, c_float, c_void_p],
@@ -150,6 +150,8 @@ def lib():
         l.gi_gemm_bf16_scratch_floats.restype = c_long
         l.gi_gemm_bf16_norm_parts.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_bf16_norm_parts.restype = c_int
+        l.gi_attention_prompt_share_floats.argtypes = [c_int, c_int, c_int, c_int, c_int, c_int, c_int]
+        l.gi_attention_prompt_share_floats.restype = c_long
         l.gi_gemm_bf16_tall_shares.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_bf16_tall_shares.restype = c_int
         l.gi_gemm_bf16_counters.argtypes = []
@@ -1175,7 +1177,7 @@ class AttentionPlan:
         plan = cls.__new__(cls)
         plan.n_decode, plan.n_tiles, plan.max_decode_context, plan.single_rows = n_rows, 0, max_context, True
         plan.decode_rows = None                                  # rows 0 .. n_rows-1
-        plan.decode_positions = None
+        plan.decode_positions = plan.tile_contexts = None
         plan.tiles = torch.empty(0, dtype=torch.int32, device=device)
         plan.n_tile_rows, plan.max_tile_context, plan.tile_first, plan.tile_rows, plan.paired, plan.tile = 0, 0, None, None, False, 128
         return plan
@@ -1207,7 +1209,8 @@ class AttentionPlan:
                 tiles.extend((late, early if early is not late else (late[0], 0, late[2], late[3])))
         self.n_decode, self.n_tiles = len(dec), len(tiles)
         self.n_tile_rows = sum(t[1] for t in tiles)
-        self.max_tile_context = max((t[2] + t[1] for t in tiles), default=0)
+        self.tile_contexts = [t[2] + t[1] for t in tiles if t[1]]        # positions each tile of rows sees; None: of a step still to come
+        self.max_tile_context = max(self.tile_contexts, default=0)
         # for sharing a tile's keys out over workgroups: rows before each tile, and the tiles' rows in order
         firsts, count = [], 0
         for t in tiles:
@@ -1237,6 +1240,26 @@ def prompt_attention_splits(n_groups, n_heads, span, target_groups=512):
     if groups >= target_groups // 2:
         return 1
     return max(1, min(-(-target_groups // groups), span // 256, 64))
+
+
+PROMPT_SHARE_COUNTERS = 4096
+
+
+def prompt_attention_shares(contexts, n_heads, hd):
+    """(shares, keys) for the tiles of a step that fill the chip: a tile's keys are shared out over up to so many workgroups of so many keys each, (1, 0) where
+    none should be.  The chip holds two workgroups a compute unit (three at heads of 64 channels); a tile that sees far more keys than there are for each of
+    those places keeps one busy when the others have ended.  Measured, one workgroup a tile and shared: 24 heads of 128 over 1,350 rows behind 1,000 and 674 more
+    87.6 -> 71 us (77 in two shares, 79 in four), 2,000 rows 74.6 -> 52 (57 in three), 32 heads over 1,000 rows 40 -> 31, over 1,500 58 -> 41, but over 2,048
+    62.5 -> 71.6 and over 800 the same; 32 heads of 64 over 2,560 rows 52.4 -> 49.8, over 3,500 99.5 -> 82, over 900 behind 1,000 and 1,100 more 52 -> 40 (44 in
+    three).  The lines: the longest walk 2.1 (64 channels: 1.5) times a place's even share and 16 tiles of 64 keys, and every share from the third on
+    leaves each 12 (16) of them."""
+    walks = [-(-c // 64) for c in contexts]
+    wide = hd == 128
+    longest, even = max(walks), sum(walks) * n_heads / (lib().gi_compute_units() * (2 if wide else 3))
+    if longest < 16 or longest < (2.1 if wide else 1.5) * even:
+        return (1, 0)
+    most = max(2, min(4, longest // (12 if wide else 16)))
+    return (most, 64 * -(-longest // most))
 
 
 def _decode_piece(span, n_pieces):
@@ -1420,10 +1443,20 @@ def attention_bf16(q, cache, out, plan: AttentionPlan, positions, slots, table, 
         n_splits = prompt_attention_splits(plan.n_tiles // 2 if plan.paired else plan.n_tiles, n_heads, seen(plan.max_tile_context, plan.tile),
                                            target_groups=PAIRED_TARGET_GROUPS if plan.paired else 512)      # a pair's workgroup has twice the waves
         n_part = plan.n_tile_rows * n_heads * n_splits * (hd + 2) if n_splits > 1 else 0
+        most, keys, counters = 1, 0, None
+        if n_splits == 1 and memo is not None and plan.tile_contexts is not None and plan.n_tiles * n_heads <= PROMPT_SHARE_COUNTERS // 2:
+            most, keys = prompt_attention_shares([min(c, seen(c, plan.tile)) for c in plan.tile_contexts], n_heads, hd)
+            n_part = lib().gi_attention_prompt_share_floats(plan.n_tiles, plan.tile, n_heads, hd, 1, 1 if plan.paired else 0, most)
+            if n_part:
+                counters = memo.get("attention_counters")
+                if counters is None:
+                    counters = memo["attention_counters"] = torch.zeros(PROMPT_SHARE_COUNTERS, dtype=torch.int32, device=out.device)
+            else:
+                most, keys = 1, 0
         part = torch.empty(n_part, dtype=torch.float32, device=out.device) if n_part else None
         _call("gi_attention_prompt_bf16", q.data_ptr(), cache.data_ptr(), out.data_ptr(), plan.tiles.data_ptr(), plan.n_tiles, plan.tile,
               1 if plan.paired else 0, table.data_ptr(), table.stride(0), cache.stride(0), page_size, n_heads, n_kv, hd, window, scale, n_splits,
-              _ptr(plan.tile_first), _ptr(plan.tile_rows), plan.n_tile_rows, _ptr(part), n_part, *extras, _stream())
+              _ptr(plan.tile_first), _ptr(plan.tile_rows), plan.n_tile_rows, _ptr(part), n_part, *extras, keys, most, _ptr(counters), _stream())
     if plan.n_decode:
         span = seen(plan.max_decode_context, 31)
         n_splits, n_waves = decode_attention_shape(plan.n_decode, n_heads, n_kv, hd, span, target_waves, products is not None)

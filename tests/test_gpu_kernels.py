@@ -844,6 +844,35 @@ def test_many_prompt_tiles_of_many_heads(window):
     assert rel(out, want) < 8e-3, rel(out, want)
 
 
+@pytest.mark.parametrize("n_heads,n_kv,hd,segs,window,known", [
+    (24, 8, 128, [(0, 1020, 1350), (1, 0, 674), (2, 49, 1)], None, "3"), (32, 8, 128, [(0, 0, 1000)], None, "2"), (16, 8, 128, [(0, 4000, 260), (1, 0, 1900)], None, "4"), (24, 8, 128, [(0, 1020, 1350), (1, 0, 674)], None, "sinks"),
+    (24, 8, 128, [(0, 1020, 1350), (1, 0, 674)], None, "cap"), (64, 16, 64, [(0, 3000, 900), (1, 0, 401)], None, "3"), (64, 16, 64, [(0, 3000, 130), (1, 0, 960)], 2000, "2")])
+def test_long_walks_of_prompt_tiles_share_their_keys_out(n_heads, n_kv, hd, segs, window, known):
+    """Portions far behind others whose tiles fill the chip all the same: the tiles with long walks are made by several workgroups that meet in the kernel.
+    Against 64 bits where that is stated plainly, against one workgroup a tile, and in bits against themselves, whoever came last."""
+    o = ops()
+    contexts = [pos0 + n for _, pos0, n in segs]
+    cache, table, dense = build_paged(contexts, n_kv, hd, 16, torch.bfloat16, seed=5, scale_one=(77, 3.0))
+    rows = [(slot, pos0 + i) for slot, pos0, n in segs for i in range(n)]
+    starts = [sum(n for _, _, n in segs[:i]) for i in range(len(segs))]
+    plan = o.AttentionPlan(starts, [n for _, _, n in segs], [p for _, p, _ in segs], [s_ + 1 for s_, _, _ in segs], DEV)
+    most, keys = o.prompt_attention_shares([min(c, (window or c) + plan.tile) for c in plan.tile_contexts], n_heads, hd)
+    assert plan.n_tiles and most > 1 and (known not in "234" or most == int(known)), (most, keys)
+    q = randn(len(rows), n_heads * hd, dtype=torch.bfloat16, seed=3)
+    pos = torch.tensor([p for _, p in rows], dtype=torch.int32, device=DEV)
+    slots = torch.tensor([s_ + 1 for s_, _ in rows], dtype=torch.int32, device=DEV)
+    extras = dict(sinks=randn(n_heads, seed=9)) if known == "sinks" else dict(cap=20.0) if known == "cap" else {}
+    seen, memo = [], {}
+    for m in (memo, memo, {}, None):
+        seen.append(torch.full((len(rows), n_heads * hd), float("nan"), dtype=torch.bfloat16, device=DEV))
+        o.attention_bf16(q, cache, seen[-1], plan, pos, slots, table, n_heads, n_kv, hd, window, memo=m, **extras)
+    assert torch.equal(seen[0], seen[1]) and torch.equal(seen[0], seen[2]) and not bool(memo["attention_counters"].any())
+    # (the probabilities are rounded to bfloat16 about another maximum, 2^-9 of each at most on either side, and the results, 2^-8 between the two)
+    assert rel(seen[0], seen[3]) < 2 * 2.0 ** -9 + 2.0 ** -8, rel(seen[0], seen[3])
+    if not extras:
+        assert rel(seen[0], plain_attention_rows(q, dense, rows, n_heads, n_kv, hd, window)) < 8e-3
+
+
 @pytest.mark.parametrize("n_heads,n_kv,hd", [(4, 2, 64), (4, 2, 128), (64, 16, 64)])
 def test_prompt_attention_with_scores_that_climb_along_the_context(n_heads, n_kv, hd):
     """Every query points along one direction and the keys' share of that direction climbs with their position, by 2 to 12
