@@ -299,16 +299,23 @@ __global__ __launch_bounds__(256) void gemm_exact_add_parts_kernel(const float* 
 // (5.8); one lane per column, each walking all of k alone, took 290 us, 1.15 ms and 400 us.
 constexpr int FEW_ROWS = 16, AHEAD = 8;
 
-template <int STRIP, typename TA, typename TW, typename TC, bool ACCUMULATE>
+// GATED: W is [gate; up], a strip of 16 is 8 gates and the 8 ups of the same columns, and act(gate) * up goes out in the bits of the gate's own kernel, which
+// read both again (3 rows of 16,384 x 2,048: 27.4 us and 5 for the gate, 28 in one).  The norm of the rows was tried here too (every workgroup working the rows'
+// factors out for itself while its first weights are on their way, in the bits of the norm's kernel): 1,024 workgroups that each read all rows once more took 39 us
+// for 27.4 and the norm's 5, 3,072 x 2,048 13 for 8.6 and 5.  Not kept.
+struct Gate { int act; float limit; };
+
+template <int STRIP, typename TA, typename TW, typename TC, bool ACCUMULATE, bool GATED>
 __global__ __launch_bounds__(STRIP == 16 ? 512 : 256) void gemm_exact_few_rows_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C,
-                                                                                      int M, int N, int K, long lda, long ldw, long ldc) {
+                                                                                      int M, int N, int K, long lda, long ldw, long ldc, Gate gate) {
+    static_assert(!GATED || STRIP == 16, "a strip of gates and ups");
     __shared__ f32x4 sums[RANGES][STRIP == 16 ? 64 : 16];                 // per range: [group of 4 columns][row]
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
-    const int n0 = blockIdx.x * STRIP, L = range_length(K);
+    const int n0 = blockIdx.x * (GATED ? 8 : STRIP), L = range_length(K), inter = N / 2;
     const int q = STRIP == 16 ? wave : 2 * wave + (r >> 3), row = STRIP == 16 ? r : r & 7;
     const int q_last = STRIP == 16 ? wave : 2 * wave + 1, q_first = STRIP == 16 ? wave : 2 * wave;       // of the wave
     const int base = q * L + 4 * g;
-    const TW* w_row = W + (size_t)min(n0 + row, N - 1) * ldw;
+    const TW* w_row = W + (size_t)(GATED ? min(n0 + (row & 7), inter - 1) + (row >> 3) * inter : min(n0 + row, N - 1)) * ldw;
     const TA* a_row = A + (size_t)min(row, M - 1) * lda;
     const int blocks = max(0, min(L, K - q_first * L) + 15) / 16;             // until both of the wave's ranges are through
     const int whole = max(0, min(L, K - q_last * L)) / 16 / AHEAD * AHEAD;    // ... of them with nothing to guard, in groups
@@ -338,14 +345,24 @@ __global__ __launch_bounds__(STRIP == 16 ? 512 : 256) void gemm_exact_few_rows_k
     const int e = threadIdx.x;
     if (e >= STRIP * STRIP / 4) return;
     const int m = e % STRIP, n = n0 + 4 * (e / STRIP);
-    if (m >= M) return;
+    if (!GATED && m >= M) return;
     f32x4 v[RANGES];
 #pragma unroll
     for (int z = 0; z < RANGES; ++z) v[z] = sums[z][e];
     const f32x4 sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    if constexpr (GATED) {                                      // lanes 0 .. 31 hold gates, the lane 32 further the ups of the same columns and row
+        f32x4 up;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (n + i < N) put<TC, ACCUMULATE>(C, (size_t)m * ldc + n + i, sum[i]);
+        for (int i = 0; i < 4; ++i) up[i] = __shfl_xor(sum[i], 32, 64);
+        if (e >= 32 || m >= M) return;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (n + i < inter) store_f32(C, (size_t)m * ldc + n + i, gated_act(sum[i], up[i], gate.act, gate.limit));
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (n + i < N) put<TC, ACCUMULATE>(C, (size_t)m * ldc + n + i, sum[i]);
+    }
 }
 
 // ------------------------------------------------------------------------------------------- dispatch
@@ -386,9 +403,9 @@ int launch(const TA* A, const TW* W, TC* C, float* part, long part_floats, int M
     if (vector && few_rows(M, N, K)) {
         // strips of 8 where strips of 16 would give fewer than two workgroups a compute unit
         if (M <= 8 && N < 32 * gi_compute_units())
-            gemm_exact_few_rows_kernel<8, TA, TW, TC, ACC><<<(N + 7) / 8, 256, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc);
+            gemm_exact_few_rows_kernel<8, TA, TW, TC, ACC, false><<<(N + 7) / 8, 256, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, Gate{-1, 0.f});
         else
-            gemm_exact_few_rows_kernel<16, TA, TW, TC, ACC><<<(N + 15) / 16, 512, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc);
+            gemm_exact_few_rows_kernel<16, TA, TW, TC, ACC, false><<<(N + 15) / 16, 512, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, Gate{-1, 0.f});
         return 0;
     }
     Cut c = cut_for(M, N, K);
@@ -445,5 +462,18 @@ GI_API int gi_gemm_exact(const void* A, int a_dtype, const void* W, int w_dtype,
 #undef GO
     if (rc) return rc;
     GI_CHECK_LAUNCH("gemm_exact");
+    return 0;
+}
+
+// Whether gi_gemm_exact_gated takes a product of these sizes.
+GI_API int gi_gemm_exact_gated_takes(int M, int N, int K) { return M > 0 && N > 0 && N % 2 == 0 && K > 0 && K % 4 == 0 && few_rows(M, N, K); }
+
+// C [M, N / 2] = act(gate) * up of A W^T with W = [gate; up] (N rows in all), 32-bit throughout: the bits of gi_gemm_exact and gi_act_mul.  C must not be what A reads.
+GI_API int gi_gemm_exact_gated(const float* A, const float* W, float* C, int act, float limit, int M, int N, int K, long lda, long ldw, long ldc, hipStream_t stream) {
+    GI_REQUIRE(act >= 0 && act < GI_N_ACTIVATIONS && gi_gemm_exact_gated_takes(M, N, K), "gemm_exact (gated): sizes M %d, N %d, K %d or activation %d are not taken", M, N, K, act);
+    GI_REQUIRE(lda >= K && ldw >= K && ldc >= N / 2 && lda % 4 == 0 && ldw % 4 == 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0,
+               "gemm_exact (gated): rows must be 16-byte aligned (strides %ld, %ld, %ld)", lda, ldw, ldc);
+    gemm_exact_few_rows_kernel<16, float, float, float, false, true><<<(N / 2 + 7) / 8, 512, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, Gate{act, limit});
+    GI_CHECK_LAUNCH("gemm_exact (gated)");
     return 0;
 }

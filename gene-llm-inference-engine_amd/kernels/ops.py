@@ -33,6 +33,7 @@ _SIGNATURES = {
     "gi_gather_rows": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
     "gi_scale_rows": [c_void_p, c_int, c_int, c_long, c_float, c_void_p],
     "gi_softcap_rows": [c_void_p, c_int, c_int, c_long, c_float, c_void_p],
+    "gi_gemm_exact_gated": [c_void_p, c_void_p, c_void_p, c_int, c_float, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p],
     "gi_gemm_exact": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long, c_void_p],
     "gi_attention_exact": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_long, c_int,
                            c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_void_p, c_long, c_int, c_void_p],
@@ -144,6 +145,8 @@ def lib():
         l.gi_attention_decode_workgroups_per_unit.restype = c_int
         l.gi_attention_bf16_supports.argtypes = [c_int, c_int, c_int]
         l.gi_attention_bf16_supports.restype = c_int
+        l.gi_gemm_exact_gated_takes.argtypes = [c_int, c_int, c_int]
+        l.gi_gemm_exact_gated_takes.restype = c_int
         l.gi_gemm_exact_scratch_floats.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_exact_scratch_floats.restype = c_long
         l.gi_gemm_bf16_scratch_floats.argtypes = [c_int, c_int, c_int]
@@ -562,6 +565,31 @@ def gemm_exact(a, w, out, accumulate=False):
     part = torch.empty(n_part, dtype=torch.float32, device=out.device) if n_part else None
     _call("gi_gemm_exact", a.data_ptr(), _code(a, "gemm: a"), w.data_ptr(), _code(w, "gemm: w"), out.data_ptr(), _code(out, "gemm: out"),
           1 if accumulate else 0, m, n, k, a.stride(0), w.stride(0), out.stride(0), _ptr(part), n_part, _stream())
+    return out
+
+
+@lru_cache(maxsize=8192)
+def _exact_gated_takes(m, n, k) -> bool:
+    return bool(lib().gi_gemm_exact_gated_takes(m, n, k))
+
+
+def gemm_exact_gated_takes(a, w, out) -> bool:
+    """Whether `gemm_exact_gated` takes these operands: a few float32 rows, 16-byte aligned, and results that are not written over what it reads."""
+    return (a.dtype == w.dtype == out.dtype == torch.float32 and a.stride(1) == 1 and w.stride(1) == 1 and out.stride(1) == 1 and a.stride(0) % 4 == 0 and w.stride(0) % 4 == 0
+            and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and out.untyped_storage().data_ptr() != a.untyped_storage().data_ptr()
+            and _exact_gated_takes(a.shape[0], w.shape[0], w.shape[1]))
+
+
+def gemm_exact_gated(a, w, out, activation="silu", limit=0.0):
+    """out = act(a @ gate.T) * (a @ up.T) for a few rows in 32-bit, w being [gate; up], in the bits of `gemm_exact` and `act_mul`."""
+    _dev(a, w, out)
+    if not (a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1] and out.shape == (a.shape[0], w.shape[0] // 2) and gemm_exact_gated_takes(a, w, out)
+            and activation in ACTIVATIONS):
+        raise KernelError("gemm_exact_gated: float32 operands [rows, k], [2 * columns, k] with aligned rows, a result [rows, columns] of its own, and sizes that are taken")
+    if _profile is not None:
+        _profile.note = (f"{w.shape[0]}x{w.shape[1]} gated", w.numel() * w.element_size())
+    _call("gi_gemm_exact_gated", a.data_ptr(), w.data_ptr(), out.data_ptr(), ACTIVATIONS[activation], float(limit), a.shape[0], w.shape[0], w.shape[1], a.stride(0),
+          w.stride(0), out.stride(0), _stream())
     return out
 
 

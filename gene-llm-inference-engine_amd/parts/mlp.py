@@ -9,6 +9,7 @@ from ..kernels import ops
 from ..weights.loader import TensorNeed
 from .base import FeedForward, register_feed_forward
 from .linear import activation_dtype_for, linear, linear_onto, linear_xielu, takes_handed_norm
+from .norm import NormedRows
 
 
 class SwiGlu(FeedForward):
@@ -47,10 +48,14 @@ class SwiGlu(FeedForward):
             mid = torch.empty((T, inter), dtype=torch.bfloat16, device=ctx.device)
             linear(h, self.w_gate_up, mid, gated=self.activation, gate_limit=self.limit, ctx=ctx)
         else:
-            gate_up = torch.empty((T, 2 * inter), dtype=torch.float32, device=ctx.device)
-            linear(h, self.w_gate_up, gate_up)
             mid = torch.empty((T, inter), dtype=self.mid_dtype, device=ctx.device)
-            ops.act_mul(gate_up, mid, self.activation, self.limit)
+            rows = h.materialize() if isinstance(h, NormedRows) else h
+            if ops.gemm_exact_gated_takes(rows, self.w_gate_up, mid):
+                ops.gemm_exact_gated(rows, self.w_gate_up, mid, self.activation, self.limit)
+            else:
+                gate_up = torch.empty((T, 2 * inter), dtype=torch.float32, device=ctx.device)
+                linear(h, self.w_gate_up, gate_up)
+                ops.act_mul(gate_up, mid, self.activation, self.limit)
         if overwrite:
             linear(mid, self.w_down, residual)
             return None

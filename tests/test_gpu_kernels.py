@@ -81,6 +81,18 @@ def test_gemm_exact_kernels_agree_in_bits(m, n, k):
     assert torch.equal(wide[:m], full)
 
 
+@pytest.mark.parametrize("m,n,k,gated", [(3, 16384, 2048, "silu"), (1, 1000, 4096, "gelu_tanh"), (8, 34, 36, "swish_clamped"), (16, 1004, 264, "gelu_tanh"), (9, 2, 4, "silu")])
+def test_gemm_exact_gated_has_the_bits_of_two_kernels(m, n, k, gated):
+    o = ops()
+    a, w = randn(m, k + 4, seed=5)[:, :k], randn(n, k, seed=6, scale=2.0 / k ** 0.5)
+    product = o.gemm_exact(a, w, torch.empty(m, n, device=DEV))
+    want = torch.empty(m, n // 2, device=DEV)
+    o.act_mul(product, want, gated, 1.5)
+    got = torch.full((m, n // 2 + 3), 7.0, device=DEV)
+    o.gemm_exact_gated(a, w, got[:, :n // 2], gated, 1.5)
+    assert torch.equal(got[:, :n // 2], want) and bool((got[:, n // 2:] == 7).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 16, 8), (1, 2048, 2048), (3, 100, 136), (8, 130, 264), (16, 64, 128), (17, 1000, 520),
                                    (33, 48, 72), (64, 515, 1032), (65, 128, 64), (100, 300, 200), (128, 128, 128), (200, 257, 96),
                                    (513, 384, 1024), (2048, 96, 160),
