@@ -303,19 +303,55 @@ constexpr int FEW_ROWS = 16, AHEAD = 8;
 // read both again (3 rows of 16,384 x 2,048: 27.4 us and 5 for the gate, 28 in one).  The norm of the rows was tried here too (every workgroup working the rows'
 // factors out for itself while its first weights are on their way, in the bits of the norm's kernel): 1,024 workgroups that each read all rows once more took 39 us
 // for 27.4 and the norm's 5, 3,072 x 2,048 13 for 8.6 and 5.  Not kept.
-struct Gate { int act; float limit; };
+struct Plain { static constexpr int KIND = 0; };
+struct Gate { static constexpr int KIND = 1; int act; float limit; };
+// Turn: the product is an attention layer's q/k/v, a strip of 8 is four channels of a head's first half and the four they are turned with, and queries and keys
+// leave turned, keys and values into the pages (rope_store_kernel's places and bits; that launch took 5 us a layer).
+struct Turn {
+    static constexpr int KIND = 2;
+    const float *cos_t, *sin_t;                // [M, hd / 2], null: not turned
+    const int *pos, *slot, *table;
+    int table_stride;
+    float *q_out, *cache;
+    long page_stride;
+    int page_size, n_heads, n_kv, hd;
+};
 
-template <int STRIP, typename TA, typename TW, typename TC, bool ACCUMULATE, bool GATED>
+template <int STRIP, typename TA, typename TW, typename TC, bool ACCUMULATE, typename End>
 __global__ __launch_bounds__(STRIP == 16 ? 512 : 256) void gemm_exact_few_rows_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C,
-                                                                                      int M, int N, int K, long lda, long ldw, long ldc, Gate gate) {
+                                                                                      int M, int N, int K, long lda, long ldw, long ldc, End end) {
+    constexpr bool GATED = End::KIND == 1, TURNED = End::KIND == 2;
     static_assert(!GATED || STRIP == 16, "a strip of gates and ups");
+    static_assert(!TURNED || STRIP == 8, "a strip of pairs");
     __shared__ f32x4 sums[RANGES][STRIP == 16 ? 64 : 16];                 // per range: [group of 4 columns][row]
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
     const int n0 = blockIdx.x * (GATED ? 8 : STRIP), L = range_length(K), inter = N / 2;
     const int q = STRIP == 16 ? wave : 2 * wave + (r >> 3), row = STRIP == 16 ? r : r & 7;
     const int q_last = STRIP == 16 ? wave : 2 * wave + 1, q_first = STRIP == 16 ? wave : 2 * wave;       // of the wave
     const int base = q * L + 4 * g;
-    const TW* w_row = W + (size_t)(GATED ? min(n0 + (row & 7), inter - 1) + (row >> 3) * inter : min(n0 + row, N - 1)) * ldw;
+    int first_row = GATED ? min(n0 + (row & 7), inter - 1) + (row >> 3) * inter : min(n0 + row, N - 1);
+    f32x4 cs = f32x4{1.f, 1.f, 1.f, 1.f}, sn = f32x4{0.f, 0.f, 0.f, 0.f};
+    int head = 0, channel = 0, place = 0;
+    long page = 0;
+    if constexpr (TURNED) {
+        const int strips = end.hd / 8, half = end.hd / 2;       // of a head
+        head = blockIdx.x / strips;
+        channel = (blockIdx.x % strips) * 4;
+        first_row = head * end.hd + channel + (row & 3) + (row >> 2) * half;
+        if (threadIdx.x < 16 && (threadIdx.x & 7) < M) {        // what the end needs of row threadIdx.x % 8, on its way while the products run
+            const int m = threadIdx.x & 7;
+            if (end.cos_t != nullptr) {
+                cs = load4(end.cos_t + (size_t)m * half + channel);
+                sn = load4(end.sin_t + (size_t)m * half + channel);
+            }
+            if (head >= end.n_heads) {
+                const int p = end.pos[m];
+                page = end.table[(size_t)end.slot[m] * end.table_stride + p / end.page_size];
+                place = p % end.page_size;
+            }
+        }
+    }
+    const TW* w_row = W + (size_t)first_row * ldw;
     const TA* a_row = A + (size_t)min(row, M - 1) * lda;
     const int blocks = max(0, min(L, K - q_first * L) + 15) / 16;             // until both of the wave's ranges are through
     const int whole = max(0, min(L, K - q_last * L)) / 16 / AHEAD * AHEAD;    // ... of them with nothing to guard, in groups
@@ -345,7 +381,7 @@ __global__ __launch_bounds__(STRIP == 16 ? 512 : 256) void gemm_exact_few_rows_k
     const int e = threadIdx.x;
     if (e >= STRIP * STRIP / 4) return;
     const int m = e % STRIP, n = n0 + 4 * (e / STRIP);
-    if (!GATED && m >= M) return;
+    if (!GATED && !TURNED && m >= M) return;
     f32x4 v[RANGES];
 #pragma unroll
     for (int z = 0; z < RANGES; ++z) v[z] = sums[z][e];
@@ -357,7 +393,33 @@ __global__ __launch_bounds__(STRIP == 16 ? 512 : 256) void gemm_exact_few_rows_k
         if (e >= 32 || m >= M) return;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            if (n + i < inter) store_f32(C, (size_t)m * ldc + n + i, gated_act(sum[i], up[i], gate.act, gate.limit));
+            if (n + i < inter) store_f32(C, (size_t)m * ldc + n + i, gated_act(sum[i], up[i], end.act, end.limit));
+    } else if constexpr (TURNED) {                              // threads 0 .. 7 hold the first halves' channels of their row, the thread 8 further those they are turned with
+        f32x4 other;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) other[i] = __shfl_xor(sum[i], 8, 64);
+        if (m >= M) return;
+        const bool second = e >= 8;
+        const int at = channel + (second ? end.hd / 2 : 0);
+        f32x4 turned;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float a = second ? other[i] : sum[i], b = second ? sum[i] : other[i];
+            turned[i] = second ? fmaf(a, sn[i], b * cs[i]) : fmaf(a, cs[i], -(b * sn[i]));      // (rounded where rope_store_kernel's a sin + b cos and a cos - b sin are)
+        }
+        if (head < end.n_heads) {
+            *reinterpret_cast<f32x4*>(end.q_out + ((size_t)m * end.n_heads + head) * end.hd + at) = turned;
+            return;
+        }
+        float* keys = end.cache + page * end.page_stride;
+        const int kv = head - end.n_heads;
+        if (kv < end.n_kv) {
+            *reinterpret_cast<f32x4*>(keys + ((size_t)kv * end.page_size + place) * end.hd + at) = turned;
+            return;
+        }
+        float* values = keys + (size_t)end.n_kv * end.page_size * end.hd + ((size_t)(kv - end.n_kv) * end.hd + at) * end.page_size + place;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) values[(size_t)i * end.page_size] = sum[i];
     } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -403,9 +465,9 @@ int launch(const TA* A, const TW* W, TC* C, float* part, long part_floats, int M
     if (vector && few_rows(M, N, K)) {
         // strips of 8 where strips of 16 would give fewer than two workgroups a compute unit
         if (M <= 8 && N < 32 * gi_compute_units())
-            gemm_exact_few_rows_kernel<8, TA, TW, TC, ACC, false><<<(N + 7) / 8, 256, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, Gate{-1, 0.f});
+            gemm_exact_few_rows_kernel<8, TA, TW, TC, ACC, Plain><<<(N + 7) / 8, 256, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, Plain{});
         else
-            gemm_exact_few_rows_kernel<16, TA, TW, TC, ACC, false><<<(N + 15) / 16, 512, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, Gate{-1, 0.f});
+            gemm_exact_few_rows_kernel<16, TA, TW, TC, ACC, Plain><<<(N + 15) / 16, 512, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, Plain{});
         return 0;
     }
     Cut c = cut_for(M, N, K);
@@ -473,7 +535,30 @@ GI_API int gi_gemm_exact_gated(const float* A, const float* W, float* C, int act
     GI_REQUIRE(act >= 0 && act < GI_N_ACTIVATIONS && gi_gemm_exact_gated_takes(M, N, K), "gemm_exact (gated): sizes M %d, N %d, K %d or activation %d are not taken", M, N, K, act);
     GI_REQUIRE(lda >= K && ldw >= K && ldc >= N / 2 && lda % 4 == 0 && ldw % 4 == 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0,
                "gemm_exact (gated): rows must be 16-byte aligned (strides %ld, %ld, %ld)", lda, ldw, ldc);
-    gemm_exact_few_rows_kernel<16, float, float, float, false, true><<<(N / 2 + 7) / 8, 512, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, Gate{act, limit});
+    gemm_exact_few_rows_kernel<16, float, float, float, false, Gate><<<(N / 2 + 7) / 8, 512, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, Gate{act, limit});
     GI_CHECK_LAUNCH("gemm_exact (gated)");
+    return 0;
+}
+
+// Whether gi_gemm_exact_qkv_rope_store takes a q/k/v product of these sizes with heads of hd channels.
+GI_API int gi_gemm_exact_qkv_rope_store_takes(int M, int N, int K, int hd) {
+    return M > 0 && M <= 8 && N > 0 && N < 32 * gi_compute_units() && K > 0 && K % 4 == 0 && hd >= 8 && hd % 8 == 0 && N % hd == 0;
+}
+
+// The q/k/v product of an attention layer in 32-bit for a few rows, A [M, K] x W [N, K]^T with N = (n_heads + 2 n_kv) * hd, whose results do not come back: the bits
+// and places of gi_gemm_exact and gi_rope_store.
+GI_API int gi_gemm_exact_qkv_rope_store(const float* A, const float* W, int M, int N, int K, long lda, long ldw, const float* cos_t, const float* sin_t, const int* pos,
+                                        const int* slot, const int* table, int table_stride, float* q_out, float* cache, long page_stride, int page_size, int n_heads, int n_kv,
+                                        int hd, hipStream_t stream) {
+    GI_REQUIRE(n_heads > 0 && n_kv > 0 && N == (n_heads + 2 * n_kv) * hd && gi_gemm_exact_qkv_rope_store_takes(M, N, K, hd),
+               "gemm_exact (q/k/v): M %d, N %d, K %d with %d heads and %d key/value heads of %d are not taken", M, N, K, n_heads, n_kv, hd);
+    GI_REQUIRE(lda >= K && ldw >= K && lda % 4 == 0 && ldw % 4 == 0 && (((uintptr_t)A | (uintptr_t)W | (uintptr_t)q_out | (uintptr_t)cache | (uintptr_t)cos_t | (uintptr_t)sin_t) & 15) == 0,
+               "gemm_exact (q/k/v): operands must be 16-byte aligned (strides %ld, %ld)", lda, ldw);
+    GI_REQUIRE((cos_t == nullptr) == (sin_t == nullptr) && pos != nullptr && slot != nullptr && table != nullptr && q_out != nullptr && cache != nullptr && page_size > 0 &&
+                   page_stride >= 2L * n_kv * page_size * hd && page_stride % 4 == 0,
+               "gemm_exact (q/k/v): positions, slots, a table, q_out, both tables of the rotation or none, and a cache with a page stride of at least 2*n_kv*page_size*hd are needed");
+    const Turn turn = {cos_t, sin_t, pos, slot, table, table_stride, q_out, cache, page_stride, page_size, n_heads, n_kv, hd};
+    gemm_exact_few_rows_kernel<8, float, float, float, false, Turn><<<N / 8, 256, 0, stream>>>(A, W, nullptr, M, N, K, lda, ldw, 0L, turn);
+    GI_CHECK_LAUNCH("gemm_exact (q/k/v)");
     return 0;
 }

@@ -33,6 +33,8 @@ _SIGNATURES = {
     "gi_gather_rows": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
     "gi_scale_rows": [c_void_p, c_int, c_int, c_long, c_float, c_void_p],
     "gi_softcap_rows": [c_void_p, c_int, c_int, c_long, c_float, c_void_p],
+    "gi_gemm_exact_qkv_rope_store": [c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
+                                     c_long, c_int, c_int, c_int, c_int, c_void_p],
     "gi_gemm_exact_gated": [c_void_p, c_void_p, c_void_p, c_int, c_float, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p],
     "gi_gemm_exact": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long, c_void_p],
     "gi_attention_exact": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_long, c_int,
@@ -145,6 +147,8 @@ def lib():
         l.gi_attention_decode_workgroups_per_unit.restype = c_int
         l.gi_attention_bf16_supports.argtypes = [c_int, c_int, c_int]
         l.gi_attention_bf16_supports.restype = c_int
+        l.gi_gemm_exact_qkv_rope_store_takes.argtypes = [c_int, c_int, c_int, c_int]
+        l.gi_gemm_exact_qkv_rope_store_takes.restype = c_int
         l.gi_gemm_exact_gated_takes.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_exact_gated_takes.restype = c_int
         l.gi_gemm_exact_scratch_floats.argtypes = [c_int, c_int, c_int]
@@ -591,6 +595,41 @@ def gemm_exact_gated(a, w, out, activation="silu", limit=0.0):
     _call("gi_gemm_exact_gated", a.data_ptr(), w.data_ptr(), out.data_ptr(), ACTIVATIONS[activation], float(limit), a.shape[0], w.shape[0], w.shape[1], a.stride(0),
           w.stride(0), out.stride(0), _stream())
     return out
+
+
+@lru_cache(maxsize=8192)
+def _exact_qkv_takes(m, n, k, hd) -> bool:
+    return bool(lib().gi_gemm_exact_qkv_rope_store_takes(m, n, k, hd))
+
+
+def gemm_exact_qkv_rope_store_takes(a, w, cache, hd) -> bool:
+    """Whether `gemm_exact_qkv_rope_store` takes these operands: a few float32 rows, 16-byte aligned, and a float32 cache."""
+    return (a.dtype == w.dtype == cache.dtype == torch.float32 and a.stride(1) == 1 and w.stride(1) == 1 and a.stride(0) % 4 == 0 and w.stride(0) % 4 == 0
+            and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and cache.data_ptr() % 16 == 0 and cache.stride(0) % 4 == 0 and _exact_qkv_takes(a.shape[0], w.shape[0], w.shape[1], hd))
+
+
+def gemm_exact_qkv_rope_store(a, w, cos, sin, positions, slots, table, q_out, cache, n_heads, n_kv, hd):
+    """The q/k/v product a @ w.T of an attention layer in 32-bit for a few rows: the queries go, rotated, into q_out, the keys (rotated) and the values into the
+    cache's pages, in the bits of `gemm_exact` and `rope_store`.  cos, sin: float32 [m, hd/2] or None."""
+    _dev(a, w, cos, sin, positions, slots, table, q_out, cache)
+    m, k = a.shape
+    n = w.shape[0]
+    if not (w.shape == (n, k) and n == (n_heads + 2 * n_kv) * hd and gemm_exact_qkv_rope_store_takes(a, w, cache, hd) and q_out.dtype == torch.float32
+            and q_out.shape == (m, n_heads * hd) and q_out.is_contiguous() and q_out.data_ptr() % 16 == 0):
+        raise KernelError(f"gemm_exact (q/k/v): a product of {m} x {n} x {k} with heads of {hd}, or these operands, are not taken")
+    if cos is not None:
+        for t in (cos, sin):
+            if not (t.dtype == torch.float32 and t.shape == (m, hd // 2) and t.is_contiguous() and t.data_ptr() % 16 == 0):
+                raise KernelError("gemm_exact (q/k/v): cos/sin must be float32 [m, hd/2], 16-byte aligned")
+    page_size = cache.shape[3]
+    _check_cache(cache, table, page_size, n_kv, hd, "gemm_exact (q/k/v)")
+    _i32(positions, "gemm_exact (q/k/v): positions", m)
+    _i32(slots, "gemm_exact (q/k/v): slots", m)
+    if _profile is not None:
+        _profile.note = (f"{n}x{k}", n * k * w.element_size())
+    _call("gi_gemm_exact_qkv_rope_store", a.data_ptr(), w.data_ptr(), m, n, k, a.stride(0), w.stride(0), _ptr(cos), _ptr(sin), positions.data_ptr(), slots.data_ptr(),
+          table.data_ptr(), table.stride(0), q_out.data_ptr(), cache.data_ptr(), cache.stride(0), page_size, n_heads, n_kv, hd, _stream())
+    return q_out
 
 
 def attention_max_head_size() -> int:

@@ -58,6 +58,13 @@ def qkv_rotate_store_attend(h, w_qkv, ctx, cache, *, n_heads, n_kv_heads, head_d
             return ops.attention(q_rot, cache.kv, att, ctx, cache.table, n_heads, n_kv_heads, head_dim, window)
         if norm_in is None:
             h = rows                  # (whole rows: what `linear` below would make of h)
+    if before_rotation is None and cache.writes and (tables is not None or position is None) and in_dtype == torch.float32 and w_qkv.dtype == torch.float32:
+        # the same for a few rows in 32-bit, in the product's own kernel
+        rows = h.materialize() if isinstance(h, NormedRows) else h
+        if ops.gemm_exact_qkv_rope_store_takes(rows, w_qkv, cache.kv, head_dim) and (cos is None or (cos.data_ptr() | sin.data_ptr()) % 16 == 0):
+            q_rot = torch.empty((T, a_dim), dtype=torch.float32, device=ctx.device)
+            ops.gemm_exact_qkv_rope_store(rows, w_qkv, cos, sin, ctx.row_pos, ctx.row_slot, cache.table, q_rot, cache.kv, n_heads, n_kv_heads, head_dim)
+            return ops.attention(q_rot, cache.kv, att, ctx, cache.table, n_heads, n_kv_heads, head_dim, window)
     if cache.writes:
         qkv = torch.empty((T, a_dim + 2 * kv_dim), dtype=torch.float32, device=ctx.device)
         linear(h, w_qkv, qkv, ctx=ctx)

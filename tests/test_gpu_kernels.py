@@ -81,6 +81,24 @@ def test_gemm_exact_kernels_agree_in_bits(m, n, k):
     assert torch.equal(wide[:m], full)
 
 
+@pytest.mark.parametrize("m,hidden,n_heads,n_kv,hd,page_size,rotate", [(3, 2048, 32, 8, 64, 16, True), (8, 264, 6, 3, 8, 4, True), (1, 1000, 5, 1, 128, 12, True), (5, 36, 2, 2, 24, 7, False)])
+def test_gemm_exact_qkv_has_the_bits_of_two_kernels(m, hidden, n_heads, n_kv, hd, page_size, rotate):
+    """A few rows' q/k/v product in 32-bit that rotates and fills the pages itself: queries and pages in the bits of product and `rope_store`, and nothing else touched."""
+    o = ops()
+    n, a_dim, kv_dim = (n_heads + 2 * n_kv) * hd, n_heads * hd, n_kv * hd
+    a, w = randn(m, hidden, seed=1), randn(n, hidden, seed=2, scale=0.05)
+    cos, sin = (torch.cos(randn(m, hd // 2, seed=3)), torch.sin(randn(m, hd // 2, seed=3))) if rotate else (None, None)
+    table = torch.randperm(12, generator=torch.Generator().manual_seed(4)).view(4, 3).to(torch.int32).to(DEV)
+    slots = torch.tensor([i % 4 for i in range(m)], dtype=torch.int32, device=DEV)
+    positions = torch.tensor([(page_size - 1 + (i // 4) * page_size + i % 4) % (3 * page_size) for i in range(m)], dtype=torch.int32, device=DEV)
+    caches = [torch.full((12, 2, n_kv, page_size, hd), 7.0, device=DEV) for _ in range(2)]
+    qkv, want, got = torch.empty(m, n, device=DEV), torch.empty(m, a_dim, device=DEV), torch.empty(m, a_dim, device=DEV)
+    o.gemm_exact(a, w, qkv)
+    o.rope_store(qkv[:, :a_dim], qkv[:, a_dim:a_dim + kv_dim], qkv[:, a_dim + kv_dim:], cos, sin, positions, slots, table, want, caches[0], n_heads, n_kv, hd)
+    o.gemm_exact_qkv_rope_store(a, w, cos, sin, positions, slots, table, got, caches[1], n_heads, n_kv, hd)
+    assert torch.equal(got, want) and torch.equal(caches[0], caches[1]) and bool((caches[1] != 7).any())
+
+
 @pytest.mark.parametrize("m,n,k,gated", [(3, 16384, 2048, "silu"), (1, 1000, 4096, "gelu_tanh"), (8, 34, 36, "swish_clamped"), (16, 1004, 264, "gelu_tanh"), (9, 2, 4, "silu")])
 def test_gemm_exact_gated_has_the_bits_of_two_kernels(m, n, k, gated):
     o = ops()
