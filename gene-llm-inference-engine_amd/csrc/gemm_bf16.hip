@@ -392,6 +392,15 @@ __device__ __forceinline__ void tile_add_handing_norm(const float* tile, const T
     }
 }
 
+// Results of a prompt's product that nobody reads soon from the same L2 leave it as they come: what an L2 holds of them at a kernel's end is written back before
+// the next begins.  2,048 rows of 16,384 x 2,048 gated 121 -> 116.5 us, 8,192 of 28,672 x 4,096 1,470 -> 1,433, 1,777 of 8,192 x 2,048 through xielu in its
+// step 72 -> 66, 32-bit stores of 1,777 x 5,376 there 34 -> 32.  Not the rows a product adds onto, nor queries, keys and values: what reads those next got
+// slower by as much (attention behind them 82.5 -> 84.3 us, the products onto 3,072 columns 90.7 -> 92.4).
+typedef unsigned gi_uint4 __attribute__((ext_vector_type(4)));
+typedef unsigned gi_uint2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void store_streaming(void* p, uint4 v) { __builtin_nontemporal_store(gi_uint4{v.x, v.y, v.z, v.w}, (gi_uint4*)p); }
+__device__ __forceinline__ void store_streaming(void* p, uint2 v) { __builtin_nontemporal_store(gi_uint2{v.x, v.y}, (gi_uint2*)p); }
+
 // ------------------------------------------------------------------------------------------ piped
 // The same product for large shapes, with the operands going from global memory straight into LDS
 // (global_load_lds_dwordx4: no registers in between) through a ring of blocks of 64 k, so that
@@ -793,7 +802,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
             for (int it = 0; it < WM / 8; ++it) {
                 const int row = it * 8 + frow, m = m0 + wm + row, c = (n0 + wn) / 2 + part * 64 + fchunk * 8;      // output column
                 const uint4 v = *reinterpret_cast<const uint4*>(mine + row * STAGE_ROW + fchunk * 16);
-                if (m < M && c + 7 < N / 2 && (ldc & 7) == 0) *reinterpret_cast<uint4*>((bf16_t*)C + (size_t)m * ldc + c) = v;
+                if (m < M && c + 7 < N / 2 && (ldc & 7) == 0) store_streaming((bf16_t*)C + (size_t)m * ldc + c, v);
                 else if (m < M) {
                     const bf16_t* e = reinterpret_cast<const bf16_t*>(&v);
 #pragma unroll
@@ -829,7 +838,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
             for (int it = 0; it < WM / 8; ++it) {
                 const int row = it * 8 + frow, m = m0 + wm + row, c = n0 + wn + part * 64 + fchunk * 8;
                 const uint4 v = *reinterpret_cast<const uint4*>(mine + row * STAGE_ROW + fchunk * 16);
-                if (m < M && c + 7 < N && (ldc & 7) == 0) *reinterpret_cast<uint4*>((bf16_t*)C + (size_t)m * ldc + c) = v;
+                if (m < M && c + 7 < N && (ldc & 7) == 0) store_streaming((bf16_t*)C + (size_t)m * ldc + c, v);
                 else if (m < M) {
                     const bf16_t* e = reinterpret_cast<const bf16_t*>(&v);
 #pragma unroll
@@ -858,8 +867,10 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
                     if constexpr (EPI == EPI_ADD_F32) {
                         const float4 old = *reinterpret_cast<const float4*>(dst);
                         v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
+                        *reinterpret_cast<float4*>(dst) = v;
+                    } else {
+                        store_streaming(dst, uint4{__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)});
                     }
-                    *reinterpret_cast<float4*>(dst) = v;
                 } else {
                     const float e[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
@@ -911,7 +922,6 @@ __global__ void clear_counters_kernel(unsigned* counters, int n) {
     for (int i = threadIdx.x; i < n; i += blockDim.x) counters[i] = 0;
 }
 constexpr int TALL_MAX_SHARES = 4;
-typedef unsigned gi_uint4 __attribute__((ext_vector_type(4)));
 constexpr int DEVICE_SCOPE = 16;               // sc1 in a buffer access's cache policy
 template <int EPI>
 __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ C, int M, int N, int K,
@@ -1093,13 +1103,15 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
                 const size_t at = (size_t)m * ldc + c;
                 if (whole) {
                     if constexpr (ELEM == 2) {
-                        *reinterpret_cast<uint2*>((bf16_t*)C + at) = uint2{f32x2_to_bf16x2(v.x, v.y), f32x2_to_bf16x2(v.z, v.w)};
+                        store_streaming((bf16_t*)C + at, uint2{f32x2_to_bf16x2(v.x, v.y), f32x2_to_bf16x2(v.z, v.w)});
                     } else {
                         if constexpr (EPI == EPI_ADD_F32) {
                             const float4 o = *reinterpret_cast<const float4*>((const float*)C + at);
                             v.x += o.x; v.y += o.y; v.z += o.z; v.w += o.w;
+                            *reinterpret_cast<float4*>((float*)C + at) = v;
+                        } else {
+                            store_streaming((float*)C + at, uint4{__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)});
                         }
-                        *reinterpret_cast<float4*>((float*)C + at) = v;
                     }
                 } else {
                     const float e[4] = {v.x, v.y, v.z, v.w};
