@@ -1175,14 +1175,14 @@ GI_API int gi_attention_bf16_supports(int hd, int page_size, int prompt) {
     return hd == 32 || hd == 64 || hd == 96 || hd == 128 || hd == 256;
 }
 
-static bool takes_wide(int n_tiles, int n_heads, int hd, int n_splits, int paired) {
+static bool takes_wide(int n_tiles, int n_heads, int hd, int n_splits, int paired, bool shared) {
     const bool one_round = (long)(paired ? n_tiles / 2 : n_tiles) * n_heads <= gi_compute_units();
-    return hd == 128 || (hd == 64 && n_splits == 1 && !one_round);
+    return hd == 128 || (hd == 64 && n_splits == 1 && (!one_round || shared));
 }
 // Floats of scratch for gi_attention_prompt_bf16 with `most_shares` shares; 0 where the kernel that takes these sizes shares no keys out.  The counters it
 // wants are 2 * n_tiles * n_heads of 32 bits, all 0, and are left so.
 GI_API long gi_attention_prompt_share_floats(int n_tiles, int rows_per_tile, int n_heads, int hd, int n_splits, int paired, int most_shares) {
-    if (n_splits != 1 || most_shares < 2 || most_shares > WIDE_MAX_SHARES || (long)n_tiles * most_shares > 65535 || !takes_wide(n_tiles, n_heads, hd, n_splits, paired)) return 0;
+    if (n_splits != 1 || most_shares < 2 || most_shares > WIDE_MAX_SHARES || (long)n_tiles * most_shares > 65535 || !takes_wide(n_tiles, n_heads, hd, n_splits, paired, true)) return 0;
     const int waves = hd == 64 && rows_per_tile == 64 ? 2 : 4;
     return (long)n_tiles * n_heads * most_shares * (hd == 128 ? wide_share_bytes<128>(waves) : wide_share_bytes<64>(waves)) / 4;
 }
@@ -1217,7 +1217,8 @@ GI_API int gi_attention_prompt_bf16(const void* q, const void* cache, void* out,
     // first kernel's pairs of tiles are the better balance while they fit the chip in one round (a workgroup of 16 waves a compute
     // unit: 2,048 rows of 32 heads take 56 against 61 us) and where few tiles share their keys out; beyond one round its time
     // doubles at once and the wide kernel's many small workgroups win (2,560 rows: 68 against 100 us; 8,192: 360 against 572).
-    if (takes_wide(n_tiles, n_heads, hd, n_splits, paired)) {
+    // With its long walks shared out the wide kernel is the faster one within a round too, from so many rows or keys on that the caller shares them out.
+    if (takes_wide(n_tiles, n_heads, hd, n_splits, paired, most_shares > 1)) {
         GI_REQUIRE((long)n_tiles * n_splits * (most_shares > 1 ? most_shares : 1) <= 65535, "attention_prompt: %d tiles in %d splits are too many for one launch", n_tiles, n_splits);
         WideShares shares = {1, 0, nullptr, nullptr};
         if (most_shares > 1) {

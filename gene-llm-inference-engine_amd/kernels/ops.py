@@ -1312,16 +1312,23 @@ def prompt_attention_splits(n_groups, n_heads, span, target_groups=512):
 PROMPT_SHARE_COUNTERS = 4096
 
 
-def prompt_attention_shares(contexts, n_heads, hd):
+def prompt_attention_shares(contexts, n_heads, hd, tile=128, one_round=False):
     """(shares, keys) for the tiles of a step that fill the chip: a tile's keys are shared out over up to so many workgroups of so many keys each, (1, 0) where
     none should be.  The chip holds two workgroups a compute unit (three at heads of 64 channels); a tile that sees far more keys than there are for each of
     those places keeps one busy when the others have ended.  Measured, one workgroup a tile and shared: 24 heads of 128 over 1,350 rows behind 1,000 and 674 more
     87.6 -> 71 us (77 in two shares, 79 in four), 2,000 rows 74.6 -> 52 (57 in three), 32 heads over 1,000 rows 40 -> 31, over 1,500 58 -> 41, but over 2,048
     62.5 -> 71.6 and over 800 the same; 32 heads of 64 over 2,560 rows 52.4 -> 49.8, over 3,500 99.5 -> 82, over 900 behind 1,000 and 1,100 more 52 -> 40 (44 in
-    three).  The lines: the longest walk 2.1 (64 channels: 1.5) times a place's even share and 16 tiles of 64 keys, and every share from the third on
-    leaves each 12 (16) of them."""
+    three).  The lines there: the longest walk 2.1 (64 channels: 1.5) times a place's even share and 16 tiles of 64 keys, and every share from the third on
+    leaves each 12 (16) of them.
+    one_round: heads of 64 channels whose pairs of tiles are at most one for a compute unit.  Their kernel walks a pair's keys with one workgroup of 16 waves; a
+    workgroup a tile and up to three shares of 512 keys or more take 39.6 us for 40.8 (32 heads over 2,048 rows), 29.3 for 34 (1,500), 18.5 for 23 (1,024),
+    17.1 for 20.4 (800), 36.5 for 47 (600 behind 2,000).  Tiles of 64 rows (steps of up to 768) only where a walk has 20 tiles of keys: 300 rows behind 1,000
+    and 200 more 24 for 27.4, but 760 rows from the beginning 19.7 for 18.2."""
     walks = [-(-c // 64) for c in contexts]
     wide = hd == 128
+    if hd == 64 and one_round:
+        longest = max(walks)
+        return (3, 64 * max(8, -(-longest // 3))) if longest >= (20 if tile == 64 else 9) else (1, 0)
     longest, even = max(walks), sum(walks) * n_heads / (lib().gi_compute_units() * (2 if wide else 3))
     if longest < 16 or longest < (2.1 if wide else 1.5) * even:
         return (1, 0)
@@ -1511,8 +1518,10 @@ def attention_bf16(q, cache, out, plan: AttentionPlan, positions, slots, table, 
                                            target_groups=PAIRED_TARGET_GROUPS if plan.paired else 512)      # a pair's workgroup has twice the waves
         n_part = plan.n_tile_rows * n_heads * n_splits * (hd + 2) if n_splits > 1 else 0
         most, keys, counters = 1, 0, None
-        if n_splits == 1 and memo is not None and plan.tile_contexts is not None and plan.n_tiles * n_heads <= PROMPT_SHARE_COUNTERS // 2:
-            most, keys = prompt_attention_shares([min(c, seen(c, plan.tile)) for c in plan.tile_contexts], n_heads, hd)
+        one_round = (plan.n_tiles // 2 if plan.paired else plan.n_tiles) * n_heads <= lib().gi_compute_units()
+        contexts = plan.tile_contexts if plan.tile_contexts is not None else [plan.max_tile_context] if hd == 64 and one_round else None
+        if n_splits == 1 and memo is not None and contexts is not None and hd in (64, 128) and plan.n_tiles * n_heads <= PROMPT_SHARE_COUNTERS // 2:
+            most, keys = prompt_attention_shares([min(c, seen(c, plan.tile)) for c in contexts], n_heads, hd, plan.tile, one_round)
             n_part = lib().gi_attention_prompt_share_floats(plan.n_tiles, plan.tile, n_heads, hd, 1, 1 if plan.paired else 0, most)
             if n_part:
                 counters = memo.get("attention_counters")

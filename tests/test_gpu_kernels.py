@@ -876,7 +876,8 @@ def test_many_prompt_tiles_of_many_heads(window):
 
 @pytest.mark.parametrize("n_heads,n_kv,hd,segs,window,known", [
     (24, 8, 128, [(0, 1020, 1350), (1, 0, 674), (2, 49, 1)], None, "3"), (32, 8, 128, [(0, 0, 1000)], None, "2"), (16, 8, 128, [(0, 4000, 260), (1, 0, 1900)], None, "4"), (24, 8, 128, [(0, 1020, 1350), (1, 0, 674)], None, "sinks"),
-    (24, 8, 128, [(0, 1020, 1350), (1, 0, 674)], None, "cap"), (64, 16, 64, [(0, 3000, 900), (1, 0, 401)], None, "3"), (64, 16, 64, [(0, 3000, 130), (1, 0, 960)], 2000, "2")])
+    (24, 8, 128, [(0, 1020, 1350), (1, 0, 674)], None, "cap"), (64, 16, 64, [(0, 3000, 900), (1, 0, 401)], None, "3"), (64, 16, 64, [(0, 3000, 130), (1, 0, 960)], 2000, "2"),
+    (32, 8, 64, [(0, 0, 1500)], None, "3"), (32, 8, 64, [(0, 0, 1777)], 1024, "3"), (32, 8, 64, [(0, 1300, 300), (1, 0, 200)], None, "3")])
 def test_long_walks_of_prompt_tiles_share_their_keys_out(n_heads, n_kv, hd, segs, window, known):
     """Portions far behind others whose tiles fill the chip all the same: the tiles with long walks are made by several workgroups that meet in the kernel.
     Against 64 bits where that is stated plainly, against one workgroup a tile, and in bits against themselves, whoever came last."""
@@ -886,7 +887,8 @@ def test_long_walks_of_prompt_tiles_share_their_keys_out(n_heads, n_kv, hd, segs
     rows = [(slot, pos0 + i) for slot, pos0, n in segs for i in range(n)]
     starts = [sum(n for _, _, n in segs[:i]) for i in range(len(segs))]
     plan = o.AttentionPlan(starts, [n for _, _, n in segs], [p for _, p, _ in segs], [s_ + 1 for s_, _, _ in segs], DEV)
-    most, keys = o.prompt_attention_shares([min(c, (window or c) + plan.tile) for c in plan.tile_contexts], n_heads, hd)
+    most, keys = o.prompt_attention_shares([min(c, (window or c) + plan.tile) for c in plan.tile_contexts], n_heads, hd, plan.tile,
+                                           plan.n_tiles // 2 * n_heads <= o.lib().gi_compute_units())
     assert plan.n_tiles and most > 1 and (known not in "234" or most == int(known)), (most, keys)
     q = randn(len(rows), n_heads * hd, dtype=torch.bfloat16, seed=3)
     pos = torch.tensor([p for _, p in rows], dtype=torch.int32, device=DEV)
