@@ -905,6 +905,40 @@ def test_long_walks_of_prompt_tiles_share_their_keys_out(n_heads, n_kv, hd, segs
         assert rel(seen[0], plain_attention_rows(q, dense, rows, n_heads, n_kv, hd, window)) < 8e-3
 
 
+def test_workgroups_that_meet_in_a_kernel_under_capture():
+    """A product with shared tiles and an attention with shared walks in one captured pass, whose counters are filled in the pass: every replay gives the bits of
+    the same calls made one by one, with other work and a synchronization between."""
+    from types import SimpleNamespace
+    o = ops()
+    m, n_heads, n_kv, hd = 1000, 32, 8, 128
+    width = n_heads * hd
+    cache, table, _ = build_paged([m], n_kv, hd, 16, torch.bfloat16, seed=5)
+    plan = o.AttentionPlan([0], [m], [0], [1], DEV)
+    assert o.prompt_attention_shares(plan.tile_contexts, n_heads, hd)[0] > 1 and o.gemm_bf16_tall_shares(2 * m, width // 2, 2 * width) == 2
+    pos, slots = torch.arange(m, dtype=torch.int32, device=DEV), torch.ones(m, dtype=torch.int32, device=DEV)
+    q, a, w = randn(m, width, dtype=torch.bfloat16, seed=3), randn(2 * m, 2 * width, dtype=torch.bfloat16, seed=4), randn(width // 2, 2 * width, dtype=torch.bfloat16, seed=6)
+    att, out = torch.empty(m, width, dtype=torch.bfloat16, device=DEV), torch.empty(2 * m, width // 2, device=DEV)
+
+    def step():
+        ctx = SimpleNamespace(memo={}, device=torch.device(DEV))
+        for _ in range(2):
+            o.attention_bf16(q, cache, att, plan, pos, slots, table, n_heads, n_kv, hd, memo=ctx.memo)
+            o.gemm_bf16(a, w, out, counters=o.step_counters(ctx, 2 * m, *w.shape))
+
+    step()
+    want = att.clone(), out.clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step()
+    for _ in range(4):
+        att.fill_(7), out.fill_(7)
+        graph.replay()
+        assert torch.equal(att, want[0]) and torch.equal(out, want[1])
+        torch.cuda.synchronize()
+        o.gemm_bf16(a, w, torch.empty_like(out))
+
+
 @pytest.mark.parametrize("n_heads,n_kv,hd", [(4, 2, 64), (4, 2, 128), (64, 16, 64)])
 def test_prompt_attention_with_scores_that_climb_along_the_context(n_heads, n_kv, hd):
     """Every query points along one direction and the keys' share of that direction climbs with their position, by 2 to 12
