@@ -300,13 +300,14 @@ __global__ __launch_bounds__(256) void gemm_exact_add_parts_kernel(const float* 
 constexpr int FEW_ROWS = 16, AHEAD = 8;
 
 // GATED: W is [gate; up], a strip of 16 is 8 gates and the 8 ups of the same columns, and act(gate) * up goes out in the bits of the gate's own kernel, which
-// read both again (3 rows of 16,384 x 2,048: 27.4 us and 5 for the gate, 28 in one).  The norm of the rows was tried here too (every workgroup working the rows'
+// read both again (3 rows of 16,384 x 2,048: 27.4 us and 5 for the gate, 27.4 in one).  The norm of the rows was tried here too (every workgroup working the rows'
 // factors out for itself while its first weights are on their way, in the bits of the norm's kernel): 1,024 workgroups that each read all rows once more took 39 us
 // for 27.4 and the norm's 5, 3,072 x 2,048 13 for 8.6 and 5.  Not kept.
 struct Plain { static constexpr int KIND = 0; };
 struct Gate { static constexpr int KIND = 1; int act; float limit; };
 // Turn: the product is an attention layer's q/k/v, a strip of 8 is four channels of a head's first half and the four they are turned with, and queries and keys
-// leave turned, keys and values into the pages (rope_store_kernel's places and bits; that launch took 5 us a layer).
+// leave turned, keys and values into the pages (rope_store_kernel's places and bits; 3 rows of 3,072 x 2,048: 8.6 us and 5 for that
+// launch, 10.5 in one).
 struct Turn {
     static constexpr int KIND = 2;
     const float *cos_t, *sin_t;                // [M, hd / 2], null: not turned
