@@ -418,7 +418,7 @@ __global__ __launch_bounds__(128 * NW * PAIR) void attention_prompt_kernel(const
 // A walk that is much longer than the others' share of the chip is cut into shares of keys, up to WideShares::most of them by its own length, whose workgroups meet
 // in the kernel: the one that comes last merges the others' {m, l, O} with its own, in the order of the keys whoever it is, and writes the rows; the
 // others leave theirs in the order of their registers and end.  Who has come is counted, and the sums go past the L2s of the dies, as in the products'
-// kernel for the last tiles of a round (`TileShares` in gemm_bf16.hip): the last waits only for workgroups that have nothing left to wait for.
+// kernel for the last tiles of a round (`TileShares` in gemm_bf16.hip): the last waits only for workgroups that have nothing left to wait for, and not for ever.
 // 24 heads of 128 over a portion of 1,350 rows behind 1,000 positions and one of 674 (264 workgroups that walk up to 37 tiles of keys beside 144 short ones).
 struct WideShares {
     int most, keys;                            // shares at most (1: none), and keys a share should have
@@ -641,6 +641,7 @@ __global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_w
         if (extra.sinks != nullptr && split == 0) add_sink(extra.sinks[head], m, l);
         constexpr int PIECES = DT * 4 + 1;                    // 16 bytes a lane each; the last holds m and l
         unsigned& drawn = *reinterpret_cast<unsigned*>(lds);   // (everybody is past the last tile)
+        float& start = *reinterpret_cast<float*>(lds + 4);     // 0, or no number where the others never came
         const size_t walk = (size_t)group * n_heads + head;
         unsigned* const counter = shares.counters + 2 * walk;
         const int at = (wv * PIECES * 64 + lane) * 16;
@@ -663,8 +664,7 @@ __global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_w
             if (tid == 0) __hip_atomic_fetch_add(counter + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return;
         }
-        if (tid == 0)
-            while ((int)__hip_atomic_load(counter + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 < n_splits) __builtin_amdgcn_s_sleep(1);
+        if (tid == 0) start = others_came(counter + 1, n_splits - 1) ? 0.f : __builtin_nanf("");
         __syncthreads();
         if (tid < 2) __hip_atomic_store(counter + tid, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         float weight[WIDE_MAX_SHARES], share_l[WIDE_MAX_SHARES], big = -INFINITY;
@@ -680,7 +680,7 @@ __global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_w
         }
 #pragma unroll
         for (int of = 0; of < WIDE_MAX_SHARES; ++of) big = fmaxf(big, weight[of]);
-        l = 0.f;
+        l = start;
 #pragma unroll
         for (int of = 0; of < WIDE_MAX_SHARES; ++of) {
             weight[of] = weight[of] == -INFINITY ? 0.f : exp2_fast(weight[of] - big);

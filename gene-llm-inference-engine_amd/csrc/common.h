@@ -100,3 +100,15 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
     for (int w = 0; w < NT / 64; ++w) t += red[w];
     return t;
 }
+
+// For workgroups of one launch that meet: waits (one thread of a workgroup) until `counter` says that `n` others have come.  A wait ends whatever the counter
+// held at the start: false after so many polls of about a microsecond each, of which a meeting takes some dozens at most, for a caller whose counters were
+// not 0 or that gave them to two launches at once.  The workgroup then leaves no numbers (NaN) where its sums would have gone.
+constexpr int MEETING_POLLS = 1 << 18;
+__device__ __forceinline__ bool others_came(unsigned* counter, int n) {
+    for (int polls = 0; (int)__hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < n; ++polls) {
+        if (polls == MEETING_POLLS) return false;
+        __builtin_amdgcn_s_sleep(1);
+    }
+    return true;
+}

@@ -910,7 +910,8 @@ struct TileOrder {
 // The tiles of the last, incomplete round share their k out: with at most half as many left as there are compute units, each is made by
 // `shares` workgroups, every one of which sums a part of k.  The one that comes last to its end adds the others' sums to its own, in the order of k whoever it
 // is, and goes on to the epilogue.  An earlier one leaves its sums in its place and ends.  A tile's two counters are drawn from when a workgroup has its sums
-// and raised when these are in memory: the last waits, but only for workgroups that have drawn, whose way to the second counter holds no wait of their own.
+// and raised when these are in memory: the last waits, but only for workgroups that have drawn, whose way to the second counter holds no wait of their own
+// (and not for ever: `others_came`).
 // The sums go past the L2s, which belong to one die each (stores and loads of device scope): no fence, whose write-back of a whole L2 costs more than
 // all of this.
 struct TileShares {
@@ -1145,6 +1146,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
     }
     // A half at a time: first the one that another share would rather finish.
     __shared__ unsigned drawn[2];
+    __shared__ float start[2];                                                           // 0, or no number where the others never came
     unsigned* const counters = shared.counters + (u - shared.whole) * 4;
     float* const places_of_tile = shared.sums + (size_t)(u - shared.whole) * shared.shares * (BM * BN);
     auto place = [&](int of) { return __builtin_amdgcn_make_buffer_rsrc(places_of_tile + (size_t)of * (BM * BN), 0, BM * BN * 4, 0x00027000); };
@@ -1175,8 +1177,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
         }
         TileOld<NT> old;
         if (hands_norm) tile_old<NT>(old, (const float*)C, ldc, m0 + half * 128, n0, M);
-        if (tid == 0)
-            while ((int)__hip_atomic_load(counter + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 < shared.shares) __builtin_amdgcn_s_sleep(1);
+        if (tid == 0) start[turn_of] = others_came(counter + 1, shared.shares - 1) ? 0.f : __builtin_nanf("");
         __syncthreads();
         if (tid < 2) __hip_atomic_store(counter + tid, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // as the next product of the step wants them
         if (group == half) {
@@ -1184,7 +1185,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
             for (int i = 0; i < TM; ++i) {
                 floatx16 total[TN];
 #pragma unroll
-                for (int j = 0; j < TN; ++j) total[j] = floatx16{};
+                for (int j = 0; j < TN; ++j) total[j] = floatx16{} + start[turn_of];
 #pragma unroll 1
                 for (int of = 0; of < shared.shares; ++of) {
                     if (of == share) {

@@ -939,6 +939,39 @@ def test_workgroups_that_meet_in_a_kernel_under_capture():
         o.gemm_bf16(a, w, torch.empty_like(out))
 
 
+def test_a_meeting_of_workgroups_ends_whatever_its_counters_held():
+    """Counters that were not 0 (a workgroup has been counted that never comes): the launch ends, the results that are not whole are no numbers, all others are right,
+    and the counters are 0 again."""
+    o = ops()
+    m, n, k = 2048, 2048, 8192                                # 128 tiles of 256 x 128, each in two shares; a tile's counters: {drawn, raised} of its upper half, of its lower half
+    a, w = randn(m, k, dtype=torch.bfloat16, seed=4), randn(n, k, dtype=torch.bfloat16, seed=6)
+    counters = torch.zeros(o.lib().gi_gemm_bf16_counters(), dtype=torch.int32, device=DEV)
+    right = o.gemm_bf16(a, w, torch.empty(m, n, device=DEV), counters=counters)
+    assert o.gemm_bf16_tall_shares(m, n, k) == 2 and bool(torch.isfinite(right).all())
+    counters[4 * 5 + 2] = 1                                   # the sixth tile's lower half
+    hurt = o.gemm_bf16(a, w, torch.empty(m, n, device=DEV), counters=counters)
+    bad = torch.isnan(hurt)
+    rows, columns = bad.any(1).nonzero().flatten(), bad.any(0).nonzero().flatten()
+    assert rows.numel() == columns.numel() == 128 and int(rows[0]) % 256 == 128 and int(columns[0]) % 128 == 0 and int(bad.sum()) == 128 * 128
+    assert torch.equal(hurt[~bad], right[~bad]) and not bool(counters.any())
+    m, n_heads, n_kv, hd = 1000, 32, 8, 128
+    cache, table, _ = build_paged([m], n_kv, hd, 16, torch.bfloat16, seed=5)
+    plan = o.AttentionPlan([0], [m], [0], [1], DEV)
+    pos, slots = torch.arange(m, dtype=torch.int32, device=DEV), torch.ones(m, dtype=torch.int32, device=DEV)
+    q, memo = randn(m, n_heads * hd, dtype=torch.bfloat16, seed=3), {}
+
+    def attend():
+        return o.attention_bf16(q, cache, torch.empty_like(q), plan, pos, slots, table, n_heads, n_kv, hd, memo=memo)
+
+    right = attend()
+    late = plan.tiles.view(-1, 4)[:, 0].argmax().item()       # the tile of the last rows: two shares
+    memo["attention_counters"][2 * (late * n_heads + 7)] = 1
+    hurt = attend()
+    bad = torch.isnan(hurt).view(m, n_heads, hd)
+    assert bool(bad[896:, 7].all()) and int(bad.sum()) == (m - 896) * hd and torch.equal(hurt[~bad.view(m, -1)], right[~bad.view(m, -1)])
+    assert not bool(memo["attention_counters"].any()) and torch.equal(attend(), right)
+
+
 @pytest.mark.parametrize("n_heads,n_kv,hd", [(4, 2, 64), (4, 2, 128), (64, 16, 64)])
 def test_prompt_attention_with_scores_that_climb_along_the_context(n_heads, n_kv, hd):
     """Every query points along one direction and the keys' share of that direction climbs with their position, by 2 to 12
