@@ -795,13 +795,13 @@ GI_API int gi_heads_product(const void* a, long lda, const void* w, void* out, i
                n_rows, n_heads, k_dim, n_out);
     GI_REQUIRE(lda % 8 == 0 && lda >= (long)n_heads * k_dim && ((uintptr_t)a & 15) == 0 && ((uintptr_t)w & 15) == 0 && out_head_stride >= n_out &&
                ldo >= (long)(n_heads - 1) * out_head_stride + n_out, "heads_product: operands must be 16-byte aligned with row strides that are multiples of 8, and rows long enough");
-    GI_REQUIRE((n_out + 15) / 16 <= 65535, "heads_product: too many columns");
+    GI_REQUIRE((n_out + 63) / 64 <= 65535, "heads_product: too many columns");
 #define GO_AS(TO, RT, J)                                                                                                                            \
     heads_product_kernel<TO, RT, J><<<dim3((n_rows + 16 * RT - 1) / (16 * RT), n_heads, (n_out + 16 * J - 1) / (16 * J)), 64, 0, stream>>>(           \
         (const bf16_t*)a, lda, (const bf16_t*)w, (TO*)out, ldo, out_head_stride, n_rows, k_dim, n_out, gate, ldg)
 #define GO(TO)                                  \
     do {                                        \
-        if (n_rows <= 16) GO_AS(TO, 1, 1);      \
+        if (n_rows <= 16 && (n_out + 15) / 16 <= 65535) GO_AS(TO, 1, 1);      \
         else if (n_rows <= 256) GO_AS(TO, 1, 4); \
         else GO_AS(TO, 4, 4);                   \
     } while (0)

@@ -616,6 +616,16 @@ def test_every_head_s_product_in_one_launch(rows, H, k, n):
     assert not ops.heads_product(a.to(DEV)[:, 1:], w.to(DEV), out, H, n)           # operands it does not take: the caller goes head by head
 
 
+@pytest.mark.parametrize("rows, n", [(2, 65535 * 16), (2, 65535 * 16 + 5), (17, 65535 * 16 + 5)])
+def test_a_head_s_product_of_more_columns_than_a_grid_has_strips_of_16(rows, n):
+    from geneinfer_amd.kernels import ops
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    a, w = torch.randn(rows, 8, generator=g, device=DEV).to(torch.bfloat16), torch.randn(1, n, 8, generator=g, device=DEV).to(torch.bfloat16)
+    out = torch.zeros(rows, n + 3, device=DEV)
+    assert ops.heads_product(a, w, out[:, :n], 1)
+    assert relative_error(out[:, :n], a.double() @ w[0].double().T) < 1e-5 and (out[:, n:] == 0).all()
+
+
 # =============================================================================================== whole models
 def _portions(n, sizes=(7, 2, 5, 3, 2, 11, 1, 4, 2, 19)):
     out, i = [], 0
