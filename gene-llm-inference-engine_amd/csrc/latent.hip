@@ -148,7 +148,10 @@ constexpr float LOG2E = 1.4426950408889634f;
 // result is multiplied by sigmoid(gate).
 // A few rows are bound by a round trip to memory (16 columns a wave, all of k asked for at once), the rows of prompts by how often w is read (64 rows a
 // wave) and by the stores: 1,777 rows of 32 heads, 64 -> 256 and 256 -> 64 channels together 45.0 us with 16 rows a wave and stores of 2 bytes, so 29.4;
-// 5 rows 11.8 with 64 columns a wave, so 7.5.
+// 5 rows 11.8 with 64 columns a wave, so 7.5.  Where 64 rows a wave leave fewer waves than three quarters of the compute units, 16 rows a wave are
+// the faster ones: 257 rows of 4 heads, 64 -> 36 channels 3.1 us (5.0 with 64 rows a wave), of 8 heads, 512 -> 128 6.5 (8.9), 500 rows 6.7 (8.9; 128 waves),
+// but 700 rows 9.1 (8.9; 176 waves), 400 rows of 32 heads, 256 -> 64 6.7 (5.9; 224 waves).  And where strips of 16 columns are more than eight waves a compute
+// unit, so are 64 columns a wave for a few rows: 128 heads, 128 -> 512 (4,096 waves), 8 rows 4.7 us (5.4), 16 rows 5.0 (6.3).
 template <typename TO, int RT, int J>
 __global__ __launch_bounds__(64) void heads_product_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restrict__ w, TO* __restrict__ out, long ldo,
                                                           long out_head_stride, int n_rows, int k_dim, int n_out, const float* __restrict__ gate, long ldg) {
@@ -796,13 +799,15 @@ GI_API int gi_heads_product(const void* a, long lda, const void* w, void* out, i
     GI_REQUIRE(lda % 8 == 0 && lda >= (long)n_heads * k_dim && ((uintptr_t)a & 15) == 0 && ((uintptr_t)w & 15) == 0 && out_head_stride >= n_out &&
                ldo >= (long)(n_heads - 1) * out_head_stride + n_out, "heads_product: operands must be 16-byte aligned with row strides that are multiples of 8, and rows long enough");
     GI_REQUIRE((n_out + 63) / 64 <= 65535, "heads_product: too many columns");
+    const bool few_strips = (long)n_heads * ((n_out + 15) / 16) <= 8L * gi_compute_units();      // (of one row of 16; so the grid takes them)
+    const bool few_waves = (long)((n_rows + 63) / 64) * n_heads * ((n_out + 63) / 64) < gi_compute_units() * 3 / 4;
 #define GO_AS(TO, RT, J)                                                                                                                            \
     heads_product_kernel<TO, RT, J><<<dim3((n_rows + 16 * RT - 1) / (16 * RT), n_heads, (n_out + 16 * J - 1) / (16 * J)), 64, 0, stream>>>(           \
         (const bf16_t*)a, lda, (const bf16_t*)w, (TO*)out, ldo, out_head_stride, n_rows, k_dim, n_out, gate, ldg)
 #define GO(TO)                                  \
     do {                                        \
-        if (n_rows <= 16 && (n_out + 15) / 16 <= 65535) GO_AS(TO, 1, 1);      \
-        else if (n_rows <= 256) GO_AS(TO, 1, 4); \
+        if (n_rows <= 16 && few_strips) GO_AS(TO, 1, 1);      \
+        else if (n_rows <= 256 || few_waves) GO_AS(TO, 1, 4); \
         else GO_AS(TO, 4, 4);                   \
     } while (0)
     if (out_dtype == GI_F32) GO(float);

@@ -602,7 +602,8 @@ def test_latent_attention_with_scores_that_climb_along_the_context_and_sinks(pag
     assert relative_error(out, want) < 1.5e-2                                   # (probabilities and outputs are kept in bfloat16)
 
 
-@pytest.mark.parametrize("rows, H, k, n", [(1, 8, 32, 128), (37, 3, 72, 40), (300, 32, 64, 256), (16, 2, 256, 64), (5, 1, 8, 7)])
+@pytest.mark.parametrize("rows, H, k, n", [(1, 8, 32, 128), (37, 3, 72, 40), (300, 32, 64, 256), (16, 2, 256, 64), (5, 1, 8, 7),
+                                           (300, 3, 72, 40), (575, 21, 64, 36), (577, 19, 40, 100), (13, 65, 64, 512), (16, 64, 40, 500)])
 def test_every_head_s_product_in_one_launch(rows, H, k, n):
     from geneinfer_amd.kernels import ops
     g = torch.Generator().manual_seed(rows + k)
