@@ -64,16 +64,21 @@ def norm_to_hand_on(reader, n_rows: int):
 
 class NormToMake:
     """A norm that whoever writes its rows may make whole on the way (`ReadyRows`), as a part's `then`: the parts whose `then` goes to `linear_onto` alone
-    (`hands_whole_norms`) take it."""
+    (`hands_whole_norms`, said by the class whose `forward` that is: a part built on one may have a `forward` of its own, to which `then` is a norm) take it."""
 
     def __init__(self, norm: "RmsNorm"):
         self.norm = norm
 
 
+def _takes_norm_to_make(part) -> bool:
+    cls = next(c for c in type(part).__mro__ if "forward" in vars(c))
+    return bool(vars(cls).get("hands_whole_norms", False))
+
+
 def norm_to_make(reader, part):
     """reader: as above.  The norm as `part`'s `then`, if the part may make it whole and its reader takes it so in bfloat16; None otherwise."""
     norm, reads = reader if reader is not None else (None, None)
-    if (not getattr(part, "hands_whole_norms", False) or not hasattr(norm, "handed_weight") or not getattr(reads, "accepts_deferred_norm", False)
+    if (not getattr(part, "hands_whole_norms", False) or not _takes_norm_to_make(part) or not hasattr(norm, "handed_weight") or not getattr(reads, "accepts_deferred_norm", False)
             or getattr(reads, "in_dtype", None) != torch.bfloat16):
         return None
     return NormToMake(norm)
