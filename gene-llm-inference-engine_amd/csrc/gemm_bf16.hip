@@ -1994,8 +1994,12 @@ enum Large { PIPED_128, TALL_256, PINGPONG_256 };
 // some 5 us later for the exchange, and 2 for every share.  Alone, 2,048 rows of 2,048 x 8,192 take 76 us in two shares (95 as 128 x 128 tiles, one a unit),
 // of 2,048 x 4,096 47 (58), of 2,048 x 2,048 33 (31: not taken); 3,000 rows of 3,072 x 8,192, one round and 32 tiles, 163 in four shares and 180 in two
 // (203 in two rounds), of 3,072 x 3,072 83 (96); 2,048 rows of 5,120 x 3,072 76 in four (78).  Fewer than 8 blocks a share are not worth the exchange.
+// Of 874 products that were shared out where these times alone spoke for it, 35 were slower than before by up to a quarter; the lines here and in `large_kernel` leave those
+// out.  Beside whole tiles the times have to promise 7.5 %: 1,161 rows of 8,192 x 2,048, promised 7 %, took 69 us for 62.
+// clears: no counters are given, and the launch that clears them takes 4 us (2 to 5).
+constexpr double CLEAR_US = 4;
 struct TallCut { int whole, rest, shares; double us; };
-static TallCut tall_cut(int M, int N, int K, bool may_share) {
+static TallCut tall_cut(int M, int N, int K, bool may_share, bool clears) {
     const int units = gi_compute_units(), tiles = ((M + 255) / 256) * ((N + 127) / 128), rest = tiles % units;
     const double blocks = K / PK, each = blocks * 0.715 + 13;
     TallCut cut = {tiles, 0, 1, (tiles + units - 1) / units * each};
@@ -2003,7 +2007,7 @@ static TallCut tall_cut(int M, int N, int K, bool may_share) {
     const double before = tiles / units * each, whole = cut.us;
     for (int shares = 2; shares * rest <= units && shares <= TALL_MAX_SHARES && blocks >= 8 * shares; ++shares) {
         const double us = before + ((int)blocks + shares - 1) / shares * 0.85 + 16 + 2 * shares;
-        if (us < 0.95 * whole && us < cut.us) cut = {tiles - rest, rest, shares, us};
+        if (us < 0.925 * whole && us + (clears ? CLEAR_US : 0) < 0.95 * whole && us < cut.us) cut = {tiles - rest, rest, shares, us};
     }
     return cut;
 }
@@ -2011,7 +2015,8 @@ static TallCut tall_cut(int M, int N, int K, bool may_share) {
 static long tall_counter_floats(const TallCut& cut) { return (4L * cut.rest + 63) / 64 * 64; }
 static long tall_scratch_floats(const TallCut& cut) { return cut.shares > 1 ? tall_counter_floats(cut) + (long)cut.rest * cut.shares * 256 * 128 : 0; }
 
-static Large large_kernel(int M, int N, int K, int epi, bool rope, bool hands_norm, bool scaled_rows, bool may_share) {
+struct LargeChoice { Large kernel; TallCut cut; };              // cut: how the tall kernel makes its tiles, where that is the one
+static LargeChoice large_kernel(int M, int N, int K, int epi, bool rope, bool hands_norm, bool scaled_rows, bool may_share, bool clears) {
     const long units = gi_compute_units(), m128 = (M + 127) / 128, m256 = (M + 255) / 256, n128 = (N + 127) / 128, n256 = (N + 255) / 256;
     const auto rounds = [&](long tiles) { return (double)((tiles + units - 1) / units); };
     const bool many = many_tiles(M, N), gated = !rope && is_gated(epi);
@@ -2025,28 +2030,47 @@ static Large large_kernel(int M, int N, int K, int epi, bool rope, bool hands_no
     // (one: measured 31 us at 32 blocks, 50 to 58 at 64, 95 at 128)
     double piped = small > 1 ? small * (blocks * 0.45 + ends.each) * (small > 2 ? 1.15 : 1) - ends.less : blocks * 0.65 + 10.5;      // (several: two workgroups a unit)
     if (scaled_rows && !rope) piped = 1e30;
-    const double tall = tall_cut(M, N, K, may_share).us;
+    const TallCut whole = tall_cut(M, N, K, false, false), cut = tall_cut(M, N, K, may_share, clears);
     const double pingpong = many && !rope ? rounds(m256 * n256) * (blocks * 1.45 + 14) : 1e30;
     // (gating 256 x 128 sums at a time costs the tall kernel 3 us a round more: 1,500 rows by 16,384 of 2,048, three rounds of it against one and a
-    // half of the ping-pong kernel: 114 us against 103)
-    if (pingpong < piped && 0.95 * pingpong <= tall + (gated ? 3 * rounds(m256 * n128) : 0)) return PINGPONG_256;
-    return tall < piped ? TALL_256 : PIPED_128;
+    // half of the ping-pong kernel: 114 us against 103.  Shares do not take its products: with 160 to 192 tiles a block takes it 1.3 us, and 4,096 rows of
+    // 3,072 x 8,192 added took 182 with it and 198 shared, 1,368 of 8,192 x 6,784 stored 149 and 160)
+    if (pingpong < piped && 0.95 * pingpong <= whole.us + (gated ? 3 * rounds(m256 * n128) : 0)) return {PINGPONG_256, whole};
+    if (whole.us < piped) return {TALL_256, cut};
+    if (cut.shares > 1) {
+        if (small > 1) return cut.us + (clears ? CLEAR_US : 0) < piped ? LargeChoice{TALL_256, cut} : LargeChoice{PIPED_128, whole};
+        // Both in one round that may leave units idle, which the times above do not know: fitted to 534 products of 128 to 1,024 rows and of more by few columns, whose
+        // 128 x 128 tiles take so long within 5 % and whose shares within 7.  3 us ahead they are never the slower ones (273 rows of 8,192 x 3,072 handing a norm on: 34 us
+        // as 128 x 128 tiles, 42 in shares, 31 expected), and what is left out by that gains 2 %.
+        const bool through_lds = rope || hands_norm, added = !rope && epi == EPI_ADD_F32;
+        const double fill = (double)(m128 * n128) / units, shared_fill = (double)(cut.rest * cut.shares) / units;
+        const double one_round = 4.7 + blocks * (0.41 + 0.207 * fill) + (through_lds ? 1.4 : added ? 7.4 : 0);
+        const double shared = 6 + ((int)blocks + cut.shares - 1) / cut.shares * (0.45 + 0.476 * shared_fill) + 1.77 * cut.shares + (through_lds ? 2.9 : added ? 3.3 : gated ? 1.9 : 0);
+        if (shared + (clears ? CLEAR_US : 0) + 3 < one_round) return {TALL_256, cut};
+    }
+    return {PIPED_128, whole};
 }
-static Large large_kernel_of_kind(int M, int N, int K, int kind) {               // kinds as for gi_gemm_bf16_large_kernel
-    const int epi = kind == 0 ? EPI_STORE_F32 : kind <= 2 ? EPI_ADD_F32 : kind == 6 ? EPI_XIELU : EPI_GATED_BF16;
-    return large_kernel(M, N, K, epi, kind == 5, kind == 2, kind == 4, kind != 6);
+// Kinds as for gi_gemm_bf16_large_kernel.
+static LargeChoice large_kernel_of_kind(int M, int N, int K, int kind, bool counters) {
+    const int epi = kind == 0 ? EPI_STORE_F32 : kind <= 2 ? EPI_ADD_F32 : kind == 6 ? EPI_XIELU : kind == 7 ? EPI_STORE_BF16 : EPI_GATED_BF16;
+    return large_kernel(M, N, K, epi, kind == 5, kind == 2, kind == 4, kind != 6, !counters);
+}
+static bool takes_large(int M, int N, int K) { return M > SKINNY_MAX_ROWS && K % PK == 0 && N >= 128; }
+
+// By how many workgroups each tile of the last round of a product is made that has all the scratch it asks for (1: one), with or without counters.
+GI_API int gi_gemm_bf16_shares(int M, int N, int K, int kind, int counters) {
+    if (!takes_large(M, N, K) || gi_gemm_bf16_piped_splits(M, N, K) > 1) return 1;
+    const LargeChoice choice = large_kernel_of_kind(M, N, K, kind, counters != 0);
+    return choice.kernel == TALL_256 ? choice.cut.shares : 1;
 }
 
-// Floats of scratch a product of these sizes needs (partial sums where k is shared out), 0 if none.
-GI_API long gi_gemm_bf16_scratch_floats(int M, int N, int K) {
+// Floats of scratch a product of these sizes and kind asks for (partial sums where k is shared out), 0 if none.  It does without where gi_gemm_bf16_shares says
+// more than one: the kernels that share nothing out serve then.
+GI_API long gi_gemm_bf16_scratch_floats(int M, int N, int K, int kind, int counters) {
     if (M <= SKINNY_MAX_ROWS) return (long)gi_gemm_bf16_skinny_splits(N, K) * M * N;
     const int splits = gi_gemm_bf16_piped_splits(M, N, K);
     if (splits > 1) return (long)splits * M * N;
-    if (K % PK != 0 || N < 128) return 0;
-    const long shared = tall_scratch_floats(tall_cut(M, N, K, true));
-    for (int kind = 0; shared > 0 && kind < 6; ++kind)
-        if (large_kernel_of_kind(M, N, K, kind) == TALL_256) return shared;
-    return 0;
+    return gi_gemm_bf16_shares(M, N, K, kind, counters) > 1 ? tall_scratch_floats(large_kernel_of_kind(M, N, K, kind, counters != 0).cut) : 0;
 }
 
 static const NormIn NO_NORM_IN = {nullptr, 0, 0.f, 1, 0.f};
@@ -2321,10 +2345,13 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
     GI_REQUIRE(norm_in.squares == nullptr || rope != nullptr || (is_gated(epi) && many_tiles(M, N) && norm_in.parts <= PIPED_MAX_PARTS),
                "gemm_bf16: a product of M %d, N %d, K %d takes no norm handed on in %d pieces", M, N, K, norm_in.parts);
     GI_REQUIRE(!many_tiles(M, N) || (lda < (1L << 22) && ldw < (1L << 22)), "gemm_bf16: row strides %ld, %ld are too large for the tile-relative addressing", lda, ldw);
-    const long sharing = tall_scratch_floats(tall_cut(M, N, K, true));
+    const bool clears = counters == nullptr;
+    const long sharing = tall_scratch_floats(tall_cut(M, N, K, true, clears));
     const bool may_share = sharing > 0 && scratch != nullptr && scratch_floats >= sharing && ((uintptr_t)scratch & 15) == 0;
-    const Large which = lda < (1L << 22) && ldw < (1L << 22)
-                            ? large_kernel(M, N, K, epi, rope != nullptr, norm_out.scaled != nullptr, norm_in.squares != nullptr, may_share) : PIPED_128;
+    LargeChoice choice = {PIPED_128, {}};
+    if (lda < (1L << 22) && ldw < (1L << 22))
+        choice = large_kernel(M, N, K, epi, rope != nullptr, norm_out.scaled != nullptr, norm_in.squares != nullptr, may_share, clears);
+    const Large which = choice.kernel;
     if (which == PINGPONG_256) {
 #define PINGPONG(EPI_)                                                                                                                  \
     do {                                                                                                                                \
@@ -2346,10 +2373,10 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
         return 0;
     }
     if (which == TALL_256) {
-        const TallCut cut = tall_cut(M, N, K, may_share);
+        const TallCut& cut = choice.cut;
         const TileOrder order = tall_order(M, N, cut.whole);
         const TileShares shared = {cut.whole, cut.rest, cut.shares, cut.shares > 1 ? scratch + tall_counter_floats(cut) : nullptr, counters != nullptr ? counters : (unsigned*)scratch};
-        if (cut.shares > 1 && counters == nullptr) {                                     // (5.5 us)
+        if (cut.shares > 1 && clears) {
             clear_counters_kernel<<<1, 256, 0, stream>>>(shared.counters, 4 * cut.rest);
             GI_CHECK_LAUNCH("gemm_bf16 (counters)");
         }
@@ -2520,16 +2547,16 @@ GI_API int gi_gemm_bf16_qkv_rope_store(const void* A, const void* W, int M, int 
 
 // Which kernel makes a product of more than 128 rows whose rows lie whole in memory: 0 the tiles of 128 x 128, 1 those of 256 x 128, 2 those of 256 x 256,
 // 3 the first with k shared out over workgroups; -1 for sizes that none of these takes.  kind: 0 stored, 1 added, 2 added with a norm handed on, 3 gated,
-// 4 gated with a norm taken, 5 rotated into the pages, 6 through xielu.
+// 4 gated with a norm taken, 5 rotated into the pages, 6 through xielu, 7 stored in bfloat16.  With counters, and the scratch it asks for.
 GI_API int gi_gemm_bf16_large_kernel(int M, int N, int K, int kind) {
-    if (M <= SKINNY_MAX_ROWS || K % PK != 0 || N < 128 || kind < 0 || kind > 6) return -1;
+    if (!takes_large(M, N, K) || kind < 0 || kind > 7) return -1;
     if (gi_gemm_bf16_piped_splits(M, N, K) > 1) return 3;
-    return large_kernel_of_kind(M, N, K, kind);
+    return large_kernel_of_kind(M, N, K, kind, true).kernel;
 }
 
-// By how many workgroups each tile of the last round is made where the tiles of 256 x 128 make such a product with all the scratch it asks for (1: one).
+// The same where the tiles of 256 x 128 make such a product, of whatever kind, with counters.
 GI_API int gi_gemm_bf16_tall_shares(int M, int N, int K) {
-    return M <= SKINNY_MAX_ROWS || K % PK != 0 || N < 128 || gi_gemm_bf16_piped_splits(M, N, K) > 1 ? 1 : tall_cut(M, N, K, true).shares;
+    return !takes_large(M, N, K) || gi_gemm_bf16_piped_splits(M, N, K) > 1 ? 1 : tall_cut(M, N, K, true, false).shares;
 }
 
 // So many 32-bit counters, all 0, are what a product may be given as `counters`; it leaves them 0 again.  Without (null) it makes its own with a launch.  Products

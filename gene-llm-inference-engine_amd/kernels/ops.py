@@ -153,7 +153,7 @@ def lib():
         l.gi_gemm_exact_gated_takes.restype = c_int
         l.gi_gemm_exact_scratch_floats.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_exact_scratch_floats.restype = c_long
-        l.gi_gemm_bf16_scratch_floats.argtypes = [c_int, c_int, c_int]
+        l.gi_gemm_bf16_scratch_floats.argtypes = [c_int, c_int, c_int, c_int, c_int]
         l.gi_gemm_bf16_scratch_floats.restype = c_long
         l.gi_gemm_bf16_norm_parts.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_bf16_norm_parts.restype = c_int
@@ -161,6 +161,8 @@ def lib():
         l.gi_attention_prompt_share_floats.restype = c_long
         l.gi_gemm_bf16_tall_shares.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_bf16_tall_shares.restype = c_int
+        l.gi_gemm_bf16_shares.argtypes = [c_int, c_int, c_int, c_int, c_int]
+        l.gi_gemm_bf16_shares.restype = c_int
         l.gi_gemm_bf16_counters.argtypes = []
         l.gi_gemm_bf16_counters.restype = c_int
         l.gi_gemm_bf16_large_kernel.argtypes = [c_int, c_int, c_int, c_int]
@@ -1648,9 +1650,22 @@ def _exact_scratch_floats(m, n, k) -> int:
     return lib().gi_gemm_exact_scratch_floats(m, n, k)
 
 
+# What becomes of a product's sums, by the library's numbers.
+PRODUCT_KINDS = ("stored", "added", "added handing a norm on", "gated", "gated with a norm", "rotated", "xielu", "stored in bfloat16")
+
+
+def product_kind(out, accumulate=False, gated=False, norm_in=None, norm_out=None) -> int:
+    """The number of what `gemm_bf16` does with these arguments."""
+    if norm_out is not None:
+        return 2
+    if gated:
+        return 4 if norm_in is not None else 3
+    return 1 if accumulate else 7 if out.dtype == torch.bfloat16 else 0
+
+
 @lru_cache(maxsize=8192)
-def _scratch_floats(m, n, k) -> int:
-    return lib().gi_gemm_bf16_scratch_floats(m, n, k)
+def _scratch_floats(m, n, k, kind, counted) -> int:
+    return lib().gi_gemm_bf16_scratch_floats(m, n, k, kind, 1 if counted else 0)
 
 
 @lru_cache(maxsize=8192)
@@ -1659,10 +1674,15 @@ def gemm_bf16_tall_shares(m, n, k) -> int:
     return lib().gi_gemm_bf16_tall_shares(m, n, k)
 
 
-def step_counters(ctx, m, n, k):
-    """`counters` for a product of these sizes in the step `ctx`: the step's own, filled once and left as they were by every product (a step's products run one
-    after the other); None for a product that has no use for them."""
-    if ctx is None or gemm_bf16_tall_shares(m, n, k) == 1:
+@lru_cache(maxsize=8192)
+def _shares(m, n, k, kind, counted) -> int:
+    return lib().gi_gemm_bf16_shares(m, n, k, kind, 1 if counted else 0)
+
+
+def step_counters(ctx, m, n, k, kind=0):
+    """`counters` for a product of these sizes and kind (`product_kind`) in the step `ctx`: the step's own, filled once and left as they were by every product (a
+    step's products run one after the other); None for a product that has no use for them."""
+    if ctx is None or _shares(m, n, k, kind, True) == 1:
         return None
     counters = ctx.memo.get("product_counters")
     if counters is None:
@@ -1710,7 +1730,7 @@ def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=N
         raise KernelError(f"gemm: out is {tuple(out.shape)}, ({m}, {n // 2 if gated else n}) is needed")
     if not (checked or gemm_bf16_supports(a, w, out)):
         raise KernelError("gemm_bf16: operands must be bfloat16 with K and row strides multiples of 8, 16-byte aligned")
-    n_scratch = _scratch_floats(m, n, k)                             # partial sums where k is split over workgroups
+    n_scratch = _scratch_floats(m, n, k, product_kind(out, accumulate, gated, norm_in, norm_out), counters is not None)      # partial sums where k is split over workgroups
     scratch = torch.empty(n_scratch, dtype=torch.float32, device=a.device) if n_scratch else None
     if gated and gated is not True and gated not in ACTIVATIONS:
         raise KernelError(f"gemm: unknown activation {gated!r} of a gated product; known: {', '.join(ACTIVATIONS)}")
@@ -1754,7 +1774,7 @@ def gemm_bf16_onto_norm(a, w, x, g, eps, normed):
     if not (w.shape == (n, k) and x.shape == (m, n) and gemm_bf16_supports(a, w, x) and x.dtype == torch.float32 and gemm_bf16_onto_norm_takes(m, n, k)
             and g.dtype == torch.float32 and g.shape == (n,) and g.is_contiguous() and normed.dtype == torch.bfloat16 and normed.shape == (m, n) and normed.stride(1) == 1):
         raise KernelError("gemm_bf16_onto_norm: bfloat16 operands, float32 rows [m, n] and weights [n], bfloat16 [m, n] for the normed rows, and sizes that are taken")
-    n_scratch = _scratch_floats(m, n, k)
+    n_scratch = _scratch_floats(m, n, k, 1, False)
     scratch = torch.empty(n_scratch, dtype=torch.float32, device=a.device)
     if _profile is not None:
         _profile.note = (f"{n}x{k}", n * k * w.element_size())
@@ -1765,9 +1785,8 @@ def gemm_bf16_onto_norm(a, w, x, g, eps, normed):
 
 def gemm_bf16_large_kernel(m, n, k, kind):
     """Which kernel makes a product of more than 128 rows (None: none of these): "128x128", "256x128", "256x256" or "128x128 shared" (k shared out over
-    workgroups).  kind: "stored", "added", "added handing a norm on", "gated", "gated with a norm", "rotated" or "xielu"."""
-    kinds = ("stored", "added", "added handing a norm on", "gated", "gated with a norm", "rotated", "xielu")
-    which = lib().gi_gemm_bf16_large_kernel(m, n, k, kinds.index(kind))
+    workgroups).  kind: one of `PRODUCT_KINDS`; with counters (`step_counters`)."""
+    which = lib().gi_gemm_bf16_large_kernel(m, n, k, PRODUCT_KINDS.index(kind))
     return None if which < 0 else ("128x128", "256x128", "256x256", "128x128 shared")[which]
 
 
@@ -1834,7 +1853,7 @@ def gemm_bf16_qkv_rope_store(a, w, cos, sin, positions, slots, table, q_out, cac
     squares_in, eps = norm_in if norm_in is not None else (None, 0.0)
     if squares_in is not None and not (squares_in.dtype == torch.float32 and squares_in.is_contiguous() and squares_in.dim() == 2 and squares_in.shape[0] == m):
         raise KernelError("gemm: the pieces of the sums of squares must be float32 [m, pieces]")
-    n_scratch = _scratch_floats(m, n, k)
+    n_scratch = _scratch_floats(m, n, k, 5, counters is not None)
     scratch = torch.empty(n_scratch, dtype=torch.float32, device=a.device) if n_scratch else None
     if _profile is not None:
         _profile.note = (f"{n}x{k}", n * k * w.element_size())

@@ -54,7 +54,7 @@ def qkv_rotate_store_attend(h, w_qkv, ctx, cache, *, n_heads, n_kv_heads, head_d
         if ops.gemm_bf16_supports(rows, w_qkv, att):
             q_rot = torch.empty((T, a_dim), dtype=torch.bfloat16, device=ctx.device)
             ops.gemm_bf16_qkv_rope_store(rows, w_qkv, cos, sin, ctx.row_pos, ctx.row_slot, cache.table, q_rot, cache.kv, n_heads, n_kv_heads,
-                                         head_dim, norm_in, ops.step_counters(ctx, T, *w_qkv.shape))
+                                         head_dim, norm_in, ops.step_counters(ctx, T, *w_qkv.shape, ops.PRODUCT_KINDS.index("rotated")))
             return ops.attention(q_rot, cache.kv, att, ctx, cache.table, n_heads, n_kv_heads, head_dim, window)
         if norm_in is None:
             h = rows                  # (whole rows: what `linear` below would make of h)
@@ -71,7 +71,7 @@ def qkv_rotate_store_attend(h, w_qkv, ctx, cache, *, n_heads, n_kv_heads, head_d
         q, k, v = qkv[:, :a_dim], qkv[:, a_dim:a_dim + kv_dim], qkv[:, a_dim + kv_dim:]
     else:                       # the pages are another layer's: only the queries are made
         q, k, v = torch.empty((T, a_dim), dtype=torch.float32, device=ctx.device), None, None
-        linear(h, w_qkv[:a_dim], q)
+        linear(h, w_qkv[:a_dim], q, ctx=ctx)
     if before_rotation is not None:
         before_rotation(q, k)
     if position is not None and tables is None:          # an encoding with kernels of its own: q and k are turned in place
@@ -289,7 +289,7 @@ class Attention(Mixer):
             if att.dtype != self.att_dtype:
                 att = att.to(self.att_dtype)
             if overwrite:
-                linear(att, self.w_o, residual)
+                linear(att, self.w_o, residual, ctx=ctx)
                 return None
             return linear_onto(att, self.w_o, residual, then, ctx)
         if overwrite:

@@ -137,7 +137,7 @@ class GatedDelta(Mixer):
             low = proj[:, self.low[0]:self.low[1]]
             low = ops.concat_rows(low, None, torch.empty(low.shape, dtype=self.low_dtype, device=dev))
             up = torch.empty((T, self.w_low.shape[0]), dtype=torch.float32, device=dev)
-            linear(low, self.w_low, up)
+            linear(low, self.w_low, up, ctx=ctx)
             if "low_a" in o:
                 a = up[:, :self.n_decays]
             if "low_g" in o:
@@ -155,7 +155,7 @@ class GatedDelta(Mixer):
         mid = torch.empty((T, vv), dtype=self.mid_dtype, device=dev)
         ops.head_norm_gate(read, gate, self.out_norm, s.norm_eps, mid, H, dv, gate_activation=s.gate_activation, gate_up=gate_up)
         if overwrite:
-            linear(mid, self.w_o, residual)
+            linear(mid, self.w_o, residual, ctx=ctx)
             return None
         return linear_onto(mid, self.w_o, residual, then, ctx)
 

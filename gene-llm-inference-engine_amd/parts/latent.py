@@ -132,7 +132,7 @@ class LatentAttention(Mixer):
         down = projected
         if down is None:
             down = torch.empty((T, self.w_down.shape[0]), dtype=torch.float32, device=dev)
-            linear(h, self.w_down, down)
+            linear(h, self.w_down, down, ctx=ctx)
         cos, sin = (None, None) if self.position is None else self.position.half_split_tables(ctx) if self.half_split else self.position.pair_tables(ctx)
         plain = torch.empty((T, H * s.head_dim), dtype=self.plain_dtype, device=dev)
         folded = torch.empty((T, H * kd), dtype=cache.kv.dtype, device=dev)
@@ -144,7 +144,7 @@ class LatentAttention(Mixer):
             ops.latent_prepare(down, s.q_rank, s.kv_rank, s.rotary_dim, self.q_norm, self.kv_norm, s.norm_eps, cos, sin, ctx.row_pos, ctx.row_slot,
                                cache.table, cq, cache.kv, cache.page_size, self.half_split)
             q = torch.empty((T, H * (s.head_dim + s.rotary_dim)), dtype=torch.float32, device=dev)
-            linear(cq, self.w_uq, q)
+            linear(cq, self.w_uq, q, ctx=ctx)
             ops.latent_queries(q, cos, sin, plain, folded, H, s.head_dim, s.rotary_dim, s.kv_rank, self.half_split)
         heads_product(plain, self.w_uk_t, folded, H, kd)
         attended = torch.empty((T, H * s.kv_rank), dtype=cache.kv.dtype, device=dev)
@@ -160,7 +160,7 @@ class LatentAttention(Mixer):
         if self.gated:
             ops.head_gate(att, down[:, self.gate_at:self.gate_at + H], H, s.value_dim)
         if overwrite:
-            linear(att, self.w_o, residual)
+            linear(att, self.w_o, residual, ctx=ctx)
             return None
         return linear_onto(att, self.w_o, residual, then, ctx)
 

@@ -75,7 +75,7 @@ class Lightning(Mixer):
         mid = torch.empty((T, vv), dtype=self.mid_dtype, device=ctx.device)
         ops.row_norm_gate(out, proj[:, self.g_at:self.g_at + vv], self.out_norm, s.norm_eps, mid)
         if overwrite:
-            linear(mid, self.w_o, residual)
+            linear(mid, self.w_o, residual, ctx=ctx)
             return None
         return linear_onto(mid, self.w_o, residual, then, ctx)
 

@@ -25,12 +25,14 @@ def linear(a, weight: torch.Tensor, out: torch.Tensor, accumulate: bool = False,
     if isinstance(a, HandedRows):
         if (weight.dtype == torch.bfloat16 and ops.gemm_bf16_supports(a.scaled, weight, out)
                 and ops.gemm_bf16_takes_norm(a.scaled.shape[0], weight.shape[0], weight.shape[1], gated)):
-            return ops.gemm_bf16(a.scaled, weight, out, accumulate, gated, checked=True, norm_in=(a.squares, a.eps), gate_limit=gate_limit,
-                                 counters=ops.step_counters(ctx, a.scaled.shape[0], *weight.shape))
+            norm_in = (a.squares, a.eps)
+            return ops.gemm_bf16(a.scaled, weight, out, accumulate, gated, checked=True, norm_in=norm_in, gate_limit=gate_limit,
+                                 counters=ops.step_counters(ctx, a.scaled.shape[0], *weight.shape, ops.product_kind(out, accumulate, gated, norm_in)))
     if isinstance(a, NormedRows):
         a = a.materialize()
     if a.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and ops.gemm_bf16_supports(a, weight, out):
-        return ops.gemm_bf16(a, weight, out, accumulate, gated, checked=True, gate_limit=gate_limit, counters=ops.step_counters(ctx, a.shape[0], *weight.shape))
+        return ops.gemm_bf16(a, weight, out, accumulate, gated, checked=True, gate_limit=gate_limit,
+                             counters=ops.step_counters(ctx, a.shape[0], *weight.shape, ops.product_kind(out, accumulate, gated)))
     if gated:
         raise ops.KernelError("the gated product exists for bfloat16 operands only")
     return ops.gemm_exact(a, weight, out, accumulate)
@@ -75,8 +77,9 @@ def linear_onto(a: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor, t
         if parts:
             scaled = torch.empty((rows, width), dtype=torch.bfloat16, device=residual.device)
             squares = torch.empty((rows, parts), dtype=torch.float32, device=residual.device)
-            ops.gemm_bf16(a, weight, residual, accumulate=True, checked=True, norm_out=(then.handed_weight(), scaled, squares),
-                          counters=ops.step_counters(ctx, rows, *weight.shape))
+            norm_out = (then.handed_weight(), scaled, squares)
+            ops.gemm_bf16(a, weight, residual, accumulate=True, checked=True, norm_out=norm_out,
+                          counters=ops.step_counters(ctx, rows, *weight.shape, ops.product_kind(residual, True, norm_out=norm_out)))
             return HandedRows(then, residual, scaled, squares)
     linear(a, weight, residual, accumulate=True, ctx=ctx)
     return None

@@ -57,7 +57,7 @@ class SwiGlu(FeedForward):
                 linear(h, self.w_gate_up, gate_up)
                 ops.act_mul(gate_up, mid, self.activation, self.limit)
         if overwrite:
-            linear(mid, self.w_down, residual)
+            linear(mid, self.w_down, residual, ctx=ctx)
             return None
         return linear_onto(mid, self.w_down, residual, then, ctx)
 
@@ -113,11 +113,11 @@ class DenseMlp(FeedForward):
             up = projected
             if up is None:
                 up = torch.empty((T, inter), dtype=torch.float32, device=ctx.device)
-                linear(h, self.w_up, up)
+                linear(h, self.w_up, up, ctx=ctx)
             mid = torch.empty((T, inter), dtype=self.mid_dtype, device=ctx.device)
             ops.xielu(up, mid, self.params)
         if overwrite:
-            linear(mid, self.w_down, residual)
+            linear(mid, self.w_down, residual, ctx=ctx)
             return None
         return linear_onto(mid, self.w_down, residual, then, ctx)
 

@@ -58,7 +58,7 @@ class Mlstm(Mixer):
         s, T, o = self.spec, ctx.n_rows, self.offsets
         vv = s.n_heads * s.value_dim
         proj = torch.empty((T, self.w_in.shape[0]), dtype=torch.float32, device=ctx.device)
-        linear(h, self.w_in, proj)
+        linear(h, self.w_in, proj, ctx=ctx)
         seg_start, seg_len = ops.segments(ctx)
         sums = torch.empty((T, vv), dtype=torch.float32, device=ctx.device)          # the heads' S^T q, and what to divide them by
         divisors = torch.empty((T, s.n_heads), dtype=torch.float32, device=ctx.device)
@@ -67,9 +67,9 @@ class Mlstm(Mixer):
         mid = torch.empty((T, vv), dtype=self.mid_dtype, device=ctx.device)
         ops.head_norm_gate(sums, proj[:, o["g"]:o["g"] + vv], self.out_norm, s.norm_eps, mid, s.n_heads, s.value_dim, den=divisors)
         if overwrite:
-            linear(mid, self.w_o, residual)
+            linear(mid, self.w_o, residual, ctx=ctx)
         else:
-            linear_onto(mid, self.w_o, residual)
+            linear_onto(mid, self.w_o, residual, ctx=ctx)
 
 
 register_mixer("mlstm", Mlstm)

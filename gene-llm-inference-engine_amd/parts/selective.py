@@ -84,7 +84,7 @@ class SelectiveScan(Mixer):
         proj = projected
         if proj is None:
             proj = torch.empty((T, self.w_in.shape[0]), dtype=torch.float32, device=dev)
-            linear(h, self.w_in, proj)
+            linear(h, self.w_in, proj, ctx=ctx)
         pre, z = proj[:, :inner], proj[:, inner:2 * inner]
         seg_start, seg_len = ops.segments(ctx)
         x = torch.empty((T, inner), dtype=torch.float32, device=dev)
@@ -94,20 +94,20 @@ class SelectiveScan(Mixer):
         if not single_rows:
             ops.ssm_tail(pre, s.conv_taps, seg_start, seg_len, ctx.row_slot, cache.state, inner, N)
         low = torch.empty((T, self.w_x.shape[0]), dtype=torch.float32, device=dev)
-        linear(x_low, self.w_x, low)
+        linear(x_low, self.w_x, low, ctx=ctx)
         mid = torch.empty((T, inner), dtype=self.mid_dtype, device=dev)
         dt_pre = dt_proj = None
         if single_rows and self.mid_dtype == torch.bfloat16 and self.w_dt.dtype == torch.bfloat16:
             dt_proj = (self.w_dt, 0)                    # (a step of single rows: the scan's kernel makes the step sizes' product on its way)
         else:
             dt_pre = torch.empty((T, inner), dtype=torch.float32, device=dev)
-            linear(low[:, :R], self.w_dt, dt_pre)       # (32-bit rows: the step sizes' product keeps them)
+            linear(low[:, :R], self.w_dt, dt_pre, ctx=ctx)       # (32-bit rows: the step sizes' product keeps them)
         ops.ssm_scan(x, dt_pre, self.dt_bias, low, R, R + N, z, self.a_log, self.d_skip, seg_start, seg_len, ctx.row_slot, cache.state, mid, N,
                      rows_per_request=ctx.seg_len, out_scale=self.out_scale, dt_proj=dt_proj)
         if overwrite:
-            linear(mid, self.w_o, residual)
+            linear(mid, self.w_o, residual, ctx=ctx)
             return None
-        return linear_onto(mid, self.w_o, residual, then)
+        return linear_onto(mid, self.w_o, residual, then, ctx)
 
 
 register_mixer("selective_scan", SelectiveScan)

@@ -84,7 +84,7 @@ class SideBySide(Mixer):
         told = [{} for _ in self.members]
         if self.w_first is not None:
             both = torch.empty((ctx.n_rows, self.w_first.shape[0]), dtype=torch.float32, device=residual.device)
-            linear(rows, self.w_first, both)
+            linear(rows, self.w_first, both, ctx=ctx)
             for own, (lo, hi) in zip(told, self._cuts):
                 own["projected"] = both[:, lo:hi]
         if self.weigh_inside:

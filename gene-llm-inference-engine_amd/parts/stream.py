@@ -67,15 +67,15 @@ class TokenSideInput(StreamPart):
             rows = handed.materialize() if handed is not None and handed.norm is self.rows else x
             ops.gate_token_columns_rows(rows if ops.gate_token_columns_rows_takes(rows, self.w_gate) else x, self.w_gate, self.table, s.first_column, ctx.tokens, g, s.activation)
             y = torch.empty((T, s.hidden_size), dtype=torch.float32, device=dev)
-            linear(g, self.w_out, y)
+            linear(g, self.w_out, y, ctx=ctx)
             return self._join(y, x, ctx, next_reader)
         rows = handed.materialize() if handed is not None and handed.norm is self.rows else self.rows(x, self.in_dtype)
         u = torch.empty((T, s.dim), dtype=torch.float32, device=dev)
-        linear(rows, self.w_gate, u)
+        linear(rows, self.w_gate, u, ctx=ctx)
         g = torch.empty((T, s.dim), dtype=self.mid_dtype, device=dev)
         ops.gate_token_columns(u, self.table, s.first_column, ctx.tokens, g, s.activation)
         y = torch.empty((T, s.hidden_size), dtype=torch.float32, device=dev)
-        linear(g, self.w_out, y)
+        linear(g, self.w_out, y, ctx=ctx)
         return self._join(y, x, ctx, next_reader)
 
 
@@ -104,7 +104,7 @@ class Rejoin(StreamPart):
     def forward(self, x, ctx):
         T, d = x.shape
         both = ops.concat_rows(x, ctx.memo["token_rows"], torch.empty((T, 2 * d), dtype=self.in_dtype, device=ctx.device))
-        linear(both, self.weight, x)                   # (x is free to be overwritten: `both` holds what the product reads)
+        linear(both, self.weight, x, ctx=ctx)                   # (x is free to be overwritten: `both` holds what the product reads)
         if self.offset is not None:
             ops.add_vector(x, self.offset)
 

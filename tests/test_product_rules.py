@@ -24,6 +24,41 @@ def test_the_faster_kernel_is_chosen(m, n, k, kind, kernel):
     assert ops.gemm_bf16_large_kernel(m, n, k, kind) == kernel
 
 
+# m, n, k, what becomes of the sums, the kernel that was the faster one, by how many workgroups it makes its last tiles, and without counters
+SHARED_OR_NOT = [
+    (4096, 3072, 8192, "added", "256x256", 1, 1), (4096, 3072, 8192, "stored in bfloat16", "256x256", 1, 1), (1368, 8192, 6784, "stored in bfloat16", "256x256", 1, 1),
+    (573, 16384, 6464, "added", "256x256", 1, 1), (709, 16384, 10176, "gated", "256x256", 1, 1), (1161, 8192, 2048, "added", "256x128", 1, 1), (588, 14336, 2048, "added", "256x128", 1, 1),
+    (273, 8192, 3072, "added handing a norm on", "128x128", 1, 1), (489, 6144, 3072, "added handing a norm on", "128x128", 1, 1), (793, 2048, 2496, "stored in bfloat16", "128x128", 1, 1),
+    (740, 4096, 4096, "added handing a norm on", "256x128", 2, 1), (206, 10240, 2624, "stored in bfloat16", "128x128", 1, 1), (496, 6144, 3136, "rotated", "128x128", 1, 1),
+    (318, 512, 4416, "added handing a norm on", "256x128", 4, 4), (437, 8192, 7168, "added handing a norm on", "256x128", 2, 2),
+    (2048, 2048, 8192, "added", "256x128", 2, 2), (1777, 2048, 8192, "added handing a norm on", "256x128", 2, 2), (2048, 5120, 3072, "rotated", "256x128", 4, 4),
+    (3000, 3072, 8192, "stored", "256x128", 4, 4), (2600, 4064, 4160, "gated", "256x128", 2, 2), (2048, 2048, 2048, "added", "128x128", 1, 1), (2048, 3072, 2048, "xielu", "256x128", 1, 1),
+]
+
+
+@pytest.mark.parametrize("m,n,k,kind,kernel,shares,without", SHARED_OR_NOT)
+def test_tiles_are_shared_out_where_that_is_faster(m, n, k, kind, kernel, shares, without):
+    number = ops.PRODUCT_KINDS.index(kind)
+    assert ops.gemm_bf16_large_kernel(m, n, k, kind) == kernel
+    assert (ops._shares(m, n, k, number, True), ops._shares(m, n, k, number, False)) == (shares, without)
+
+
+def test_only_a_product_whose_tiles_are_shared_out_asks_for_their_scratch():
+    """Counters, and 128 KB a share: at most one for every compute unit, so 33.6 MB."""
+    asked = 0
+    for m in (129, 300, 777, 1000, 1500, 2048, 3000, 4096, 8192):
+        for n in (512, 2048, 3072, 5120, 8192, 16384):
+            for k in (512, 2048, 3136, 8192):
+                for number in range(len(ops.PRODUCT_KINDS)):
+                    if ops.gemm_bf16_large_kernel(m, n, k, ops.PRODUCT_KINDS[number]) == "128x128 shared":
+                        continue
+                    for counted in (True, False):
+                        floats, shares = ops._scratch_floats(m, n, k, number, counted), ops._shares(m, n, k, number, counted)
+                        assert floats == 0 if shares == 1 else 2 * 32768 <= floats <= 256 * 32768 + 512
+                        asked += shares > 1
+    assert asked > 100
+
+
 @pytest.mark.parametrize("rows,seen,spans", [(1, 256, 0), (1, 257, 3), (3, 4096, 17), (1, 65534 * 256, 65535), (1, 65534 * 256 + 1, 0), (1, 1 << 30, 0)])
 def test_a_context_is_shared_out_over_so_many_spans_as_a_grid_takes(rows, seen, spans):
     """One head of 16 channels, whose parts are small: longer contexts stay whole (0), they are not refused."""
