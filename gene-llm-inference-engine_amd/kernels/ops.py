@@ -284,6 +284,14 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 _raw_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
+def _room(floats, device):
+    """Scratch for a way that another does without: float32 [floats], or None where the device has no room for it (the caller then takes the other way)."""
+    try:
+        return torch.empty(floats, dtype=torch.float32, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def _stream():
     if _raw_stream is not None and _raw_device is not None:
         return _raw_stream(_raw_device())
@@ -1133,7 +1141,8 @@ def delta_chunks_pay(rows_per_request, least, n_heads) -> bool:
 
 def delta_chunks(qkv, gates, seg_start, seg_len, rows_per_request, least, row_slot, state, out, n_heads, n_kv, dk, dv):
     """`delta_scan` for the requests of at least `least` rows, 64 rows at a time on the 32-bit matrix instructions (csrc/recurrent.hip states it; sums in
-    another order than the scan's, no further from 64 bits).  rows_per_request: the numbers in seg_len, on the host."""
+    another order than the scan's, no further from 64 bits).  rows_per_request: the numbers in seg_len, on the host.  None, and nothing done, where there is no
+    room for what the blocks hand on (98 KB a block and head at heads of 64 x 128)."""
     _dev(qkv, gates, seg_start, seg_len, row_slot, state, out)
     n, n_segs = qkv.shape[0], seg_start.numel()
     if not (qkv.dtype == torch.float32 and qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.shape[1] >= 2 * n_kv * dk + n_heads * dv and gates.dtype == torch.float32
@@ -1151,7 +1160,9 @@ def delta_chunks(qkv, gates, seg_start, seg_len, rows_per_request, least, row_sl
     blocks = sum(-(-m // DELTA_CHUNK) for m in rows_per_request if m >= least)
     if blocks == 0:
         return out
-    scratch = torch.empty(lib().gi_delta_chunk_floats(blocks, n_heads, dv), dtype=torch.float32, device=out.device)
+    scratch = _room(lib().gi_delta_chunk_floats(blocks, n_heads, dv), out.device)
+    if scratch is None:
+        return None
     _call("gi_delta_chunks", qkv.data_ptr(), qkv.stride(0), gates.data_ptr(), seg_start.data_ptr(), seg_len.data_ptr(), n_segs, int(least), blocks, row_slot.data_ptr(),
           state.data_ptr(), state.stride(0), scratch.data_ptr(), out.data_ptr(), out.stride(0), n_heads, n_kv, dv, _stream())
     return out
@@ -1525,13 +1536,15 @@ def attention_bf16(q, cache, out, plan: AttentionPlan, positions, slots, table, 
         if n_splits == 1 and memo is not None and contexts is not None and hd in (64, 128) and plan.n_tiles * n_heads <= PROMPT_SHARE_COUNTERS // 2:
             most, keys = prompt_attention_shares([min(c, seen(c, plan.tile)) for c in contexts], n_heads, hd, plan.tile, one_round)
             n_part = lib().gi_attention_prompt_share_floats(plan.n_tiles, plan.tile, n_heads, hd, 1, 1 if plan.paired else 0, most)
-            if n_part:
+            part = _room(n_part, out.device) if n_part else None
+            if part is not None:
                 counters = memo.get("attention_counters")
                 if counters is None:
                     counters = memo["attention_counters"] = torch.zeros(PROMPT_SHARE_COUNTERS, dtype=torch.int32, device=out.device)
             else:
-                most, keys = 1, 0
-        part = torch.empty(n_part, dtype=torch.float32, device=out.device) if n_part else None
+                most, keys, n_part = 1, 0, 0
+        else:
+            part = torch.empty(n_part, dtype=torch.float32, device=out.device) if n_part else None
         _call("gi_attention_prompt_bf16", q.data_ptr(), cache.data_ptr(), out.data_ptr(), plan.tiles.data_ptr(), plan.n_tiles, plan.tile,
               1 if plan.paired else 0, table.data_ptr(), table.stride(0), cache.stride(0), page_size, n_heads, n_kv, hd, window, scale, n_splits,
               _ptr(plan.tile_first), _ptr(plan.tile_rows), plan.n_tile_rows, _ptr(part), n_part, *extras, keys, most, _ptr(counters), _stream())
@@ -1679,6 +1692,18 @@ def _shares(m, n, k, kind, counted) -> int:
     return lib().gi_gemm_bf16_shares(m, n, k, kind, 1 if counted else 0)
 
 
+def _product_scratch(m, n, k, kind, counted, device):
+    """(scratch, its floats) of a product: partial sums where k is shared out over workgroups.  Without the room for shared tiles' sums the product's other
+    kernels make it."""
+    floats = _scratch_floats(m, n, k, kind, counted)
+    if not floats:
+        return None, 0
+    if _shares(m, n, k, kind, counted) > 1:
+        scratch = _room(floats, device)
+        return scratch, floats if scratch is not None else 0
+    return torch.empty(floats, dtype=torch.float32, device=device), floats
+
+
 def step_counters(ctx, m, n, k, kind=0):
     """`counters` for a product of these sizes and kind (`product_kind`) in the step `ctx`: the step's own, filled once and left as they were by every product (a
     step's products run one after the other); None for a product that has no use for them."""
@@ -1730,8 +1755,7 @@ def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=N
         raise KernelError(f"gemm: out is {tuple(out.shape)}, ({m}, {n // 2 if gated else n}) is needed")
     if not (checked or gemm_bf16_supports(a, w, out)):
         raise KernelError("gemm_bf16: operands must be bfloat16 with K and row strides multiples of 8, 16-byte aligned")
-    n_scratch = _scratch_floats(m, n, k, product_kind(out, accumulate, gated, norm_in, norm_out), counters is not None)      # partial sums where k is split over workgroups
-    scratch = torch.empty(n_scratch, dtype=torch.float32, device=a.device) if n_scratch else None
+    scratch, n_scratch = _product_scratch(m, n, k, product_kind(out, accumulate, gated, norm_in, norm_out), counters is not None, a.device)
     if gated and gated is not True and gated not in ACTIVATIONS:
         raise KernelError(f"gemm: unknown activation {gated!r} of a gated product; known: {', '.join(ACTIVATIONS)}")
     gate_code = 0 if not gated else 1 + (0 if gated is True else ACTIVATIONS[gated])        # 1: SiLU, 2: GELU (tanh form)
@@ -1853,8 +1877,7 @@ def gemm_bf16_qkv_rope_store(a, w, cos, sin, positions, slots, table, q_out, cac
     squares_in, eps = norm_in if norm_in is not None else (None, 0.0)
     if squares_in is not None and not (squares_in.dtype == torch.float32 and squares_in.is_contiguous() and squares_in.dim() == 2 and squares_in.shape[0] == m):
         raise KernelError("gemm: the pieces of the sums of squares must be float32 [m, pieces]")
-    n_scratch = _scratch_floats(m, n, k, 5, counters is not None)
-    scratch = torch.empty(n_scratch, dtype=torch.float32, device=a.device) if n_scratch else None
+    scratch, n_scratch = _product_scratch(m, n, k, 5, counters is not None, a.device)
     if _profile is not None:
         _profile.note = (f"{n}x{k}", n * k * w.element_size())
     _call("gi_gemm_bf16_qkv_rope_store", a.data_ptr(), w.data_ptr(), m, n, k, a.stride(0), w.stride(0), _ptr(scratch), n_scratch,

@@ -148,8 +148,8 @@ class GatedDelta(Mixer):
             ops.delta_tail(proj, o["conv"], s.conv_taps, seg_start, seg_len, ctx.row_slot, cache.state, H, G, dk, dv)
         read = torch.empty((T, vv), dtype=torch.float32, device=dev)
         chunked = self.in_blocks and ops.delta_chunks_pay(ctx.seg_len, self.ROWS_IN_BLOCKS, H)
-        if chunked:
-            ops.delta_chunks(qkv, gates, seg_start, seg_len, ctx.seg_len, self.ROWS_IN_BLOCKS, ctx.row_slot, cache.state, read, H, G, dk, dv)
+        if chunked:                # (not where there is no room for it)
+            chunked = ops.delta_chunks(qkv, gates, seg_start, seg_len, ctx.seg_len, self.ROWS_IN_BLOCKS, ctx.row_slot, cache.state, read, H, G, dk, dv) is not None
         if not chunked or min(ctx.seg_len) < self.ROWS_IN_BLOCKS:
             ops.delta_scan(qkv, gates, seg_start, seg_len, ctx.row_slot, cache.state, read, H, G, dk, dv, s.channel_decay, single_rows, self.ROWS_IN_BLOCKS if chunked else 0)
         mid = torch.empty((T, vv), dtype=self.mid_dtype, device=dev)

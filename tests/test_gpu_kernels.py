@@ -939,6 +939,32 @@ def test_workgroups_that_meet_in_a_kernel_under_capture():
         o.gemm_bf16(a, w, torch.empty_like(out))
 
 
+@pytest.mark.parametrize("hd, m", [(128, 1000), (64, 1500)])
+def test_without_room_for_scratch_nothing_is_shared_out(hd, m, monkeypatch):
+    """A device that has no room for the sums of shared tiles and walks: the kernels that share nothing out serve, as without a step's memory of its own."""
+    o = ops()
+    n_heads, n_kv, rows, n, k = 32, 8, 2048, 2048, 8192
+    cache, table, _ = build_paged([m], n_kv, hd, 16, torch.bfloat16, seed=5)
+    plan = o.AttentionPlan([0], [m], [0], [1], DEV)
+    pos, slots = torch.arange(m, dtype=torch.int32, device=DEV), torch.ones(m, dtype=torch.int32, device=DEV)
+    q, a, w = randn(m, n_heads * hd, dtype=torch.bfloat16, seed=3), randn(rows, k, dtype=torch.bfloat16, seed=4), randn(n, k, dtype=torch.bfloat16, seed=6)
+
+    def attend(memo):
+        return o.attention_bf16(q, cache, torch.empty_like(q), plan, pos, slots, table, n_heads, n_kv, hd, memo=memo)
+
+    alone, memo = attend(None), {}
+    shared, product = attend(memo), o.gemm_bf16(a, w, torch.empty(rows, n, device=DEV))
+    assert "attention_counters" in memo and o._shares(rows, n, k, 0, False) == 2
+    asked = []
+    monkeypatch.setattr(o, "_room", lambda floats, device: asked.append(4 * floats))
+    memo = {}
+    assert torch.equal(attend(memo), alone) and not torch.equal(shared, alone) and "attention_counters" not in memo
+    whole = o.gemm_bf16(a, w, torch.empty(rows, n, device=DEV))
+    assert rel(whole, a.double() @ w.double().T) < 1e-5 and not torch.equal(whole, product)
+    # 68 KB (heads of 128 channels; 36) for every share of every tile and head, 128 KB for every share of a product's tile
+    assert asked == [plan.n_tiles * n_heads * {128: 2 * 69632, 64: 3 * 36864}[hd], 4 * (512 + 128 * 2 * 32768)]
+
+
 def test_a_meeting_of_workgroups_ends_whatever_its_counters_held():
     """Counters that were not 0 (a workgroup has been counted that never comes): the launch ends, the results that are not whole are no numbers, all others are right,
     and the counters are 0 again."""

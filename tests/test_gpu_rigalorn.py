@@ -377,6 +377,29 @@ def test_delta_rule_in_blocks_with_no_numbers(what, value):
         assert relative_error(ours[keep].double(), scans[keep].double()) < 2e-6
 
 
+def test_a_prompt_without_room_for_the_blocks_goes_token_by_token(tmp_path, monkeypatch):
+    """A device that has no room for what the blocks of a long prompt hand on: the scan's logits and memories, which need none."""
+    from geneinfer_amd.engine import Runner, StepEntry, load_model
+    from geneinfer_amd.kernels import ops
+    layer = dict(type="delta", mlp=dict(kind="dense", ff=128), mixer=dict(heads=2, kv_heads=1, dim=64, vdim=64, conv=4))
+    cfg = dict(architecture="Rigalorn", vocab=97, width=64, embedding=dict(scale=8.0), norm=dict(eps=1e-5), max_positions=1024, layers=[layer])
+    write_model(tmp_path, cfg, seed=5)
+    model, tokens = load_model(tmp_path, "bfloat16", DEV), _prompt(cfg, 400, 6)
+    assert ops.delta_chunks_pay([400], 65, 2)
+    got = {}
+    for what in ("blocks", "no room", "scan"):
+        with monkeypatch.context() as patch:
+            if what == "no room":
+                patch.setattr(ops, "_room", lambda floats, device: None)
+            if what == "scan":
+                patch.setattr(ops, "delta_chunks_pay", lambda *a: False)
+            runner = Runner(model, page_size=16, max_tokens=1024, max_requests=2)
+            runner.open("r")
+            got[what] = [runner.step([StepEntry("r", tokens[:399], tuple(range(399)))]).cpu().clone(), runner.step([StepEntry("r", tokens[399:], (0,))]).cpu().clone()]
+    assert all(torch.equal(x, y) for x, y in zip(got["no room"], got["scan"])) and not torch.equal(got["blocks"][0], got["scan"][0])
+    assert relative_error(got["blocks"][0], got["scan"][0].double()) < 1e-2
+
+
 def test_delta_rule_takes_very_wide_values():
     """More tiles of four value channels than half of what a launch's third dimension holds."""
     from geneinfer_amd.kernels import ops

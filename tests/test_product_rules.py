@@ -1,6 +1,7 @@
 """The library's own rules at sizes on both sides of their lines, on 256 compute units (which it assumes where there is no GPU): which kernel
 makes a product of a prompt's rows, and which contexts the 32-bit attention shares out."""
 import pytest
+import torch
 
 from geneinfer_amd.kernels import ops
 
@@ -63,3 +64,12 @@ def test_only_a_product_whose_tiles_are_shared_out_asks_for_their_scratch():
 def test_a_context_is_shared_out_over_so_many_spans_as_a_grid_takes(rows, seen, spans):
     """One head of 16 channels, whose parts are small: longer contexts stay whole (0), they are not refused."""
     assert ops.lib().gi_attention_exact_spans(rows, rows, 1, 1, 16, 16, 16, seen) == spans
+
+
+def test_no_room_for_scratch_is_no_error(monkeypatch):
+    def full(*args, **kw):
+        raise torch.OutOfMemoryError("full")
+
+    assert ops._room(5, "cpu").shape == (5,)
+    monkeypatch.setattr(torch, "empty", full)
+    assert ops._room(5, "cpu") is None
