@@ -1258,6 +1258,7 @@ class AttentionPlan:
         plan.n_decode, plan.n_tiles, plan.max_decode_context, plan.single_rows = n_rows, 0, max_context, True
         plan.decode_rows = None                                  # rows 0 .. n_rows-1
         plan.decode_positions = plan.tile_contexts = None
+        plan.tile_places, plan.walk_shares = [], {}
         plan.tiles = torch.empty(0, dtype=torch.int32, device=device)
         plan.n_tile_rows, plan.max_tile_context, plan.tile_first, plan.tile_rows, plan.paired, plan.tile = 0, 0, None, None, False, 128
         return plan
@@ -1275,7 +1276,7 @@ class AttentionPlan:
                 self.max_decode_context = max(self.max_decode_context, pos0 + n)
                 self.decode_positions += n * pos0 + n * (n + 1) // 2
             else:
-                portions.append([(start + off, min(self.tile, n - off), pos0 + off, slot) for off in range(0, n, self.tile)])
+                portions.append([(start + off, min(self.tile, n - off), pos0 + off, slot, max(0, n - off - self.tile)) for off in range(0, n, self.tile)])
         # Tile i of a portion sees the keys of the tiles before it: the last tile goes with the first, the last but
         # one with the second, ... so that every pair has about the same number of keys to visit and reads them once
         # for both (a tile of no rows fills the middle pair of an odd number).  Without a portion of two tiles, no pairs.
@@ -1286,10 +1287,12 @@ class AttentionPlan:
                 continue
             for i in range((len(p) + 1) // 2):
                 late, early = p[len(p) - 1 - i], p[i]
-                tiles.extend((late, early if early is not late else (late[0], 0, late[2], late[3])))
+                tiles.extend((late, early if early is not late else (late[0], 0, *late[2:])))
         self.n_decode, self.n_tiles = len(dec), len(tiles)
         self.n_tile_rows = sum(t[1] for t in tiles)
         self.tile_contexts = [t[2] + t[1] for t in tiles if t[1]]        # positions each tile of rows sees; None: of a step still to come
+        self.tile_places = [(t[2], t[1], t[4]) for t in tiles]           # every tile's first position, its rows, the rows behind it in its portion
+        self.walk_shares = {}                                            # what `_walk_shares` found for the step's layers
         self.max_tile_context = max(self.tile_contexts, default=0)
         # for sharing a tile's keys out over workgroups: rows before each tile, and the tiles' rows in order
         firsts, count = [], 0
@@ -1300,7 +1303,7 @@ class AttentionPlan:
         self.decode_rows = self.tile_first = self.tile_rows = None      # no prompt rows: the decode rows are all rows, in order
         self.tiles = torch.empty(0, dtype=torch.int32, device=device)
         if tiles:                            # (every piece starts at a multiple of 16 bytes: the kernel reads a tile's four numbers at once)
-            self.tiles, self.tile_first, self.tile_rows, *rest = put([v for t in tiles for v in t], firsts, [r for t in tiles for r in range(t[0], t[0] + t[1])],
+            self.tiles, self.tile_first, self.tile_rows, *rest = put([v for t in tiles for v in t[:4]], firsts, [r for t in tiles for r in range(t[0], t[0] + t[1])],
                                                                      *([dec] if dec else []))
             self.decode_rows = rest[0] if rest else None
 
@@ -1325,28 +1328,61 @@ def prompt_attention_splits(n_groups, n_heads, span, target_groups=512):
 PROMPT_SHARE_COUNTERS = 4096
 
 
-def prompt_attention_shares(contexts, n_heads, hd, tile=128, one_round=False):
+def prompt_attention_shares(contexts, n_heads, hd, tile=128, one_round=False, pairs=None):
     """(shares, keys) for the tiles of a step that fill the chip: a tile's keys are shared out over up to so many workgroups of so many keys each, (1, 0) where
     none should be.  The chip holds two workgroups a compute unit (three at heads of 64 channels); a tile that sees far more keys than there are for each of
     those places keeps one busy when the others have ended.  Measured, one workgroup a tile and shared: 24 heads of 128 over 1,350 rows behind 1,000 and 674 more
     87.6 -> 71 us (77 in two shares, 79 in four), 2,000 rows 74.6 -> 52 (57 in three), 32 heads over 1,000 rows 40 -> 31, over 1,500 58 -> 41, but over 2,048
     62.5 -> 71.6 and over 800 the same; 32 heads of 64 over 2,560 rows 52.4 -> 49.8, over 3,500 99.5 -> 82, over 900 behind 1,000 and 1,100 more 52 -> 40 (44 in
-    three).  The lines there: the longest walk 2.1 (64 channels: 1.5) times a place's even share and 16 tiles of 64 keys, and every share from the third on
-    leaves each 12 (16) of them.
+    three).  The lines there: the longest walk 2.1 (64 channels: 1.5) times a place's even share and 16 tiles of 64 keys (under 20 tiles 2.5 and 1.6 times:
+    24 heads over two prompts of 1,024 rows, 2.37 times, 37 us and 43 shared), and every share from the third on leaves each 12 (16) of them.
     one_round: heads of 64 channels whose pairs of tiles are at most one for a compute unit.  Their kernel walks a pair's keys with one workgroup of 16 waves; a
     workgroup a tile and up to three shares of 512 keys or more take 39.6 us for 40.8 (32 heads over 2,048 rows), 29.3 for 34 (1,500), 18.5 for 23 (1,024),
     17.1 for 20.4 (800), 36.5 for 47 (600 behind 2,000).  Tiles of 64 rows (steps of up to 768) only where a walk has 20 tiles of keys: 300 rows behind 1,000
-    and 200 more 24 for 27.4, but 760 rows from the beginning 19.7 for 18.2."""
+    and 200 more 24 for 27.4, but 760 rows from the beginning 19.7 for 18.2.  pairs: the tiles of keys that each pair sees, where they are known.  Fitted to 320 steps
+    of one to six portions, with windows and without: the pairs take 4.2 us, 1.12 for each tile of keys of the busiest and 4.6 for each pair a compute unit, the shares
+    2.6, 1 for each of a place's even share, 1.32 for each of a share's and 3.2 for each workgroup a unit; where that promises 5 % one of them is slower shared, by
+    5 % (16 were, by up to a half: two prompts of 1,000 rows 28 and 31 us, 2,048 rows under a window of 1,024 36.7 and 39.3).  Tiles of 64 rows have four
+    workgroups a unit at once: 479 rows of 64 heads behind 839 positions, 1,408 workgroups, took 42 us for 28; up to 1,024 all were faster shared."""
     walks = [-(-c // 64) for c in contexts]
-    wide = hd == 128
+    wide, longest, units = hd == 128, max(walks), lib().gi_compute_units()
+    even = sum(walks) * n_heads / (units * (2 if wide else 3))
     if hd == 64 and one_round:
-        longest = max(walks)
-        return (3, 64 * max(8, -(-longest // 3))) if longest >= (20 if tile == 64 else 9) else (1, 0)
-    longest, even = max(walks), sum(walks) * n_heads / (lib().gi_compute_units() * (2 if wide else 3))
-    if longest < 16 or longest < (2.1 if wide else 1.5) * even:
+        keys = max(8, -(-longest // 3))
+        if longest < (20 if tile == 64 else 9):
+            return (1, 0)
+        if pairs is not None:
+            workgroups = sum(min(3, -(-w // keys)) for w in walks) * n_heads / units
+            if workgroups > 4 if tile == 64 else 4.2 + 1.12 * max(pairs) + 4.6 * len(pairs) * n_heads / units < 1.05 * (2.6 + even + 1.32 * keys + 3.2 * workgroups):
+                return (1, 0)
+        return (3, 64 * keys)
+    if longest < 16 or longest < ((2.1 if wide else 1.5) if longest >= 20 else 2.5 if wide else 1.6) * even:
         return (1, 0)
     most = max(2, min(4, longest // (12 if wide else 16)))
     return (most, 64 * -(-longest // most))
+
+
+def _walk_shares(plan, n_heads, hd, window, chunk, one_round):
+    """`prompt_attention_shares` for the tiles of a plan, once a step for all layers of one kind.  A step still to come (a captured pass) is taken to reach the
+    end of its bracket with every portion; at heads of 128 channels, and beyond one round, it shares nothing out (the shares of such tiles are fitted to the walks
+    a step has, and a replay's can be half as long)."""
+    key = (n_heads, hd, window, chunk, one_round)
+    if key not in plan.walk_shares:
+        places = plan.tile_places
+        if plan.tile_contexts is None:
+            if not (hd == 64 and one_round):
+                plan.walk_shares[key] = (1, 0)
+                return plan.walk_shares[key]
+            places = [(plan.max_tile_context - behind - rows if rows else pos0, rows, behind) for pos0, rows, behind in places]
+        first = lambda pos0: max(pos0 - window + 1 if window else 0, pos0 - pos0 % chunk if chunk else 0, 0)
+        contexts = [min([pos0 + rows] + ([window + plan.tile] if window else []) + ([chunk + plan.tile] if chunk else [])) for pos0, rows, _ in places if rows]
+        pairs = None
+        if hd == 64 and one_round:
+            seen = [(first(pos0) // 64, (pos0 + rows - 1) // 64) if rows else (0, -1) for pos0, rows, _ in places]
+            groups = zip(seen[::2], seen[1::2]) if plan.paired else ((t, (0, -1)) for t in seen)
+            pairs = [l1 - l0 + 1 + max(0, min(e1, l0 - 1) - e0 + 1) for (l0, l1), (e0, e1) in groups]               # (the late tile's, and what the early one sees before them)
+        plan.walk_shares[key] = prompt_attention_shares(contexts, n_heads, hd, plan.tile, one_round, pairs)
+    return plan.walk_shares[key]
 
 
 def _decode_piece(span, n_pieces):
@@ -1532,9 +1568,8 @@ def attention_bf16(q, cache, out, plan: AttentionPlan, positions, slots, table, 
         n_part = plan.n_tile_rows * n_heads * n_splits * (hd + 2) if n_splits > 1 else 0
         most, keys, counters = 1, 0, None
         one_round = (plan.n_tiles // 2 if plan.paired else plan.n_tiles) * n_heads <= lib().gi_compute_units()
-        contexts = plan.tile_contexts if plan.tile_contexts is not None else [plan.max_tile_context] if hd == 64 and one_round else None
-        if n_splits == 1 and memo is not None and contexts is not None and hd in (64, 128) and plan.n_tiles * n_heads <= PROMPT_SHARE_COUNTERS // 2:
-            most, keys = prompt_attention_shares([min(c, seen(c, plan.tile)) for c in contexts], n_heads, hd, plan.tile, one_round)
+        if n_splits == 1 and memo is not None and hd in (64, 128) and plan.n_tiles * n_heads <= PROMPT_SHARE_COUNTERS // 2:
+            most, keys = _walk_shares(plan, n_heads, hd, window, chunk, one_round)
             n_part = lib().gi_attention_prompt_share_floats(plan.n_tiles, plan.tile, n_heads, hd, 1, 1 if plan.paired else 0, most)
             part = _room(n_part, out.device) if n_part else None
             if part is not None:

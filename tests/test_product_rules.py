@@ -66,6 +66,40 @@ def test_a_context_is_shared_out_over_so_many_spans_as_a_grid_takes(rows, seen, 
     assert ops.lib().gi_attention_exact_spans(rows, rows, 1, 1, 16, 16, 16, seen) == spans
 
 
+# (first position, rows) of every portion, heads, channels, window -> shares, as measured faster
+WALKS = [
+    ([(0, 1500)], 32, 64, 0, 3), ([(0, 1024)], 32, 64, 0, 3), ([(0, 800)], 32, 64, 0, 3), ([(2000, 600)], 32, 64, 0, 3), ([(1300, 300), (0, 200)], 32, 64, 0, 3), ([(0, 1777)], 32, 64, 1024, 3),
+    ([(0, 1000)] * 2, 32, 64, 0, 1), ([(839, 479)], 64, 64, 0, 1), ([(866, 254)] * 4, 64, 64, 1024, 1), ([(0, 2048)], 32, 64, 1024, 1), ([(0, 950)] * 2, 32, 64, 512, 1), ([(522, 1961)], 32, 64, 0, 1),
+    ([(0, 760)], 32, 64, 0, 1), ([(347, 409), (0, 1638), (133, 157), (0, 171), (0, 289), (0, 701)], 32, 64, 1024, 1), ([(0, 2581)], 32, 64, 0, 2),
+    ([(0, 1000)], 32, 128, 0, 2), ([(0, 2000)], 24, 128, 0, 2), ([(1000, 1350), (0, 674)], 24, 128, 0, 3), ([(0, 1024)] * 2, 24, 128, 0, 1), ([(0, 2972)], 12, 128, 1024, 1), ([(0, 2048)], 32, 128, 0, 1),
+    ([(0, 800)], 32, 128, 0, 1), ([(3000, 700), (0, 700)], 32, 128, 0, 4),
+]
+
+
+def _plan(portions):
+    starts = [sum(n for _, n in portions[:i]) for i in range(len(portions))]
+    return ops.AttentionPlan(starts, [n for _, n in portions], [p for p, _ in portions], list(range(len(portions))), "cpu")
+
+
+@pytest.mark.parametrize("portions,heads,hd,window,shares", WALKS)
+def test_walks_over_keys_are_shared_out_where_that_is_faster(portions, heads, hd, window, shares):
+    plan = _plan(portions)
+    one_round = (plan.n_tiles // 2 if plan.paired else plan.n_tiles) * heads <= 256
+    assert ops._walk_shares(plan, heads, hd, window, 0, one_round)[0] == shares
+    assert list(plan.walk_shares.values())[0][0] == shares
+
+
+@pytest.mark.parametrize("portions,bracket,heads,hd,shares", [([(0, 1000)], 1024, 32, 64, 3), ([(0, 1000)], 1024, 32, 128, 1), ([(839, 479)], 2048, 64, 64, 1), ([(900, 600)], 2048, 32, 64, 3)])
+def test_walks_of_a_captured_pass_go_by_its_bracket(portions, bracket, heads, hd, shares):
+    """Whatever the positions of the step it was captured with."""
+    found = set()
+    for back in (0, 100):
+        plan = _plan([(max(0, p - back), n) for p, n in portions])
+        plan.max_tile_context, plan.tile_contexts = bracket, None
+        found.add(ops._walk_shares(plan, heads, hd, 0, 0, True))
+    assert len(found) == 1 and found.pop()[0] == shares
+
+
 def test_no_room_for_scratch_is_no_error(monkeypatch):
     def full(*args, **kw):
         raise torch.OutOfMemoryError("full")
