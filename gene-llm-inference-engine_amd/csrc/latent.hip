@@ -231,7 +231,7 @@ __global__ __launch_bounds__(64) void heads_product_kernel(const bf16_t* __restr
 // Shares of one row meet in `part` ([row][head][share]{m, l, o[vd]}, 32-bit) and `latent_merge_kernel` adds them; with one share
 // the wave writes the heads' outputs itself.  `rows`: the step's rows that this launch serves (nullptr: all, in order).
 // `sinks` [heads], where given: a score per head that joins the softmax's sum and has no value; the row's first share starts from it.
-template <int KS, int DT>
+template <int KS, int DT, bool EARLY>
 __global__ __launch_bounds__(64) void latent_attention_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache, bf16_t* __restrict__ out,
                                                              float* __restrict__ part, const int* __restrict__ rows, const int* __restrict__ pos,
                                                              const int* __restrict__ slot, const int* __restrict__ table, int table_stride, long page_stride,
@@ -274,9 +274,8 @@ __global__ __launch_bounds__(64) void latent_attention_kernel(const bf16_t* __re
             page[b] = cache + (long)tab[j0 / page_size] * page_stride;
             place[b] = j0 % page_size;
         }
-        // The values are asked for with the keys (up to keys of 288 channels: registers): behind the scores they were a second round trip to memory, most of
-        // the time of a share of one tile (5 rows of 32 heads at 212 positions: 13.4 us, so 8.7).
-        constexpr bool EARLY = KS <= 9;
+        // EARLY: the values are asked for with the keys (up to keys of 288 channels: registers): behind the scores they were a second round trip to memory, most of
+        // the time of a share of one tile (5 rows of 32 heads at 212 positions: 13.4 us, so 8.7).  See the launch for where they are not.
         uint4 k_early[2][EARLY ? KS : 1];
         uint2 v_early[2][EARLY ? DT : 1];
         const auto value = [&](int b, int i) {
@@ -828,10 +827,11 @@ GI_API long gi_latent_attention_scratch_floats(int n_rows, int n_heads, int vd, 
 }
 
 // q: bfloat16 [n_rows, n_heads*kd] (folded queries); cache: bfloat16 pages [place][kd] then [vd][place]; out: bfloat16 [n_rows, n_heads*vd].
-// rows: the n_rows rows of the step to serve (nullptr: rows 0 .. n_rows - 1).
+// rows: the n_rows rows of the step to serve (nullptr: rows 0 .. n_rows - 1).  share_tiles: how many tiles of 32 positions the longest share has, as far as the
+// caller knows (for the choice of a kernel alone: any number gives the same results).
 GI_API int gi_latent_attention_bf16(const void* q, const void* cache, void* out, float* part, long part_floats, const int* rows, const int* pos, const int* slot,
                                     const int* table, int table_stride, long page_stride, int page_size, int n_rows, int n_heads, int kd, int vd, int window,
-                                    float scale, int n_splits, const float* sinks, hipStream_t stream) {
+                                    float scale, int n_splits, int share_tiles, const float* sinks, hipStream_t stream) {
     GI_REQUIRE(n_rows > 0 && n_heads > 0 && gi_latent_attention_supports(kd, vd, page_size), "latent_attention: sizes (rows %d, heads %d, keys %d, values %d, pages of %d) are not taken",
                n_rows, n_heads, kd, vd, page_size);
     GI_REQUIRE(window >= 0 && n_splits >= 1 && n_splits <= 64 && page_stride >= (long)page_size * (kd + vd) && page_stride % 8 == 0 && ((uintptr_t)cache & 15) == 0 &&
@@ -841,13 +841,18 @@ GI_API int gi_latent_attention_bf16(const void* q, const void* cache, void* out,
     GI_REQUIRE((long)n_rows * n_heads < 2147483647L && (n_heads + 15) / 16 <= 65535, "latent_attention: too many rows or heads");
     dim3 grid(n_rows, (n_heads + 15) / 16, n_splits);
     const float scale2 = scale * 1.4426950408889634f;
-#define GO(KS, DT)                                                                                                                                      \
-    latent_attention_kernel<KS, DT><<<grid, 64, 0, stream>>>((const bf16_t*)q, (const bf16_t*)cache, (bf16_t*)out, part, rows, pos, slot, table, table_stride, \
-                                                             page_stride, page_size, n_heads, kd, vd, window, scale2, n_splits, sinks)
-    if (kd <= 96 && vd <= 64) GO(3, 4);
-    else if (kd <= 160 && vd <= 128) GO(5, 8);
-    else if (kd <= 288 && vd <= 256) GO(9, 16);
-    else GO(18, 32);
+#define GO(KS, DT, EARLY_)                                                                                                                              \
+    latent_attention_kernel<KS, DT, EARLY_><<<grid, 64, 0, stream>>>((const bf16_t*)q, (const bf16_t*)cache, (bf16_t*)out, part, rows, pos, slot, table, table_stride, \
+                                                                     page_stride, page_size, n_heads, kd, vd, window, scale2, n_splits, sinks)
+    // At keys of 288 channels the values' registers leave a SIMD one wave (two without): shares of one tile of positions that are more than that, or of two that
+    // are at most half as many again, wait for a second round behind it.  40 rows of 32 heads at 500 positions (1,280 waves) 35.5 us, values behind the scores 31.7; 12
+    // rows at 4,000 (1,536 waves of two tiles) 51.6 and 49.0; but 40 rows at 1,000 (2,000 waves of two) 39.9 and 41.8, 64 rows at 4,000 (eight tiles) 88 and 115.
+    const long waves = (long)n_rows * grid.y * n_splits, places = 4L * gi_compute_units();
+    const bool second_round = waves > places && (share_tiles == 1 || (share_tiles == 2 && 2 * waves <= 3 * places));
+    if (kd <= 96 && vd <= 64) GO(3, 4, true);
+    else if (kd <= 160 && vd <= 128) GO(5, 8, true);
+    else if (kd <= 288 && vd <= 256) { if (second_round) GO(9, 16, false); else GO(9, 16, true); }
+    else GO(18, 32, false);
 #undef GO
     GI_CHECK_LAUNCH("latent_attention");
     if (n_splits > 1) {

@@ -81,7 +81,7 @@ _SIGNATURES = {
                           c_void_p, c_int, c_long, c_void_p, c_int, c_long, c_int, c_int, c_int, c_void_p],
     "gi_heads_product": [c_void_p, c_long, c_void_p, c_void_p, c_int, c_long, c_long, c_int, c_int, c_int, c_int, c_void_p, c_long, c_void_p],
     "gi_latent_attention_bf16": [c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int, c_int,
-                                 c_float, c_int, c_void_p, c_void_p],
+                                 c_float, c_int, c_int, c_void_p, c_void_p],
     "gi_latent_attention_tiles_bf16": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p, c_void_p],
     "gi_latent_queries": [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_long, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "gi_act_mul": [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_float, c_void_p],
@@ -2088,11 +2088,13 @@ def latent_attention_bf16(q, cache, out, ctx, table, n_heads, kd, vd, page_size,
         span = min(span, int(window) + 31)
     groups = n_single * (-(-n_heads // 16))
     n_splits = max(1, min(LATENT_MAX_SPLITS, LATENT_WAVES // groups, (span + LATENT_SHARE - 1) // LATENT_SHARE))
+    tiles = -(-span // 32)                # (a captured pass serves contexts from half its bracket on)
+    share_tiles = max(1, -(-(tiles if plan.decode_positions is not None else tiles // 2) // n_splits))
     n_part = n_single * n_heads * n_splits * (vd + 2) if n_splits > 1 else 0
     part = torch.empty(n_part, dtype=torch.float32, device=out.device) if n_part else None
     _call("gi_latent_attention_bf16", q.data_ptr(), cache.data_ptr(), out.data_ptr(), _ptr(part), n_part, _ptr(rows), ctx.row_pos.data_ptr(), ctx.row_slot.data_ptr(),
-          table.data_ptr(), table.stride(0), cache.stride(0), int(page_size), n_single, n_heads, kd, vd, int(window or 0), float(scale), n_splits, _ptr(sinks),
-          _stream())
+          table.data_ptr(), table.stride(0), cache.stride(0), int(page_size), n_single, n_heads, kd, vd, int(window or 0), float(scale), n_splits, share_tiles,
+          _ptr(sinks), _stream())
     return out
 
 

@@ -586,6 +586,36 @@ def test_matrix_core_attention_over_latent_pages_with_heads_in_groups_of_32(H, k
     test_matrix_core_attention_over_latent_pages(H, kd, vd, window, lens, pos0)
 
 
+@pytest.mark.parametrize("n, H, context, window", [(40, 32, 500, None), (12, 32, 4000, None), (60, 32, 511, 300), (32, 32, 500, None), (65, 20, 333, None)])
+def test_single_rows_over_latent_pages_in_more_waves_than_places(n, H, context, window):
+    """Shares of one and two tiles, on both sides of a wave for every place of the chip: the kernels that ask for the values before and behind the scores give the
+    same bits, and the right ones."""
+    from geneinfer_amd.kernels import ops
+    from geneinfer_amd.parts import StepContext
+    kd, vd, page = 288, 256, 16
+    g = torch.Generator(device=DEV).manual_seed(n)
+    pages = -(-context // page)
+    cache = torch.randn(n * pages, page * (kd + vd), generator=g, device=DEV).to(torch.bfloat16)
+    keys = cache[:, :page * kd].reshape(n, pages * page, kd)
+    cache[:, page * kd:] = keys.reshape(n * pages, page, kd)[:, :, :vd].transpose(1, 2).reshape(n * pages, -1)
+    table = torch.arange(n * pages, dtype=torch.int32, device=DEV).view(n, pages)
+    at = [context - 1 - (7 * i) % (context // 2) for i in range(n)]
+    q = torch.randn(n, H, kd, generator=g, device=DEV).to(torch.bfloat16)
+    pos, slots = torch.tensor(at, dtype=torch.int32, device=DEV), torch.arange(n, dtype=torch.int32, device=DEV)
+    seen = []
+    for known in (True, False):
+        ctx = StepContext(n_rows=n, dtype=torch.bfloat16, device=torch.device(DEV), tokens=pos, row_pos=pos, row_slot=slots, seg_slot=list(range(n)), seg_start=list(range(n)), seg_len=[1] * n, seg_pos0=at)
+        plan = ops._plan_of(ctx)
+        plan.decode_positions = plan.decode_positions if known else None
+        seen.append(torch.empty(n, H * vd, dtype=torch.bfloat16, device=DEV))
+        ops.latent_attention_bf16(q.view(n, -1), cache, seen[-1], ctx, table, H, kd, vd, page, window, 0.06)
+    assert torch.equal(*seen)
+    for i in (0, 1, n // 2, n - 1):
+        k = keys[i, max(0, at[i] - window + 1) if window else 0:at[i] + 1].double()
+        want = torch.softmax(0.06 * (q[i].double() @ k.T), -1) @ k[:, :vd]
+        assert relative_error(seen[0][i], want.reshape(-1).cpu()) < 1e-2
+
+
 @pytest.mark.parametrize("page, window", [(16, None), (48, 130), (64, None)])
 def test_latent_attention_with_scores_that_climb_along_the_context_and_sinks(page, window):
     """Scores grow along the context by 0 to 12 units a tile of 32 positions, up to 60 and more: a column's maximum moves in every tile, by less and by more than what
