@@ -530,6 +530,15 @@ GI_API int gi_gemm_exact(const void* A, int a_dtype, const void* W, int w_dtype,
 
 // Whether gi_gemm_exact_gated takes a product of these sizes.
 GI_API int gi_gemm_exact_gated_takes(int M, int N, int K) { return M > 0 && N > 0 && N % 2 == 0 && K > 0 && K % 4 == 0 && few_rows(M, N, K); }
+// And whether it is the faster way.  Its strips are 16 rows of weights; where the product alone has strips of 8 and its busiest compute unit so reads fewer
+// rows, the two launches are the faster ones from k = 2,048 on: 1,024 x 4,096 10.5 us apart and 13.4 in one for 1 row, 2,048 x 3,072 11.0 and 11.9, 5,632 x 4,096
+// 23.2 and 26.8 (8 rows 28.8 and 29.5); at k = 2,048 only for a strip a unit or two rows (1,024 columns 7.4 and 7.8, 6,144 for 1 row 14.8 and 15.5, for 8
+// 17.9 and 16.5).
+GI_API int gi_gemm_exact_gated_pays(int M, int N, int K) {
+    const int units = gi_compute_units(), strips16 = (N + 15) / 16, strips8 = (N + 7) / 8;
+    const bool more_rows = M <= 8 && N < 32 * units && (strips16 + units - 1) / units * 2 > (strips8 + units - 1) / units;
+    return gi_gemm_exact_gated_takes(M, N, K) && !(more_rows && (K > 2048 || (K == 2048 && (N <= 4 * units || (M <= 2 && N > 16 * units)))));
+}
 
 // C [M, N / 2] = act(gate) * up of A W^T with W = [gate; up] (N rows in all), 32-bit throughout: the bits of gi_gemm_exact and gi_act_mul.  C must not be what A reads.
 GI_API int gi_gemm_exact_gated(const float* A, const float* W, float* C, int act, float limit, int M, int N, int K, long lda, long ldw, long ldc, hipStream_t stream) {

@@ -151,6 +151,8 @@ def lib():
         l.gi_gemm_exact_qkv_rope_store_takes.restype = c_int
         l.gi_gemm_exact_gated_takes.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_exact_gated_takes.restype = c_int
+        l.gi_gemm_exact_gated_pays.argtypes = [c_int, c_int, c_int]
+        l.gi_gemm_exact_gated_pays.restype = c_int
         l.gi_gemm_exact_scratch_floats.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_exact_scratch_floats.restype = c_long
         l.gi_gemm_bf16_scratch_floats.argtypes = [c_int, c_int, c_int, c_int, c_int]
@@ -585,6 +587,12 @@ def gemm_exact(a, w, out, accumulate=False):
 @lru_cache(maxsize=8192)
 def _exact_gated_takes(m, n, k) -> bool:
     return bool(lib().gi_gemm_exact_gated_takes(m, n, k))
+
+
+@lru_cache(maxsize=8192)
+def gemm_exact_gated_pays(m, n, k) -> bool:
+    """Whether `gemm_exact_gated` is faster than `gemm_exact` and `act_mul` at these sizes."""
+    return bool(lib().gi_gemm_exact_gated_pays(m, n, k))
 
 
 def gemm_exact_gated_takes(a, w, out) -> bool:

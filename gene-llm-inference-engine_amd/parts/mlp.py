@@ -50,7 +50,7 @@ class SwiGlu(FeedForward):
         else:
             mid = torch.empty((T, inter), dtype=self.mid_dtype, device=ctx.device)
             rows = h.materialize() if self.in_dtype == torch.float32 and isinstance(h, NormedRows) else h
-            if torch.is_tensor(rows) and ops.gemm_exact_gated_takes(rows, self.w_gate_up, mid):
+            if torch.is_tensor(rows) and ops.gemm_exact_gated_takes(rows, self.w_gate_up, mid) and ops.gemm_exact_gated_pays(T, *self.w_gate_up.shape):
                 ops.gemm_exact_gated(rows, self.w_gate_up, mid, self.activation, self.limit)
             else:
                 gate_up = torch.empty((T, 2 * inter), dtype=torch.float32, device=ctx.device)

@@ -66,6 +66,12 @@ def test_a_context_is_shared_out_over_so_many_spans_as_a_grid_takes(rows, seen, 
     assert ops.lib().gi_attention_exact_spans(rows, rows, 1, 1, 16, 16, 16, seen) == spans
 
 
+@pytest.mark.parametrize("m,n,k,taken", [(3, 16384, 2048, 1), (1, 4096, 4096, 1), (8, 8192, 4096, 1), (1, 6656, 4096, 1), (16, 1024, 4096, 1), (1, 1024, 1024, 1), (1, 2048, 2048, 1), (8, 5120, 2048, 1),
+                                         (9, 1000, 4096, 1), (1, 1000, 4096, 0), (1, 1024, 4096, 0), (8, 2048, 3072, 0), (1, 5632, 4096, 0), (4, 4608, 3072, 0), (8, 1024, 2048, 0), (2, 6144, 2048, 0), (17, 4096, 1024, 0), (3, 4095, 1024, 0)])
+def test_gates_in_the_product_where_that_is_faster(m, n, k, taken):
+    assert ops.gemm_exact_gated_pays(m, n, k) == taken
+
+
 # (first position, rows) of every portion, heads, channels, window -> shares, as measured faster
 WALKS = [
     ([(0, 1500)], 32, 64, 0, 3), ([(0, 1024)], 32, 64, 0, 3), ([(0, 800)], 32, 64, 0, 3), ([(2000, 600)], 32, 64, 0, 3), ([(1300, 300), (0, 200)], 32, 64, 0, 3), ([(0, 1777)], 32, 64, 1024, 3),
