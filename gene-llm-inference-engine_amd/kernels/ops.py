@@ -1444,10 +1444,11 @@ def _decode_ragged_split(groups, longest, mean, hd, n_waves):
     """(splits, waves) for contexts whose lengths are known, where the plain rule cuts none: one workgroup per (row, group of heads) takes the time of the
     longest context; cut in two or more and dealt out there and back (`_decode_order`), the compute units share the bytes more evenly, for the merge.  24
     rows of 8 groups of 128 channels at 380 to 3,000 positions beside a prompt's portions: 44.6 -> 35.3 us a layer and 5 for the merge (expected: 49.5 and
-    34; so it has to promise a fifth)."""
+    34).  It has to promise three tenths: of 253 steps that were cut where it promised two, 16 were slower, by up to a tenth (42 rows of 4 groups of 128 channels
+    at 1,500 to 3,000 positions, promised 21 %, 37.9 and 41.2 us); of the 120 that promise three none is, and they gain 18 %."""
     units, row_mb = lib().gi_compute_units(), hd * 4 / 1e6
     even_us = max(groups * mean * row_mb / units / _DECODE_SHARED_UNIT_MB_PER_S, groups * mean * row_mb / _DECODE_CHIP_MB_PER_S) * 1e6
-    best, best_us = (1, n_waves), 0.8 * max(even_us, longest * row_mb / _DECODE_UNIT_MB_PER_S * 1e6)
+    best, best_us = (1, n_waves), 0.7 * max(even_us, longest * row_mb / _DECODE_UNIT_MB_PER_S * 1e6)
     for splits in (2, 3, 4):
         if longest / splits < 256:
             break

@@ -72,6 +72,13 @@ def test_gates_in_the_product_where_that_is_faster(m, n, k, taken):
     assert ops.gemm_exact_gated_pays(m, n, k) == taken
 
 
+# workgroups uncut, longest context, mean, channels -> cuts, as measured faster
+@pytest.mark.parametrize("groups,longest,mean,hd,splits", [(192, 3000, 1640, 128, 2), (168, 2988, 2247, 128, 1), (144, 1709, 1282, 128, 1), (152, 4064, 3041, 64, 1), (176, 6694, 3350, 64, 3), (148, 3501, 1400, 64, 4),
+                                                           (128, 1123, 645, 128, 1), (224, 4589, 2300, 128, 2), (64, 500, 100, 128, 1)])
+def test_known_contexts_are_cut_where_that_is_faster(groups, longest, mean, hd, splits):
+    assert ops._decode_ragged_split(groups, longest, mean, hd, 8) == ((splits, 4) if splits > 1 else (1, 8))
+
+
 # (first position, rows) of every portion, heads, channels, window -> shares, as measured faster
 WALKS = [
     ([(0, 1500)], 32, 64, 0, 3), ([(0, 1024)], 32, 64, 0, 3), ([(0, 800)], 32, 64, 0, 3), ([(2000, 600)], 32, 64, 0, 3), ([(1300, 300), (0, 200)], 32, 64, 0, 3), ([(0, 1777)], 32, 64, 1024, 3),
