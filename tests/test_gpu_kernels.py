@@ -845,6 +845,73 @@ def test_decoded_rows_of_unequal_contexts_dealt_out_over_the_chip(n_single, port
     assert torch.equal(*both)
 
 
+@pytest.mark.parametrize("n_single, n_heads, n_kv, hd, splits", [(24, 24, 8, 128, 3), (38, 32, 4, 64, 4)])
+def test_ordered_rows_whose_contexts_are_cut(n_single, n_heads, n_kv, hd, splits):
+    """Single rows at 500 to 3,000 positions beside a prompt's portion: taken longest context first, and each context cut.  The pieces are kept by the place in that
+    order and come back to their rows."""
+    from geneinfer_amd.parts import StepContext
+    o = ops()
+    g = torch.Generator().manual_seed(n_single)
+    contexts = [int(c) for c in torch.randint(500, 1700, (n_single,), generator=g)]
+    contexts[5], contexts[n_single - 2] = 3000, 2900
+    contexts.insert(n_single // 2, 300)                        # a portion of 100 rows in the middle
+    cache, table, dense = build_paged(contexts, n_kv, hd, 16, torch.bfloat16, seed=5, scale_one=(2000, 3.0))
+    rows, seg_start, seg_len, seg_pos0, seg_slot = [], [], [], [], []
+    for slot, c in enumerate(contexts):
+        n = 100 if slot == n_single // 2 else 1
+        seg_start.append(len(rows)); seg_len.append(n); seg_pos0.append(c - n); seg_slot.append(slot + 1)
+        rows += [(slot, c - n + i) for i in range(n)]
+    T = len(rows)
+    q = randn(T, n_heads * hd, dtype=torch.bfloat16, seed=3)
+    pos = torch.tensor([p for _, p in rows], dtype=torch.int32, device=DEV)
+    slots = torch.tensor([s_ + 1 for s_, _ in rows], dtype=torch.int32, device=DEV)
+    ctx = StepContext(n_rows=T, dtype=torch.bfloat16, device=torch.device(DEV), tokens=pos, row_pos=pos, row_slot=slots, seg_slot=seg_slot,
+                      seg_start=seg_start, seg_len=seg_len, seg_pos0=seg_pos0)
+    plan = o._plan_of(ctx)
+    assert o.decode_attention_shape(n_single, n_heads, n_kv, hd, 3000)[0] == 1
+    assert o._decode_ragged_split(n_single * n_kv, 3000, plan.decode_positions / n_single, hd, 8)[0] == splits
+    out = torch.full((T, n_heads * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    o.attention(q, cache, out, ctx, table, n_heads, n_kv, hd)
+    assert "decode_order" in ctx.memo
+    want = plain_attention_rows(q, dense, rows, n_heads, n_kv, hd, None)
+    worst = float(((out.double().cpu() - want).norm(dim=1) / want.norm(dim=1)).max())
+    assert rel(out, want) < 8e-3 and worst < 3e-2, (rel(out, want), worst)
+
+
+@pytest.mark.parametrize("n_heads", [32, 24])
+def test_ordered_rows_in_the_kernel_that_rotates_and_stores(n_heads):
+    """The rows of a decode step whose contexts are cut and whose workgroups are more than the compute units: each still writes its own key and value, once."""
+    from geneinfer_amd.parts import StepContext
+    o = ops()
+    n, longest, n_kv, hd = 17, 4096, 8, 64
+    g = torch.Generator().manual_seed(n_heads)
+    contexts = [int(c) for c in torch.randint(2, longest, (n,), generator=g)]
+    contexts[3] = longest
+    cache, table, dense = build_paged(contexts, n_kv, hd, 16, torch.bfloat16, seed=5)
+    a, kv = n_heads * hd, n_kv * hd
+    pos = torch.tensor([c - 1 for c in contexts], dtype=torch.int32, device=DEV)
+    slots = torch.arange(1, n + 1, dtype=torch.int32, device=DEV)
+    qkv = randn(n, a + 2 * kv, seed=31)
+    inv = torch.tensor([1.0 / (10000.0 ** (2 * k / hd)) for k in range(hd // 2)], dtype=torch.float64, device=DEV)
+    cos, sin = torch.empty(n, hd // 2, device=DEV), torch.empty(n, hd // 2, device=DEV)
+    o.rope_cos_sin(pos, inv, cos, sin)
+    want_cache, q_rot = cache.clone(), torch.empty(n, a, dtype=torch.bfloat16, device=DEV)
+    o.rope_store(qkv[:, :a], qkv[:, a:a + kv], qkv[:, a + kv:], cos, sin, pos, slots, table, q_rot, want_cache, n_heads, n_kv, hd)
+    for i, c in enumerate(contexts):
+        page, place = int(table[i + 1, (c - 1) // 16]), (c - 1) % 16
+        dense[i][0][c - 1], dense[i][1][c - 1] = want_cache[page, 0, :, place].cpu(), want_cache[page, 1].view(n_kv, hd, 16)[:, :, place].cpu()
+    ctx = StepContext(n_rows=n, dtype=torch.bfloat16, device=torch.device(DEV), tokens=pos, row_pos=pos, row_slot=slots, seg_slot=list(range(1, n + 1)), seg_start=list(range(n)),
+                      seg_len=[1] * n, seg_pos0=[c - 1 for c in contexts])
+    splits = o.decode_attention_shape(n, n_heads, n_kv, hd, longest, fused=True)[0]
+    assert splits > 1 and n * n_kv * splits > o.lib().gi_compute_units()
+    out = torch.full((n, a), float("nan"), dtype=torch.bfloat16, device=DEV)
+    assert o.attention_from_products(qkv[:, :a], qkv[:, a:a + kv], qkv[:, a + kv:], cos, sin, cache, out, ctx, table, n_heads, n_kv, hd) and "decode_order" in ctx.memo
+    got, kept = torch.nan_to_num(cache.float(), nan=-1.0), torch.nan_to_num(want_cache.float(), nan=-1.0)
+    assert rel(got, kept) < 1e-3 and float(((got - kept).abs() > 0.02 * kept.abs() + 1e-6).sum()) == 0           # (a rotated key may round the other way in 32-bit)
+    want = plain_attention_rows(q_rot, dense, [(i, c - 1) for i, c in enumerate(contexts)], n_heads, n_kv, hd, None)
+    assert rel(out, want) < 8e-3
+
+
 @pytest.mark.parametrize("window", [None, 200])
 def test_many_prompt_tiles_of_many_heads(window):
     """More workgroups than compute units at head size 64 (5 pairs of tiles x 64 heads): the step takes the kernel with a
@@ -937,6 +1004,36 @@ def test_workgroups_that_meet_in_a_kernel_under_capture():
         assert torch.equal(att, want[0]) and torch.equal(out, want[1])
         torch.cuda.synchronize()
         o.gemm_bf16(a, w, torch.empty_like(out))
+
+
+def test_workgroups_that_meet_on_two_streams_at_once():
+    """Two steps side by side, each with counters of its own, and products that clear their own: every result has the bits it has alone."""
+    from types import SimpleNamespace
+    o = ops()
+    m, n_heads, n_kv, hd, rows, n, k = 1000, 32, 8, 128, 2048, 2048, 8192
+    cache, table, _ = build_paged([m], n_kv, hd, 16, torch.bfloat16, seed=5)
+    plan = o.AttentionPlan([0], [m], [0], [1], DEV)
+    pos, slots = torch.arange(m, dtype=torch.int32, device=DEV), torch.ones(m, dtype=torch.int32, device=DEV)
+    q, a, w = randn(m, n_heads * hd, dtype=torch.bfloat16, seed=3), randn(rows, k, dtype=torch.bfloat16, seed=4), randn(n, k, dtype=torch.bfloat16, seed=6)
+    assert o._shares(rows, n, k, 0, False) == o._shares(rows, n, k, 0, True) == 2
+
+    def step(times):
+        ctx, got = SimpleNamespace(memo={}, device=torch.device(DEV)), []
+        for _ in range(times):
+            got.append(o.attention_bf16(q, cache, torch.empty_like(q), plan, pos, slots, table, n_heads, n_kv, hd, memo=ctx.memo))
+            got.append(o.gemm_bf16(a, w, torch.empty(rows, n, device=DEV), counters=o.step_counters(ctx, rows, n, k)))
+            got.append(o.gemm_bf16(a, w, torch.empty(rows, n, device=DEV)))
+        return got
+
+    want = step(1)
+    torch.cuda.synchronize()
+    streams, got = [torch.cuda.Stream(), torch.cuda.Stream()], []
+    for stream in streams:
+        with torch.cuda.stream(stream):
+            got.append(step(6))
+    torch.cuda.synchronize()
+    for results in got:
+        assert all(torch.equal(x, want[i % 3]) for i, x in enumerate(results))
 
 
 @pytest.mark.parametrize("hd, m", [(128, 1000), (64, 1500)])

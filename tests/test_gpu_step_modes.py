@@ -219,6 +219,33 @@ def test_steps_whose_shape_comes_again_are_replayed_from_a_captured_pass(tmp_pat
         assert_within_bfloat16_noise(got, lambda k: exact[k[0]][k[1]], lambda k: near[k[0]][k[1]], "tiny D, captured steps")
 
 
+@pytest.mark.parametrize("hd, eager, captured", [(128, 2, 1), (64, 3, 3)])
+def test_a_prompt_that_comes_again_with_walks_that_are_shared_out(tmp_path, hd, eager, captured, monkeypatch):
+    """A prompt of 1,000 rows of 32 heads: the first time its long walks over keys are shared out by the step's own lengths, from the second time on it is a captured
+    pass, which goes by its bracket (at 128 channels it shares none out).  Both are the plain model's logits, and every replay has the same bits."""
+    from geneinfer_amd.engine import Runner, StepEntry, load_model
+    from geneinfer_amd.kernels import ops
+    config = dict(CONFIGS["D"], hidden_size=128, num_attention_heads=32, num_key_value_heads=8, head_dim=hd, num_hidden_layers=2, max_position_embeddings=2048)
+    write_model(tmp_path, config, seed=3)
+    rng = random.Random(9)
+    tokens = [rng.randrange(config["vocab_size"]) for _ in range(1000)]
+    wanted = (3, 127, 128, 640, 999)
+    plain = PlainLlama(tmp_path)
+    exact, near = plain.logits(tokens), plain.with_storage(torch.bfloat16).logits(tokens)
+    runner = Runner(load_model(tmp_path, "bfloat16", "cuda:0"), page_size=16, max_tokens=4096, max_requests=2, max_rows=1024)
+    shares, asked = [], ops._walk_shares
+    monkeypatch.setattr(ops, "_walk_shares", lambda *a: shares.append(asked(*a)[0]) or asked(*a))
+    got = []
+    for i in range(4):
+        runner.open(i)
+        got.append(runner.step([StepEntry(i, tokens, wanted)]).cpu().clone())
+        runner.close(i)
+    assert shares == [eager] * 2 + [captured] * 2 and next(iter(runner._step_graphs.values())).calls == 4
+    assert torch.equal(got[1], got[2]) and torch.equal(got[1], got[3])
+    for rows in got[:2]:
+        assert_within_bfloat16_noise({p: rows[j] for j, p in enumerate(wanted)}, exact.__getitem__, near.__getitem__, f"heads of {hd}, 1,000 rows")
+
+
 def test_a_runner_with_captured_steps_is_freed_without_the_cycle_collector(case):
     """A runner and its captured graphs form no reference cycle: dropping the runner frees them at once, not at a
     moment of the cycle collector's choosing (which may fall inside another capture, where freeing aborts)."""
