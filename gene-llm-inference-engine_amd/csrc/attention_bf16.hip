@@ -1213,11 +1213,11 @@ GI_API int gi_attention_prompt_bf16(const void* q, const void* cache, void* out,
     GI_REQUIRE(!paired || n_tiles % 2 == 0, "attention_prompt: %d tiles cannot go in pairs", n_tiles);
     // Two tiles share a workgroup of 1024 threads up to head size 64; larger heads need more registers than such a
     // workgroup leaves a thread, and take the same list tile by tile (a filling tile of 0 rows then does nothing).
-    // Head size 128 takes the wide kernel (measured at 8,192 rows: 726 against 1,577 us a layer of 32 heads).  At head size 64 the
-    // first kernel's pairs of tiles are the better balance while they fit the chip in one round (a workgroup of 16 waves a compute
-    // unit: 2,048 rows of 32 heads take 56 against 61 us) and where few tiles share their keys out; beyond one round its time
-    // doubles at once and the wide kernel's many small workgroups win (2,560 rows: 68 against 100 us; 8,192: 360 against 572).
-    // With its long walks shared out the wide kernel is the faster one within a round too, from so many rows or keys on that the caller shares them out.
+    // Head size 128 takes the wide kernel (measured at 8,192 rows: 726 against 1,577 us a layer of 32 heads).  At head size 64 the first kernel walks a
+    // pair's keys with one workgroup of 16 waves, and its time doubles at once beyond one round of those: there the wide kernel's many small workgroups
+    // win (32 heads: 2,560 rows 52.4 us, 49.8 shared out; 8,192: 360 against 572).  Within a round it wins where the caller shares the walks out (2,048 rows of
+    // 32 heads 39.6 against 40.8 us, 1,024 rows 18.5 against 23).  The first kernel keeps the steps within a round whose walks are short or that a rule of
+    // the caller's does not share out (300 rows from the beginning, 2,048 rows under a window of 1,024: 36.7 against 39.3), and all whose keys are cut into splits.
     if (takes_wide(n_tiles, n_heads, hd, n_splits, paired, most_shares > 1)) {
         GI_REQUIRE((long)n_tiles * n_splits * (most_shares > 1 ? most_shares : 1) <= 65535, "attention_prompt: %d tiles in %d splits are too many for one launch", n_tiles, n_splits);
         WideShares shares = {1, 0, nullptr, nullptr};

@@ -730,7 +730,9 @@ __global__ __launch_bounds__(256) void delta_single_kernel(const float* __restri
 }
 
 // ------------------------------------------------------------------------------------- gated delta rule, a prompt's rows in blocks
-// The same rule for requests that bring many rows (keys of 64 channels, one decay a head).  With d_t the decays, R_ti = d_{i+1} .. d_t and
+// The same rule for requests that bring many rows (keys of 64 channels, one decay a head), by the published chunked form of the delta rule: the block's updates
+// in their WY form, from a unit lower triangular system (the UT transform; Yang and others, "Parallelizing Linear Transformers with the Delta Rule over Sequence
+// Length", 2024, with the decays of "Gated Delta Networks", 2024).  With d_t the decays, R_ti = d_{i+1} .. d_t and
 // g_t = d_0 .. d_t inside a block of 64 rows, S_0 the memory before it, the rule's updates w_t = s_t (v_t - d_t S_{t-1}^T k_t) are the
 // solution of (1 + A) W = s (V - g K S_0), A_ti = s_t R_ti (k_t . k_i) below the diagonal.  So with U = (1 + A)^-1 s V and P = (1 + A)^-1 s g K,
 // which need no memory,
