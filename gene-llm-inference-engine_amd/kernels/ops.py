@@ -1736,13 +1736,18 @@ def _shares(m, n, k, kind, counted) -> int:
     return lib().gi_gemm_bf16_shares(m, n, k, kind, 1 if counted else 0)
 
 
+# Rows up to which a product's scratch depends on its sizes alone and no tile is shared out: decoding asks for nothing else on the way to each launch (the kind, the
+# shares and the scratch by kind took 1 us of the host's 10 to 20 a product).
+FEW_ROWS = 128
+
+
 def _product_scratch(m, n, k, kind, counted, device):
     """(scratch, its floats) of a product: partial sums where k is shared out over workgroups.  Without the room for shared tiles' sums the product's other
     kernels make it."""
     floats = _scratch_floats(m, n, k, kind, counted)
     if not floats:
         return None, 0
-    if _shares(m, n, k, kind, counted) > 1:
+    if m > FEW_ROWS and _shares(m, n, k, kind, counted) > 1:
         scratch = _room(floats, device)
         return scratch, floats if scratch is not None else 0
     return torch.empty(floats, dtype=torch.float32, device=device), floats
@@ -1751,7 +1756,7 @@ def _product_scratch(m, n, k, kind, counted, device):
 def step_counters(ctx, m, n, k, kind=0):
     """`counters` for a product of these sizes and kind (`product_kind`) in the step `ctx`: the step's own, filled once and left as they were by every product (a
     step's products run one after the other); None for a product that has no use for them."""
-    if ctx is None or _shares(m, n, k, kind, True) == 1:
+    if ctx is None or m <= FEW_ROWS or _shares(m, n, k, kind, True) == 1:
         return None
     counters = ctx.memo.get("product_counters")
     if counters is None:
@@ -1778,7 +1783,7 @@ def gemm_bf16_takes_norm(m, n, k, gated=False) -> bool:
     return bool(lib().gi_gemm_bf16_takes_norm(m, n, k, 1 if gated else 0))
 
 
-def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=None, norm_out=None, gate_limit=0.0, counters=None):
+def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=None, norm_out=None, gate_limit=0.0, counters=None, ctx=None):
     """out (=|+=) a @ w.T with bfloat16 operands on the matrix cores, float32 sums.
     gated: w is [gate; up] interleaved in groups of 16 rows and out = act(a @ gate.T) * (a @ up.T), bfloat16 [m, n/2]; act is
     SiLU (gated = True or "silu"), the tanh form of GELU (gated = "gelu_tanh") or the clamped form (gated = "swish_clamped", with
@@ -1788,7 +1793,7 @@ def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=N
     norm_out = (g, scaled, squares), with accumulate: beside out += a @ w.T, scaled = bfloat16(g * out) and squares
     [m, gemm_bf16_norm_parts(m, n, k)] = the pieces of the rows' sums of out^2;
     norm_in = (squares, eps): a is such a `scaled`, and the results are multiplied by rsqrt(sum of the row's pieces / k + eps).
-    counters: see `step_counters`; the product clears its own where it needs them and has none."""
+    counters: see `step_counters`; the product clears its own where it needs them and has none.  ctx: the step whose counters it may take, where none are given."""
     _dev(a, w, out, counters)
     _check_counters(counters)
     m, k = a.shape
@@ -1799,7 +1804,10 @@ def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=N
         raise KernelError(f"gemm: out is {tuple(out.shape)}, ({m}, {n // 2 if gated else n}) is needed")
     if not (checked or gemm_bf16_supports(a, w, out)):
         raise KernelError("gemm_bf16: operands must be bfloat16 with K and row strides multiples of 8, 16-byte aligned")
-    scratch, n_scratch = _product_scratch(m, n, k, product_kind(out, accumulate, gated, norm_in, norm_out), counters is not None, a.device)
+    kind = product_kind(out, accumulate, gated, norm_in, norm_out) if m > FEW_ROWS else 0
+    if counters is None:
+        counters = step_counters(ctx, m, n, k, kind)
+    scratch, n_scratch = _product_scratch(m, n, k, kind, counters is not None, a.device)
     if gated and gated is not True and gated not in ACTIVATIONS:
         raise KernelError(f"gemm: unknown activation {gated!r} of a gated product; known: {', '.join(ACTIVATIONS)}")
     gate_code = 0 if not gated else 1 + (0 if gated is True else ACTIVATIONS[gated])        # 1: SiLU, 2: GELU (tanh form)

@@ -25,14 +25,11 @@ def linear(a, weight: torch.Tensor, out: torch.Tensor, accumulate: bool = False,
     if isinstance(a, HandedRows):
         if (weight.dtype == torch.bfloat16 and ops.gemm_bf16_supports(a.scaled, weight, out)
                 and ops.gemm_bf16_takes_norm(a.scaled.shape[0], weight.shape[0], weight.shape[1], gated)):
-            norm_in = (a.squares, a.eps)
-            return ops.gemm_bf16(a.scaled, weight, out, accumulate, gated, checked=True, norm_in=norm_in, gate_limit=gate_limit,
-                                 counters=ops.step_counters(ctx, a.scaled.shape[0], *weight.shape, ops.product_kind(out, accumulate, gated, norm_in)))
+            return ops.gemm_bf16(a.scaled, weight, out, accumulate, gated, checked=True, norm_in=(a.squares, a.eps), gate_limit=gate_limit, ctx=ctx)
     if isinstance(a, NormedRows):
         a = a.materialize()
     if a.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and ops.gemm_bf16_supports(a, weight, out):
-        return ops.gemm_bf16(a, weight, out, accumulate, gated, checked=True, gate_limit=gate_limit,
-                             counters=ops.step_counters(ctx, a.shape[0], *weight.shape, ops.product_kind(out, accumulate, gated)))
+        return ops.gemm_bf16(a, weight, out, accumulate, gated, checked=True, gate_limit=gate_limit, ctx=ctx)
     if gated:
         raise ops.KernelError("the gated product exists for bfloat16 operands only")
     return ops.gemm_exact(a, weight, out, accumulate)
@@ -77,9 +74,7 @@ def linear_onto(a: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor, t
         if parts:
             scaled = torch.empty((rows, width), dtype=torch.bfloat16, device=residual.device)
             squares = torch.empty((rows, parts), dtype=torch.float32, device=residual.device)
-            norm_out = (then.handed_weight(), scaled, squares)
-            ops.gemm_bf16(a, weight, residual, accumulate=True, checked=True, norm_out=norm_out,
-                          counters=ops.step_counters(ctx, rows, *weight.shape, ops.product_kind(residual, True, norm_out=norm_out)))
+            ops.gemm_bf16(a, weight, residual, accumulate=True, checked=True, norm_out=(then.handed_weight(), scaled, squares), ctx=ctx)
             return HandedRows(then, residual, scaled, squares)
     linear(a, weight, residual, accumulate=True, ctx=ctx)
     return None

@@ -14,6 +14,8 @@ this saves the norm's kernel; `linear` decides where it applies, and `materializ
 rows the ordinary way."""
 from __future__ import annotations
 
+from functools import lru_cache
+
 import torch
 
 from ..kernels import ops
@@ -70,15 +72,16 @@ class NormToMake:
         self.norm = norm
 
 
-def _takes_norm_to_make(part) -> bool:
-    cls = next(c for c in type(part).__mro__ if "forward" in vars(c))
-    return bool(vars(cls).get("hands_whole_norms", False))
+@lru_cache(maxsize=256)
+def _takes_norm_to_make(cls) -> bool:
+    owner = next(c for c in cls.__mro__ if "forward" in vars(c))
+    return bool(vars(owner).get("hands_whole_norms", False))
 
 
 def norm_to_make(reader, part):
     """reader: as above.  The norm as `part`'s `then`, if the part may make it whole and its reader takes it so in bfloat16; None otherwise."""
     norm, reads = reader if reader is not None else (None, None)
-    if (not getattr(part, "hands_whole_norms", False) or not _takes_norm_to_make(part) or not hasattr(norm, "handed_weight") or not getattr(reads, "accepts_deferred_norm", False)
+    if (not getattr(part, "hands_whole_norms", False) or not _takes_norm_to_make(type(part)) or not hasattr(norm, "handed_weight") or not getattr(reads, "accepts_deferred_norm", False)
             or getattr(reads, "in_dtype", None) != torch.bfloat16):
         return None
     return NormToMake(norm)

@@ -1,9 +1,12 @@
 """The library's own rules at sizes on both sides of their lines, on 256 compute units (which it assumes where there is no GPU): which kernel
 makes a product of a prompt's rows, and which contexts the 32-bit attention shares out."""
+from types import SimpleNamespace
+
 import pytest
 import torch
 
 from geneinfer_amd.kernels import ops
+from geneinfer_amd.parts.linear import linear, linear_onto
 
 # m, n, k, what becomes of the sums -> the kernel that was the faster one there, by more than 4 %
 MEASURED = [
@@ -120,3 +123,23 @@ def test_no_room_for_scratch_is_no_error(monkeypatch):
     assert ops._room(5, "cpu").shape == (5,)
     monkeypatch.setattr(torch, "empty", full)
     assert ops._room(5, "cpu") is None
+
+
+def test_products_of_few_rows_ask_for_nothing_by_kind(monkeypatch):
+    for m, n, k in [(1, 3072, 2048), (17, 2048, 8192), (128, 16384, 2048), (128, 28672, 4096)]:
+        assert m <= ops.FEW_ROWS and len({ops._scratch_floats(m, n, k, kind, counted) for kind in range(len(ops.PRODUCT_KINDS)) for counted in (False, True)}) == 1
+        assert all(ops._shares(m, n, k, kind, True) == 1 for kind in range(len(ops.PRODUCT_KINDS)))
+    asked = []
+    for name in ("product_kind", "_shares"):
+        monkeypatch.setattr(ops, name, lambda *a, _inner=getattr(ops, name), _name=name, **k: (asked.append(_name), _inner(*a, **k))[1])
+    monkeypatch.setattr(ops, "_dev", lambda *tensors: None)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_call", lambda *a: None)
+    step = SimpleNamespace(memo={}, device="cpu")
+    bf16 = lambda *shape: torch.zeros(shape, dtype=torch.bfloat16)
+    for m in (1, 128):
+        linear(bf16(m, 2048), bf16(3072, 2048), torch.zeros(m, 3072), ctx=step)
+        linear_onto(bf16(m, 2048), bf16(2048, 2048), torch.zeros(m, 2048), None, step)
+    assert not asked and not step.memo
+    linear(bf16(2048, 8192), bf16(2048, 8192), torch.zeros(2048, 2048), accumulate=True, ctx=step)
+    assert asked and step.memo["product_counters"].numel() >= ops.lib().gi_gemm_bf16_counters()
