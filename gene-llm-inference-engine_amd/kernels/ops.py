@@ -1266,7 +1266,7 @@ class AttentionPlan:
         plan.n_decode, plan.n_tiles, plan.max_decode_context, plan.single_rows = n_rows, 0, max_context, True
         plan.decode_rows = None                                  # rows 0 .. n_rows-1
         plan.decode_positions = plan.tile_contexts = None
-        plan.tile_places, plan.walk_shares = [], {}
+        plan.tile_places, plan.walk_shares, plan.cuts = [], {}, {}
         plan.tiles = torch.empty(0, dtype=torch.int32, device=device)
         plan.n_tile_rows, plan.max_tile_context, plan.tile_first, plan.tile_rows, plan.paired, plan.tile = 0, 0, None, None, False, 128
         return plan
@@ -1300,7 +1300,7 @@ class AttentionPlan:
         self.n_tile_rows = sum(t[1] for t in tiles)
         self.tile_contexts = [t[2] + t[1] for t in tiles if t[1]]        # positions each tile of rows sees; None: of a step still to come
         self.tile_places = [(t[2], t[1], t[4]) for t in tiles]           # every tile's first position, its rows, the rows behind it in its portion
-        self.walk_shares = {}                                            # what `_walk_shares` found for the step's layers
+        self.walk_shares, self.cuts = {}, {}                             # what `_walk_shares`, `_prompt_cut` and `_single_cut` found for the step's layers
         self.max_tile_context = max(self.tile_contexts, default=0)
         # for sharing a tile's keys out over workgroups: rows before each tile, and the tiles' rows in order
         firsts, count = [], 0
@@ -1374,7 +1374,7 @@ def _walk_shares(plan, n_heads, hd, window, chunk, one_round):
     """`prompt_attention_shares` for the tiles of a plan, once a step for all layers of one kind.  A step still to come (a captured pass) is taken to reach the
     end of its bracket with every portion; at heads of 128 channels, and beyond one round, it shares nothing out (the shares of such tiles are fitted to the walks
     a step has, and a replay's can be half as long)."""
-    key = (n_heads, hd, window, chunk, one_round)
+    key = (plan.max_tile_context, plan.tile_contexts is None, n_heads, hd, window, chunk, one_round)
     if key not in plan.walk_shares:
         places = plan.tile_places
         if plan.tile_contexts is None:
@@ -1523,6 +1523,31 @@ def decode_attention_shape(n_decode, n_heads, n_kv, hd, span, target_waves=4096,
     return best or base
 
 
+def _prompt_cut(plan, n_heads, hd, window, chunk, seen, shares):
+    """(splits, floats of scratch, most shares, keys a share) for the tiles of a plan: the same for all layers of one kind, and kept by the plan."""
+    groups = plan.n_tiles // 2 if plan.paired else plan.n_tiles
+    n_splits = prompt_attention_splits(groups, n_heads, seen(plan.max_tile_context, plan.tile), target_groups=PAIRED_TARGET_GROUPS if plan.paired else 512)      # a pair's workgroup has twice the waves
+    if n_splits > 1:
+        return n_splits, plan.n_tile_rows * n_heads * n_splits * (hd + 2), 1, 0
+    if shares and hd in (64, 128) and plan.n_tiles * n_heads <= PROMPT_SHARE_COUNTERS // 2:
+        most, keys = _walk_shares(plan, n_heads, hd, window, chunk, groups * n_heads <= lib().gi_compute_units())
+        n_part = lib().gi_attention_prompt_share_floats(plan.n_tiles, plan.tile, n_heads, hd, 1, 1 if plan.paired else 0, most)
+        if n_part:
+            return 1, n_part, most, keys
+    return 1, 0, 1, 0
+
+
+def _single_cut(plan, n_heads, n_kv, hd, seen, target_waves, fused, orders):
+    """(splits, waves, whether the longest context comes first, floats of scratch) for the single rows of a plan, kept by the plan as well."""
+    span = seen(plan.max_decode_context, 31)
+    n_splits, n_waves = decode_attention_shape(plan.n_decode, n_heads, n_kv, hd, span, target_waves, fused)
+    groups = plan.n_decode * n_kv * ((n_heads // n_kv + 15) // 16)
+    if plan.decode_positions is not None and n_splits == 1 and not fused and span == plan.max_decode_context:
+        n_splits, n_waves = _decode_ragged_split(groups, span, plan.decode_positions / plan.n_decode, hd, n_waves)
+    ordered = orders and 16 < plan.n_decode <= 1024 and groups * n_splits > lib().gi_compute_units()
+    return n_splits, n_waves, ordered, plan.n_decode * n_heads * n_splits * (hd + 2) if n_splits > 1 else 0
+
+
 def attention_bf16(q, cache, out, plan: AttentionPlan, positions, slots, table, n_heads, n_kv, hd, window=None, scale=None,
                    target_waves: int = 4096, products=None, chunk=None, sinks=None, gate=None, cap=None, channel_gate=None, memo=None):
     """Attention of a step's rows with the matrix-core kernels (bfloat16 cache and out).  memo: what the pass keeps for its layers (the order of its rows).
@@ -1572,37 +1597,32 @@ def attention_bf16(q, cache, out, plan: AttentionPlan, positions, slots, table, 
             if not (t is None or (t.dtype == torch.float32 and t.shape == (n, hd // 2) and t.is_contiguous())):
                 raise KernelError("attention: cos/sin must be float32 [n, hd/2]")
     if plan.n_tiles:
-        n_splits = prompt_attention_splits(plan.n_tiles // 2 if plan.paired else plan.n_tiles, n_heads, seen(plan.max_tile_context, plan.tile),
-                                           target_groups=PAIRED_TARGET_GROUPS if plan.paired else 512)      # a pair's workgroup has twice the waves
-        n_part = plan.n_tile_rows * n_heads * n_splits * (hd + 2) if n_splits > 1 else 0
-        most, keys, counters = 1, 0, None
-        one_round = (plan.n_tiles // 2 if plan.paired else plan.n_tiles) * n_heads <= lib().gi_compute_units()
-        if n_splits == 1 and memo is not None and hd in (64, 128) and plan.n_tiles * n_heads <= PROMPT_SHARE_COUNTERS // 2:
-            most, keys = _walk_shares(plan, n_heads, hd, window, chunk, one_round)
-            n_part = lib().gi_attention_prompt_share_floats(plan.n_tiles, plan.tile, n_heads, hd, 1, 1 if plan.paired else 0, most)
-            part = _room(n_part, out.device) if n_part else None
+        key = (plan.max_tile_context, plan.tile_contexts is None, PAIRED_TARGET_GROUPS, n_heads, hd, window, chunk, memo is not None)
+        cut = plan.cuts.get(key)
+        if cut is None:
+            cut = plan.cuts[key] = _prompt_cut(plan, n_heads, hd, window, chunk, seen, memo is not None)
+        n_splits, n_part, most, keys = cut
+        part = counters = None
+        if most > 1:
+            part = _room(n_part, out.device)
             if part is not None:
                 counters = memo.get("attention_counters")
                 if counters is None:
                     counters = memo["attention_counters"] = torch.zeros(PROMPT_SHARE_COUNTERS, dtype=torch.int32, device=out.device)
             else:
                 most, keys, n_part = 1, 0, 0
-        else:
-            part = torch.empty(n_part, dtype=torch.float32, device=out.device) if n_part else None
+        elif n_part:
+            part = torch.empty(n_part, dtype=torch.float32, device=out.device)
         _call("gi_attention_prompt_bf16", q.data_ptr(), cache.data_ptr(), out.data_ptr(), plan.tiles.data_ptr(), plan.n_tiles, plan.tile,
               1 if plan.paired else 0, table.data_ptr(), table.stride(0), cache.stride(0), page_size, n_heads, n_kv, hd, window, scale, n_splits,
               _ptr(plan.tile_first), _ptr(plan.tile_rows), plan.n_tile_rows, _ptr(part), n_part, *extras, keys, most, _ptr(counters), _stream())
     if plan.n_decode:
-        span = seen(plan.max_decode_context, 31)
-        n_splits, n_waves = decode_attention_shape(plan.n_decode, n_heads, n_kv, hd, span, target_waves, products is not None)
-        groups = plan.n_decode * n_kv * ((n_heads // n_kv + 15) // 16)
-        if plan.decode_positions is not None and n_splits == 1 and products is None and span == plan.max_decode_context:
-            n_splits, n_waves = _decode_ragged_split(groups, span, plan.decode_positions / plan.n_decode, hd, n_waves)
-        rows = plan.decode_rows
-        ordered = memo is not None and 16 < plan.n_decode <= 1024 and groups * n_splits > lib().gi_compute_units()
-        if ordered:
-            rows = _decode_order(memo, plan, positions)
-        n_part = plan.n_decode * n_heads * n_splits * (hd + 2) if n_splits > 1 else 0
+        key = (plan.max_decode_context, plan.decode_positions, n_heads, n_kv, hd, window, chunk, target_waves, products is not None, memo is not None)
+        cut = plan.cuts.get(key)
+        if cut is None:
+            cut = plan.cuts[key] = _single_cut(plan, n_heads, n_kv, hd, seen, target_waves, products is not None, memo is not None)
+        n_splits, n_waves, ordered, n_part = cut
+        rows = _decode_order(memo, plan, positions) if ordered else plan.decode_rows
         part = torch.empty(n_part, dtype=torch.float32, device=out.device) if n_part else None
         _call("gi_attention_decode_bf16", _ptr(q), _ptr(qf), _ptr(kf), _ptr(vf), qf.stride(0) if qf is not None else 0,
               kf.stride(0) if kf is not None else 0, vf.stride(0) if vf is not None else 0, _ptr(cos), _ptr(sin), cache.data_ptr(),
@@ -1736,8 +1756,7 @@ def _shares(m, n, k, kind, counted) -> int:
     return lib().gi_gemm_bf16_shares(m, n, k, kind, 1 if counted else 0)
 
 
-# Rows up to which a product's scratch depends on its sizes alone and no tile is shared out: decoding asks for nothing else on the way to each launch (the kind, the
-# shares and the scratch by kind took 1 us of the host's 10 to 20 a product).
+# Rows up to which a product's scratch depends on its sizes alone and no tile is shared out: decoding asks for nothing else on the way to each launch.
 FEW_ROWS = 128
 
 
@@ -1747,7 +1766,7 @@ def _product_scratch(m, n, k, kind, counted, device):
     floats = _scratch_floats(m, n, k, kind, counted)
     if not floats:
         return None, 0
-    if m > FEW_ROWS and _shares(m, n, k, kind, counted) > 1:
+    if _shares(m, n, k, kind, counted) > 1:
         scratch = _room(floats, device)
         return scratch, floats if scratch is not None else 0
     return torch.empty(floats, dtype=torch.float32, device=device), floats
@@ -1765,7 +1784,8 @@ def step_counters(ctx, m, n, k, kind=0):
 
 
 def _check_counters(counters):
-    if counters is not None and not (counters.dtype == torch.int32 and counters.is_contiguous() and counters.numel() >= lib().gi_gemm_bf16_counters()):
+    _dev(counters)
+    if not (counters.dtype == torch.int32 and counters.is_contiguous() and counters.numel() >= lib().gi_gemm_bf16_counters()):
         raise KernelError("gemm: the counters must be int32, as many as gi_gemm_bf16_counters says, contiguous")
 
 
@@ -1794,8 +1814,9 @@ def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=N
     [m, gemm_bf16_norm_parts(m, n, k)] = the pieces of the rows' sums of out^2;
     norm_in = (squares, eps): a is such a `scaled`, and the results are multiplied by rsqrt(sum of the row's pieces / k + eps).
     counters: see `step_counters`; the product clears its own where it needs them and has none.  ctx: the step whose counters it may take, where none are given."""
-    _dev(a, w, out, counters)
-    _check_counters(counters)
+    _dev(a, w, out)
+    if counters is not None:
+        _check_counters(counters)
     m, k = a.shape
     n = w.shape[0]
     if not (w.shape == (n, k)):
@@ -1804,10 +1825,14 @@ def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=N
         raise KernelError(f"gemm: out is {tuple(out.shape)}, ({m}, {n // 2 if gated else n}) is needed")
     if not (checked or gemm_bf16_supports(a, w, out)):
         raise KernelError("gemm_bf16: operands must be bfloat16 with K and row strides multiples of 8, 16-byte aligned")
-    kind = product_kind(out, accumulate, gated, norm_in, norm_out) if m > FEW_ROWS else 0
-    if counters is None:
-        counters = step_counters(ctx, m, n, k, kind)
-    scratch, n_scratch = _product_scratch(m, n, k, kind, counters is not None, a.device)
+    if m <= FEW_ROWS:
+        n_scratch = _scratch_floats(m, n, k, 0, False)
+        scratch = torch.empty(n_scratch, dtype=torch.float32, device=a.device) if n_scratch else None
+    else:
+        kind = product_kind(out, accumulate, gated, norm_in, norm_out)
+        if counters is None:
+            counters = step_counters(ctx, m, n, k, kind)
+        scratch, n_scratch = _product_scratch(m, n, k, kind, counters is not None, a.device)
     if gated and gated is not True and gated not in ACTIVATIONS:
         raise KernelError(f"gemm: unknown activation {gated!r} of a gated product; known: {', '.join(ACTIVATIONS)}")
     gate_code = 0 if not gated else 1 + (0 if gated is True else ACTIVATIONS[gated])        # 1: SiLU, 2: GELU (tanh form)
@@ -1841,13 +1866,13 @@ def gemm_bf16_onto_norm_takes(m, n, k) -> bool:
     return bool(lib().gi_gemm_bf16_onto_norm_takes(m, n, k))
 
 
-def gemm_bf16_onto_norm(a, w, x, g, eps, normed):
+def gemm_bf16_onto_norm(a, w, x, g, eps, normed, checked=False):
     """x += a @ w.T onto float32 rows, and normed = bfloat16(g * (x * rsqrt(mean(x^2) + eps))), as `rmsnorm` makes it of the new rows, in the kernel that adds
-    the shares of k up."""
+    the shares of k up.  checked: the caller has asked `gemm_bf16_supports` and `gemm_bf16_onto_norm_takes`."""
     _dev(a, w, x, g, normed)
     m, k = a.shape
     n = w.shape[0]
-    if not (w.shape == (n, k) and x.shape == (m, n) and gemm_bf16_supports(a, w, x) and x.dtype == torch.float32 and gemm_bf16_onto_norm_takes(m, n, k)
+    if not (w.shape == (n, k) and x.shape == (m, n) and x.dtype == torch.float32 and (checked or (gemm_bf16_supports(a, w, x) and gemm_bf16_onto_norm_takes(m, n, k)))
             and g.dtype == torch.float32 and g.shape == (n,) and g.is_contiguous() and normed.dtype == torch.bfloat16 and normed.shape == (m, n) and normed.stride(1) == 1):
         raise KernelError("gemm_bf16_onto_norm: bfloat16 operands, float32 rows [m, n] and weights [n], bfloat16 [m, n] for the normed rows, and sizes that are taken")
     n_scratch = _scratch_floats(m, n, k, 1, False)
@@ -1906,12 +1931,13 @@ def gemm_bf16_qkv_rope_store_max_parts(m, n, k) -> int:
     return lib().gi_gemm_bf16_qkv_rope_store_max_parts(m, n, k)
 
 
-def gemm_bf16_qkv_rope_store(a, w, cos, sin, positions, slots, table, q_out, cache, n_heads, n_kv, hd, norm_in=None, counters=None):
+def gemm_bf16_qkv_rope_store(a, w, cos, sin, positions, slots, table, q_out, cache, n_heads, n_kv, hd, norm_in=None, counters=None, ctx=None):
     """The q/k/v product a @ w.T of an attention layer whose results do not come back: the queries go, rotated, into q_out
     (bfloat16 [m, heads*hd]), the keys (rotated) and the values into the cache's pages, as `rope_store` puts them.
-    cos, sin: float32 [m, hd/2] or None; norm_in as for `gemm_bf16`."""
-    _dev(a, w, cos, sin, positions, slots, table, q_out, cache, counters)
-    _check_counters(counters)
+    cos, sin: float32 [m, hd/2] or None; norm_in, counters and ctx as for `gemm_bf16`."""
+    _dev(a, w, cos, sin, positions, slots, table, q_out, cache)
+    if counters is not None:
+        _check_counters(counters)
     m, k = a.shape
     n = w.shape[0]
     if not (gemm_bf16_supports(a, w, q_out) and w.shape == (n, k) and n == (n_heads + 2 * n_kv) * hd and gemm_bf16_qkv_rope_store_takes(m, n, k, hd)):
@@ -1929,7 +1955,13 @@ def gemm_bf16_qkv_rope_store(a, w, cos, sin, positions, slots, table, q_out, cac
     squares_in, eps = norm_in if norm_in is not None else (None, 0.0)
     if squares_in is not None and not (squares_in.dtype == torch.float32 and squares_in.is_contiguous() and squares_in.dim() == 2 and squares_in.shape[0] == m):
         raise KernelError("gemm: the pieces of the sums of squares must be float32 [m, pieces]")
-    scratch, n_scratch = _product_scratch(m, n, k, 5, counters is not None, a.device)
+    if m <= FEW_ROWS:
+        n_scratch = _scratch_floats(m, n, k, 0, False)
+        scratch = torch.empty(n_scratch, dtype=torch.float32, device=a.device) if n_scratch else None
+    else:
+        if counters is None:
+            counters = step_counters(ctx, m, n, k, 5)
+        scratch, n_scratch = _product_scratch(m, n, k, 5, counters is not None, a.device)
     if _profile is not None:
         _profile.note = (f"{n}x{k}", n * k * w.element_size())
     _call("gi_gemm_bf16_qkv_rope_store", a.data_ptr(), w.data_ptr(), m, n, k, a.stride(0), w.stride(0), _ptr(scratch), n_scratch,

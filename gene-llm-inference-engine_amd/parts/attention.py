@@ -54,7 +54,7 @@ def qkv_rotate_store_attend(h, w_qkv, ctx, cache, *, n_heads, n_kv_heads, head_d
         if ops.gemm_bf16_supports(rows, w_qkv, att):
             q_rot = torch.empty((T, a_dim), dtype=torch.bfloat16, device=ctx.device)
             ops.gemm_bf16_qkv_rope_store(rows, w_qkv, cos, sin, ctx.row_pos, ctx.row_slot, cache.table, q_rot, cache.kv, n_heads, n_kv_heads,
-                                         head_dim, norm_in, ops.step_counters(ctx, T, *w_qkv.shape, ops.PRODUCT_KINDS.index("rotated")))
+                                         head_dim, norm_in, ctx=ctx)
             return ops.attention(q_rot, cache.kv, att, ctx, cache.table, n_heads, n_kv_heads, head_dim, window)
         if norm_in is None:
             h = rows                  # (whole rows: what `linear` below would make of h)

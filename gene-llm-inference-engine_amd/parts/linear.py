@@ -62,10 +62,10 @@ def linear_onto(a: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor, t
     `NormToMake`, for a reader that takes no other than a whole one: the rows come back normed where the product's kernel can."""
     if isinstance(then, NormToMake):
         norm, n, k = then.norm, weight.shape[0], weight.shape[1]
-        if (a.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and residual.dtype == torch.float32 and residual.stride(0) % 4 == 0 and residual.data_ptr() % 16 == 0
-                and norm.handed_weight().data_ptr() % 16 == 0 and ops.gemm_bf16_supports(a, weight, residual) and ops.gemm_bf16_onto_norm_takes(residual.shape[0], n, k)):
+        if (a.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and residual.dtype == torch.float32 and ops.gemm_bf16_onto_norm_takes(residual.shape[0], n, k)
+                and residual.stride(0) % 4 == 0 and residual.data_ptr() % 16 == 0 and norm.handed_weight().data_ptr() % 16 == 0 and ops.gemm_bf16_supports(a, weight, residual)):
             normed = torch.empty(residual.shape, dtype=torch.bfloat16, device=residual.device)
-            return ReadyRows(norm, residual, ops.gemm_bf16_onto_norm(a, weight, residual, norm.handed_weight(), norm.eps, normed))
+            return ReadyRows(norm, residual, ops.gemm_bf16_onto_norm(a, weight, residual, norm.handed_weight(), norm.eps, normed, checked=True))
         then = None
     if (then is not None and a.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and residual.dtype == torch.float32
             and residual.is_contiguous() and ops.gemm_bf16_supports(a, weight, residual)):

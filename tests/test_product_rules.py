@@ -143,3 +143,32 @@ def test_products_of_few_rows_ask_for_nothing_by_kind(monkeypatch):
     assert not asked and not step.memo
     linear(bf16(2048, 8192), bf16(2048, 8192), torch.zeros(2048, 2048), accumulate=True, ctx=step)
     assert asked and step.memo["product_counters"].numel() >= ops.lib().gi_gemm_bf16_counters()
+
+
+def test_how_a_step_s_attention_is_cut_is_found_once_for_its_layers(monkeypatch):
+    asked = []
+    for name in ("_decode_ragged_split", "prompt_attention_splits"):
+        monkeypatch.setattr(ops, name, lambda *a, _inner=getattr(ops, name), _name=name, **k: (asked.append(_name), _inner(*a, **k))[1])
+    launched = []
+    monkeypatch.setattr(ops, "_dev", lambda *tensors: None)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_call", lambda name, *a: launched.append((name, a)))
+    n_single, heads, n_kv, hd, page = 24, 24, 8, 128, 16
+    lens, befores = [1] * n_single + [900], [400 + 110 * i for i in range(n_single)] + [64]
+    starts = list(range(n_single)) + [n_single]
+    plan = ops.AttentionPlan(starts, lens, befores, list(range(n_single + 1)), "cpu")
+    n = sum(lens)
+    q = torch.zeros(n, heads * hd, dtype=torch.bfloat16)
+    cache, table = torch.zeros(8, 2, n_kv, page, hd, dtype=torch.bfloat16), torch.zeros(n_single + 1, 256, dtype=torch.int32)
+    at = torch.zeros(n, dtype=torch.int32)
+    memo = {}
+    layer = lambda window: ops.attention_bf16(q, cache, torch.zeros_like(q), plan, at, at, table, heads, n_kv, hd, window=window, memo=memo)
+    for _ in range(3):
+        layer(None)
+    assert sorted(asked) == ["_decode_ragged_split", "prompt_attention_splits"]
+    layer(512)                                   # (another kind of layer: its own cut)
+    assert asked.count("prompt_attention_splits") == 2
+    plan.decode_positions = None                 # (a step still to come: nothing that was found of this one holds)
+    layer(None)
+    splits = [args[-10] for name, args in launched if name == "gi_attention_decode_bf16"]
+    assert splits[0] == splits[1] == splits[2] > 1 and splits[-1] == 1
