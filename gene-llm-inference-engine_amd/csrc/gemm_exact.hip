@@ -193,6 +193,12 @@ __global__ __launch_bounds__(256) void gemm_exact_tiled_kernel(const TA* __restr
 // The same for 32-bit operands whose rows are whole blocks of 32 k: the operands go from memory straight into LDS, a ring of three
 // stages with two in flight while one is multiplied (asked for and waited for as the bfloat16 ring kernel does), so a stage costs a
 // wave four loads and a barrier beside its matrix instructions.
+// What bounds it is how much of a wave's time the matrix instructions do not fill, wherever a compute unit has fewer than three workgroups.  So a half of a
+// stage is read from LDS while the half before it is multiplied, and the barrier that hands the next stage over lies between a stage's halves: behind it a wave
+// has 16 matrix instructions whose operands are in registers, under which the next stage's loads go out and its first half is read.  With reads, barrier
+// and loads at the beginning of a stage, ahead of its products, 301 rows of 16,384 x 2,048 (five tiles a unit: three together, then two) took 200 us,
+// 177 now, of 2,048 x 8,192 112 and 101, 600 of 2,048 x 2,048 59 and 55; where three workgroups share a unit all the time it makes no difference (600 rows
+// of 16,384 x 2,048 331 and 328, 120 to 133 TFLOP/s).  Two stages (five workgroups fit the LDS, but not the registers) or four are no faster.
 template <int BM, bool ACCUMULATE>
 __global__ __launch_bounds__(256) void gemm_exact_ring_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, float* __restrict__ part,
                                                              int M, int N, int K, long lda, long ldw, long ldc, int m_tiles, int n_tiles, int splits) {
@@ -229,43 +235,62 @@ __global__ __launch_bounds__(256) void gemm_exact_ring_kernel(const float* __res
     };
     f32x4 acc[TN * TM], t[3][TN * TM];
 #pragma unroll
-    for (int i = 0; i < STAGES - 1; ++i)
+    for (int i = 0; i < STAGES; ++i)
         if (s_begin + i < s_end) issue(s_begin + i, i);
     const int a_at[2] = {chunk_at(wm + r, g), chunk_at(wm + r, 4 + g)}, w_at[2] = {BM * BK + chunk_at(wn + r, g), BM * BK + chunk_at(wn + r, 4 + g)};
+    f32x4 a[2][TM], w[2][TN];
+    auto read_half = [&](int slot, int b) {                 // (rows 16 apart have the same permutation of chunks)
+        const float* stage = ring + slot * ROWS * BK;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) a[b][i] = *reinterpret_cast<const f32x4*>(stage + a_at[b] + i * 16 * BK);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) w[b][j] = *reinterpret_cast<const f32x4*>(stage + w_at[b] + j * 16 * BK);
+    };
+    auto multiply_half = [&](int b) {
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int i = 0; i < TM; ++i) acc[j * TM + i] = mfma(w[b][j][kk], a[b][i][kk], acc[j * TM + i]);
+    };
     int s = s_begin, slot = 0;
+    if (s < s_end) {
+        const int behind = min(s_end - s, STAGES) - 1;      // stages asked for behind the first
+        if (behind == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LOADS) : "memory");
+        else if (behind == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        read_half(0, 0);
+    }
     const int q_end = max(q0, min(q1, (s_end + per_range - 1) / per_range));              // (short k leaves ranges empty)
 #pragma unroll
     for (int i = 0; i < TN * TM; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int q = q0; q < q_end; ++q) {
 #pragma unroll
         for (int i = 0; i < TN * TM; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < TN * TM; ++i) asm volatile("" : "+v"(acc[i]));        // (four zeros, not one in four places: the compiler else moves the sums about in every stage)
         const int stop = min((q + 1) * per_range, s_end);
         for (; s < stop; ++s) {
-            if (s + 1 < s_end) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");        // this wave's part of stage s has landed
-            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __builtin_amdgcn_s_barrier();                                                          // everyone's has, and everyone has read stage s - 1
-            asm volatile("" ::: "memory");
-            if (s + STAGES - 1 < s_end) issue(s + STAGES - 1, slot == 0 ? STAGES - 1 : slot - 1);      // into the place of stage s - 1
-            const float* stage = ring + slot * ROWS * BK;
+            read_half(slot, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply_half(0);
+            __builtin_amdgcn_sched_barrier(0);
+            const int here = slot;
             slot = slot + 1 == STAGES ? 0 : slot + 1;
-            f32x4 a[2][TM], w[2][TN];
-            // (rows 16 apart have the same permutation of chunks)
-#pragma unroll
-            for (int b = 0; b < BK / 16; ++b) {
-#pragma unroll
-                for (int i = 0; i < TM; ++i) a[b][i] = *reinterpret_cast<const f32x4*>(stage + a_at[b] + i * 16 * BK);
-#pragma unroll
-                for (int j = 0; j < TN; ++j) w[b][j] = *reinterpret_cast<const f32x4*>(stage + w_at[b] + j * 16 * BK);
+            __builtin_amdgcn_s_waitcnt(0xc07f);                // lgkmcnt(0), in a form that the compiler counts with: this wave's reads of stage s are done
+            if (s + 1 < s_end) {
+                if (s + 2 < s_end) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");        // its part of stage s + 1 has landed
+                else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __builtin_amdgcn_s_barrier();                                                  // everyone's
+                asm volatile("" ::: "memory");
+                read_half(slot, 0);
+                if (s + STAGES < s_end) issue(s + STAGES, here);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            __builtin_amdgcn_sched_barrier(0);             // (the second half's operands arrive while the first half is multiplied)
-#pragma unroll
-            for (int b = 0; b < BK / 16; ++b)
-#pragma unroll
-                for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-#pragma unroll
-                        for (int i = 0; i < TM; ++i) acc[j * TM + i] = mfma(w[b][j][kk], a[b][i][kk], acc[j * TM + i]);
+            multiply_half(1);
         }
         fold(q - q0, acc, t);
     }
@@ -438,8 +463,8 @@ struct Cut { int bm, m_tiles, n_tiles, splits; };
 
 // Tiles of 64 rows, or of 32 where those hold at least a tenth fewer rows beyond M.  The ranges of k go to 1, 2, 4 or 8 workgroups: what
 // counts is the compute unit with the most of them (they share its matrix cores, and reach about half, two thirds and 0.72 of its 0.6
-// TFLOP/s when there are one, two and three or more), against writing and reading the parts.  301 rows of 2,048 x 2,048 (160 tiles): 50
-// us with one workgroup a tile, 41 with four.
+// TFLOP/s when there are one, two and three or more), against writing and reading the parts.  301 rows of 2,048 x 2,048 (160 tiles): 42
+// us with one workgroup a tile, 35 with four.  Of 54 products of 17 to 600 rows it takes the fastest cut or one within 6 %, but for four (9 to 11 %).
 Cut cut_for(int M, int N, int K) {
     const int units = gi_compute_units();
     Cut c;
