@@ -1,7 +1,7 @@
 // C[m, n] (=|+=) sum_k A[m, k] * W[n, k] with bfloat16 operands on the matrix cores, 32-bit sums.
 //
 // Both operands are row-major with k contiguous, so each lane's operand of a matrix instruction is
-// one 16-byte load of 8 consecutive k.  Six kernels:
+// one 16-byte load of 8 consecutive k.  Seven kernels:
 //
 //   pingpong  large prompt-sized products (256 x 256 tiles for most of the compute units): operands loaded
 //           from global memory straight into LDS, two stages of A and three of W; the workgroup's eight waves form two
@@ -12,10 +12,11 @@
 //           blocks of k in flight; v_mfma_f32_32x32x16_bf16.
 //   tiled   the other shapes above 64 rows: a BM x 128 tile of C per workgroup of 4 waves,
 //           operands staged through registers into LDS in k-blocks of 64.
-//   skinny  up to 128 rows of A: weights stream from HBM straight into registers and are used
-//           once, activations go through LDS; v_mfma_f32_16x16x32_bf16.  Wide outputs are
-//           finished by the workgroup that sees all of k; for narrow ones k is split over
-//           workgroups and the partial sums are added in a fixed order by a second kernel.
+//   strips  up to 256 rows of A (K a multiple of 64): 64 rows of weights and all rows of A a workgroup, both
+//           straight into a ring of LDS stages.  Wide outputs are finished by the workgroup that sees all of k;
+//           for narrow ones k is split over workgroups and the partial sums are added in a fixed order by a second kernel.
+//   skinny  the other shapes of up to 128 rows: weights stream from HBM straight into registers and are used
+//           once, activations go through LDS; v_mfma_f32_16x16x32_bf16.  Wide and narrow outputs likewise.
 //   slim    at most 16 rows of A (decode): a workgroup of 8 waves owns 16 (or 2 x 16) weight
 //           rows, its waves take interleaved blocks of k and add their sums through LDS in a
 //           fixed order, so one launch does the whole product and its epilogue.
@@ -1253,19 +1254,16 @@ constexpr int REDUCE_COLUMNS = 1024, REDUCE_MAX_PARTS = 8;
 // before the use.  With many pieces (the writer was a kernel for at most 32 rows with a piece per workgroup: at most
 // TILES_MAX_PARTS for 17 to 32 rows, slim_max_parts for fewer) 16 or 32 threads share a row and ask for 16 pieces each at once.
 constexpr int TILES_MAX_PARTS = 256;
-__device__ __forceinline__ void row_scales_into(float* scales, const NormIn& n, int M) {
-    const int tid = threadIdx.x;
-    if (n.parts <= REDUCE_MAX_PARTS) {
-        if (tid < M) scales[tid] = row_scale_of(n, tid);
-        return;
-    }
-    const int sharing = M <= 16 ? 32 : 16, row = tid / sharing, at = tid % sharing;        // M <= 32 here
-    float piece[16];
+__device__ __forceinline__ void row_pieces_shared(const NormIn& n, int M, int sharing, float (&piece)[16]) {
+    const int row = threadIdx.x / sharing, at = threadIdx.x % sharing;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const int p = at + sharing * i;
         piece[i] = (row < M && p < n.parts) ? n.squares[(size_t)row * n.parts + p] : 0.f;
     }
+}
+__device__ __forceinline__ void row_scales_shared(float* scales, const NormIn& n, int M, int sharing, const float (&piece)[16]) {
+    const int row = threadIdx.x / sharing, at = threadIdx.x % sharing;
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) sum += piece[i];
@@ -1273,6 +1271,17 @@ __device__ __forceinline__ void row_scales_into(float* scales, const NormIn& n, 
 #pragma unroll
     for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
     if (at == 0 && row < M) scales[row] = 1.0f / sqrtf(sum / (float)n.dim + n.eps);
+}
+__device__ __forceinline__ void row_scales_into(float* scales, const NormIn& n, int M) {
+    const int tid = threadIdx.x;
+    if (n.parts <= REDUCE_MAX_PARTS) {
+        if (tid < M) scales[tid] = row_scale_of(n, tid);
+        return;
+    }
+    const int sharing = M <= 16 ? 32 : 16;                                                 // M <= 32 here
+    float piece[16];
+    row_pieces_shared(n, M, sharing, piece);
+    row_scales_shared(scales, n, M, sharing, piece);
 }
 
 template <int MT, int EPI, bool PARTIAL>
@@ -1400,6 +1409,187 @@ __global__ __launch_bounds__(512, MT == 2 ? 4 : 2) void gemm_bf16_skinny_kernel(
                 if constexpr (PARTIAL) P[((size_t)blockIdx.y * M + m) * N + n] = acc[t][v];
                 else write_out<EPI>(C, (size_t)m * ldc + n, scaled_rows ? acc[t][v] * row_scale[m] : acc[t][v]);
             }
+    }
+}
+
+// ------------------------------------------------------------------------------------------ strips
+// All rows of A (up to 32 TM of them) against 64 rows of W and the k range of the workgroup's grid row: both operands go from memory straight into
+// a ring of LDS stages of 64 k (chunks placed as in the kernels above), STAGES - 1 of them in flight.  Eight waves: two halves of 32
+// columns times four quarters of every stage's k, so that a wave's one fragment of weights meets all rows and a fragment of rows is read by two waves only; the
+// quarters' sums meet in LDS, (0 + 2) + (1 + 3).  A wave reads the next stage's operands while it multiplies this one's.
+// Bound by the weights on their way from memory (a strip of 64 rows gives 256 workgroups 28 to 56 KB each of them in flight), and from 100 rows or so on by what
+// a unit takes in of A besides: one tile for all rows reads the weights once, where 131 rows in two tiles of 128 had half of the units load them for three rows.  Microseconds
+// in a captured chain, before (weights through registers up to 128 rows, tiles of 128 x 128 above; where k is shared out with the kernel that adds up) and now:
+//   rows                     17            64            128           131           192
+//   16,384 x 2,048 gated     18.2, 17.1    22.4, 19.5    30.7, 24.7    31.0, 25.6    31.9, 29.0
+//   28,672 x 4,096 gated     53.5, 46.8    65.4, 55.5    93.2, 71.7    (as before)
+//   2,048 x 2,048 added      (other)       10.7, 8.8     14.4, 12.4    14.8, 13.0    17.2, 14.9
+//   2,048 x 8,192 added      13.9, 12.8    15.8, 14.5    20.0, 19.2    24.5, 19.9    26.0, 22.4
+//   3,072 x 8,192 added      19.1, 16.7    22.0, 19.0    28.6, 24.4    38.6, 25.2    41.0, 29.0
+//   4,096 x 14,336 added     28.6, 27.5    35.1, 32.9    46.0, 42.9    61.5, 43.7    63.9, 50.4
+//   128,256 x 2,048 stored   107.5, 102.2  130, 122      182, 150
+// The sums of a product have fewer and longer chains than before; against 64 bits they are nearer (2,048 x 8,192: 1.1e-7 for 1.4 to 1.9e-7).
+constexpr int strip_ring(int tm, int stages) { return stages * (64 + 32 * tm) * 128; }
+constexpr int strip_chunk(int tm, int stages) { return strip_ring(tm, stages) / 32768 < tm ? strip_ring(tm, stages) / 32768 : tm; }       // fragments whose quarters' sums fit the ring
+constexpr int strip_bytes(int tm, int stages) {
+    const int end = strip_chunk(tm, stages) * 32768 + (tm <= 4 ? 32 * tm * 4 : 0);
+    return strip_ring(tm, stages) > end ? strip_ring(tm, stages) : end;
+}
+template <int TM, int STAGES, int EPI, bool PARTIAL>
+__global__ __launch_bounds__(512, TM <= 2 ? 4 : 2) void gemm_bf16_strip_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ C,
+                                                                              float* __restrict__ P, int M, int N, int K, long lda, long ldw, long ldc, int k_per_split, NormIn norm_in) {
+    constexpr int BM = 32 * TM, STAGE_BYTES = (64 + BM) * 128, CHUNK = strip_chunk(TM, STAGES);
+    extern __shared__ __attribute__((aligned(16))) unsigned char ring[];               // strip_bytes(TM, STAGES)
+    float* const row_scale = reinterpret_cast<float*>(ring + CHUNK * 32768);            // (behind the sums of the end)
+    const bool scaled_rows = TM <= 4 && !PARTIAL && norm_in.squares != nullptr;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // The pieces of the rows' sums of squares: asked for ahead of everything, used at the end.  Up to 32 rows they may be many (`row_scales_into`).
+    constexpr int EACH = TM == 1 ? 16 : 1;
+    const int sharing = M <= 16 ? 32 : 16;
+    [[maybe_unused]] RowPieces pieces;
+    [[maybe_unused]] float piece[EACH];
+    if constexpr (TM == 1) {
+        if (scaled_rows) row_pieces_shared(norm_in, M, sharing, piece);
+    } else {
+        if (scaled_rows && tid < M) pieces = row_pieces(norm_in, tid);
+    }
+    const int half = wave & 1, quarter = wave >> 1, n0 = blockIdx.x * 64;
+    const int k_begin = blockIdx.y * k_per_split, n_k = (min(K, k_begin + k_per_split) - k_begin) / PK;
+    // A wave loads eight rows of W and every eighth group of eight rows of A; groups beyond M are left out (what then lies in LDS makes rows that nobody writes).
+    constexpr int MOST = (BM / 8 + 7) / 8;                                              // (M > BM - 32: a wave has so many groups, or one fewer)
+    const bool most = wave + 8 * (MOST - 1) < (M + 7) / 8;
+    const bf16_t *w_tile = W + (size_t)n0 * ldw + k_begin, *a_tile = A + k_begin;
+    unsigned w_src, a_src[MOST];
+    {
+        const int row = wave * 8 + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
+        w_src = (unsigned)(((size_t)min(row, N - 1 - n0) * ldw + 8 * c) * 2);
+#pragma unroll
+        for (int i = 0; i < MOST; ++i) {
+            const int r = row + 64 * i;
+            a_src[i] = (unsigned)(((size_t)min(r, M - 1) * lda + 8 * c) * 2);           // (rows 64 apart have the same permutation of chunks)
+        }
+    }
+    const unsigned ring_base = (unsigned)(size_t)(lds_ptr_t)ring;
+    auto issue = [&](int block, int slot) {
+        const unsigned at = ring_base + slot * STAGE_BYTES + wave * 1024;
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(w_src), "s"(w_tile + block * PK) : "memory", "m0");
+#pragma unroll
+        for (int i = 0; i < MOST; ++i)
+            if (i + 1 < MOST || most)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at + (64 + 64 * i) * 128), "v"(a_src[i]), "s"(a_tile + block * PK) : "memory", "m0");
+    };
+    // waits until at most the loads of so many stages are outstanding
+#define LOADS_OF(N_)                                                                                                                    \
+    do {                                                                                                                                \
+        if (most) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((N_) * (1 + MOST)) : "memory");                                              \
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((N_) * MOST) : "memory");                                                         \
+    } while (0)
+    auto wait = [&](int stages) {
+        static_assert(STAGES >= 3 && STAGES <= 8 && (STAGES - 1) * (1 + MOST) < 64, "waits for 0 to 7 stages");
+        if (stages >= STAGES - 1) LOADS_OF(STAGES - 1);
+        else if (stages == STAGES - 2) LOADS_OF(STAGES - 2);
+        else if (stages == 1) LOADS_OF(1);
+        else if (stages == 2) LOADS_OF(2);
+        else if (stages == 3) LOADS_OF(3);
+        else if (stages == 4) LOADS_OF(4);
+        else if (stages == 5) LOADS_OF(5);
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    };
+#undef LOADS_OF
+    floatx16 acc[TM];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) acc[i] = floatx16{};
+#pragma unroll
+    for (int s = 0; s < STAGES; ++s)
+        if (s < n_k) issue(s, s);
+    const int r = lane & 31, chunk = ((quarter * 2 + (lane >> 5)) ^ ((r >> 1) & 7)) * 16;
+    const unsigned char *w_at = ring + (half * 32 + r) * 128 + chunk, *a_at = ring + (64 + r) * 128 + chunk;
+    bf16x8 w[2], a[2][TM];
+    auto read = [&](int slot, int into) {
+        w[into] = as_bf16x8(*reinterpret_cast<const uint4*>(w_at + slot * STAGE_BYTES));
+#pragma unroll
+        for (int i = 0; i < TM; ++i) a[into][i] = as_bf16x8(*reinterpret_cast<const uint4*>(a_at + slot * STAGE_BYTES + i * 32 * 128));
+    };
+    auto meet = [&]() {
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    wait(min(n_k, STAGES) - 1);
+    meet();
+    read(0, 0);
+    int slot = 0;
+    auto step = [&](int it, int now) __attribute__((always_inline)) {
+        const int here = slot;
+        slot = slot + 1 == STAGES ? 0 : slot + 1;
+        __builtin_amdgcn_s_waitcnt(0xc07f);                                             // lgkmcnt(0), in a form that the compiler counts with: this wave has read stage `it`
+        if (it + 1 < n_k) {
+            if (it + STAGES <= n_k) wait(STAGES - 2);                                   // its part of stage it + 1 has landed
+            else wait(n_k - 2 - it);
+            meet();                                                                     // everyone's; everyone has read stage `it`
+            read(slot, now ^ 1);
+            if (it + STAGES < n_k) issue(it + STAGES, here);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[now][i], w[now], acc[i], 0, 0, 0);
+    };
+    for (int it = 0; it < n_k; it += 2) {
+        step(it, 0);
+        if (it + 1 < n_k) step(it + 1, 1);
+    }
+    // Element v of a lane's 32x32 result: row 8*(v/4) + 4*(lane/32) + v%4, column lane%32.  CHUNK fragments of rows at a time.
+    float4* const sums = reinterpret_cast<float4*>(ring);                               // [quarter][half][fragment][v / 4][lane]
+    auto at = [&](int of_quarter, int of_half, int f, int vg, int of_lane) { return (((of_quarter * 2 + of_half) * CHUNK + f) * 4 + vg) * 64 + of_lane; };
+    auto sum_of = [&](int of_half, int f, int vg, int of_lane) {
+        const float4 s0 = sums[at(0, of_half, f, vg, of_lane)], s1 = sums[at(1, of_half, f, vg, of_lane)], s2 = sums[at(2, of_half, f, vg, of_lane)], s3 = sums[at(3, of_half, f, vg, of_lane)];
+        return float4{(s0.x + s2.x) + (s1.x + s3.x), (s0.y + s2.y) + (s1.y + s3.y), (s0.z + s2.z) + (s1.z + s3.z), (s0.w + s2.w) + (s1.w + s3.w)};
+    };
+#pragma unroll
+    for (int first = 0; first < TM; first += CHUNK) {
+        __syncthreads();
+        if (first == 0 && scaled_rows) {
+            if constexpr (TM == 1) row_scales_shared(row_scale, norm_in, M, sharing, piece);
+            else if (tid < M) row_scale[tid] = row_scale_from(norm_in, tid, pieces);
+        }
+#pragma unroll
+        for (int f = 0; f < CHUNK; ++f)
+            if (first + f < TM) {
+#pragma unroll
+                for (int vg = 0; vg < 4; ++vg) {
+                    const floatx16& from = acc[first + f < TM ? first + f : 0];
+                    sums[at(quarter, half, f, vg, lane)] = float4{from[4 * vg], from[4 * vg + 1], from[4 * vg + 2], from[4 * vg + 3]};
+                }
+            }
+        __syncthreads();
+        const int here = min(CHUNK, TM - first);
+        if constexpr (is_gated(EPI) && !PARTIAL) {
+            // columns 0 .. 15 of a half are gates, 16 .. 31 the ups of the same outputs
+            for (int e = wave; e < here * 4; e += 8) {
+                const int f = e >> 2, vg = e & 3, o = lane & 31, from = (o & 15) + (lane & 32), row = (first + f) * 32 + 8 * vg + 4 * (lane >> 5);
+                const float4 g = sum_of(o >> 4, f, vg, from), u = sum_of(o >> 4, f, vg, from + 16);
+                const float gs[4] = {g.x, g.y, g.z, g.w}, us[4] = {u.x, u.y, u.z, u.w};
+                if (n0 + (o >> 4) * 32 >= N) continue;
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (row + v < M) {
+                        const float rs = scaled_rows ? row_scale[row + v] : 1.0f;
+                        ((bf16_t*)C)[(size_t)(row + v) * ldc + n0 / 2 + o] = f32_to_bf16(gate_of<EPI>(gs[v] * rs, us[v] * rs, norm_in.limit));
+                    }
+            }
+        } else {
+            for (int e = wave; e < here * 8; e += 8) {
+                const int f = e >> 3, vg = e & 3, of_half = (e >> 2) & 1, n = n0 + of_half * 32 + (lane & 31), row = (first + f) * 32 + 8 * vg + 4 * (lane >> 5);
+                const float4 s = sum_of(of_half, f, vg, lane);
+                const float ss[4] = {s.x, s.y, s.z, s.w};
+                if (n >= N) continue;
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (row + v < M) {
+                        if constexpr (PARTIAL) P[((size_t)blockIdx.y * M + row + v) * N + n] = ss[v];
+                        else write_out<EPI>(C, (size_t)(row + v) * ldc + n, scaled_rows ? ss[v] * row_scale[row + v] : ss[v]);
+                    }
+            }
+        }
     }
 }
 
@@ -2062,9 +2252,33 @@ static LargeChoice large_kernel_of_kind(int M, int N, int K, int kind, bool coun
 }
 static bool takes_large(int M, int N, int K) { return M > SKINNY_MAX_ROWS && K % PK == 0 && N >= 128; }
 
+// Whether the strips' kernel makes a product; `whole`: with all of k in a workgroup, which ends it, else k is shared out.  Above 128 rows the tiles of 128 x 128 are the better ones
+// where the strips do not fit one round (160 rows of 28,672 x 4,096 gated: 75 us and 82) or leave half of the units without one (10,240 x 2,048: 26.2 and 27.3), and above 192
+// rows where k is short (256 rows of 2,048 x 2,048 18.8 and 18.1, of 3,072 x 2,048 20.9 and 21.3, 200 of 2,048 x 1,024 12.6 and 13.6).
+constexpr int STRIP_MAX_ROWS = 256;
+static bool strips_take(int M, int N, int K, bool whole) {
+    if (K % PK != 0 || M > STRIP_MAX_ROWS) return false;
+    if (M <= SKINNY_MAX_ROWS) return true;
+    const int strips = (N + 63) / 64, units = gi_compute_units();
+    return whole ? M <= 192 && strips <= units : 2 * strips <= units && (M <= 192 || K > 8 * M);
+}
+static bool strip_strides(long lda, long ldw) { return lda < (1L << 22) && ldw < (1L << 22); }       // (a tile's rows within 32-bit offsets)
+// Shares of k: as many as there are units for, with at least 512 of k each (64 rows of 2,048 x 2,048, 32 strips: 9.1 us in four, 10.3 in eight; of 2,048 x 8,192 14.5
+// in eight, 18.4 in four; of 5,120 x 3,072, 80 strips, 13.9 in three, 16.4 in four and 15.3 in two).
+static int strip_splits(int M, int N, int K) {
+    const int strips = (N + 63) / 64, units = gi_compute_units(), most = 2 * strips <= units ? units / strips : M <= 64 ? 2 : 1;
+    return most < K / 512 ? most : K / 512 > 0 ? K / 512 : 1;
+}
+// The most shares of k that a product may be cut into, which the kernels beside the strips' cut into `splits` (0: none).
+static int shared_out(int M, int N, int K, int splits) {
+    if (splits == 0 || !strips_take(M, N, K, false)) return splits;
+    const int strips = strip_splits(M, N, K);
+    return strips > splits ? strips : splits;
+}
+
 // By how many workgroups each tile of the last round of a product is made that has all the scratch it asks for (1: one), with or without counters.
 GI_API int gi_gemm_bf16_shares(int M, int N, int K, int kind, int counters) {
-    if (!takes_large(M, N, K) || gi_gemm_bf16_piped_splits(M, N, K) > 1) return 1;
+    if (!takes_large(M, N, K) || gi_gemm_bf16_piped_splits(M, N, K) > 1 || (kind == 3 && strips_take(M, N, K, true))) return 1;
     const LargeChoice choice = large_kernel_of_kind(M, N, K, kind, counters != 0);
     return choice.kernel == TALL_256 ? choice.cut.shares : 1;
 }
@@ -2072,9 +2286,9 @@ GI_API int gi_gemm_bf16_shares(int M, int N, int K, int kind, int counters) {
 // Floats of scratch a product of these sizes and kind asks for (partial sums where k is shared out), 0 if none.  It does without where gi_gemm_bf16_shares says
 // more than one: the kernels that share nothing out serve then.
 GI_API long gi_gemm_bf16_scratch_floats(int M, int N, int K, int kind, int counters) {
-    if (M <= SKINNY_MAX_ROWS) return (long)gi_gemm_bf16_skinny_splits(N, K) * M * N;
+    if (M <= SKINNY_MAX_ROWS) return (long)shared_out(M, N, K, gi_gemm_bf16_skinny_splits(N, K)) * M * N;
     const int splits = gi_gemm_bf16_piped_splits(M, N, K);
-    if (splits > 1) return (long)splits * M * N;
+    if (splits > 1) return (long)shared_out(M, N, K, splits) * M * N;
     return gi_gemm_bf16_shares(M, N, K, kind, counters) > 1 ? tall_scratch_floats(large_kernel_of_kind(M, N, K, kind, counters != 0).cut) : 0;
 }
 
@@ -2111,17 +2325,23 @@ static int reduce_partials(const float* scratch, void* C, int epi, int M, int N,
 }
 
 // Up to 16 rows the slim kernel (no LDS staging, one launch) is the faster one, except for wide outputs with more
-// than a few rows, where its per-workgroup reading of the activations costs more than the skinny kernel's staging
-// (measured crossovers, whole decode steps: 12 rows for 256 strips of 64 columns at K = 2048, 8 to 9 rows for 256 strips at
-// K = 3072, 3 rows for 448 strips at K = 4096, where the 8B shape's step lost 3 to 5 % at 6 to 10 rows with the crossover at 12;
-// 5 rows for the 2004 strips of the vocabulary at K = 2048): the longer the rows and the more strips, the sooner, as
-// 12 * (2048 / K) * (256 / strips), between 3 and 12.
-static bool takes_slim(int M, int N, int K) {
-    const int strips64 = (N + 63) / 64;
+// than a few rows, where its per-workgroup reading of the activations costs more than staging them.  Beside the strips' kernel that is so from 8 rows on (16,384 x 2,048
+// gated with a norm: 17.8 and 18.3 us at 6 rows, 18.6 and 18.3 at 8, 21.5 and 18.4 at 16), from 6 for longer rows (22,016 x 4,096: 43.3 and 41.0 at 8), from 10 for
+// short rows and several rounds of strips (24,576 x 1,024: 13.3 and 13.1), from 5 for a vocabulary (128,256 x 2,048: 92.4 and 95.9 at 4, 101.6 and 96.4 at 6); and always where the strips fill one round
+// of workgroups incompletely (12,288 x 2,048: 15.0 and 13.8 at 1 row, 18.8 and 14.3 at 16) or long rows' rounds well (28,672 x 4,096: 49.3 and 46.0 at 1, 55.1 and 45.7 at 8).
+// Where the skinny kernel is the other one (K no multiple of 64, measured at the time at K = 2,048 to 4,096) the longer the rows and the more strips, the sooner, between 3 and 12.
+// xielu: the product ends through that activation, which of the two only the slim kernel has.
+static bool takes_slim(int M, int N, int K, bool xielu = false) {
+    const int strips64 = (N + 63) / 64, units = gi_compute_units();
+    if (M > 16 || gi_gemm_bf16_skinny_splits(N, K) > 0) return M <= 16;
+    if (strips64 >= 1024) return M < 5;
+    if (K % PK == 0 && !xielu) {
+        const double filled = (double)strips64 / ((strips64 + units - 1) / units * units);
+        if (strips64 * 5 <= units * 4 || (K >= 3072 && filled >= 0.85)) return false;
+        return M < (K > 2048 ? 6 : K > 1024 || strips64 <= units ? 8 : 10);
+    }
     const double fitted = 12.0 * (2048.0 / K) * (256.0 / strips64);
-    const int wide_rows = strips64 >= 1024 ? 5 : fitted < 3 ? 3 : fitted > 12 ? 12 : (int)(fitted + 0.5);
-    const bool wide_skinny = gi_gemm_bf16_skinny_splits(N, K) == 0 && M >= wide_rows;
-    return M <= 16 && !wide_skinny;
+    return M < (fitted < 3 ? 3 : fitted > 12 ? 12 : (int)(fitted + 0.5));
 }
 
 // Workgroups of the slim kernel for an output of N columns that is not gated: the pieces a row's sum of squares comes in.
@@ -2237,6 +2457,52 @@ static int launch_slim_tiles(const void* A, const void* W, void* C, int epi, int
     return 0;
 }
 
+// splits == 0: all of k is one workgroup's, which ends the product with `epi`; else the sums go to `scratch`.
+static int launch_strips(const void* A, const void* W, void* C, int epi, int M, int N, int K, long lda, long ldw, long ldc, float* scratch, int splits, NormIn norm_in, hipStream_t stream) {
+    const int k_per_split = splits == 0 ? K : ((K + splits - 1) / splits + PK - 1) / PK * PK;
+    dim3 grid((N + 63) / 64, splits == 0 ? 1 : splits);
+#define STRIP(TM_, ST_, EPI_, PARTIAL_)                                                                                                 \
+    do {                                                                                                                                \
+        constexpr int bytes = strip_bytes(TM_, ST_);                                                                                    \
+        static bool raised = false;                                                                                                     \
+        if (!raised) {                                                                                                                  \
+            if (hipFuncSetAttribute((const void*)gemm_bf16_strip_kernel<TM_, ST_, EPI_, PARTIAL_>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) \
+                return gi_fail("gemm_bf16: cannot reserve %d bytes of LDS", bytes);                                                     \
+            raised = true;                                                                                                              \
+        }                                                                                                                               \
+        gemm_bf16_strip_kernel<TM_, ST_, EPI_, PARTIAL_><<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, scratch, M, N, K, lda, ldw, ldc, k_per_split, norm_in); \
+    } while (0)
+#define STRIP_TM(EPI_, PARTIAL_)                                                                                                        \
+    do {                                                                                                                                \
+        if (M <= 32) STRIP(1, 6, EPI_, PARTIAL_); else if (M <= 64) STRIP(2, 4, EPI_, PARTIAL_); else if (M <= 96) STRIP(3, 4, EPI_, PARTIAL_);     \
+        else if (!one_round) STRIP(4, 3, EPI_, PARTIAL_); else STRIP(4, 6, EPI_, PARTIAL_);                                             \
+    } while (0)
+#define STRIP_GATED(EPI_)                                                                                                               \
+    do {                                                                                                                                \
+        if (M <= 128) STRIP_TM(EPI_, false); else if (M <= 160) STRIP(5, 5, EPI_, false); else STRIP(6, 4, EPI_, false);                \
+    } while (0)
+    // Up to 128 rows two workgroups fit a compute unit's LDS, but where there are no more workgroups than units a deeper ring serves better (128 rows of 16,384 x 2,048
+    // gated 24.2 us with six stages, 25.4 with three; of 28,672 x 4,096 75.6 and 71.5).
+    const bool one_round = (long)grid.x * grid.y <= gi_compute_units();
+    if (splits != 0 && M <= 128) STRIP_TM(EPI_STORE_F32, true);
+    else if (splits != 0) {
+        if (M <= 160) STRIP(5, 5, EPI_STORE_F32, true); else if (M <= 192) STRIP(6, 4, EPI_STORE_F32, true);
+        else if (M <= 224) STRIP(7, 4, EPI_STORE_F32, true); else STRIP(8, 4, EPI_STORE_F32, true);
+    }
+    else if (epi == EPI_GATED_BF16) STRIP_GATED(EPI_GATED_BF16);
+    else if (epi == EPI_GATED_GELU_BF16) STRIP_GATED(EPI_GATED_GELU_BF16);
+    else if (epi == EPI_GATED_CLAMP_BF16) STRIP_GATED(EPI_GATED_CLAMP_BF16);
+    else if (M > 128) return gi_fail("gemm_bf16 (strips): %d rows are not taken", M);
+    else if (epi == EPI_STORE_F32) STRIP_TM(EPI_STORE_F32, false);
+    else if (epi == EPI_ADD_F32) STRIP_TM(EPI_ADD_F32, false);
+    else STRIP_TM(EPI_STORE_BF16, false);
+#undef STRIP_GATED
+#undef STRIP_TM
+#undef STRIP
+    GI_CHECK_LAUNCH("gemm_bf16 (strips)");
+    return 0;
+}
+
 // Up to 128 rows the weights are the traffic and every workgroup streams its share of them once (measured on the decode step of
 // the Llama-3.2-1B shape: 72 rows took 2.69 ms through the tiles of 128 rows of the kernels for more rows, against 2.11 ms at 64 rows).
 static int launch_skinny(const void* A, const void* W, void* C, int epi, int M, int N, int K, long lda, long ldw, long ldc, float* scratch,
@@ -2257,6 +2523,7 @@ static int launch_skinny(const void* A, const void* W, void* C, int epi, int M, 
                norm_in.parts, consumer_max_parts(M), M);
     if (splits == 0) {                             // a wide output: every workgroup sees all of k and finishes its columns
         GI_REQUIRE(norm_out.scaled == nullptr && rope == nullptr, "gemm_bf16: a product this wide does not hand a norm on, or its rows to the cache");
+        if (strips_take(M, N, K, true) && strip_strides(lda, ldw)) return launch_strips(A, W, C, epi, M, N, K, lda, ldw, ldc, nullptr, 0, norm_in, stream);
         const int k_per_split = K;
         dim3 grid((N + 63) / 64, 1);
         if (epi == EPI_GATED_BF16) SKINNY_MT(EPI_GATED_BF16, false); else if (epi == EPI_GATED_GELU_BF16) SKINNY_MT(EPI_GATED_GELU_BF16, false); else if (epi == EPI_GATED_CLAMP_BF16) SKINNY_MT(EPI_GATED_CLAMP_BF16, false); else if (epi == EPI_STORE_F32) SKINNY_MT(EPI_STORE_F32, false);
@@ -2266,18 +2533,23 @@ static int launch_skinny(const void* A, const void* W, void* C, int epi, int M, 
     }
     GI_REQUIRE(scratch != nullptr && scratch_floats >= (long)splits * M * N, "gemm_bf16: scratch of %ld floats needed, %ld given",
                (long)splits * M * N, scratch_floats);
-    int k_per_split = (K + splits - 1) / splits;
-    k_per_split = (k_per_split + KB - 1) / KB * KB;
-    dim3 grid((N + 63) / 64, splits);
-    SKINNY_MT(EPI_STORE_F32, true);
+    int parts = splits;
+    if (strips_take(M, N, K, false) && strip_strides(lda, ldw) && scratch_floats >= (long)strip_splits(M, N, K) * M * N) {
+        parts = strip_splits(M, N, K);
+        if (int rc = launch_strips(A, W, nullptr, EPI_STORE_F32, M, N, K, lda, ldw, (long)N, scratch, parts, NO_NORM_IN, stream)) return rc;
+    } else {
+        const int k_per_split = ((K + splits - 1) / splits + KB - 1) / KB * KB;
+        dim3 grid((N + 63) / 64, splits);
+        SKINNY_MT(EPI_STORE_F32, true);
+    }
 #undef SKINNY_MT
     GI_CHECK_LAUNCH("gemm_bf16 (skinny)");
     if (rope != nullptr) {                         // the sums go where an attention layer wants its queries, keys and values
-        skinny_reduce_rope_store_kernel<<<(unsigned)(((size_t)M * N / 4 + 255) / 256), 256, 0, stream>>>(scratch, M, N, splits, norm_in, *rope);
+        skinny_reduce_rope_store_kernel<<<(unsigned)(((size_t)M * N / 4 + 255) / 256), 256, 0, stream>>>(scratch, M, N, parts, norm_in, *rope);
         GI_CHECK_LAUNCH("gemm_bf16 (reduce, rotate, store)");
         return 0;
     }
-    return reduce_partials(scratch, C, epi, M, N, splits, ldc, stream, norm_in, norm_out, whole);
+    return reduce_partials(scratch, C, epi, M, N, parts, ldc, stream, norm_in, norm_out, whole);
 }
 
 static TileOrder tall_order(int M, int N, int whole) {
@@ -2335,16 +2607,22 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
     if (splits > 1) {                              // few tiles: k is shared out, the sums are finished by the reduce kernel
         GI_REQUIRE(scratch != nullptr && scratch_floats >= (long)splits * M * N, "gemm_bf16: scratch of %ld floats needed, %ld given",
                    (long)splits * M * N, scratch_floats);
-        const int k_per_split = K / splits;
-        PIPED(128, 128, 2, 2, 2, EPI_STORE_F32, scratch, (long)N, splits, k_per_split, (long)M * N, NO_NORM_IN, NO_ROPE);
+        int parts = splits;
+        if (strips_take(M, N, K, false) && strip_strides(lda, ldw) && scratch_floats >= (long)strip_splits(M, N, K) * M * N) {
+            parts = strip_splits(M, N, K);
+            if (int rc = launch_strips(A, W, nullptr, EPI_STORE_F32, M, N, K, lda, ldw, (long)N, scratch, parts, NO_NORM_IN, stream)) return rc;
+        } else {
+            PIPED(128, 128, 2, 2, 2, EPI_STORE_F32, scratch, (long)N, splits, K / splits, (long)M * N, NO_NORM_IN, NO_ROPE);
+        }
         GI_CHECK_LAUNCH("gemm_bf16 (piped, split)");
         if (rope != nullptr) {
-            skinny_reduce_rope_store_kernel<<<(unsigned)(((size_t)M * N / 4 + 255) / 256), 256, 0, stream>>>(scratch, M, N, splits, norm_in, *rope);
+            skinny_reduce_rope_store_kernel<<<(unsigned)(((size_t)M * N / 4 + 255) / 256), 256, 0, stream>>>(scratch, M, N, parts, norm_in, *rope);
             GI_CHECK_LAUNCH("gemm_bf16 (reduce, rotate, store)");
             return 0;
         }
-        return reduce_partials(scratch, C, epi, M, N, splits, ldc, stream, norm_in, norm_out, whole);
+        return reduce_partials(scratch, C, epi, M, N, parts, ldc, stream, norm_in, norm_out, whole);
     }
+    if (rope == nullptr && is_gated(epi) && norm_in.squares == nullptr && strips_take(M, N, K, true) && strip_strides(lda, ldw)) return launch_strips(A, W, C, epi, M, N, K, lda, ldw, ldc, nullptr, 0, limit_in, stream);
     const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
     GI_REQUIRE(norm_out.scaled == nullptr || (!many_tiles(M, N) && large_norm_parts(M, N, K) > 0), "gemm_bf16: a product of M %d, N %d, K %d hands no norm on", M, N, K);
     GI_REQUIRE(norm_in.squares == nullptr || rope != nullptr || (is_gated(epi) && many_tiles(M, N) && norm_in.parts <= PIPED_MAX_PARTS),
@@ -2557,11 +2835,12 @@ GI_API int gi_gemm_bf16_qkv_rope_store(const void* A, const void* W, int M, int 
 }
 
 // Which kernel makes a product of more than 128 rows whose rows lie whole in memory: 0 the tiles of 128 x 128, 1 those of 256 x 128, 2 those of 256 x 256,
-// 3 the first with k shared out over workgroups; -1 for sizes that none of these takes.  kind: 0 stored, 1 added, 2 added with a norm handed on, 3 gated,
+// 3 the first or strips with k shared out over workgroups, 4 strips; -1 for sizes that none of these takes.  kind: 0 stored, 1 added, 2 added with a norm handed on, 3 gated,
 // 4 gated with a norm taken, 5 rotated into the pages, 6 through xielu, 7 stored in bfloat16.  With counters, and the scratch it asks for.
 GI_API int gi_gemm_bf16_large_kernel(int M, int N, int K, int kind) {
     if (!takes_large(M, N, K) || kind < 0 || kind > 7) return -1;
     if (gi_gemm_bf16_piped_splits(M, N, K) > 1) return 3;
+    if (kind == 3 && strips_take(M, N, K, true)) return 4;
     return large_kernel_of_kind(M, N, K, kind, true).kernel;
 }
 
@@ -2578,7 +2857,7 @@ GI_API int gi_gemm_bf16_counters() { return 2 * gi_compute_units(); }
 // where all of a tile's k is one workgroup's, with all columns through the activation.
 GI_API int gi_gemm_bf16_xielu_takes(int M, int N, int K, int first) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 8 != 0 || first < 0 || first >= N) return 0;
-    if (takes_slim(M, N, K)) return 1;
+    if (takes_slim(M, N, K, true)) return 1;
     return M > SKINNY_MAX_ROWS && first == 0 && K % PK == 0 && N >= 128 && gi_gemm_bf16_piped_splits(M, N, K) == 1;
 }
 
@@ -2592,7 +2871,7 @@ GI_API int gi_gemm_bf16_xielu(const void* A, const void* W, void* C, int M, int 
     GI_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && lda >= K && ldw >= K && ((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0,
                "gemm_bf16 (xielu): rows must be 16-byte aligned (strides %ld, %ld)", lda, ldw);
     GI_REQUIRE(params != nullptr && act_out != nullptr && ld_act >= N - first && (first == 0 || (C != nullptr && ldc >= first)), "gemm_bf16 (xielu): outputs or parameters are missing");
-    const bool slim = takes_slim(M, N, K);
+    const bool slim = takes_slim(M, N, K, true);
     GI_REQUIRE(squares_in == nullptr || (slim && parts_in > 0 && parts_in <= slim_max_parts(M)), "gemm_bf16 (xielu): %d pieces of a sum of squares are not taken", parts_in);
     NormIn in = {squares_in, parts_in, eps, K, 0.f};
     in.first = first;

@@ -1885,10 +1885,10 @@ def gemm_bf16_onto_norm(a, w, x, g, eps, normed, checked=False):
 
 
 def gemm_bf16_large_kernel(m, n, k, kind):
-    """Which kernel makes a product of more than 128 rows (None: none of these): "128x128", "256x128", "256x256" or "128x128 shared" (k shared out over
-    workgroups).  kind: one of `PRODUCT_KINDS`; with counters (`step_counters`)."""
+    """Which kernel makes a product of more than 128 rows (None: none of these): "128x128", "256x128", "256x256", "strips" (64 columns by all rows) or
+    "128x128 shared" (k shared out over workgroups, which make strips of up to 256 rows where those are the faster ones).  kind: one of `PRODUCT_KINDS`; with counters (`step_counters`)."""
     which = lib().gi_gemm_bf16_large_kernel(m, n, k, PRODUCT_KINDS.index(kind))
-    return None if which < 0 else ("128x128", "256x128", "256x256", "128x128 shared")[which]
+    return None if which < 0 else ("128x128", "256x128", "256x256", "128x128 shared", "strips")[which]
 
 
 @lru_cache(maxsize=8192)

@@ -279,6 +279,39 @@ def test_gated_products_have_one_gate(m, inter, k, few, columns, stride, gated, 
     assert torch.equal(out[:few, :columns], alone) and bool((out[:, inter:] == 3.0).all())
 
 
+@pytest.mark.parametrize("m", [1, 17, 33, 64, 65, 97, 128, 129, 160, 161, 192, 193, 225, 256])
+@pytest.mark.parametrize("n,k", [(12320, 64), (12288 + 48, 192), (16384, 576), (200, 1088), (3072, 1536), (2048, 2112)])
+def test_gemm_bf16_strips(m, n, k):
+    """64 columns by all rows: on both sides of every height, one to more blocks of k than the ring has stages, a last strip of 32 and of 48 columns, k in one to four shares
+    (uneven ones too), stored, added, in bfloat16 and gated."""
+    a, w = randn(m, k, dtype=torch.bfloat16, seed=1), randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.1)
+    want = a.double() @ w.double().T
+    out = torch.full((m, n + 4), 3.0, device=DEV)
+    ops().gemm_bf16(a, w, out[:, :n])
+    assert rel(out[:, :n], want) < 2e-6 and bool((out[:, n:] == 3.0).all())
+    ops().gemm_bf16(a, w, out[:, :n], accumulate=True)
+    assert rel(out[:, :n], 2 * want) < 2e-6 and bool((out[:, n:] == 3.0).all())
+    rounded = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    ops().gemm_bf16(a, w, rounded)
+    assert torch.equal(rounded, (out[:, :n] / 2).bfloat16()) or rel(rounded, want) < 4.1e-3          # half of bfloat16's last place
+    if n % 32 == 0:
+        gate, up = want.view(m, n // 32, 2, 16).unbind(2)
+        gated = torch.full((m + 1, n // 2), 3.0, dtype=torch.bfloat16, device=DEV)
+        ops().gemm_bf16(a, w, gated[:m], gated=True)
+        assert rel(gated[:m], (torch.nn.functional.silu(gate) * up).reshape(m, n // 2)) < 4.1e-3 and bool((gated[m:] == 3.0).all())
+
+
+@pytest.mark.parametrize("m,parts", [(1, 512), (8, 300), (9, 256), (16, 3), (17, 256), (32, 2), (33, 8), (64, 1), (128, 5)])
+def test_gemm_bf16_strips_finish_a_norm(m, parts):
+    n, k = 28672, 3072                                                     # (strips from one row on)
+    a, w, squares = randn(m, k, dtype=torch.bfloat16, seed=1), randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.1), randn(m, parts, seed=3).abs() * k / parts
+    product = (a.double() @ w.double().T) * torch.rsqrt(squares.double().sum(1, keepdim=True) / k + 1e-5)
+    gate, up = product.view(m, n // 32, 2, 16).unbind(2)
+    out = torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV)
+    ops().gemm_bf16(a, w, out, gated=True, norm_in=(squares, 1e-5))
+    assert rel(out, (torch.nn.functional.silu(gate) * up).reshape(m, n // 2)) < 4.1e-3
+
+
 @pytest.mark.parametrize("m,n,k", [(4109, 4120, 192), (4096, 4096, 448)])
 def test_gemm_bf16_ping_pong_with_whole_lines(m, n, k):
     """Outputs whose rows are 16-byte aligned leave the ping-pong kernel in whole cache lines: every epilogue, with edge tiles."""

@@ -28,6 +28,17 @@ def test_the_faster_kernel_is_chosen(m, n, k, kind, kernel):
     assert ops.gemm_bf16_large_kernel(m, n, k, kind) == kernel
 
 
+@pytest.mark.parametrize("m,n,k,kernel", [(129, 16384, 2048, "strips"), (192, 16384, 3072, "strips"), (193, 16384, 2048, "128x128"), (131, 28672, 4096, "256x128"), (131, 16384, 2056, None)])
+def test_strips_where_one_round_of_them_is_faster(m, n, k, kernel):
+    assert ops.gemm_bf16_large_kernel(m, n, k, "gated") == kernel
+
+
+# m, n, k -> shares of k, as the scratch shows them
+@pytest.mark.parametrize("m,n,k,shares", [(64, 2048, 2048, 8), (131, 3072, 8192, 5), (40, 5120, 3072, 4), (131, 10240, 2048, 2), (256, 2048, 2048, 8), (256, 3072, 8192, 5), (300, 2048, 2048, 4)])
+def test_scratch_holds_as_many_shares_as_either_kernel_makes(m, n, k, shares):
+    assert ops._scratch_floats(m, n, k, 0, False) == shares * m * n
+
+
 # m, n, k, what becomes of the sums, the kernel that was the faster one, by how many workgroups it makes its last tiles, and without counters
 SHARED_OR_NOT = [
     (4096, 3072, 8192, "added", "256x256", 1, 1), (4096, 3072, 8192, "stored in bfloat16", "256x256", 1, 1), (1368, 8192, 6784, "stored in bfloat16", "256x256", 1, 1),
