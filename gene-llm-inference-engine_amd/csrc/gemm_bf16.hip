@@ -12,8 +12,8 @@
 //           blocks of k in flight; v_mfma_f32_32x32x16_bf16.
 //   tiled   the other shapes above 64 rows: a BM x 128 tile of C per workgroup of 4 waves,
 //           operands staged through registers into LDS in k-blocks of 64.
-//   strips  up to 256 rows of A (K a multiple of 64): 64 rows of weights and all rows of A a workgroup, both
-//           straight into a ring of LDS stages.  Wide outputs are finished by the workgroup that sees all of k;
+//   strips  up to 128 rows of A (K a multiple of 64), and more where k is shared out: 64 rows of weights and all rows of A, or a tile of up
+//           to 256, a workgroup, both straight into a ring of LDS stages.  Wide outputs are finished by the workgroup that sees all of k;
 //           for narrow ones k is split over workgroups and the partial sums are added in a fixed order by a second kernel.
 //   skinny  the other shapes of up to 128 rows: weights stream from HBM straight into registers and are used
 //           once, activations go through LDS; v_mfma_f32_16x16x32_bf16.  Wide and narrow outputs likewise.
@@ -1437,7 +1437,8 @@ constexpr int strip_bytes(int tm, int stages) {
 }
 template <int TM, int STAGES, int EPI, bool PARTIAL>
 __global__ __launch_bounds__(512, TM <= 2 ? 4 : 2) void gemm_bf16_strip_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ C,
-                                                                              float* __restrict__ P, int M, int N, int K, long lda, long ldw, long ldc, int k_per_split, NormIn norm_in) {
+                                                                              float* __restrict__ P, int all_rows, int N, int K, long lda, long ldw, long ldc, int k_per_split, int tile_rows, NormIn norm_in) {
+    const int m_first = PARTIAL ? blockIdx.z * tile_rows : 0, M = PARTIAL ? min(tile_rows, all_rows - m_first) : all_rows;       // of this tile
     constexpr int BM = 32 * TM, STAGE_BYTES = (64 + BM) * 128, CHUNK = strip_chunk(TM, STAGES);
     extern __shared__ __attribute__((aligned(16))) unsigned char ring[];               // strip_bytes(TM, STAGES)
     float* const row_scale = reinterpret_cast<float*>(ring + CHUNK * 32768);            // (behind the sums of the end)
@@ -1458,7 +1459,7 @@ __global__ __launch_bounds__(512, TM <= 2 ? 4 : 2) void gemm_bf16_strip_kernel(c
     // A wave loads eight rows of W and every eighth group of eight rows of A; groups beyond M are left out (what then lies in LDS makes rows that nobody writes).
     constexpr int MOST = (BM / 8 + 7) / 8;                                              // (M > BM - 32: a wave has so many groups, or one fewer)
     const bool most = wave + 8 * (MOST - 1) < (M + 7) / 8;
-    const bf16_t *w_tile = W + (size_t)n0 * ldw + k_begin, *a_tile = A + k_begin;
+    const bf16_t *w_tile = W + (size_t)n0 * ldw + k_begin, *a_tile = A + (size_t)m_first * lda + k_begin;
     unsigned w_src, a_src[MOST];
     {
         const int row = wave * 8 + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
@@ -1585,7 +1586,7 @@ __global__ __launch_bounds__(512, TM <= 2 ? 4 : 2) void gemm_bf16_strip_kernel(c
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
                     if (row + v < M) {
-                        if constexpr (PARTIAL) P[((size_t)blockIdx.y * M + row + v) * N + n] = ss[v];
+                        if constexpr (PARTIAL) P[((size_t)blockIdx.y * all_rows + m_first + row + v) * N + n] = ss[v];
                         else write_out<EPI>(C, (size_t)(row + v) * ldc + n, scaled_rows ? ss[v] * row_scale[row + v] : ss[v]);
                     }
             }
@@ -2252,33 +2253,56 @@ static LargeChoice large_kernel_of_kind(int M, int N, int K, int kind, bool coun
 }
 static bool takes_large(int M, int N, int K) { return M > SKINNY_MAX_ROWS && K % PK == 0 && N >= 128; }
 
-// Whether the strips' kernel makes a product; `whole`: with all of k in a workgroup, which ends it, else k is shared out.  Above 128 rows the tiles of 128 x 128 are the better ones
-// where the strips do not fit one round (160 rows of 28,672 x 4,096 gated: 75 us and 82) or leave half of the units without one (10,240 x 2,048: 26.2 and 27.3), and above 192
-// rows where k is short (256 rows of 2,048 x 2,048 18.8 and 18.1, of 3,072 x 2,048 20.9 and 21.3, 200 of 2,048 x 1,024 12.6 and 13.6).
-constexpr int STRIP_MAX_ROWS = 256;
-static bool strips_take(int M, int N, int K, bool whole) {
-    if (K % PK != 0 || M > STRIP_MAX_ROWS) return false;
-    if (M <= SKINNY_MAX_ROWS) return true;
-    const int strips = (N + 63) / 64, units = gi_compute_units();
-    return whole ? M <= 192 && strips <= units : 2 * strips <= units && (M <= 192 || K > 8 * M);
+// Products whose k is shared out, in strips: tiles of rows (one to some, of equal height), shares of k, and about how long it takes with the kernel that adds up.  The times are fitted
+// to 4,600 products (24 numbers of rows from 17 to 1,400, 12 sizes of weights, every cut), which they meet within 6 %; the cut they choose is 0.7 % slower than the best one on average, 11 % at worst.
+// 128 rows of 2,048 x 2,048 take 12.2 us as one tile in four shares, 10.2 as two in three; 301 of 2,048 x 8,192 27 as two in four, 32 as three in two.
+struct StripCut { int tiles, splits; double us; };
+static StripCut strip_cut(int M, int N, int K) {
+    const int strips = (N + 63) / 64, units = gi_compute_units(), all = K / PK;
+    StripCut best = {0, 0, 0};
+    double least = 0;
+    for (int tiles = (M + 255) / 256; tiles <= (M + 63) / 64; ++tiles) {
+        const int rows = (M + tiles - 1) / tiles, height = (rows + 31) / 32, together = height <= 3 ? 2 : 1;       // (workgroups that a unit's LDS holds)
+        for (int want = 1; want <= 16 && (want == 1 || all / want >= 3); ++want) {
+            const int blocks = (all + want - 1) / want, splits = (all + blocks - 1) / blocks;
+            if (splits != want) continue;
+            const long groups = (long)strips * tiles * splits;
+            if (best.tiles && (groups > 2 * units || (groups > units && rows > 64 && (tiles > 1 || rows > 96)))) break;
+            const long a_unit = (groups + units - 1) / units;
+            const double one = blocks * (0.121 + 0.00116 * rows + 0.0283 * height) + 0.39, sums = 1.85e-6 * splits * M * N;
+            const double busy = 5.2 + (a_unit / together * (together == 2 ? 1.38 : 1) + a_unit % together) * one + sums;
+            const double memory = 5.2 + 0.27e-6 * N * K + sums + 4.5e-6 * (rows + 64) * groups * blocks;
+            const double both = busy * busy * busy * busy + memory * memory * memory * memory;
+            if (best.tiles == 0 || both < least) { least = both; best = {tiles, splits, 0}; }
+        }
+    }
+    best.us = sqrt(sqrt(least));
+    return best;
+}
+// Whether a product ends in strips, with all of k in a workgroup.  Above 128 rows the tiles of 128 x 128 are the better ones for gated products whose strips do not fit one
+// round (160 rows of 28,672 x 4,096: 75 us and 82).
+static bool ends_in_strips(int M, int N, int K) { return K % PK == 0 && (M <= SKINNY_MAX_ROWS || (M <= 192 && (N + 63) / 64 <= gi_compute_units())); }
+// How strips make a product whose k is shared out, which the kernels beside them cut into `splits`; no tiles where they do not: from 129 rows on where the tiles of 128 x 128 promise to
+// be as fast (a fit like the one above; 350 rows of 3,072 x 8,192 43.1 us and 44.5, 600 71 and 58).
+constexpr int STRIP_MAX_ROWS = 1536;
+static StripCut shared_strips(int M, int N, int K, int splits) {
+    const StripCut none = {0, 0, 0};
+    if (K % PK != 0 || M > STRIP_MAX_ROWS || splits == 0) return none;
+    const StripCut cut = strip_cut(M, N, K);
+    if (M <= SKINNY_MAX_ROWS) return cut;
+    const bool two = (long)((M + 127) / 128) * ((N + 127) / 128) * splits > gi_compute_units();
+    return cut.us < 0.98 * (6.6 + K / splits / PK * (two ? 0.951 : 0.882) + 1.55e-6 * splits * M * N) ? cut : none;
 }
 static bool strip_strides(long lda, long ldw) { return lda < (1L << 22) && ldw < (1L << 22); }       // (a tile's rows within 32-bit offsets)
-// Shares of k: as many as there are units for, with at least 512 of k each (64 rows of 2,048 x 2,048, 32 strips: 9.1 us in four, 10.3 in eight; of 2,048 x 8,192 14.5
-// in eight, 18.4 in four; of 5,120 x 3,072, 80 strips, 13.9 in three, 16.4 in four and 15.3 in two).
-static int strip_splits(int M, int N, int K) {
-    const int strips = (N + 63) / 64, units = gi_compute_units(), most = 2 * strips <= units ? units / strips : M <= 64 ? 2 : 1;
-    return most < K / 512 ? most : K / 512 > 0 ? K / 512 : 1;
-}
-// The most shares of k that a product may be cut into, which the kernels beside the strips' cut into `splits` (0: none).
+// The most shares of k that a product may be cut into.
 static int shared_out(int M, int N, int K, int splits) {
-    if (splits == 0 || !strips_take(M, N, K, false)) return splits;
-    const int strips = strip_splits(M, N, K);
+    const int strips = shared_strips(M, N, K, splits).splits;
     return strips > splits ? strips : splits;
 }
 
 // By how many workgroups each tile of the last round of a product is made that has all the scratch it asks for (1: one), with or without counters.
 GI_API int gi_gemm_bf16_shares(int M, int N, int K, int kind, int counters) {
-    if (!takes_large(M, N, K) || gi_gemm_bf16_piped_splits(M, N, K) > 1 || (kind == 3 && strips_take(M, N, K, true))) return 1;
+    if (!takes_large(M, N, K) || gi_gemm_bf16_piped_splits(M, N, K) > 1 || (kind == 3 && ends_in_strips(M, N, K))) return 1;
     const LargeChoice choice = large_kernel_of_kind(M, N, K, kind, counters != 0);
     return choice.kernel == TALL_256 ? choice.cut.shares : 1;
 }
@@ -2457,10 +2481,11 @@ static int launch_slim_tiles(const void* A, const void* W, void* C, int epi, int
     return 0;
 }
 
-// splits == 0: all of k is one workgroup's, which ends the product with `epi`; else the sums go to `scratch`.
-static int launch_strips(const void* A, const void* W, void* C, int epi, int M, int N, int K, long lda, long ldw, long ldc, float* scratch, int splits, NormIn norm_in, hipStream_t stream) {
-    const int k_per_split = splits == 0 ? K : ((K + splits - 1) / splits + PK - 1) / PK * PK;
-    dim3 grid((N + 63) / 64, splits == 0 ? 1 : splits);
+// cut.splits == 0: all of k is one workgroup's, which ends the product with `epi`; else the sums go to `scratch`.
+static int launch_strips(const void* A, const void* W, void* C, int epi, int M, int N, int K, long lda, long ldw, long ldc, float* scratch, StripCut cut, NormIn norm_in, hipStream_t stream) {
+    const int splits = cut.splits, k_per_split = splits == 0 ? K : (K / PK + splits - 1) / splits * PK;
+    const int tile_rows = (M + cut.tiles - 1) / cut.tiles;
+    dim3 grid((N + 63) / 64, splits == 0 ? 1 : splits, cut.tiles);
 #define STRIP(TM_, ST_, EPI_, PARTIAL_)                                                                                                 \
     do {                                                                                                                                \
         constexpr int bytes = strip_bytes(TM_, ST_);                                                                                    \
@@ -2470,11 +2495,11 @@ static int launch_strips(const void* A, const void* W, void* C, int epi, int M, 
                 return gi_fail("gemm_bf16: cannot reserve %d bytes of LDS", bytes);                                                     \
             raised = true;                                                                                                              \
         }                                                                                                                               \
-        gemm_bf16_strip_kernel<TM_, ST_, EPI_, PARTIAL_><<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, scratch, M, N, K, lda, ldw, ldc, k_per_split, norm_in); \
+        gemm_bf16_strip_kernel<TM_, ST_, EPI_, PARTIAL_><<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, scratch, M, N, K, lda, ldw, ldc, k_per_split, tile_rows, norm_in); \
     } while (0)
 #define STRIP_TM(EPI_, PARTIAL_)                                                                                                        \
     do {                                                                                                                                \
-        if (M <= 32) STRIP(1, 6, EPI_, PARTIAL_); else if (M <= 64) STRIP(2, 4, EPI_, PARTIAL_); else if (M <= 96) STRIP(3, 4, EPI_, PARTIAL_);     \
+        if (tile_rows <= 32) STRIP(1, 6, EPI_, PARTIAL_); else if (tile_rows <= 64) STRIP(2, 4, EPI_, PARTIAL_); else if (tile_rows <= 96) STRIP(3, 4, EPI_, PARTIAL_); \
         else if (!one_round) STRIP(4, 3, EPI_, PARTIAL_); else STRIP(4, 6, EPI_, PARTIAL_);                                             \
     } while (0)
 #define STRIP_GATED(EPI_)                                                                                                               \
@@ -2483,11 +2508,11 @@ static int launch_strips(const void* A, const void* W, void* C, int epi, int M, 
     } while (0)
     // Up to 128 rows two workgroups fit a compute unit's LDS, but where there are no more workgroups than units a deeper ring serves better (128 rows of 16,384 x 2,048
     // gated 24.2 us with six stages, 25.4 with three; of 28,672 x 4,096 75.6 and 71.5).
-    const bool one_round = (long)grid.x * grid.y <= gi_compute_units();
-    if (splits != 0 && M <= 128) STRIP_TM(EPI_STORE_F32, true);
+    const bool one_round = (long)grid.x * grid.y * grid.z <= gi_compute_units();
+    if (splits != 0 && tile_rows <= 128) STRIP_TM(EPI_STORE_F32, true);
     else if (splits != 0) {
-        if (M <= 160) STRIP(5, 5, EPI_STORE_F32, true); else if (M <= 192) STRIP(6, 4, EPI_STORE_F32, true);
-        else if (M <= 224) STRIP(7, 4, EPI_STORE_F32, true); else STRIP(8, 4, EPI_STORE_F32, true);
+        if (tile_rows <= 160) STRIP(5, 5, EPI_STORE_F32, true); else if (tile_rows <= 192) STRIP(6, 4, EPI_STORE_F32, true);
+        else if (tile_rows <= 224) STRIP(7, 4, EPI_STORE_F32, true); else STRIP(8, 4, EPI_STORE_F32, true);
     }
     else if (epi == EPI_GATED_BF16) STRIP_GATED(EPI_GATED_BF16);
     else if (epi == EPI_GATED_GELU_BF16) STRIP_GATED(EPI_GATED_GELU_BF16);
@@ -2523,7 +2548,7 @@ static int launch_skinny(const void* A, const void* W, void* C, int epi, int M, 
                norm_in.parts, consumer_max_parts(M), M);
     if (splits == 0) {                             // a wide output: every workgroup sees all of k and finishes its columns
         GI_REQUIRE(norm_out.scaled == nullptr && rope == nullptr, "gemm_bf16: a product this wide does not hand a norm on, or its rows to the cache");
-        if (strips_take(M, N, K, true) && strip_strides(lda, ldw)) return launch_strips(A, W, C, epi, M, N, K, lda, ldw, ldc, nullptr, 0, norm_in, stream);
+        if (ends_in_strips(M, N, K) && strip_strides(lda, ldw)) return launch_strips(A, W, C, epi, M, N, K, lda, ldw, ldc, nullptr, StripCut{1, 0, 0}, norm_in, stream);
         const int k_per_split = K;
         dim3 grid((N + 63) / 64, 1);
         if (epi == EPI_GATED_BF16) SKINNY_MT(EPI_GATED_BF16, false); else if (epi == EPI_GATED_GELU_BF16) SKINNY_MT(EPI_GATED_GELU_BF16, false); else if (epi == EPI_GATED_CLAMP_BF16) SKINNY_MT(EPI_GATED_CLAMP_BF16, false); else if (epi == EPI_STORE_F32) SKINNY_MT(EPI_STORE_F32, false);
@@ -2534,9 +2559,10 @@ static int launch_skinny(const void* A, const void* W, void* C, int epi, int M, 
     GI_REQUIRE(scratch != nullptr && scratch_floats >= (long)splits * M * N, "gemm_bf16: scratch of %ld floats needed, %ld given",
                (long)splits * M * N, scratch_floats);
     int parts = splits;
-    if (strips_take(M, N, K, false) && strip_strides(lda, ldw) && scratch_floats >= (long)strip_splits(M, N, K) * M * N) {
-        parts = strip_splits(M, N, K);
-        if (int rc = launch_strips(A, W, nullptr, EPI_STORE_F32, M, N, K, lda, ldw, (long)N, scratch, parts, NO_NORM_IN, stream)) return rc;
+    const StripCut cut = strip_strides(lda, ldw) ? shared_strips(M, N, K, splits) : StripCut{0, 0, 0};
+    if (cut.tiles && scratch_floats >= (long)cut.splits * M * N) {
+        parts = cut.splits;
+        if (int rc = launch_strips(A, W, nullptr, EPI_STORE_F32, M, N, K, lda, ldw, (long)N, scratch, cut, NO_NORM_IN, stream)) return rc;
     } else {
         const int k_per_split = ((K + splits - 1) / splits + KB - 1) / KB * KB;
         dim3 grid((N + 63) / 64, splits);
@@ -2608,9 +2634,10 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
         GI_REQUIRE(scratch != nullptr && scratch_floats >= (long)splits * M * N, "gemm_bf16: scratch of %ld floats needed, %ld given",
                    (long)splits * M * N, scratch_floats);
         int parts = splits;
-        if (strips_take(M, N, K, false) && strip_strides(lda, ldw) && scratch_floats >= (long)strip_splits(M, N, K) * M * N) {
-            parts = strip_splits(M, N, K);
-            if (int rc = launch_strips(A, W, nullptr, EPI_STORE_F32, M, N, K, lda, ldw, (long)N, scratch, parts, NO_NORM_IN, stream)) return rc;
+        const StripCut cut = strip_strides(lda, ldw) ? shared_strips(M, N, K, splits) : StripCut{0, 0, 0};
+        if (cut.tiles && scratch_floats >= (long)cut.splits * M * N) {
+            parts = cut.splits;
+            if (int rc = launch_strips(A, W, nullptr, EPI_STORE_F32, M, N, K, lda, ldw, (long)N, scratch, cut, NO_NORM_IN, stream)) return rc;
         } else {
             PIPED(128, 128, 2, 2, 2, EPI_STORE_F32, scratch, (long)N, splits, K / splits, (long)M * N, NO_NORM_IN, NO_ROPE);
         }
@@ -2622,7 +2649,7 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
         }
         return reduce_partials(scratch, C, epi, M, N, parts, ldc, stream, norm_in, norm_out, whole);
     }
-    if (rope == nullptr && is_gated(epi) && norm_in.squares == nullptr && strips_take(M, N, K, true) && strip_strides(lda, ldw)) return launch_strips(A, W, C, epi, M, N, K, lda, ldw, ldc, nullptr, 0, limit_in, stream);
+    if (rope == nullptr && is_gated(epi) && norm_in.squares == nullptr && ends_in_strips(M, N, K) && strip_strides(lda, ldw)) return launch_strips(A, W, C, epi, M, N, K, lda, ldw, ldc, nullptr, StripCut{1, 0, 0}, limit_in, stream);
     const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
     GI_REQUIRE(norm_out.scaled == nullptr || (!many_tiles(M, N) && large_norm_parts(M, N, K) > 0), "gemm_bf16: a product of M %d, N %d, K %d hands no norm on", M, N, K);
     GI_REQUIRE(norm_in.squares == nullptr || rope != nullptr || (is_gated(epi) && many_tiles(M, N) && norm_in.parts <= PIPED_MAX_PARTS),
@@ -2840,7 +2867,7 @@ GI_API int gi_gemm_bf16_qkv_rope_store(const void* A, const void* W, int M, int 
 GI_API int gi_gemm_bf16_large_kernel(int M, int N, int K, int kind) {
     if (!takes_large(M, N, K) || kind < 0 || kind > 7) return -1;
     if (gi_gemm_bf16_piped_splits(M, N, K) > 1) return 3;
-    if (kind == 3 && strips_take(M, N, K, true)) return 4;
+    if (kind == 3 && ends_in_strips(M, N, K)) return 4;
     return large_kernel_of_kind(M, N, K, kind, true).kernel;
 }
 

@@ -301,6 +301,18 @@ def test_gemm_bf16_strips(m, n, k):
         assert rel(gated[:m], (torch.nn.functional.silu(gate) * up).reshape(m, n // 2)) < 4.1e-3 and bool((gated[m:] == 3.0).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(257, 2048, 2112), (301, 3072, 192), (450, 1024, 1984), (700, 200, 576), (897, 2048, 8192), (1000, 960, 704), (1400, 2048, 1088), (1536, 64 * 30, 640), (1537, 1920, 640)])
+def test_gemm_bf16_strips_in_several_tiles_of_rows(m, n, k):
+    """Tiles of equal height, the last one a few rows lower (52 of 65 at 897 rows), k in uneven shares; on both sides of the most rows."""
+    a, w = randn(m, k, dtype=torch.bfloat16, seed=1), randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.1)
+    want = a.double() @ w.double().T
+    out = torch.full((m + 1, n + 4), 3.0, device=DEV)
+    ops().gemm_bf16(a, w, out[:m, :n])
+    assert rel(out[:m, :n], want) < 2e-6 and bool((out[:, n:] == 3.0).all()) and bool((out[m:] == 3.0).all())
+    ops().gemm_bf16(a, w, out[:m, :n], accumulate=True)
+    assert rel(out[:m, :n], 2 * want) < 2e-6 and bool((out[m:] == 3.0).all())
+
+
 @pytest.mark.parametrize("m,parts", [(1, 512), (8, 300), (9, 256), (16, 3), (17, 256), (32, 2), (33, 8), (64, 1), (128, 5)])
 def test_gemm_bf16_strips_finish_a_norm(m, parts):
     n, k = 28672, 3072                                                     # (strips from one row on)

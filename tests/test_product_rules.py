@@ -33,8 +33,8 @@ def test_strips_where_one_round_of_them_is_faster(m, n, k, kernel):
     assert ops.gemm_bf16_large_kernel(m, n, k, "gated") == kernel
 
 
-# m, n, k -> shares of k, as the scratch shows them
-@pytest.mark.parametrize("m,n,k,shares", [(64, 2048, 2048, 8), (131, 3072, 8192, 5), (40, 5120, 3072, 4), (131, 10240, 2048, 2), (256, 2048, 2048, 8), (256, 3072, 8192, 5), (300, 2048, 2048, 4)])
+# m, n, k -> the most shares of k that either kernel makes, as the scratch shows them
+@pytest.mark.parametrize("m,n,k,shares", [(131, 3072, 8192, 5), (40, 5120, 3072, 4), (131, 10240, 2048, 2), (256, 3072, 8192, 5), (300, 2048, 2048, 4), (600, 3072, 8192, 2), (17, 200, 64, 1), (40, 128, 12288, 32)])
 def test_scratch_holds_as_many_shares_as_either_kernel_makes(m, n, k, shares):
     assert ops._scratch_floats(m, n, k, 0, False) == shares * m * n
 
