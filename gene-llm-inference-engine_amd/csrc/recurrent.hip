@@ -702,8 +702,8 @@ __global__ __launch_bounds__(256) void delta_single_kernel(const float* __restri
     constexpr int C = 4, RG = 16;
     const int seg = blockIdx.x, h = blockIdx.y, vt = blockIdx.z * 4 + (threadIdx.x >> 6), n_tiles = (dv + C - 1) / C;
     const int lane = threadIdx.x & 63, c = lane / RG, rg = lane % RG;
-    if (vt >= n_tiles || seg_len[seg] <= 0) return;
-    const size_t t = seg_start[seg];
+    if (vt >= n_tiles || (seg_len && seg_len[seg] <= 0)) return;
+    const size_t t = seg_start ? seg_start[seg] : seg;
     const int col = vt * C + c, kvh = h / (n_heads / n_kv), dn = CHANNEL ? dk : 1;
     float* st = state + (size_t)row_slot[t] * state_stride + ((size_t)h * n_tiles + vt) * ((size_t)dk * C);
     const float* row = qkv + t * ld;
@@ -1193,7 +1193,7 @@ GI_API int gi_delta_tail(const float* proj, long ld, int conv_off, int n_taps, c
 }
 
 // qkv: float32 [n_rows, ld], a row's unit queries [n_kv][dk], unit keys [n_kv][dk], values [n_heads][dv]; gates: float32 [n_rows, 2 n_heads],
-// or [n_rows, n_heads dk + n_heads] with a decay per head and key channel (channel != 0);
+// or [n_rows, n_heads dk + n_heads] with a decay per head and key channel (channel != 0); with `single`, seg_start and seg_len null: run i is row i;
 // out: float32 [n_rows, ldo] gets the heads' read-outs [n_heads][dv].  below > 0: only the runs of fewer rows than that (not with `single`).
 GI_API int gi_delta_scan(const float* qkv, long ld, const float* gates, const int* seg_start, const int* seg_len, int n_segs, const int* row_slot,
                          float* state, long state_stride, float* out, long ldo, int n_heads, int n_kv, int dk, int dv, int channel, int single, int below, hipStream_t stream) {
@@ -1202,6 +1202,7 @@ GI_API int gi_delta_scan(const float* qkv, long ld, const float* gates, const in
     GI_REQUIRE(ld >= 2L * n_kv * dk + (long)n_heads * dv && ldo >= (long)n_heads * dv && state_stride >= gi_delta_memory_floats(n_heads, dk, dv), "delta_scan: row or state strides too small");
     const int tiles = (dv + 3) / 4;
     GI_REQUIRE(n_heads <= 65535 && tiles <= 65535, "delta_scan: too many heads or value channels");
+    GI_REQUIRE((seg_start == nullptr) == (seg_len == nullptr) && (seg_start != nullptr || single), "delta_scan: the runs of a step that is not of single rows are missing");
     dim3 grid(n_segs, n_heads, tiles);
 #define ARGS qkv, ld, gates, seg_start, seg_len, row_slot, state, state_stride, out, ldo, n_heads, n_kv, dk, dv
     const bool aligned = ld % 4 == 0 && ((uintptr_t)qkv & 15) == 0 && (!channel || (((long)n_heads * (dk + 1)) % 4 == 0 && ((uintptr_t)gates & 15) == 0));

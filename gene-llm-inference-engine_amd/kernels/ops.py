@@ -1105,7 +1105,7 @@ def delta_scan(qkv, gates, seg_start, seg_len, row_slot, state, out, n_heads, n_
     """The gated delta rule over every request's rows of the step, in order (csrc/recurrent.hip states it): qkv and gates as
     `delta_prepare` leaves them, out float32 [n, heads*dv] gets the read-outs M^T q; the memories come from the request's state
     slot and go back into it.  channel: the decays are one per head and key channel.  single_rows: every request of the step has one row
-    (a kernel without staging; the same bits).  below: only requests of fewer rows than that (0: all; `delta_chunks` serves the others)."""
+    (a kernel without staging; the same bits); seg_start and seg_len may then be None, request i's row being row i.  below: only requests of fewer rows than that (0: all; `delta_chunks` serves the others)."""
     _dev(qkv, gates, seg_start, seg_len, row_slot, state, out)
     n = qkv.shape[0]
     if single_rows and below:
@@ -1118,11 +1118,14 @@ def delta_scan(qkv, gates, seg_start, seg_len, row_slot, state, out, n_heads, n_
         raise KernelError("delta_scan: state must be float32 [slots, at least delta_memory_floats]")
     if not (0 < dk <= DELTA_MAX_KEY_DIM and n_heads % n_kv == 0):
         raise KernelError(f"delta_scan: keys of 1 to {DELTA_MAX_KEY_DIM} channels and heads in whole groups are served")
-    n_segs = seg_start.numel()
-    _i32(seg_start, "delta_scan: seg_start", n_segs)
-    _i32(seg_len, "delta_scan: seg_len", n_segs)
+    if (seg_start is None) != (seg_len is None) or (seg_start is None and not single_rows):
+        raise KernelError("delta_scan: the runs of a step that is not of single rows are needed")
+    n_segs = n if seg_start is None else seg_start.numel()
+    if seg_start is not None:
+        _i32(seg_start, "delta_scan: seg_start", n_segs)
+        _i32(seg_len, "delta_scan: seg_len", n_segs)
     _i32(row_slot, "delta_scan: slots", n)
-    _call("gi_delta_scan", qkv.data_ptr(), qkv.stride(0), gates.data_ptr(), seg_start.data_ptr(), seg_len.data_ptr(), n_segs, row_slot.data_ptr(), state.data_ptr(),
+    _call("gi_delta_scan", qkv.data_ptr(), qkv.stride(0), gates.data_ptr(), _ptr(seg_start), _ptr(seg_len), n_segs, row_slot.data_ptr(), state.data_ptr(),
           state.stride(0), out.data_ptr(), out.stride(0), n_heads, n_kv, dk, dv, 1 if channel else 0, 1 if single_rows else 0, int(below), _stream())
     return out
 

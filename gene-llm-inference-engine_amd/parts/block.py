@@ -16,7 +16,7 @@ import torch
 
 from ..kernels import ops
 from .base import feed_forward_class, mixer_class, norm_class, register_block
-from .linear import linear, linear_xielu, takes_handed_norm
+from .linear import linear, linear_onto, linear_xielu, takes_handed_norm
 from .norm import NormedRows, ReadyRows, norm_to_apply, norm_to_hand_on, norm_to_make
 
 
@@ -194,6 +194,12 @@ class _Readers:
         return self.in_dtype is not None and all(hasattr(p, "takes_handed_norm") and p.takes_handed_norm(n_rows) for p in self.parts)
 
 
+class _Held:
+    """A matrix that parts hold views of: what a step reads of it counts with them."""
+    def __init__(self, weight):
+        self.weight = weight
+
+
 class ParallelBlock:
     """x += mixer(h) + feed_forward(h) with h = norm_1(x): both halves read the same normed rows, which are made once, and each
     adds its result onto x (the two sums reach x one after the other; neither half reads x).  The block plays the game of
@@ -202,7 +208,7 @@ class ParallelBlock:
     (asked beforehand: the second half must not fall back on rows that the first has changed by then).  A norm that does not commute
     with a product may be made whole by the half that writes x last, if it can (`makes_next_norm`)."""
     hands_norm_on = True
-    STACK = True                     # the two halves' first products as one (off: each half makes its own)
+    STACK = True                     # the two halves' first products as one, and their last (off: each half makes its own)
     # ... in steps of up to so many rows and with both matrices together up to so many bytes: one launch less a layer where launches
     # are what a step costs (8 decoded rows, 8 layers: 0.563 -> 0.536 ms a step with 44 MB a layer); with 160 MB a layer the one product
     # took longer than the two (1.142 -> 1.169 ms), and so did it for the rows of prompts at both sizes (5.19 -> 5.28, 11.28 -> 11.37 ms).
@@ -233,6 +239,18 @@ class ParallelBlock:
                 self.w_first = torch.cat(first, dim=0).contiguous()
                 self.mixer.use_input_weight(self.w_first[:self._split])
                 self.feed_forward.use_input_weight(self.w_first[self._split:])
+        # Both halves end with a product onto the same rows: where both say which matrix that is (`output_weight`, bfloat16), the two are laid side by side along k and the halves
+        # write the rows they would multiply into one buffer (`into=`): one product of all of it.  5 rows of 2,048 x 2,048 and 2,048 x 8,192 14.8 us, in one 12.2; 200 rows 34.1
+        # and 26.3, 1,777 105.5 and 92.2.
+        self._last, self._last_split = None, 0
+        last = [getattr(p, "output_weight", lambda: None)() for p in (self.mixer, self.feed_forward)] if self.feed_forward is not None else []
+        if (self.STACK and len(last) == 2 and all(w is not None and w.dtype == torch.bfloat16 and w.shape[1] % 8 == 0 for w in last) and last[0].shape[0] == last[1].shape[0]
+                and all("into" in inspect.signature(p.forward).parameters for p in (self.mixer, self.feed_forward))):
+            self._last_split = last[0].shape[1]
+            whole = torch.cat(last, dim=1).contiguous()
+            self.mixer.use_output_weight(whole[:, :self._last_split])
+            self.feed_forward.use_output_weight(whole[:, self._last_split:])
+            self._last = _Held(whole)
         # (a feed-forward built on one that takes activated columns may have a `forward` of its own that does not)
         self._activates = hasattr(self.feed_forward, "input_activation") and "activated" in inspect.signature(self.feed_forward.forward).parameters
         self._readers = _Readers(self._parts()[1:], self._stacked)
@@ -275,21 +293,30 @@ class ParallelBlock:
         last = self.feed_forward if self.feed_forward is not None else self.mixer
         then = norm_to_hand_on(next_reader, ctx.n_rows) if getattr(last, "hands_norm_on", False) else norm_to_apply(next_reader, last)
         own = [{}, {}]                            # what each half is told beyond its rows
+        into = (None, None)
+        if self._last is not None and ctx.trace is None:          # (a trace wants the rows between the halves)
+            ends = torch.empty((ctx.n_rows, self._last.weight.shape[1]), dtype=torch.bfloat16, device=x.device)
+            into = ends[:, :self._last_split], ends[:, self._last_split:]
+            for told, columns in zip(own, into):
+                told["into"] = columns
         w_first = self._stacked(ctx.n_rows)
         if w_first is not None:
             both = torch.empty((ctx.n_rows, w_first.shape[0]), dtype=torch.float32, device=x.device)
-            activated = linear_xielu(rows(self.mixer), w_first, *self.feed_forward.input_activation(), both) if self._activates else None
+            to = {"into": into[1]} if into[1] is not None else {}
+            activated = linear_xielu(rows(self.mixer), w_first, *self.feed_forward.input_activation(), both, **to) if self._activates else None
             if activated is None:
                 linear(rows(self.mixer), w_first, both)
             own[0]["projected"] = both[:, :self._split]
             own[1].update(activated=activated) if activated is not None else own[1].update(projected=both[:, self._split:])
-        if then is not None:
+        if then is not None and into[0] is None:
             own[0 if last is self.mixer else 1]["then"] = then
         out = self.mixer.forward(rows(self.mixer), x, ctx, cache, **own[0])
         if ctx.trace is not None:
             ctx.trace("attn_out", x)
         if self.feed_forward is not None:
             out = self.feed_forward.forward(rows(self.feed_forward), x, ctx, **own[1])
+        if into[0] is not None:
+            out = linear_onto(ends, self._last.weight, x, then, ctx)
         if ctx.trace is not None:
             ctx.trace("ffn_out", x)
         return out if then is not None else None

@@ -100,6 +100,13 @@ class GatedDelta(Mixer):
     def use_input_weight(self, view):
         self.w_in = view
 
+    # ... and the last product's, whose rows the part then writes into columns it is handed (`forward(..., into=)`), leaving the product to the block.
+    def output_weight(self):
+        return self.w_o if self.mid_dtype == torch.bfloat16 else None
+
+    def use_output_weight(self, view):
+        self.w_o = view
+
     @classmethod
     def tensor_needs(cls, spec):
         s, d = spec, spec.hidden_size
@@ -115,7 +122,7 @@ class GatedDelta(Mixer):
     def cache_need(cls, spec):
         return StateNeed((ops.delta_state_floats(spec.n_heads, spec.n_kv_heads, spec.key_dim, spec.value_dim, spec.conv_taps),), torch.float32)
 
-    def forward(self, h, residual, ctx, cache, then=None, overwrite=False, projected=None):
+    def forward(self, h, residual, ctx, cache, then=None, overwrite=False, projected=None, into=None):
         s, T, o, dev = self.spec, ctx.n_rows, self.offsets, ctx.device
         H, G, dk, dv = s.n_heads, s.n_kv_heads, s.key_dim, s.value_dim
         vv = H * dv
@@ -123,10 +130,10 @@ class GatedDelta(Mixer):
         if proj is None:
             proj = torch.empty((T, self.w_in.shape[0]), dtype=torch.float32, device=dev)
             linear(h, self.w_in, proj, ctx=ctx)
-        seg_start, seg_len = ops.segments(ctx)
         qkv = torch.empty((T, 2 * G * dk + vv), dtype=torch.float32, device=dev)
         gates = torch.empty((T, self.n_decays + H), dtype=torch.float32, device=dev)
         single_rows = ctx.max_seg_len == 1            # (a step's shape, which a captured pass shares with its replays)
+        seg_start, seg_len = (None, None) if single_rows else ops.segments(ctx)
         a, gate, a_up, gate_up = o.get("a"), proj[:, o["g"]:o["g"] + vv] if "g" in o else None, None, None
         if self.w_low is not None and T <= self.few_rows:
             if "low_a" in o:
@@ -152,8 +159,10 @@ class GatedDelta(Mixer):
             chunked = ops.delta_chunks(qkv, gates, seg_start, seg_len, ctx.seg_len, self.ROWS_IN_BLOCKS, ctx.row_slot, cache.state, read, H, G, dk, dv) is not None
         if not chunked or min(ctx.seg_len) < self.ROWS_IN_BLOCKS:
             ops.delta_scan(qkv, gates, seg_start, seg_len, ctx.row_slot, cache.state, read, H, G, dk, dv, s.channel_decay, single_rows, self.ROWS_IN_BLOCKS if chunked else 0)
-        mid = torch.empty((T, vv), dtype=self.mid_dtype, device=dev)
+        mid = into if into is not None else torch.empty((T, vv), dtype=self.mid_dtype, device=dev)
         ops.head_norm_gate(read, gate, self.out_norm, s.norm_eps, mid, H, dv, gate_activation=s.gate_activation, gate_up=gate_up)
+        if into is not None:
+            return None
         if overwrite:
             linear(mid, self.w_o, residual, ctx=ctx)
             return None

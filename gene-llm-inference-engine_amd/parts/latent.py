@@ -110,6 +110,12 @@ class LatentAttention(Mixer):
     def use_input_weight(self, view):
         self.w_down = view
 
+    def output_weight(self):         # (see `GatedDelta.output_weight`)
+        return self.w_o if self.att_dtype == torch.bfloat16 else None
+
+    def use_output_weight(self, view):
+        self.w_o = view
+
     @classmethod
     def tensor_needs(cls, spec):
         s, d = spec, spec.hidden_size
@@ -126,7 +132,7 @@ class LatentAttention(Mixer):
     def cache_need(cls, spec):
         return PagedKvNeed(1, spec.kv_rank + spec.rotary_dim, spec.window, spec.kv_rank, None)
 
-    def forward(self, h, residual, ctx, cache, then=None, overwrite=False, projected=None):
+    def forward(self, h, residual, ctx, cache, then=None, overwrite=False, projected=None, into=None):
         s, T, dev = self.spec, ctx.n_rows, ctx.device
         H, kd = s.n_heads, self.key_dim
         down = projected
@@ -155,10 +161,12 @@ class LatentAttention(Mixer):
                                   window=s.window, scale=s.scale, sinks=self.sinks)
         if attended.dtype != activation_dtype_for(self.w_uv, self.dtype):
             attended = attended.to(activation_dtype_for(self.w_uv, self.dtype))
-        att = torch.empty((T, H * s.value_dim), dtype=self.att_dtype, device=dev)
+        att = into if into is not None else torch.empty((T, H * s.value_dim), dtype=self.att_dtype, device=dev)
         heads_product(attended, self.w_uv, att, H, channel_gate=down[:, self.gate_at:self.gate_at + H * s.value_dim] if self.channel_gated else None)
         if self.gated:
             ops.head_gate(att, down[:, self.gate_at:self.gate_at + H], H, s.value_dim)
+        if into is not None:
+            return None
         if overwrite:
             linear(att, self.w_o, residual, ctx=ctx)
             return None

@@ -35,9 +35,9 @@ def linear(a, weight: torch.Tensor, out: torch.Tensor, accumulate: bool = False,
     return ops.gemm_exact(a, weight, out, accumulate)
 
 
-def linear_xielu(a, weight: torch.Tensor, params: torch.Tensor, columns: int, dtype: torch.dtype, out: torch.Tensor = None):
+def linear_xielu(a, weight: torch.Tensor, params: torch.Tensor, columns: int, dtype: torch.dtype, out: torch.Tensor = None, into: torch.Tensor = None):
     """The product of `linear` with the activation of a feed-forward that has no gate in its epilogue, where a kernel does both
-    (`ops.gemm_bf16_xielu`): its last `columns` columns come back activated, as `dtype`, the ones before go to out.  None where no
+    (`ops.gemm_bf16_xielu`): its last `columns` columns come back activated, as `dtype` (in `into`, if given), the ones before go to out.  None where no
     kernel does, and out is as it was."""
     n, k = weight.shape
     rows = a.n_rows if isinstance(a, NormedRows) else a.shape[0]
@@ -52,7 +52,7 @@ def linear_xielu(a, weight: torch.Tensor, params: torch.Tensor, columns: int, dt
         a = a.materialize()                      # (kept by `a` for whoever asks next)
     if not ops.gemm_bf16_supports(a, weight, weight):
         return None
-    mid = torch.empty((rows, columns), dtype=dtype, device=weight.device)
+    mid = into if into is not None else torch.empty((rows, columns), dtype=dtype, device=weight.device)
     return ops.gemm_bf16_xielu(a, weight, params, mid, out, norm_in)
 
 

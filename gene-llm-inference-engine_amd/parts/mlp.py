@@ -99,23 +99,33 @@ class DenseMlp(FeedForward):
     def use_input_weight(self, view):
         self.w_up = view
 
+    # ... and the last product's, for a block that makes several parts' last products in one: it then hands the part the columns of a common
+    # buffer that its rows go to (`forward(..., into=)`), and the part leaves the product to the block.
+    def output_weight(self):
+        return self.w_down if self.mid_dtype == torch.bfloat16 else None
+
+    def use_output_weight(self, view):
+        self.w_down = view
+
     def input_activation(self):
         """What a block's product of several parts' first matrices does to this one's columns where it can (`linear_xielu`), which `forward`
         then takes as `activated`: the activation's parameters, the number of columns, what they are stored as."""
         return self.params, self.spec.intermediate_size, self.mid_dtype
 
-    def forward(self, h, residual, ctx, then=None, overwrite=False, projected=None, activated=None):
+    def forward(self, h, residual, ctx, then=None, overwrite=False, projected=None, activated=None, into=None):
         T, inter = ctx.n_rows, self.spec.intermediate_size
         mid = activated
         if mid is None and projected is None:        # (the activation in the epilogue of the product where that can be: of its own it costs 27 us a layer for 1,777 rows of 8,192)
-            mid = linear_xielu(h, self.w_up, *self.input_activation())
+            mid = linear_xielu(h, self.w_up, *self.input_activation(), into=into)
         if mid is None:
             up = projected
             if up is None:
                 up = torch.empty((T, inter), dtype=torch.float32, device=ctx.device)
                 linear(h, self.w_up, up, ctx=ctx)
-            mid = torch.empty((T, inter), dtype=self.mid_dtype, device=ctx.device)
+            mid = into if into is not None else torch.empty((T, inter), dtype=self.mid_dtype, device=ctx.device)
             ops.xielu(up, mid, self.params)
+        if into is not None:
+            return None
         if overwrite:
             linear(mid, self.w_down, residual, ctx=ctx)
             return None

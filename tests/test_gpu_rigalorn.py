@@ -291,6 +291,24 @@ def test_delta_rule_sums_in_one_order(heads, kv, dk, dv, spare, channel):
     assert torch.equal(one, out[21:22]) and torch.equal(one_state[0], state[0])
 
 
+@pytest.mark.parametrize("channel", [False, True])
+def test_delta_rule_of_single_rows_needs_no_runs(channel):
+    from geneinfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(9)
+    heads, kv, dk, dv, n = 4, 2, 40, 10, 5
+    qkv, gates = torch.randn(n, 2 * kv * dk + heads * dv, generator=g).to(DEV), torch.rand(n, heads * ((dk if channel else 1) + 1), generator=g).to(DEV)
+    slot, rows = torch.tensor([3, 0, 5, 1, 2], dtype=torch.int32, device=DEV), torch.arange(n, dtype=torch.int32, device=DEV)
+    first = torch.randn(6, ops.delta_memory_floats(heads, dk, dv), generator=g).to(DEV)
+    got = []
+    for runs in ((rows, torch.ones_like(rows)), (None, None)):
+        state, out = first.clone(), torch.empty(n, heads * dv, device=DEV)
+        ops.delta_scan(qkv, gates, *runs, slot, state, out, heads, kv, dk, dv, channel=channel, single_rows=True)
+        got.append((state, out))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    with pytest.raises(ops.KernelError):
+        ops.delta_scan(qkv, gates, None, None, slot, state, out, heads, kv, dk, dv, channel=channel)
+
+
 def _delta_inputs(lens, heads, kv, dv, seed, steps=None, spare=0):
     """Rows as `delta_prepare` leaves them: unit keys, queries of length 1/8, decays as at initialisation, and where given one step size for all."""
     g = torch.Generator().manual_seed(seed)

@@ -77,3 +77,52 @@ def test_a_feed_forward_gets_its_columns_as_it_takes_them(kind, taken, monkeypat
         assert told["activated"] is ready and told["projected"] is None
     else:
         assert torch.equal(told["projected"], x.bfloat16().float() @ up.float().T) and told.get("activated") is None
+
+
+class EndingMixer(Mixer):
+    def __init__(self, spec, tensors, dtype, device):
+        super().__init__(spec, tensors, dtype, device)
+        self.w_o = tensors["o"]
+
+    def output_weight(self):
+        return self.w_o
+
+    def use_output_weight(self, view):
+        self.w_o = view
+
+    def forward(self, h, residual, ctx, cache, then=None, projected=None, into=None):
+        ends = torch.arange(h.shape[0] * MIX).view(-1, MIX).bfloat16()
+        if into is None:
+            residual += ends.float() @ self.w_o.float().T
+        else:
+            into.copy_(ends)
+
+
+@pytest.mark.parametrize("traced", [False, True])
+def test_both_halves_end_in_one_product(traced, monkeypatch):
+    """The halves write the two parts of one buffer, which meets the matrices side by side; a traced pass, which looks at the rows between the halves, has two products.  Either way the
+    weights count once."""
+    base.register_mixer("ending", EndingMixer)
+    tensors = dict(mix=torch.randn(MIX, D).bfloat16(), o=torch.randn(D, MIX).bfloat16(), up=torch.randn(INTER, D).bfloat16(), down=torch.randn(D, INTER).bfloat16(), act=torch.tensor([0.3, 0.1]))
+    ff = Spec(kind="dense_mlp", activation="xielu", activation_params="act", up_proj="up", down_proj="down", intermediate_size=INTER, hidden_size=D)
+    spec = Spec(feed_forward_norm=None, mixer_post_norm=None, feed_forward_post_norm=None, mixer_norm=Spec(kind="stand_in"), mixer=Spec(kind="ending"), feed_forward=ff)
+    b = block.ParallelBlock(spec, tensors, torch.bfloat16, "cpu")
+    matrices = sum(tensors[n].numel() * 2 for n in ("mix", "o", "up", "down"))
+    assert matrices <= base.weight_bytes(b) <= matrices + 2 * (MIX + INTER) * D + 64          # (the first products' common matrix is named beside its second half)
+    x, seen, products = torch.randn(3, D), [], []
+    mid = torch.randn(3, INTER).bfloat16()
+
+    def activated(a, weight, params, columns, dtype, out, into=None):
+        return mid if into is None else into.copy_(mid)
+
+    def onto(a, weight, residual, then=None, ctx=None):
+        products.append((a.shape[1], weight.shape[1]))
+        residual += a.float() @ weight.float().T
+
+    monkeypatch.setattr(block, "linear_xielu", activated)
+    for module in (block, __import__("geneinfer_amd.parts.mlp", fromlist=["mlp"])):
+        monkeypatch.setattr(module, "linear_onto", onto)
+    want = x + torch.arange(3 * MIX).view(3, MIX).bfloat16().float() @ tensors["o"].float().T + mid.float() @ tensors["down"].float().T
+    b.forward(x, Spec(n_rows=3, dtype=torch.bfloat16, trace=(lambda name, rows: seen.append(name)) if traced else None), None)
+    assert torch.allclose(x, want, rtol=1e-5, atol=1e-3)
+    assert (products, seen) == (([(INTER, INTER)], ["attn_out", "ffn_out"]) if traced else ([(MIX + INTER, MIX + INTER)], []))
