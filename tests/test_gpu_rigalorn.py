@@ -500,6 +500,38 @@ def test_attention_with_biases_blended_values_and_one_key_that_stands_out(T, win
     assert relative_error(out.view(T, heads, dv)[T - 1], want[T - 1]) < 2e-5
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads, kv, dk, dv, rot, page, extras", [(4, 2, 64, 64, 32, 16, "all"), (6, 3, 24, 10, 8, 8, "all"), (2, 2, 4, 7, 0, 24, "biases"), (5, 1, 128, 128, 128, 4, "none"), (4, 2, 64, 33, 16, 16, "growth")])
+def test_rows_of_prompts_are_turned_and_stored_as_rows_one_by_one(heads, kv, dk, dv, rot, page, extras, dtype):
+    """64 rows or more of three requests (one from the middle of eight positions on, one of a few rows that shares windows with both others, one from a multiple of eight) in the kernel
+    for many rows, and the same rows ten at a time: queries, pages and kept values in bits."""
+    from geneinfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(dk + dv)
+    lens, firsts = [75, 4, 90], [5, 63, 16]
+    n = sum(lens)
+    q, k, v, other = (torch.randn(n, width, generator=g).to(DEV) for width in (heads * dk, kv * dk, kv * dv, kv * dv))
+    biases = tuple(torch.randn(width, generator=g).to(DEV) for width in (heads * dk, kv * dk, kv * dv)) if extras in ("all", "biases") else None
+    blend = (other, torch.tensor([0.35], device=DEV)) if extras == "all" else None
+    pos = torch.cat([torch.arange(p, p + m) for p, m in zip(firsts, lens)]).to(DEV, torch.int32)
+    slot = torch.cat([torch.full((m,), s) for s, m in zip((2, 0, 1), lens)]).to(DEV, torch.int32)
+    pages = 3 * -(-106 // page)
+    table = torch.randperm(pages, generator=g).view(3, -1).to(DEV, torch.int32)
+    cos, sin = (torch.randn(n, rot // 2, generator=g).to(DEV) for _ in range(2)) if rot else (None, None)
+    got = []
+    for step in (n, 10):
+        cache = torch.full((pages, kv * (dk + dv) * page), 9.0, dtype=dtype, device=DEV).view(pages, 1, kv * (dk + dv), page)
+        q_out, keep = torch.empty(n, heads * dk, dtype=dtype, device=DEV), torch.empty(n, kv * dv, device=DEV) if extras == "all" else None
+        for a in range(0, n, step):
+            b = min(n, a + step)
+            cut = lambda x: None if x is None else x[a:b]
+            ops.norm_rope_store(q[a:b], k[a:b], v[a:b], None, None, 1e-6, cut(cos), cut(sin), rot, pos[a:b], slot[a:b], table, q_out[a:b], cache, page, heads, kv, dk, dv, biases=biases,
+                                blend=None if blend is None else (other[a:b], blend[1]), keep=cut(keep), v_scale=0.7 if extras == "biases" else 1.0,
+                                query_growth=(0.1, 20.0) if extras == "growth" else None)
+        got.append((q_out, cache, keep))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and (got[0][2] is None or torch.equal(got[0][2], got[1][2]))
+    assert bool((got[0][1] != 9.0).any())
+
+
 @pytest.mark.parametrize("T, window, far", [(200, None, 2), (200, 50, 150), (200, 50, 149), (45, 16, 29), (45, 16, 30)])
 def test_attention_through_latents_against_keys_and_values_made_in_full(T, window, far):
     """The kernels around the latent cache and the attention over it, with the up projections folded into query and output by hand
