@@ -21,7 +21,7 @@
 //
 // Two kernels.  Which one serves depends on the data types and on hd, vd, the page size, the window and the chunk alone, so one layer meets one of them:
 //   tiles    32-bit throughout, hd and vd multiples of 16 up to 128, pages of a multiple of 4, rows that may see more than 16 keys: both products
-//            on the 32-bit matrix instructions, four waves a workgroup, long contexts shared out over workgroups;
+//            on the 32-bit matrix instructions, four waves a workgroup, long contexts shared out over workgroups (in blocks of 64 keys, by a kernel of the same sums, where the tiles are few);
 //   rows     everything else: one wave per (row, query head), keys 64 at a time.
 #include "common.h"
 
@@ -320,6 +320,217 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attention_exact_tiles_ke
     }
 }
 
+// The same numbers where the tiles are few: a workgroup per block of 64 keys, its four waves each with 16 of the keys for the scores and with every fourth 16 channels for the second product
+// (the probabilities change hands in LDS).  Every sum is the one above, of the same operands in the same order.  What a block gives is left in `part` (per (row, head, block): vd
+// sums, then l and m); the meeting of a span's blocks is the join kernel's too.  Bound by a wave's chain of
+// instructions, which is a third of the one above, and by its loads' two round trips.  With the join, spans to a workgroup and blocks: 3 rows at 600 positions, 32/8 heads of 64, 17.5 us and 10.7;
+// 1 row 15.3 and 9.6, 8 rows at 1,000 18.1 and 15.7; 24/8 heads of 128, 3 rows at 600 25.7 and 12.9, 16 at 1,000 51 and 41.
+template <int D>
+__global__ __launch_bounds__(256, 2) void attention_exact_blocks_kernel(const float* __restrict__ q, const float* __restrict__ cache, const int* __restrict__ pos, const int* __restrict__ slot,
+                                                                       const int* __restrict__ table, int table_stride, long page_stride, Divisor pages, int n_rows, int n_heads, int n_kv,
+                                                                       int hd, int vd, int window, int chunk, float scale, float cap, int n_single, int rows_a_tile, float* __restrict__ part,
+                                                                       int n_blocks) {
+    constexpr int OWN = D / 64;                                    // groups of 16 channels a wave has: wave, wave + 4, ...
+    __shared__ float m_s[4][PAIRS];
+    __shared__ f32x4 p_s[4][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+    const int group = n_heads / n_kv, head_tiles = (group + PAIRS - 1) / PAIRS;
+    const int tile = blockIdx.x / (n_kv * head_tiles), kv = blockIdx.x / head_tiles % n_kv, ht = blockIdx.x % head_tiles;
+    const int heads_here = min(PAIRS, group - ht * PAIRS);
+    const int rows_here = tile < n_single ? 1 : rows_a_tile, t_first = tile < n_single ? tile : n_single + (tile - n_single) * rows_a_tile;
+    const int place = r / heads_here, t = t_first + place, h = kv * group + ht * PAIRS + r % heads_here;
+    const bool valid = place < rows_here && t < n_rows;
+    const int my_pos = valid ? pos[t] : 0, my_slot = valid ? slot[t] : -1, my_lo = valid ? first_key(my_pos, window, chunk) : 0;
+    f32x4 qv[D / 16];
+#pragma unroll
+    for (int c = 0; c < D / 16; ++c)
+        qv[c] = valid && c * 16 < hd ? *reinterpret_cast<const f32x4*>(q + ((size_t)t * n_heads + h) * hd + c * 16 + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
+    const int page_size = pages.size;
+    const long v_plane = (long)n_kv * page_size * hd;
+    bool todo = valid;
+    unsigned turn = 0;
+    while (__ballot(todo) != 0) {                                  // (a request's rows at a time, as above)
+        const int run_slot = __builtin_amdgcn_readfirstlane(__shfl(my_slot, (int)__ffsll((unsigned long long)__ballot(todo)) - 1, 64));
+        const bool in_run = todo && my_slot == run_slot;
+        todo = todo && !in_run;
+        if (turn++ % gridDim.z != blockIdx.z) continue;
+        int lo_min = in_run ? my_lo : 2147483647, lo_max = in_run ? my_lo : 0, p_min = in_run ? my_pos : 2147483647, p_max = in_run ? my_pos : 0;
+#pragma unroll
+        for (int off = 1; off < PAIRS; off <<= 1) {
+            lo_min = min(lo_min, __shfl_xor(lo_min, off, 64));
+            lo_max = max(lo_max, __shfl_xor(lo_max, off, 64));
+            p_min = min(p_min, __shfl_xor(p_min, off, 64));
+            p_max = max(p_max, __shfl_xor(p_max, off, 64));
+        }
+        lo_min = __builtin_amdgcn_readfirstlane(lo_min);
+        p_max = __builtin_amdgcn_readfirstlane(p_max);
+        const int* tab = table + (size_t)run_slot * table_stride;
+        for (int block = lo_min / BLOCK + blockIdx.y; block <= p_max / BLOCK; block += gridDim.y) {
+            const int b0 = block * BLOCK;
+            bool live[4];
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) live[kt] = b0 + kt * 16 <= p_max && b0 + kt * 16 + 16 > lo_min;
+            f32x4 kk[D / 16], vv[4][OWN];
+            {
+                const int key = max(min(b0 + wave * 16 + r, p_max), lo_min), page = quotient(key, pages);
+                const float* from = cache + (size_t)tab[page] * page_stride + ((size_t)kv * page_size + key - page * page_size) * hd + 4 * g;
+#pragma unroll
+                for (int c = 0; c < D / 16; ++c) kk[c] = c * 16 < hd ? *reinterpret_cast<const f32x4*>(from + c * 16) : f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) {
+                const int key = max(min(b0 + kt * 16 + 4 * g, p_max), lo_min) & ~3, page = quotient(key, pages);
+                const float* from = cache + (size_t)tab[page] * page_stride + v_plane + ((size_t)kv * vd + r) * page_size + key - page * page_size;
+#pragma unroll
+                for (int e = 0; e < OWN; ++e) {
+                    const int c = wave + 4 * e;
+                    vv[kt][e] = c * 16 < vd ? *reinterpret_cast<const f32x4*>(from + (size_t)c * 16 * page_size) : f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+            }
+            f32x4 sc = {0.f, 0.f, 0.f, 0.f};
+            float m = -INFINITY;
+            const bool mine = b0 + wave * 16 <= p_max && b0 + wave * 16 + 16 > lo_min;
+            if (mine) {
+#pragma unroll
+                for (int c = 0; c < D / 16; ++c)
+                    if (c * 16 < hd) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) sc = mfma(kk[c][j], qv[c][j], sc);
+                    }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int key = b0 + wave * 16 + 4 * g + i;
+                    float x = sc[i] * scale;
+                    if (cap > 0.f) x = cap * tanhf(x / cap);
+                    sc[i] = in_run && key <= my_pos && key >= my_lo ? x : -INFINITY;
+                    m = fmaxf(m, sc[i]);
+                }
+                m = fmaxf(m, __shfl_xor(m, 16, 64));
+                m = fmaxf(m, __shfl_xor(m, 32, 64));
+            }
+            if (g == 0) m_s[wave][r] = m;
+            __syncthreads();
+            m = fmaxf(fmaxf(m_s[0][r], m_s[1][r]), fmaxf(m_s[2][r], m_s[3][r]));
+            if (mine) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sc[i] = sc[i] == -INFINITY ? 0.f : expf(sc[i] - m);
+                p_s[wave][lane] = sc;
+            }
+            __syncthreads();
+            f32x4 p[4];
+            float l = 0.f;
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) {
+                p[kt] = p_s[kt][lane];                             // (nobody has written what is not live)
+                if (!live[kt]) continue;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) l += p[kt][i];
+            }
+            l += __shfl_xor(l, 16, 64);
+            l += __shfl_xor(l, 32, 64);
+            __syncthreads();                                       // the next block writes them anew
+            bool odd = false;                                      // (values that are no numbers: as above)
+            if (!(b0 >= lo_max && b0 + BLOCK - 1 <= p_min)) {
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt) {
+                    if (!live[kt]) continue;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int key = b0 + kt * 16 + 4 * g + i;
+#pragma unroll
+                        for (int e = 0; e < OWN; ++e) {
+                            if (key > p_max || key < lo_min) vv[kt][e][i] = 0.f;
+                            odd = odd || !(fabsf(vv[kt][e][i]) < INFINITY);
+                        }
+                    }
+                }
+            }
+            f32x4 o[OWN];
+#pragma unroll
+            for (int e = 0; e < OWN; ++e) o[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) {
+                if (!live[kt]) continue;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int e = 0; e < OWN; ++e) o[e] = mfma(vv[kt][e][j], p[kt][j], o[e]);
+            }
+            if (__ballot(odd) != 0) {
+                for (int row = 0; row < rows_here; ++row) {
+                    const int row_pos = __shfl(my_pos, row * heads_here, 64), row_lo = __shfl(my_lo, row * heads_here, 64);
+#pragma unroll
+                    for (int e = 0; e < OWN; ++e) {
+                        f32x4 own = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int kt = 0; kt < 4; ++kt) {
+                            if (!live[kt]) continue;
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) {
+                                const int key = b0 + kt * 16 + 4 * g + j;
+                                own = mfma(key > row_pos || key < row_lo ? 0.f : vv[kt][e][j], p[kt][j], own);
+                            }
+                        }
+                        if (place == row) o[e] = own;
+                    }
+                }
+            }
+            const int at = block - my_lo / BLOCK;
+            if (!in_run || at < 0 || block > my_pos / BLOCK || at >= n_blocks) continue;
+            float* to = part + (((size_t)t * n_heads + h) * n_blocks + at) * part_floats(vd);
+#pragma unroll
+            for (int e = 0; e < OWN; ++e)
+                if ((wave + 4 * e) * 16 < vd) *reinterpret_cast<f32x4*>(to + (wave + 4 * e) * 16 + 4 * g) = o[e];
+            if (wave == 0 && g == 0) *reinterpret_cast<float2*>(to + vd) = float2{l, m};
+        }
+    }
+}
+
+// What those blocks left of a (row, head), joined: a span's four blocks as the kernel above joins them, then span after span.  Four spans' numbers are asked for at once.
+__global__ __launch_bounds__(128) void attention_exact_join_blocks_kernel(const float* __restrict__ part, float* __restrict__ out, const int* __restrict__ pos, int n_heads, int vd,
+                                                                         int window, int chunk, const float* __restrict__ sinks, const float* __restrict__ gate, long gate_stride,
+                                                                         int gate_channels, int n_blocks) {
+    const int t = blockIdx.x / n_heads, h = blockIdx.x % n_heads, d = threadIdx.x, p = pos[t], lo = first_key(p, window, chunk);
+    const int first = lo / BLOCK, last = min(p / BLOCK, first + n_blocks - 1), channel = min(d, vd - 1);
+    const float* from = part + (size_t)blockIdx.x * n_blocks * part_floats(vd);
+    float m = sinks ? sinks[h] : -INFINITY, o = 0.f;
+    double l = sinks ? 1.0 : 0.0;
+    constexpr int AT_ONCE = 4;
+    for (int s0 = first / 4; s0 <= last / 4; s0 += AT_ONCE) {
+        float o_block[4 * AT_ONCE];
+        float2 lm[4 * AT_ONCE];
+#pragma unroll
+        for (int b = 0; b < 4 * AT_ONCE; ++b) {
+            const float* block = from + (size_t)(min(max(s0 * 4 + b, first), last) - first) * part_floats(vd);
+            o_block[b] = block[channel];
+            lm[b] = *reinterpret_cast<const float2*>(block + vd);
+        }
+#pragma unroll
+        for (int s = 0; s < AT_ONCE; ++s) {
+            if (s0 + s > last / 4) break;
+            float top = -INFINITY;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const int block = (s0 + s) * 4 + b;
+                if (block >= first && block <= last) top = fmaxf(top, lm[4 * s + b].y);
+            }
+            double l_span = 0.0;
+            float o_span = 0.f;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const int block = (s0 + s) * 4 + b;
+                if (block < first || block > last) continue;
+                const float f = lm[4 * s + b].y == -INFINITY ? 0.f : expf(lm[4 * s + b].y - top);
+                l_span = fma((double)lm[4 * s + b].x, (double)f, l_span);
+                o_span = fmaf(o_block[4 * s + b], f, o_span);
+            }
+            const Join f = join(m, l, true, top, l_span);
+            o = joined(o, o_span, f);
+        }
+    }
+    if (d < vd) out[(size_t)blockIdx.x * vd + d] = finished(o, l, gate, gate_stride, gate_channels, t, h, d);
+}
+
 // The spans of a (row, head), left by several workgroups, joined in order.
 __global__ __launch_bounds__(128) void attention_exact_join_kernel(const float* __restrict__ part, float* __restrict__ out, const int* __restrict__ pos, int n_heads, int vd,
                                                                   int window, int chunk, const float* __restrict__ sinks, const float* __restrict__ gate, long gate_stride,
@@ -434,7 +645,18 @@ GI_API int gi_attention_exact_spans(int n_rows, int n_single, int n_heads, int n
     if (tiles >= 2L * gi_compute_units() || spans > MAX_SPANS || spans * n_rows * n_heads * part_floats(vd) > (16L << 20)) return 0;
     return (int)spans;
 }
-GI_API long gi_attention_exact_part_floats(int n_rows, int n_heads, int vd, int n_spans) { return (long)n_rows * n_heads * n_spans * part_floats(vd); }
+// Whether the spans' blocks of 64 keys then go out one by one: with heads of more than 64 channels (spans and blocks, 24/8 heads of 128: 40 rows of their own at 1,000 positions 117 us and 80, 60 at 4,000
+// 574 and 403, a prompt of 64 rows at 1,000 47 and 41; 32 such rows 26.3 and 27.4, 250 at 300 56 and 57), else up to so many blocks as the tiles see at most, fewer where contexts are long, and while the
+// join has few parts to read (32/8 heads of 64: 12 rows at 300, 600, 1,000 positions 18.6 and 12.4, 18.7 and 15.1, 22.2 and 21.6; 16 at 1,000 23.2 and 25.6; 5 at 2,000 22.6 and 22.3, 8 at 2,000 24.9 and
+// 28.0; 1 at 4,000 22.5 and 20.8, 3 at 4,000 26.4 and 29.5; a prompt of 16 rows at 1,000 16.6 and 13.3, of 32 17.2 and 19.2).
+static bool by_blocks(int n_rows, int n_single, int n_heads, int n_kv, int hd, int vd, int n_spans) {
+    const long blocks = count_tiles(n_rows, n_single, n_kv, n_heads / n_kv) * 4 * (n_spans - 1);
+    return 4L * n_spans * n_rows * n_heads * part_floats(vd) <= (16L << 20) && 4 * n_spans <= MAX_SPANS && 
+           (hd > 64 || vd > 64 || ((long)n_rows * n_heads <= 512 && blocks <= (n_spans <= 5 ? 1536 : n_spans <= 9 ? 1280 : 512)));
+}
+GI_API long gi_attention_exact_part_floats(int n_rows, int n_single, int n_heads, int n_kv, int hd, int vd, int n_spans) {
+    return (long)n_rows * n_heads * n_spans * (by_blocks(n_rows, n_single, n_heads, n_kv, hd, vd, n_spans) ? 4 : 1) * part_floats(vd);
+}
 
 GI_API int gi_attention_exact(const void* q, int q_dtype, const void* cache, int cache_dtype, void* out, int out_dtype, const int* pos,
                               const int* slot, const int* table, int table_stride, long page_stride, int page_size, int n_rows,
@@ -454,8 +676,8 @@ GI_API int gi_attention_exact(const void* q, int q_dtype, const void* cache, int
         GI_REQUIRE(n_single >= 0 && n_single <= n_rows, "attention_exact: %d single rows of %d", n_single, n_rows);
         const int a_tile = rows_a_tile(n_heads / n_kv), turns = n_single == n_rows ? 1 : n_requests > 0 && n_requests < a_tile ? n_requests : a_tile;
         if (n_spans > 0) {
-            GI_REQUIRE(part != nullptr && aligned(part) && part_size >= gi_attention_exact_part_floats(n_rows, n_heads, vd, n_spans) && n_spans <= MAX_SPANS,
-                       "attention_exact: sharing the keys out needs %ld floats", gi_attention_exact_part_floats(n_rows, n_heads, vd, n_spans));
+            GI_REQUIRE(part != nullptr && aligned(part) && part_size >= (long)n_rows * n_heads * n_spans * part_floats(vd) && n_spans <= MAX_SPANS,
+                       "attention_exact: sharing the keys out needs %ld floats", (long)n_rows * n_heads * n_spans * part_floats(vd));
         } else {
             part = nullptr;
         }
@@ -463,6 +685,20 @@ GI_API int gi_attention_exact(const void* q, int q_dtype, const void* cache, int
         while ((1LL << pages.shift) < page_size) ++pages.shift;
         pages.magic = (unsigned)((((1ULL << pages.shift) - page_size) << 32) / page_size + 1);
         const dim3 tiles((unsigned)count_tiles(n_rows, n_single, n_kv, n_heads / n_kv), part ? n_spans : 1, turns);
+        if (part && by_blocks(n_rows, n_single, n_heads, n_kv, hd, vd, n_spans) && part_size >= 4L * n_rows * n_heads * n_spans * part_floats(vd)) {
+            const int n_blocks = 4 * n_spans;
+            const dim3 blocks(tiles.x, n_blocks, tiles.z);
+#define BLOCKS(D)                                                                                                                          \
+    attention_exact_blocks_kernel<D><<<blocks, 256, 0, stream>>>((const float*)q, (const float*)cache, pos, slot, table, table_stride, page_stride, pages, n_rows, n_heads, n_kv, hd, vd, window, \
+                                                                 chunk, scale, cap, n_single, a_tile, part, n_blocks)
+            if (hd <= 64 && vd <= 64) BLOCKS(64);
+            else BLOCKS(128);
+#undef BLOCKS
+            GI_CHECK_LAUNCH("attention_exact (blocks)");
+            attention_exact_join_blocks_kernel<<<grid, 128, 0, stream>>>(part, (float*)out, pos, n_heads, vd, window, chunk, sinks, gate, gate_stride, gate_channels, n_blocks);
+            GI_CHECK_LAUNCH("attention_exact (join)");
+            return 0;
+        }
 #define TILES(D)                                                                                                                           \
     attention_exact_tiles_kernel<D><<<tiles, 256, 0, stream>>>((const float*)q, (const float*)cache, (float*)out, pos, slot, table, table_stride, page_stride, pages, n_rows, \
                                                                n_heads, n_kv, hd, vd, window, chunk, scale, cap, sinks, gate, gate_stride, gate_channels, n_single, a_tile, part, n_spans)

@@ -139,7 +139,7 @@ def lib():
         l.gi_sample_filtered_histogram_bytes.restype = c_int
         l.gi_attention_exact_spans.argtypes = [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int]
         l.gi_attention_exact_spans.restype = c_int
-        l.gi_attention_exact_part_floats.argtypes = [c_int, c_int, c_int, c_int]
+        l.gi_attention_exact_part_floats.argtypes = [c_int, c_int, c_int, c_int, c_int, c_int, c_int]
         l.gi_attention_exact_part_floats.restype = c_long
         l.gi_attention_exact_max_head_size.argtypes = []
         l.gi_attention_exact_max_head_size.restype = c_int
@@ -695,9 +695,8 @@ def attention_exact(q, cache, out, positions, slots, table, n_heads, n_kv, hd, w
     part, n_part, n_spans = None, 0, 0
     if max_context is not None and q.dtype == torch.float32:
         seen = min([int(max_context)] + ([int(window)] if window else []) + ([int(chunk)] if chunk else []))
-        n_spans = _exact_spans(n, n_single, n_heads, n_kv, hd, vd, page_size, -(-seen // 256) * 256)
+        n_spans, n_part = _exact_spans(n, n_single, n_heads, n_kv, hd, vd, page_size, -(-seen // 256) * 256)
         if n_spans:
-            n_part = lib().gi_attention_exact_part_floats(n, n_heads, vd, n_spans)
             part = torch.empty(n_part, dtype=torch.float32, device=out.device)
     _call("gi_attention_exact", q.data_ptr(), _code(q, "attention: q"), cache.data_ptr(), _code(cache, "attention: cache"), out.data_ptr(),
           _code(out, "attention: out"), positions.data_ptr(), slots.data_ptr(), table.data_ptr(), table.stride(0), cache.stride(0),
@@ -707,8 +706,10 @@ def attention_exact(q, cache, out, positions, slots, table, n_heads, n_kv, hd, w
 
 
 @lru_cache(maxsize=1024)
-def _exact_spans(n, n_single, n_heads, n_kv, hd, vd, page_size, seen) -> int:
-    return lib().gi_attention_exact_spans(n, n_single, n_heads, n_kv, hd, vd, page_size, seen)
+def _exact_spans(n, n_single, n_heads, n_kv, hd, vd, page_size, seen):
+    """(spans a row has at most where they are shared out, else 0; floats for their parts)"""
+    spans = lib().gi_attention_exact_spans(n, n_single, n_heads, n_kv, hd, vd, page_size, seen)
+    return spans, lib().gi_attention_exact_part_floats(n, n_single, n_heads, n_kv, hd, vd, spans) if spans else 0
 
 
 def _gates(gate, channel_gate, n, n_heads, vd):

@@ -1344,6 +1344,46 @@ def test_attention_exact_shares_contexts_out_with_all_it_takes(n_heads, n_kv, hd
         assert torch.equal(attend(**known), whole), known
 
 
+@pytest.mark.parametrize("n_heads,n_kv,hd,vd,window,chunk", [(32, 8, 64, 64, None, None), (16, 16, 48, 64, 300, None), (8, 8, 64, 16, None, 320), (6, 2, 64, 80, None, None), (34, 2, 128, 128, 520, None)])
+def test_attention_exact_of_blocks_one_by_one(n_heads, n_kv, hd, vd, window, chunk):
+    """32-bit: contexts around the ends of blocks of 64 and spans of 256 keys, shared out block by block (few rows), span by span (many) and not at all, rows of their own
+    and rows of one request in a tile: the same bits, and the kernel of each number of rows is the one that the rule's line names."""
+    ps, seen = 16, 1040
+    pages = -(-seen // ps)
+    g = torch.Generator(device=DEV).manual_seed(hd + vd)
+    cache = torch.randn(2 * pages, n_kv * ps * (hd + vd), device=DEV, generator=g)
+    cache[pages + 300 // ps].fill_(float("inf"))                               # met by the rows of the second request that see it
+    table = torch.randperm(pages, device=DEV, generator=g).int()
+    table = torch.stack([table, table + pages])
+    picked = [0, 15, 16, 63, 64, 65, 127, 128, 255, 256, 257, 319, 320, 511, 512, 767, 1023, 1024, 1039]
+    T = 160
+    pos = torch.tensor([picked[i % len(picked)] for i in range(T)], dtype=torch.int32, device=DEV)
+    slots = torch.tensor([i // len(picked) % 2 for i in range(T)], dtype=torch.int32, device=DEV)
+    q = torch.randn(T, n_heads * hd, device=DEV, generator=g)
+    sinks = torch.randn(n_heads, device=DEV, generator=g)
+
+    def attend(first, n, **known):
+        out = torch.full((n, n_heads * vd), 7.0, device=DEV)
+        return ops().attention_exact(q[first:first + n], cache, out, pos[first:first + n], slots[first:first + n], table, n_heads, n_kv, hd, window, page_size=ps, value_dim=vd, cap=30.0,
+                                     sinks=sinks, chunk=chunk, **known).view(torch.int32)
+
+    wide = -(-min(seen, window or seen, chunk or seen) // 256) * 256           # as the wrapper asks
+    spans = ops().lib().gi_attention_exact_spans(2, 2, n_heads, n_kv, hd, vd, ps, wide)
+
+    def parts(n):                                                              # that a span of a (row, head) leaves
+        return ops().lib().gi_attention_exact_part_floats(n, n, n_heads, n_kv, hd, vd, spans) // (n * n_heads * spans * (vd + 4))
+
+    whole = attend(0, T, single_rows=True)
+    few, many = 2, (1536 if spans <= 5 else 1280) // (n_kv * 4 * (spans - 1)) + 1
+    assert spans > 1 and parts(1) == parts(few) == 4 and parts(many) == (1 if hd <= 64 and vd <= 64 else 4)
+    for n, known in ((1, dict(single_rows=True)), (few, dict(single_rows=True)), (19, dict(single_rows=True)), (many, dict(single_rows=True)), (19, dict()), (few + 19, dict(single_rows=few))):
+        for first in (0, 18, T - n if n < T else 0):
+            got = attend(first, n, max_context=seen, **known)
+            assert torch.equal(got, whole[first:first + n]), (n, known, first)
+    clean = torch.isfinite(whole.view(torch.float32)).all(1).tolist()
+    assert clean[0] and any(clean[len(picked):2 * len(picked)]) and all(clean[:len(picked)]) and not all(clean)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_finds_one_far_key(dtype):
     """Among 700 keys one is scaled so that its score stands out: the output must be its value."""
