@@ -571,7 +571,9 @@ __global__ __launch_bounds__(512) void latent_attention_tiles_kernel(const bf16_
 // banks.  A lane reads the key rows in the order that makes its 16 scores the positions 8 h + 0 .. 7 and 16 + 8 h + 0 .. 7 (h: which half of the
 // wave): as they lie, packed, they are the second operand of O^T = V^T P^T, and its first operand is one piece.  A column's maximum follows its scores
 // only when it lags by more than LATENT_SLACK (in units of log2 e; any reference gives the same O / l), which takes the rescaling of the sums off most tiles.
-// 1,777 rows of 32 heads, keys of 288 and values of 256 channels, a window of 1,024: 84 us, 223 in the kernel above.
+// A wave's pieces of a tile are asked for some ahead of their products: with each waited for in turn 1,777 rows of 32 heads, keys of 288 and values of 256 channels, a window of
+// 1,024, took 87 us for now 78 (223 in the kernel above), 500 rows at 3,000 to 3,500 positions 226 and 188.  What bounds it: of the 3,900 clocks of a tile the matrix instructions take 2,180, the
+// other wave of the SIMD beside it mostly doing the same; more pieces ahead have no registers (at 256 of them), and half of the waves a step behind the others was slower (85 us).
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 constexpr float LATENT_SLACK = 8.f;
 template <int KS, int VT>          // keys of up to 32 KS channels, values of up to 32 VT
@@ -580,6 +582,7 @@ __global__ __launch_bounds__(512) void latent_attention_wide_kernel(const bf16_t
                                                                    const int* __restrict__ table, int table_stride, long page_stride, int page_size,
                                                                    int n_heads, int kd, int vd, int window, float scale2, const float* __restrict__ sinks) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    constexpr int AHEAD = KS > 5 ? 3 : 4;                 // pieces of a tile asked for ahead of their product (as many as there are registers for)
     constexpr int KPIECES = 4 * KS, K_BYTES = 32 * KPIECES * 16, V_BYTES = VT * 32 * 64, STAGE = K_BYTES + V_BYTES, PARTS = STAGE / 1024, MOST = (PARTS + 7) / 8;
     static_assert(K_BYTES % 1024 == 0 && V_BYTES % 1024 == 0, "a wave-wide load fills 1 KB");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, half = lane >> 5;
@@ -610,30 +613,51 @@ __global__ __launch_bounds__(512) void latent_attention_wide_kernel(const bf16_t
         }
     }
     const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) void*)lds;
-    auto load_tile = [&](int tk, int place) {
+    int tk = lo_all >> 5;
+    const int tk_last = p_last >> 5;
+    // Where the two blocks of the next tile to ask for lie: their pages are looked up a tile ahead, so that no load waits for the table's answer.
+    int page_next = (tk << 5) / page_size, place_next = (tk << 5) % page_size, pages[2], places[2];
+    auto look_up = [&](int tk) {
+        int at_page[2], at_place[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            at_page[b] = page_next;
+            at_place[b] = place_next;
+            place_next += 16;
+            if (place_next == page_size) { place_next = 0; ++page_next; }
+        }
+        // a block that nobody sees is read from the tile's other one
+        const int b0 = (tk << 5) + 16 <= lo_all ? 1 : 0, b1 = (tk << 5) + 16 > p_last ? 0 : 1;
+        places[0] = b0 ? at_place[1] : at_place[0];
+        places[1] = b1 ? at_place[1] : at_place[0];
+        pages[0] = tab[b0 ? at_page[1] : at_page[0]];
+        pages[1] = tab[b1 ? at_page[1] : at_page[0]];
+    };
+    auto load_tile = [&](int place) {
         const char *keys[2], *values[2];
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {                    // a block that nobody sees is read from one that somebody does
-            const int j0 = __builtin_amdgcn_readfirstlane(min(max((tk << 5) + 16 * b, lo_all & ~15), p_last & ~15)), at = j0 % page_size;
-            const bf16_t* page = cache + (long)tab[j0 / page_size] * page_stride;
-            keys[b] = (const char*)(page + (long)at * kd);
-            values[b] = (const char*)(page + (long)page_size * kd + at);
+        for (int b = 0; b < 2; ++b) {
+            const bf16_t* page = cache + (long)pages[b] * page_stride;
+            keys[b] = (const char*)(page + (long)places[b] * kd);
+            values[b] = (const char*)(page + (long)page_size * kd + places[b]);
         }
 #pragma unroll
         for (int i = 0; i < MOST; ++i) {
             const int part = wave + i * 8;
             if (part < PARTS) {
-                const bool is_key = part * 1024 < K_BYTES, second = (int)from[i] < 0;
-                const char* src = (is_key ? (second ? keys[1] : keys[0]) : (second ? values[1] : values[0])) + (from[i] & 0x7fffffffu);
+                unsigned where = from[i];
+                asm volatile("" : "+v"(where));          // (or what follows from it is kept in registers from tile to tile)
+                const bool is_key = part * 1024 < K_BYTES, second = (int)where < 0;
+                const char* src = (is_key ? (second ? keys[1] : keys[0]) : (second ? values[1] : values[0])) + (where & 0x7fffffffu);
                 const unsigned dst = __builtin_amdgcn_readfirstlane(lds_base + place * STAGE + part * 1024);
                 // (as assembly, so that the compiler does not wait for them before every read of LDS: the wait and the barrier below order them)
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src) : "memory", "m0");
             }
         }
     };
-    int tk = lo_all >> 5;
-    const int tk_last = p_last >> 5;
-    load_tile(tk, 0);
+    look_up(tk);
+    load_tile(0);
+    if (tk < tk_last) look_up(tk + 1);
     bf16x8 qreg[2 * KS];
 #pragma unroll
     for (int s = 0; s < 2 * KS; ++s) {
@@ -652,25 +676,45 @@ __global__ __launch_bounds__(512) void latent_attention_wide_kernel(const bf16_t
     const unsigned char* v_row = lds + K_BYTES + r * 64;
     const int k_off[2] = {(half ^ k_swz) * 16, ((2 + half) ^ k_swz) * 16}, v_off[2] = {(half ^ v_swz) * 16, ((2 + half) ^ v_swz) * 16};
 
+    auto lane_again = [] {                               // (what is rarely used is not kept in registers across the tiles, which take all there are)
+        int l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+        asm volatile("" : "+v"(l));
+        return l;
+    };
     for (int place = 0; tk <= tk_last; ++tk, place ^= 1) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                               // this wave's loads of the tile have landed
         __builtin_amdgcn_s_barrier();                                                  // everyone's have, and nobody reads the other place any more
         asm volatile("" ::: "memory");
-        if (tk < tk_last) load_tile(tk + 1, place ^ 1);
+        if (tk < tk_last) load_tile(place ^ 1);
+        if (tk + 1 < tk_last) look_up(tk + 2);
         const int kv0 = tk << 5;
         if (!works || kv0 + 31 < lo || kv0 > p) continue;
         const unsigned char *kr = k_row + place * STAGE, *vr = v_row + place * STAGE;
+        // piece f of the tile: the keys' along the channels, then the values', all channels of the first 16 positions before the others
+        auto piece_at = [&](int f) {
+            const int i = f - 2 * KS;
+            return as_bf16x8(*reinterpret_cast<const uint4*>(i < 0 ? kr + (f >> 1) * 64 + k_off[f & 1] : vr + (i % VT) * 2048 + v_off[i / VT]));
+        };
+        bf16x8 piece_of[AHEAD];
+#pragma unroll
+        for (int f = 0; f < AHEAD; ++f) piece_of[f] = piece_at(f);
+        __builtin_amdgcn_sched_barrier(0);
         floatx16 s = floatx16{};
 #pragma unroll
-        for (int ks = 0; ks < 2 * KS; ++ks)
-            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(*reinterpret_cast<const uint4*>(kr + (ks >> 1) * 64 + k_off[ks & 1])), qreg[ks], s, 0, 0, 0);
+        for (int f = 0; f < 2 * KS; ++f) {
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(piece_of[f % AHEAD], qreg[f], s, 0, 0, 0);
+            piece_of[f % AHEAD] = piece_at(f + AHEAD);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         // element v: position kv0 + 16 (v / 8) + 8 half + v % 8, head `head`
 #pragma unroll
         for (int v = 0; v < 16; ++v) s[v] *= scale2;
+        asm volatile("" : "+v"(s));                         // (one set of registers either way)
         if (kv0 < lo || kv0 + 31 > p) {
+            const int first = kv0 + 8 * (lane_again() >> 5);
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                const int j = kv0 + 16 * (v >> 3) + 8 * half + (v & 7);
+                const int j = first + 16 * (v >> 3) + (v & 7);
                 s[v] = j >= lo && j <= p ? s[v] : -INFINITY;
             }
         }
@@ -695,20 +739,22 @@ __global__ __launch_bounds__(512) void latent_attention_wide_kernel(const bf16_t
         const bf16x8 pb[2] = {as_bf16x8(uint4{f32x2_to_bf16x2(s[0], s[1]), f32x2_to_bf16x2(s[2], s[3]), f32x2_to_bf16x2(s[4], s[5]), f32x2_to_bf16x2(s[6], s[7])}),
                               as_bf16x8(uint4{f32x2_to_bf16x2(s[8], s[9]), f32x2_to_bf16x2(s[10], s[11]), f32x2_to_bf16x2(s[12], s[13]), f32x2_to_bf16x2(s[14], s[15])})};
 #pragma unroll
-        for (int i = 0; i < VT; ++i)
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-                o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(*reinterpret_cast<const uint4*>(vr + i * 2048 + v_off[ks])), pb[ks], o[i], 0, 0, 0);
+        for (int f = 0; f < 2 * VT; ++f) {
+            o[f % VT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(piece_of[(2 * KS + f) % AHEAD], pb[f / VT], o[f % VT], 0, 0, 0);
+            if (f + AHEAD < 2 * VT) piece_of[(2 * KS + f) % AHEAD] = piece_at(2 * KS + f + AHEAD);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
     if (!works) return;
     l += __shfl_xor(l, 32, 64);
     const float inv = 1.0f / l;                          // (a row always sees itself)
-    bf16_t* to = out + ((size_t)t * n_heads + head) * vd;
+    const int end_lane = lane_again(), end_half = end_lane >> 5;
+    bf16_t* to = out + ((size_t)t * n_heads + (wave % HG) * 32 + (end_lane & 31)) * vd;
 #pragma unroll
     for (int i = 0; i < VT; ++i)
 #pragma unroll
         for (int v = 0; v < 16; v += 4) {
-            const int c = 32 * i + 2 * v + 4 * half;      // element v: channel 32 i + 8 (v / 4) + 4 half + v % 4
+            const int c = 32 * i + 2 * v + 4 * end_half;  // element v: channel 32 i + 8 (v / 4) + 4 half + v % 4
             if (c < vd) *reinterpret_cast<uint2*>(to + c) = uint2{f32x2_to_bf16x2(o[i][v] * inv, o[i][v + 1] * inv), f32x2_to_bf16x2(o[i][v + 2] * inv, o[i][v + 3] * inv)};
         }
 }

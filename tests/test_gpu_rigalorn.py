@@ -636,6 +636,38 @@ def test_matrix_core_attention_over_latent_pages_with_heads_in_groups_of_32(H, k
     test_matrix_core_attention_over_latent_pages(H, kd, vd, window, lens, pos0)
 
 
+@pytest.mark.parametrize("H, kd, vd", [(32, 288, 256), (64, 160, 128), (32, 88, 56)])
+@pytest.mark.parametrize("window, pos0, n", [(None, 0, 70), (None, 47, 33), (5, 31, 66), (33, 96, 40), (100, 200, 17), (1, 15, 34)])
+def test_prompt_rows_over_latent_pages_of_any_size(H, kd, vd, window, pos0, n):
+    """Tiles of 32 positions over pages of 16 (two a tile), 48 (one or two), 32 and 112, looked up a tile ahead: first and last tiles of which half is seen, walks of one, two and more
+    tiles; the same numbers in the same order, so the same bits, and pages that no row sees hold no number at all."""
+    from geneinfer_amd.kernels import ops
+    from geneinfer_amd.parts import StepContext
+    g = torch.Generator().manual_seed(pos0 + n + kd)
+    total = pos0 + n
+    k, q = torch.randn(total, kd, generator=g).to(torch.bfloat16), torch.randn(n, H * kd, generator=g).to(torch.bfloat16)
+    pos = torch.arange(pos0, total, dtype=torch.int32, device=DEV)
+    ctx = StepContext(n_rows=n, dtype=torch.bfloat16, device=torch.device(DEV), tokens=pos, row_pos=pos, row_slot=torch.zeros_like(pos), seg_slot=[0], seg_start=[0], seg_len=[n], seg_pos0=[pos0])
+    first, outs = max(0, pos0 - (window or total) + 1), []
+    for page in (16, 48, 32, 112):
+        pages = -(-total // page)
+        cache = torch.full((pages + 1, page * (kd + vd)), float("nan"), dtype=torch.bfloat16)
+        table = torch.full((1, pages), pages, dtype=torch.int32)                   # (pages behind every window are somebody else's)
+        for i in range(first // page, pages):
+            block = torch.zeros(page, kd, dtype=torch.bfloat16)
+            block[:len(k[i * page:(i + 1) * page])] = k[i * page:(i + 1) * page]
+            table[0, i] = pages - 1 - i
+            cache[pages - 1 - i] = torch.cat([block.reshape(-1), block[:, :vd].T.reshape(-1)])
+        out = torch.empty(n, H * vd, dtype=torch.bfloat16, device=DEV)
+        outs.append(ops.latent_attention_bf16(q.to(DEV), cache.to(DEV), out, ctx, table.to(DEV), H, kd, vd, page, window, 0.2))
+    i_, j_ = torch.arange(pos0, total)[:, None], torch.arange(total)[None]
+    scores = torch.einsum("thd,sd->hts", q.double().view(n, H, kd), k.double()) * 0.2
+    want = torch.einsum("hts,sd->thd", torch.softmax(scores.masked_fill(~((j_ <= i_) & (i_ - j_ < (window or total + 1)))[None], float("-inf")), -1), k[:, :vd].double()).reshape(n, -1)
+    assert relative_error(outs[0], want) < 1.5e-2                                  # (as above)
+    for out in outs[1:]:
+        assert torch.equal(out, outs[0])
+
+
 @pytest.mark.parametrize("n, H, context, window", [(40, 32, 500, None), (12, 32, 4000, None), (60, 32, 511, 300), (32, 32, 500, None), (65, 20, 333, None)])
 def test_single_rows_over_latent_pages_in_more_waves_than_places(n, H, context, window):
     """Shares of one and two tiles, on both sides of a wave for every place of the chip: the kernels that ask for the values before and behind the scores give the
