@@ -2280,8 +2280,9 @@ static StripCut strip_cut(int M, int N, int K) {
     return best;
 }
 // Whether a product ends in strips, with all of k in a workgroup.  Above 128 rows the tiles of 128 x 128 are the better ones for gated products whose strips do not fit one
-// round (160 rows of 28,672 x 4,096: 75 us and 82).
-static bool ends_in_strips(int M, int N, int K) { return K % PK == 0 && (M <= SKINNY_MAX_ROWS || (M <= 192 && (N + 63) / 64 <= gi_compute_units())); }
+// round (160 rows of 28,672 x 4,096: 75 us and 82).  Shorter k stays with those tiles too, whose sums in bits are those of the larger tiles that more rows take: there is little to gain
+// (131 rows of 16,384 x 512 12.8 us and 10.7 in strips; of 16,384 x 1,024 17.9 and 14.3).
+static bool ends_in_strips(int M, int N, int K) { return K % PK == 0 && (M <= SKINNY_MAX_ROWS || (M <= 192 && K >= 1024 && (N + 63) / 64 <= gi_compute_units())); }
 // How strips make a product whose k is shared out, which the kernels beside them cut into `splits`; no tiles where they do not: from 129 rows on where the tiles of 128 x 128 promise to
 // be as fast (a fit like the one above; 350 rows of 3,072 x 8,192 43.1 us and 44.5, 600 71 and 58).
 constexpr int STRIP_MAX_ROWS = 1536;
