@@ -294,7 +294,7 @@ class ParallelBlock:
         then = norm_to_hand_on(next_reader, ctx.n_rows) if getattr(last, "hands_norm_on", False) else norm_to_apply(next_reader, last)
         own = [{}, {}]                            # what each half is told beyond its rows
         into = (None, None)
-        if self._last is not None and ctx.trace is None:          # (a trace wants the rows between the halves)
+        if self._last is not None:
             ends = torch.empty((ctx.n_rows, self._last.weight.shape[1]), dtype=torch.bfloat16, device=x.device)
             into = ends[:, :self._last_split], ends[:, self._last_split:]
             for told, columns in zip(own, into):
@@ -312,7 +312,11 @@ class ParallelBlock:
             own[0 if last is self.mixer else 1]["then"] = then
         out = self.mixer.forward(rows(self.mixer), x, ctx, cache, **own[0])
         if ctx.trace is not None:
-            ctx.trace("attn_out", x)
+            between = x
+            if into[0] is not None:               # (the rows between the halves, made for the trace alone: what the pass computes is the same with one and without)
+                between = x.clone()
+                linear_onto(into[0], self._last.weight[:, :self._last_split], between, None, ctx)
+            ctx.trace("attn_out", between)
         if self.feed_forward is not None:
             out = self.feed_forward.forward(rows(self.feed_forward), x, ctx, **own[1])
         if into[0] is not None:

@@ -883,6 +883,38 @@ def test_long_decoding_carries_state_and_passes_windows(folders):
         check_against_plain(folders, "A", dtype, tokens, got, f"A decoding ({dtype})")
 
 
+@pytest.mark.parametrize("n", [2, 20, 131, 300])
+def test_a_traced_prompt_makes_the_numbers_of_an_untraced_one(folders, n, monkeypatch):
+    """bfloat16, with layers whose two halves end in one product: the rows behind every layer and the last position's logits, in bits (with every row's logits wanted the last norm is
+    handed on, which a traced pass does not do); the trace is shown the same rows."""
+    from geneinfer_amd.engine import StepEntry
+    runner = make_runner(folders, "A", "bfloat16")
+    layers = runner.model.layers
+    assert sum(layer._last is not None for layer in layers) >= 2
+    tokens, got, seen, behind = _prompt(CONFIGS["A"], n, 5), [], [], []
+
+    def watched(forward):
+        def run(x, *args, **kw):
+            out = forward(x, *args, **kw)
+            behind.append(x.clone())
+            return out
+        return run
+
+    for layer in layers:
+        monkeypatch.setattr(layer, "forward", watched(layer.forward))
+    for trace in (None, lambda tag, entry, rows: seen.append((tag, entry, rows.clone()))):
+        runner.model.set_trace(trace)
+        runner.open("r")
+        got.append(runner.step([StepEntry("r", tokens, (n - 1,))]).cpu())
+        runner.close("r")
+    assert torch.equal(got[0], got[1]) and len(behind) == 2 * len(layers)
+    assert [(tag, entry) for tag, entry, _ in seen if tag.endswith("_out")] == [(tag, i) for i in range(len(layers)) for tag in ("attn_out", "ffn_out")]
+    rows = {(tag, entry): x for tag, entry, x in seen}
+    for i in range(len(layers)):
+        assert torch.equal(behind[i], behind[len(layers) + i]) and torch.equal(behind[i], rows["ffn_out", i]), i
+        assert rows["attn_out", i].shape == (n, CONFIGS["A"]["width"]) and not torch.equal(rows["attn_out", i], behind[i - 1] if i else rows["embedding", -1])
+
+
 def test_first_layer_of_a_family_of_blended_values_may_come_anywhere(folders, tmp_path):
     """The same layers in another order: the family's first layer is now the model's last-but-one, and a layer that does not blend
     lies between."""

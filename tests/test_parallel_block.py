@@ -100,8 +100,8 @@ class EndingMixer(Mixer):
 
 @pytest.mark.parametrize("traced", [False, True])
 def test_both_halves_end_in_one_product(traced, monkeypatch):
-    """The halves write the two parts of one buffer, which meets the matrices side by side; a traced pass, which looks at the rows between the halves, has two products.  Either way the
-    weights count once."""
+    """The halves write the two parts of one buffer, which meets the matrices side by side; a traced pass makes the rows between the halves besides, and its own results by the same one product.
+    Either way the weights count once."""
     base.register_mixer("ending", EndingMixer)
     tensors = dict(mix=torch.randn(MIX, D).bfloat16(), o=torch.randn(D, MIX).bfloat16(), up=torch.randn(INTER, D).bfloat16(), down=torch.randn(D, INTER).bfloat16(), act=torch.tensor([0.3, 0.1]))
     ff = Spec(kind="dense_mlp", activation="xielu", activation_params="act", up_proj="up", down_proj="down", intermediate_size=INTER, hidden_size=D)
@@ -122,7 +122,10 @@ def test_both_halves_end_in_one_product(traced, monkeypatch):
     monkeypatch.setattr(block, "linear_xielu", activated)
     for module in (block, __import__("geneinfer_amd.parts.mlp", fromlist=["mlp"])):
         monkeypatch.setattr(module, "linear_onto", onto)
+    between = x + torch.arange(3 * MIX).view(3, MIX).bfloat16().float() @ tensors["o"].float().T
     want = x + torch.arange(3 * MIX).view(3, MIX).bfloat16().float() @ tensors["o"].float().T + mid.float() @ tensors["down"].float().T
-    b.forward(x, Spec(n_rows=3, dtype=torch.bfloat16, trace=(lambda name, rows: seen.append(name)) if traced else None), None)
+    b.forward(x, Spec(n_rows=3, dtype=torch.bfloat16, trace=(lambda name, rows: seen.append((name, rows.clone()))) if traced else None), None)
     assert torch.allclose(x, want, rtol=1e-5, atol=1e-3)
-    assert (products, seen) == (([(INTER, INTER)], ["attn_out", "ffn_out"]) if traced else ([(MIX + INTER, MIX + INTER)], []))
+    assert products == [(MIX, MIX)] * traced + [(MIX + INTER, MIX + INTER)] and [name for name, _ in seen] == ["attn_out", "ffn_out"] * traced
+    if traced:
+        assert torch.allclose(seen[0][1], between, rtol=1e-5, atol=1e-3) and torch.equal(seen[1][1], x)
