@@ -2282,7 +2282,13 @@ static StripCut strip_cut(int M, int N, int K) {
 // Whether a product ends in strips, with all of k in a workgroup.  Above 128 rows the tiles of 128 x 128 are the better ones for gated products whose strips do not fit one
 // round (160 rows of 28,672 x 4,096: 75 us and 82).  Shorter k stays with those tiles too, whose sums in bits are those of the larger tiles that more rows take: there is little to gain
 // (131 rows of 16,384 x 512 12.8 us and 10.7 in strips; of 16,384 x 1,024 17.9 and 14.3).
-static bool ends_in_strips(int M, int N, int K) { return K % PK == 0 && (M <= SKINNY_MAX_ROWS || (M <= 192 && K >= 1024 && (N + 63) / 64 <= gi_compute_units())); }
+// A few rows with k of two blocks of the skinny kernel, or nearly, stay with that: it asks for all its weights at once (16 rows of 16,384 x 512 stored 5.8 us and 6.4 in strips, of
+// 16,384 x 768 9.1 and 7.6; from 20 rows and beyond two rounds of strips they are level).
+static bool ends_in_strips(int M, int N, int K) {
+    const int strips = (N + 63) / 64, units = gi_compute_units();
+    if (K % PK != 0 || (M < 20 && K > 384 && K <= 512 && strips <= 2 * units)) return false;
+    return M <= SKINNY_MAX_ROWS || (M <= 192 && K >= 1024 && strips <= units);
+}
 // How strips make a product whose k is shared out, which the kernels beside them cut into `splits`; no tiles where they do not: from 129 rows on where the tiles of 128 x 128 promise to
 // be as fast (a fit like the one above; 350 rows of 3,072 x 8,192 43.1 us and 44.5, 600 71 and 58).
 constexpr int STRIP_MAX_ROWS = 1536;
@@ -2349,24 +2355,47 @@ static int reduce_partials(const float* scratch, void* C, int epi, int M, int N,
     return 0;
 }
 
-// Up to 16 rows the slim kernel (no LDS staging, one launch) is the faster one, except for wide outputs with more
-// than a few rows, where its per-workgroup reading of the activations costs more than staging them.  Beside the strips' kernel that is so from 8 rows on (16,384 x 2,048
-// gated with a norm: 17.8 and 18.3 us at 6 rows, 18.6 and 18.3 at 8, 21.5 and 18.4 at 16), from 6 for longer rows (22,016 x 4,096: 43.3 and 41.0 at 8), from 10 for
-// short rows and several rounds of strips (24,576 x 1,024: 13.3 and 13.1), from 5 for a vocabulary (128,256 x 2,048: 92.4 and 95.9 at 4, 101.6 and 96.4 at 6); and always where the strips fill one round
-// of workgroups incompletely (12,288 x 2,048: 15.0 and 13.8 at 1 row, 18.8 and 14.3 at 16) or long rows' rounds well (28,672 x 4,096: 49.3 and 46.0 at 1, 55.1 and 45.7 at 8).
+// Up to 16 rows the slim kernel (no LDS staging, one launch) is the faster one, except for wide outputs with more than a few rows, where its per-workgroup reading of the activations
+// costs more than staging them: from 5 rows on for a vocabulary (128,256 x 2,048: 92.4 us and 95.9 in strips at 4 rows, 101.6 and 96.4 at 6), else from the row that
+// slim_until_row or, where strips are not the other ones, streamed_from_row says.
 // Where the skinny kernel is the other one (K no multiple of 64, measured at the time at K = 2,048 to 4,096) the longer the rows and the more strips, the sooner, between 3 and 12.
-// xielu: the product ends through that activation, which of the two only the slim kernel has.
-static bool takes_slim(int M, int N, int K, bool xielu = false) {
-    const int strips64 = (N + 63) / 64, units = gi_compute_units();
-    if (M > 16 || gi_gemm_bf16_skinny_splits(N, K) > 0) return M <= 16;
-    if (strips64 >= 1024) return M < 5;
-    if (K % PK == 0 && !xielu) {
-        const double filled = (double)strips64 / ((strips64 + units - 1) / units * units);
-        if (strips64 * 5 <= units * 4 || (K >= 3072 && filled >= 0.85)) return false;
-        return M < (K > 2048 ? 6 : K > 1024 || strips64 <= units ? 8 : 10);
+static int streamed_from_row(int strips, int K) {
+    const double fitted = 12.0 * (2048.0 / K) * (256.0 / strips);
+    return fitted < 3 ? 3 : fitted > 12 ? 12 : (int)(fitted + 0.5);
+}
+// Beside the strips' kernel (14 widths from 12,288 to 49,152 columns, 19 k from 64 to 14,336, 1 to 16 rows, slim and strips each for all of them, stored, gated and gated with a norm: the choice is 1.3 %
+// slower than the faster of the two on average, 15 % at worst).  What decides it: gated columns leave a strip more cheaply than 32-bit ones; a round of workgroups that strips of 64 columns fill badly is
+// slim's, whose strips are narrower, in the second round, and the strips' in the first, where their workgroups have a unit to themselves; and rows of weights a multiple of 4,096 bytes apart
+// cost the strips, which ask for 64 of them at once, more than slim (whole).  Microseconds, slim and strips:
+//   gated                        1 row         8 rows        16 rows            stored                       1 row         8 rows        16 rows
+//   12,288 x 2,048               14.2, 13.1    15.7, 13.3    18.2, 13.4         12,288 x 2,048               11.1, 13.0    12.9, 13.1    15.9, 13.1
+//   16,384 x 2,048 (a norm)      16.7, 17.5    17.2, 17.9    19.6, 18.1         16,384 x 2,048               13.5, 16.6    16.1, 16.7    20.1, 16.7
+//   28,672 x 4,096               48.2, 44.3    54.0, 45.1    63.4, 45.4         18,432 x 8,192               58.8, 79.0    64.7, 79.8    80.4, 80.3
+//   12,288 x 256                 3.5, 4.1      3.9, 4.6      4.2, 4.6           12,288 x 3,072               14.2, 15.4    18.2, 15.8    22.7, 16.2
+// Decoding 8 requests of the 1B shape, whose gated product has 16,384 x 2,048, takes 900 us with either; 9 take 957 with slim and 949 with strips.
+static int slim_until_row(int strips, int K, bool gated) {
+    const int units = gi_compute_units();
+    const bool three_quarters = strips * 4 <= units * 3, narrow = strips * 5 <= units * 4, second = strips > units && strips * 2 <= units * 3, barely = strips * 4 <= units * 5, whole = K % 2048 == 0;
+    const double filled = (double)strips / ((strips + units - 1) / units * units);
+    if (!gated) {
+        if (K <= 512) return three_quarters ? 12 : 0;
+        if (K < 1536) return strips > units && barely ? 10 : 0;
+        if (whole) return three_quarters ? 8 : narrow ? 4 : !second ? (filled > 0.9 ? 8 : 7) : barely ? 12 : 9;
+        return three_quarters ? 4 : narrow ? 0 : !second ? 2 : barely ? 10 : 6;
     }
-    const double fitted = 12.0 * (2048.0 / K) * (256.0 / strips64);
-    return M < (fitted < 3 ? 3 : fitted > 12 ? 12 : (int)(fitted + 0.5));
+    int until;
+    if (K < 1024) until = narrow && K > 512 ? 8 : strips * 2 <= units * 3 ? 12 : 10;
+    else if (narrow) until = 0;
+    else if (K >= 3072 && filled >= 0.85) until = !whole ? 0 : filled > 0.9 ? 6 : strips <= units ? 3 : 0;
+    else until = K > 2048 ? 6 : whole && strips <= units && filled > 0.9 ? 9 : K > 1024 || strips <= units ? 8 : 10;
+    return strips * 2 > units * 3 ? min(until, streamed_from_row(strips, K)) : until;
+}
+// xielu: the product ends through that activation, which of the kernels only slim has.
+static bool takes_slim(int M, int N, int K, bool gated, bool xielu = false) {
+    const int strips = (N + 63) / 64;
+    if (M > 16 || gi_gemm_bf16_skinny_splits(N, K) > 0) return M <= 16;
+    if (strips >= 1024) return M < 5;
+    return M < (K % PK != 0 || xielu ? streamed_from_row(strips, K) : slim_until_row(strips, K, gated));
 }
 
 // Workgroups of the slim kernel for an output of N columns that is not gated: the pieces a row's sum of squares comes in.
@@ -2448,7 +2477,7 @@ static int launch_slim(const void* A, const void* W, void* C, int epi, int M, in
 // second grid dimension: 256 workgroups at 64 rows and N = 2048, each with 64 KB of weights and its own 128 KB of A) measured
 // equal at 33 to 64 rows and 3 % slower in the whole step from 65 rows on: not kept.
 static bool takes_slim_tiles(int M, int N, int K, int epi) {
-    return !takes_slim(M, N, K) && M <= 32 && K <= 2048 && !is_gated(epi) && gi_gemm_bf16_skinny_splits(N, K) > 0;
+    return !takes_slim(M, N, K, is_gated(epi)) && M <= 32 && K <= 2048 && !is_gated(epi) && gi_gemm_bf16_skinny_splits(N, K) > 0;
 }
 
 // Weight rows per workgroup of that kernel: 16, or 12 or 8 where strips of 16 fill the compute units unevenly and those fill
@@ -2731,7 +2760,7 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
 // 16 or 32 rows in one launch; up to 128 rows one per 1024 columns, from the kernel that adds the partial sums of the shares of k
 // onto the rows.
 GI_API int gi_gemm_bf16_norm_parts(int M, int N, int K) {
-    if (takes_slim(M, N, K)) {
+    if (takes_slim(M, N, K, false)) {
         const int parts = slim_parts(M, N);
         return parts <= slim_max_parts(M) ? parts : 0;
     }
@@ -2747,7 +2776,7 @@ GI_API int gi_gemm_bf16_norm_parts(int M, int N, int K) {
 // Whether a product of these sizes can read rows whose norm was handed on (gi_gemm_bf16_handing with `squares_in`) by a product
 // of as many rows.
 GI_API int gi_gemm_bf16_takes_norm(int M, int N, int K, int gated) {
-    if (takes_slim(M, N, K) || takes_slim_tiles(M, N, K, gated ? EPI_GATED_BF16 : EPI_STORE_F32)) return 1;
+    if (takes_slim(M, N, K, gated != 0) || takes_slim_tiles(M, N, K, gated ? EPI_GATED_BF16 : EPI_STORE_F32)) return 1;
     if (M > SKINNY_MAX_ROWS)                      // the rows of prompts: the gated product with many tiles scales in its epilogue
         return gated && K % PK == 0 && N >= 128 && many_tiles(M, N) ? 1 : 0;
     if (gi_gemm_bf16_skinny_splits(N, K) == 0) return 1;      // the weight-streaming kernel finishes its columns and scales them
@@ -2779,7 +2808,7 @@ GI_API int gi_gemm_bf16_handing(const void* A, const void* W, void* C, int c_dty
                "room for the sums of squares", M, N, K);
     const NormIn norm_in = {squares_in, parts_in, eps, K, gate_limit};
     const NormOut norm_out = {g, (bf16_t*)scaled_out, ld_scaled, squares_out};
-    if (takes_slim(M, N, K)) {
+    if (takes_slim(M, N, K, gated != 0)) {
         GI_REQUIRE(squares_in == nullptr || parts_in <= slim_max_parts(M), "gemm_bf16: %d pieces of a sum of squares, at most %d", parts_in, slim_max_parts(M));
         return launch_slim(A, W, C, epi, M, N, K, lda, ldw, ldc, norm_in, norm_out, stream);
     }
@@ -2799,7 +2828,7 @@ GI_API int gi_gemm_bf16_handing(const void* A, const void* W, void* C, int c_dty
 // that adds the shares up sees whole rows.
 GI_API int gi_gemm_bf16_onto_norm_takes(int M, int N, int K) {
     if (M <= 0 || N <= 0 || N % 4 != 0 || N > WHOLE_NORM_COLUMNS || K <= 0 || K % 8 != 0) return 0;
-    if (M <= SKINNY_MAX_ROWS) return !takes_slim(M, N, K) && !takes_slim_tiles(M, N, K, EPI_ADD_F32) && gi_gemm_bf16_skinny_splits(N, K) > 0;
+    if (M <= SKINNY_MAX_ROWS) return !takes_slim(M, N, K, false) && !takes_slim_tiles(M, N, K, EPI_ADD_F32) && gi_gemm_bf16_skinny_splits(N, K) > 0;
     return K % PK == 0 && N >= 128 && gi_gemm_bf16_piped_splits(M, N, K) > 1;
 }
 
@@ -2824,7 +2853,7 @@ GI_API int gi_gemm_bf16_onto_norm(const void* A, const void* W, float* C, int M,
 GI_API int gi_gemm_bf16_qkv_rope_store_takes(int M, int N, int K, int hd) {
     if (hd < 8 || hd > 256 || (hd & (hd - 1)) != 0) return 0;
     if (M <= SKINNY_MAX_ROWS)
-        return !takes_slim(M, N, K) && !takes_slim_tiles(M, N, K, EPI_STORE_F32) && gi_gemm_bf16_skinny_splits(N, K) > 0 && N % 256 == 0 ? 1 : 0;
+        return !takes_slim(M, N, K, false) && !takes_slim_tiles(M, N, K, EPI_STORE_F32) && gi_gemm_bf16_skinny_splits(N, K) > 0 && N % 256 == 0 ? 1 : 0;
     if (K % PK != 0 || N < 128) return 0;
     return gi_gemm_bf16_piped_splits(M, N, K) > 1 ? N % 256 == 0 : hd <= 128;
 }
@@ -2872,6 +2901,15 @@ GI_API int gi_gemm_bf16_large_kernel(int M, int N, int K, int kind) {
     return large_kernel_of_kind(M, N, K, kind, true).kernel;
 }
 
+// Which kernel makes a product of up to 128 rows: 0 slim, 1 slim's tiles of 17 to 32 rows, 2 strips, 3 the weight-streaming one; -1 for more rows.
+GI_API int gi_gemm_bf16_small_kernel(int M, int N, int K, int gated) {
+    if (M <= 0 || N <= 0 || K <= 0 || M > SKINNY_MAX_ROWS) return -1;
+    if (takes_slim(M, N, K, gated != 0)) return 0;
+    if (takes_slim_tiles(M, N, K, gated ? EPI_GATED_BF16 : EPI_STORE_F32)) return 1;
+    const int splits = gi_gemm_bf16_skinny_splits(N, K);
+    return splits == 0 ? ends_in_strips(M, N, K) ? 2 : 3 : shared_strips(M, N, K, splits).tiles ? 2 : 3;
+}
+
 // The same where the tiles of 256 x 128 make such a product, of whatever kind, with counters.
 GI_API int gi_gemm_bf16_tall_shares(int M, int N, int K) {
     return !takes_large(M, N, K) || gi_gemm_bf16_piped_splits(M, N, K) > 1 ? 1 : tall_cut(M, N, K, true, false).shares;
@@ -2885,7 +2923,7 @@ GI_API int gi_gemm_bf16_counters() { return 2 * gi_compute_units(); }
 // where all of a tile's k is one workgroup's, with all columns through the activation.
 GI_API int gi_gemm_bf16_xielu_takes(int M, int N, int K, int first) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 8 != 0 || first < 0 || first >= N) return 0;
-    if (takes_slim(M, N, K, true)) return 1;
+    if (takes_slim(M, N, K, false, true)) return 1;
     return M > SKINNY_MAX_ROWS && first == 0 && K % PK == 0 && N >= 128 && gi_gemm_bf16_piped_splits(M, N, K) == 1;
 }
 
@@ -2899,7 +2937,7 @@ GI_API int gi_gemm_bf16_xielu(const void* A, const void* W, void* C, int M, int 
     GI_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && lda >= K && ldw >= K && ((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0,
                "gemm_bf16 (xielu): rows must be 16-byte aligned (strides %ld, %ld)", lda, ldw);
     GI_REQUIRE(params != nullptr && act_out != nullptr && ld_act >= N - first && (first == 0 || (C != nullptr && ldc >= first)), "gemm_bf16 (xielu): outputs or parameters are missing");
-    const bool slim = takes_slim(M, N, K, true);
+    const bool slim = takes_slim(M, N, K, false, true);
     GI_REQUIRE(squares_in == nullptr || (slim && parts_in > 0 && parts_in <= slim_max_parts(M)), "gemm_bf16 (xielu): %d pieces of a sum of squares are not taken", parts_in);
     NormIn in = {squares_in, parts_in, eps, K, 0.f};
     in.first = first;
@@ -2923,7 +2961,7 @@ GI_API int gi_gemm_bf16(const void* A, const void* W, void* C, int c_dtype, int 
     GI_REQUIRE(epi >= 0, "gemm_bf16: output dtype %d with accumulate %d is not supported", c_dtype, accumulate);
 
     const NormIn plain_in = {nullptr, 0, 0.f, 1, gate_limit};          // no norm to finish; the clamped gate's limit
-    if (takes_slim(M, N, K)) return launch_slim(A, W, C, epi, M, N, K, lda, ldw, ldc, plain_in, NO_NORM_OUT, stream);
+    if (takes_slim(M, N, K, gated != 0)) return launch_slim(A, W, C, epi, M, N, K, lda, ldw, ldc, plain_in, NO_NORM_OUT, stream);
 
     if (takes_slim_tiles(M, N, K, epi)) return launch_slim_tiles(A, W, C, epi, M, N, K, lda, ldw, ldc, plain_in, NO_NORM_OUT, stream);
     if (M <= SKINNY_MAX_ROWS) return launch_skinny(A, W, C, epi, M, N, K, lda, ldw, ldc, scratch, scratch_floats, plain_in, NO_NORM_OUT, stream);

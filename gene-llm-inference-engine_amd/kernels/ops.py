@@ -169,6 +169,8 @@ def lib():
         l.gi_gemm_bf16_counters.restype = c_int
         l.gi_gemm_bf16_large_kernel.argtypes = [c_int, c_int, c_int, c_int]
         l.gi_gemm_bf16_large_kernel.restype = c_int
+        l.gi_gemm_bf16_small_kernel.argtypes = [c_int, c_int, c_int, c_int]
+        l.gi_gemm_bf16_small_kernel.restype = c_int
         l.gi_gemm_bf16_onto_norm_takes.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_bf16_onto_norm_takes.restype = c_int
         l.gi_gemm_bf16_xielu_takes.argtypes = [c_int, c_int, c_int, c_int]
@@ -1893,6 +1895,12 @@ def gemm_bf16_large_kernel(m, n, k, kind):
     "128x128 shared" (k shared out over workgroups, which make strips of up to 256 rows where those are the faster ones).  kind: one of `PRODUCT_KINDS`; with counters (`step_counters`)."""
     which = lib().gi_gemm_bf16_large_kernel(m, n, k, PRODUCT_KINDS.index(kind))
     return None if which < 0 else ("128x128", "256x128", "256x256", "128x128 shared", "strips")[which]
+
+
+def gemm_bf16_small_kernel(m, n, k, gated=False):
+    """Which kernel makes a product of up to 128 rows (None: more rows): "slim", "slim tiles", "strips" or "streamed" (weights through registers)."""
+    which = lib().gi_gemm_bf16_small_kernel(m, n, k, 1 if gated else 0)
+    return None if which < 0 else ("slim", "slim tiles", "strips", "streamed")[which]
 
 
 @lru_cache(maxsize=8192)

@@ -33,6 +33,23 @@ def test_strips_where_one_round_of_them_is_faster(m, n, k, kernel):
     assert ops.gemm_bf16_large_kernel(m, n, k, "gated") == kernel
 
 
+# m, n, k, gated -> the kernel of up to 128 rows that was the faster one there, by more than 4 % or (on one side of a line) as fast
+FEW_ROWS = [
+    (1, 12288, 2048, True, "strips"), (8, 16384, 2048, True, "slim"), (9, 16384, 2048, True, "strips"), (1, 16384, 3072, True, "strips"), (1, 28672, 4096, True, "strips"), (4, 16384, 4096, True, "slim"),
+    (8, 16384, 4096, True, "strips"), (8, 12288, 256, True, "slim"), (2, 20480, 3072, True, "slim"), (8, 20480, 3072, True, "strips"),
+    (1, 12288, 2048, False, "slim"), (12, 12288, 2048, False, "strips"), (1, 12288, 3072, False, "slim"), (1, 13056, 3072, False, "strips"), (4, 16384, 2048, False, "slim"),
+    (12, 16384, 2048, False, "strips"), (2, 18432, 8192, False, "slim"), (4, 24576, 4096, False, "slim"), (4, 24576, 512, False, "streamed"), (4, 24576, 768, False, "strips"), (1, 32768, 4096, False, "slim"), (8, 32768, 3072, False, "strips"),
+    (16, 16384, 512, False, "streamed"), (16, 16384, 768, False, "strips"), (20, 16384, 512, False, "strips"), (4, 128256, 2048, False, "slim"), (5, 128256, 2048, False, "strips"),
+    (11, 16384, 2056, True, "slim"), (12, 16384, 2056, True, "streamed"), (16, 3072, 2048, False, "slim"), (17, 3072, 2048, False, "slim tiles"), (17, 3072, 2048, True, "strips"),
+    (128, 3072, 2048, False, "strips"), (128, 3072, 2056, False, "streamed"), (129, 3072, 2048, False, None),
+]
+
+
+@pytest.mark.parametrize("m,n,k,gated,kernel", FEW_ROWS)
+def test_the_faster_kernel_is_chosen_for_few_rows(m, n, k, gated, kernel):
+    assert ops.gemm_bf16_small_kernel(m, n, k, gated) == kernel
+
+
 # m, n, k -> the most shares of k that either kernel makes, as the scratch shows them
 @pytest.mark.parametrize("m,n,k,shares", [(131, 3072, 8192, 5), (40, 5120, 3072, 4), (131, 10240, 2048, 2), (256, 3072, 8192, 5), (300, 2048, 2048, 4), (600, 3072, 8192, 2), (17, 200, 64, 1), (40, 128, 12288, 32)])
 def test_scratch_holds_as_many_shares_as_either_kernel_makes(m, n, k, shares):
