@@ -2279,15 +2279,16 @@ static StripCut strip_cut(int M, int N, int K) {
     best.us = sqrt(sqrt(least));
     return best;
 }
-// Whether a product ends in strips, with all of k in a workgroup.  Above 128 rows the tiles of 128 x 128 are the better ones for gated products whose strips do not fit one
-// round (160 rows of 28,672 x 4,096: 75 us and 82).  Shorter k stays with those tiles too, whose sums in bits are those of the larger tiles that more rows take: there is little to gain
-// (131 rows of 16,384 x 512 12.8 us and 10.7 in strips; of 16,384 x 1,024 17.9 and 14.3).
+// Whether a product ends in strips, with all of k in a workgroup.  Above 128 rows the tiles of 128 or 256 x 128 are the better ones for gated products whose strips do not fit one
+// round (160 rows of 28,672 x 4,096: 75 us and 82), for k above 4,096, where what a strip takes in of A tells (160 rows of 12,288 x 4,096 42.0 us and 39.2, x 6,144 60.1 and 61.3, x 14,336 112 and 128), and from 169 rows on
+// for k above 2,048 where the strips leave a tenth of the units idle (184 rows of 12,288 x 3,072 33.1 and 34.4, of 16,384 x 3,072 40.5 and 37.2).
+// Below 1,024 of k strips would be faster too (131 rows of 16,384 x 512 12.8 us and 10.7), but there a gated product's sums are in bits those of the larger tiles that more rows take, and stay so.
 // A few rows with k of two blocks of the skinny kernel, or nearly, stay with that: it asks for all its weights at once (16 rows of 16,384 x 512 stored 5.8 us and 6.4 in strips, of
 // 16,384 x 768 9.1 and 7.6; from 20 rows and beyond two rounds of strips they are level).
 static bool ends_in_strips(int M, int N, int K) {
     const int strips = (N + 63) / 64, units = gi_compute_units();
     if (K % PK != 0 || (M < 20 && K > 384 && K <= 512 && strips <= 2 * units)) return false;
-    return M <= SKINNY_MAX_ROWS || (M <= 192 && K >= 1024 && strips <= units);
+    return M <= SKINNY_MAX_ROWS || (M <= 192 && K >= 1024 && K <= 4096 && strips <= units && (M <= 168 || K <= 2048 || strips * 10 >= units * 9));
 }
 // How strips make a product whose k is shared out, which the kernels beside them cut into `splits`; no tiles where they do not: from 129 rows on where the tiles of 128 x 128 promise to
 // be as fast (a fit like the one above; 350 rows of 3,072 x 8,192 43.1 us and 44.5, 600 71 and 58).

@@ -28,7 +28,9 @@ def test_the_faster_kernel_is_chosen(m, n, k, kind, kernel):
     assert ops.gemm_bf16_large_kernel(m, n, k, kind) == kernel
 
 
-@pytest.mark.parametrize("m,n,k,kernel", [(129, 16384, 2048, "strips"), (192, 16384, 3072, "strips"), (193, 16384, 2048, "128x128"), (131, 28672, 4096, "256x128"), (131, 16384, 2056, None)])
+@pytest.mark.parametrize("m,n,k,kernel", [(129, 16384, 2048, "strips"), (192, 16384, 3072, "strips"), (193, 16384, 2048, "128x128"), (131, 28672, 4096, "256x128"), (131, 16384, 2056, None),
+                                          (184, 12288, 2048, "strips"), (160, 12288, 3072, "strips"), (184, 12288, 3072, "128x128"), (160, 12288, 4096, "strips"), (160, 12288, 6144, "256x128"),
+                                          (150, 13056, 14336, "256x128"), (192, 16384, 4096, "strips"), (192, 16384, 6144, "256x128")])
 def test_strips_where_one_round_of_them_is_faster(m, n, k, kernel):
     assert ops.gemm_bf16_large_kernel(m, n, k, "gated") == kernel
 
