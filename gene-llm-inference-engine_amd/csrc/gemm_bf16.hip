@@ -2291,15 +2291,22 @@ static bool ends_in_strips(int M, int N, int K) {
     return M <= SKINNY_MAX_ROWS || (M <= 192 && K >= 1024 && K <= 4096 && strips <= units && (M <= 168 || K <= 2048 || strips * 10 >= units * 9));
 }
 // How strips make a product whose k is shared out, which the kernels beside them cut into `splits`; no tiles where they do not: from 129 rows on where the tiles of 128 x 128 promise to
-// be as fast (a fit like the one above; 350 rows of 3,072 x 8,192 43.1 us and 44.5, 600 71 and 58).
+// be as fast (a fit like the one above; 350 rows of 3,072 x 8,192 43.1 us and 44.5, 600 71 and 58).  Strips have to promise more where the fit knows less of what they take in (1,900 products
+// of 14 sizes of columns, 128 to 11,264, and nine of k, 512 to 28,672: with these lines none of more than 128 rows is over 5 % slower than the tiles, without them 40 are, up to 27 %):
+//   many workgroups with long shares (300 rows of 6,144 x 14,336 116 us in tiles and 125 in strips), one tile of more than 192 rows (256 of 11,264 x 768 23.6 and 25.2), and
+//   few columns, whose strips read more of A than of the weights (900 rows of 500 x 8,192 22.8 and 26.4, 1,400 of 320 x 28,672 66 and 81; 400 of 500 x 4,096 15.2 and 12.4).
 constexpr int STRIP_MAX_ROWS = 1536;
 static StripCut shared_strips(int M, int N, int K, int splits) {
     const StripCut none = {0, 0, 0};
     if (K % PK != 0 || M > STRIP_MAX_ROWS || splits == 0) return none;
+    const int strips = (N + 63) / 64;
+    if (N < 768 && M > 256 && (double)M * K * strips > 24e6) return none;
     const StripCut cut = strip_cut(M, N, K);
     if (M <= SKINNY_MAX_ROWS) return cut;
     const bool two = (long)((M + 127) / 128) * ((N + 127) / 128) * splits > gi_compute_units();
-    return cut.us < 0.98 * (6.6 + K / splits / PK * (two ? 0.951 : 0.882) + 1.55e-6 * splits * M * N) ? cut : none;
+    const int groups = strips * cut.tiles * cut.splits, blocks = (K / PK + cut.splits - 1) / cut.splits;
+    const double least = groups > gi_compute_units() && blocks > 64 ? 0.88 : cut.tiles * cut.splits == 1 && M > 192 ? 0.9 : 0.98;
+    return cut.us < least * (6.6 + K / splits / PK * (two ? 0.951 : 0.882) + 1.55e-6 * splits * M * N) ? cut : none;
 }
 static bool strip_strides(long lda, long ldw) { return lda < (1L << 22) && ldw < (1L << 22); }       // (a tile's rows within 32-bit offsets)
 // The most shares of k that a product may be cut into.
@@ -2909,6 +2916,13 @@ GI_API int gi_gemm_bf16_small_kernel(int M, int N, int K, int gated) {
     if (takes_slim_tiles(M, N, K, gated ? EPI_GATED_BF16 : EPI_STORE_F32)) return 1;
     const int splits = gi_gemm_bf16_skinny_splits(N, K);
     return splits == 0 ? ends_in_strips(M, N, K) ? 2 : 3 : shared_strips(M, N, K, splits).tiles ? 2 : 3;
+}
+
+// How strips make a product whose k is shared out: 100 times the tiles of rows and the shares of k (at most 16); 0 where they do not.
+GI_API int gi_gemm_bf16_strip_cut(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || (M <= SKINNY_MAX_ROWS ? gi_gemm_bf16_small_kernel(M, N, K, 0) != 2 : !takes_large(M, N, K) || gi_gemm_bf16_piped_splits(M, N, K) == 1)) return 0;
+    const StripCut cut = shared_strips(M, N, K, M <= SKINNY_MAX_ROWS ? gi_gemm_bf16_skinny_splits(N, K) : gi_gemm_bf16_piped_splits(M, N, K));
+    return 100 * cut.tiles + cut.splits;
 }
 
 // The same where the tiles of 256 x 128 make such a product, of whatever kind, with counters.

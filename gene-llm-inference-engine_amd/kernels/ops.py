@@ -171,6 +171,8 @@ def lib():
         l.gi_gemm_bf16_large_kernel.restype = c_int
         l.gi_gemm_bf16_small_kernel.argtypes = [c_int, c_int, c_int, c_int]
         l.gi_gemm_bf16_small_kernel.restype = c_int
+        l.gi_gemm_bf16_strip_cut.argtypes = [c_int, c_int, c_int]
+        l.gi_gemm_bf16_strip_cut.restype = c_int
         l.gi_gemm_bf16_onto_norm_takes.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_bf16_onto_norm_takes.restype = c_int
         l.gi_gemm_bf16_xielu_takes.argtypes = [c_int, c_int, c_int, c_int]
@@ -1895,6 +1897,12 @@ def gemm_bf16_large_kernel(m, n, k, kind):
     "128x128 shared" (k shared out over workgroups, which make strips of up to 256 rows where those are the faster ones).  kind: one of `PRODUCT_KINDS`; with counters (`step_counters`)."""
     which = lib().gi_gemm_bf16_large_kernel(m, n, k, PRODUCT_KINDS.index(kind))
     return None if which < 0 else ("128x128", "256x128", "256x256", "128x128 shared", "strips")[which]
+
+
+def gemm_bf16_strip_cut(m, n, k):
+    """(tiles of rows, shares of k) with which strips make a product whose k is shared out over workgroups, or None: another kernel does, or nobody shares k out."""
+    cut = lib().gi_gemm_bf16_strip_cut(m, n, k)
+    return divmod(cut, 100) if cut else None
 
 
 def gemm_bf16_small_kernel(m, n, k, gated=False):

@@ -52,6 +52,15 @@ def test_the_faster_kernel_is_chosen_for_few_rows(m, n, k, gated, kernel):
     assert ops.gemm_bf16_small_kernel(m, n, k, gated) == kernel
 
 
+# m, n, k -> tiles of rows and shares of k in strips, or None where the other kernels were the faster ones
+@pytest.mark.parametrize("m,n,k,cut", [(131, 3072, 8192, (1, 5)), (256, 3072, 8192, (1, 5)), (301, 2048, 2048, (4, 2)), (300, 3072, 8192, (5, 2)), (300, 3072, 20480, None), (300, 6144, 14336, None),
+                                       (131, 10240, 2048, (3, 1)), (131, 10240, 6144, None), (129, 11264, 768, (1, 1)), (256, 11264, 768, None), (400, 500, 4096, (7, 4)), (900, 500, 8192, None),
+                                       (256, 500, 8192, (4, 8)), (1400, 320, 28672, None), (1536, 1920, 640, (8, 1)), (1537, 1920, 640, None), (64, 2048, 2048, (1, 4)), (64, 2048, 2056, None),
+                                       (64, 16384, 2048, None), (2048, 2048, 2048, None)])
+def test_products_are_cut_into_strips_where_that_is_faster(m, n, k, cut):
+    assert ops.gemm_bf16_strip_cut(m, n, k) == cut
+
+
 # m, n, k -> the most shares of k that either kernel makes, as the scratch shows them
 @pytest.mark.parametrize("m,n,k,shares", [(131, 3072, 8192, 5), (40, 5120, 3072, 4), (131, 10240, 2048, 2), (256, 3072, 8192, 5), (300, 2048, 2048, 4), (600, 3072, 8192, 2), (17, 200, 64, 1), (40, 128, 12288, 32)])
 def test_scratch_holds_as_many_shares_as_either_kernel_makes(m, n, k, shares):
