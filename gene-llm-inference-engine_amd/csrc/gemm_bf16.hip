@@ -2296,7 +2296,7 @@ static bool ends_in_strips(int M, int N, int K) {
 //   many workgroups with long shares (300 rows of 6,144 x 14,336 116 us in tiles and 125 in strips), one tile of more than 192 rows (256 of 11,264 x 768 23.6 and 25.2), and
 //   few columns, whose strips read more of A than of the weights (900 rows of 500 x 8,192 22.8 and 26.4, 1,400 of 320 x 28,672 66 and 81; 400 of 500 x 4,096 15.2 and 12.4).
 constexpr int STRIP_MAX_ROWS = 1536;
-static StripCut shared_strips(int M, int N, int K, int splits) {
+static StripCut find_shared_strips(int M, int N, int K, int splits) {
     const StripCut none = {0, 0, 0};
     if (K % PK != 0 || M > STRIP_MAX_ROWS || splits == 0) return none;
     const int strips = (N + 63) / 64;
@@ -2307,6 +2307,15 @@ static StripCut shared_strips(int M, int N, int K, int splits) {
     const int groups = strips * cut.tiles * cut.splits, blocks = (K / PK + cut.splits - 1) / cut.splits;
     const double least = groups > gi_compute_units() && blocks > 64 ? 0.88 : cut.tiles * cut.splits == 1 && M > 192 ? 0.9 : 0.98;
     return cut.us < least * (6.6 + K / splits / PK * (two ? 0.951 : 0.882) + 1.55e-6 * splits * M * N) ? cut : none;
+}
+// Found once for the sizes that a thread asks for again and again (a step's layers have the same few): looking at up to 140 cuts takes 0.3 to 2 us of the host's time, for every product of a pass
+// that is not captured.
+static StripCut shared_strips(int M, int N, int K, int splits) {
+    struct Found { int M, N, K, splits; StripCut cut; };
+    static thread_local Found found[32] = {};
+    Found& at = found[(unsigned)(M + 5 * (N / 64) + 11 * (K / 64)) % 32];
+    if (at.M != M || at.N != N || at.K != K || at.splits != splits) at = {M, N, K, splits, find_shared_strips(M, N, K, splits)};
+    return at.cut;
 }
 static bool strip_strides(long lda, long ldw) { return lda < (1L << 22) && ldw < (1L << 22); }       // (a tile's rows within 32-bit offsets)
 // The most shares of k that a product may be cut into.

@@ -61,6 +61,17 @@ def test_products_are_cut_into_strips_where_that_is_faster(m, n, k, cut):
     assert ops.gemm_bf16_strip_cut(m, n, k) == cut
 
 
+def test_a_cut_does_not_depend_on_what_was_asked_before():
+    """Answers are kept by size: asked in other orders, between others whose answers lie in the same places, and from another thread they are the same."""
+    from concurrent.futures import ThreadPoolExecutor
+    sizes = [(m, n, k) for m in (17, 49, 131, 163, 300, 332, 1400) for n in (500, 2048, 3072) for k in (512, 2048, 8192)]
+    ask = lambda order: {size: ops.lib().gi_gemm_bf16_strip_cut(*size) for size in order}
+    first = ask(sizes)
+    assert len(set(first.values())) > 10 and ask(sizes[::-1]) == first and ask(sizes[::5] + sizes) == first
+    with ThreadPoolExecutor(2) as pool:
+        assert all(got == first for got in pool.map(ask, [sizes, sizes[::-1]]))
+
+
 # m, n, k -> the most shares of k that either kernel makes, as the scratch shows them
 @pytest.mark.parametrize("m,n,k,shares", [(131, 3072, 8192, 5), (40, 5120, 3072, 4), (131, 10240, 2048, 2), (256, 3072, 8192, 5), (300, 2048, 2048, 4), (600, 3072, 8192, 2), (17, 200, 64, 1), (40, 128, 12288, 32)])
 def test_scratch_holds_as_many_shares_as_either_kernel_makes(m, n, k, shares):
