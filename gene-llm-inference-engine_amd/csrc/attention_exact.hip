@@ -645,14 +645,23 @@ GI_API int gi_attention_exact_spans(int n_rows, int n_single, int n_heads, int n
     if (tiles >= 2L * gi_compute_units() || spans > MAX_SPANS || spans * n_rows * n_heads * part_floats(vd) > (16L << 20)) return 0;
     return (int)spans;
 }
-// Whether the spans' blocks of 64 keys then go out one by one: with heads of more than 64 channels (spans and blocks, 24/8 heads of 128: 40 rows of their own at 1,000 positions 117 us and 80, 60 at 4,000
-// 574 and 403, a prompt of 64 rows at 1,000 47 and 41; 32 such rows 26.3 and 27.4, 250 at 300 56 and 57), else up to so many blocks as the tiles see at most, fewer where contexts are long, and while the
-// join has few parts to read (32/8 heads of 64: 12 rows at 300, 600, 1,000 positions 18.6 and 12.4, 18.7 and 15.1, 22.2 and 21.6; 16 at 1,000 23.2 and 25.6; 5 at 2,000 22.6 and 22.3, 8 at 2,000 24.9 and
-// 28.0; 1 at 4,000 22.5 and 20.8, 3 at 4,000 26.4 and 29.5; a prompt of 16 rows at 1,000 16.6 and 13.3, of 32 17.2 and 19.2).
+// Whether the spans' blocks of 64 keys then go out one by one, by `walks`, the spans that the tiles see at most (workgroups of the kernel of spans), and how many rounds those make on the compute
+// units.  3,094 steps (1 to 400 rows of their own, of a prompt and of both, 280 to 40,000 positions, 11 shapes of heads; both kernels with their joins): nowhere more than 2 % slower than spans and 30 % less
+// time in the mean where blocks serve, which are 2 to 54 % slower in 160 of the others.
+// Heads of more than 64 channels, one workgroup of spans or two of blocks a unit.  Microseconds, spans and blocks:
+//   not where the spans' workgroups nearly fill their first round, for the blocks are then two full ones (24/8 heads of 128, 1,000 positions: a prompt of 24 rows 25.5 and 20.8, of 32 25.7 and 28.4, of 60 46.0 and
+//   36.3; 3 rows of their own at 2,000 28.2 and 21.9, 2 at 4,000 32.4 and 34.4).  With up to three spans a row that tells later, and only where many rows join (500 positions: a prompt of 64 rows 26.7 and 27.3,
+//   of 80 27.6 and 29.9; 16/16 heads, 100 rows at 300 26.4 and 19.3);
+//   not where rows have more spans than the rounds saved are worth, for the join walks four parts a span (16/2 heads of 128, 8 rows of their own at 8,000 58.7 and 59.8, 10 of 8/1 heads at 12,000 70 and 74, 24/8 heads, 1 row
+//   at 8,000 37.2 and 44.2, 3 of 8/1 heads at 40,000 105 and 144).
+// Heads of up to 64 channels, two workgroups of spans a unit: up to so many blocks, fewer where contexts are long, and while the join has few parts to read (32/8 heads of 64: 12 rows at 300, 600 positions
+// 15.9 and 11.6, 19.5 and 15.3, at 1,000 22.6 and 23.4; 5 at 2,000 23.3 and 24.2; 1 at 4,000 20.8 and 19.7, 16/2 heads, 1 row at 8,000 26.9 and 28.8; a prompt of 16 rows at 1,000 16.6 and 13.3, at 2,000 18.9 and 21.2).
 static bool by_blocks(int n_rows, int n_single, int n_heads, int n_kv, int hd, int vd, int n_spans) {
-    const long blocks = count_tiles(n_rows, n_single, n_kv, n_heads / n_kv) * 4 * (n_spans - 1);
-    return 4L * n_spans * n_rows * n_heads * part_floats(vd) <= (16L << 20) && 4 * n_spans <= MAX_SPANS && 
-           (hd > 64 || vd > 64 || ((long)n_rows * n_heads <= 512 && blocks <= (n_spans <= 5 ? 1536 : n_spans <= 9 ? 1280 : 512)));
+    if (4L * n_spans * n_rows * n_heads * part_floats(vd) > (16L << 20) || 4 * n_spans > MAX_SPANS) return false;
+    const long pairs = (long)n_rows * n_heads, walks = count_tiles(n_rows, n_single, n_kv, n_heads / n_kv) * (n_spans - 1), units = gi_compute_units();
+    if (hd <= 64 && vd <= 64) return pairs <= 512 && n_spans <= 17 && 4 * walks <= (n_spans <= 5 ? 1152 : n_spans <= 9 ? 896 : 512);
+    const bool nearly_one_round = walks <= units && (n_spans > 4 ? 4 * walks > 3 * units : 8 * walks > 7 * units && pairs >= 900);
+    return !nearly_one_round && n_spans - 1 <= 22 * ((walks + units - 1) / units) + 2;
 }
 GI_API long gi_attention_exact_part_floats(int n_rows, int n_single, int n_heads, int n_kv, int hd, int vd, int n_spans) {
     return (long)n_rows * n_heads * n_spans * (by_blocks(n_rows, n_single, n_heads, n_kv, hd, vd, n_spans) ? 4 : 1) * part_floats(vd);

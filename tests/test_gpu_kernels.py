@@ -1374,8 +1374,9 @@ def test_attention_exact_of_blocks_one_by_one(n_heads, n_kv, hd, vd, window, chu
         return ops().lib().gi_attention_exact_part_floats(n, n, n_heads, n_kv, hd, vd, spans) // (n * n_heads * spans * (vd + 4))
 
     whole = attend(0, T, single_rows=True)
-    few, many = 2, (1536 if spans <= 5 else 1280) // (n_kv * 4 * (spans - 1)) + 1
-    assert spans > 1 and parts(1) == parts(few) == 4 and parts(many) == (1 if hd <= 64 and vd <= 64 else 4)
+    small = hd <= 64 and vd <= 64
+    few, many = 2, (1280 if not small else 1152 if spans <= 5 else 896) // (n_kv * 4 * (spans - 1)) + 1
+    assert spans > 1 and parts(1) == parts(few) == 4 and parts(many) == (1 if small else 4)
     for n, known in ((1, dict(single_rows=True)), (few, dict(single_rows=True)), (19, dict(single_rows=True)), (many, dict(single_rows=True)), (19, dict()), (few + 19, dict(single_rows=few))):
         for first in (0, 18, T - n if n < T else 0):
             got = attend(first, n, max_context=seen, **known)

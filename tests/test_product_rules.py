@@ -119,6 +119,19 @@ def test_a_context_is_shared_out_over_so_many_spans_as_a_grid_takes(rows, seen, 
     assert ops.lib().gi_attention_exact_spans(rows, rows, 1, 1, 16, 16, 16, seen) == spans
 
 
+# rows, rows of their own, heads, key heads, channels, positions seen -> whether a span's blocks go out one by one; beside it what was measured, microseconds of spans and of blocks
+@pytest.mark.parametrize("rows,single,heads,kv,hd,seen,blocks", [(3, 3, 24, 8, 128, 600, True),                                                   # 25.7, 12.9
+                                                                 (24, 0, 24, 8, 128, 1000, True), (32, 0, 24, 8, 128, 1000, False), (60, 0, 24, 8, 128, 1000, True),          # 25.5, 20.8; 25.7, 28.4; 46.0, 36.3
+                                                                 (100, 0, 16, 16, 128, 300, True), (128, 0, 16, 2, 128, 500, False),               # 26.4, 19.3; 27.8, 30.5
+                                                                 (1, 1, 24, 8, 128, 8000, False), (5, 5, 24, 8, 128, 8000, True), (3, 3, 8, 1, 128, 40000, False),              # 37.2, 44.2; 134, 106; 105, 144
+                                                                 (10, 10, 8, 1, 128, 12000, False), (14, 14, 8, 1, 128, 12000, True),              # 70.1, 74.1; 91.5, 86.1
+                                                                 (12, 12, 32, 8, 64, 600, True), (12, 12, 32, 8, 64, 1000, False), (16, 0, 32, 8, 64, 1000, True), (16, 0, 32, 8, 64, 2000, False),
+                                                                 (1, 1, 32, 8, 64, 4000, True), (1, 1, 16, 2, 64, 8000, False)])                   # 20.8, 19.7; 26.9, 28.8
+def test_blocks_of_keys_go_out_one_by_one_where_that_is_faster(rows, single, heads, kv, hd, seen, blocks):
+    spans, floats = ops._exact_spans(rows, single, heads, kv, hd, hd, 16, -(-seen // 256) * 256)
+    assert spans > 1 and floats == rows * heads * spans * (hd + 4) * (4 if blocks else 1)
+
+
 @pytest.mark.parametrize("m,n,k,taken", [(3, 16384, 2048, 1), (1, 4096, 4096, 1), (8, 8192, 4096, 1), (1, 6656, 4096, 1), (16, 1024, 4096, 1), (1, 1024, 1024, 1), (1, 2048, 2048, 1), (8, 5120, 2048, 1),
                                          (9, 1000, 4096, 1), (1, 1000, 4096, 0), (1, 1024, 4096, 0), (8, 2048, 3072, 0), (1, 5632, 4096, 0), (4, 4608, 3072, 0), (8, 1024, 2048, 0), (2, 6144, 2048, 0), (17, 4096, 1024, 0), (3, 4095, 1024, 0)])
 def test_gates_in_the_product_where_that_is_faster(m, n, k, taken):
