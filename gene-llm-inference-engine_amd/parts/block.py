@@ -241,10 +241,12 @@ class ParallelBlock:
                 self.feed_forward.use_input_weight(self.w_first[self._split:])
         # Both halves end with a product onto the same rows: where both say which matrix that is (`output_weight`, bfloat16), the two are laid side by side along k and the halves
         # write the rows they would multiply into one buffer (`into=`): one product of all of it.  5 rows of 2,048 x 2,048 and 2,048 x 8,192 14.8 us, in one 12.2; 200 rows 34.1
-        # and 26.3, 1,777 105.5 and 92.2.
+        # and 26.3, 1,777 105.5 and 92.2; so over 308 products of 1 to 4,096 rows, 512 to 8,192 columns.  Not where one matrix is whole blocks of 64 along k and both together are not, which the kernels for more than
+        # 128 rows want (2,048 x (200 + 8,192): 131 rows 33.2 us and 136.6, 2,048 90.6 and 153.8; 2,048 x (2,048 + 5,464) 103.5 and 128.2).
         self._last, self._last_split = None, 0
         last = [getattr(p, "output_weight", lambda: None)() for p in (self.mixer, self.feed_forward)] if self.feed_forward is not None else []
         if (self.STACK and len(last) == 2 and all(w is not None and w.dtype == torch.bfloat16 and w.shape[1] % 8 == 0 for w in last) and last[0].shape[0] == last[1].shape[0]
+                and ((last[0].shape[1] + last[1].shape[1]) % 64 == 0 or all(w.shape[1] % 64 for w in last))
                 and all("into" in inspect.signature(p.forward).parameters for p in (self.mixer, self.feed_forward))):
             self._last_split = last[0].shape[1]
             whole = torch.cat(last, dim=1).contiguous()

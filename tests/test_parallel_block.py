@@ -129,3 +129,14 @@ def test_both_halves_end_in_one_product(traced, monkeypatch):
     assert products == [(MIX, MIX)] * traced + [(MIX + INTER, MIX + INTER)] and [name for name, _ in seen] == ["attn_out", "ffn_out"] * traced
     if traced:
         assert torch.allclose(seen[0][1], between, rtol=1e-5, atol=1e-3) and torch.equal(seen[1][1], x)
+
+
+@pytest.mark.parametrize("mix,inter,joined", [(24, 32, True), (64, 128, True), (24, 40, True), (64, 40, False), (200, 128, False), (200, 72, True), (24, 20, False)])
+def test_matrices_lie_side_by_side_where_the_kernels_for_many_rows_take_them(mix, inter, joined):
+    """Not where one is whole blocks of 64 along k and both together are not (nor where one is not 16 bytes long)."""
+    base.register_mixer("ending", EndingMixer)
+    tensors = dict(mix=torch.randn(mix, D).bfloat16(), o=torch.randn(D, mix).bfloat16(), up=torch.randn(inter, D).bfloat16(), down=torch.randn(D, inter).bfloat16(), act=torch.tensor([0.3, 0.1]))
+    ff = Spec(kind="dense_mlp", activation="xielu", activation_params="act", up_proj="up", down_proj="down", intermediate_size=inter, hidden_size=D)
+    b = block.ParallelBlock(Spec(feed_forward_norm=None, mixer_post_norm=None, feed_forward_post_norm=None, mixer_norm=Spec(kind="stand_in"), mixer=Spec(kind="ending"), feed_forward=ff), tensors, torch.bfloat16, "cpu")
+    assert (b._last is not None) == joined
+    assert torch.equal(b.mixer.w_o, tensors["o"]) and torch.equal(b.feed_forward.w_down, tensors["down"])
