@@ -758,9 +758,9 @@ GI_API int gi_norm_rope_store(const float* q, const float* k, const float* v, lo
         GI_CHECK_LAUNCH("norm_rope_store (plain)");
         return 0;
     }
-    // (from 64 rows on: 32 + 8 + 8 heads of 64, 5 rows 3.4 us a wave a head and 4.5 here, 48 rows 3.7 and 3.6, 64 4.0 and 3.7, 200 6.0 and 3.8)
+    // (not where the queries are turned in their own place, whose partners two threads read; from 64 rows on: 32 + 8 + 8 heads of 64, 5 rows 3.4 us a wave a head and 4.5 here, 48 rows 3.7 and 3.6, 64 4.0 and 3.7, 200 6.0 and 3.8)
     const auto by16 = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
-    const bool rows = k != nullptr && n_rows >= TURN_STORE_ROWS && q_norm == nullptr && k_norm == nullptr && flags == 0 && hd % 4 == 0 && rot % 8 == 0 && ldq % 4 == 0 && ldk % 4 == 0 &&
+    const bool rows = k != nullptr && (const void*)q != q_out && n_rows >= TURN_STORE_ROWS && q_norm == nullptr && k_norm == nullptr && flags == 0 && hd % 4 == 0 && rot % 8 == 0 && ldq % 4 == 0 && ldk % 4 == 0 &&
                       page_stride % 4 == 0 && (page_size % 8 != 0 || ((long)n_kv * page_size * hd) % 4 == 0) && by16(q) && by16(k) && by16(q_out) && by16(cache) && by16(cos_t) && by16(sin_t) &&
                       by16(q_bias) && by16(k_bias) && (long)n_rows * (n_heads + n_kv) * (hd / 4) < 2147483647L && (long)(n_rows + 7) / 8 * n_kv * vd < 2147483647L;
     if (rows && ((q_dtype == GI_F32 && cache_dtype == GI_F32) || (q_dtype == GI_BF16 && cache_dtype == GI_BF16))) {

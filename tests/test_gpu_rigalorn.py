@@ -532,6 +532,22 @@ def test_rows_of_prompts_are_turned_and_stored_as_rows_one_by_one(heads, kv, dk,
     assert bool((got[0][1] != 9.0).any())
 
 
+def test_queries_of_many_rows_may_be_turned_in_their_own_place():
+    """32-bit queries written over themselves, heads of 24 channels, whose pairs lie in two waves now and then: the numbers of queries written elsewhere."""
+    from geneinfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(3)
+    n, heads, kv, dk, page, rot = 200, 21, 1, 24, 8, 24
+    q, k, v = (torch.randn(n, width * dk, generator=g).to(DEV) for width in (heads, kv, kv))
+    cos, sin = (torch.randn(n, rot // 2, generator=g).to(DEV) for _ in range(2))
+    pos, slot, table = torch.arange(n, dtype=torch.int32, device=DEV), torch.zeros(n, dtype=torch.int32, device=DEV), torch.arange(n // page, dtype=torch.int32, device=DEV).view(1, -1)
+    got = []
+    for out in (torch.empty_like(q), q):
+        cache = torch.zeros(n // page, 1, 2 * kv * dk, page, device=DEV)
+        ops.norm_rope_store(q, k, v, None, None, 1e-6, cos, sin, rot, pos, slot, table, out, cache, page, heads, kv, dk, dk)
+        got.append((out, cache))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("T, window, far", [(200, None, 2), (200, 50, 150), (200, 50, 149), (45, 16, 29), (45, 16, 30)])
 def test_attention_through_latents_against_keys_and_values_made_in_full(T, window, far):
     """The kernels around the latent cache and the attention over it, with the up projections folded into query and output by hand
