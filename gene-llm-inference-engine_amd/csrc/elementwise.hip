@@ -705,7 +705,7 @@ __global__ __launch_bounds__(256) void turn_store_rows_kernel(const float* __res
     }
 }
 
-constexpr int TURN_STORE_ROWS = 64;
+constexpr int TURN_STORE_ROWS = 64, TURN_STORE_HEADS = 10000;
 GI_API int gi_norm_rope_store(const float* q, const float* k, const float* v, long ldq, long ldk, long ldv, const void* q_norm, const void* k_norm,
                               int norm_dtype, float eps, const float* cos_t, const float* sin_t, int rot, const int* pos, const int* slot,
                               const int* table, int table_stride, void* q_out, int q_dtype, void* cache, int cache_dtype, long page_stride,
@@ -758,9 +758,11 @@ GI_API int gi_norm_rope_store(const float* q, const float* k, const float* v, lo
         GI_CHECK_LAUNCH("norm_rope_store (plain)");
         return 0;
     }
-    // (not where the queries are turned in their own place, whose partners two threads read; from 64 rows on: 32 + 8 + 8 heads of 64, 5 rows 3.4 us a wave a head and 4.5 here, 48 rows 3.7 and 3.6, 64 4.0 and 3.7, 200 6.0 and 3.8)
+    // Not where the queries are turned in their own place, whose partners two threads read.  And from so many rows and heads on, for with fewer the kernel above, which spreads them over more waves, is as fast or
+    // faster, above all for rows that are no run of positions, whose values leave one by one (microseconds above and here: 32 + 8 + 8 heads of 64, 100 rows of a prompt 4.1 and 4.0, 200 5.5 and 3.5, 100 rows of
+    // their own 4.1 and 5.4, 200 5.7 and 5.7; 6 + 3 + 3 heads of 24 and 10, 200 rows of a prompt 3.3 and 3.2, of their own 3.3 and 5.0; 64 + 4 + 4 heads of 128 and 64, 131 5.8 and 3.9, 5.8 and 5.5).
     const auto by16 = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
-    const bool rows = k != nullptr && (const void*)q != q_out && n_rows >= TURN_STORE_ROWS && q_norm == nullptr && k_norm == nullptr && flags == 0 && hd % 4 == 0 && rot % 8 == 0 && ldq % 4 == 0 && ldk % 4 == 0 &&
+    const bool rows = k != nullptr && (const void*)q != q_out && n_rows >= TURN_STORE_ROWS && (long)n_rows * (n_heads + 2 * n_kv) >= TURN_STORE_HEADS && q_norm == nullptr && k_norm == nullptr && flags == 0 && hd % 4 == 0 && rot % 8 == 0 && ldq % 4 == 0 && ldk % 4 == 0 &&
                       page_stride % 4 == 0 && (page_size % 8 != 0 || ((long)n_kv * page_size * hd) % 4 == 0) && by16(q) && by16(k) && by16(q_out) && by16(cache) && by16(cos_t) && by16(sin_t) &&
                       by16(q_bias) && by16(k_bias) && (long)n_rows * (n_heads + n_kv) * (hd / 4) < 2147483647L && (long)(n_rows + 7) / 8 * n_kv * vd < 2147483647L;
     if (rows && ((q_dtype == GI_F32 && cache_dtype == GI_F32) || (q_dtype == GI_BF16 && cache_dtype == GI_BF16))) {

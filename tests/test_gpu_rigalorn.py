@@ -503,22 +503,23 @@ def test_attention_with_biases_blended_values_and_one_key_that_stands_out(T, win
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("heads, kv, dk, dv, rot, page, extras", [(4, 2, 64, 64, 32, 16, "all"), (6, 3, 24, 10, 8, 8, "all"), (2, 2, 4, 7, 0, 24, "biases"), (5, 1, 128, 128, 128, 4, "none"), (4, 2, 64, 33, 16, 16, "growth")])
 def test_rows_of_prompts_are_turned_and_stored_as_rows_one_by_one(heads, kv, dk, dv, rot, page, extras, dtype):
-    """64 rows or more of three requests (one from the middle of eight positions on, one of a few rows that shares windows with both others, one from a multiple of eight) in the kernel
-    for many rows, and the same rows ten at a time: queries, pages and kept values in bits."""
+    """Rows of three requests (one from the middle of eight positions on, one of a few rows that shares windows with both others, one from a multiple of eight) in the kernel
+    for many rows and heads (10,000 together), and the same rows 100 at a time: queries, pages and kept values in bits."""
     from geneinfer_amd.kernels import ops
     g = torch.Generator().manual_seed(dk + dv)
-    lens, firsts = [75, 4, 90], [5, 63, 16]
+    lens, firsts = [875, 4, 890], [5, 863, 16]
     n = sum(lens)
     q, k, v, other = (torch.randn(n, width, generator=g).to(DEV) for width in (heads * dk, kv * dk, kv * dv, kv * dv))
     biases = tuple(torch.randn(width, generator=g).to(DEV) for width in (heads * dk, kv * dk, kv * dv)) if extras in ("all", "biases") else None
     blend = (other, torch.tensor([0.35], device=DEV)) if extras == "all" else None
     pos = torch.cat([torch.arange(p, p + m) for p, m in zip(firsts, lens)]).to(DEV, torch.int32)
     slot = torch.cat([torch.full((m,), s) for s, m in zip((2, 0, 1), lens)]).to(DEV, torch.int32)
-    pages = 3 * -(-106 // page)
+    pages = 3 * -(-906 // page)
+    assert n * (heads + 2 * kv) >= 10000 > 100 * (heads + 2 * kv)
     table = torch.randperm(pages, generator=g).view(3, -1).to(DEV, torch.int32)
     cos, sin = (torch.randn(n, rot // 2, generator=g).to(DEV) for _ in range(2)) if rot else (None, None)
     got = []
-    for step in (n, 10):
+    for step in (n, 100):
         cache = torch.full((pages, kv * (dk + dv) * page), 9.0, dtype=dtype, device=DEV).view(pages, 1, kv * (dk + dv), page)
         q_out, keep = torch.empty(n, heads * dk, dtype=dtype, device=DEV), torch.empty(n, kv * dv, device=DEV) if extras == "all" else None
         for a in range(0, n, step):
@@ -536,7 +537,7 @@ def test_queries_of_many_rows_may_be_turned_in_their_own_place():
     """32-bit queries written over themselves, heads of 24 channels, whose pairs lie in two waves now and then: the numbers of queries written elsewhere."""
     from geneinfer_amd.kernels import ops
     g = torch.Generator().manual_seed(3)
-    n, heads, kv, dk, page, rot = 200, 21, 1, 24, 8, 24
+    n, heads, kv, dk, page, rot = 600, 21, 1, 24, 8, 24
     q, k, v = (torch.randn(n, width * dk, generator=g).to(DEV) for width in (heads, kv, kv))
     cos, sin = (torch.randn(n, rot // 2, generator=g).to(DEV) for _ in range(2))
     pos, slot, table = torch.arange(n, dtype=torch.int32, device=DEV), torch.zeros(n, dtype=torch.int32, device=DEV), torch.arange(n // page, dtype=torch.int32, device=DEV).view(1, -1)
