@@ -2383,12 +2383,14 @@ static int streamed_from_row(int strips, int K) {
 // Beside the strips' kernel (14 widths from 12,288 to 49,152 columns, 19 k from 64 to 14,336, 1 to 16 rows, slim and strips each for all of them, stored, gated and gated with a norm: the choice is 1.3 %
 // slower than the faster of the two on average, 15 % at worst).  What decides it: gated columns leave a strip more cheaply than 32-bit ones; a round of workgroups that strips of 64 columns fill badly is
 // slim's, whose strips are narrower, in the second round, and the strips' in the first, where their workgroups have a unit to themselves; and rows of weights a multiple of 4,096 bytes apart
-// cost the strips, which ask for 64 of them at once, more than slim (whole).  Microseconds, slim and strips:
+// cost the strips, which ask for 64 of them at once, more than slim (whole).  Of 4,020 other products (20 widths up to 64,000 columns, 28 k) the choice is 0.3 % slower than the faster of the two on average
+// for stored columns and 1.0 % for gated ones; a third round and more that is badly filled is slim's for some rows longer too.  Microseconds, slim and strips:
 //   gated                        1 row         8 rows        16 rows            stored                       1 row         8 rows        16 rows
 //   12,288 x 2,048               14.2, 13.1    15.7, 13.3    18.2, 13.4         12,288 x 2,048               11.1, 13.0    12.9, 13.1    15.9, 13.1
 //   16,384 x 2,048 (a norm)      16.7, 17.5    17.2, 17.9    19.6, 18.1         16,384 x 2,048               13.5, 16.6    16.1, 16.7    20.1, 16.7
 //   28,672 x 4,096               48.2, 44.3    54.0, 45.1    63.4, 45.4         18,432 x 8,192               58.8, 79.0    64.7, 79.8    80.4, 80.3
 //   12,288 x 256                 3.5, 4.1      3.9, 4.6      4.2, 4.6           12,288 x 3,072               14.2, 15.4    18.2, 15.8    22.7, 16.2
+//   33,280 x 3,072               43.5, 46.4    50.9, 46.1    60.7, 46.5         33,280 x 3,072               38.0, 46.5    48.6, 46.2    59.7, 46.9 (4 rows 41.0, 45.7, 6 44.4, 46.0)
 // Decoding 8 requests of the 1B shape, whose gated product has 16,384 x 2,048, takes 900 us with either; 9 take 957 with slim and 949 with strips.
 static int slim_until_row(int strips, int K, bool gated) {
     const int units = gi_compute_units();
@@ -2396,9 +2398,10 @@ static int slim_until_row(int strips, int K, bool gated) {
     const double filled = (double)strips / ((strips + units - 1) / units * units);
     if (!gated) {
         if (K <= 512) return three_quarters ? 12 : 0;
-        if (K < 1536) return strips > units && barely ? 10 : 0;
-        if (whole) return three_quarters ? 8 : narrow ? 4 : !second ? (filled > 0.9 ? 8 : 7) : barely ? 12 : 9;
-        return three_quarters ? 4 : narrow ? 0 : !second ? 2 : barely ? 10 : 6;
+        const bool third = strips > 2 * units;
+        if (K < 1536) return strips > units && barely ? 10 : third && filled < 0.8 && K > 1024 ? 4 : 0;
+        if (whole) return three_quarters ? 8 : narrow ? 4 : second ? (barely ? 12 : 9) : third && filled < 0.85 ? 10 : filled > 0.9 ? 8 : 7;
+        return three_quarters ? 4 : narrow ? 0 : second ? (barely ? 10 : 6) : third ? (filled < 0.8 ? 6 : filled < 0.9 ? 4 : 3) : strips > units ? 3 : 2;
     }
     int until;
     if (K < 1024) until = narrow && K > 512 ? 8 : strips * 2 <= units * 3 ? 12 : 10;

@@ -41,6 +41,7 @@ FEW_ROWS = [
     (8, 16384, 4096, True, "strips"), (8, 12288, 256, True, "slim"), (2, 20480, 3072, True, "slim"), (8, 20480, 3072, True, "strips"),
     (1, 12288, 2048, False, "slim"), (12, 12288, 2048, False, "strips"), (1, 12288, 3072, False, "slim"), (1, 13056, 3072, False, "strips"), (4, 16384, 2048, False, "slim"),
     (12, 16384, 2048, False, "strips"), (2, 18432, 8192, False, "slim"), (4, 24576, 4096, False, "slim"), (4, 24576, 512, False, "streamed"), (4, 24576, 768, False, "strips"), (1, 32768, 4096, False, "slim"), (8, 32768, 3072, False, "strips"),
+    (4, 33280, 3072, False, "slim"), (8, 33280, 3072, False, "strips"), (3, 33280, 1280, False, "slim"), (4, 40960, 3072, False, "strips"), (3, 40960, 3072, False, "slim"), (8, 33280, 2048, False, "slim"), (3, 28672, 3072, False, "strips"),
     (16, 16384, 512, False, "streamed"), (16, 16384, 768, False, "strips"), (20, 16384, 512, False, "strips"), (4, 128256, 2048, False, "slim"), (5, 128256, 2048, False, "strips"),
     (11, 16384, 2056, True, "slim"), (12, 16384, 2056, True, "streamed"), (16, 3072, 2048, False, "slim"), (17, 3072, 2048, False, "slim tiles"), (17, 3072, 2048, True, "strips"),
     (128, 3072, 2048, False, "strips"), (128, 3072, 2056, False, "streamed"), (129, 3072, 2048, False, None),
