@@ -282,8 +282,8 @@ def test_gated_products_have_one_gate(m, inter, k, few, columns, stride, gated, 
 @pytest.mark.parametrize("m", [1, 17, 33, 64, 65, 97, 128, 129, 160, 161, 192, 193, 225, 256])
 @pytest.mark.parametrize("n,k", [(12320, 64), (12288 + 48, 192), (16384, 576), (200, 1088), (3072, 1536), (2048, 2112)])
 def test_gemm_bf16_strips(m, n, k):
-    """64 columns by all rows: on both sides of every height, one to more blocks of k than the ring has stages, a last strip of 32 and of 48 columns, k in one to four shares
-    (uneven ones too), stored, added, in bfloat16 and gated."""
+    """64 columns by all rows, up to 128 of them: on both sides of every height, one to more blocks of k than the ring has stages, a last strip of 8, 32 and 48 columns, k whole and in two to seven shares
+    (uneven ones too), stored, added, in bfloat16 and gated.  With more rows strips make some of these products: two tiles of rows in two shares (3,072 x 1,536), gated ones with all of k."""
     a, w = randn(m, k, dtype=torch.bfloat16, seed=1), randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.1)
     want = a.double() @ w.double().T
     out = torch.full((m, n + 4), 3.0, device=DEV)
@@ -301,16 +301,89 @@ def test_gemm_bf16_strips(m, n, k):
         assert rel(gated[:m], (torch.nn.functional.silu(gate) * up).reshape(m, n // 2)) < 4.1e-3 and bool((gated[m:] == 3.0).all())
 
 
-@pytest.mark.parametrize("m,n,k", [(257, 2048, 2112), (301, 3072, 192), (450, 1024, 1984), (700, 200, 576), (897, 2048, 8192), (1000, 960, 704), (1400, 2048, 1088), (1536, 64 * 30, 640), (1537, 1920, 640)])
-def test_gemm_bf16_strips_in_several_tiles_of_rows(m, n, k):
-    """Tiles of equal height, the last one a few rows lower (52 of 65 at 897 rows), k in uneven shares; on both sides of the most rows."""
-    a, w = randn(m, k, dtype=torch.bfloat16, seed=1), randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.1)
+# m, n, k -> tiles of rows, rows of the last one, shares of k, blocks of 64 of a share and of the last one
+@pytest.mark.parametrize("m,n,k,tiles,last,shares,blocks,last_blocks",
+                         [(m, 3072, 8192, 1, m, 5, 26, 24) for m in (17, 33, 65, 97, 128, 129, 160, 161, 192, 193, 224, 225, 256)] +
+                         [(33, 200, 1088, 1, 33, 5, 4, 1), (129, 200, 4096, 3, 43, 13, 5, 4), (193, 2048, 2048, 4, 46, 2, 16, 16), (257, 2048, 8192, 2, 128, 4, 32, 32), (301, 2048, 2048, 4, 73, 2, 16, 16),
+                          (400, 500, 4096, 7, 52, 4, 16, 16), (897, 2048, 8192, 4, 222, 2, 64, 64), (897, 2048, 2048, 8, 106, 1, 32, 32), (1536, 1920, 640, 8, 192, 1, 10, 10), (225, 3072, 1536, 4, 54, 1, 24, 24)])
+def test_gemm_bf16_strips_of_shared_k(m, n, k, tiles, last, shares, blocks, last_blocks):
+    """k in even and uneven shares, one tile of every height (both ends of the rows that each has) or several of equal height, the last of them a few rows lower: stored, added and in bfloat16, whole
+    matrices and columns of wider ones; the cut is the one named."""
+    assert ops().gemm_bf16_strip_cut(m, n, k) == (tiles, shares)
+    tile_rows, per = -(-m // tiles), -(-(k // 64) // shares)
+    assert (m - (tiles - 1) * tile_rows, per, k // 64 - (shares - 1) * per) == (last, blocks, last_blocks)
+    wide_a, wide_w = randn(m, k + 24, dtype=torch.bfloat16, seed=1), randn(n, k + 40, dtype=torch.bfloat16, seed=2, scale=0.1)
+    a, w = wide_a[:, 8:8 + k], wide_w[:, 16:16 + k]
     want = a.double() @ w.double().T
-    out = torch.full((m + 1, n + 4), 3.0, device=DEV)
+    seen = []
+    for left, right in ((a, w), (a.contiguous(), w.contiguous())):
+        out = torch.full((m + 1, n + 4), 3.0, device=DEV)
+        ops().gemm_bf16(left, right, out[:m, :n])
+        assert rel(out[:m, :n], want) < 2e-6 and bool((out[:, n:] == 3.0).all()) and bool((out[m:] == 3.0).all())
+        rounded = torch.full((m + 1, n), 3.0, dtype=torch.bfloat16, device=DEV)
+        ops().gemm_bf16(left, right, rounded[:m])
+        assert torch.equal(rounded[:m], out[:m, :n].bfloat16()) and bool((rounded[m:] == 3.0).all())
+        ops().gemm_bf16(left, right, out[:m, :n], accumulate=True)
+        assert rel(out[:m, :n], 2 * want) < 2e-6 and bool((out[m:] == 3.0).all())
+        seen.append(out)
+    assert torch.equal(*seen)
+
+
+@pytest.mark.parametrize("gated,limit", [(True, 0.0), ("gelu_tanh", 0.0), ("swish_clamped", 1.5)])
+@pytest.mark.parametrize("m", [129, 160, 161, 192])
+def test_gemm_bf16_strips_gate_up_to_192_rows(m, gated, limit):
+    """Every gate at both heights of strips above 128 rows, the last strip of 32 columns; whole matrices and columns of wider ones in bits."""
+    inter, k = 6160, 1088
+    assert ops().gemm_bf16_large_kernel(m, 2 * inter, k, "gated") == "strips"
+    wide_a, wide_w = randn(m, k + 24, dtype=torch.bfloat16, seed=1), randn(2 * inter, k + 40, dtype=torch.bfloat16, seed=2, scale=0.05)
+    a, w = wide_a[:, 8:8 + k], wide_w[:, 16:16 + k]
+    gate, up = (a.double() @ w.double().T).view(m, inter // 16, 2, 16).unbind(2)
+    if gated == "swish_clamped":
+        gate, up = gate.clamp(max=limit), up.clamp(-limit, limit) + 1
+        want = gate * torch.sigmoid(1.702 * gate) * up
+    else:
+        want = (torch.nn.functional.silu(gate) if gated is True else 0.5 * gate * (1 + torch.tanh((2 / torch.pi) ** 0.5 * (gate + 0.044715 * gate ** 3)))) * up
+    seen = []
+    for left, right in ((a, w), (a.contiguous(), w.contiguous())):
+        out = torch.full((m + 1, inter + 2), 3.0, dtype=torch.bfloat16, device=DEV)
+        ops().gemm_bf16(left, right, out[:m, :inter], gated=gated, gate_limit=limit)
+        assert rel(out[:m, :inter], want.reshape(m, inter)) < 4.1e-3 and bool((out[m:] == 3.0).all()) and bool((out[:, inter:] == 3.0).all())
+        seen.append(out)
+    assert torch.equal(*seen)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 12320, 64), (20, 16384, 576), (64, 12320, 192), (97, 12320, 576), (128, 16384, 1088)])
+def test_gemm_bf16_strips_of_columns_of_wider_matrices(m, n, k):
+    """All of k in a workgroup: rows of A and W further apart than k, in bits as whole matrices."""
+    assert ops().gemm_bf16_small_kernel(m, n, k) == "strips"
+    wide_a, wide_w = randn(m, k + 24, dtype=torch.bfloat16, seed=1), randn(n, k + 40, dtype=torch.bfloat16, seed=2, scale=0.1)
+    a, w = wide_a[:, 8:8 + k], wide_w[:, 16:16 + k]
+    out, whole = torch.full((m + 1, n + 4), 3.0, device=DEV), torch.empty(m, n, device=DEV)
     ops().gemm_bf16(a, w, out[:m, :n])
-    assert rel(out[:m, :n], want) < 2e-6 and bool((out[:, n:] == 3.0).all()) and bool((out[m:] == 3.0).all())
-    ops().gemm_bf16(a, w, out[:m, :n], accumulate=True)
-    assert rel(out[:m, :n], 2 * want) < 2e-6 and bool((out[m:] == 3.0).all())
+    ops().gemm_bf16(a.contiguous(), w.contiguous(), whole)
+    assert torch.equal(out[:m, :n], whole) and rel(whole, a.double() @ w.double().T) < 2e-6 and bool((out[:, n:] == 3.0).all()) and bool((out[m:] == 3.0).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 3072, 8192), (131, 3072, 8192)])
+@pytest.mark.parametrize("short_of", ["scratch", "strides"])
+def test_products_that_strips_do_not_make_go_the_way_before(m, n, k, short_of, monkeypatch):
+    """With the scratch of the kernels before strips, fewer shares of k than strips make, and with rows of A further apart than a strip's 32-bit offsets are asked to reach."""
+    o = ops()
+    before = o.lib().gi_gemm_bf16_skinny_splits(n, k) if m <= 128 else o.lib().gi_gemm_bf16_piped_splits(m, n, k)
+    assert 0 < before < o.gemm_bf16_strip_cut(m, n, k)[1]
+    a, w = randn(m, k, dtype=torch.bfloat16, seed=1), randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.1)
+    strips, out = torch.empty(m, n, device=DEV), torch.full((m + 1, n + 4), 3.0, device=DEV)
+    o.gemm_bf16(a, w, strips)
+    if short_of == "scratch":
+        monkeypatch.setattr(o, "_scratch_floats", lambda *_: before * m * n)
+    else:
+        far = torch.empty(m, 1 << 22, dtype=torch.bfloat16, device=DEV)[:, :k]
+        far.copy_(a)
+        a = far
+    o.gemm_bf16(a, w, out[:m, :n])
+    want = a.double() @ w.double().T
+    assert rel(out[:m, :n], want) < 2e-6 and rel(strips, want) < 2e-6 and bool((out[:, n:] == 3.0).all()) and bool((out[m:] == 3.0).all())
+    assert not torch.equal(out[:m, :n], strips)                            # (the sums of other shares)
 
 
 @pytest.mark.parametrize("m,parts", [(1, 512), (8, 300), (9, 256), (16, 3), (17, 256), (32, 2), (33, 8), (64, 1), (128, 5)])
