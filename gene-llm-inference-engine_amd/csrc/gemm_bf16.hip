@@ -1419,15 +1419,16 @@ __global__ __launch_bounds__(512, MT == 2 ? 4 : 2) void gemm_bf16_skinny_kernel(
 // quarters' sums meet in LDS, (0 + 2) + (1 + 3).  A wave reads the next stage's operands while it multiplies this one's.
 // Bound by the weights on their way from memory (a strip of 64 rows gives 256 workgroups 28 to 56 KB each of them in flight), and from 100 rows or so on by what
 // a unit takes in of A besides: one tile for all rows reads the weights once, where 131 rows in two tiles of 128 had half of the units load them for three rows.  Microseconds
-// in a captured chain, before (weights through registers up to 128 rows, tiles of 128 x 128 above; where k is shared out with the kernel that adds up) and now:
+// a product, in a captured chain of products that each have weights of their own (640 MB of them a chain), with the kernel that adds up where k is shared out; before (weights
+// through registers up to 128 rows, tiles of 128 x 128 above) and now:
 //   rows                     17            64            128           131           192
-//   16,384 x 2,048 gated     18.2, 17.1    22.4, 19.5    30.7, 24.7    31.0, 25.6    31.9, 29.0
-//   28,672 x 4,096 gated     53.5, 46.8    65.4, 55.5    93.2, 71.7    (as before)
-//   2,048 x 2,048 added      (other)       10.7, 8.8     14.4, 12.4    14.8, 13.0    17.2, 14.9
-//   2,048 x 8,192 added      13.9, 12.8    15.8, 14.5    20.0, 19.2    24.5, 19.9    26.0, 22.4
-//   3,072 x 8,192 added      19.1, 16.7    22.0, 19.0    28.6, 24.4    38.6, 25.2    41.0, 29.0
-//   4,096 x 14,336 added     28.6, 27.5    35.1, 32.9    46.0, 42.9    61.5, 43.7    63.9, 50.4
-//   128,256 x 2,048 stored   107.5, 102.2  130, 122      182, 150
+//   16,384 x 2,048 gated     18.2, 17.4    21.8, 18.5    29.8, 23.1    28.4, 23.4    28.9, 27.3
+//   28,672 x 4,096 gated     53.2, 47.8    63.3, 53.0    90.0, 68.2    (as before)
+//   2,048 x 2,048 added      (other)       10.1, 9.4     14.0, 11.0    14.5, 11.1    16.7, 11.9
+//   2,048 x 8,192 added      12.8, 11.8    15.1, 13.5    20.4, 17.9    23.8, 19.0    25.4, 21.6
+//   3,072 x 8,192 added      17.9, 15.4    21.2, 17.7    27.2, 22.5    37.5, 23.3    39.7, 28.3
+//   4,096 x 14,336 added     27.2, 26.0    33.6, 30.0    42.9, 39.5    57.0, 38.5    59.9, 46.9
+//   128,256 x 2,048 stored   107.1, 101.9  134.7, 121.1  184.7, 149.2  (as before)
 // The sums of a product have fewer and longer chains than before; against 64 bits they are nearer (2,048 x 8,192: 1.1e-7 for 1.4 to 1.9e-7).
 constexpr int strip_ring(int tm, int stages) { return stages * (64 + 32 * tm) * 128; }
 constexpr int strip_chunk(int tm, int stages) { return strip_ring(tm, stages) / 32768 < tm ? strip_ring(tm, stages) / 32768 : tm; }       // fragments whose quarters' sums fit the ring
@@ -2143,9 +2144,8 @@ int epilogue_of(int c_dtype, int accumulate) {
 
 }  // namespace
 
-// Number of k-splits of the skinny kernel for a product with 17..64 rows, so that the caller can size
-// the scratch (splits * M * N floats); 0: the output is wide enough to fill the chip without a split,
-// no scratch is needed.  Workgroups for three quarters of the chip or more, each with at least one block of k (measured at 33 to
+// Number of k-splits of the skinny kernel for a product with 17..128 rows (what scratch a product wants, strips' shares among it, gi_gemm_bf16_scratch_floats says);
+// 0: the output is wide enough to fill the chip without a split, no scratch is needed.  Workgroups for three quarters of the chip or more, each with at least one block of k (measured at 33 to
 // 64 rows, product and reduce kernel together: 192 to 384 workgroups on 256 compute units, with two blocks of k each, take 11 us for N = 3072, K = 2048 and
 // 16 us for N = 2048, K = 8192; twice the workgroups with one block each 12.5 and 17.5 us, half of them 13 and 22 us).
 GI_API int gi_gemm_bf16_skinny_splits(int N, int K) {
@@ -2255,7 +2255,7 @@ static bool takes_large(int M, int N, int K) { return M > SKINNY_MAX_ROWS && K %
 
 // Products whose k is shared out, in strips: tiles of rows (one to some, of equal height), shares of k, and about how long it takes with the kernel that adds up.  The times are fitted
 // to 4,600 products (24 numbers of rows from 17 to 1,400, 12 sizes of weights, every cut), which they meet within 6 %; the cut they choose is 0.7 % slower than the best one on average, 11 % at worst.
-// 128 rows of 2,048 x 2,048 take 12.2 us as one tile in four shares, 10.2 as two in three; 301 of 2,048 x 8,192 27 as two in four, 32 as three in two.
+// What the fit misses at other sizes (few columns, long shares) find_shared_strips allows for.  128 rows of 2,048 x 2,048 take 12.2 us as one tile in four shares, 10.2 as two in three; 301 of 2,048 x 8,192 27 as two in four, 32 as three in two.
 struct StripCut { int tiles, splits; double us; };
 static StripCut strip_cut(int M, int N, int K) {
     const int strips = (N + 63) / 64, units = gi_compute_units(), all = K / PK;

@@ -132,6 +132,13 @@ class FeedForward(Part):
 #                                  None; with it `use_input_weight(view)` (the same matrix as a view of a larger one, to keep instead of its
 #                                  own) and a keyword `projected` of `forward` (float32 [rows, that matrix's rows]: the product, already made).
 #                                  A block whose parts read the same rows may then make their first products as one (`ParallelBlock`).
+#   input_activation()             beside `input_weight()`: (parameters, columns, dtype) of the activation that follows the first product, if the block's product may end in it
+#                                  (`linear_xielu`); a keyword `activated` of `forward` is then the activated columns.
+#   output_weight()                the matrix of the part's last product, or None where a block may not make that product (rows that are not bfloat16 before it); with it
+#                                  `use_output_weight(view)` (the same matrix as columns of a wider one) and a keyword `into` of `forward` (bfloat16 [rows, that matrix's columns], a
+#                                  range of columns of a wider buffer): the part writes there what it would have multiplied, leaves `residual` as it is, makes no product and
+#                                  returns None.  It is given no `then` beside `into`, whose norm goes to the block's product.  A block whose parts add onto the same rows may
+#                                  then make their last products as one (`ParallelBlock`).
 #   makes_next_norm(norm)          whether the part, where it writes the residual last, can also make the rows of `norm`, the norm that reads the
 #                                  residual next; `forward` then takes `then` (that norm) and returns the rows ready (`ReadyRows`) or None.
 
