@@ -663,8 +663,10 @@ static bool by_blocks(int n_rows, int n_single, int n_heads, int n_kv, int hd, i
     const bool nearly_one_round = walks <= units && (n_spans > 4 ? 4 * walks > 3 * units : 8 * walks > 7 * units && pairs >= 900);
     return !nearly_one_round && n_spans - 1 <= 22 * ((walks + units - 1) / units) + 2;
 }
+// Floats for the parts: what spans leave, and what the call asks for (with fewer than blocks leave it goes by spans).
+GI_API long gi_attention_exact_span_floats(int n_rows, int n_heads, int vd, int n_spans) { return (long)n_rows * n_heads * n_spans * part_floats(vd); }
 GI_API long gi_attention_exact_part_floats(int n_rows, int n_single, int n_heads, int n_kv, int hd, int vd, int n_spans) {
-    return (long)n_rows * n_heads * n_spans * (by_blocks(n_rows, n_single, n_heads, n_kv, hd, vd, n_spans) ? 4 : 1) * part_floats(vd);
+    return gi_attention_exact_span_floats(n_rows, n_heads, vd, n_spans) * (by_blocks(n_rows, n_single, n_heads, n_kv, hd, vd, n_spans) ? 4 : 1);
 }
 
 GI_API int gi_attention_exact(const void* q, int q_dtype, const void* cache, int cache_dtype, void* out, int out_dtype, const int* pos,
@@ -685,8 +687,8 @@ GI_API int gi_attention_exact(const void* q, int q_dtype, const void* cache, int
         GI_REQUIRE(n_single >= 0 && n_single <= n_rows, "attention_exact: %d single rows of %d", n_single, n_rows);
         const int a_tile = rows_a_tile(n_heads / n_kv), turns = n_single == n_rows ? 1 : n_requests > 0 && n_requests < a_tile ? n_requests : a_tile;
         if (n_spans > 0) {
-            GI_REQUIRE(part != nullptr && aligned(part) && part_size >= (long)n_rows * n_heads * n_spans * part_floats(vd) && n_spans <= MAX_SPANS,
-                       "attention_exact: sharing the keys out needs %ld floats", (long)n_rows * n_heads * n_spans * part_floats(vd));
+            GI_REQUIRE(part != nullptr && aligned(part) && part_size >= gi_attention_exact_span_floats(n_rows, n_heads, vd, n_spans) && n_spans <= MAX_SPANS,
+                       "attention_exact: sharing the keys out needs %ld floats", gi_attention_exact_span_floats(n_rows, n_heads, vd, n_spans));
         } else {
             part = nullptr;
         }
@@ -694,7 +696,7 @@ GI_API int gi_attention_exact(const void* q, int q_dtype, const void* cache, int
         while ((1LL << pages.shift) < page_size) ++pages.shift;
         pages.magic = (unsigned)((((1ULL << pages.shift) - page_size) << 32) / page_size + 1);
         const dim3 tiles((unsigned)count_tiles(n_rows, n_single, n_kv, n_heads / n_kv), part ? n_spans : 1, turns);
-        if (part && by_blocks(n_rows, n_single, n_heads, n_kv, hd, vd, n_spans) && part_size >= 4L * n_rows * n_heads * n_spans * part_floats(vd)) {
+        if (part && by_blocks(n_rows, n_single, n_heads, n_kv, hd, vd, n_spans) && part_size >= 4 * gi_attention_exact_span_floats(n_rows, n_heads, vd, n_spans)) {
             const int n_blocks = 4 * n_spans;
             const dim3 blocks(tiles.x, n_blocks, tiles.z);
 #define BLOCKS(D)                                                                                                                          \

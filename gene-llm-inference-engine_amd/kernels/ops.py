@@ -141,6 +141,8 @@ def lib():
         l.gi_attention_exact_spans.restype = c_int
         l.gi_attention_exact_part_floats.argtypes = [c_int, c_int, c_int, c_int, c_int, c_int, c_int]
         l.gi_attention_exact_part_floats.restype = c_long
+        l.gi_attention_exact_span_floats.argtypes = [c_int, c_int, c_int, c_int]
+        l.gi_attention_exact_span_floats.restype = c_long
         l.gi_attention_exact_max_head_size.argtypes = []
         l.gi_attention_exact_max_head_size.restype = c_int
         l.gi_attention_decode_workgroups_per_unit.argtypes = [c_int, c_int, c_int, c_int]
@@ -701,7 +703,10 @@ def attention_exact(q, cache, out, positions, slots, table, n_heads, n_kv, hd, w
         seen = min([int(max_context)] + ([int(window)] if window else []) + ([int(chunk)] if chunk else []))
         n_spans, n_part = _exact_spans(n, n_single, n_heads, n_kv, hd, vd, page_size, -(-seen // 256) * 256)
         if n_spans:
-            part = torch.empty(n_part, dtype=torch.float32, device=out.device)
+            part = _room(n_part, out.device)
+            if part is None:                         # (with a quarter of it blocks of keys go by spans, in the same bits)
+                n_part = lib().gi_attention_exact_span_floats(n, n_heads, vd, n_spans)
+                part = torch.empty(n_part, dtype=torch.float32, device=out.device)
     _call("gi_attention_exact", q.data_ptr(), _code(q, "attention: q"), cache.data_ptr(), _code(cache, "attention: cache"), out.data_ptr(),
           _code(out, "attention: out"), positions.data_ptr(), slots.data_ptr(), table.data_ptr(), table.stride(0), cache.stride(0),
           page_size, n, n_heads, n_kv, hd, vd, int(window or 0), int(chunk or 0), float(scale if scale is not None else hd ** -0.5),

@@ -1458,6 +1458,21 @@ def test_attention_exact_of_blocks_one_by_one(n_heads, n_kv, hd, vd, window, chu
     assert clean[0] and any(clean[len(picked):2 * len(picked)]) and all(clean[:len(picked)]) and not all(clean)
 
 
+@pytest.mark.parametrize("rows,n_heads,n_kv,hd,seen", [(3, 24, 8, 128, 600), (12, 32, 8, 64, 600)])
+def test_attention_exact_without_room_for_blocks_goes_by_spans(rows, n_heads, n_kv, hd, seen, monkeypatch):
+    """A device that has no room for what blocks of keys leave: spans leave a quarter of it, and the bits are the same."""
+    ps, g = 16, torch.Generator(device=DEV).manual_seed(hd)
+    pages = -(-seen // ps)
+    cache, q = torch.randn(pages, n_kv * ps * 2 * hd, device=DEV, generator=g), torch.randn(rows, n_heads * hd, device=DEV, generator=g)
+    table, slots = torch.arange(pages, dtype=torch.int32, device=DEV).view(1, -1), torch.zeros(rows, dtype=torch.int32, device=DEV)
+    pos = torch.tensor([seen - 1 - 37 * i for i in range(rows)], dtype=torch.int32, device=DEV)
+    attend = lambda: ops().attention_exact(q, cache, torch.full_like(q, 7.0), pos, slots, table, n_heads, n_kv, hd, page_size=ps, single_rows=True, max_context=seen)
+    blocks, asked = attend(), []
+    monkeypatch.setattr(ops(), "_room", lambda floats, device: asked.append(floats))
+    spans = attend()
+    assert torch.equal(spans, blocks) and asked == [4 * ops().lib().gi_attention_exact_span_floats(rows, n_heads, hd, ops()._exact_spans(rows, rows, n_heads, n_kv, hd, hd, ps, 768)[0])]
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_finds_one_far_key(dtype):
     """Among 700 keys one is scaled so that its score stands out: the output must be its value."""

@@ -189,6 +189,37 @@ def test_no_room_for_scratch_is_no_error(monkeypatch):
     assert ops._room(5, "cpu") is None
 
 
+def _launches_with_room_for(floats, monkeypatch):
+    """What is launched from here on, on a device with room for allocations of up to so many numbers."""
+    launched, empty = [], torch.empty
+
+    def bounded(*size, **kw):
+        if torch.Size(size[0] if len(size) == 1 and not isinstance(size[0], int) else size).numel() > floats:
+            raise torch.OutOfMemoryError("full")
+        return empty(*size, **kw)
+
+    monkeypatch.setattr(ops, "_dev", lambda *tensors: None)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_call", lambda name, *a: launched.append((name, a)))
+    monkeypatch.setattr(torch, "empty", bounded)
+    return launched
+
+
+@pytest.mark.parametrize("rows,hd,seen", [(3, 128, 600), (12, 64, 600)])
+def test_attention_without_room_for_blocks_of_keys_goes_by_spans(rows, hd, seen, monkeypatch):
+    """The blocks of keys leave four times the numbers that the spans leave: a step that fits with spans is not refused."""
+    spans, floats = ops._exact_spans(rows, rows, 24, 8, hd, hd, 16, -(-seen // 256) * 256)
+    least = rows * 24 * spans * (hd + 4)
+    assert floats == 4 * least
+    q, at, cache = torch.zeros(rows, 24 * hd), torch.zeros(rows, dtype=torch.int32), torch.zeros(4, 8 * 16 * 2 * hd)
+    out, table = torch.zeros_like(q), torch.zeros(rows, 4, dtype=torch.int32)
+    for room, given in ((floats, floats), (floats - 1, least), (least, least)):
+        with monkeypatch.context() as patch:
+            launched = _launches_with_room_for(room, patch)
+            ops.attention_exact(q, cache, out, at, at, table, 24, 8, hd, page_size=16, single_rows=True, max_context=seen)
+            assert [(name, a[-3:-1]) for name, a in launched] == [("gi_attention_exact", (given, spans))]
+
+
 def test_products_of_few_rows_ask_for_nothing_by_kind(monkeypatch):
     for m, n, k in [(1, 3072, 2048), (17, 2048, 8192), (128, 16384, 2048), (128, 28672, 4096)]:
         assert m <= ops.FEW_ROWS and len({ops._scratch_floats(m, n, k, kind, counted) for kind in range(len(ops.PRODUCT_KINDS)) for counted in (False, True)}) == 1
