@@ -2340,6 +2340,13 @@ GI_API long gi_gemm_bf16_scratch_floats(int M, int N, int K, int kind, int count
     return gi_gemm_bf16_shares(M, N, K, kind, counters) > 1 ? tall_scratch_floats(large_kernel_of_kind(M, N, K, kind, counters != 0).cut) : 0;
 }
 
+// The least that such a product does with: with less than the above the kernels beside strips make it, and beside shared tiles (0: they need none).
+GI_API long gi_gemm_bf16_least_scratch_floats(int M, int N, int K) {
+    if (M <= SKINNY_MAX_ROWS) return (long)gi_gemm_bf16_skinny_splits(N, K) * M * N;
+    const int splits = gi_gemm_bf16_piped_splits(M, N, K);
+    return splits > 1 ? (long)splits * M * N : 0;
+}
+
 static const NormIn NO_NORM_IN = {nullptr, 0, 0.f, 1, 0.f};
 static const NormOut NO_NORM_OUT = {nullptr, nullptr, 0, nullptr};
 

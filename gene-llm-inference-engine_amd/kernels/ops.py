@@ -159,6 +159,8 @@ def lib():
         l.gi_gemm_exact_scratch_floats.restype = c_long
         l.gi_gemm_bf16_scratch_floats.argtypes = [c_int, c_int, c_int, c_int, c_int]
         l.gi_gemm_bf16_scratch_floats.restype = c_long
+        l.gi_gemm_bf16_least_scratch_floats.argtypes = [c_int, c_int, c_int]
+        l.gi_gemm_bf16_least_scratch_floats.restype = c_long
         l.gi_gemm_bf16_norm_parts.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_bf16_norm_parts.restype = c_int
         l.gi_attention_prompt_share_floats.argtypes = [c_int, c_int, c_int, c_int, c_int, c_int, c_int]
@@ -1773,16 +1775,24 @@ def _shares(m, n, k, kind, counted) -> int:
 FEW_ROWS = 128
 
 
+def _split_scratch(floats, m, n, k, device):
+    """(scratch, its floats) of a product whose k is shared out and whose kernels ask for so many: without room for those, what the kernels beside strips make it with."""
+    scratch = _room(floats, device)
+    if scratch is None:
+        floats = lib().gi_gemm_bf16_least_scratch_floats(m, n, k)
+        scratch = torch.empty(floats, dtype=torch.float32, device=device)
+    return scratch, floats
+
+
 def _product_scratch(m, n, k, kind, counted, device):
-    """(scratch, its floats) of a product: partial sums where k is shared out over workgroups.  Without the room for shared tiles' sums the product's other
-    kernels make it."""
+    """(scratch, its floats) of a product: partial sums where k is shared out over workgroups.  Without the room for them the product's other kernels make it."""
     floats = _scratch_floats(m, n, k, kind, counted)
     if not floats:
         return None, 0
     if _shares(m, n, k, kind, counted) > 1:
         scratch = _room(floats, device)
         return scratch, floats if scratch is not None else 0
-    return torch.empty(floats, dtype=torch.float32, device=device), floats
+    return _split_scratch(floats, m, n, k, device)
 
 
 def step_counters(ctx, m, n, k, kind=0):
@@ -1840,7 +1850,7 @@ def gemm_bf16(a, w, out, accumulate=False, gated=False, checked=False, norm_in=N
         raise KernelError("gemm_bf16: operands must be bfloat16 with K and row strides multiples of 8, 16-byte aligned")
     if m <= FEW_ROWS:
         n_scratch = _scratch_floats(m, n, k, 0, False)
-        scratch = torch.empty(n_scratch, dtype=torch.float32, device=a.device) if n_scratch else None
+        scratch, n_scratch = _split_scratch(n_scratch, m, n, k, a.device) if n_scratch else (None, 0)
     else:
         kind = product_kind(out, accumulate, gated, norm_in, norm_out)
         if counters is None:
@@ -1888,8 +1898,7 @@ def gemm_bf16_onto_norm(a, w, x, g, eps, normed, checked=False):
     if not (w.shape == (n, k) and x.shape == (m, n) and x.dtype == torch.float32 and (checked or (gemm_bf16_supports(a, w, x) and gemm_bf16_onto_norm_takes(m, n, k)))
             and g.dtype == torch.float32 and g.shape == (n,) and g.is_contiguous() and normed.dtype == torch.bfloat16 and normed.shape == (m, n) and normed.stride(1) == 1):
         raise KernelError("gemm_bf16_onto_norm: bfloat16 operands, float32 rows [m, n] and weights [n], bfloat16 [m, n] for the normed rows, and sizes that are taken")
-    n_scratch = _scratch_floats(m, n, k, 1, False)
-    scratch = torch.empty(n_scratch, dtype=torch.float32, device=a.device)
+    scratch, n_scratch = _split_scratch(_scratch_floats(m, n, k, 1, False), m, n, k, a.device)
     if _profile is not None:
         _profile.note = (f"{n}x{k}", n * k * w.element_size())
     _call("gi_gemm_bf16_onto_norm", a.data_ptr(), w.data_ptr(), x.data_ptr(), m, n, k, a.stride(0), w.stride(0), x.stride(0), scratch.data_ptr(), n_scratch, g.data_ptr(),
@@ -1982,7 +1991,7 @@ def gemm_bf16_qkv_rope_store(a, w, cos, sin, positions, slots, table, q_out, cac
         raise KernelError("gemm: the pieces of the sums of squares must be float32 [m, pieces]")
     if m <= FEW_ROWS:
         n_scratch = _scratch_floats(m, n, k, 0, False)
-        scratch = torch.empty(n_scratch, dtype=torch.float32, device=a.device) if n_scratch else None
+        scratch, n_scratch = _split_scratch(n_scratch, m, n, k, a.device) if n_scratch else (None, 0)
     else:
         if counters is None:
             counters = step_counters(ctx, m, n, k, 5)

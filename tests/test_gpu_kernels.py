@@ -1154,6 +1154,19 @@ def test_workgroups_that_meet_on_two_streams_at_once():
         assert all(torch.equal(x, want[i % 3]) for i, x in enumerate(results))
 
 
+@pytest.mark.parametrize("m", [33, 131])
+def test_a_product_without_room_for_strips_is_made_beside_them(m, monkeypatch):
+    """A device that has no room for the sums of strips' shares of k (five here): those of the kernels before them (four) are enough."""
+    o, n, k = ops(), 3072, 8192
+    a, w = randn(m, k, dtype=torch.bfloat16, seed=1), randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.1)
+    strips, out, asked = o.gemm_bf16(a, w, torch.empty(m, n, device=DEV)), torch.full((m + 1, n), 3.0, device=DEV), []
+    monkeypatch.setattr(o, "_room", lambda floats, device: asked.append(floats))
+    o.gemm_bf16(a, w, out[:m])
+    want = a.double() @ w.double().T
+    assert asked == [5 * m * n] and o.lib().gi_gemm_bf16_least_scratch_floats(m, n, k) == 4 * m * n
+    assert rel(out[:m], want) < 2e-6 and rel(strips, want) < 2e-6 and not torch.equal(out[:m], strips) and bool((out[m:] == 3.0).all())
+
+
 @pytest.mark.parametrize("hd, m", [(128, 1000), (64, 1500)])
 def test_without_room_for_scratch_nothing_is_shared_out(hd, m, monkeypatch):
     """A device that has no room for the sums of shared tiles and walks: the kernels that share nothing out serve, as without a step's memory of its own."""

@@ -220,6 +220,30 @@ def test_attention_without_room_for_blocks_of_keys_goes_by_spans(rows, hd, seen,
             assert [(name, a[-3:-1]) for name, a in launched] == [("gi_attention_exact", (given, spans))]
 
 
+@pytest.mark.parametrize("m,n,k,before", [(33, 3072, 8192, 4), (131, 3072, 8192, 4), (96, 10240, 8192, 2), (40, 128, 12288, 32), (64, 2048, 2056, 8)])
+def test_a_product_without_room_for_strips_shares_of_k_has_those_of_before(m, n, k, before, monkeypatch):
+    """A step that fits with the sums of the kernels beside strips is not refused, whichever way its product is asked for."""
+    wanted, least = ops._scratch_floats(m, n, k, 0, False), before * m * n
+    assert wanted >= least and (wanted > least) == ((m, n, k) in [(33, 3072, 8192), (131, 3072, 8192), (96, 10240, 8192)])
+    bf16 = lambda *shape: torch.zeros(shape, dtype=torch.bfloat16)
+    a, w, x, normed, at = bf16(m, k), bf16(n, k), torch.zeros(m, n), bf16(m, n), torch.zeros(m, dtype=torch.int32)
+    cache, table, turns = bf16(2, 2, 8, 64, 64), torch.zeros(1, 2, dtype=torch.int32), torch.zeros(m, 32)
+    calls = [(ops.gemm_bf16, (a, w, x))]
+    if ops.gemm_bf16_onto_norm_takes(m, n, k):
+        calls.append((ops.gemm_bf16_onto_norm, (a, w, x, torch.zeros(n), 1e-6, normed)))
+    if n == 3072:
+        calls.append((ops.gemm_bf16_qkv_rope_store, (a, w, turns, turns, at, at, table, bf16(m, 32 * 64), cache, 32, 8, 64)))
+    for call, args in calls:
+        for room, given in ((wanted, wanted), (wanted - 1, least if wanted > least else None), (least, least)):
+            if given is None:
+                continue
+            with monkeypatch.context() as patch:
+                launched = _launches_with_room_for(room, patch)
+                call(*args)
+            (name, passed), = launched
+            assert given in passed and (wanted == given or wanted not in passed), name
+
+
 def test_products_of_few_rows_ask_for_nothing_by_kind(monkeypatch):
     for m, n, k in [(1, 3072, 2048), (17, 2048, 8192), (128, 16384, 2048), (128, 28672, 4096)]:
         assert m <= ops.FEW_ROWS and len({ops._scratch_floats(m, n, k, kind, counted) for kind in range(len(ops.PRODUCT_KINDS)) for counted in (False, True)}) == 1
