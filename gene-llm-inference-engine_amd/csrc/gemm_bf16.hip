@@ -17,9 +17,9 @@
 //           for narrow ones k is split over workgroups and the partial sums are added in a fixed order by a second kernel.
 //   skinny  the other shapes of up to 128 rows: weights stream from HBM straight into registers and are used
 //           once, activations go through LDS; v_mfma_f32_16x16x32_bf16.  Wide and narrow outputs likewise.
-//   slim    at most 16 rows of A (decode): a workgroup of 8 waves owns 16 (or 2 x 16) weight
-//           rows, its waves take interleaved blocks of k and add their sums through LDS in a
-//           fixed order, so one launch does the whole product and its epilogue.
+//   slim    at most 16 rows of A (decode): a workgroup of 8 waves owns 8 to 32 weight rows, its
+//           waves take interleaved steps of k and add their sums through LDS in a fixed order, so
+//           one launch does the whole product and its epilogue.  Strips of so few rows are its too.
 //
 // The "gated" epilogue serves SwiGLU: the weight is [gate; up] interleaved in groups of 16 rows
 // (16 gate rows, the 16 up rows of the same outputs, and so on), and the output column c of a
@@ -75,6 +75,11 @@ __device__ __forceinline__ float gate_fast_of(float g, float u, float limit) {
 }
 
 __device__ __forceinline__ uint4 load16(const bf16_t* p) { return *reinterpret_cast<const uint4*>(p); }
+__device__ __forceinline__ uint4 load16_once(const bf16_t* p) {              // of bytes that this launch reads no second time
+    typedef uint32_t gi_load4 __attribute__((ext_vector_type(4)));
+    const gi_load4 v = __builtin_nontemporal_load(reinterpret_cast<const gi_load4*>(p));
+    return uint4{v.x, v.y, v.z, v.w};
+}
 __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
 
 template <int EPI>
@@ -1239,12 +1244,6 @@ constexpr int KB = 2 * SK, X_STRIDE = KB + 8;         // k per block of the work
 // The kernel for at most 16 rows: a thread keeps 8 pieces while the products run (more would cost the kernel its second
 // workgroup per compute unit); 64 threads share a row where there are at most 8 rows, 32 otherwise.
 constexpr int SLIM_PIECES = 8;
-// Outputs of fewer than so many strips of 16 weight rows take strips of 8, twice the workgroups; with up to 8 rows of A, where a
-// strip of 8 leaves no lane idle (FOLD = 1 below), of fewer than twice as many (measured at N = 4096 to 6144: 1 to 2 % of the
-// decode step at 1 to 8 rows, and 7 % the other way at 12 and 16 rows); a product that adds onto rows and hands a norm on does
-// so up to 3 rows only (N = 4096, K = 4096 and 14336 at 8 rows: 18.5 us with strips of 16 against 20.5, the step of the 8B shape
-// 4.47 -> 4.3 ms; equal at 4 rows, 0.5 % the other way at 1 and 2).
-constexpr int SLIM_NARROW_STRIPS = 256;
 __host__ __device__ constexpr int slim_max_parts(int M) { return SLIM_PIECES * (M <= 8 ? 64 : 32); }
 // The kernels for 17 to 128 rows: the kernel that adds the partial sums onto x writes one piece per 1024 columns.
 constexpr int REDUCE_COLUMNS = 1024, REDUCE_MAX_PARTS = 8;
@@ -1833,71 +1832,100 @@ __global__ __launch_bounds__(256) void skinny_reduce_rope_store_kernel(const flo
 }
 
 // ------------------------------------------------------------------------------------------- slim
-// At most 16 rows of A.  Workgroup: 8 waves = STRIPS strips of ROWS weight rows x (8 / STRIPS)
-// slices of k; slice s takes the 128-wide blocks of k numbered s, s + slices, ...  Both operands go
-// from global memory straight into registers (the activations are few and stay in cache): for the
-// j-th product of a block, lane (r = lane%16, q = lane/16) holds k0 + 32j + 8q .. +8 of weight row r
-// and of activation row r, so the four lanes of a row read 64 contiguous bytes per load.  Loads run
-// two blocks ahead of the products.  The slices' sums meet in LDS and are added in slice order.
-// ROWS = 8 leaves half of each product idle and doubles the number of workgroups for narrow outputs.
+// At most 16 rows of A.  A workgroup of 8 waves owns `rows` weight rows in GROUPS groups of 8 (the last may be partly full); k goes in steps of 64, and wave w takes the steps w, w + 8, ...,
+// counted from a place of the workgroup's own.  Both operands go from global memory straight into registers (the activations are few and stay in cache):
+// lane l holds row l % 8 of a group, and of a step's 64 k the 8 from 8 (l / 16) + 32 (l / 8 % 2) on, for weights and activations alike, so the eight
+// lanes of a row read 128 contiguous bytes, a cache line, in one load.  To the matrix instruction that is 16 rows by 32 k on either side, rows 8 to 15 being
+// the same 8 rows' next 32 k: of the 16 x 16 result the two 8 x 8 blocks on the diagonal are the two halves' sums (the other two mix the halves and are dropped).
+// XT groups of 8 rows of A share the weights; GROUPS groups of weights share the activations.
+// Loads run DEPTH steps ahead of the products.  The waves' sums meet in LDS and are added in the order of the waves, the lower halves before the upper.
+//
+// What bounds it is weights on their way from memory, and behind them the activations, of which every workgroup reads all.  67 MB of weights in a bare read take
+// 12.8 us, 11.4 past the caches (each line is read once, by one load; with 16 rows' 64 bytes a load, as this kernel read them before, 14.1 and 14.8).  All workgroups
+// starting at the same k would ask the same memory channels first (rows lie a multiple of 4 KB apart): 12.6 us, 11.9 from a place of their own.  Microseconds, before and now, in chains
+// of products with weights of their own:
+//   rows                        1               8               16
+//   16,384 x 2,048 gated        15.8, 12.2      16.7, 12.4      16.8, 13.9
+//   28,672 x 4,096 gated        45.9, 37.0      46.6, 43.1      46.8, 47.9
+//   2,048 x 8,192 added         8.9, 7.6        11.0, 9.6       13.6, 13.4
+//   2,048 x 2,048 added         3.9, 3.8        4.6, 4.4        5.3, 5.4
+//   4,096 x 14,336 added        25.3, 20.1      26.1, 22.7      32.3, 28.4
+//   6,144 x 4,096 stored        11.3, 9.9       14.1, 10.3      17.1, 12.1
+//   128,256 x 2,048 stored      84.4, 77.7      98.7, 80.9      100.9, 93.1
+//   1,024 x 512 stored          2.2, 2.4        2.5, 2.6        2.7, 2.9
 // HAND: with the two halves of a norm handed from product to product (`NormIn`, `NormOut` above).
-// FOLD (ROWS = 8): the product's rows 8..15, idle otherwise on the weights' side, take the same 8 weight rows at the next 32 of k, and
-// the other operand 8 rows of A at both places likewise, so that a block is 256 wide, every lane loads weights, and a row's eight
-// lanes read 128 contiguous bytes; of the 16 x 16 result the two 8 x 8 blocks on the diagonal are the two halves' sums (the other
-// two mix the halves and are dropped).  FOLD = 1: at most 8 rows of A, one product per weight fragment; FOLD = 2: up to 16, in two
-// groups of 8 rows that share the weight fragment.
-// (A struct's numbers do not come in registers with the launch.  With the strides among those that do, as for the kernels of more rows, which are the
-// faster ones so, a decoded step of 3 rows takes 800 us instead of 796.)
-struct Strides {
-    long a, w, c;
-};
-template <int STRIPS, int ROWS, int EPI, bool HAND, int FOLD = 0>
-__global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ C,
-                                                            int M, int N, int K, Strides strides, NormIn norm_in, NormOut norm_out) {
-    const long lda = strides.a, ldw = strides.w, ldc = strides.c;
+// Strides come in pieces of 16 bytes, so that all that the first loads need is in the registers that are filled with the launch.
+template <int GROUPS, int EPI, bool HAND, int XT>
+__global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int lda8, int ldw8, int M, int N, int K, int rows, int turn,
+                                                                void* __restrict__ C, long ldc, NormIn norm_in, NormOut norm_out) {
+    constexpr bool GATED = is_gated(EPI);                              // the weights are 16 gates, their 16 ups, and so on
+    constexpr int DEPTH = GROUPS == 1 ? 4 : GROUPS == 2 ? 4 : 2;
+    static_assert(!GATED || GROUPS == 2 || GROUPS == 4, "as many groups of gates as of ups");
+    const int out = GATED ? 4 * GROUPS : rows;                         // columns of the output
     float act_p = 0.f, act_q = 0.f;
     if constexpr (EPI == EPI_XIELU) { act_p = norm_out.g[0]; act_q = norm_out.g[1]; }
-    static_assert(FOLD == 0 || ROWS == 8, "folding k into the idle rows needs strips of 8 weight rows");
-    constexpr int BLOCK = FOLD ? 2 * SK : SK, SPAN = BLOCK / 4;       // k of a block, and of one of its four products
-    constexpr int XT = FOLD == 2 ? 2 : 1;                             // groups of rows of A
-    constexpr int SLICES = 8 / STRIPS, STEP = SLICES * BLOCK, DEPTH = FOLD == 2 ? 2 : 3;
-    __shared__ float red[8][XT][64][4];
+    __shared__ float red[8][XT][GROUPS][2][8][8];                      // [wave][rows of A][weights][half of a step][row][weight row]
     __shared__ float row_scale[16];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int strip = wave % STRIPS, slice = wave / STRIPS;
-    const int r = FOLD ? lane & 7 : lane & 15, q = lane >> 4;
-    const int k_lane = 8 * q + (FOLD ? 32 * ((lane >> 3) & 1) : 0);   // where in a product's span of k this lane reads
-    const int n = (blockIdx.x * STRIPS + strip) * ROWS + (r < ROWS ? r : ROWS - 1);      // (lanes beyond a strip of 10 or 12 rows ask for its last row again)
-    // Every lane issues every load of a block (a row beyond the operand is clamped into it and lands in results that are never
-    // written; in a row's last, ragged block k is clamped too and the activations beyond K become zeros), and what a wave skips it
-    // skips as a whole: the compiler then counts the loads in flight, and a block's products wait for that block alone.
-    const bf16_t* wrow = W + (size_t)min(n, N - 1) * ldw + k_lane;
-    const bf16_t* xrow[XT];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 7, k_lane = 8 * (lane >> 4) + 32 * ((lane >> 3) & 1);
+    // A row beyond an operand is clamped into it and lands in results that are never written.  In a row's last, ragged step k is clamped too and the activations
+    // beyond K become zeros.
+    const int base = GATED ? (blockIdx.x / (4 / GROUPS)) * 32 + (blockIdx.x % (4 / GROUPS)) * 8 : blockIdx.x * rows;
+    const bf16_t* w_base[GROUPS];
+    // Where the lane's rows begin, in pieces of 16 bytes, or in bytes where the registers are scarce (one 32-bit distance from a scalar address; the host sees to strides that it holds).
+    constexpr int PIECE = GROUPS == 4 ? 1 : 16;
+    unsigned w_at[GROUPS], x_at[XT];
 #pragma unroll
-    for (int t = 0; t < XT; ++t) xrow[t] = A + (size_t)min(8 * t + r, M - 1) * lda + k_lane;
-    const int k_last = K - 8 - k_lane;                        // the last 16 bytes of a row, from `wrow` and `xrow`
-
-    floatx4 acc[XT];
+    for (int g = 0; g < GROUPS; ++g) {
+        w_base[g] = W + 8 * ((size_t)(base + (GATED ? 32 / GROUPS * g : 0)) * ldw8);
+        const int row = GATED ? r : min(8 * g + r, min(rows, N - base) - 1);
+        w_at[g] = ((unsigned)row * (unsigned)ldw8 + k_lane / 8) * (16 / PIECE);
+    }
 #pragma unroll
-    for (int t = 0; t < XT; ++t) acc[t] = floatx4{};
-    uint4 w_buf[DEPTH][4], x_buf[DEPTH][XT][4];
-    auto fetch = [&](int k0, uint4* w, uint4 (*x)[4]) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int at = min(k0 + SPAN * j, k_last);
-            w[j] = load16(wrow + at);
-#pragma unroll
-            for (int t = 0; t < XT; ++t) x[t][j] = load16(xrow[t] + at);
-        }
+    for (int t = 0; t < XT; ++t) x_at[t] = ((unsigned)min(8 * t + r, M - 1) * (unsigned)lda8 + k_lane / 8) * (16 / PIECE);
+    const int k_last = K - 8 - k_lane;                                 // the last 16 bytes of a row, from `w_row` and `x_row`
+    const int steps = (K + 63) / 64, first = blockIdx.x & turn;           // (`turn` + 1: the largest power of two of steps)
+    const int mine = (steps - wave + 7) / 8;                           // of this wave
+    auto place = [&](int i) {                                          // k where the wave's step i begins
+        const int step = wave + 8 * i + first;
+        return 64 * (step < steps ? step : step - steps);
     };
-    // What the epilogue adds onto (the thread's element of the 32-bit rows, and the next norm's gain for its column) is asked for
-    // before anything else: it comes from the memory-side cache while the weights stream, not behind them as one more round trip.
+    uint4 w_buf[DEPTH][GROUPS], x_buf[DEPTH][XT];
+    auto fetch = [&](int i, uint4 (&w)[GROUPS], uint4 (&x)[XT]) __attribute__((always_inline)) {
+        const unsigned at = (unsigned)((min(place(i), k_last) >> 3) * (16 / PIECE));         // (below 0 for a lane beyond a K under 64: the sums with it are not)
+        auto whereof = [](const bf16_t* p, unsigned pieces) { return (const bf16_t*)((const char*)p + (PIECE == 1 ? (size_t)pieces : (size_t)pieces * PIECE)); };
+#pragma unroll
+        for (int t = 0; t < XT; ++t) x[t] = load16(whereof(A, x_at[t] + at));
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) w[g] = load16_once(whereof(w_base[g], w_at[g] + at));
+    };
+    floatx4 acc[XT][GROUPS];
+#pragma unroll
+    for (int t = 0; t < XT; ++t)
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) acc[t][g] = floatx4{};
+    auto products = [&](int i, const uint4 (&w)[GROUPS], uint4 (&x)[XT]) __attribute__((always_inline)) {
+        const int at = place(i);
+        if (at + 64 > K) {                                             // the row's end lies in this step
+#pragma unroll
+            for (int t = 0; t < XT; ++t)
+                if (at + k_lane >= K) x[t] = uint4{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int t = 0; t < XT; ++t)
+#pragma unroll
+            for (int g = 0; g < GROUPS; ++g) acc[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(x[t]), as_bf16x8(w[g]), acc[t][g], 0, 0, 0);
+    };
+    // The thread's element of the output: row `m`, the workgroup's column `c`.  What the epilogue adds onto (the 32-bit rows, and the next norm's gain for
+    // the column) is asked for before anything else: it comes from the memory-side cache while the weights stream, not behind them as one more round trip.
+    constexpr int SHARE = GATED ? 4 * GROUPS : GROUPS == 3 ? 32 : 8 * GROUPS;       // threads to a row
+    const int m = tid / SHARE, c = tid % SHARE;
+    const int col = blockIdx.x * out + c;
     [[maybe_unused]] float old_value = 0.f, gain = 0.f;
     if constexpr (EPI == EPI_ADD_F32) {
-        const int e_m = (tid & 255) >> 4, e_col = (blockIdx.x * STRIPS + (tid >> 8) % STRIPS) * ROWS + (tid & 15);
-        old_value = ((const float*)C)[(size_t)min(e_m, M - 1) * ldc + min(e_col, N - 1)];
+        old_value = ((const float*)C)[(size_t)min(m, M - 1) * ldc + min(col, N - 1)];
         if constexpr (HAND) {
-            if (norm_out.scaled != nullptr) gain = norm_out.g[min(e_col, N - 1)];
+            if (norm_out.scaled != nullptr) gain = norm_out.g[min(col, N - 1)];
         }
     }
     // The pieces of the rows' sums of squares, 32 or 64 threads a row: asked for ahead of the first weights (loads come back in
@@ -1905,60 +1933,70 @@ __global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __
     float piece[HAND ? SLIM_PIECES : 1];
     [[maybe_unused]] float pieces_sum = 0.f;
     const int sharing = M <= 8 ? 64 : 32, piece_row = M <= 8 ? tid >> 6 : tid >> 5;
-    if constexpr (HAND) {
-        if (norm_in.squares != nullptr) {
-            const float* row_pieces = norm_in.squares + (size_t)min(piece_row, M - 1) * norm_in.parts;
+    auto ask_pieces = [&]() __attribute__((always_inline)) {
+        if constexpr (HAND) {
+            if (norm_in.squares != nullptr) {
+                const float* row_pieces = norm_in.squares + (size_t)min(piece_row, M - 1) * norm_in.parts;
 #pragma unroll
-            for (int i = 0; i < SLIM_PIECES; ++i) piece[i] = row_pieces[min((tid & (sharing - 1)) + sharing * i, norm_in.parts - 1)];
+                for (int i = 0; i < SLIM_PIECES; ++i) piece[i] = row_pieces[min((tid & (sharing - 1)) + sharing * i, norm_in.parts - 1)];
+            }
         }
-    }
-    const int k_first = slice * BLOCK;
-    const int n_blocks = k_first < K ? (K - k_first + STEP - 1) / STEP : 0;       // of this wave
-#pragma unroll
-    for (int d = 0; d < DEPTH - 1; ++d)
-        if (d < n_blocks) fetch(k_first + d * STEP, w_buf[d], x_buf[d]);
-    if constexpr (HAND) {
-        if (norm_in.squares != nullptr) {
-#pragma unroll
-            for (int i = 0; i < SLIM_PIECES; ++i)
-                if (piece_row < M && (tid & (sharing - 1)) + sharing * i < norm_in.parts) pieces_sum += piece[i];
-        }
-    }
-    // Block b of the wave lies in buffer b % DEPTH; its products are behind the request for block b + DEPTH - 1.
-    auto products = [&](int b, uint4* w, uint4 (*x)[4]) __attribute__((always_inline)) {
-        const int kb = k_first + b * STEP;
-        if (kb + BLOCK > K) {                                 // the row's end lies in this block
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (kb + SPAN * j + k_lane >= K) {
-#pragma unroll
-                    for (int t = 0; t < XT; ++t) x[t][j] = uint4{0, 0, 0, 0};
-                }
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int t = 0; t < XT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(x[t][j]), as_bf16x8(w[j]), acc[t], 0, 0, 0);
     };
-    int b = 0;
-    for (; b + 2 * DEPTH - 1 <= n_blocks; b += DEPTH) {      // trips in which nothing is skipped: exact waits
+    auto add_pieces = [&]() __attribute__((always_inline)) {
+        if constexpr (HAND) {
+            if (norm_in.squares != nullptr) {
 #pragma unroll
-        for (int d = 0; d < DEPTH; ++d) {
-            fetch(k_first + (b + d + DEPTH - 1) * STEP, w_buf[(d + DEPTH - 1) % DEPTH], x_buf[(d + DEPTH - 1) % DEPTH]);
-            products(b + d, w_buf[d], x_buf[d]);
+                for (int i = 0; i < SLIM_PIECES; ++i)
+                    if (piece_row < M && (tid & (sharing - 1)) + sharing * i < norm_in.parts) pieces_sum += piece[i];
+            }
         }
-    }
-    for (; b < n_blocks; b += DEPTH) {                        // the end of the wave's blocks
+    };
+    ask_pieces();
+    if (__builtin_expect(mine >= DEPTH, 1)) {                          // (the usual way lies straight ahead for the instruction fetch)
+        // Every load of a trip is issued and nothing is skipped: the compiler counts the loads in flight, and a step's products wait for that step alone.
 #pragma unroll
-        for (int d = 0; d < DEPTH; ++d) {
-            if (b + d + DEPTH - 1 < n_blocks) fetch(k_first + (b + d + DEPTH - 1) * STEP, w_buf[(d + DEPTH - 1) % DEPTH], x_buf[(d + DEPTH - 1) % DEPTH]);
-            if (b + d < n_blocks) products(b + d, w_buf[d], x_buf[d]);
+        for (int d = 0; d < DEPTH; ++d) fetch(d, w_buf[d], x_buf[d]);
+        add_pieces();
+        int i = 0;
+        for (; i + 2 * DEPTH <= mine; i += DEPTH) {
+#pragma unroll
+            for (int d = 0; d < DEPTH; ++d) {
+                products(i + d, w_buf[d], x_buf[d]);
+                fetch(i + DEPTH + d, w_buf[d], x_buf[d]);
+            }
         }
+        const int rest = mine - i - DEPTH;                             // steps not asked for yet, fewer than DEPTH
+        if (__builtin_expect(rest > 0, 0)) {
+#pragma unroll
+            for (int d = 0; d < DEPTH; ++d) {
+                products(i + d, w_buf[d], x_buf[d]);
+                if (d < rest) fetch(i + DEPTH + d, w_buf[d], x_buf[d]);
+            }
+#pragma unroll
+            for (int d = 0; d < DEPTH - 1; ++d)
+                if (d < rest) products(i + DEPTH + d, w_buf[d], x_buf[d]);
+        } else {
+#pragma unroll
+            for (int d = 0; d < DEPTH; ++d) products(i + d, w_buf[d], x_buf[d]);
+        }
+    } else {
+#pragma unroll
+        for (int d = 0; d < DEPTH - 1; ++d)
+            if (d < mine) fetch(d, w_buf[d], x_buf[d]);
+        add_pieces();
+#pragma unroll
+        for (int d = 0; d < DEPTH - 1; ++d)
+            if (d < mine) products(d, w_buf[d], x_buf[d]);
     }
+    // Element v of a lane's result: row 4 (lane / 16) + v, weight row lane % 16, each modulo 8; on the diagonal where both are below 8 or both are not.
+    if ((lane < 32) == ((lane & 8) == 0)) {
 #pragma unroll
-    for (int t = 0; t < XT; ++t)
+        for (int t = 0; t < XT; ++t)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) red[wave][t][lane][v] = acc[t][v];
+            for (int g = 0; g < GROUPS; ++g)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) red[wave][t][g][lane >> 5][4 * ((lane >> 4) & 1) + v][r] = acc[t][g][v];
+    }
     if constexpr (HAND) {
         if (norm_in.squares != nullptr) {
             float sum = pieces_sum;
@@ -1969,59 +2007,48 @@ __global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __
         }
     }
     __syncthreads();
-    // Element v of a lane's result: activation row 4*q + v, weight row r of the strip (folded: of the group's 8 rows, and the
-    // second half of k at row + 8, weight row + 8).
-    if (tid < 256 * (is_gated(EPI) ? 1 : STRIPS)) {
-        const int st = tid >> 8, e = tid & 255, m = e >> 4, c = e & 15;
-        const int group = FOLD ? m >> 3 : 0, m_in = FOLD ? m & 7 : m;
-        const int src_lane = c + 16 * (m_in >> 2), v = m_in & 3;
-        float r = 1.0f;
-        if constexpr (HAND) r = norm_in.squares != nullptr ? row_scale[m] : 1.0f;
+    auto sum_of = [&](int column) {
+        float sum = 0.f;
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int w = 0; w < 8; ++w) sum += red[w][XT == 1 ? 0 : m >> 3][column >> 3][half][m & 7][column & 7];
+        return sum;
+    };
+    if (tid < 8 * XT * SHARE) {
+        float scale = 1.0f;
+        if constexpr (HAND) scale = norm_in.squares != nullptr ? row_scale[m] : 1.0f;
         float square = 0.f;
-        if (m < M && c < ROWS && group < XT) {
-            if constexpr (is_gated(EPI)) {
-                float gate = 0.f, up = 0.f;
-#pragma unroll
-                for (int s = 0; s < SLICES; ++s) {
-                    gate += red[s * STRIPS + 0][0][src_lane][v];
-                    up += red[s * STRIPS + 1][0][src_lane][v];
-                }
-                if constexpr (HAND) { gate *= r; up *= r; }
-                ((bf16_t*)C)[(size_t)m * ldc + blockIdx.x * 16 + c] = f32_to_bf16(gate_of<EPI>(gate, up, norm_in.limit));
-            } else {
-                float sum = 0.f;
-#pragma unroll
-                for (int s = 0; s < SLICES; ++s) sum += red[s * STRIPS + st][group][src_lane][v];
-                if constexpr (FOLD != 0) {                      // the other half of k: row + 8, column + 8 of the product
-#pragma unroll
-                    for (int s = 0; s < SLICES; ++s) sum += red[s * STRIPS + st][group][src_lane + 40][v];
-                }
-                if constexpr (HAND) sum *= r;
-                const int col = (blockIdx.x * STRIPS + st) * ROWS + c;
-                if (col < N) {
-                    if constexpr (EPI == EPI_ADD_F32) {
-                        const float x = old_value + sum;
-                        ((float*)C)[(size_t)m * ldc + col] = x;
-                        if constexpr (HAND) {
-                            if (norm_out.scaled != nullptr) {
-                                norm_out.scaled[(size_t)m * norm_out.ld + col] = f32_to_bf16(gain * x);
-                                square = x * x;
-                            }
+        if (m < M && c < out) {
+            if constexpr (GATED) {
+                float gate = sum_of(c), up = sum_of(4 * GROUPS + c);
+                if constexpr (HAND) { gate *= scale; up *= scale; }
+                ((bf16_t*)C)[(size_t)m * ldc + col] = f32_to_bf16(gate_of<EPI>(gate, up, norm_in.limit));
+            } else if (col < N) {
+                float sum = sum_of(c);
+                if constexpr (HAND) sum *= scale;
+                if constexpr (EPI == EPI_ADD_F32) {
+                    const float x = old_value + sum;
+                    ((float*)C)[(size_t)m * ldc + col] = x;
+                    if constexpr (HAND) {
+                        if (norm_out.scaled != nullptr) {
+                            norm_out.scaled[(size_t)m * norm_out.ld + col] = f32_to_bf16(gain * x);
+                            square = x * x;
                         }
-                    } else if constexpr (EPI == EPI_XIELU) {
-                        if (col < norm_in.first) ((float*)C)[(size_t)m * ldc + col] = sum;
-                        else norm_out.scaled[(size_t)m * norm_out.ld + col - norm_in.first] = f32_to_bf16(xielu(sum, softplus_f32(act_p), 0.5f + softplus_f32(act_q)));
-                    } else {
-                        write_out<EPI>(C, (size_t)m * ldc + col, sum);
                     }
+                } else if constexpr (EPI == EPI_XIELU) {
+                    if (col < norm_in.first) ((float*)C)[(size_t)m * ldc + col] = sum;
+                    else norm_out.scaled[(size_t)m * norm_out.ld + col - norm_in.first] = f32_to_bf16(xielu(sum, softplus_f32(act_p), 0.5f + softplus_f32(act_q)));
+                } else {
+                    write_out<EPI>(C, (size_t)m * ldc + col, sum);
                 }
             }
         }
         if constexpr (HAND && EPI == EPI_ADD_F32) {
-            if (norm_out.scaled != nullptr) {                   // the 16 threads of a row: its columns of this workgroup
+            if (norm_out.scaled != nullptr) {                   // the threads of a row: its columns of this workgroup
 #pragma unroll
-                for (int off = 8; off > 0; off >>= 1) square += __shfl_xor(square, off, 64);
-                if (c == 0 && m < M) norm_out.squares[(size_t)m * (gridDim.x * STRIPS) + blockIdx.x * STRIPS + st] = square;
+                for (int off = SHARE / 2; off > 0; off >>= 1) square += __shfl_xor(square, off, 64);
+                if (c == 0 && m < M) norm_out.squares[(size_t)m * gridDim.x + blockIdx.x] = square;
             }
         }
     }
@@ -2379,26 +2406,15 @@ static int reduce_partials(const float* scratch, void* C, int epi, int M, int N,
     return 0;
 }
 
-// Up to 16 rows the slim kernel (no LDS staging, one launch) is the faster one, except for wide outputs with more than a few rows, where its per-workgroup reading of the activations
-// costs more than staging them: from 5 rows on for a vocabulary (128,256 x 2,048: 92.4 us and 95.9 in strips at 4 rows, 101.6 and 96.4 at 6), else from the row that
-// slim_until_row or, where strips are not the other ones, streamed_from_row says.
-// Where the skinny kernel is the other one (K no multiple of 64, measured at the time at K = 2,048 to 4,096) the longer the rows and the more strips, the sooner, between 3 and 12.
+// Up to 16 rows the slim kernel (no LDS staging, one launch) is the faster one, except where its per-workgroup reading of the activations costs more than staging them.
+// Where the weight-streaming kernel is the other one (K no multiple of 64) the longer the rows and the more strips, the sooner, between 3 and 12: 16,384 x 2,056 gated takes 16.6 us
+// and 17.7 at 8 rows, 17.1 and 17.8 at 12, 18.1 and 17.9 at 16; 32,000 x 1,000 stored 14.9, 15.3; 15.9, 15.6; 16.7, 15.9.
 static int streamed_from_row(int strips, int K) {
     const double fitted = 12.0 * (2048.0 / K) * (256.0 / strips);
     return fitted < 3 ? 3 : fitted > 12 ? 12 : (int)(fitted + 0.5);
 }
-// Beside the strips' kernel (14 widths from 12,288 to 49,152 columns, 19 k from 64 to 14,336, 1 to 16 rows, slim and strips each for all of them, stored, gated and gated with a norm: the choice is 1.3 %
-// slower than the faster of the two on average, 15 % at worst).  What decides it: gated columns leave a strip more cheaply than 32-bit ones; a round of workgroups that strips of 64 columns fill badly is
-// slim's, whose strips are narrower, in the second round, and the strips' in the first, where their workgroups have a unit to themselves; and rows of weights a multiple of 4,096 bytes apart
-// cost the strips, which ask for 64 of them at once, more than slim (whole).  Of 4,020 other products (20 widths up to 64,000 columns, 28 k) the choice is 0.3 % slower than the faster of the two on average
-// for stored columns and 1.0 % for gated ones; a third round and more that is badly filled is slim's for some rows longer too.  Microseconds, slim and strips:
-//   gated                        1 row         8 rows        16 rows            stored                       1 row         8 rows        16 rows
-//   12,288 x 2,048               14.2, 13.1    15.7, 13.3    18.2, 13.4         12,288 x 2,048               11.1, 13.0    12.9, 13.1    15.9, 13.1
-//   16,384 x 2,048 (a norm)      16.7, 17.5    17.2, 17.9    19.6, 18.1         16,384 x 2,048               13.5, 16.6    16.1, 16.7    20.1, 16.7
-//   28,672 x 4,096               48.2, 44.3    54.0, 45.1    63.4, 45.4         18,432 x 8,192               58.8, 79.0    64.7, 79.8    80.4, 80.3
-//   12,288 x 256                 3.5, 4.1      3.9, 4.6      4.2, 4.6           12,288 x 3,072               14.2, 15.4    18.2, 15.8    22.7, 16.2
-//   33,280 x 3,072               43.5, 46.4    50.9, 46.1    60.7, 46.5         33,280 x 3,072               38.0, 46.5    48.6, 46.2    59.7, 46.9 (4 rows 41.0, 45.7, 6 44.4, 46.0)
-// Decoding 8 requests of the 1B shape, whose gated product has 16,384 x 2,048, takes 900 us with either; 9 take 957 with slim and 949 with strips.
+// Where K is a multiple of 64, from which row on a product counts as strips of columns, which take no norm's pieces beyond a reader's and hand none on: lines drawn between the slim
+// kernel as it was and the strips' ring in LDS.  Since it reads whole cache lines the slim kernel makes most strips of up to 16 rows too (`strips_in_registers` below).
 static int slim_until_row(int strips, int K, bool gated) {
     const int units = gi_compute_units();
     const bool three_quarters = strips * 4 <= units * 3, narrow = strips * 5 <= units * 4, second = strips > units && strips * 2 <= units * 3, barely = strips * 4 <= units * 5, whole = K % 2048 == 0;
@@ -2426,32 +2442,42 @@ static bool takes_slim(int M, int N, int K, bool gated, bool xielu = false) {
 }
 
 // Workgroups of the slim kernel for an output of N columns that is not gated: the pieces a row's sum of squares comes in.
-// (A product that adds onto rows may hand a norm on, with one piece of the rows' sums of squares per workgroup: it takes strips
-// of 8 only where the reader takes that many pieces.  N = 3072 at 9 to 16 rows: 384 strips of 8 would be more than the 256 pieces
-// a reader of so many rows takes, and the norm's own kernel would run twice a layer; 192 strips of 16 hand it on.)
-static bool slim_wide_strips(int M, int N, int epi) {
-    const bool doubled = M <= 8 && (epi != EPI_ADD_F32 || M <= 3);
-    const bool few = (N + 15) / 16 <= (doubled ? 2 * SLIM_NARROW_STRIPS : SLIM_NARROW_STRIPS) - 1;
-    return !(few && (epi != EPI_ADD_F32 || (N + 7) / 8 <= slim_max_parts(M)));
-}
-// Weight rows per workgroup of the slim kernel for an output that is not gated: 16 or 8 by the rules above, unless that many
-// workgroups fill the compute units unevenly (384 strips of 8 or 192 of 16 on 256 units: a quarter of the chip waits for the
-// rest) and strips of 12 or 10 rows fill them evenly (3,072 columns: 256 strips of 12) with no more pieces than a reader takes.
-// A product's 16 weight rows beyond such a strip repeat its last row (the same cache line, no further traffic) and their results
-// are dropped.  Measured on the decode step: the 1B shape (q/k/v of 3,072 columns) 1 to 2 % faster at 1 to 16 rows, the 3B shape
-// (rows of 3,072: 11.7 against 12.9 us a product at 8 rows) 3 to 5 %.  640 strips of 8 (5,120 columns, five sixths even) are
-// faster than 512 of 10 (11.9 against 12.9 us): the even strips are taken where the usual ones are less than four fifths even.
+// Weight rows per workgroup of the slim kernel.  A round of workgroups, one per compute unit, takes as long as its weights, an eighth to a third of a weight row more for
+// every row of A (all of which every workgroup reads) and two rows' time to begin and end; a round that is not full costs four fifths of one at least.  So an output that
+// 256 workgroups of at most 32 rows cover has one round, and wider ones as few as fill it well.  28 outputs of 640 to 128,256 columns, k of 768 to 14,336, 1 to 16 rows, seven to
+// eight heights each: the choice is 0.3 % slower than the fastest on average, 9.6 % at worst (10,240 x 2,048 at one row).  Microseconds by weight rows a workgroup:
+//                                      8       12      16      20      24      32
+//   6,144 x 4,096 at 1 row             10.05   10.53   11.21   13.65   9.87    11.47
+//   6,144 x 4,096 at 8 rows            13.09   12.33   13.26   15.56   10.26   12.33
+//   2,048 x 8,192 at 8 rows            9.78    11.93   13.13   15.59   16.82
+//   128,256 x 2,048 at 8 rows          119.1   107.0   90.8    91.0    84.7    80.9
+//   28,672 x 4,096 gated, 1 and 12                     37.0, 48.7              42.1, 45.7
+// Gated columns come in pairs of 16 weight rows, half of which or all a workgroup takes; what adds onto rows stays below 32, whose registers it lacks, and where it hands a norm on
+// makes no more pieces of a row's sum of squares than a reader takes.
 static int slim_strip_rows(int M, int N, int epi) {
-    const int usual = slim_wide_strips(M, N, epi) ? 16 : 8, units = gi_compute_units();
-    auto evenness = [&](int rows) {
-        const int groups = (N + rows - 1) / rows;
-        return (double)groups / ((groups + units - 1) / units * units);
+    const int units = gi_compute_units();
+    auto cost = [&](int rows) {
+        const int groups = (N + rows - 1) / rows, whole = groups / units, rest = groups % units;
+        const double share = rest == 0 ? 0.0 : whole == 0 ? 1.0 : rest * 5 < units * 4 ? 0.8 : (double)rest / units;
+        return (whole + share) * (rows + (M <= 8 ? 0.2 : 0.6) * M + 2);
     };
-    if (evenness(usual) >= 0.8) return usual;
-    for (int rows : {12, 10})
-        if (evenness(rows) >= 0.95 && (epi != EPI_ADD_F32 || (N + rows - 1) / rows <= slim_max_parts(M))) return rows;
-    return usual;
+    if (is_gated(epi)) return cost(16) < cost(32) ? 16 : 32;
+    int best = 8;
+    for (int rows = 9; rows <= (epi == EPI_ADD_F32 ? 24 : 32); ++rows)
+        if (cost(rows) < cost(best) || (epi == EPI_ADD_F32 && (N + best - 1) / best > slim_max_parts(M))) best = rows;
+    return best;
 }
+// Strips of a few rows of A, which are otherwise made through a ring in LDS, in the slim kernel's workgroups of 16 or 32 weight rows: faster to 14 rows for 18
+// sizes measured, and at 16 by 9 % on average and at most 3 % slower; but stored columns of a short k, whose end weighs most there, from 9 rows on.
+// Microseconds, strips through LDS and in registers:
+//   rows                     4              8              12             16
+//   28,672 x 4,096 gated     46.4, 40.9     46.4, 43.1     46.7, 45.5     46.7, 47.9
+//   24,576 x 2,048 gated     23.2, 17.1     23.6, 17.4     24.2, 18.5     24.4, 19.5
+//   128,256 x 2,048 stored   94.2, 78.3     98.7, 80.9     99.9, 88.6     100.9, 93.1
+//   16,384 x 8,192 stored    66.2, 44.4     65.5, 44.5     65.1, 46.9     65.8, 49.7
+//   65,536 x 512 stored      15.1, 14.9     15.2, 15.2     15.3, 18.0     15.5, 18.3
+static bool strips_in_registers(int M, int K, int epi) { return M <= 8 || (M <= 16 && (is_gated(epi) || K > 512)); }
+
 static int slim_parts(int M, int N) {
     const int rows = slim_strip_rows(M, N, EPI_ADD_F32);
     return (N + rows - 1) / rows;
@@ -2460,39 +2486,41 @@ static int slim_parts(int M, int N) {
 static int launch_slim(const void* A, const void* W, void* C, int epi, int M, int N, int K, long lda, long ldw, long ldc, NormIn norm_in,
                        NormOut norm_out, hipStream_t stream) {
     const bool hand = norm_in.squares != nullptr || (norm_out.scaled != nullptr && epi != EPI_XIELU);
-#define SLIM(STRIPS_, ROWS_, EPI_)                                                                                                                     \
+    int rows = slim_strip_rows(M, N, epi);
+    // The kernel reckons distances between rows in 32 bits: in bytes for 32 weight rows, in pieces of 16 bytes for fewer.
+    if (rows > 24 && (31 * ldw * 2 >= 1l << 32 || 15 * lda * 2 >= 1l << 32)) rows = is_gated(epi) ? 16 : 24;
+    GI_REQUIRE((N == 1 || 31 * (ldw / 8) < 1l << 32) && (M == 1 || 15 * (lda / 8) < 1l << 32), "gemm_bf16: rows %ld and %ld elements apart are not taken", lda, ldw);
+    const dim3 grid((N + rows - 1) / rows);
+    int turn = 1;
+    while (2 * turn <= (K + 63) / 64) turn *= 2;
+    --turn;
+#define SLIM_XT(GROUPS_, EPI_, XT_)                                                                                                                    \
     do {                                                                                                                                               \
-        if (hand) gemm_bf16_slim_kernel<STRIPS_, ROWS_, EPI_, true><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, Strides{lda, ldw, ldc}, norm_in, norm_out); \
-        else gemm_bf16_slim_kernel<STRIPS_, ROWS_, EPI_, false><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, Strides{lda, ldw, ldc}, norm_in, norm_out);     \
+        if (hand) gemm_bf16_slim_kernel<GROUPS_, EPI_, true, XT_><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, (int)(lda / 8), (int)(ldw / 8), M, N, K, rows, turn, C, ldc, norm_in, norm_out); \
+        else gemm_bf16_slim_kernel<GROUPS_, EPI_, false, XT_><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, (int)(lda / 8), (int)(ldw / 8), M, N, K, rows, turn, C, ldc, norm_in, norm_out);     \
     } while (0)
-    if (is_gated(epi)) {
-        dim3 grid(N / 32);
-        if (epi == EPI_GATED_BF16) SLIM(2, 16, EPI_GATED_BF16); else if (epi == EPI_GATED_GELU_BF16) SLIM(2, 16, EPI_GATED_GELU_BF16); else SLIM(2, 16, EPI_GATED_CLAMP_BF16);
-    } else if (slim_strip_rows(M, N, epi) == 16) {
-        dim3 grid((N + 15) / 16);
-        if (epi == EPI_STORE_F32) SLIM(1, 16, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM(1, 16, EPI_ADD_F32); else if (epi == EPI_XIELU) SLIM(1, 16, EPI_XIELU); else SLIM(1, 16, EPI_STORE_BF16);
-    } else if (slim_strip_rows(M, N, epi) == 12) {     // (the last 4 of a product's 16 weight rows are the strip's last row again; their results are dropped)
-        dim3 grid((N + 11) / 12);
-        if (epi == EPI_STORE_F32) SLIM(1, 12, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM(1, 12, EPI_ADD_F32); else if (epi == EPI_XIELU) SLIM(1, 12, EPI_XIELU); else SLIM(1, 12, EPI_STORE_BF16);
-    } else if (slim_strip_rows(M, N, epi) == 10) {
-        dim3 grid((N + 9) / 10);
-        if (epi == EPI_STORE_F32) SLIM(1, 10, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM(1, 10, EPI_ADD_F32); else if (epi == EPI_XIELU) SLIM(1, 10, EPI_XIELU); else SLIM(1, 10, EPI_STORE_BF16);
-    } else {                                   // a narrow output: strips of 8 rows, twice the workgroups
-        dim3 grid((N + 7) / 8);
-#define SLIM_FOLD(EPI_, FOLD_)                                                                                                                         \
+#define SLIM(GROUPS_, EPI_) do { if (M <= 8) SLIM_XT(GROUPS_, EPI_, 1); else SLIM_XT(GROUPS_, EPI_, 2); } while (0)
+#define SLIM_EPI(GROUPS_)                                                                                                                              \
     do {                                                                                                                                               \
-        if (hand) gemm_bf16_slim_kernel<1, 8, EPI_, true, FOLD_><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, Strides{lda, ldw, ldc}, norm_in, norm_out); \
-        else gemm_bf16_slim_kernel<1, 8, EPI_, false, FOLD_><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, Strides{lda, ldw, ldc}, norm_in, norm_out);     \
+        if (epi == EPI_STORE_F32) SLIM(GROUPS_, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM(GROUPS_, EPI_ADD_F32);                               \
+        else if (epi == EPI_XIELU) SLIM(GROUPS_, EPI_XIELU); else SLIM(GROUPS_, EPI_STORE_BF16);                                                       \
     } while (0)
-        // the idle halves of the products take a further 32 of k: for up to 8 rows of A on both sides, for more on the weights' side
-        if (M <= 8) {
-            if (epi == EPI_STORE_F32) SLIM_FOLD(EPI_STORE_F32, 1); else if (epi == EPI_ADD_F32) SLIM_FOLD(EPI_ADD_F32, 1); else if (epi == EPI_XIELU) SLIM_FOLD(EPI_XIELU, 1); else SLIM_FOLD(EPI_STORE_BF16, 1);
-        } else {
-            if (epi == EPI_STORE_F32) SLIM_FOLD(EPI_STORE_F32, 2); else if (epi == EPI_ADD_F32) SLIM_FOLD(EPI_ADD_F32, 2); else if (epi == EPI_XIELU) SLIM_FOLD(EPI_XIELU, 2); else SLIM_FOLD(EPI_STORE_BF16, 2);
-        }
-#undef SLIM_FOLD
+#define SLIM_GATED(GROUPS_)                                                                                                                            \
+    do {                                                                                                                                               \
+        if (epi == EPI_GATED_BF16) SLIM(GROUPS_, EPI_GATED_BF16); else if (epi == EPI_GATED_GELU_BF16) SLIM(GROUPS_, EPI_GATED_GELU_BF16);             \
+        else SLIM(GROUPS_, EPI_GATED_CLAMP_BF16);                                                                                                      \
+    } while (0)
+    if (is_gated(epi)) { if (rows == 32) SLIM_GATED(4); else SLIM_GATED(2); }
+    else if (rows > 24) {
+        if (epi == EPI_STORE_F32) SLIM(4, EPI_STORE_F32); else if (epi == EPI_XIELU) SLIM(4, EPI_XIELU); else SLIM(4, EPI_STORE_BF16);
     }
+    else if (rows > 16) SLIM_EPI(3);
+    else if (rows > 8) SLIM_EPI(2);
+    else SLIM_EPI(1);
+#undef SLIM_GATED
+#undef SLIM_EPI
 #undef SLIM
+#undef SLIM_XT
     GI_CHECK_LAUNCH("gemm_bf16 (slim)");
     return 0;
 }
@@ -2605,7 +2633,11 @@ static int launch_skinny(const void* A, const void* W, void* C, int epi, int M, 
                norm_in.parts, consumer_max_parts(M), M);
     if (splits == 0) {                             // a wide output: every workgroup sees all of k and finishes its columns
         GI_REQUIRE(norm_out.scaled == nullptr && rope == nullptr, "gemm_bf16: a product this wide does not hand a norm on, or its rows to the cache");
-        if (ends_in_strips(M, N, K) && strip_strides(lda, ldw)) return launch_strips(A, W, C, epi, M, N, K, lda, ldw, ldc, nullptr, StripCut{1, 0, 0}, norm_in, stream);
+        if (ends_in_strips(M, N, K) && strip_strides(lda, ldw)) {
+            if (strips_in_registers(M, K, epi) && (norm_in.squares == nullptr || norm_in.parts <= slim_max_parts(M)))
+                return launch_slim(A, W, C, epi, M, N, K, lda, ldw, ldc, norm_in, NO_NORM_OUT, stream);
+            return launch_strips(A, W, C, epi, M, N, K, lda, ldw, ldc, nullptr, StripCut{1, 0, 0}, norm_in, stream);
+        }
         const int k_per_split = K;
         dim3 grid((N + 63) / 64, 1);
         if (epi == EPI_GATED_BF16) SKINNY_MT(EPI_GATED_BF16, false); else if (epi == EPI_GATED_GELU_BF16) SKINNY_MT(EPI_GATED_GELU_BF16, false); else if (epi == EPI_GATED_CLAMP_BF16) SKINNY_MT(EPI_GATED_CLAMP_BF16, false); else if (epi == EPI_STORE_F32) SKINNY_MT(EPI_STORE_F32, false);

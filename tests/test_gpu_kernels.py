@@ -386,6 +386,28 @@ def test_products_that_strips_do_not_make_go_the_way_before(m, n, k, short_of, m
     assert not torch.equal(out[:m, :n], strips)                            # (the sums of other shares)
 
 
+@pytest.mark.parametrize("n", [5, 2300, 4600, 7000])                      # weight rows a workgroup: 8, 9, 18 and 28, the last workgroup's fewer
+@pytest.mark.parametrize("m,k", [(1, 8), (8, 72), (9, 520), (16, 1032), (3, 1536), (8, 2056), (16, 2560), (7, 3080), (12, 4160), (1, 5120)])
+def test_gemm_bf16_few_rows_at_every_height(m, n, k):
+    """Workgroups of 8 to 32 weight rows with partly full groups, waves of none to ten steps of 64 k, the last one ragged; operands and outputs within wider ones.  The 32-bit sums' bound: 2e-6."""
+    wide_a, wide_w = randn(m, k + 24, dtype=torch.bfloat16, seed=1), randn(n, k + 8, dtype=torch.bfloat16, seed=2, scale=0.1)
+    a, w, x0 = wide_a[:, 8:8 + k], wide_w[:, :k], randn(m, n, seed=3)
+    want = a.double() @ w.double().T
+    out, x, low = torch.full((m + 1, n + 3), 3.0, device=DEV), x0.clone(), torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    ops().gemm_bf16(a, w, out[:m, :n])
+    ops().gemm_bf16(a, w, x, accumulate=True)
+    ops().gemm_bf16(a, w, low)
+    assert rel(out[:m, :n], want) < 2e-6 and rel(x, x0.double() + want) < 2e-6 and rel(low, want) < 4.1e-3
+    assert bool((out[m:] == 3.0).all()) and bool((out[:, n:] == 3.0).all())
+    cols = n // 32 * 16                                                    # gated: pairs of 16 weight rows, by halves of them or whole ones
+    if cols:
+        gate, up = want[:, :2 * cols].reshape(m, cols // 16, 2, 16).unbind(2)
+        gated = torch.full((m + 1, cols + 2), 3.0, dtype=torch.bfloat16, device=DEV)
+        ops().gemm_bf16(a, w[:2 * cols], gated[:m, :cols], gated=True)
+        assert rel(gated[:m, :cols], (torch.nn.functional.silu(gate) * up).reshape(m, cols)) < 4.1e-3
+        assert bool((gated[m:] == 3.0).all()) and bool((gated[:, cols:] == 3.0).all())
+
+
 @pytest.mark.parametrize("m,parts", [(1, 512), (8, 300), (9, 256), (16, 3), (17, 256), (32, 2), (33, 8), (64, 1), (128, 5)])
 def test_gemm_bf16_strips_finish_a_norm(m, parts):
     n, k = 28672, 3072                                                     # (strips from one row on)
