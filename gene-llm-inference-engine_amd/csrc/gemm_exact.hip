@@ -319,9 +319,11 @@ __global__ __launch_bounds__(256) void gemm_exact_add_parts_kernel(const float* 
 // range of k (strips of 16 rows, 8 waves) or two (strips of 8 rows and at most 8 rows of activations, 4 waves: the idle half of
 // every matrix instruction takes the second range, weight rows 8..15 and activation rows 8..15 of the instruction standing for the
 // same rows at the other range's k; twice the workgroups for the same waves, which is what narrow outputs lack).  The operands go
-// from memory straight into the matrix instructions' registers, AHEAD blocks of 16 k asked for at once; the ranges' sums
-// meet in LDS and are added there.  At 3 rows: 16,384 x 2,048 in 27 us (5.0 TB/s), 2,048 x 8,192 in 16 (4.1), 128,256 x 2,048 in 181
-// (5.8); one lane per column, each walking all of k alone, took 290 us, 1.15 ms and 400 us.
+// from memory straight into the matrix instructions' registers: 32-bit weights a whole cache line of 8 rows a load, past the caches, four pairs of blocks of 16 k
+// in flight behind the products (with 16 rows' 64 bytes a load, eight blocks asked for at once and all awaited: the figures before); bfloat16 weights AHEAD blocks at once.
+// The ranges' sums meet in LDS and are added there.  At 3 rows, before and now, in chains of products with weights of their own: 16,384 x 2,048 gated 28.4, 26.6 us (5.0 TB/s), 2,048 x 8,192
+// added 17.4, 15.4 (4.35; a bare read of these places 13.0), 2,048 x 2,048 added 7.4, 6.2, 3,072 x 2,048 8.8, 8.4, 128,256 x 2,048 184, 178 (5.9); what is added onto is
+// asked for first (a microsecond of the added ones); one lane per column, each walking all of k alone, took 290 us, 1.15 ms and 400 us.
 constexpr int FEW_ROWS = 16, AHEAD = 8;
 
 // GATED: W is [gate; up], a strip of 16 is 8 gates and the 8 ups of the same columns, and act(gate) * up goes out in the bits of the gate's own kernel, which
@@ -342,6 +344,18 @@ struct Turn {
     long page_stride;
     int page_size, n_heads, n_kv, hd;
 };
+
+__device__ __forceinline__ f32x4 load4_once(const float* p) { return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p)); }      // of bytes that this launch reads no second time
+// Lane l of either load holds row l % 8 and the 4 k from 4 (l / 16) + 16 (l / 8 % 2) on (`low`: rows 0 to 7, `high`: 8 to 15); afterwards row l % 16 and the 4 k from 4 (l / 16)
+// on (`low`) and those 16 further (`high`): within 16 lanes the upper half of `low` and the lower half of `high` change places.
+__device__ __forceinline__ void rows_of_halves(f32x4& low, f32x4& high) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int a = __float_as_int(low[i]), b = __float_as_int(high[i]);
+        low[i] = __int_as_float(__builtin_amdgcn_update_dpp(a, b, 0x128, 0xf, 0xc, false));         // (rotated by 8 within 16 lanes; lanes 8 to 15 take it)
+        high[i] = __int_as_float(__builtin_amdgcn_update_dpp(b, a, 0x128, 0xf, 0x3, false));        // (lanes 0 to 7)
+    }
+}
 
 template <int STRIP, typename TA, typename TW, typename TC, bool ACCUMULATE, typename End>
 __global__ __launch_bounds__(STRIP == 16 ? 512 : 256) void gemm_exact_few_rows_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C,
@@ -379,20 +393,86 @@ __global__ __launch_bounds__(STRIP == 16 ? 512 : 256) void gemm_exact_few_rows_k
     }
     const TW* w_row = W + (size_t)first_row * ldw;
     const TA* a_row = A + (size_t)min(row, M - 1) * lda;
+    // What the sums are added onto is asked for first: behind the weights it would be one more round trip.
+    [[maybe_unused]] f32x4 old;
+    if constexpr (ACCUMULATE) {
+        const int e = threadIdx.x % (STRIP * STRIP / 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) old[i] = load_f32(C, (size_t)min(e % STRIP, M - 1) * ldc + min(n0 + 4 * (e / STRIP) + i, N - 1));
+    }
     const int blocks = max(0, min(L, K - q_first * L) + 15) / 16;             // until both of the wave's ranges are through
-    const int whole = max(0, min(L, K - q_last * L)) / 16 / AHEAD * AHEAD;    // ... of them with nothing to guard, in groups
+    const int guarded = max(0, min(L, K - q_last * L)) / 16;                  // ... of them with nothing to guard
     f32x4 acc[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
-    for (int b = 0; b < whole; b += AHEAD) {
-        f32x4 w[AHEAD], a[AHEAD];
+    int whole;
+    if constexpr (sizeof(TW) == 4) {
+        // 32-bit weights: a load brings 32 k of 8 rows, a whole cache line of each, past the caches; two of them hold two blocks of 16 rows' (or 8 rows' in both
+        // ranges) operands, whose halves then change places.  DEPTH such pairs are in flight.
+        constexpr int DEPTH = 4;
+        const int w_k = 4 * (g + 4 * (r >> 3)), low_row = __shfl(first_row, r & 7, 64), high_row = STRIP == 16 ? __shfl(first_row, 8 + (r & 7), 64) : low_row;
+        const float *w_low = W + (size_t)low_row * ldw + q_first * L + w_k, *w_high = W + (size_t)high_row * ldw + q_last * L + w_k;
+        const int pairs = guarded / 2;
+        whole = 2 * pairs;
+        f32x4 w[DEPTH][2], a[DEPTH][2];
+        auto fetch = [&](int i, int d) __attribute__((always_inline)) {
+            w[d][0] = load4_once(w_low + 32 * i);
+            w[d][1] = load4_once(w_high + 32 * i);
+            a[d][0] = load4(a_row + base + 32 * i);
+            a[d][1] = load4(a_row + base + 32 * i + 16);
+        };
+        auto products = [&](int d) __attribute__((always_inline)) {
+            rows_of_halves(w[d][0], w[d][1]);
 #pragma unroll
-        for (int i = 0; i < AHEAD; ++i) w[i] = load4(w_row + base + (b + i) * 16);
+            for (int half = 0; half < 2; ++half)
 #pragma unroll
-        for (int i = 0; i < AHEAD; ++i) a[i] = load4(a_row + base + (b + i) * 16);
-        __builtin_amdgcn_sched_barrier(0);                     // all of them in flight before the first product
+                for (int kk = 0; kk < 4; ++kk) acc[0] = mfma(w[d][half][kk], a[d][half][kk], acc[0]);
+        };
+        if (__builtin_expect(pairs >= DEPTH, 1)) {                            // nothing is skipped in a trip: a pair's products wait for that pair alone
 #pragma unroll
-        for (int i = 0; i < AHEAD; ++i)
+            for (int d = 0; d < DEPTH; ++d) fetch(d, d);
+            int i = 0;
+            for (; i + 2 * DEPTH <= pairs; i += DEPTH) {
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk) acc[0] = mfma(w[i][kk], a[i][kk], acc[0]);
+                for (int d = 0; d < DEPTH; ++d) {
+                    products(d);
+                    fetch(i + DEPTH + d, d);
+                }
+            }
+            const int rest = pairs - i - DEPTH;                               // not asked for yet, fewer than DEPTH
+            if (__builtin_expect(rest > 0, 0)) {
+#pragma unroll
+                for (int d = 0; d < DEPTH; ++d) {
+                    products(d);
+                    if (d < rest) fetch(i + DEPTH + d, d);
+                }
+#pragma unroll
+                for (int d = 0; d < DEPTH - 1; ++d)
+                    if (d < rest) products(d);
+            } else {
+#pragma unroll
+                for (int d = 0; d < DEPTH; ++d) products(d);
+            }
+        } else {
+#pragma unroll
+            for (int d = 0; d < DEPTH - 1; ++d)
+                if (d < pairs) fetch(d, d);
+#pragma unroll
+            for (int d = 0; d < DEPTH - 1; ++d)
+                if (d < pairs) products(d);
+        }
+    } else {
+        whole = guarded / AHEAD * AHEAD;                                      // in groups
+        for (int b = 0; b < whole; b += AHEAD) {
+            f32x4 w[AHEAD], a[AHEAD];
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i) w[i] = load4(w_row + base + (b + i) * 16);
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i) a[i] = load4(a_row + base + (b + i) * 16);
+            __builtin_amdgcn_sched_barrier(0);                     // all of them in flight before the first product
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i)
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk) acc[0] = mfma(w[i][kk], a[i][kk], acc[0]);
+        }
     }
     for (int b = whole; b < blocks; ++b) {
         const int k = base + b * 16, at = min(k, K - 4);
@@ -448,8 +528,11 @@ __global__ __launch_bounds__(STRIP == 16 ? 512 : 256) void gemm_exact_few_rows_k
         for (int i = 0; i < 4; ++i) values[(size_t)i * end.page_size] = sum[i];
     } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (n + i < N) put<TC, ACCUMULATE>(C, (size_t)m * ldc + n + i, sum[i]);
+        for (int i = 0; i < 4; ++i) {
+            if (n + i >= N) continue;
+            if constexpr (ACCUMULATE) store_f32(C, (size_t)m * ldc + n + i, old[i] + sum[i]);
+            else store_f32(C, (size_t)m * ldc + n + i, sum[i]);
+        }
     }
 }
 

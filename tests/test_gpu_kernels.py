@@ -58,6 +58,19 @@ def test_gemm_exact_rows_alone_have_the_same_bits(w_dtype, k):
         assert torch.equal(few, wide[:rows])                                # adding onto what is there, the same in both kernels
 
 
+@pytest.mark.parametrize("k", [4, 36, 260, 1056, 2052, 2820, 4100])            # a range of k in 32-bit: none to sixteen whole lines of 32 k, four in flight, and what is left
+@pytest.mark.parametrize("m,n", [(1, 5), (8, 520), (9, 130), (3, 8200)])       # strips of 8 and of 16 weight rows, the last ones partly beyond the output
+def test_gemm_exact_few_rows_line_by_line(m, n, k):
+    """In the bits of the kernel with tiles, which serves more rows, stored and added, and near the 64-bit product (the bound of the tests above)."""
+    a, w, x0 = randn(40, k, seed=5), randn(n, k + 4, seed=6)[:, :k], randn(m, n + 2, seed=7)
+    tiles, few, x = torch.empty(40, n, device=DEV), torch.empty(m, n, device=DEV), x0.clone()
+    ops().gemm_exact(a, w, tiles)
+    ops().gemm_exact(a[:m], w, few)
+    ops().gemm_exact(a[:m], w, x[:, :n], accumulate=True)
+    assert torch.equal(few, tiles[:m]) and rel(few, a[:m].double() @ w.double().T) < 2e-6
+    assert torch.equal(x[:, :n], x0[:, :n] + few) and torch.equal(x[:, n:], x0[:, n:])
+
+
 @pytest.mark.parametrize("m,n,k", [(64, 256, 8192), (33, 130, 2080), (300, 160, 64), (129, 65, 4128), (16, 2048, 8192), (17, 90, 32), (70, 100, 1000), (40, 70, 203),
                                    # three, five, six and seven ranges of k that are not empty, the last ones whole or not
                                    (40, 70, 96), (300, 160, 160), (33, 90, 192), (70, 100, 224), (40, 70, 75), (70, 90, 141), (40, 70, 201)])
