@@ -19,6 +19,11 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint4 load16(const bf16_t* p) { return *reinterpret_cast<const uint4*>(p); }
+__device__ __forceinline__ uint2 load8_once(const bf16_t* p) {
+    typedef uint32_t gi_load2 __attribute__((ext_vector_type(2)));
+    const gi_load2 v = __builtin_nontemporal_load(reinterpret_cast<const gi_load2*>(p));
+    return uint2{v.x, v.y};
+}
 __device__ __forceinline__ uint2 load8(const bf16_t* p) { return *reinterpret_cast<const uint2*>(p); }
 __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
 __device__ __forceinline__ uint32_t pack2(float a, float b) { return f32x2_to_bf16x2(a, b); }
@@ -821,7 +826,9 @@ __global__ __launch_bounds__(ORDER_MAX_ROWS) void decode_order_kernel(const int*
     order[before] = row;
 }
 
-template <int HD, bool FUSED, bool CAP>
+// PAGE16: pages of 16 positions, the usual ones, in which 16 channels' values lie in one piece and go past the caches.  (The kernel is not told more of it: with the size a
+// constant the compiler keeps addresses in 12 to 22 more registers, a wave of a SIMD's four or five.)
+template <int HD, bool FUSED, bool CAP, bool PAGE16 = false>
 __global__ __launch_bounds__(64 * DecodeShape<HD>::MAX_WAVES) void attention_decode_kernel(
     const bf16_t* __restrict__ q, const float* __restrict__ qf, const float* __restrict__ kf, const float* __restrict__ vf, long ldq, long ldk,
     long ldv, const float* __restrict__ cos_t, const float* __restrict__ sin_t, bf16_t* __restrict__ cache, float* __restrict__ part,
@@ -887,13 +894,28 @@ __global__ __launch_bounds__(64 * DecodeShape<HD>::MAX_WAVES) void attention_dec
         for (int t = 0; t < 2; ++t) pg[t] = tab[__builtin_amdgcn_readfirstlane(min(max(page_index(kv0 + 16 * t), first_page), last_page))];
     };
     uint4 k_a[2][KSTEPS], k_b[2][KSTEPS];
+    // Heads of 64 and 128 channels: a load brings 128 bytes of 8 positions' keys, whole cache lines that are used once; two of them hold 64 channels of 16 positions,
+    // whose halves change places before they are used (`rows_of_halves`).  A block of 16 positions is read whole, from one scalar address: what lies in its page beyond the
+    // row's own range is masked with its scores.
+    // (Caps of scores and heads of 256 channels leave no registers for that.)
+    constexpr bool LINES = !CAP && (HD == 64 || HD == 128);
+    const unsigned key_lane = LINES ? (lane & 7) * HD + 8 * q4 + 32 * ((lane >> 3) & 1) : r * HD + 8 * q4;
     auto load_keys = [&](int kv0, const int (&pg)[2], uint4 (&dst)[2][KSTEPS]) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            const int kv = min(max(kv0 + 16 * t + r, lo), my_pos);
-            const bf16_t* krow = kbase + (long)pg[t] * page_stride + (long)place_of(kv) * HD + 8 * q4;
+            if constexpr (HD == 256) {
+                const int kv = min(max(kv0 + 16 * t + r, lo), my_pos);
+                const bf16_t* krow = kbase + (long)pg[t] * page_stride + (long)place_of(kv) * HD + 8 * q4;
 #pragma unroll
-            for (int ks = 0; ks < KSTEPS; ++ks) dst[t][ks] = load16(krow + 32 * ks);
+                for (int ks = 0; ks < KSTEPS; ++ks) dst[t][ks] = load16(krow + 32 * ks);
+                continue;
+            }
+            const bf16_t* block = kbase + (long)pg[t] * page_stride + (long)place_of(kv0 + 16 * t) * HD;
+#pragma unroll
+            for (int ks = 0; ks < KSTEPS; ++ks) {
+                if constexpr (LINES) dst[t][ks] = load16_once(block + key_lane + 8 * HD * (ks & 1) + 32 * (ks & ~1));
+                else dst[t][ks] = load16(block + key_lane + 32 * ks);
+            }
         }
     };
     // The values of a tile are asked for behind the products of the tile before it (the first tile's behind its keys), into the
@@ -905,8 +927,9 @@ __global__ __launch_bounds__(64 * DecodeShape<HD>::MAX_WAVES) void attention_dec
         const bf16_t* vb = vbase + (long)pg[1] * page_stride + place_of(kvb) + (long)r * page_size;
 #pragma unroll
         for (int i = 0; i < DT; ++i) {
-            vx[i] = load8(va + (long)(16 * i) * page_size);
-            vy[i] = load8(vb + (long)(16 * i) * page_size);
+            const long at = (long)(16 * i) * page_size;
+            vx[i] = PAGE16 ? load8_once(va + at) : load8(va + at);
+            vy[i] = PAGE16 ? load8_once(vb + at) : load8(vb + at);
         }
     };
     int pg_cur[2] = {0, 0}, pg_nxt[2] = {0, 0};
@@ -971,6 +994,12 @@ __global__ __launch_bounds__(64 * DecodeShape<HD>::MAX_WAVES) void attention_dec
         int pg_far[2] = {0, 0};
         if constexpr (NEXT) pages_of(kv0 + 64, pg_far);
         if constexpr (NEXT) load_keys(kv0 + 32, pg_nxt, k_fill);
+        if constexpr (LINES) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int ks = 0; ks < KSTEPS; ks += 2) rows_of_halves(k_use[t][ks], k_use[t][ks + 1]);
+        }
         if constexpr (FUSED && !NEXT) {
             if (has_own) {                                // the last tile of the piece: the row's own key and value go in
                 const int off = my_pos - kv0;             // 0 .. 31
@@ -1360,21 +1389,23 @@ GI_API int gi_attention_decode_bf16(const void* q, const float* qf, const float*
     dim3 grid(n_rows, n_kv * hg, n_splits);
     GI_REQUIRE(!ordered || (rows != nullptr && (long)n_rows * n_kv * hg * n_splits < 2147483647L), "attention_decode: an order needs its rows, and fewer workgroups");
     const int units = ordered ? gi_compute_units() : 0;
-#define GO2(HD, FUSED_, CAP_)                                                                                                              \
-    attention_decode_kernel<HD, FUSED_, CAP_><<<grid, 64 * n_waves, lds, stream>>>((const bf16_t*)q, qf, kf, vf, ldq, ldk, ldv, cos_t, sin_t, \
+#define GO3(HD, FUSED_, CAP_, PAGE16_)                                                                                                              \
+    attention_decode_kernel<HD, FUSED_, CAP_, PAGE16_><<<grid, 64 * n_waves, lds, stream>>>((const bf16_t*)q, qf, kf, vf, ldq, ldk, ldv, cos_t, sin_t, \
                                                                                    (bf16_t*)cache, part, (bf16_t*)out, rows, pos, slots, table, \
                                                                                    table_stride, page_stride, page_size, n_heads, n_kv, window, \
                                                                                    scale, n_splits, gh, units, extra)
     GI_REQUIRE(!(qf && extra.cap > 0.f), "attention_decode: capped scores are not served from unrotated products");
-#define GO(HD)                                         \
-    do {                                               \
-        if (qf) GO2(HD, true, false);                  \
-        else if (extra.cap > 0.f) GO2(HD, false, true); \
-        else GO2(HD, false, false);                    \
+#define GO2(HD, PAGE16_)                                       \
+    do {                                                       \
+        if (qf) GO3(HD, true, false, PAGE16_);                 \
+        else if (extra.cap > 0.f) GO3(HD, false, true, false); \
+        else GO3(HD, false, false, PAGE16_);                   \
     } while (0)
-    if (hd == 32) GO(32); else if (hd == 64) GO(64); else if (hd == 96) GO(96); else if (hd == 128) GO(128); else GO(256);
+#define GO(HD) do { if (page_size == 16) GO2(HD, true); else GO2(HD, false); } while (0)
+    if (hd == 32) GO2(32, false); else if (hd == 64) GO(64); else if (hd == 96) GO2(96, false); else if (hd == 128) GO(128); else GO2(256, false);
 #undef GO
 #undef GO2
+#undef GO3
     GI_CHECK_LAUNCH("attention_decode");
     if (n_splits > 1) {
         dim3 cgrid(n_rows, n_heads);

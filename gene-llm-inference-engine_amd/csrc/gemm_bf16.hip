@@ -75,11 +75,6 @@ __device__ __forceinline__ float gate_fast_of(float g, float u, float limit) {
 }
 
 __device__ __forceinline__ uint4 load16(const bf16_t* p) { return *reinterpret_cast<const uint4*>(p); }
-__device__ __forceinline__ uint4 load16_once(const bf16_t* p) {              // of bytes that this launch reads no second time
-    typedef uint32_t gi_load4 __attribute__((ext_vector_type(4)));
-    const gi_load4 v = __builtin_nontemporal_load(reinterpret_cast<const gi_load4*>(p));
-    return uint4{v.x, v.y, v.z, v.w};
-}
 __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
 
 template <int EPI>

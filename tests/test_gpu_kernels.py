@@ -1541,6 +1541,24 @@ def test_attention_finds_one_far_key(dtype):
     assert rel(out.view(n_heads, hd)[0], v[target, 0]) < 2e-2          # the softmax is nearly one-hot on the target
 
 
+@pytest.mark.parametrize("hd", [32, 64, 96, 128])
+@pytest.mark.parametrize("ps,window", [(16, None), (16, 19), (48, None)])
+def test_decoded_rows_read_whole_blocks_of_keys(hd, ps, window):
+    """Single rows whose ranges begin and end anywhere in a block of 16 positions, by whole cache lines or not; what lies beyond a row in its pages is NaN and reaches no result."""
+    from geneinfer_amd.parts import StepContext
+    contexts = list(range(1, 35)) + [47, 48, 49, 63, 64, 65, 129, 500]
+    cache, table, dense = build_paged(contexts, 2, hd, ps, torch.bfloat16, seed=hd)
+    T = len(contexts)
+    q = randn(T, 6 * hd, dtype=torch.bfloat16, seed=3)
+    pos = torch.tensor([n - 1 for n in contexts], dtype=torch.int32, device=DEV)
+    ctx = StepContext(n_rows=T, dtype=torch.bfloat16, device=torch.device(DEV), tokens=pos, row_pos=pos, row_slot=torch.arange(1, T + 1, dtype=torch.int32, device=DEV),
+                      seg_slot=list(range(1, T + 1)), seg_start=list(range(T)), seg_len=[1] * T, seg_pos0=[n - 1 for n in contexts])
+    out = torch.full((T, 6 * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops().attention(q, cache, out, ctx, table, 6, 2, hd, window)
+    want = plain_attention_rows(q, dense, [(i, n - 1) for i, n in enumerate(contexts)], 6, 2, hd, window)
+    assert rel(out, want) < 8e-3, rel(out, want)
+
+
 @pytest.mark.parametrize("n_heads,n_kv,hd,ps,window", ATT_CASES)
 @pytest.mark.parametrize("target_waves", [4096, 64])
 def test_decode_attention_from_unrotated_products(n_heads, n_kv, hd, ps, window, target_waves, monkeypatch):
