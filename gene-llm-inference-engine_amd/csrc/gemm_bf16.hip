@@ -1406,6 +1406,17 @@ __global__ __launch_bounds__(512, MT == 2 ? 4 : 2) void gemm_bf16_skinny_kernel(
     }
 }
 
+// Where in its steps of 64 k a workgroup of the kernels for few rows begins: all at the same k would ask the same memory channels, and the same of an L2's for the rows that they
+// share.  Workgroups go to the eight compute dies in turn, so those of one die take the places 3, 6, 9, ... apart, modulo a power of two (`turn` + 1).  Microseconds with one place for
+// all, with the workgroup's number, and so: 16,384 x 2,048 gated at 64 rows 18.2, 17.1, 16.1, at 24 rows 17.2, 15.8, 14.5, at one row 12.6, 12.1, 12.2; 28,672 x 4,096 gated at 8 rows
+// 43.0 with its number, 41.4, at 64 rows 54.1, 50.7, 49.9; 128,256 x 2,048 at 64 rows 119.7, 120.9, 115.9.
+__device__ __forceinline__ int first_step(int turn) { return (int)((blockIdx.x >> 3) * 3) & turn; }
+static int turn_of_steps(int steps) {
+    int turn = 1;
+    while (2 * turn <= steps) turn *= 2;
+    return turn - 1;
+}
+
 // ------------------------------------------------------------------------------------------ strips
 // All rows of A (up to 32 TM of them) against 64 rows of W and the k range of the workgroup's grid row: both operands go from memory straight into
 // a ring of LDS stages of 64 k (chunks placed as in the kernels above), STAGES - 1 of them in flight.  Eight waves: two halves of 32
@@ -1416,8 +1427,8 @@ __global__ __launch_bounds__(512, MT == 2 ? 4 : 2) void gemm_bf16_skinny_kernel(
 // a product, in a captured chain of products that each have weights of their own (640 MB of them a chain), with the kernel that adds up where k is shared out; before (weights
 // through registers up to 128 rows, tiles of 128 x 128 above) and now:
 //   rows                     17            64            128           131           192
-//   16,384 x 2,048 gated     18.2, 17.4    21.8, 18.5    29.8, 23.1    28.4, 23.4    28.9, 27.3
-//   28,672 x 4,096 gated     53.2, 47.8    63.3, 53.0    90.0, 68.2    (as before)
+//   16,384 x 2,048 gated     18.2, 14.7    21.8, 16.1    29.8, 21.5    28.4, 21.8    28.9, 25.8
+//   28,672 x 4,096 gated     53.2, 43.0    63.3, 49.9    90.0, 65.0    (as before)
 //   2,048 x 2,048 added      (other)       10.1, 9.4     14.0, 11.0    14.5, 11.1    16.7, 11.9
 //   2,048 x 8,192 added      12.8, 11.8    15.1, 13.5    20.4, 17.9    23.8, 19.0    25.4, 21.6
 //   3,072 x 8,192 added      17.9, 15.4    21.2, 17.7    27.2, 22.5    37.5, 23.3    39.7, 28.3
@@ -1432,7 +1443,7 @@ constexpr int strip_bytes(int tm, int stages) {
 }
 template <int TM, int STAGES, int EPI, bool PARTIAL>
 __global__ __launch_bounds__(512, TM <= 2 ? 4 : 2) void gemm_bf16_strip_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ C,
-                                                                              float* __restrict__ P, int all_rows, int N, int K, long lda, long ldw, long ldc, int k_per_split, int tile_rows, NormIn norm_in) {
+                                                                              float* __restrict__ P, int all_rows, int N, int K, long lda, long ldw, long ldc, int k_per_split, int tile_rows, int turn, NormIn norm_in) {
     const int m_first = PARTIAL ? blockIdx.z * tile_rows : 0, M = PARTIAL ? min(tile_rows, all_rows - m_first) : all_rows;       // of this tile
     constexpr int BM = 32 * TM, STAGE_BYTES = (64 + BM) * 128, CHUNK = strip_chunk(TM, STAGES);
     extern __shared__ __attribute__((aligned(16))) unsigned char ring[];               // strip_bytes(TM, STAGES)
@@ -1466,7 +1477,9 @@ __global__ __launch_bounds__(512, TM <= 2 ? 4 : 2) void gemm_bf16_strip_kernel(c
         }
     }
     const unsigned ring_base = (unsigned)(size_t)(lds_ptr_t)ring;
-    auto issue = [&](int block, int slot) {
+    const int first_block = first_step(turn + 1 > n_k ? 0 : turn);
+    auto issue = [&](int step_, int slot) {
+        const int ahead = step_ + first_block, block = ahead < n_k ? ahead : ahead - n_k;
         const unsigned at = ring_base + slot * STAGE_BYTES + wave * 1024;
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(w_src), "s"(w_tile + block * PK) : "memory", "m0");
 #pragma unroll
@@ -1879,7 +1892,7 @@ __global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __
 #pragma unroll
     for (int t = 0; t < XT; ++t) x_at[t] = ((unsigned)min(8 * t + r, M - 1) * (unsigned)lda8 + k_lane / 8) * (16 / PIECE);
     const int k_last = K - 8 - k_lane;                                 // the last 16 bytes of a row, from `w_row` and `x_row`
-    const int steps = (K + 63) / 64, first = blockIdx.x & turn;           // (`turn` + 1: the largest power of two of steps)
+    const int steps = (K + 63) / 64, first = first_step(turn);
     const int mine = (steps - wave + 7) / 8;                           // of this wave
     auto place = [&](int i) {                                          // k where the wave's step i begins
         const int step = wave + 8 * i + first;
@@ -2486,9 +2499,7 @@ static int launch_slim(const void* A, const void* W, void* C, int epi, int M, in
     if (rows > 24 && (31 * ldw * 2 >= 1l << 32 || 15 * lda * 2 >= 1l << 32)) rows = is_gated(epi) ? 16 : 24;
     GI_REQUIRE((N == 1 || 31 * (ldw / 8) < 1l << 32) && (M == 1 || 15 * (lda / 8) < 1l << 32), "gemm_bf16: rows %ld and %ld elements apart are not taken", lda, ldw);
     const dim3 grid((N + rows - 1) / rows);
-    int turn = 1;
-    while (2 * turn <= (K + 63) / 64) turn *= 2;
-    --turn;
+    const int turn = turn_of_steps((K + 63) / 64);
 #define SLIM_XT(GROUPS_, EPI_, XT_)                                                                                                                    \
     do {                                                                                                                                               \
         if (hand) gemm_bf16_slim_kernel<GROUPS_, EPI_, true, XT_><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, (int)(lda / 8), (int)(ldw / 8), M, N, K, rows, turn, C, ldc, norm_in, norm_out); \
@@ -2566,6 +2577,7 @@ static int launch_strips(const void* A, const void* W, void* C, int epi, int M, 
     const int splits = cut.splits, k_per_split = splits == 0 ? K : (K / PK + splits - 1) / splits * PK;
     const int tile_rows = (M + cut.tiles - 1) / cut.tiles;
     dim3 grid((N + 63) / 64, splits == 0 ? 1 : splits, cut.tiles);
+    const int turn = turn_of_steps(k_per_split / PK);
 #define STRIP(TM_, ST_, EPI_, PARTIAL_)                                                                                                 \
     do {                                                                                                                                \
         constexpr int bytes = strip_bytes(TM_, ST_);                                                                                    \
@@ -2575,7 +2587,7 @@ static int launch_strips(const void* A, const void* W, void* C, int epi, int M, 
                 return gi_fail("gemm_bf16: cannot reserve %d bytes of LDS", bytes);                                                     \
             raised = true;                                                                                                              \
         }                                                                                                                               \
-        gemm_bf16_strip_kernel<TM_, ST_, EPI_, PARTIAL_><<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, scratch, M, N, K, lda, ldw, ldc, k_per_split, tile_rows, norm_in); \
+        gemm_bf16_strip_kernel<TM_, ST_, EPI_, PARTIAL_><<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, scratch, M, N, K, lda, ldw, ldc, k_per_split, tile_rows, turn, norm_in); \
     } while (0)
 #define STRIP_TM(EPI_, PARTIAL_)                                                                                                        \
     do {                                                                                                                                \
