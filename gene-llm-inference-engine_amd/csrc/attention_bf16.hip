@@ -434,13 +434,15 @@ constexpr int WIDE_MAX_SHARES = 4;
 typedef unsigned gi_uint4 __attribute__((ext_vector_type(4)));
 constexpr int DEVICE_SCOPE = 16;               // sc1 in a buffer access's cache policy
 template <int HD> constexpr int wide_share_bytes(int nw) { return nw * (HD / 32 * 4 + 1) * 1024; }
+template <int HD> constexpr int wide_lds_bytes() { return 2 * (KV_TILE * HD * 2 + HD * KV_TILE * 2); }
+// head, at, n_at: the workgroup's place in the launch.
 template <int HD, int NW, bool CAP>
-__global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache,
-                                                                       bf16_t* __restrict__ out, const int4* __restrict__ tiles,
-                                                                       const int* __restrict__ table, int table_stride, long page_stride,
-                                                                       int page_size, int n_heads, int n_kv, int window, float scale,
-                                                                       int n_splits, const int* __restrict__ tile_first, float* __restrict__ part,
-                                                                       int list_order, Extras extra, WideShares shares) {
+__device__ __forceinline__ void prompt_wide(unsigned char* lds, int head, int at, int n_at, const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache,
+                                            bf16_t* __restrict__ out, const int4* __restrict__ tiles,
+                                            const int* __restrict__ table, int table_stride, long page_stride,
+                                            int page_size, int n_heads, int n_kv, int window, float scale,
+                                            int n_splits, const int* __restrict__ tile_first, float* __restrict__ part,
+                                            int list_order, const Extras& extra, const WideShares& shares) {
     static_assert(HD == 128 || HD == 64, "the chunk swizzle is made for key rows of 256 or 128 bytes");
     constexpr int QSTEPS = HD / 16, DT = HD / 32;
     constexpr int K_BYTES = KV_TILE * HD * 2, V_BYTES = HD * KV_TILE * 2, STAGE = K_BYTES + V_BYTES;
@@ -448,14 +450,13 @@ __global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_w
     constexpr int K_LOADS = K_BYTES / 1024, V_LOADS = V_BYTES / 1024, LOADS = (K_LOADS + V_LOADS) / NW;      // wave-wide loads of 1 KB: per tile, per wave
     static_assert((K_LOADS + V_LOADS) % NW == 0 && K_LOADS % LOADS == 0, "a wave's loads are all keys or all values");
     static_assert(LOADS % (16 / (64 / CK)) == 0, "a wave's loads begin with a group's first rows");
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * STAGE];
 
     // Workgroups start in the order of their numbers, heads fastest: the long walks (late tiles) of all heads first, so that the
     // short ones fill the end.  A plain list runs from early tiles to late ones and is taken backwards; a list of pairs names a
     // late tile, an early one, the next later one, the next earlier one, ...: first its late tiles in their order, then its early
     // ones backwards.
     const int places = shares.most > 1 ? shares.most : n_splits;
-    const int n_groups = gridDim.y / places, turn = blockIdx.y / places, split = blockIdx.y % places;
+    const int n_groups = n_at / places, turn = at / places, split = at % places;
     const int group = !list_order ? n_groups - 1 - turn : turn < n_groups / 2 ? 2 * turn : 2 * (n_groups - 1 - turn) + 1;
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int4 tile = tiles[group];
@@ -466,7 +467,7 @@ __global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_w
         n_splits = min(shares.most, (walk + shares.keys - 1) / shares.keys);
         if (split >= n_splits) return;
     }
-    const int head = blockIdx.x, g = head / (n_heads / n_kv);
+    const int g = head / (n_heads / n_kv);
     const int col = lane & 31, hf = lane >> 5;
     const int* tab = table + (size_t)slot * table_stride;
 
@@ -649,7 +650,7 @@ __global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_w
         float& start = *reinterpret_cast<float*>(lds + 4);     // 0, or no number where the others never came
         const size_t walk = (size_t)group * n_heads + head;
         unsigned* const counter = shares.counters + 2 * walk;
-        const int at = (wv * PIECES * 64 + lane) * 16;
+        const int mine_at = (wv * PIECES * 64 + lane) * 16;
         auto place = [&](int of) {
             return __builtin_amdgcn_make_buffer_rsrc(shares.sums + (walk * shares.most + of) * wide_share_bytes<HD>(NW), 0, wide_share_bytes<HD>(NW), 0x00027000);
         };
@@ -661,9 +662,9 @@ __global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_w
             for (int f = 0; f < DT * 4; ++f) {
                 const int v = (f & 3) * 4;
                 __builtin_amdgcn_raw_buffer_store_b128(gi_uint4{__float_as_uint(o[f >> 2][v]), __float_as_uint(o[f >> 2][v + 1]), __float_as_uint(o[f >> 2][v + 2]),
-                                                                __float_as_uint(o[f >> 2][v + 3])}, mine, at, f * 1024, DEVICE_SCOPE);
+                                                                __float_as_uint(o[f >> 2][v + 3])}, mine, mine_at, f * 1024, DEVICE_SCOPE);
             }
-            __builtin_amdgcn_raw_buffer_store_b128(gi_uint4{__float_as_uint(m), __float_as_uint(l), 0u, 0u}, mine, at, DT * 4 * 1024, DEVICE_SCOPE);
+            __builtin_amdgcn_raw_buffer_store_b128(gi_uint4{__float_as_uint(m), __float_as_uint(l), 0u, 0u}, mine, mine_at, DT * 4 * 1024, DEVICE_SCOPE);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's sums are in memory
             __syncthreads();
             if (tid == 0) __hip_atomic_fetch_add(counter + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -678,7 +679,7 @@ __global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_w
             weight[of] = of == split ? m : -INFINITY;
             share_l[of] = of == split ? l : 0.f;
             if (of < n_splits && of != split) {
-                const gi_uint4 v = __builtin_amdgcn_raw_buffer_load_b128(place(of), at, DT * 4 * 1024, DEVICE_SCOPE);
+                const gi_uint4 v = __builtin_amdgcn_raw_buffer_load_b128(place(of), mine_at, DT * 4 * 1024, DEVICE_SCOPE);
                 weight[of] = __uint_as_float(v[0]);
                 share_l[of] = __uint_as_float(v[1]);
             }
@@ -703,7 +704,7 @@ __global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_w
                     const auto theirs = place(of);
                     gi_uint4 sums[4];
 #pragma unroll
-                    for (int f = 0; f < 4; ++f) sums[f] = __builtin_amdgcn_raw_buffer_load_b128(theirs, at, (i * 4 + f) * 1024, DEVICE_SCOPE);
+                    for (int f = 0; f < 4; ++f) sums[f] = __builtin_amdgcn_raw_buffer_load_b128(theirs, mine_at, (i * 4 + f) * 1024, DEVICE_SCOPE);
 #pragma unroll
                     for (int v = 0; v < 16; ++v) total[v] = fmaf(weight[of], __uint_as_float(sums[v >> 2][v & 3]), total[v]);
                 }
@@ -737,6 +738,17 @@ __global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_w
             *reinterpret_cast<uint2*>(orow + d) = gated4(extra, (size_t)(row0 + my_row), head, d, o[i][4 * v4] * inv, o[i][4 * v4 + 1] * inv, o[i][4 * v4 + 2] * inv,
                                                          o[i][4 * v4 + 3] * inv);
         }
+}
+template <int HD, int NW, bool CAP>
+__global__ __launch_bounds__(64 * NW, HD == 128 ? 2 : 3) void attention_prompt_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache,
+                                                                       bf16_t* __restrict__ out, const int4* __restrict__ tiles,
+                                                                       const int* __restrict__ table, int table_stride, long page_stride,
+                                                                       int page_size, int n_heads, int n_kv, int window, float scale,
+                                                                       int n_splits, const int* __restrict__ tile_first, float* __restrict__ part,
+                                                                       int list_order, Extras extra, WideShares shares) {
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[wide_lds_bytes<HD>()];
+    prompt_wide<HD, NW, CAP>(lds, blockIdx.x, blockIdx.y, gridDim.y, q, cache, out, tiles, table, table_stride, page_stride, page_size, n_heads, n_kv, window, scale,
+                             n_splits, tile_first, part, list_order, extra, shares);
 }
 
 // =========================================================================================== decode
@@ -828,17 +840,17 @@ __global__ __launch_bounds__(ORDER_MAX_ROWS) void decode_order_kernel(const int*
 
 // PAGE16: pages of 16 positions, the usual ones, in which 16 channels' values lie in one piece and go past the caches.  (The kernel is not told more of it: with the size a
 // constant the compiler keeps addresses in 12 to 22 more registers, a wave of a SIMD's four or five.)
-template <int HD, bool FUSED, bool CAP, bool PAGE16 = false>
-__global__ __launch_bounds__(64 * DecodeShape<HD>::MAX_WAVES) void attention_decode_kernel(
+// merged: [wave][gh][HD + 2] in LDS.
+template <int HD, bool FUSED, bool CAP, bool PAGE16>
+__device__ __forceinline__ void decode_rows(
+    float* merged, const DecodeItem& item,
     const bf16_t* __restrict__ q, const float* __restrict__ qf, const float* __restrict__ kf, const float* __restrict__ vf, long ldq, long ldk,
     long ldv, const float* __restrict__ cos_t, const float* __restrict__ sin_t, bf16_t* __restrict__ cache, float* __restrict__ part,
     bf16_t* __restrict__ out, const int* __restrict__ rows, const int* __restrict__ pos, const int* __restrict__ slots,
     const int* __restrict__ table, int table_stride, long page_stride, int page_size, int n_heads, int n_kv, int window, float scale,
-    int n_splits, int gh, int units, Extras extra) {
+    int n_splits, int gh, const Extras& extra) {
     constexpr int KSTEPS = HD / 32, DT = HD / 16;
-    extern __shared__ float merged[];                        // [wave][gh][HD + 2]
     const int group = n_heads / n_kv, hg_per_kv = (group + 15) / 16;
-    const DecodeItem item = decode_item(units);
     const int row = rows ? rows[item.row] : item.row, g = item.heads / hg_per_kv, hg = item.heads % hg_per_kv, split = item.split;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n_waves = blockDim.x >> 6;
     const int r = lane & 15, q4 = lane >> 4;
@@ -1136,6 +1148,47 @@ __global__ __launch_bounds__(64 * DecodeShape<HD>::MAX_WAVES) void attention_dec
     }
 }
 
+template <int HD, bool FUSED, bool CAP, bool PAGE16 = false>
+__global__ __launch_bounds__(64 * DecodeShape<HD>::MAX_WAVES) void attention_decode_kernel(
+    const bf16_t* __restrict__ q, const float* __restrict__ qf, const float* __restrict__ kf, const float* __restrict__ vf, long ldq, long ldk,
+    long ldv, const float* __restrict__ cos_t, const float* __restrict__ sin_t, bf16_t* __restrict__ cache, float* __restrict__ part,
+    bf16_t* __restrict__ out, const int* __restrict__ rows, const int* __restrict__ pos, const int* __restrict__ slots,
+    const int* __restrict__ table, int table_stride, long page_stride, int page_size, int n_heads, int n_kv, int window, float scale,
+    int n_splits, int gh, int units, Extras extra) {
+    extern __shared__ float merged[];
+    decode_rows<HD, FUSED, CAP, PAGE16>(merged, decode_item(units), q, qf, kf, vf, ldq, ldk, ldv, cos_t, sin_t, cache, part, out, rows, pos, slots, table, table_stride,
+                                        page_stride, page_size, n_heads, n_kv, window, scale, n_splits, gh, extra);
+}
+
+// ------------------------------------------------------------------------------------------- both
+// Portions of prompts and single rows of one step in one launch (`prompt_wide`, `decode_rows`): the former are bound by the matrix cores and by walks of uneven length, which leave
+// units idle towards the end, the latter by the memory.  Workgroups go to the eight dies in turn, on each to its units in turn: the two kinds take turns eight by eight, and change places
+// every 32 of a die, so that a unit's first two are one of each as long as there are both.
+// Two launches and in one, 24 heads of 128 channels: portions of 1,350 rows behind 1,000 positions and of 674, 24 single rows at up to 2,990 positions, 110 and 93 us (the tiles alone 69);
+// 300 rows and 4 at up to 428 25.8 and 16.3; 32 heads of 64: 1,812 rows and 26 at up to 1,643 53.1 and 41.7.
+struct BothSplit { int prompt, decode; };               // workgroups of each kind, both padded to multiples of 8
+template <int HD, bool PAGE16>
+__global__ __launch_bounds__(256, HD == 128 ? 2 : 3) void attention_both_kernel(
+    const bf16_t* __restrict__ q, bf16_t* __restrict__ cache, bf16_t* __restrict__ out, const int4* __restrict__ tiles, int n_at, const int* __restrict__ table, int table_stride,
+    long page_stride, int page_size, int n_heads, int n_kv, int window, float scale, int tile_splits, const int* __restrict__ tile_first, float* __restrict__ tile_part, int list_order,
+    Extras extra, WideShares shares, const int* __restrict__ rows, int n_rows, const int* __restrict__ pos, const int* __restrict__ slots, float* __restrict__ part, int n_splits, int gh,
+    BothSplit count) {
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[wide_lds_bytes<HD>()];
+    const int turn = blockIdx.x >> 3, both = min(count.prompt, count.decode) >> 3;
+    const bool paired = turn < 2 * both, decodes = paired ? ((turn ^ (turn >> 5)) & 1) == 0 : count.decode > count.prompt;
+    const int of_kind = ((paired ? turn >> 1 : turn - both) << 3) + (blockIdx.x & 7);
+    if (decodes) {
+        const int each = n_kv * ((n_heads / n_kv + 15) / 16) * n_splits, row = of_kind / each, rest = of_kind % each, heads = each / n_splits;
+        if (row >= n_rows) return;
+        decode_rows<HD, false, false, PAGE16>(reinterpret_cast<float*>(lds), DecodeItem{row, rest % heads, rest / heads}, q, nullptr, nullptr, nullptr, 0, 0, 0, nullptr, nullptr, cache,
+                                              part, out, rows, pos, slots, table, table_stride, page_stride, page_size, n_heads, n_kv, window, scale, n_splits, gh, extra);
+    } else {
+        if (of_kind >= n_at * n_heads) return;
+        prompt_wide<HD, 4, false>(lds, of_kind % n_heads, of_kind / n_heads, n_at, q, cache, out, tiles, table, table_stride, page_stride, page_size, n_heads, n_kv, window, scale,
+                                  tile_splits, tile_first, tile_part, list_order, extra, shares);
+    }
+}
+
 // Merges the splits of one (row, head): out = sum_s e^(m_s - M) O_s / sum_s e^(m_s - M) l_s, the sums
 // taken in split order.  One wave: lane s first fetches split s's {m, l} (all splits at once), then
 // lane d adds channel d over the splits with the weights read from LDS.
@@ -1411,6 +1464,68 @@ GI_API int gi_attention_decode_bf16(const void* q, const float* qf, const float*
         dim3 cgrid(n_rows, n_heads);
         attention_decode_combine_kernel<<<cgrid, 64, 0, stream>>>(part, (bf16_t*)out, rows, n_heads, hd, n_splits, extra);
         GI_CHECK_LAUNCH("attention_decode (combine)");
+    }
+    return 0;
+}
+
+// Whether gi_attention_both_bf16 takes a step whose tiles and single rows these are.
+GI_API int gi_attention_both_takes(int n_tiles, int rows_per_tile, int paired, int tile_splits, int most_shares, int n_rows, int n_splits, int n_heads, int n_kv, int hd, int page_size) {
+    if (n_tiles <= 0 || n_rows <= 0 || tile_splits < 1 || tile_splits > MAX_SPLITS || n_splits < 1 || n_splits > MAX_SPLITS || n_heads <= 0 || n_kv <= 0 || n_heads % n_kv != 0) return 0;
+    if (page_size % 16 != 0 || !(hd == 128 || (hd == 64 && rows_per_tile == 128)) || most_shares < 1 || (tile_splits > 1 && most_shares > 1)) return 0;
+    if (!takes_wide(n_tiles, n_heads, hd, tile_splits, paired, most_shares > 1)) return 0;
+    return (long)n_tiles * tile_splits * most_shares <= 65535 && (long)n_tiles * tile_splits * most_shares * n_heads + (long)n_rows * n_heads * n_splits < (1L << 30);
+}
+
+// gi_attention_prompt_bf16 and gi_attention_decode_bf16 (of rotated queries, workgroups of four waves) of one step in one launch; arguments as theirs: `tile_part` for the tiles' shares or
+// splits, `part` for the rows' splits.
+GI_API int gi_attention_both_bf16(const void* q, void* cache, void* out, const int* tiles, int n_tiles, int rows_per_tile, int paired, const int* table, int table_stride,
+                                  long page_stride, int page_size, int n_heads, int n_kv, int hd, int window, float scale, int tile_splits, const int* tile_first, const int* tile_rows,
+                                  int n_tile_rows, float* tile_part, long tile_floats, int chunk, const float* sinks, const float* gate, long gate_stride, int gate_channels, int share_keys,
+                                  int most_shares, unsigned* counters, const int* rows, int n_rows, const int* pos, const int* slots, float* part, long part_floats, int n_splits,
+                                  hipStream_t stream) {
+    GI_REQUIRE(chunk >= 0 && (gate_channels == 0 || gate_channels == hd) && (gate == nullptr || gate_stride >= (long)n_heads * (gate_channels ? hd : 1)) &&
+                   (gate == nullptr || gate_channels == 0 || (gate_stride % 4 == 0 && ((uintptr_t)gate & 15) == 0)),
+               "attention_both: bad chunk or gate stride, or a channels' gate whose rows do not start at multiples of 16 bytes");
+    const Extras extra = {chunk, sinks, gate, gate_stride, gate_channels, 0.f};
+    GI_REQUIRE(rows_per_tile == 64 || rows_per_tile == 128, "attention_both: tiles of %d rows are not supported (64 or 128)", rows_per_tile);
+    GI_REQUIRE(gi_attention_both_takes(n_tiles, rows_per_tile, paired, tile_splits, most_shares, n_rows, n_splits, n_heads, n_kv, hd, page_size),
+               "attention_both: %d tiles of %d rows in %d splits or %d shares beside %d rows in %d splits, %d heads of %d with pages of %d, are not served", n_tiles, rows_per_tile,
+               tile_splits, most_shares, n_rows, n_splits, n_heads, hd, page_size);
+    GI_REQUIRE(page_stride >= 2L * n_kv * page_size * hd && page_stride % 8 == 0, "attention_both: bad page stride %ld", page_stride);
+    GI_REQUIRE(!paired || n_tiles % 2 == 0, "attention_both: %d tiles cannot go in pairs", n_tiles);
+    GI_REQUIRE(q != nullptr && pos != nullptr && slots != nullptr && rows != nullptr, "attention_both: queries, positions, slots and the single rows must be given");
+    GI_REQUIRE(n_splits == 1 || (part != nullptr && part_floats >= (long)n_rows * n_heads * n_splits * (hd + 2)), "attention_both: scratch too small");
+    GI_REQUIRE(tile_splits == 1 || (tile_first && tile_rows && tile_part && n_tile_rows > 0 && tile_floats >= (long)n_tile_rows * n_heads * tile_splits * (hd + 2)),
+               "attention_both: splitting needs the tiles' row offsets, their rows and scratch for the partial results");
+    WideShares shares = {1, 0, nullptr, nullptr};
+    if (most_shares > 1) {
+        const long floats = gi_attention_prompt_share_floats(n_tiles, rows_per_tile, n_heads, hd, 1, paired, most_shares);
+        GI_REQUIRE(floats > 0 && share_keys > 0 && counters != nullptr && tile_part != nullptr && ((uintptr_t)tile_part & 15) == 0 && tile_floats >= floats,
+                   "attention_both: %d shares of %d keys need counters and scratch that were not given, or sizes that are not shared out", most_shares, share_keys);
+        shares = {most_shares, share_keys, counters, (unsigned char*)tile_part};
+    }
+    const int group = n_heads / n_kv, hg = (group + 15) / 16, gh = group < 16 ? group : 16, n_at = n_tiles * tile_splits * shares.most;
+    const BothSplit count = {(n_at * n_heads + 7) / 8 * 8, (n_rows * n_kv * hg * n_splits + 7) / 8 * 8};
+#define BOTH(HD, PAGE16_)                                                                                                                                              \
+    do {                                                                                                                                                               \
+        static_assert(4 * 16 * (HD + 2) * (int)sizeof(float) <= wide_lds_bytes<HD>(), "the single rows' results fit the tiles' LDS");                                  \
+        attention_both_kernel<HD, PAGE16_><<<count.prompt + count.decode, 256, 0, stream>>>((const bf16_t*)q, (bf16_t*)cache, (bf16_t*)out, (const int4*)tiles, n_at, table, table_stride, \
+                                                                                            page_stride, page_size, n_heads, n_kv, window, scale, tile_splits, tile_first, tile_part, \
+                                                                                            paired ? 1 : 0, extra, shares, rows, n_rows, pos, slots, part, n_splits, gh, count); \
+    } while (0)
+    if (hd == 64) { if (page_size == 16) BOTH(64, true); else BOTH(64, false); }
+    else { if (page_size == 16) BOTH(128, true); else BOTH(128, false); }
+#undef BOTH
+    GI_CHECK_LAUNCH("attention_both");
+    if (tile_splits > 1) {
+        dim3 cgrid(n_tile_rows, n_heads);
+        attention_decode_combine_kernel<<<cgrid, 64, 0, stream>>>(tile_part, (bf16_t*)out, tile_rows, n_heads, hd, tile_splits, extra);
+        GI_CHECK_LAUNCH("attention_both (combine the tiles')");
+    }
+    if (n_splits > 1) {
+        dim3 cgrid(n_rows, n_heads);
+        attention_decode_combine_kernel<<<cgrid, 64, 0, stream>>>(part, (bf16_t*)out, rows, n_heads, hd, n_splits, extra);
+        GI_CHECK_LAUNCH("attention_both (combine the rows')");
     }
     return 0;
 }

@@ -105,6 +105,9 @@ _SIGNATURES = {
     "gi_gemm_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long, c_void_p, c_void_p],
     "gi_attention_prompt_bf16": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int,
                                  c_float, c_int, c_void_p, c_void_p, c_int, c_void_p, c_long, c_int, c_void_p, c_void_p, c_long, c_int, c_float, c_int, c_int, c_void_p, c_void_p],
+    "gi_attention_both_bf16": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p,
+                               c_void_p, c_int, c_void_p, c_long, c_int, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_long,
+                               c_int, c_void_p],
     "gi_attention_decode_bf16": [c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_long, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                  c_long, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int,
                                  c_float, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_long, c_int, c_float, c_void_p],
@@ -1563,9 +1566,41 @@ def _single_cut(plan, n_heads, n_kv, hd, seen, target_waves, fused, orders):
     return n_splits, n_waves, ordered, plan.n_decode * n_heads * n_splits * (hd + 2) if n_splits > 1 else 0
 
 
+def _both_splits(plan, n_heads, n_kv, hd, span, tile_splits, most):
+    """By how many workgroups each context of a step's single rows is read where they go out in one launch with the tiles; 0: in a launch of their own.
+    The tiles' workgroups take about 11 us, half a microsecond for each tile of keys of the longest share and 2.6 for each of a place's even share; one that reads a context
+    13.1 (64 channels: 9.8) for every 1,000 positions alone and nearly twice that beside the others.  So as few as keep the longest context within 0.8 of the
+    tiles' time: its splits would cost a merge of theirs.  Of 135 drawn steps (1 to 48 single rows at up to 30,000 positions, 256 to 2,048 rows in all) two got
+    slower, by 2 and 6 % (many single rows at under 350 positions, 45.6 and 48.3 us), and attention took 0.82 of the two launches' time in the mean: 24 heads of 128 over portions of 1,350 rows behind 1,000 positions and of 674, 24 single rows at up to
+    2,990, 110 -> 93 us; 32 heads of 64 over 1,812 rows, 26 at up to 1,643, 53.1 -> 41.7.  Where the single rows' reading is more than four times the tiles' (more
+    than was measured) the places that tiles leave them, two workgroups a unit, are too few."""
+    walks = [-(-c // 64) for c in plan.tile_contexts]
+    even = sum(walks) * n_heads / (lib().gi_compute_units() * (2 if hd == 128 else 3))
+    tiles_us = 11 + 0.5 * -(-max(walks) // max(tile_splits, most)) + 2.6 * even
+    if plan.decode_positions * n_kv * hd * 4 > 4 * tiles_us * _DECODE_CHIP_MB_PER_S:
+        return 0
+    splits = 1
+    while splits < 16 and span >= 128 * (splits + 1) and 3 + span / splits * (0.0131 if hd == 128 else 0.0098) > 0.8 * tiles_us:
+        splits += 1
+    return splits
+
+
+def _both_cut(plan, n_heads, n_kv, hd, window, chunk, page_size, seen, tile_splits, most):
+    """`_both_splits` for a plan, once a step for all layers of one kind; 0 too for sizes and options that the one launch does not take, and for a step still to come."""
+    if not plan.n_decode or plan.tile_contexts is None or plan.decode_positions is None:
+        return 0
+    key = ("both", n_heads, n_kv, hd, window, chunk, page_size, tile_splits, most)
+    if key not in plan.cuts:
+        splits = _both_splits(plan, n_heads, n_kv, hd, seen(plan.max_decode_context, 31), tile_splits, most) if hd in (64, 128) else 0
+        takes = splits and lib().gi_attention_both_takes(plan.n_tiles, plan.tile, 1 if plan.paired else 0, tile_splits, most, plan.n_decode, splits, n_heads, n_kv, hd, page_size)
+        plan.cuts[key] = splits if takes else 0
+    return plan.cuts[key]
+
+
 def attention_bf16(q, cache, out, plan: AttentionPlan, positions, slots, table, n_heads, n_kv, hd, window=None, scale=None,
-                   target_waves: int = 4096, products=None, chunk=None, sinks=None, gate=None, cap=None, channel_gate=None, memo=None):
+                   target_waves: int = 4096, products=None, chunk=None, sinks=None, gate=None, cap=None, channel_gate=None, memo=None, together=False):
     """Attention of a step's rows with the matrix-core kernels (bfloat16 cache and out).  memo: what the pass keeps for its layers (the order of its rows).
+    together: single rows may go out in one launch with the tiles of prompts (`_both_splits`).
 
     `q` holds the rotated queries in bfloat16 and the cache the rows' keys and values; or, for a step
     of single decoded rows only, `q` is None and `products = (q, k, v, cos, sin)` holds the unrotated
@@ -1628,6 +1663,16 @@ def attention_bf16(q, cache, out, plan: AttentionPlan, positions, slots, table, 
                 most, keys, n_part = 1, 0, 0
         elif n_part:
             part = torch.empty(n_part, dtype=torch.float32, device=out.device)
+        both = _both_cut(plan, n_heads, n_kv, hd, window, chunk, page_size, seen, n_splits, most) if together and memo is not None and cap is None else 0
+        if both:
+            rows = _decode_order(memo, plan, positions) if 16 < plan.n_decode <= 1024 else plan.decode_rows
+            n_rows_part = plan.n_decode * n_heads * both * (hd + 2) if both > 1 else 0
+            rows_part = torch.empty(n_rows_part, dtype=torch.float32, device=out.device) if n_rows_part else None
+            _call("gi_attention_both_bf16", q.data_ptr(), cache.data_ptr(), out.data_ptr(), plan.tiles.data_ptr(), plan.n_tiles, plan.tile, 1 if plan.paired else 0, table.data_ptr(),
+                  table.stride(0), cache.stride(0), page_size, n_heads, n_kv, hd, window, scale, n_splits, _ptr(plan.tile_first),
+                  _ptr(plan.tile_rows), plan.n_tile_rows, _ptr(part), n_part, *extras[:-1], keys, most, _ptr(counters), rows.data_ptr(),
+                  plan.n_decode, positions.data_ptr(), slots.data_ptr(), _ptr(rows_part), n_rows_part, both, _stream())
+            return out
         _call("gi_attention_prompt_bf16", q.data_ptr(), cache.data_ptr(), out.data_ptr(), plan.tiles.data_ptr(), plan.n_tiles, plan.tile,
               1 if plan.paired else 0, table.data_ptr(), table.stride(0), cache.stride(0), page_size, n_heads, n_kv, hd, window, scale, n_splits,
               _ptr(plan.tile_first), _ptr(plan.tile_rows), plan.n_tile_rows, _ptr(part), n_part, *extras, keys, most, _ptr(counters), _stream())
@@ -1669,7 +1714,7 @@ def attention(q, cache, out, ctx, table, n_heads, n_kv, hd, window=None):
     if q.dtype == torch.bfloat16 and cache.dtype == torch.bfloat16 and out.dtype == torch.bfloat16:
         plan = _plan_of(ctx)
         if (not plan.n_tiles or attention_bf16_supports(hd, page_size, True)) and (not plan.n_decode or attention_bf16_supports(hd, page_size, False)):
-            return attention_bf16(q, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, memo=ctx.memo)
+            return attention_bf16(q, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, memo=ctx.memo, together=True)
     return attention_exact(q, cache, out, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, **_known_of(ctx))
 
 
@@ -1698,7 +1743,7 @@ def attention_general(q, cache, out, ctx, table, n_heads, n_kv, hd, *, page_size
         plan = _plan_of(ctx)
         if (not plan.n_tiles or attention_bf16_supports(hd, page_size, True)) and (not plan.n_decode or attention_bf16_supports(hd, page_size, False)):
             return attention_bf16(q, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, scale, chunk=chunk, sinks=sinks, gate=gate, cap=cap,
-                                  channel_gate=channel_gate, memo=ctx.memo)
+                                  channel_gate=channel_gate, memo=ctx.memo, together=True)
     return attention_exact(q, cache, out, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, scale, page_size=page_size,
                            value_dim=value_dim, chunk=chunk, sinks=sinks, gate=gate, cap=cap, channel_gate=channel_gate, **_known_of(ctx))
 

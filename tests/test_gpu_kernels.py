@@ -1125,6 +1125,54 @@ def test_long_walks_of_prompt_tiles_share_their_keys_out(n_heads, n_kv, hd, segs
         assert rel(seen[0], plain_attention_rows(q, dense, rows, n_heads, n_kv, hd, window)) < 8e-3
 
 
+@pytest.mark.parametrize("n_heads,n_kv,hd,ps,portions,singles,splits,window,extra", [
+    # walks in shares; one more single row than a workgroup of eight fills, contexts of 1 and 33; pages of 16, 32 and 48; several splits; a window and chunks; more workgroups of either kind
+    (24, 8, 128, 16, [(1020, 1350), (0, 674)], [1, 33, 700, 2990] * 6, 1, None, None), (24, 8, 128, 32, [(500, 600)], [900, 64, 31], 2, None, None),
+    (32, 8, 64, 16, [(0, 1500)], [1, 1200, 16, 17, 500], 1, None, None), (64, 16, 64, 48, [(3000, 900), (0, 401)], [2000] * 9, 3, None, None), (64, 16, 64, 16, [(300, 1200)], [900, 30, 1700], 2, 200, None),
+    (20, 1, 128, 16, [(0, 300)], [40, 999, 1], 1, None, None), (40, 2, 128, 16, [(100, 800)], [640, 65], 3, None, None), (4, 4, 128, 48, [(1400, 100), (600, 130)], [300, 800], 1, 450, None),
+    (4, 1, 128, 16, [(0, 200)], [500] * 70, 4, None, None), (16, 8, 128, 16, [(640, 900)], [300, 129, 128, 1], 1, None, "chunk"), (16, 8, 128, 16, [(0, 900)], [300, 129], 2, None, "sinks"),
+    (24, 8, 128, 16, [(0, 700)], [800, 2], 2, None, "gate"), (32, 8, 64, 16, [(0, 1500)], [600, 3], 2, None, "channels")])
+def test_single_rows_and_tiles_in_one_launch(n_heads, n_kv, hd, ps, portions, singles, splits, window, extra, monkeypatch):
+    """A step's single rows beside portions of prompts: the tiles' rows are in bits those of a launch of their own, the single rows those of another cut of their contexts; every time the
+    same bits; and without room for shares."""
+    o = ops()
+    segs = [(c - 1, 1) for c in singles[:len(singles) // 2]] + portions + [(c - 1, 1) for c in singles[len(singles) // 2:]]
+    contexts = [p + n for p, n in segs]
+    gone = {s: max(0, p - window + 1) for s, (p, _) in enumerate(segs)} if window else None
+    cache, table, dense = build_paged(contexts, n_kv, hd, ps, torch.bfloat16, seed=5, scale_one=(0, 2.0), gone_before=gone)
+    rows = [(s, p + i) for s, (p, n) in enumerate(segs) for i in range(n)]
+    starts = [sum(n for _, n in segs[:i]) for i in range(len(segs))]
+    q = randn(len(rows), n_heads * hd, dtype=torch.bfloat16, seed=3)
+    pos = torch.tensor([p for _, p in rows], dtype=torch.int32, device=DEV)
+    slots = torch.tensor([s + 1 for s, _ in rows], dtype=torch.int32, device=DEV)
+    extras = {None: {}, "chunk": dict(chunk=128), "sinks": dict(sinks=randn(n_heads, seed=9)), "gate": dict(gate=randn(len(rows), n_heads, seed=9)),
+              "channels": dict(channel_gate=randn(len(rows), n_heads * hd, seed=9))}[extra]
+    asked, call = [], o._call
+    monkeypatch.setattr(o, "_call", lambda name, *a: (asked.append(name), call(name, *a))[1])
+    monkeypatch.setattr(o, "_both_splits", lambda *a: splits)
+
+    def made(together, memo):
+        plan = o.AttentionPlan(starts, [n for _, n in segs], [p for p, _ in segs], [s + 1 for s in range(len(segs))], DEV)
+        out = torch.full((len(rows), n_heads * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+        return o.attention_bf16(q, cache, out, plan, pos, slots, table, n_heads, n_kv, hd, window, memo=memo, together=together, **extras)
+
+    before, memo = cache.clone(), {}
+    apart, got, again = made(False, {}), made(True, memo), made(True, memo)
+    assert asked.count("gi_attention_both_bf16") == 2 and asked.count("gi_attention_prompt_bf16") == 1
+    single = torch.tensor([s for s, (_, n) in zip(starts, segs) if n == 1], device=DEV)
+    tiles = torch.ones(len(rows), dtype=torch.bool, device=DEV).index_fill_(0, single, False)
+    assert torch.equal(got, again) and torch.equal(got[tiles], apart[tiles])
+    # (probabilities are rounded to bfloat16 about other maxima, 2^-9 of each at most on either side, and the results, 2^-8 between the two)
+    assert rel(got[single], apart[single]) < 2 * 2.0 ** -9 + 2.0 ** -8
+    if extra is None:
+        assert rel(got, plain_attention_rows(q, dense, rows, n_heads, n_kv, hd, window)) < 8e-3
+    assert torch.equal(torch.nan_to_num(cache, nan=-1.0), torch.nan_to_num(before, nan=-1.0)) and ("attention_counters" not in memo or not bool(memo["attention_counters"].any()))
+    monkeypatch.setattr(o, "_room", lambda *_: None)
+    asked.clear()
+    without = made(True, {})
+    assert rel(without, got) < 2 * 2.0 ** -9 + 2.0 ** -8 and len(asked) <= 3
+
+
 def test_workgroups_that_meet_in_a_kernel_under_capture():
     """A product with shared tiles and an attention with shared walks in one captured pass, whose counters are filled in the pass: every replay gives the bits of
     the same calls made one by one, with other work and a synchronization between."""
