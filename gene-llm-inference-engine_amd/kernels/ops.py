@@ -23,8 +23,8 @@ class KernelError(RuntimeError):
 
 
 _SIGNATURES = {
-    "gi_embed": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p],
-    "gi_embed_handing": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
+    "gi_embed": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
+    "gi_embed_handing": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p, c_void_p, c_void_p, c_void_p],
     "gi_rmsnorm": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_float, c_long, c_long, c_void_p],
     "gi_rope_cos_sin": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
     "gi_rope_store": [c_void_p, c_void_p, c_void_p, c_long, c_long, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
@@ -101,6 +101,7 @@ _SIGNATURES = {
     "gi_segments": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p],
     "gi_mlstm_scan": [c_void_p, c_long, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float, c_float, c_void_p, c_void_p, c_int, c_void_p,
                       c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_int, c_int, c_void_p],
+    "gi_latent_fold": [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "gi_head_norm_gate": [c_void_p, c_long, c_void_p, c_void_p, c_long, c_void_p, c_int, c_void_p, c_int, c_long, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p],
     "gi_gemm_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_long, c_void_p, c_void_p],
     "gi_attention_prompt_bf16": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int,
@@ -345,8 +346,8 @@ def device_arch() -> str:
 
 
 # ------------------------------------------------------------------------------------------------
-def embed(table, tokens, out):
-    """out[t, :] = table[tokens[t], :] widened to float32."""
+def embed(table, tokens, out, factor=1.0):
+    """out[t, :] = table[tokens[t], :] * factor, widened to float32."""
     _dev(table, tokens, out)
     n, dim = out.shape
     if not (table.dim() == 2 and table.shape[1] == dim and table.is_contiguous()):
@@ -354,11 +355,11 @@ def embed(table, tokens, out):
     if not (out.dtype == torch.float32 and out.is_contiguous()):
         raise KernelError("embed: out must be contiguous float32")
     _i32(tokens, "embed: tokens", n)
-    _call("gi_embed", table.data_ptr(), _code(table, "embed: table"), tokens.data_ptr(), out.data_ptr(), n, dim, _stream())
+    _call("gi_embed", table.data_ptr(), _code(table, "embed: table"), tokens.data_ptr(), out.data_ptr(), n, dim, float(factor), _stream())
     return out
 
 
-def embed_handing(table, tokens, out, g, scaled, squares):
+def embed_handing(table, tokens, out, g, scaled, squares, factor=1.0):
     """`embed`, and on the way the first half of an RMS norm of the rows for a product that finishes it (`gemm_bf16(..., norm_in=...)`):
     scaled = bfloat16(g * out) and squares [n, 1] = the rows' sums of out^2."""
     _dev(table, tokens, out, g, scaled, squares)
@@ -369,7 +370,7 @@ def embed_handing(table, tokens, out, g, scaled, squares):
             and scaled.is_contiguous() and squares.dtype == torch.float32 and squares.is_contiguous() and squares.shape == (n, 1)):
         raise KernelError("embed: handing a norm on needs float32 weights [dim], bfloat16 [n, dim] for the scaled rows and float32 [n, 1] for the sums of squares")
     _i32(tokens, "embed: tokens", n)
-    _call("gi_embed_handing", table.data_ptr(), _code(table, "embed: table"), tokens.data_ptr(), out.data_ptr(), n, dim, g.data_ptr(), scaled.data_ptr(),
+    _call("gi_embed_handing", table.data_ptr(), _code(table, "embed: table"), tokens.data_ptr(), out.data_ptr(), n, dim, float(factor), g.data_ptr(), scaled.data_ptr(),
           squares.data_ptr(), _stream())
     return out
 
@@ -1237,6 +1238,31 @@ def latent_queries(q, cos, sin, plain, folded, n_heads, dim, rot, kv_rank, half_
                 raise KernelError("latent_queries: cos/sin must be float32 [n, rot/2]")
     _call("gi_latent_queries", q.data_ptr(), q.stride(0), _ptr(cos), _ptr(sin), plain.data_ptr(), _code(plain, "latent_queries: plain"), plain.stride(0),
           folded.data_ptr(), _code(folded, "latent_queries: folded"), folded.stride(0), n, n_heads, dim, rot, kv_rank, 1 if half_split else 0, _stream())
+
+
+@lru_cache(maxsize=None)
+def _latent_fold_takes(n, n_heads, dim, rot, kv_rank) -> bool:
+    return bool(lib().gi_latent_fold_takes(n, n_heads, dim, rot, kv_rank))
+
+
+def latent_fold(q, cos, sin, w, folded, n_heads, dim, rot, kv_rank, half_split=False):
+    """`latent_queries` and `heads_product` of the unrotated channels with w bfloat16 [heads, kv_rank, dim], in one launch and with their bits: folded bfloat16
+    [n, heads*(kv_rank + rot)].  For a few rows: False, and nothing done, where the kernel does not take the operands."""
+    _dev(q, cos, sin, w, folded)
+    n = q.shape[0]
+    if not (w.dtype == torch.bfloat16 and folded.dtype == torch.bfloat16 and w.shape == (n_heads, kv_rank, dim) and w.is_contiguous() and q.stride(0) % 4 == 0
+            and (q.data_ptr() | w.data_ptr()) % 16 == 0 and _latent_fold_takes(n, n_heads, dim, rot, kv_rank)):
+        return False
+    if not (q.dtype == torch.float32 and q.shape == (n, n_heads * (dim + rot)) and q.stride(1) == 1 and folded.shape == (n, n_heads * (kv_rank + rot)) and folded.stride(1) == 1):
+        raise KernelError("latent_fold: q must be float32 [n, heads*(dim+rot)], folded [n, heads*(kv_rank+rot)]")
+    if rot:
+        for t in (cos, sin):
+            if not (t.dtype == torch.float32 and t.shape == (n, rot // 2) and t.is_contiguous()):
+                raise KernelError("latent_fold: cos/sin must be float32 [n, rot/2]")
+    if _profile is not None:
+        _profile.note = (f"{n_heads}x{kv_rank}x{dim}", w.numel() * w.element_size())
+    _call("gi_latent_fold", q.data_ptr(), q.stride(0), _ptr(cos), _ptr(sin), w.data_ptr(), folded.data_ptr(), folded.stride(0), n, n_heads, dim, rot, kv_rank, 1 if half_split else 0, _stream())
+    return True
 
 
 def latent_direct(q, kv, kv_norm, eps, cos, sin, positions, slots, table, plain, folded, cache, page_size, n_heads, dim, rot, kv_rank, half_split=False):

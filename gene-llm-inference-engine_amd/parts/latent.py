@@ -140,9 +140,11 @@ class LatentAttention(Mixer):
             down = torch.empty((T, self.w_down.shape[0]), dtype=torch.float32, device=dev)
             linear(h, self.w_down, down, ctx=ctx)
         cos, sin = (None, None) if self.position is None else self.position.half_split_tables(ctx) if self.half_split else self.position.pair_tables(ctx)
-        plain = torch.empty((T, H * s.head_dim), dtype=self.plain_dtype, device=dev)
+        new_plain = lambda: torch.empty((T, H * s.head_dim), dtype=self.plain_dtype, device=dev)
         folded = torch.empty((T, H * kd), dtype=cache.kv.dtype, device=dev)
+        plain = None                      # the queries' unrotated channels, where they are not folded yet
         if self.direct:
+            plain = new_plain()
             ops.latent_direct(down[:, :self.kv_at], down[:, self.kv_at:self.gate_at], self.kv_norm, s.norm_eps, cos, sin, ctx.row_pos, ctx.row_slot, cache.table, plain, folded,
                               cache.kv, cache.page_size, H, s.head_dim, s.rotary_dim, s.kv_rank, self.half_split)
         else:
@@ -151,8 +153,11 @@ class LatentAttention(Mixer):
                                cache.table, cq, cache.kv, cache.page_size, self.half_split)
             q = torch.empty((T, H * (s.head_dim + s.rotary_dim)), dtype=torch.float32, device=dev)
             linear(cq, self.w_uq, q, ctx=ctx)
-            ops.latent_queries(q, cos, sin, plain, folded, H, s.head_dim, s.rotary_dim, s.kv_rank, self.half_split)
-        heads_product(plain, self.w_uk_t, folded, H, kd)
+            if not (self.plain_dtype == torch.bfloat16 and ops.latent_fold(q, cos, sin, self.w_uk_t, folded, H, s.head_dim, s.rotary_dim, s.kv_rank, self.half_split)):
+                plain = new_plain()
+                ops.latent_queries(q, cos, sin, plain, folded, H, s.head_dim, s.rotary_dim, s.kv_rank, self.half_split)
+        if plain is not None:
+            heads_product(plain, self.w_uk_t, folded, H, kd)
         attended = torch.empty((T, H * s.kv_rank), dtype=cache.kv.dtype, device=dev)
         if cache.kv.dtype == torch.bfloat16 and ops.latent_attention_bf16_supports(kd, s.kv_rank, cache.page_size):
             ops.latent_attention_bf16(folded, cache.kv, attended, ctx, cache.table, H, kd, s.kv_rank, cache.page_size, s.window, s.scale, self.sinks)

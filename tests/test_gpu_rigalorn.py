@@ -309,6 +309,24 @@ def test_delta_rule_of_single_rows_needs_no_runs(channel):
         ops.delta_scan(qkv, gates, None, None, slot, state, out, heads, kv, dk, dv, channel=channel)
 
 
+@pytest.mark.parametrize("H,d,r,rank,n,half_split", [(32, 64, 32, 256, 5, False), (3, 40, 8, 36, 16, True), (1, 8, 0, 16, 1, False), (4, 136, 64, 500, 7, True)])
+def test_queries_of_a_few_rows_are_folded_in_one_launch(H, d, r, rank, n, half_split):
+    """The bits of the two launches, whole and ragged strips of 16 columns and pieces of 32 channels, with and without turned channels; what it does not take is left alone."""
+    from geneinfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(4)
+    q = torch.randn(n, H * (d + r) + 4, generator=g).to(DEV)[:, :H * (d + r)]
+    w = (torch.randn(H, rank, d, generator=g) * d ** -0.5).to(DEV, torch.bfloat16)
+    angle = torch.randn(n, max(r // 2, 1), generator=g).to(DEV)
+    cos, sin = (torch.cos(angle), torch.sin(angle)) if r else (None, None)
+    plain, want = torch.empty(n, H * d, dtype=torch.bfloat16, device=DEV), torch.full((n, H * (rank + r)), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.latent_queries(q, cos, sin, plain, want, H, d, r, rank, half_split)
+    assert ops.heads_product(plain, w, want, H, rank + r)
+    got = torch.full_like(want, 7.0)
+    assert ops.latent_fold(q, cos, sin, w, got, H, d, r, rank, half_split) and torch.equal(got, want)
+    many = torch.zeros(17, H * (d + r), device=DEV)
+    assert not ops.latent_fold(many, cos, sin, w, torch.empty(17, H * (rank + r), dtype=torch.bfloat16, device=DEV), H, d, r, rank, half_split)
+
+
 def _delta_inputs(lens, heads, kv, dv, seed, steps=None, spare=0):
     """Rows as `delta_prepare` leaves them: unit keys, queries of length 1/8, decays as at initialisation, and where given one step size for all."""
     g = torch.Generator().manual_seed(seed)
