@@ -174,21 +174,35 @@ struct TilePlaces {
     int run[16];
 };
 
-// Filled by the workgroup's first 128 threads (each row's page is two loads that depend on each other: done once per row here,
-// not once per piece of a row); the caller puts a barrier before the use.
-__device__ __forceinline__ void tile_places(TilePlaces& t, int m0, int M, const RopeStore& rs) {
-    const int row = threadIdx.x;
-    if (row >= 128) return;
+// One row's of it, for the row's thread (rows 64 .. and the threads of a wave go together; each row's page is two loads that depend on each other: done once per row here,
+// not once per piece of a row).
+struct RowPlace {
+    long page;
+    int place, run;
+};
+__device__ __forceinline__ RowPlace row_place(int row, int m0, int M, const RopeStore& rs) {
+    RowPlace t;
     const int m = min(m0 + row, M - 1), p = rs.pos[m], slot = rs.slot[m];
-    t.page[row] = (long)rs.table[(size_t)slot * rs.table_stride + p / rs.page_size] * rs.page_stride;
-    t.place[row] = p % rs.page_size;
+    t.page = (long)rs.table[(size_t)slot * rs.table_stride + p / rs.page_size] * rs.page_stride;
+    t.place = p % rs.page_size;
     bool begins = p % 8 == 0 && rs.page_size % 8 == 0 && row + 7 < 128 && m0 + row + 7 < M;
     if (begins) {
 #pragma unroll
         for (int i = 1; i < 8; ++i) begins = begins & (rs.pos[m + i] == p + i) & (rs.slot[m + i] == slot);
     }
     const unsigned here = (unsigned)(__ballot(begins) >> (row & 56)) & 0xffu;         // (two such rows are eight apart or more)
-    if ((row & 7) == 0) t.run[row >> 3] = here ? row + __ffs(here) - 1 : -1;
+    t.run = here ? (row & ~7) + __ffs(here) - 1 : -1;                                   // of the row's window
+    return t;
+}
+__device__ __forceinline__ void keep_place(TilePlaces& t, int row, const RowPlace& of) {
+    t.page[row] = of.page;
+    t.place[row] = of.place;
+    if ((row & 7) == 0) t.run[row >> 3] = of.run;
+}
+// Filled by the workgroup's first 128 threads; the caller puts a barrier before the use.
+__device__ __forceinline__ void tile_places(TilePlaces& t, int m0, int M, const RopeStore& rs) {
+    const int row = threadIdx.x;
+    if (row < 128) keep_place(t, row, row_place(row, m0, M, rs));
 }
 
 // A tile of 128 x 128 sums of a q/k/v product, row-major in LDS, goes where `RopeStore` says.  Whole heads lie inside the
@@ -609,7 +623,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_grouped_kernel(const bf16_t* __
 // of 16,384 gated 104.8 and 102.6 us, 2,048 rows 118.4 and 118.0, 3,000 rows 174.8 and 174.1, 8,192 rows 460 and 451.
 template <int BN, int EPI>
 __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ C,
-                                                                int M, int N, int K, long lda, long ldw, long ldc, NormIn norm_in) {
+                                                                int M, int N, int K, long lda, long ldw, long ldc, NormIn norm_in, RopeStore rope) {
     static_assert(BN == 256, "the sharing of the loads below is written for 256 x 256 tiles");
     constexpr int BM = 256, WAVES = 8, WM = 64, WN = BN / 2, TM = WM / 32, TN = WN / 32;
     constexpr int ROWS = BM + BN, A_BYTES = BM * 128, W_BYTES = BN * 128, LOADS = ROWS / 8 / WAVES;      // a wave-wide load fills 8 rows of 128 bytes
@@ -707,7 +721,14 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
             }
         }
     }
-    if (n_k > 1 && !(is_gated(EPI) && norm_in.squares != nullptr)) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    // Likewise where the rows' keys and values go.
+    [[maybe_unused]] RowPlace my_place = {0, 0, -1};
+    [[maybe_unused]] bool places_wanted = false;
+    if constexpr (EPI == EPI_QKV_ROPE) {
+        places_wanted = n0 + BN > rope.n_heads * rope.hd;                               // (a tile of queries alone needs no pages)
+        if (places_wanted && wave < 4) my_place = row_place(tid & 127, m0 + (tid & 128), M, rope);
+    }
+    if (n_k > 1 && !(is_gated(EPI) && norm_in.squares != nullptr) && !places_wanted) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     phase_barrier();
     if (group == 1) phase_barrier();            // group 1 runs one barrier behind group 0's phases
@@ -754,7 +775,10 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[step][j], a[step][i], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < TN; ++j) {
+                    if constexpr (EPI == EPI_QKV_ROPE) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[step][i], b[step][j], acc[i][j], 0, 0, 0);
+                    else acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[step][j], a[step][i], acc[i][j], 0, 0, 0);
+                }
         if (group == 0) {                                                           // the half of W sent for a block ago has landed
             if (more) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
             else if (last_rows) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
@@ -763,6 +787,33 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
         phase_barrier();
     }
     if (group == 0) phase_barrier();
+    if constexpr (EPI == EPI_QKV_ROPE) {
+        // The sums (element v of a lane's result: row 8*(v/4) + 4*(lane/32) + v%4, column lane%32) are laid into LDS as two tiles of 128 x 128, a group's 128 rows at a
+        // time, and leave rotated, queries to their rows, keys and values to their pages (some 8 us a tile beyond what stored ones take: 8,192 rows of 6,144 x 4,096 298 and 318 us).
+        TilePlaces* places = reinterpret_cast<TilePlaces*>(ring + 2 * 128 * 128 * 4);
+        static_assert(2 * 128 * 128 * 4 + 2 * sizeof(TilePlaces) <= 2 * A_BYTES + 3 * W_BYTES, "two tiles and their rows' places fit the ring");
+        if (places_wanted && wave < 4) keep_place(places[tid >> 7], tid & 127, my_place);
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            if (m0 + half * 128 >= M) break;
+            if (group == half) {
+                float* tile = reinterpret_cast<float*>(ring) + (wave & 1) * (128 * 128);
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v)
+                            tile[(wm - half * 128 + i * 32 + 8 * (v / 4) + 4 * (lane >> 5) + (v & 3)) * 128 + j * 32 + (lane & 31)] = acc[i][j][v];
+            }
+            __syncthreads();
+            const float* tiles = reinterpret_cast<const float*>(ring);
+            qkv_tile_rope_store<512>(tiles, places[half], m0 + half * 128, n0, M, N, rope);
+            qkv_tile_rope_store<512>(tiles + 128 * 128, places[half], m0 + half * 128, n0 + 128, M, N, rope);
+            __syncthreads();
+        }
+        return;
+    }
     float* row_scale = reinterpret_cast<float*>(ring + 2 * A_BYTES + W_BYTES);      // (behind what the waves' results pass through)
     if constexpr (is_gated(EPI)) {
         if (norm_in.squares != nullptr) {
@@ -2246,6 +2297,9 @@ static TallCut tall_cut(int M, int N, int K, bool may_share, bool clears) {
 static long tall_counter_floats(const TallCut& cut) { return (4L * cut.rest + 63) / 64 * 64; }
 static long tall_scratch_floats(const TallCut& cut) { return cut.shares > 1 ? tall_counter_floats(cut) + (long)cut.rest * cut.shares * 256 * 128 : 0; }
 
+// (the ping-pong kernel's rotated ends; 8 us a round leave out what is no faster.  33 products, 2,048 to 8,192 rows, in tiles of 256 x 128 or 128 x 128 and of 256 x 256: 4,096 rows of 3,072 x 2,048
+// 64.6 us and 52.9, 3,072 of 5,120 x 3,072 97.8 and 83.8, 8,192 of 6,144 x 4,096 368.9 and 317.6; of the 14 that it takes none gains less than 14 %)
+constexpr double ROPE_US = 8;
 struct LargeChoice { Large kernel; TallCut cut; };              // cut: how the tall kernel makes its tiles, where that is the one
 static LargeChoice large_kernel(int M, int N, int K, int epi, bool rope, bool hands_norm, bool scaled_rows, bool may_share, bool clears) {
     const long units = gi_compute_units(), m128 = (M + 127) / 128, m256 = (M + 255) / 256, n128 = (N + 127) / 128, n256 = (N + 255) / 256;
@@ -2262,7 +2316,7 @@ static LargeChoice large_kernel(int M, int N, int K, int epi, bool rope, bool ha
     double piped = small > 1 ? small * (blocks * 0.45 + ends.each) * (small > 2 ? 1.15 : 1) - ends.less : blocks * 0.65 + 10.5;      // (several: two workgroups a unit)
     if (scaled_rows && !rope) piped = 1e30;
     const TallCut whole = tall_cut(M, N, K, false, false), cut = tall_cut(M, N, K, may_share, clears);
-    const double pingpong = many && !rope ? rounds(m256 * n256) * (blocks * 1.45 + 14) : 1e30;
+    const double pingpong = many && !(rope && scaled_rows) ? rounds(m256 * n256) * (blocks * 1.45 + 14 + (rope ? ROPE_US : 0)) : 1e30;
     // (gating 256 x 128 sums at a time costs the tall kernel 3 us a round more: 1,500 rows by 16,384 of 2,048, three rounds of it against one and a
     // half of the ping-pong kernel: 114 us against 103.  Shares do not take its products: with 160 to 192 tiles a block takes it 1.3 us, and 4,096 rows of
     // 3,072 x 8,192 added took 182 with it and 198 shared, 1,368 of 8,192 x 6,784 stored 149 and 160)
@@ -2769,9 +2823,10 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
             raised = true;                                                                                                              \
         }                                                                                                                               \
         dim3 grid((N + 255) / 256, (M + 255) / 256);                                                                                    \
-        gemm_bf16_pingpong_kernel<256, EPI_><<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldw, ldc, norm_in); \
+        gemm_bf16_pingpong_kernel<256, EPI_><<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldw, ldc, norm_in, rope != nullptr ? *rope : NO_ROPE); \
     } while (0)
-        if (epi == EPI_STORE_F32) PINGPONG(EPI_STORE_F32); else if (epi == EPI_ADD_F32) PINGPONG(EPI_ADD_F32);
+        if (rope != nullptr) PINGPONG(EPI_QKV_ROPE);
+        else if (epi == EPI_STORE_F32) PINGPONG(EPI_STORE_F32); else if (epi == EPI_ADD_F32) PINGPONG(EPI_ADD_F32);
         else if (epi == EPI_XIELU) { norm_in.squares = norm_out.g; PINGPONG(EPI_XIELU); }
         else if (epi == EPI_STORE_BF16) PINGPONG(EPI_STORE_BF16); else if (epi == EPI_GATED_BF16) PINGPONG(EPI_GATED_BF16); else if (epi == EPI_GATED_GELU_BF16) PINGPONG(EPI_GATED_GELU_BF16); else PINGPONG(EPI_GATED_CLAMP_BF16);
 #undef PINGPONG

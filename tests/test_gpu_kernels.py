@@ -674,6 +674,32 @@ def test_qkv_product_that_rotates_and_fills_the_pages(m, hidden, n_heads, n_kv, 
     assert float((got_q.float() != want_q.float()).float().mean()) < 0.01 and float((got_cache.float() != want_cache.float()).float().mean()) < 0.01
 
 
+@pytest.mark.parametrize("m,hidden,n_heads,n_kv,hd,page_size,rotate", [(2500, 3072, 24, 8, 128, 16, True), (2390, 3072, 23, 8, 128, 12, True), (4000, 2048, 32, 8, 64, 16, True), (2330, 4096, 40, 4, 128, 24, False),
+                                                                       (2305, 3072, 128, 16, 32, 8, True)])
+def test_qkv_product_of_many_tiles_rotates_and_fills_the_pages(m, hidden, n_heads, n_kv, hd, page_size, rotate):
+    """Tiles of 256 x 256 whose halves of rows and of columns end anywhere: a last tile of one row, without a second half of rows or of columns; portions that begin anywhere, and single rows."""
+    o = ops()
+    n = (n_heads + 2 * n_kv) * hd
+    assert o.gemm_bf16_qkv_rope_store_takes(m, n, hidden, hd) and o.gemm_bf16_large_kernel(m, n, hidden, "rotated") == "256x256"
+    a, w = randn(m, hidden, dtype=torch.bfloat16, seed=1), randn(n, hidden, dtype=torch.bfloat16, seed=2, scale=hidden ** -0.5)
+    ang = 6.28 * torch.rand(m, hd // 2, generator=torch.Generator().manual_seed(9))
+    cos, sin = (torch.cos(ang).to(DEV), torch.sin(ang).to(DEV)) if rotate else (None, None)
+    starts, pos0 = [0, 1, 2, 3, 24, 1000, m], [5, 16, 7, 0, 701, 3]
+    positions = torch.cat([p + torch.arange(e - b, dtype=torch.int32) for b, e, p in zip(starts, starts[1:], pos0)]).to(DEV)
+    slots = torch.cat([torch.full((e - b,), i, dtype=torch.int32) for i, (b, e) in enumerate(zip(starts, starts[1:]))]).to(DEV)
+    pages = -(-(m + 800) // page_size)
+    table = torch.randperm(6 * pages, generator=torch.Generator().manual_seed(3)).view(6, pages).to(torch.int32).to(DEV)
+    want_cache, got_cache = (torch.full((6 * pages, 2, n_kv, page_size, hd), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    want_q, got_q = (torch.full((m + 1, n_heads * hd), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    qkv = (a.double() @ w.double().T).float()
+    a_dim, kv_dim = n_heads * hd, n_kv * hd
+    o.rope_store(qkv[:, :a_dim], qkv[:, a_dim:a_dim + kv_dim], qkv[:, a_dim + kv_dim:], cos, sin, positions, slots, table, want_q[:m], want_cache, n_heads, n_kv, hd)
+    o.gemm_bf16_qkv_rope_store(a, w, cos, sin, positions, slots, table, got_q[:m], got_cache, n_heads, n_kv, hd)
+    step = lambda t: t.float().abs() * 2.0 ** -7 + 2.0 ** -16             # a rounding step of bfloat16 at most, and what 32-bit sums of numbers about 1 may be off
+    for got, want in ((got_q, want_q), (got_cache, want_cache)):
+        assert ((got.float() - want.float()).abs() <= step(want)).all() and float((got.float() != want.float()).float().mean()) < 0.01
+
+
 @pytest.mark.parametrize("m,page_size,portions", [(2048, 16, [(0, 24, 0), (24, 1300, 701), (1324, 724, 3)]),      # single rows, then portions that begin anywhere
                                                   (1500, 16, [(0, 3, 0), (3, 9, 5), (12, 8, 16), (20, 1, 7), (21, 1479, 1000)]),
                                                   (2048, 12, [(0, 1000, 5), (1000, 1048, 0)]), (1410, 24, [(0, 1410, 23)])])
