@@ -91,7 +91,7 @@ GI_API int gi_embed(const void* table, int table_dtype, const int* tokens, float
 // The same for a step of a few rows whose first norm the product behind it finishes (see the products' `NormIn`): beside x the
 // row goes out times the norm's weights in bfloat16, and its sum of squares as one number.
 template <typename TT>
-__global__ __launch_bounds__(256) void embed_handing_kernel(const TT* __restrict__ table, const int* __restrict__ tokens, float* __restrict__ x, int dim, float factor,
+__global__ __launch_bounds__(256) void embed_handing_kernel(const TT* __restrict__ table, const int* __restrict__ tokens, float* __restrict__ x, int dim,
                                                             const float* __restrict__ g, bf16_t* __restrict__ scaled, float* __restrict__ squares) {
     __shared__ float red[4];
     const int t = blockIdx.x;
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256) void embed_handing_kernel(const TT* __restrict
     if (dim % 4 == 0 && (((uintptr_t)table | (uintptr_t)x | (uintptr_t)g | (uintptr_t)scaled) & 15) == 0) {      // four neighbouring channels a thread
         for (int d = threadIdx.x * 4; d < dim; d += 1024) {
             float v[4];
-            four_of(row + d, factor, v);
+            four_of(row + d, 1.0f, v);
             const float4 gd = *reinterpret_cast<const float4*>(g + d);
             *reinterpret_cast<float4*>(x + (size_t)t * dim + d) = float4{v[0], v[1], v[2], v[3]};
             *reinterpret_cast<uint2*>(scaled + (size_t)t * dim + d) = uint2{f32x2_to_bf16x2(gd.x * v[0], gd.y * v[1]), f32x2_to_bf16x2(gd.z * v[2], gd.w * v[3])};
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256) void embed_handing_kernel(const TT* __restrict
         }
     } else {
         for (int d = threadIdx.x; d < dim; d += 256) {
-            const float v = load_f32(row, d) * factor;
+            const float v = load_f32(row, d);
             x[(size_t)t * dim + d] = v;
             scaled[(size_t)t * dim + d] = f32_to_bf16(g[d] * v);
             sum = fmaf(v, v, sum);
@@ -118,13 +118,13 @@ __global__ __launch_bounds__(256) void embed_handing_kernel(const TT* __restrict
     if (threadIdx.x == 0) squares[t] = sum;
 }
 
-GI_API int gi_embed_handing(const void* table, int table_dtype, const int* tokens, float* x, int n_rows, int dim, float factor, const float* g, void* scaled,
+GI_API int gi_embed_handing(const void* table, int table_dtype, const int* tokens, float* x, int n_rows, int dim, const float* g, void* scaled,
                             float* squares, hipStream_t stream) {
     GI_REQUIRE(n_rows > 0 && dim > 0 && g != nullptr && scaled != nullptr && squares != nullptr, "embed: n_rows %d and dim %d must be positive, and the norm's operands given", n_rows, dim);
     if (table_dtype == GI_F32)
-        embed_handing_kernel<float><<<n_rows, 256, 0, stream>>>((const float*)table, tokens, x, dim, factor, g, (bf16_t*)scaled, squares);
+        embed_handing_kernel<float><<<n_rows, 256, 0, stream>>>((const float*)table, tokens, x, dim, g, (bf16_t*)scaled, squares);
     else if (table_dtype == GI_BF16)
-        embed_handing_kernel<bf16_t><<<n_rows, 256, 0, stream>>>((const bf16_t*)table, tokens, x, dim, factor, g, (bf16_t*)scaled, squares);
+        embed_handing_kernel<bf16_t><<<n_rows, 256, 0, stream>>>((const bf16_t*)table, tokens, x, dim, g, (bf16_t*)scaled, squares);
     else
         return gi_fail("embed: unknown table dtype %d", table_dtype);
     GI_CHECK_LAUNCH("embed");

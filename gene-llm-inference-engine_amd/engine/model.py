@@ -165,18 +165,15 @@ class DecoderModel:
         single rows of decoding requests in bfloat16, a norm of the form g * x * rsqrt(mean square + eps), a reader whose product
         finishes it), the kernel that fetches the rows does the norm's first half too and the `HandedRows` are returned; None otherwise."""
         first = self.layers[self.run_order[0].layer] if self.run_order else None
-        transforms = self.after_embedding
-        factor = 1.0                              # (a scale behind the token table is a factor of the fetch)
-        if transforms and type(transforms[0]) is ScaleRows and (len(transforms) == 1 or type(transforms[-1]) is not LearnedPositions):
-            factor, transforms = float(transforms[0].spec.factor), transforms[1:]
-        if (first is not None and not transforms and self.trace is None and self.dtype == torch.bfloat16 and self.before_entry[0] is None
+        if (first is not None and not self.after_embedding and self.trace is None and self.dtype == torch.bfloat16 and self.before_entry[0] is None
                 and getattr(first, "hands_norm_on", False) and ctx.max_seg_len == 1):         # (decode steps: the one norm kernel of a step that is all launches)
             norm = norm_to_hand_on(first.first_reader(), ctx.n_rows)
             if norm is not None:
                 scaled = torch.empty((ctx.n_rows, self.spec.hidden_size), dtype=torch.bfloat16, device=self.device)
                 squares = torch.empty((ctx.n_rows, 1), dtype=torch.float32, device=self.device)
-                ops.embed_handing(self.embedding, ctx.tokens, x, norm.handed_weight(), scaled, squares, factor)
+                ops.embed_handing(self.embedding, ctx.tokens, x, norm.handed_weight(), scaled, squares)
                 return HandedRows(norm, x, scaled, squares)
+        transforms = self.after_embedding
         # a scale and a table of positions behind the token table are one kernel with the fetch, which also leaves the rows as the
         # first product reads them where they are read without a norm
         if transforms and type(transforms[-1]) is LearnedPositions and all(type(t) is ScaleRows for t in transforms[:-1]):
@@ -193,8 +190,11 @@ class DecoderModel:
                 ctx.memo["token_rows"] = torch.empty_like(x)          # (the same kernel writes both)
             transforms[0].fetch(self.embedding, x, ctx, None if entry is None else cache.layer_cache(entry), ctx.memo.get("token_rows"))
             transforms = transforms[1:]
+        elif transforms and type(transforms[0]) is ScaleRows:         # (a factor of the fetch)
+            ops.embed(self.embedding, ctx.tokens, x, float(transforms[0].spec.factor))
+            transforms = transforms[1:]
         else:
-            ops.embed(self.embedding, ctx.tokens, x, factor)
+            ops.embed(self.embedding, ctx.tokens, x)
         for transform in transforms:
             if transform.needs_context:
                 transform(x, ctx)
