@@ -381,6 +381,11 @@ __device__ __forceinline__ void tile_old(TileOld<NT>& old, const float* C, long 
     for (int it = 0; it < 128 / (NT / 32); ++it)
         old.v[it] = *reinterpret_cast<const float4*>(C + (size_t)min(m0 + (int)(threadIdx.x >> 5) + it * (NT / 32), M - 1) * ldc + n0 + (threadIdx.x & 31) * 4);
 }
+// ... where N or the rows' stride need not be whole tiles or pieces: a lane whose four columns are not whole in the rows asks for nothing.
+template <int NT>
+__device__ __forceinline__ void tile_old_within(TileOld<NT>& old, const float* C, long ldc, int m0, int n0, int M, int N) {
+    if (n0 + (int)(threadIdx.x & 31) * 4 + 3 < N && (ldc & 3) == 0 && ((uintptr_t)C & 15) == 0) tile_old<NT>(old, C, ldc, m0, n0, M);
+}
 // ... with a norm handed on: the rows' new values, the same times the norm's weights in bfloat16, and the tile's piece of every row's
 // sum of squares (N is a multiple of 128).
 template <int NT>
@@ -562,7 +567,13 @@ __device__ __forceinline__ void piped_tile(const bf16_t* __restrict__ A, const b
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+        for (int j = 0; j < TN; ++j) {
+            [[maybe_unused]] float before[16];                                     // what sums are added onto, a result's sixteen at once (one by one 2,048 rows of 2,048 x 2,048 took 34.3 us for 30.0, 900 of 5,000 x 1,024 24.4 for 21.7)
+            if constexpr (EPI == EPI_ADD_F32) {
+                const int n = min(n0 + wn + j * 32 + (lane & 31), N - 1);
+#pragma unroll
+                for (int v = 0; v < 16; ++v) before[v] = ((const float*)C)[(size_t)min(m0 + wm + i * 32 + 8 * (v / 4) + 4 * (lane >> 5) + (v & 3), M - 1) * ldc + n];
+            }
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int m = m0 + wm + i * 32 + 8 * (v / 4) + 4 * (lane >> 5) + (v & 3);
@@ -571,12 +582,15 @@ __device__ __forceinline__ void piped_tile(const bf16_t* __restrict__ A, const b
                     const float up = __shfl_xor(acc[i][j][v], 16, 64);
                     if ((lane & 16) == 0 && m < M && n < N)
                         ((bf16_t*)C)[(size_t)m * ldc + (n >> 5) * 16 + (lane & 15)] = f32_to_bf16(gate_of<EPI>(acc[i][j][v], up, norm_in.limit));
+                } else if constexpr (EPI == EPI_ADD_F32) {
+                    if (m < M && n < N) ((float*)C)[(size_t)m * ldc + n] = before[v] + acc[i][j][v];
                 } else if constexpr (EPI != EPI_QKV_ROPE) {
                     float sum = acc[i][j][v];
                     if constexpr (EPI == EPI_XIELU) sum = xielu(sum, act_a, act_b);
                     if (m < M && n < N) write_out<EPI>(C, (size_t)m * ldc + n, sum);
                 }
             }
+        }
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int EPI>
@@ -900,8 +914,24 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
             }
         }
     } else {
+        // What the sums are added onto is asked for 32 columns ahead, all of a lane's rows at once (a row beyond M is clamped and not written): read row by row as each leaves,
+        // behind the store of the one before, it was 32 round trips to memory at the end of a tile.  8,192 rows of 4,096 x 4,096 added 231.9 -> 227.3 us, 4,096 of 4,096 x 14,336 366 -> 362.
+        constexpr int ROWS_OF_LANE = EPI == EPI_ADD_F32 ? WM / 8 : 1;
+        [[maybe_unused]] float4 before[2][ROWS_OF_LANE];
+        const bool rows_whole = (ldc & 3) == 0 && (((uintptr_t)C) & 15) == 0;
+        auto ask = [&](int j, float4 (&into)[ROWS_OF_LANE]) __attribute__((always_inline)) {
+            const int c = n0 + wn + j * 32 + fchunk * 4;
+            if (c + 3 < N && rows_whole) {
+#pragma unroll
+                for (int it = 0; it < ROWS_OF_LANE; ++it) into[it] = *reinterpret_cast<const float4*>((const float*)C + (size_t)min(m0 + wm + it * 8 + frow, M - 1) * ldc + c);
+            }
+        };
+        if constexpr (EPI == EPI_ADD_F32) ask(0, before[0]);
 #pragma unroll
         for (int j = 0; j < TN; ++j) {                                             // 32 columns = 128 bytes a row at a time
+            if constexpr (EPI == EPI_ADD_F32) {
+                if (j + 1 < TN) ask(j + 1, before[(j + 1) & 1]);
+            }
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -915,9 +945,9 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(const bf16_t* _
                 float4 v = *reinterpret_cast<const float4*>(mine + row * STAGE_ROW + fchunk * 16);
                 if (m >= M) continue;
                 float* dst = (float*)C + (size_t)m * ldc + c;
-                if (c + 3 < N && (ldc & 3) == 0 && (((uintptr_t)C) & 15) == 0) {
+                if (c + 3 < N && rows_whole) {
                     if constexpr (EPI == EPI_ADD_F32) {
-                        const float4 old = *reinterpret_cast<const float4*>(dst);
+                        const float4 old = before[j & 1][it];
                         v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
                         *reinterpret_cast<float4*>(dst) = v;
                     } else {
@@ -1164,7 +1194,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
                         store_streaming((bf16_t*)C + at, uint2{f32x2_to_bf16x2(v.x, v.y), f32x2_to_bf16x2(v.z, v.w)});
                     } else {
                         if constexpr (EPI == EPI_ADD_F32) {
-                            const float4 o = *reinterpret_cast<const float4*>((const float*)C + at);
+                            const float4 o = old.v[it];
                             v.x += o.x; v.y += o.y; v.z += o.z; v.w += o.w;
                             *reinterpret_cast<float4*>((float*)C + at) = v;
                         } else {
@@ -1181,12 +1211,11 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
         }
         __syncthreads();
     };
-    const bool hands_norm = EPI == EPI_ADD_F32 && norm_out.scaled != nullptr;
     if (!part) {
         TileOld<NT> old[2];
-        if (hands_norm) {
-            tile_old<NT>(old[0], (const float*)C, ldc, m0, n0, M);
-            tile_old<NT>(old[1], (const float*)C, ldc, m0 + 128, n0, M);
+        if constexpr (EPI == EPI_ADD_F32) {                                              // (all of a thread's rows at once: row by row as each leaves 3,000 rows of 3,072 x 3,072 took 72.3 us for 68.2)
+            tile_old_within<NT>(old[0], (const float*)C, ldc, m0, n0, M, N);
+            tile_old_within<NT>(old[1], (const float*)C, ldc, m0 + 128, n0, M, N);
         }
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
@@ -1233,7 +1262,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_tall_kernel(const bf16_t* __res
             continue;
         }
         TileOld<NT> old;
-        if (hands_norm) tile_old<NT>(old, (const float*)C, ldc, m0 + half * 128, n0, M);
+        if constexpr (EPI == EPI_ADD_F32) tile_old_within<NT>(old, (const float*)C, ldc, m0 + half * 128, n0, M, N);
         if (tid == 0) start[turn_of] = others_came(counter + 1, shared.shares - 1) ? 0.f : __builtin_nanf("");
         __syncthreads();
         if (tid < 2) __hip_atomic_store(counter + tid, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // as the next product of the step wants them
@@ -2268,7 +2297,7 @@ static bool many_tiles(int M, int N) { return (long)((M + 255) / 256) * ((N + 25
 // soonest where its sums leave as they are or through LDS (stored, rotated, added with a norm handed on) and latest where they are added one by
 // one: at short k several rounds of those are the faster ones (2,600 rows of 4,096 x 512 stored: 21 us in three, 25.5 with 256 x 128 in two; of
 // 4,096 x 1,536 the same either way; 2,048 rows of 5,120 x 1,024 rotated 36 and 42).  Only the two larger tiles finish a
-// norm handed on to a gated product; the q/k/v product's epilogue rotates tiles 128 columns wide.
+// norm handed on to a gated product; the q/k/v product takes one handed on in tiles of 128 columns alone.
 enum Large { PIPED_128, TALL_256, PINGPONG_256 };
 
 // How the tall kernel's tiles are made (`TileShares`): a last round of at most half as many tiles as there are compute units in shares of k, where
@@ -2631,7 +2660,9 @@ static int launch_strips(const void* A, const void* W, void* C, int epi, int M, 
     const int splits = cut.splits, k_per_split = splits == 0 ? K : (K / PK + splits - 1) / splits * PK;
     const int tile_rows = (M + cut.tiles - 1) / cut.tiles;
     dim3 grid((N + 63) / 64, splits == 0 ? 1 : splits, cut.tiles);
-    const int turn = turn_of_steps(k_per_split / PK);
+    // Places of their own in k (`first_step`): where k is shared out too, up to 160 rows (54 products 2 % faster in the mean, 64 rows of 2,048 x 2,048 11.2 us -> 10.0, 131 of 2,048 x 8,192 18.1 -> 17.6),
+    // but not above, where 42 products were 0.5 % slower (200 rows of 4,096 x 14,336 48.1 and 50.6).
+    const int turn = splits != 0 && M > 160 ? 0 : turn_of_steps(k_per_split / PK);
 #define STRIP(TM_, ST_, EPI_, PARTIAL_)                                                                                                 \
     do {                                                                                                                                \
         constexpr int bytes = strip_bytes(TM_, ST_);                                                                                    \
