@@ -1942,10 +1942,15 @@ __global__ __launch_bounds__(256) void skinny_reduce_rope_store_kernel(const flo
 //   128,256 x 2,048 stored      84.4, 77.7      98.7, 80.9      100.9, 93.1
 //   1,024 x 512 stored          2.2, 2.4        2.5, 2.6        2.7, 2.9
 // HAND: with the two halves of a norm handed from product to product (`NormIn`, `NormOut` above).
-// Strides come in pieces of 16 bytes, so that all that the first loads need is in the registers that are filled with the launch.
-template <int GROUPS, int EPI, bool HAND, int XT>
-__global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int lda8, int ldw8, int M, int N, int K, int rows, int turn,
+// Strides come in pieces of 16 bytes, so that all that the first loads need is in the registers that are filled with the launch.  FAR: rows so far apart that 64 bits are needed to
+// reckon with them (`slim_reach`).
+template <bool FAR> struct SlimPlaces { typedef int Stride; typedef unsigned At; };
+template <> struct SlimPlaces<true> { typedef long Stride; typedef size_t At; };
+template <int GROUPS, int EPI, bool HAND, int XT, bool FAR = false>
+__global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, typename SlimPlaces<FAR>::Stride lda8,
+                                                                typename SlimPlaces<FAR>::Stride ldw8, int M, int N, int K, int rows, int turn,
                                                                 void* __restrict__ C, long ldc, NormIn norm_in, NormOut norm_out) {
+    typedef typename SlimPlaces<FAR>::At At;
     constexpr bool GATED = is_gated(EPI);                              // the weights are 16 gates, their 16 ups, and so on
     constexpr int DEPTH = GROUPS == 1 ? 4 : GROUPS == 2 ? 4 : 2;
     static_assert(!GATED || GROUPS == 2 || GROUPS == 4, "as many groups of gates as of ups");
@@ -1960,17 +1965,18 @@ __global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __
     // beyond K become zeros.
     const int base = GATED ? (blockIdx.x / (4 / GROUPS)) * 32 + (blockIdx.x % (4 / GROUPS)) * 8 : blockIdx.x * rows;
     const bf16_t* w_base[GROUPS];
-    // Where the lane's rows begin, in pieces of 16 bytes, or in bytes where the registers are scarce (one 32-bit distance from a scalar address; the host sees to strides that it holds).
+    // Where the lane's rows begin, in pieces of 16 bytes, or in bytes where the registers are scarce (one 32-bit distance from a scalar address; the host sees to it that it holds
+    // a row's place and the one in k behind it).
     constexpr int PIECE = GROUPS == 4 ? 1 : 16;
-    unsigned w_at[GROUPS], x_at[XT];
+    At w_at[GROUPS], x_at[XT];
 #pragma unroll
     for (int g = 0; g < GROUPS; ++g) {
         w_base[g] = W + 8 * ((size_t)(base + (GATED ? 32 / GROUPS * g : 0)) * ldw8);
         const int row = GATED ? r : min(8 * g + r, min(rows, N - base) - 1);
-        w_at[g] = ((unsigned)row * (unsigned)ldw8 + k_lane / 8) * (16 / PIECE);
+        w_at[g] = ((At)row * (At)ldw8 + k_lane / 8) * (16 / PIECE);
     }
 #pragma unroll
-    for (int t = 0; t < XT; ++t) x_at[t] = ((unsigned)min(8 * t + r, M - 1) * (unsigned)lda8 + k_lane / 8) * (16 / PIECE);
+    for (int t = 0; t < XT; ++t) x_at[t] = ((At)min(8 * t + r, M - 1) * (At)lda8 + k_lane / 8) * (16 / PIECE);
     const int k_last = K - 8 - k_lane;                                 // the last 16 bytes of a row, from `w_row` and `x_row`
     const int steps = (K + 63) / 64, first = first_step(turn);
     const int mine = (steps - wave + 7) / 8;                           // of this wave
@@ -1980,8 +1986,8 @@ __global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __
     };
     uint4 w_buf[DEPTH][GROUPS], x_buf[DEPTH][XT];
     auto fetch = [&](int i, uint4 (&w)[GROUPS], uint4 (&x)[XT]) __attribute__((always_inline)) {
-        const unsigned at = (unsigned)((min(place(i), k_last) >> 3) * (16 / PIECE));         // (below 0 for a lane beyond a K under 64: the sums with it are not)
-        auto whereof = [](const bf16_t* p, unsigned pieces) { return (const bf16_t*)((const char*)p + (PIECE == 1 ? (size_t)pieces : (size_t)pieces * PIECE)); };
+        const At at = (At)((min(place(i), k_last) >> 3) * (16 / PIECE));         // (below 0 for a lane beyond a K under 64: the sums with it are not)
+        auto whereof = [](const bf16_t* p, At pieces) { return (const bf16_t*)((const char*)p + (PIECE == 1 ? (size_t)pieces : (size_t)pieces * PIECE)); };
 #pragma unroll
         for (int t = 0; t < XT; ++t) x[t] = load16(whereof(A, x_at[t] + at));
 #pragma unroll
@@ -2569,6 +2575,22 @@ static int slim_strip_rows(int M, int N, int epi) {
 //   65,536 x 512 stored      15.1, 14.9     15.2, 15.2     15.3, 18.0     15.5, 18.3
 static bool strips_in_registers(int M, int K, int epi) { return M <= 8 || (M <= 16 && (is_gated(epi) || K > 512)); }
 
+// How the slim kernel reaches rows so far apart.  It adds a row's place and the one in k behind it in 32 bits: in bytes for more than 24 weight rows a workgroup, in pieces of
+// 16 bytes for fewer, so the end of the last row that a workgroup reads, from its first, has to lie within.  Beyond the former fewer weight rows a workgroup, beyond the latter
+// (68 GB) the variant that reckons in 64 bits, of which there is one for each kind of end.
+struct SlimReach { int rows; bool far; };
+static SlimReach slim_reach(int M, int N, int K, int epi, long lda, long ldw) {
+    int rows = slim_strip_rows(M, N, epi);
+    auto pieces = [&]() {
+        const long apart = is_gated(epi) ? 7 : min(rows, N) - 1, w = apart * (ldw / 8), a = (M - 1) * (lda / 8);       // (gated: every group of 8 rows has an address of its own)
+        return (w > a ? w : a) + K / 8;
+    };
+    const int fewer = is_gated(epi) ? 16 : 24;
+    if (rows > 24 && pieces() > 1L << 28) rows = fewer;
+    const bool far = pieces() > 1L << 32;
+    return {far && rows > fewer ? fewer : rows, far};
+}
+
 static int slim_parts(int M, int N) {
     const int rows = slim_strip_rows(M, N, EPI_ADD_F32);
     return (N + rows - 1) / rows;
@@ -2577,12 +2599,18 @@ static int slim_parts(int M, int N) {
 static int launch_slim(const void* A, const void* W, void* C, int epi, int M, int N, int K, long lda, long ldw, long ldc, NormIn norm_in,
                        NormOut norm_out, hipStream_t stream) {
     const bool hand = norm_in.squares != nullptr || (norm_out.scaled != nullptr && epi != EPI_XIELU);
-    int rows = slim_strip_rows(M, N, epi);
-    // The kernel reckons distances between rows in 32 bits: in bytes for 32 weight rows, in pieces of 16 bytes for fewer.
-    if (rows > 24 && (31 * ldw * 2 >= 1l << 32 || 15 * lda * 2 >= 1l << 32)) rows = is_gated(epi) ? 16 : 24;
-    GI_REQUIRE((N == 1 || 31 * (ldw / 8) < 1l << 32) && (M == 1 || 15 * (lda / 8) < 1l << 32), "gemm_bf16: rows %ld and %ld elements apart are not taken", lda, ldw);
+    const auto [rows, far] = slim_reach(M, N, K, epi, lda, ldw);
     const dim3 grid((N + rows - 1) / rows);
     const int turn = turn_of_steps((K + 63) / 64);
+    if (far) {
+#define SLIM_FAR(GROUPS_, EPI_) gemm_bf16_slim_kernel<GROUPS_, EPI_, true, 2, true><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, lda / 8, ldw / 8, M, N, K, rows, turn, C, ldc, norm_in, norm_out)
+        if (epi == EPI_GATED_BF16) SLIM_FAR(2, EPI_GATED_BF16); else if (epi == EPI_GATED_GELU_BF16) SLIM_FAR(2, EPI_GATED_GELU_BF16); else if (is_gated(epi)) SLIM_FAR(2, EPI_GATED_CLAMP_BF16);
+        else if (epi == EPI_STORE_F32) SLIM_FAR(3, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM_FAR(3, EPI_ADD_F32);
+        else if (epi == EPI_XIELU) SLIM_FAR(3, EPI_XIELU); else SLIM_FAR(3, EPI_STORE_BF16);
+#undef SLIM_FAR
+        GI_CHECK_LAUNCH("gemm_bf16 (slim, far)");
+        return 0;
+    }
 #define SLIM_XT(GROUPS_, EPI_, XT_)                                                                                                                    \
     do {                                                                                                                                               \
         if (hand) gemm_bf16_slim_kernel<GROUPS_, EPI_, true, XT_><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, (int)(lda / 8), (int)(ldw / 8), M, N, K, rows, turn, C, ldc, norm_in, norm_out); \
@@ -3060,6 +3088,13 @@ GI_API int gi_gemm_bf16_small_kernel(int M, int N, int K, int gated) {
     if (takes_slim_tiles(M, N, K, gated ? EPI_GATED_BF16 : EPI_STORE_F32)) return 1;
     const int splits = gi_gemm_bf16_skinny_splits(N, K);
     return splits == 0 ? ends_in_strips(M, N, K) ? 2 : 3 : shared_strips(M, N, K, splits).tiles ? 2 : 3;
+}
+
+// How a product of at most 16 rows that the slim kernel makes reaches rows lda and ldw elements apart (`slim_reach`): weight rows a workgroup, and 100 more where it reckons in 64 bits.
+GI_API int gi_gemm_bf16_slim_reach(int M, int N, int K, int gated, int accumulate, long lda, long ldw) {
+    if (M <= 0 || M > 16 || N <= 0 || K <= 0) return -1;
+    const SlimReach reach = slim_reach(M, N, K, gated ? EPI_GATED_BF16 : accumulate ? EPI_ADD_F32 : EPI_STORE_F32, lda, ldw);
+    return reach.rows + (reach.far ? 100 : 0);
 }
 
 // How strips make a product whose k is shared out: 100 times the tiles of rows and the shares of k (at most 16); 0 where they do not.

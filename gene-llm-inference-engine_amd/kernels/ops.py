@@ -181,6 +181,8 @@ def lib():
         l.gi_gemm_bf16_small_kernel.restype = c_int
         l.gi_gemm_bf16_strip_cut.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_bf16_strip_cut.restype = c_int
+        l.gi_gemm_bf16_slim_reach.argtypes = [c_int, c_int, c_int, c_int, c_int, c_long, c_long]
+        l.gi_gemm_bf16_slim_reach.restype = c_int
         l.gi_gemm_bf16_onto_norm_takes.argtypes = [c_int, c_int, c_int]
         l.gi_gemm_bf16_onto_norm_takes.restype = c_int
         l.gi_gemm_bf16_xielu_takes.argtypes = [c_int, c_int, c_int, c_int]
@@ -1994,6 +1996,12 @@ def gemm_bf16_small_kernel(m, n, k, gated=False):
     """Which kernel makes a product of up to 128 rows (None: more rows): "slim", "slim tiles", "strips" or "streamed" (weights through registers)."""
     which = lib().gi_gemm_bf16_small_kernel(m, n, k, 1 if gated else 0)
     return None if which < 0 else ("slim", "slim tiles", "strips", "streamed")[which]
+
+
+def gemm_bf16_slim_reach(m, n, k, lda, ldw, gated=False, accumulate=False):
+    """(weight rows a workgroup, whether places are reckoned in 64 bits) of a product of up to 16 rows that "slim" makes, for rows lda and ldw elements apart."""
+    far, rows = divmod(lib().gi_gemm_bf16_slim_reach(m, n, k, 1 if gated else 0, 1 if accumulate else 0, lda, ldw), 100)
+    return rows, bool(far)
 
 
 @lru_cache(maxsize=8192)

@@ -421,6 +421,49 @@ def test_gemm_bf16_few_rows_at_every_height(m, n, k):
         assert bool((gated[m:] == 3.0).all()) and bool((gated[:, cols:] == 3.0).all())
 
 
+@pytest.mark.parametrize("m,n,k,lda8,reach", [(16, 8192, 256, ((1 << 28) - 32) // 15, (32, False)), (16, 8192, 256, ((1 << 28) - 32) // 15 + 1, (24, False)), (16, 8192, 264, ((1 << 32) - 33) // 15, (24, False)),
+                                              (16, 6144, 264, ((1 << 32) - 33) // 15 + 1, (24, True)), (16, 300, 56, ((1 << 32) - 7) // 15 + 1, (8, True))])
+def test_gemm_bf16_few_rows_far_apart(m, n, k, lda8, reach):
+    """Rows of A that the ends of 32 bits lie in, 4.3 and 68.7 GB behind the first: stored, added with a norm taken and handed on, gated, through xielu, and weight rows so far apart.
+    (Weights of a multiple of 64 of k beyond 12,288 columns go another way, which takes no such rows.)"""
+    o = ops()
+    assert o.gemm_bf16_slim_reach(m, n, k, 8 * lda8, k) == reach
+    torch.cuda.empty_cache()
+    far = torch.as_strided(torch.empty(8 * lda8 * (m - 1) + k, dtype=torch.bfloat16, device=DEV), (m, k), (8 * lda8, 1))
+    far.copy_(randn(m, k, dtype=torch.bfloat16, seed=1))
+    a, w, x0 = far.contiguous(), randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.1), randn(m, n, seed=3)
+    want = a.double() @ w.double().T
+    out, x, low = torch.full((m + 1, n + 3), 3.0, device=DEV), x0.clone(), torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    o.gemm_bf16(far, w, out[:m, :n])
+    o.gemm_bf16(far, w, x, accumulate=True)
+    o.gemm_bf16(far, w, low)
+    assert rel(out[:m, :n], want) < 2e-6 and rel(x, x0.double() + want) < 2e-6 and rel(low, want) < 4.1e-3
+    assert bool((out[m:] == 3.0).all()) and bool((out[:, n:] == 3.0).all())
+    cols = n // 32 * 16
+    gate, up = want[:, :2 * cols].reshape(m, cols // 16, 2, 16).unbind(2)
+    gated = torch.full((m + 1, cols + 2), 3.0, dtype=torch.bfloat16, device=DEV)
+    o.gemm_bf16(far, w[:2 * cols], gated[:m, :cols], gated=True)
+    assert rel(gated[:m, :cols], (torch.nn.functional.silu(gate) * up).reshape(m, cols)) < 4.1e-3 and bool((gated[m:] == 3.0).all()) and bool((gated[:, cols:] == 3.0).all())
+    if reach[1]:
+        weights = far[::m - 1]                                             # (the first row and the last as weight rows)
+        assert o.gemm_bf16_slim_reach(1, 2, k, k, weights.stride(0)) == (8, True)
+        o.gemm_bf16(a[:1], weights, out[:1, :2])
+        assert rel(out[:1, :2], a[:1].double() @ a[::m - 1].double().T) < 2e-6
+        mid, mid_near, params = torch.empty(m, n, dtype=torch.bfloat16, device=DEV), torch.empty(m, n, dtype=torch.bfloat16, device=DEV), torch.tensor([0.3, -0.2], device=DEV)
+        o.gemm_bf16_xielu(far, w, params, mid)
+        o.gemm_bf16_xielu(a, w, params, mid_near)
+        assert torch.equal(mid, mid_near)                                  # (as many weight rows a workgroup: the same sums)
+        squares, g = torch.rand(m, 3, device=DEV) * k, torch.rand(n, device=DEV)
+        results = []
+        for rows in (far, a):
+            y, scaled, pieces = x0.clone(), torch.empty(m, n, dtype=torch.bfloat16, device=DEV), torch.zeros(m, o.gemm_bf16_norm_parts(m, n, k), device=DEV)
+            o.gemm_bf16(rows, w, y, accumulate=True, norm_in=(squares, 1e-5), norm_out=(g, scaled, pieces))
+            results.append((y, scaled, pieces))
+        assert all(torch.equal(got, beside) for got, beside in zip(*results))
+    del far
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("m,parts", [(1, 512), (8, 300), (9, 256), (16, 3), (17, 256), (32, 2), (33, 8), (64, 1), (128, 5)])
 def test_gemm_bf16_strips_finish_a_norm(m, parts):
     n, k = 28672, 3072                                                     # (strips from one row on)

@@ -53,6 +53,26 @@ def test_the_faster_kernel_is_chosen_for_few_rows(m, n, k, gated, kernel):
     assert ops.gemm_bf16_small_kernel(m, n, k, gated) == kernel
 
 
+# rows, columns, k, distances between rows of either operand in pieces of 16 bytes (None: k), gated, added onto -> weight rows a workgroup, whether it reckons in 64 bits
+@pytest.mark.parametrize("m,n,k,lda8,ldw8,gated,added,reach", [
+    (16, 8192, 4096, None, None, False, False, (32, False)), (16, 8192, 4096, ((1 << 28) - 512) // 15, None, False, False, (32, False)), (16, 8192, 4096, ((1 << 28) - 512) // 15 + 1, None, False, False, (24, False)),
+    (16, 8192, 4096, (1 << 28) // 15, None, False, False, (24, False)), (9, 8192, 4096, ((1 << 28) - 512) // 8, None, False, False, (32, False)), (1, 8192, 4096, 1 << 40, None, False, False, (32, False)),
+    (16, 8192, 4096, ((1 << 32) - 512) // 15, None, False, False, (24, False)), (16, 8192, 4096, ((1 << 32) - 512) // 15 + 1, None, False, False, (24, True)), (2, 8192, 4096, 1 << 33, None, False, False, (24, True)),
+    (16, 16384, 4096, ((1 << 28) - 512) // 15, None, True, False, (32, False)), (16, 16384, 4096, ((1 << 28) - 512) // 15 + 1, None, True, False, (16, False)), (8, 16384, 4096, (1 << 32) // 7, None, True, False, (16, True)),
+    (4, 8192, 4096, None, ((1 << 28) - 512) // 31, False, False, (32, False)), (4, 8192, 4096, None, ((1 << 28) - 512) // 31 + 1, False, False, (24, False)),
+    (1, 2, 4096, None, (1 << 32) - 512, False, False, (8, False)), (1, 2, 4096, None, (1 << 32) - 511, False, False, (8, True)), (3, 1, 4096, None, 1 << 40, False, False, (8, False)),
+    (8, 4096, 4096, (1 << 32) // 7, None, False, True, (16, True)), (8, 4096, 4096, ((1 << 32) - 512) // 7, None, False, True, (16, False))])
+def test_few_rows_far_apart_are_reached(m, n, k, lda8, ldw8, gated, added, reach):
+    """The place of a row's last piece holds in the 32 bits that the kernel adds in, bytes or pieces; beyond them nothing is refused, and a sum of squares handed on has as many pieces as ever."""
+    lda8, ldw8 = lda8 or k // 8, ldw8 or k // 8
+    assert ops.gemm_bf16_slim_reach(m, n, k, 8 * lda8, 8 * ldw8, gated, added) == reach
+    rows, far = reach
+    last = max((m - 1) * lda8, (7 if gated else min(rows, n) - 1) * ldw8) + k // 8 - 1
+    assert far or last * (16 if rows > 24 else 1) < 1 << 32
+    if added:
+        assert -(-n // rows) == ops.lib().gi_gemm_bf16_norm_parts(m, n, k)
+
+
 # m, n, k -> tiles of rows and shares of k in strips, or None where the other kernels were the faster ones
 @pytest.mark.parametrize("m,n,k,cut", [(131, 3072, 8192, (1, 5)), (256, 3072, 8192, (1, 5)), (301, 2048, 2048, (4, 2)), (300, 3072, 8192, (5, 2)), (300, 3072, 20480, None), (300, 6144, 14336, None),
                                        (131, 10240, 2048, (3, 1)), (131, 10240, 6144, None), (129, 11264, 768, (1, 1)), (256, 11264, 768, None), (400, 500, 4096, (7, 4)), (900, 500, 8192, None),
