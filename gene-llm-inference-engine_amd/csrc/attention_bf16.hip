@@ -838,18 +838,28 @@ __global__ __launch_bounds__(ORDER_MAX_ROWS) void decode_order_kernel(const int*
     order[before] = row;
 }
 
-// PAGE16: pages of 16 positions, the usual ones, in which 16 channels' values lie in one piece and go past the caches.  (The kernel is not told more of it: with the size a
+// Heads of 64 and 128 channels: keys, and values of pages of 16 positions, go past the caches where nobody else reads them, which is faster then and slower where
+// somebody does: other rows of the same prompt (a short portion goes row by row), other requests that begin with the same pages, other groups of query heads.  LOOKS: there may be such, and a
+// wave looks for itself: does one of the four rows about its own read the page that it begins with?  (So it holds in a captured pass, whose tables are those of the step.  Looking costs
+// 0.2 to 0.5 us, so the caller asks for it only where it knows of portions or of requests that share their beginnings.)  Microseconds past the caches and through
+// them, in chains of caches of their own, 32 heads of 64 on 8 and 24 of 128 on 8:
+//   8 / 64 rows at 2,000 positions                        11.3, 12.5 / 49.0, 55.5      17.9, 20.0 / 96.1, 108.7
+//   32 rows of a portion behind 1,000 / 8,000             14.5, 11.2 / 60.4, 47.6      22.4, 16.8 / 111.5, 90.0
+//   8 / 32 rows at 2,000 that share 1,984 of them         13.5, 10.8 / 20.4, 16.7      19.4, 15.9 / 32.6, 26.7
+// PAGE16: pages of 16 positions, the usual ones, in which 16 channels' values lie in one piece.  (The kernel is not told more of it: with the size a
 // constant the compiler keeps addresses in 12 to 22 more registers, a wave of a SIMD's four or five.)
-// merged: [wave][gh][HD + 2] in LDS.
-template <int HD, bool FUSED, bool CAP, bool PAGE16>
+// step_rows: of the step, of which these rows are some.  shared: other workgroups read the row's keys and values too, whatever its neighbours do.  merged: [wave][gh][HD + 2] in LDS.
+template <int HD, bool FUSED, bool CAP, bool PAGE16, bool LOOKS>
 __device__ __forceinline__ void decode_rows(
-    float* merged, const DecodeItem& item,
+    float* merged, const DecodeItem& item, int step_rows, bool shared,
     const bf16_t* __restrict__ q, const float* __restrict__ qf, const float* __restrict__ kf, const float* __restrict__ vf, long ldq, long ldk,
     long ldv, const float* __restrict__ cos_t, const float* __restrict__ sin_t, bf16_t* __restrict__ cache, float* __restrict__ part,
     bf16_t* __restrict__ out, const int* __restrict__ rows, const int* __restrict__ pos, const int* __restrict__ slots,
     const int* __restrict__ table, int table_stride, long page_stride, int page_size, int n_heads, int n_kv, int window, float scale,
     int n_splits, int gh, const Extras& extra) {
     constexpr int KSTEPS = HD / 32, DT = HD / 16;
+    constexpr bool PAST_CACHES = !CAP && (HD == 64 || HD == 128);
+    static_assert(PAST_CACHES || !LOOKS, "nothing to look for");
     const int group = n_heads / n_kv, hg_per_kv = (group + 15) / 16;
     const int row = rows ? rows[item.row] : item.row, g = item.heads / hg_per_kv, hg = item.heads % hg_per_kv, split = item.split;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n_waves = blockDim.x >> 6;
@@ -874,14 +884,25 @@ __device__ __forceinline__ void decode_rows(
 #pragma unroll
         for (int s = 0; s < KSTEPS; ++s) q_raw[s] = load_pairs8(qf + (size_t)row * ldq + (size_t)(head_ok ? head : g * group) * HD, 32 * s + 8 * q4, HD / 2);
     }
-    const int my_pos = pos[row];
+    const int my_pos = pos[row], my_slot = slots[row];
+    [[maybe_unused]] int beside_slot[4], itself[4];               // of the rows about this one: at either end of the step one of them again, or the row itself (whose page then is none)
+    if constexpr (LOOKS) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int beside = min(max(row + (i < 2 ? i - 2 : i - 1), 0), step_rows - 1);
+            beside_slot[i] = slots[beside];
+            itself[i] = beside == row ? -1 : 0;
+        }
+    }
     const int lo = lowest_seen(my_pos, window, extra.chunk);
-    const int* tab = table + (size_t)__builtin_amdgcn_readfirstlane(slots[row]) * table_stride;
+    const int* tab = table + (size_t)__builtin_amdgcn_readfirstlane(my_slot) * table_stride;
     // every row cuts its own range into pieces (multiples of 32), one per wave of every split; short rows leave later pieces empty
     const int n_pieces = n_splits * n_waves, piece = split * n_waves + wave;
     const int span = my_pos + 1 - (lo & ~31);
     const int piece_len = (((span + n_pieces - 1) / n_pieces) + 31) & ~31;
     const int begin = (lo & ~31) + piece * piece_len, end = min(my_pos + 1, begin + piece_len);
+    if constexpr (LOOKS)          // (they come with the position and what the addresses of keys need)
+        asm volatile("" : "+s"(beside_slot[0]), "+s"(beside_slot[1]), "+s"(beside_slot[2]), "+s"(beside_slot[3]), "+s"(page_stride), "+s"(page_size), "+s"(table_stride), "+s"(n_kv));
     const int page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
     auto page_index = [&](int kv) { return page_shift >= 0 ? kv >> page_shift : kv / page_size; };
     auto place_of = [&](int kv) { return page_shift >= 0 ? kv & (page_size - 1) : kv % page_size; };
@@ -901,210 +922,275 @@ __device__ __forceinline__ void decode_rows(
     // (a page number fetched per lane is a vector load like the keys and values, and those come back in the order they were asked
     // for: waiting for it meant waiting for every key and value requested before it, several round trips to memory per tile).
     const int first_page = page_index(lo), last_page = page_index(my_pos);
+    auto page_of = [&](int kv) { return __builtin_amdgcn_readfirstlane(min(max(page_index(kv), first_page), last_page)); };
     auto pages_of = [&](int kv0, int (&pg)[2]) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t) pg[t] = tab[__builtin_amdgcn_readfirstlane(min(max(page_index(kv0 + 16 * t), first_page), last_page))];
-    };
-    uint4 k_a[2][KSTEPS], k_b[2][KSTEPS];
-    // Heads of 64 and 128 channels: a load brings 128 bytes of 8 positions' keys, whole cache lines that are used once; two of them hold 64 channels of 16 positions,
-    // whose halves change places before they are used (`rows_of_halves`).  A block of 16 positions is read whole, from one scalar address: what lies in its page beyond the
-    // row's own range is masked with its scores.
-    // (Caps of scores and heads of 256 channels leave no registers for that.)
-    constexpr bool LINES = !CAP && (HD == 64 || HD == 128);
-    const unsigned key_lane = LINES ? (lane & 7) * HD + 8 * q4 + 32 * ((lane >> 3) & 1) : r * HD + 8 * q4;
-    auto load_keys = [&](int kv0, const int (&pg)[2], uint4 (&dst)[2][KSTEPS]) {
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            if constexpr (HD == 256) {
-                const int kv = min(max(kv0 + 16 * t + r, lo), my_pos);
-                const bf16_t* krow = kbase + (long)pg[t] * page_stride + (long)place_of(kv) * HD + 8 * q4;
-#pragma unroll
-                for (int ks = 0; ks < KSTEPS; ++ks) dst[t][ks] = load16(krow + 32 * ks);
-                continue;
-            }
-            const bf16_t* block = kbase + (long)pg[t] * page_stride + (long)place_of(kv0 + 16 * t) * HD;
-#pragma unroll
-            for (int ks = 0; ks < KSTEPS; ++ks) {
-                if constexpr (LINES) dst[t][ks] = load16_once(block + key_lane + 8 * HD * (ks & 1) + 32 * (ks & ~1));
-                else dst[t][ks] = load16(block + key_lane + 32 * ks);
-            }
-        }
-    };
-    // The values of a tile are asked for behind the products of the tile before it (the first tile's behind its keys), into the
-    // registers those products have just read.  Slot e of a lane in the value product is key position kv0 + 16*(e/4) + 4*q4 + e%4.
-    uint2 vx[DT], vy[DT];
-    auto load_values = [&](int kv0, const int (&pg)[2]) {
-        const int kva = min(max(kv0 + 4 * q4, lo & ~3), my_pos & ~3), kvb = min(max(kv0 + 16 + 4 * q4, lo & ~3), my_pos & ~3);
-        const bf16_t* va = vbase + (long)pg[0] * page_stride + place_of(kva) + (long)r * page_size;
-        const bf16_t* vb = vbase + (long)pg[1] * page_stride + place_of(kvb) + (long)r * page_size;
-#pragma unroll
-        for (int i = 0; i < DT; ++i) {
-            const long at = (long)(16 * i) * page_size;
-            vx[i] = PAGE16 ? load8_once(va + at) : load8(va + at);
-            vy[i] = PAGE16 ? load8_once(vb + at) : load8(vb + at);
-        }
+        for (int t = 0; t < 2; ++t) pg[t] = tab[page_of(kv0 + 16 * t)];
     };
     int pg_cur[2] = {0, 0}, pg_nxt[2] = {0, 0};
-    if (begin < end) {
-        pages_of(begin, pg_cur);
-        pages_of(begin + 32, pg_nxt);
-        load_keys(begin, pg_cur, k_a);
-        load_values(begin, pg_cur);
-    }
-
-    bf16x8 qreg[KSTEPS];
-    uint4 own_key[KSTEPS];
-    bf16_t own_value[DT];
-    if constexpr (FUSED) {
-        // The row's own key and value (for the one wave whose piece ends at the row's position) are asked for when the first keys
-        // are on their way and rotated behind the queries: at heads of 128 channels queries, key and angles at once are 200
-        // registers a lane, which halves the waves a compute unit holds.
-        [[maybe_unused]] Pairs8 k_raw[KSTEPS];
-        [[maybe_unused]] float v_raw[DT];
-        if (has_own) {
+    [[maybe_unused]] bool once = false;
+    if constexpr (LOOKS) {
+        if (begin < end) {
+            pages_of(begin, pg_cur);
+            pages_of(begin + 32, pg_nxt);
+            const int at = page_of(begin);
+            int page[4];
 #pragma unroll
-            for (int ks = 0; ks < KSTEPS; ++ks) k_raw[ks] = load_pairs8(kf + (size_t)row * ldk + (size_t)g * HD, 32 * ks + 8 * q4, HD / 2);
+            for (int i = 0; i < 4; ++i) page[i] = table[(size_t)beside_slot[i] * table_stride + at];
+            asm volatile("" : "+s"(page[0]), "+s"(page[1]), "+s"(page[2]), "+s"(page[3]), "+s"(pg_cur[0]));          // (one after the other they would be four round trips)
+            int others = shared;
 #pragma unroll
-            for (int i = 0; i < DT; ++i) v_raw[i] = vf[(size_t)row * ldv + (size_t)g * HD + 16 * i + r];
-        }
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) qreg[s] = as_bf16x8(head_ok ? rotated8(q_raw[s], angles[s]) : uint4{0, 0, 0, 0});
-        if (has_own) {
-            bf16_t* page = cache + (long)tab[page_index(my_pos)] * page_stride;
-            const int place = place_of(my_pos);
-#pragma unroll
-            for (int ks = 0; ks < KSTEPS; ++ks) {
-                own_key[ks] = rotated8(k_raw[ks], angles[ks]);
-                if (r == 0 && hg == 0)
-                    *reinterpret_cast<uint4*>(page + (long)g * page_size * HD + (long)place * HD + 32 * ks + 8 * q4) = own_key[ks];
-            }
-#pragma unroll
-            for (int i = 0; i < DT; ++i) {
-                own_value[i] = f32_to_bf16(v_raw[i]);
-                if ((i & 3) == q4 && hg == 0) page[v_plane + ((long)g * HD + 16 * i + r) * page_size + place] = own_value[i];
-            }
-        }
-    } else {
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
-            uint4 v = {0, 0, 0, 0};
-            if (head_ok) v = load16(q + ((size_t)row * n_heads + head) * HD + 32 * s + 8 * q4);
-            qreg[s] = as_bf16x8(v);
+            for (int i = 0; i < 4; ++i) others |= (page[i] | itself[i]) == pg_cur[0];
+            once = others == 0;
         }
     }
-
+    // The walk over the keys, in registers that two of it leave no room for where it rotates too: it then looks at `once` for every tile, else it is two, one for each way.
+    constexpr int AT_EACH_LOAD = 0, PAST = 1, THROUGH = 2;
     floatx4 o[DT];
+    float m, l;
+    auto walk = [&](auto way) __attribute__((always_inline)) {
+        constexpr int WAY = decltype(way)::value;
+        if constexpr (LOOKS && WAY != AT_EACH_LOAD) asm volatile("; %0" ::"n"(WAY) : "memory");          // (nothing of the two is made one)
+        uint4 k_a[2][KSTEPS], k_b[2][KSTEPS];
+        // Heads of 64 and 128 channels (of these, where it is known here, past the caches only): a load brings 128 bytes of 8 positions' keys, whole cache lines; two of them hold 64 channels of 16 positions,
+        // whose halves change places before they are used (`rows_of_halves`).  A block of 16 positions is read whole, from one scalar address: what lies in its page beyond the
+        // row's own range is masked with its scores.
+        // (Caps of scores and heads of 256 channels leave no registers for that.)
+        constexpr bool LINES = PAST_CACHES && (HD == 64 || WAY != THROUGH);
+        const unsigned key_lane = LINES ? (lane & 7) * HD + 8 * q4 + 32 * ((lane >> 3) & 1) : r * HD + 8 * q4;
+        // Either way of loading asks for the same, so that the compiler counts the loads in flight behind them; what stands around keeps it from making one of the two.
+        auto either_way = [&](auto load) __attribute__((always_inline)) {
+            if constexpr (WAY != AT_EACH_LOAD) {
+                load(std::bool_constant<WAY == PAST>{});
+            } else if (__builtin_expect(once, 1)) {
+                asm volatile("; past the caches" ::: "memory");
+                load(std::true_type{});
+                asm volatile("; past the caches" ::: "memory");
+            } else {
+                asm volatile("; through the caches" ::: "memory");
+                load(std::false_type{});
+                asm volatile("; through the caches" ::: "memory");
+            }
+        };
+        auto load_piece = [&](auto past, const bf16_t* block, int ks) __attribute__((always_inline)) {
+            const bf16_t* piece = block + key_lane + (LINES ? 8 * HD * (ks & 1) + 32 * (ks & ~1) : 32 * ks);
+            if constexpr (decltype(past)::value) return load16_once(piece);
+            else return load16(piece);
+        };
+        auto load_keys = [&](int kv0, const int (&pg)[2], uint4 (&dst)[2][KSTEPS]) {
+            if constexpr (WAY == AT_EACH_LOAD) {
+                const bf16_t* block[2];                                               // (outside of what is there twice)
 #pragma unroll
-    for (int i = 0; i < DT; ++i) o[i] = floatx4{};
-    float m = -INFINITY, l = 0.f;
-    // One tile of 32 positions: its keys lie in `k_use`; with a tile behind it (NEXT), that tile's keys are requested into `k_fill`
-    // and the page numbers of the tile after that through the scalar unit; behind its products that tile's values.  No load of
-    // a tile is skipped by a lane or by a condition inside it, so the compiler counts the loads in flight: the scores wait for
-    // this tile's keys alone, the output's products for its values alone.
-    auto tile = [&](int kv0, auto next, uint4 (&k_use)[2][KSTEPS], uint4 (&k_fill)[2][KSTEPS]) __attribute__((always_inline)) {
-        constexpr bool NEXT = decltype(next)::value;
-        int pg_far[2] = {0, 0};
-        if constexpr (NEXT) pages_of(kv0 + 64, pg_far);
-        if constexpr (NEXT) load_keys(kv0 + 32, pg_nxt, k_fill);
-        if constexpr (LINES) {
+                for (int t = 0; t < 2; ++t) block[t] = kbase + (long)pg[t] * page_stride + (long)place_of(kv0 + 16 * t) * HD;
+                either_way([&](auto past) __attribute__((always_inline)) {
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+                    for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int ks = 0; ks < KSTEPS; ks += 2) rows_of_halves(k_use[t][ks], k_use[t][ks + 1]);
+                        for (int ks = 0; ks < KSTEPS; ++ks) dst[t][ks] = load_piece(past, block[t], ks);
+                });
+                return;
+            }
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                if constexpr (HD == 256) {
+                    const int kv = min(max(kv0 + 16 * t + r, lo), my_pos);
+                    const bf16_t* krow = kbase + (long)pg[t] * page_stride + (long)place_of(kv) * HD + 8 * q4;
+#pragma unroll
+                    for (int ks = 0; ks < KSTEPS; ++ks) dst[t][ks] = load16(krow + 32 * ks);
+                    continue;
+                }
+                const bf16_t* block = kbase + (long)pg[t] * page_stride + (long)place_of(kv0 + 16 * t) * HD;
+#pragma unroll
+                for (int ks = 0; ks < KSTEPS; ++ks) dst[t][ks] = load_piece(std::bool_constant<WAY == PAST>{}, block, ks);
+            }
+        };
+        // The values of a tile are asked for behind the products of the tile before it (the first tile's behind its keys), into the
+        // registers those products have just read.  Slot e of a lane in the value product is key position kv0 + 16*(e/4) + 4*q4 + e%4.
+        uint2 vx[DT], vy[DT];
+        auto load_values = [&](int kv0, const int (&pg)[2]) {
+            const int kva = min(max(kv0 + 4 * q4, lo & ~3), my_pos & ~3), kvb = min(max(kv0 + 16 + 4 * q4, lo & ~3), my_pos & ~3);
+            const bf16_t* va = vbase + (long)pg[0] * page_stride + place_of(kva) + (long)r * page_size;
+            const bf16_t* vb = vbase + (long)pg[1] * page_stride + place_of(kvb) + (long)r * page_size;
+            auto load = [&](auto past) __attribute__((always_inline)) {
+                constexpr bool ONCE = decltype(past)::value;
+#pragma unroll
+                for (int i = 0; i < DT; ++i) {
+                    const long at = (long)(16 * i) * page_size;
+                    vx[i] = ONCE ? load8_once(va + at) : load8(va + at);
+                    vy[i] = ONCE ? load8_once(vb + at) : load8(vb + at);
+                }
+            };
+            if constexpr (PAGE16) either_way(load);
+            else load(std::false_type{});
+        };
+        if (begin < end) {
+            if constexpr (!LOOKS) {
+                pages_of(begin, pg_cur);
+                pages_of(begin + 32, pg_nxt);
+            }
+            load_keys(begin, pg_cur, k_a);
+            load_values(begin, pg_cur);
         }
-        if constexpr (FUSED && !NEXT) {
-            if (has_own) {                                // the last tile of the piece: the row's own key and value go in
-                const int off = my_pos - kv0;             // 0 .. 31
+
+        bf16x8 qreg[KSTEPS];
+        uint4 own_key[KSTEPS];
+        bf16_t own_value[DT];
+        if constexpr (FUSED) {
+            // The row's own key and value (for the one wave whose piece ends at the row's position) are asked for when the first keys
+            // are on their way and rotated behind the queries: at heads of 128 channels queries, key and angles at once are 200
+            // registers a lane, which halves the waves a compute unit holds.
+            [[maybe_unused]] Pairs8 k_raw[KSTEPS];
+            [[maybe_unused]] float v_raw[DT];
+            if (has_own) {
+#pragma unroll
+                for (int ks = 0; ks < KSTEPS; ++ks) k_raw[ks] = load_pairs8(kf + (size_t)row * ldk + (size_t)g * HD, 32 * ks + 8 * q4, HD / 2);
+#pragma unroll
+                for (int i = 0; i < DT; ++i) v_raw[i] = vf[(size_t)row * ldv + (size_t)g * HD + 16 * i + r];
+            }
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) qreg[s] = as_bf16x8(head_ok ? rotated8(q_raw[s], angles[s]) : uint4{0, 0, 0, 0});
+            if (has_own) {
+                bf16_t* page = cache + (long)tab[page_index(my_pos)] * page_stride;
+                const int place = place_of(my_pos);
+#pragma unroll
+                for (int ks = 0; ks < KSTEPS; ++ks) {
+                    own_key[ks] = rotated8(k_raw[ks], angles[ks]);
+                    if (r == 0 && hg == 0)
+                        *reinterpret_cast<uint4*>(page + (long)g * page_size * HD + (long)place * HD + 32 * ks + 8 * q4) = own_key[ks];
+                }
+#pragma unroll
+                for (int i = 0; i < DT; ++i) {
+                    own_value[i] = f32_to_bf16(v_raw[i]);
+                    if ((i & 3) == q4 && hg == 0) page[v_plane + ((long)g * HD + 16 * i + r) * page_size + place] = own_value[i];
+                }
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) {
+                uint4 v = {0, 0, 0, 0};
+                if (head_ok) v = load16(q + ((size_t)row * n_heads + head) * HD + 32 * s + 8 * q4);
+                qreg[s] = as_bf16x8(v);
+            }
+        }
+
+#pragma unroll
+        for (int i = 0; i < DT; ++i) o[i] = floatx4{};
+        m = -INFINITY;
+        l = 0.f;
+        // One tile of 32 positions: its keys lie in `k_use`; with a tile behind it (NEXT), that tile's keys are requested into `k_fill`
+        // and the page numbers of the tile after that through the scalar unit; behind its products that tile's values.  No load of
+        // a tile is skipped by a lane or by a condition inside it, so the compiler counts the loads in flight: the scores wait for
+        // this tile's keys alone, the output's products for its values alone.
+        auto tile = [&](int kv0, auto next, uint4 (&k_use)[2][KSTEPS], uint4 (&k_fill)[2][KSTEPS]) __attribute__((always_inline)) {
+            constexpr bool NEXT = decltype(next)::value;
+            int pg_far[2] = {0, 0};
+            if constexpr (NEXT) pages_of(kv0 + 64, pg_far);
+            if constexpr (NEXT) load_keys(kv0 + 32, pg_nxt, k_fill);
+            if constexpr (LINES) {
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
-                    if ((off >> 4) == t && (off & 15) == r) {
 #pragma unroll
-                        for (int ks = 0; ks < KSTEPS; ++ks) k_use[t][ks] = own_key[ks];
-                    }
-                if (((off & 15) >> 2) == q4) {
-                    const int e = off & 3;
-                    const bool second = (off >> 4) != 0;
+                    for (int ks = 0; ks < KSTEPS; ks += 2) rows_of_halves(k_use[t][ks], k_use[t][ks + 1]);
+            }
+            if constexpr (FUSED && !NEXT) {
+                if (has_own) {                                // the last tile of the piece: the row's own key and value go in
+                    const int off = my_pos - kv0;             // 0 .. 31
 #pragma unroll
-                    for (int i = 0; i < DT; ++i) {
-                        const uint2 had = second ? vy[i] : vx[i];
-                        const uint32_t val = own_value[i];
-                        const uint32_t x = e == 0 ? (had.x & 0xffff0000u) | val : e == 1 ? (had.x & 0x0000ffffu) | (val << 16) : had.x;
-                        const uint32_t y = e == 2 ? (had.y & 0xffff0000u) | val : e == 3 ? (had.y & 0x0000ffffu) | (val << 16) : had.y;
-                        vx[i] = second ? vx[i] : uint2{x, y};
-                        vy[i] = second ? uint2{x, y} : vy[i];
+                    for (int t = 0; t < 2; ++t)
+                        if ((off >> 4) == t && (off & 15) == r) {
+#pragma unroll
+                            for (int ks = 0; ks < KSTEPS; ++ks) k_use[t][ks] = own_key[ks];
+                        }
+                    if (((off & 15) >> 2) == q4) {
+                        const int e = off & 3;
+                        const bool second = (off >> 4) != 0;
+#pragma unroll
+                        for (int i = 0; i < DT; ++i) {
+                            const uint2 had = second ? vy[i] : vx[i];
+                            const uint32_t val = own_value[i];
+                            const uint32_t x = e == 0 ? (had.x & 0xffff0000u) | val : e == 1 ? (had.x & 0x0000ffffu) | (val << 16) : had.x;
+                            const uint32_t y = e == 2 ? (had.y & 0xffff0000u) | val : e == 3 ? (had.y & 0x0000ffffu) | (val << 16) : had.y;
+                            vx[i] = second ? vx[i] : uint2{x, y};
+                            vy[i] = second ? uint2{x, y} : vy[i];
+                        }
                     }
                 }
             }
-        }
 
-        floatx4 s[2];
+            floatx4 s[2];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            s[t] = floatx4{};
+            for (int t = 0; t < 2; ++t) {
+                s[t] = floatx4{};
 #pragma unroll
-            for (int ks = 0; ks < KSTEPS; ++ks) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k_use[t][ks]), qreg[ks], s[t], 0, 0, 0);
-        }
-        // element v of s[t]: key position kv0 + 16*t + 4*q4 + v, query head r
-        if constexpr (CAP) {
+                for (int ks = 0; ks < KSTEPS; ++ks) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k_use[t][ks]), qreg[ks], s[t], 0, 0, 0);
+            }
+            // element v of s[t]: key position kv0 + 16*t + 4*q4 + v, query head r
+            if constexpr (CAP) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) s[t][v] = capped.of(s[t][v]);
+            }
+            float mx = -INFINITY;
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) s[t][v] = capped.of(s[t][v]);
-        }
-        float mx = -INFINITY;
+                for (int v = 0; v < 4; ++v) {
+                    const int kv = kv0 + 16 * t + 4 * q4 + v;
+                    s[t][v] = (kv >= lo && kv < end) ? s[t][v] * scale2 : -INFINITY;
+                    mx = fmaxf(mx, s[t][v]);
+                }
+            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            const float m_new = fmaxf(m, mx);
+            const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+            const float corr = exp2_fast(m - m_use);
+            float sum = 0.f;
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+            for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int kv = kv0 + 16 * t + 4 * q4 + v;
-                s[t][v] = (kv >= lo && kv < end) ? s[t][v] * scale2 : -INFINITY;
-                mx = fmaxf(mx, s[t][v]);
+                for (int v = 0; v < 4; ++v) {
+                    s[t][v] = exp2_fast(s[t][v] - m_use);
+                    sum += s[t][v];
+                }
+            sum += __shfl_xor(sum, 16, 64);
+            sum += __shfl_xor(sum, 32, 64);
+            l = l * corr + sum;
+            m = m_new;
+            const uint4 pb = {pack2(s[0][0], s[0][1]), pack2(s[0][2], s[0][3]), pack2(s[1][0], s[1][1]), pack2(s[1][2], s[1][3])};
+#pragma unroll
+            for (int i = 0; i < DT; ++i) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) o[i][v] *= corr;
+                o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(uint4{vx[i].x, vx[i].y, vy[i].x, vy[i].y}), as_bf16x8(pb), o[i], 0, 0, 0);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_new = fmaxf(m, mx);
-        const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-        const float corr = exp2_fast(m - m_use);
-        float sum = 0.f;
+            if constexpr (NEXT) {
+                load_values(kv0 + 32, pg_nxt);
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                s[t][v] = exp2_fast(s[t][v] - m_use);
-                sum += s[t][v];
+                for (int t = 0; t < 2; ++t) {
+                    pg_cur[t] = pg_nxt[t];
+                    pg_nxt[t] = pg_far[t];
+                }
             }
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
-        l = l * corr + sum;
-        m = m_new;
-        const uint4 pb = {pack2(s[0][0], s[0][1]), pack2(s[0][2], s[0][3]), pack2(s[1][0], s[1][1]), pack2(s[1][2], s[1][3])};
-#pragma unroll
-        for (int i = 0; i < DT; ++i) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) o[i][v] *= corr;
-            o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(uint4{vx[i].x, vx[i].y, vy[i].x, vy[i].y}), as_bf16x8(pb), o[i], 0, 0, 0);
+        };
+        // The two key buffers take turns; the piece's last tile has nothing behind it.
+        int kv0 = begin;
+        for (; kv0 + 64 < end; kv0 += 64) {
+            tile(kv0, std::true_type{}, k_a, k_b);
+            tile(kv0 + 32, std::true_type{}, k_b, k_a);
         }
-        if constexpr (NEXT) {
-            load_values(kv0 + 32, pg_nxt);
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                pg_cur[t] = pg_nxt[t];
-                pg_nxt[t] = pg_far[t];
-            }
+        if (kv0 + 32 < end) {
+            tile(kv0, std::true_type{}, k_a, k_b);
+            tile(kv0 + 32, std::false_type{}, k_b, k_a);
+        } else if (kv0 < end) {
+            tile(kv0, std::false_type{}, k_a, k_b);
         }
+        if constexpr (LOOKS && WAY != AT_EACH_LOAD) asm volatile("; %0" ::"n"(WAY) : "memory");
     };
-    // The two key buffers take turns; the piece's last tile has nothing behind it.
-    int kv0 = begin;
-    for (; kv0 + 64 < end; kv0 += 64) {
-        tile(kv0, std::true_type{}, k_a, k_b);
-        tile(kv0 + 32, std::true_type{}, k_b, k_a);
-    }
-    if (kv0 + 32 < end) {
-        tile(kv0, std::true_type{}, k_a, k_b);
-        tile(kv0 + 32, std::false_type{}, k_b, k_a);
-    } else if (kv0 < end) {
-        tile(kv0, std::false_type{}, k_a, k_b);
-    }
+    if constexpr (!LOOKS) walk(std::integral_constant<int, PAST_CACHES ? PAST : THROUGH>{});
+    else if constexpr (FUSED) walk(std::integral_constant<int, AT_EACH_LOAD>{});
+    else if (__builtin_expect(once, 1)) walk(std::integral_constant<int, PAST>{});
+    else walk(std::integral_constant<int, THROUGH>{});
 
     // The waves' results meet in LDS: element v of o[i] is channel 16*i + 4*q4 + v of query head r.
     if (r < gh) {
@@ -1148,15 +1234,15 @@ __device__ __forceinline__ void decode_rows(
     }
 }
 
-template <int HD, bool FUSED, bool CAP, bool PAGE16 = false>
+template <int HD, bool FUSED, bool CAP, bool PAGE16 = false, bool LOOKS = false>
 __global__ __launch_bounds__(64 * DecodeShape<HD>::MAX_WAVES) void attention_decode_kernel(
     const bf16_t* __restrict__ q, const float* __restrict__ qf, const float* __restrict__ kf, const float* __restrict__ vf, long ldq, long ldk,
     long ldv, const float* __restrict__ cos_t, const float* __restrict__ sin_t, bf16_t* __restrict__ cache, float* __restrict__ part,
     bf16_t* __restrict__ out, const int* __restrict__ rows, const int* __restrict__ pos, const int* __restrict__ slots,
     const int* __restrict__ table, int table_stride, long page_stride, int page_size, int n_heads, int n_kv, int window, float scale,
-    int n_splits, int gh, int units, Extras extra) {
+    int n_splits, int gh, int units, int step_rows, int shared, Extras extra) {
     extern __shared__ float merged[];
-    decode_rows<HD, FUSED, CAP, PAGE16>(merged, decode_item(units), q, qf, kf, vf, ldq, ldk, ldv, cos_t, sin_t, cache, part, out, rows, pos, slots, table, table_stride,
+    decode_rows<HD, FUSED, CAP, PAGE16, LOOKS>(merged, decode_item(units), step_rows, shared, q, qf, kf, vf, ldq, ldk, ldv, cos_t, sin_t, cache, part, out, rows, pos, slots, table, table_stride,
                                         page_stride, page_size, n_heads, n_kv, window, scale, n_splits, gh, extra);
 }
 
@@ -1167,12 +1253,12 @@ __global__ __launch_bounds__(64 * DecodeShape<HD>::MAX_WAVES) void attention_dec
 // Two launches and in one, 24 heads of 128 channels: portions of 1,350 rows behind 1,000 positions and of 674, 24 single rows at up to 2,990 positions, 110 and 93 us (the tiles alone 69);
 // 300 rows and 4 at up to 428 25.8 and 16.3; 32 heads of 64: 1,812 rows and 26 at up to 1,643 53.1 and 41.7.
 struct BothSplit { int prompt, decode; };               // workgroups of each kind, both padded to multiples of 8
-template <int HD, bool PAGE16>
+template <int HD, bool PAGE16, bool LOOKS>
 __global__ __launch_bounds__(256, HD == 128 ? 2 : 3) void attention_both_kernel(
     const bf16_t* __restrict__ q, bf16_t* __restrict__ cache, bf16_t* __restrict__ out, const int4* __restrict__ tiles, int n_at, const int* __restrict__ table, int table_stride,
     long page_stride, int page_size, int n_heads, int n_kv, int window, float scale, int tile_splits, const int* __restrict__ tile_first, float* __restrict__ tile_part, int list_order,
     Extras extra, WideShares shares, const int* __restrict__ rows, int n_rows, const int* __restrict__ pos, const int* __restrict__ slots, float* __restrict__ part, int n_splits, int gh,
-    BothSplit count) {
+    int step_rows, BothSplit count) {
     __shared__ __attribute__((aligned(1024))) unsigned char lds[wide_lds_bytes<HD>()];
     const int turn = blockIdx.x >> 3, both = min(count.prompt, count.decode) >> 3;
     const bool paired = turn < 2 * both, decodes = paired ? ((turn ^ (turn >> 5)) & 1) == 0 : count.decode > count.prompt;
@@ -1180,7 +1266,7 @@ __global__ __launch_bounds__(256, HD == 128 ? 2 : 3) void attention_both_kernel(
     if (decodes) {
         const int each = n_kv * ((n_heads / n_kv + 15) / 16) * n_splits, row = of_kind / each, rest = of_kind % each, heads = each / n_splits;
         if (row >= n_rows) return;
-        decode_rows<HD, false, false, PAGE16>(reinterpret_cast<float*>(lds), DecodeItem{row, rest % heads, rest / heads}, q, nullptr, nullptr, nullptr, 0, 0, 0, nullptr, nullptr, cache,
+        decode_rows<HD, false, false, PAGE16, LOOKS>(reinterpret_cast<float*>(lds), DecodeItem{row, rest % heads, rest / heads}, step_rows, heads > n_kv, q, nullptr, nullptr, nullptr, 0, 0, 0, nullptr, nullptr, cache,
                                               part, out, rows, pos, slots, table, table_stride, page_stride, page_size, n_heads, n_kv, window, scale, n_splits, gh, extra);
     } else {
         if (of_kind >= n_at * n_heads) return;
@@ -1396,16 +1482,16 @@ GI_API int gi_attention_decode_workgroups_per_unit(int hd, int fused, int n_wave
     return n;
 }
 
-// Rows `rows[0 .. n_rows)` of the step (`rows` null: rows 0 .. n_rows-1), one new position each.  Either `q` holds their rotated
+// Rows `rows[0 .. n_rows)` of the step's step_rows (`rows` null: rows 0 .. n_rows-1), one new position each.  Either `q` holds their rotated
 // queries in bfloat16 and the cache already holds their keys and values, or (`qf` given) `qf`,
 // `kf`, `vf` hold the unrotated 32-bit products, `cos_t`/`sin_t` the rotation (or null for none),
 // and the kernel rotates, attends and writes the new keys and values to the cache itself (`kf`
 // null: the pages belong to another layer and hold them already).  `n_waves` pieces per workgroup,
 // `n_splits` workgroups per row and head group; `part` is needed for n_splits > 1.  ordered: `rows` has the longest contexts first (gi_decode_order),
-// and the workgroups share them out evenly over the compute units.
+// and the workgroups share them out evenly over the compute units.  in_common: some of the rows may read pages in common.
 GI_API int gi_attention_decode_bf16(const void* q, const float* qf, const float* kf, const float* vf, long ldq, long ldk, long ldv,
                                     const float* cos_t, const float* sin_t, void* cache, void* out, float* part, long part_floats,
-                                    const int* rows, int n_rows, const int* pos, const int* slots, const int* table, int table_stride,
+                                    const int* rows, int n_rows, int step_rows, int in_common, const int* pos, const int* slots, const int* table, int table_stride,
                                     long page_stride, int page_size, int n_heads, int n_kv, int hd, int window, float scale, int n_splits,
                                     int n_waves, int ordered, int chunk, const float* sinks, const float* gate, long gate_stride, int gate_channels, float cap,
                                     hipStream_t stream) {
@@ -1413,8 +1499,8 @@ GI_API int gi_attention_decode_bf16(const void* q, const float* qf, const float*
                    (gate == nullptr || gate_channels == 0 || (gate_stride % 4 == 0 && ((uintptr_t)gate & 15) == 0)),
                "attention_decode: bad chunk, cap or gate stride, or a channels' gate whose rows do not start at multiples of 16 bytes");
     const Extras extra = {chunk, sinks, gate, gate_stride, gate_channels, cap};
-    GI_REQUIRE(n_rows > 0 && n_heads > 0 && n_kv > 0 && n_heads % n_kv == 0, "attention_decode: bad counts (%d rows, %d heads, %d kv heads)",
-               n_rows, n_heads, n_kv);
+    GI_REQUIRE(n_rows > 0 && step_rows >= n_rows && n_heads > 0 && n_kv > 0 && n_heads % n_kv == 0, "attention_decode: bad counts (%d rows of %d, %d heads, %d kv heads)",
+               n_rows, step_rows, n_heads, n_kv);
     GI_REQUIRE(gi_attention_bf16_supports(hd, page_size, 0), "attention_decode: head size %d with page size %d is not supported", hd, page_size);
     GI_REQUIRE(page_stride >= 2L * n_kv * page_size * hd && page_stride % 8 == 0, "attention_decode: bad page stride %ld", page_stride);
     GI_REQUIRE(n_splits >= 1 && n_splits <= MAX_SPLITS, "attention_decode: the number of splits %d is outside 1..%d", n_splits, MAX_SPLITS);
@@ -1442,20 +1528,29 @@ GI_API int gi_attention_decode_bf16(const void* q, const float* qf, const float*
     dim3 grid(n_rows, n_kv * hg, n_splits);
     GI_REQUIRE(!ordered || (rows != nullptr && (long)n_rows * n_kv * hg * n_splits < 2147483647L), "attention_decode: an order needs its rows, and fewer workgroups");
     const int units = ordered ? gi_compute_units() : 0;
-#define GO3(HD, FUSED_, CAP_, PAGE16_)                                                                                                              \
-    attention_decode_kernel<HD, FUSED_, CAP_, PAGE16_><<<grid, 64 * n_waves, lds, stream>>>((const bf16_t*)q, qf, kf, vf, ldq, ldk, ldv, cos_t, sin_t, \
+    // Groups of query heads that read the same keys: through the caches.  But where dies take the workgroups in turn as they lie in the grid and rows are a multiple of the eight
+    // dies, a row's groups lie on the same die, whose L2 brings them together anyway (8 rows at 8,000 positions, 32 heads of 128 on one, 20.2 us past the caches and 22.1; 4 rows at 4,000 16.0 and 15.2).
+    const int shared = hg > 1 && (ordered || n_rows % 8 != 0);
+    const bool looks = (in_common != 0 || shared) && extra.cap == 0.f;
+#define GO3(HD, FUSED_, CAP_, PAGE16_, LOOKS_)                                                                                                      \
+    attention_decode_kernel<HD, FUSED_, CAP_, PAGE16_, LOOKS_><<<grid, 64 * n_waves, lds, stream>>>((const bf16_t*)q, qf, kf, vf, ldq, ldk, ldv, cos_t, sin_t, \
                                                                                    (bf16_t*)cache, part, (bf16_t*)out, rows, pos, slots, table, \
                                                                                    table_stride, page_stride, page_size, n_heads, n_kv, window, \
-                                                                                   scale, n_splits, gh, units, extra)
+                                                                                   scale, n_splits, gh, units, step_rows, shared, extra)
     GI_REQUIRE(!(qf && extra.cap > 0.f), "attention_decode: capped scores are not served from unrotated products");
-#define GO2(HD, PAGE16_)                                       \
-    do {                                                       \
-        if (qf) GO3(HD, true, false, PAGE16_);                 \
-        else if (extra.cap > 0.f) GO3(HD, false, true, false); \
-        else GO3(HD, false, false, PAGE16_);                   \
+#define GO2(HD, PAGE16_, LOOKS_)                                       \
+    do {                                                               \
+        if (qf) GO3(HD, true, false, PAGE16_, LOOKS_);                 \
+        else if (extra.cap > 0.f) GO3(HD, false, true, false, false);  \
+        else GO3(HD, false, false, PAGE16_, LOOKS_);                   \
     } while (0)
-#define GO(HD) do { if (page_size == 16) GO2(HD, true); else GO2(HD, false); } while (0)
-    if (hd == 32) GO2(32, false); else if (hd == 64) GO(64); else if (hd == 96) GO2(96, false); else if (hd == 128) GO(128); else GO2(256, false);
+#define GO(HD)                                                         \
+    do {                                                               \
+        if (looks) { if (page_size == 16) GO2(HD, true, true); else GO2(HD, false, true); } \
+        else if (page_size == 16) GO2(HD, true, false);                \
+        else GO2(HD, false, false);                                    \
+    } while (0)
+    if (hd == 32) GO2(32, false, false); else if (hd == 64) GO(64); else if (hd == 96) GO2(96, false, false); else if (hd == 128) GO(128); else GO2(256, false, false);
 #undef GO
 #undef GO2
 #undef GO3
@@ -1481,7 +1576,7 @@ GI_API int gi_attention_both_takes(int n_tiles, int rows_per_tile, int paired, i
 GI_API int gi_attention_both_bf16(const void* q, void* cache, void* out, const int* tiles, int n_tiles, int rows_per_tile, int paired, const int* table, int table_stride,
                                   long page_stride, int page_size, int n_heads, int n_kv, int hd, int window, float scale, int tile_splits, const int* tile_first, const int* tile_rows,
                                   int n_tile_rows, float* tile_part, long tile_floats, int chunk, const float* sinks, const float* gate, long gate_stride, int gate_channels, int share_keys,
-                                  int most_shares, unsigned* counters, const int* rows, int n_rows, const int* pos, const int* slots, float* part, long part_floats, int n_splits,
+                                  int most_shares, unsigned* counters, const int* rows, int n_rows, int step_rows, int in_common, const int* pos, const int* slots, float* part, long part_floats, int n_splits,
                                   hipStream_t stream) {
     GI_REQUIRE(chunk >= 0 && (gate_channels == 0 || gate_channels == hd) && (gate == nullptr || gate_stride >= (long)n_heads * (gate_channels ? hd : 1)) &&
                    (gate == nullptr || gate_channels == 0 || (gate_stride % 4 == 0 && ((uintptr_t)gate & 15) == 0)),
@@ -1493,7 +1588,7 @@ GI_API int gi_attention_both_bf16(const void* q, void* cache, void* out, const i
                tile_splits, most_shares, n_rows, n_splits, n_heads, hd, page_size);
     GI_REQUIRE(page_stride >= 2L * n_kv * page_size * hd && page_stride % 8 == 0, "attention_both: bad page stride %ld", page_stride);
     GI_REQUIRE(!paired || n_tiles % 2 == 0, "attention_both: %d tiles cannot go in pairs", n_tiles);
-    GI_REQUIRE(q != nullptr && pos != nullptr && slots != nullptr && rows != nullptr, "attention_both: queries, positions, slots and the single rows must be given");
+    GI_REQUIRE(q != nullptr && pos != nullptr && slots != nullptr && rows != nullptr && step_rows >= n_rows, "attention_both: queries, positions, slots and the single rows must be given");
     GI_REQUIRE(n_splits == 1 || (part != nullptr && part_floats >= (long)n_rows * n_heads * n_splits * (hd + 2)), "attention_both: scratch too small");
     GI_REQUIRE(tile_splits == 1 || (tile_first && tile_rows && tile_part && n_tile_rows > 0 && tile_floats >= (long)n_tile_rows * n_heads * tile_splits * (hd + 2)),
                "attention_both: splitting needs the tiles' row offsets, their rows and scratch for the partial results");
@@ -1506,15 +1601,18 @@ GI_API int gi_attention_both_bf16(const void* q, void* cache, void* out, const i
     }
     const int group = n_heads / n_kv, hg = (group + 15) / 16, gh = group < 16 ? group : 16, n_at = n_tiles * tile_splits * shares.most;
     const BothSplit count = {(n_at * n_heads + 7) / 8 * 8, (n_rows * n_kv * hg * n_splits + 7) / 8 * 8};
-#define BOTH(HD, PAGE16_)                                                                                                                                              \
+#define BOTH(HD, PAGE16_, LOOKS_)                                                                                                                                      \
     do {                                                                                                                                                               \
         static_assert(4 * 16 * (HD + 2) * (int)sizeof(float) <= wide_lds_bytes<HD>(), "the single rows' results fit the tiles' LDS");                                  \
-        attention_both_kernel<HD, PAGE16_><<<count.prompt + count.decode, 256, 0, stream>>>((const bf16_t*)q, (bf16_t*)cache, (bf16_t*)out, (const int4*)tiles, n_at, table, table_stride, \
+        attention_both_kernel<HD, PAGE16_, LOOKS_><<<count.prompt + count.decode, 256, 0, stream>>>((const bf16_t*)q, (bf16_t*)cache, (bf16_t*)out, (const int4*)tiles, n_at, table, table_stride, \
                                                                                             page_stride, page_size, n_heads, n_kv, window, scale, tile_splits, tile_first, tile_part, \
-                                                                                            paired ? 1 : 0, extra, shares, rows, n_rows, pos, slots, part, n_splits, gh, count); \
+                                                                                            paired ? 1 : 0, extra, shares, rows, n_rows, pos, slots, part, n_splits, gh, step_rows, count); \
     } while (0)
-    if (hd == 64) { if (page_size == 16) BOTH(64, true); else BOTH(64, false); }
-    else { if (page_size == 16) BOTH(128, true); else BOTH(128, false); }
+#define BOTH_PAGES(HD, LOOKS_) do { if (page_size == 16) BOTH(HD, true, LOOKS_); else BOTH(HD, false, LOOKS_); } while (0)
+    const bool looks = in_common != 0 || hg > 1;
+    if (hd == 64) { if (looks) BOTH_PAGES(64, true); else BOTH_PAGES(64, false); }
+    else { if (looks) BOTH_PAGES(128, true); else BOTH_PAGES(128, false); }
+#undef BOTH_PAGES
 #undef BOTH
     GI_CHECK_LAUNCH("attention_both");
     if (tile_splits > 1) {

@@ -205,7 +205,7 @@ class Runner:
             meta_dev = meta_dev.view(3, n_rows)
             ctx = StepContext(n_rows=n_rows, dtype=self.model.dtype, device=dev, tokens=meta_dev[0], row_pos=meta_dev[1],
                               row_slot=meta_dev[2], seg_slot=seg_slot, seg_start=seg_start, seg_len=seg_len, seg_pos0=seg_pos0,
-                              upload=self._uploads.put, every_row_wanted=every_row_wanted)
+                              upload=self._uploads.put, every_row_wanted=every_row_wanted, pages_in_common=self.cache.prefix is not None)
             logits = self._forward(ctx, rows_dev, len(logit_rows))
         self._uploads.end_step()
         for e in entries:
@@ -226,13 +226,13 @@ class Runner:
             return None
         bracket = _context_bracket(max(p + n for p, n in zip(seg_pos0, seg_len)), self.max_positions)
         key = (tuple(seg_len), n_logit_rows, every_row_wanted, bracket)
-        g = self._step_graphs.get(key)
-        if g is None:
+        g, in_common = self._step_graphs.get(key), self.cache.prefix is not None
+        if g is None or g.pages_in_common != in_common:
             if len(self._step_graphs) >= self.max_step_graphs:       # (never during a capture: a graph may not be freed inside one)
                 del self._step_graphs[min(self._step_graphs, key=lambda k: self._step_graphs[k].last_used)]
             if self._graph_pool is None:
                 self._graph_pool = torch.cuda.graph_pool_handle()
-            g = self._step_graphs[key] = _StepGraph(self.model, self._view, n_rows, n_logit_rows, every_row_wanted, bracket, self._graph_pool)
+            g = self._step_graphs[key] = _StepGraph(self.model, self._view, n_rows, n_logit_rows, every_row_wanted, bracket, self._graph_pool, in_common)
         g.last_used = self.steps_run
         return g
 
@@ -300,13 +300,13 @@ class Runner:
         # The attention kernel's cut of the context into pieces is fixed at capture, for the longest context the graph
         # is to serve well: one graph per batch size and power-of-two bracket of the step's longest context.
         bracket = _context_bracket(max(seg_pos0) + 1, self.max_positions)
-        g = self._graphs.get((batch, bracket))
-        if g is None:
+        g, in_common = self._graphs.get((batch, bracket)), self.cache.prefix is not None
+        if g is None or g.pages_in_common != in_common:
             if len(self._graphs) >= self.max_graphs:         # (never during a capture: a graph may not be freed inside one)
                 del self._graphs[min(self._graphs, key=lambda k: self._graphs[k].last_used)]
             if self._graph_pool is None:
                 self._graph_pool = torch.cuda.graph_pool_handle()
-            g = self._graphs[(batch, bracket)] = _DecodeGraph(self.model, self._view, bracket, batch, self._graph_pool, self.cache.states)
+            g = self._graphs[(batch, bracket)] = _DecodeGraph(self.model, self._view, bracket, batch, self._graph_pool, self.cache.states, in_common)
         g.last_used = self.steps_run
         self.steps_replayed += 1 if g.calls >= 1 else 0
         return g.run(meta, seg_slot, seg_pos0, tokens_on_device)
@@ -432,8 +432,9 @@ class _DecodeGraph:
     its graphs must not form a reference cycle, or they would be freed by the cycle collector at a moment of its
     choosing, possibly while another graph is being captured, which the HIP runtime answers by aborting."""
 
-    def __init__(self, model: DecoderModel, view, longest_context: int, batch: int, pool=None, states=None):
+    def __init__(self, model: DecoderModel, view, longest_context: int, batch: int, pool=None, states=None, pages_in_common: bool = False):
         from ..kernels.ops import AttentionPlan
+        self.pages_in_common = pages_in_common
         self.model, self.view, self.batch, self.pool, self.last_used, self.states = model, view, batch, pool, 0, states
         dev = model.device
         self.meta = torch.zeros((3, batch), dtype=torch.int32, device=dev)
@@ -446,7 +447,8 @@ class _DecodeGraph:
     def _context(self, seg_slot, seg_pos0) -> StepContext:
         m, b = self.model, self.batch
         ctx = StepContext(n_rows=b, dtype=m.dtype, device=m.device, tokens=self.meta[0], row_pos=self.meta[1], row_slot=self.meta[2],
-                          seg_slot=list(seg_slot), seg_start=list(range(b)), seg_len=[1] * b, seg_pos0=list(seg_pos0), every_row_wanted=True)
+                          seg_slot=list(seg_slot), seg_start=list(range(b)), seg_len=[1] * b, seg_pos0=list(seg_pos0), every_row_wanted=True,
+                          pages_in_common=self.pages_in_common)
         ctx.memo["attention_plan"] = self.plan
         return ctx
 
@@ -485,9 +487,9 @@ class _StepGraph:
     over in one copy and replays.  The attention cuts contexts for the bracket's longest (`AttentionPlan` with its two context
     lengths set to the bracket), as the captured decode step does."""
 
-    def __init__(self, model: DecoderModel, view, n_rows: int, n_logit_rows: int, every_row_wanted: bool, bracket: int, pool):
+    def __init__(self, model: DecoderModel, view, n_rows: int, n_logit_rows: int, every_row_wanted: bool, bracket: int, pool, pages_in_common: bool = False):
         self.model, self.view, self.n_rows, self.n_logit_rows, self.every_row_wanted = model, view, n_rows, n_logit_rows, every_row_wanted
-        self.bracket, self.pool = bracket, pool
+        self.bracket, self.pool, self.pages_in_common = bracket, pool, pages_in_common
         self.block, self.places = None, None                 # the device block, and where each array lies in it: [(offset, size)]
         self.graph, self.logits, self.calls, self.last_used = None, None, 0, 0
 
@@ -532,7 +534,7 @@ class _StepGraph:
         meta_dev = self._view(0).view(3, self.n_rows)
         ctx = StepContext(n_rows=self.n_rows, dtype=m.dtype, device=m.device, tokens=meta_dev[0], row_pos=meta_dev[1], row_slot=meta_dev[2],
                           seg_slot=list(seg_slot), seg_start=list(seg_start), seg_len=list(seg_len), seg_pos0=list(seg_pos0),
-                          every_row_wanted=self.every_row_wanted)
+                          every_row_wanted=self.every_row_wanted, pages_in_common=self.pages_in_common)
         ctx.memo["attention_plan"] = plan
         return ctx
 

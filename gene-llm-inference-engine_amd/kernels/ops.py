@@ -107,10 +107,10 @@ _SIGNATURES = {
     "gi_attention_prompt_bf16": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int,
                                  c_float, c_int, c_void_p, c_void_p, c_int, c_void_p, c_long, c_int, c_void_p, c_void_p, c_long, c_int, c_float, c_int, c_int, c_void_p, c_void_p],
     "gi_attention_both_bf16": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p,
-                               c_void_p, c_int, c_void_p, c_long, c_int, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_long,
+                               c_void_p, c_int, c_void_p, c_long, c_int, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_long,
                                c_int, c_void_p],
     "gi_attention_decode_bf16": [c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_long, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
-                                 c_long, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int,
+                                 c_long, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_int,
                                  c_float, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_long, c_int, c_float, c_void_p],
     "gi_decode_order": [c_void_p, c_void_p, c_int, c_void_p, c_void_p],
     "gi_random_normal": [c_void_p, c_int, c_long, ctypes.c_ulonglong, ctypes.c_double, ctypes.c_double, c_void_p],
@@ -1309,7 +1309,7 @@ class AttentionPlan:
     def all_decode(cls, n_rows, max_context, device):
         """Every row is a request's single new row (what a captured decode step uses: nothing in it depends on the step)."""
         plan = cls.__new__(cls)
-        plan.n_decode, plan.n_tiles, plan.max_decode_context, plan.single_rows = n_rows, 0, max_context, True
+        plan.n_decode, plan.n_tiles, plan.max_decode_context, plan.single_rows, plan.rows_apart = n_rows, 0, max_context, True, True
         plan.decode_rows = None                                  # rows 0 .. n_rows-1
         plan.decode_positions = plan.tile_contexts = None
         plan.tile_places, plan.walk_shares, plan.cuts = [], {}, {}
@@ -1323,6 +1323,7 @@ class AttentionPlan:
         short_rows = sum(n for n in seg_len if 1 < n <= self.SHORT)
         row_by_row = self.SHORT if short_rows <= self.SHORT_TOTAL else 1
         self.single_rows = all(n == 1 for n in seg_len)          # every row is a request's only new row
+        self.rows_apart = row_by_row == 1 or short_rows == 0     # ... every row that goes one by one
         self.tile = self.TILE or (64 if sum(n for n in seg_len if n > row_by_row) <= self.SMALL_STEP else 128)
         for start, n, pos0, slot in zip(seg_start, seg_len, seg_pos0, seg_slot):
             if n <= row_by_row:
@@ -1626,9 +1627,10 @@ def _both_cut(plan, n_heads, n_kv, hd, window, chunk, page_size, seen, tile_spli
 
 
 def attention_bf16(q, cache, out, plan: AttentionPlan, positions, slots, table, n_heads, n_kv, hd, window=None, scale=None,
-                   target_waves: int = 4096, products=None, chunk=None, sinks=None, gate=None, cap=None, channel_gate=None, memo=None, together=False):
+                   target_waves: int = 4096, products=None, chunk=None, sinks=None, gate=None, cap=None, channel_gate=None, memo=None, together=False, in_common=False):
     """Attention of a step's rows with the matrix-core kernels (bfloat16 cache and out).  memo: what the pass keeps for its layers (the order of its rows).
-    together: single rows may go out in one launch with the tiles of prompts (`_both_splits`).
+    together: single rows may go out in one launch with the tiles of prompts (`_both_splits`).  in_common: requests of the step may read pages in common (portions that go row by row do anyway):
+    the kernel then looks which rows do, whose keys and values come through the caches, the others' past them; the results are the same.
 
     `q` holds the rotated queries in bfloat16 and the cache the rows' keys and values; or, for a step
     of single decoded rows only, `q` is None and `products = (q, k, v, cos, sin)` holds the unrotated
@@ -1674,6 +1676,7 @@ def attention_bf16(q, cache, out, plan: AttentionPlan, positions, slots, table, 
         for t in (cos, sin):
             if not (t is None or (t.dtype == torch.float32 and t.shape == (n, hd // 2) and t.is_contiguous())):
                 raise KernelError("attention: cos/sin must be float32 [n, hd/2]")
+    in_common = 1 if in_common or not plan.rows_apart else 0
     if plan.n_tiles:
         key = (plan.max_tile_context, plan.tile_contexts is None, PAIRED_TARGET_GROUPS, n_heads, hd, window, chunk, memo is not None)
         cut = plan.cuts.get(key)
@@ -1699,7 +1702,7 @@ def attention_bf16(q, cache, out, plan: AttentionPlan, positions, slots, table, 
             _call("gi_attention_both_bf16", q.data_ptr(), cache.data_ptr(), out.data_ptr(), plan.tiles.data_ptr(), plan.n_tiles, plan.tile, 1 if plan.paired else 0, table.data_ptr(),
                   table.stride(0), cache.stride(0), page_size, n_heads, n_kv, hd, window, scale, n_splits, _ptr(plan.tile_first),
                   _ptr(plan.tile_rows), plan.n_tile_rows, _ptr(part), n_part, *extras[:-1], keys, most, _ptr(counters), rows.data_ptr(),
-                  plan.n_decode, positions.data_ptr(), slots.data_ptr(), _ptr(rows_part), n_rows_part, both, _stream())
+                  plan.n_decode, n, in_common, positions.data_ptr(), slots.data_ptr(), _ptr(rows_part), n_rows_part, both, _stream())
             return out
         _call("gi_attention_prompt_bf16", q.data_ptr(), cache.data_ptr(), out.data_ptr(), plan.tiles.data_ptr(), plan.n_tiles, plan.tile,
               1 if plan.paired else 0, table.data_ptr(), table.stride(0), cache.stride(0), page_size, n_heads, n_kv, hd, window, scale, n_splits,
@@ -1714,7 +1717,7 @@ def attention_bf16(q, cache, out, plan: AttentionPlan, positions, slots, table, 
         part = torch.empty(n_part, dtype=torch.float32, device=out.device) if n_part else None
         _call("gi_attention_decode_bf16", _ptr(q), _ptr(qf), _ptr(kf), _ptr(vf), qf.stride(0) if qf is not None else 0,
               kf.stride(0) if kf is not None else 0, vf.stride(0) if vf is not None else 0, _ptr(cos), _ptr(sin), cache.data_ptr(),
-              out.data_ptr(), _ptr(part), n_part, _ptr(rows), plan.n_decode, positions.data_ptr(), slots.data_ptr(),
+              out.data_ptr(), _ptr(part), n_part, _ptr(rows), plan.n_decode, n, in_common, positions.data_ptr(), slots.data_ptr(),
               table.data_ptr(), table.stride(0), cache.stride(0), page_size, n_heads, n_kv, hd, window, scale, n_splits, n_waves, 1 if ordered else 0, *extras, _stream())
     return out
 
@@ -1742,7 +1745,7 @@ def attention(q, cache, out, ctx, table, n_heads, n_kv, hd, window=None):
     if q.dtype == torch.bfloat16 and cache.dtype == torch.bfloat16 and out.dtype == torch.bfloat16:
         plan = _plan_of(ctx)
         if (not plan.n_tiles or attention_bf16_supports(hd, page_size, True)) and (not plan.n_decode or attention_bf16_supports(hd, page_size, False)):
-            return attention_bf16(q, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, memo=ctx.memo, together=True)
+            return attention_bf16(q, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, memo=ctx.memo, together=True, in_common=ctx.pages_in_common)
     return attention_exact(q, cache, out, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, **_known_of(ctx))
 
 
@@ -1771,7 +1774,7 @@ def attention_general(q, cache, out, ctx, table, n_heads, n_kv, hd, *, page_size
         plan = _plan_of(ctx)
         if (not plan.n_tiles or attention_bf16_supports(hd, page_size, True)) and (not plan.n_decode or attention_bf16_supports(hd, page_size, False)):
             return attention_bf16(q, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, scale, chunk=chunk, sinks=sinks, gate=gate, cap=cap,
-                                  channel_gate=channel_gate, memo=ctx.memo, together=True)
+                                  channel_gate=channel_gate, memo=ctx.memo, together=True, in_common=ctx.pages_in_common)
     return attention_exact(q, cache, out, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, scale, page_size=page_size,
                            value_dim=value_dim, chunk=chunk, sinks=sinks, gate=gate, cap=cap, channel_gate=channel_gate, **_known_of(ctx))
 
@@ -1795,7 +1798,7 @@ def attention_from_products(q, k, v, cos, sin, cache, out, ctx, table, n_heads, 
         return False
     if q.stride(0) % 4 or q.data_ptr() % 16 or (k is not None and (k.stride(0) % 4 or k.data_ptr() % 16)):
         return False
-    attention_bf16(None, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, products=(q, k, v, cos, sin), memo=ctx.memo)
+    attention_bf16(None, cache, out, plan, ctx.row_pos, ctx.row_slot, table, n_heads, n_kv, hd, window, products=(q, k, v, cos, sin), memo=ctx.memo, in_common=ctx.pages_in_common)
     return True
 
 

@@ -1208,7 +1208,9 @@ def test_long_walks_of_prompt_tiles_share_their_keys_out(n_heads, n_kv, hd, segs
     (32, 8, 64, 16, [(0, 1500)], [1, 1200, 16, 17, 500], 1, None, None), (64, 16, 64, 48, [(3000, 900), (0, 401)], [2000] * 9, 3, None, None), (64, 16, 64, 16, [(300, 1200)], [900, 30, 1700], 2, 200, None),
     (20, 1, 128, 16, [(0, 300)], [40, 999, 1], 1, None, None), (40, 2, 128, 16, [(100, 800)], [640, 65], 3, None, None), (4, 4, 128, 48, [(1400, 100), (600, 130)], [300, 800], 1, 450, None),
     (4, 1, 128, 16, [(0, 200)], [500] * 70, 4, None, None), (16, 8, 128, 16, [(640, 900)], [300, 129, 128, 1], 1, None, "chunk"), (16, 8, 128, 16, [(0, 900)], [300, 129], 2, None, "sinks"),
-    (24, 8, 128, 16, [(0, 700)], [800, 2], 2, None, "gate"), (32, 8, 64, 16, [(0, 1500)], [600, 3], 2, None, "channels")])
+    (24, 8, 128, 16, [(0, 700)], [800, 2], 2, None, "gate"), (32, 8, 64, 16, [(0, 1500)], [600, 3], 2, None, "channels"),
+    # short portions, which go row by row among the single rows: several rows of one request in the list
+    (24, 8, 128, 16, [(1020, 900), (700, 30)], [1, 2990, 64], 1, None, None), (32, 8, 64, 16, [(0, 1500), (33, 2), (900, 17)], [600] * 5, 2, None, None), (40, 2, 128, 32, [(100, 800), (0, 40)], [640], 1, 300, None)])
 def test_single_rows_and_tiles_in_one_launch(n_heads, n_kv, hd, ps, portions, singles, splits, window, extra, monkeypatch):
     """A step's single rows beside portions of prompts: the tiles' rows are in bits those of a launch of their own, the single rows those of another cut of their contexts; every time the
     same bits; and without room for shares."""
@@ -1236,7 +1238,7 @@ def test_single_rows_and_tiles_in_one_launch(n_heads, n_kv, hd, ps, portions, si
     before, memo = cache.clone(), {}
     apart, got, again = made(False, {}), made(True, memo), made(True, memo)
     assert asked.count("gi_attention_both_bf16") == 2 and asked.count("gi_attention_prompt_bf16") == 1
-    single = torch.tensor([s for s, (_, n) in zip(starts, segs) if n == 1], device=DEV)
+    single = torch.tensor([s + i for s, (_, n) in zip(starts, segs) if n <= 64 for i in range(n)], device=DEV)
     tiles = torch.ones(len(rows), dtype=torch.bool, device=DEV).index_fill_(0, single, False)
     assert torch.equal(got, again) and torch.equal(got[tiles], apart[tiles])
     # (probabilities are rounded to bfloat16 about other maxima, 2^-9 of each at most on either side, and the results, 2^-8 between the two)
@@ -1682,6 +1684,48 @@ def test_decoded_rows_read_whole_blocks_of_keys(hd, ps, window):
     ops().attention(q, cache, out, ctx, table, 6, 2, hd, window)
     want = plain_attention_rows(q, dense, [(i, n - 1) for i, n in enumerate(contexts)], 6, 2, hd, window)
     assert rel(out, want) < 8e-3, rel(out, want)
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("rows", [2, 8, 21])
+@pytest.mark.parametrize("n_heads,n_kv,hd,ps,window", [(6, 2, 64, 16, None), (6, 2, 128, 16, None), (40, 2, 64, 48, None), (20, 1, 128, 16, 200)])
+def test_decoded_rows_that_share_their_pages(n_heads, n_kv, hd, ps, window, rows, fused):
+    """Requests of two kinds in turn that each begin alike, on pages in common and on copies of them: keys and values come through the caches or past them, the bits are the same, and
+    those of rows alone."""
+    o = ops()
+    from geneinfer_amd.parts import StepContext
+    contexts = [530 + 37 * i for i in range(rows)]
+    cache, table, dense = build_paged(contexts, n_kv, hd, ps, torch.bfloat16, seed=hd + rows)
+    alike = 500 // ps                                                     # whole pages
+    for i in range(2, rows):
+        cache[table[i + 1, :alike].long()] = cache[table[1 + i % 2, :alike].long()]
+    common = table.clone()
+    for i in range(2, rows):
+        common[i + 1, :alike] = table[1 + i % 2, :alike]
+    if rows == 2:
+        cache[table[2, :alike].long()], common[2, :alike] = cache[table[1, :alike].long()], table[1, :alike]
+    pos, slots = torch.tensor([n - 1 for n in contexts], dtype=torch.int32, device=DEV), torch.arange(1, rows + 1, dtype=torch.int32, device=DEV)
+    a, kvd = n_heads * hd, n_kv * hd
+    qkv, angle = randn(rows, a + 2 * kvd, seed=31), randn(rows, hd // 2, seed=9)
+
+    def made(table, first=0, n=rows, looks=True):
+        seen, memo = cache.clone(), {}
+        part = slice(first, first + n)
+        out = torch.full((n, a), float("nan"), dtype=torch.bfloat16, device=DEV)
+        plan = o.AttentionPlan(list(range(n)), [1] * n, [c - 1 for c in contexts[part]], list(range(first + 1, first + n + 1)), DEV)
+        if fused:
+            products = (qkv[part, :a], qkv[part, a:a + kvd], qkv[part, a + kvd:], torch.cos(angle[part]), torch.sin(angle[part]))
+            o.attention_bf16(None, seen, out, plan, pos[part], slots[part], table, n_heads, n_kv, hd, window, products=products, memo=memo, in_common=looks)
+        else:
+            o.attention_bf16(qkv[part, :a].to(torch.bfloat16).contiguous(), seen, out, plan, pos[part], slots[part], table, n_heads, n_kv, hd, window, memo=memo, in_common=looks)
+        return out, seen
+
+    (own, cache_own), (shared, cache_shared), (unseen, cache_unseen) = made(table), made(common), made(common, looks=False)
+    assert torch.equal(own, shared) and torch.equal(own, unseen) and not bool(torch.isnan(own.float()).any())
+    assert all(torch.equal(torch.nan_to_num(cache_own, nan=-1.0), torch.nan_to_num(c, nan=-1.0)) for c in (cache_shared, cache_unseen))
+    alone = torch.cat([made(table, i, 1)[0] for i in range(rows)])
+    # (probabilities are rounded to bfloat16 about other maxima, 2^-9 of each at most on either side, and the results, 2^-8 between the two)
+    assert rel(alone, own) < 2 * 2.0 ** -9 + 2.0 ** -8
 
 
 @pytest.mark.parametrize("n_heads,n_kv,hd,ps,window", ATT_CASES)

@@ -325,3 +325,20 @@ def test_single_rows_beside_tiles(portions, singles, heads, kv, hd, splits):
     assert cut() == splits and cut() == splits
     plan.decode_positions = None                 # a step still to come
     assert cut() == 0
+
+
+@pytest.mark.parametrize("rows,apart", [([1, 1, 1], True), ([1, 3], False), ([64], False), ([1, 65], True), ([1, 40, 40], True), ([1, 30, 30, 500], False), ([500, 900], True)])
+def test_short_portions_go_row_by_row_over_pages_in_common(rows, apart, monkeypatch):
+    """What the kernel is told, of itself and where the step says that requests may share pages; a captured step of single rows is told by its step."""
+    launched = []
+    monkeypatch.setattr(ops, "_dev", lambda *tensors: None)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_call", lambda name, *a: launched.append((name, a)))
+    plan, n = _plan([(700, r) for r in rows]), sum(rows)
+    q, at = torch.zeros(n, 8 * 64, dtype=torch.bfloat16), torch.zeros(n, dtype=torch.int32)
+    cache, table = torch.zeros(4, 2, 2, 16, 64, dtype=torch.bfloat16), torch.zeros(len(rows), 128, dtype=torch.int32)
+    assert plan.rows_apart == apart and ops.AttentionPlan.all_decode(3, 1000, "cpu").rows_apart
+    for in_common in (False, True):
+        ops.attention_bf16(q, cache, torch.zeros_like(q), plan, at, at, table, 8, 2, 64, memo={}, in_common=in_common)
+    told = [a[15:17] for name, a in launched if name == "gi_attention_decode_bf16"]
+    assert told == ([(n, 1 - apart), (n, 1)] if plan.n_decode else [])
