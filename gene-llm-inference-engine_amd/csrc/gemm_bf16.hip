@@ -1929,7 +1929,7 @@ __global__ __launch_bounds__(256) void skinny_reduce_rope_store_kernel(const flo
 // Loads run DEPTH steps ahead of the products.  The waves' sums meet in LDS and are added in the order of the waves, the lower halves before the upper.
 //
 // What bounds it is weights on their way from memory, and behind them the activations, of which every workgroup reads all.  67 MB of weights in a bare read take
-// 12.8 us, 11.4 past the caches (each line is read once, by one load; with 16 rows' 64 bytes a load, as this kernel read them before, 14.1 and 14.8).  All workgroups
+// 12.8 us, 11.4 past the caches (PAST: each line is read once, by one load; with 16 rows' 64 bytes a load, as this kernel read them before, 14.1 and 14.8).  All workgroups
 // starting at the same k would ask the same memory channels first (rows lie a multiple of 4 KB apart): 12.6 us, 11.9 from a place of their own.  Microseconds, before and now, in chains
 // of products with weights of their own:
 //   rows                        1               8               16
@@ -1946,7 +1946,7 @@ __global__ __launch_bounds__(256) void skinny_reduce_rope_store_kernel(const flo
 // reckon with them (`slim_reach`).
 template <bool FAR> struct SlimPlaces { typedef int Stride; typedef unsigned At; };
 template <> struct SlimPlaces<true> { typedef long Stride; typedef size_t At; };
-template <int GROUPS, int EPI, bool HAND, int XT, bool FAR = false>
+template <int GROUPS, int EPI, bool HAND, int XT, bool PAST, bool FAR = false>
 __global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, typename SlimPlaces<FAR>::Stride lda8,
                                                                 typename SlimPlaces<FAR>::Stride ldw8, int M, int N, int K, int rows, int turn,
                                                                 void* __restrict__ C, long ldc, NormIn norm_in, NormOut norm_out) {
@@ -1991,7 +1991,7 @@ __global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __
 #pragma unroll
         for (int t = 0; t < XT; ++t) x[t] = load16(whereof(A, x_at[t] + at));
 #pragma unroll
-        for (int g = 0; g < GROUPS; ++g) w[g] = load16_once(whereof(w_base[g], w_at[g] + at));
+        for (int g = 0; g < GROUPS; ++g) w[g] = PAST ? load16_once(whereof(w_base[g], w_at[g] + at)) : load16(whereof(w_base[g], w_at[g] + at));
     };
     floatx4 acc[XT][GROUPS];
 #pragma unroll
@@ -2602,8 +2602,9 @@ static int launch_slim(const void* A, const void* W, void* C, int epi, int M, in
     const auto [rows, far] = slim_reach(M, N, K, epi, lda, ldw);
     const dim3 grid((N + rows - 1) / rows);
     const int turn = turn_of_steps((K + 63) / 64);
+    const bool past = weights_past_caches(N, K);
     if (far) {
-#define SLIM_FAR(GROUPS_, EPI_) gemm_bf16_slim_kernel<GROUPS_, EPI_, true, 2, true><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, lda / 8, ldw / 8, M, N, K, rows, turn, C, ldc, norm_in, norm_out)
+#define SLIM_FAR(GROUPS_, EPI_) gemm_bf16_slim_kernel<GROUPS_, EPI_, true, 2, false, true><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, lda / 8, ldw / 8, M, N, K, rows, turn, C, ldc, norm_in, norm_out)
         if (epi == EPI_GATED_BF16) SLIM_FAR(2, EPI_GATED_BF16); else if (epi == EPI_GATED_GELU_BF16) SLIM_FAR(2, EPI_GATED_GELU_BF16); else if (is_gated(epi)) SLIM_FAR(2, EPI_GATED_CLAMP_BF16);
         else if (epi == EPI_STORE_F32) SLIM_FAR(3, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM_FAR(3, EPI_ADD_F32);
         else if (epi == EPI_XIELU) SLIM_FAR(3, EPI_XIELU); else SLIM_FAR(3, EPI_STORE_BF16);
@@ -2611,12 +2612,13 @@ static int launch_slim(const void* A, const void* W, void* C, int epi, int M, in
         GI_CHECK_LAUNCH("gemm_bf16 (slim, far)");
         return 0;
     }
-#define SLIM_XT(GROUPS_, EPI_, XT_)                                                                                                                    \
+#define SLIM_XT(GROUPS_, EPI_, XT_, PAST_)                                                                                                             \
     do {                                                                                                                                               \
-        if (hand) gemm_bf16_slim_kernel<GROUPS_, EPI_, true, XT_><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, (int)(lda / 8), (int)(ldw / 8), M, N, K, rows, turn, C, ldc, norm_in, norm_out); \
-        else gemm_bf16_slim_kernel<GROUPS_, EPI_, false, XT_><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, (int)(lda / 8), (int)(ldw / 8), M, N, K, rows, turn, C, ldc, norm_in, norm_out);     \
+        if (hand) gemm_bf16_slim_kernel<GROUPS_, EPI_, true, XT_, PAST_><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, (int)(lda / 8), (int)(ldw / 8), M, N, K, rows, turn, C, ldc, norm_in, norm_out); \
+        else gemm_bf16_slim_kernel<GROUPS_, EPI_, false, XT_, PAST_><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, (int)(lda / 8), (int)(ldw / 8), M, N, K, rows, turn, C, ldc, norm_in, norm_out);     \
     } while (0)
-#define SLIM(GROUPS_, EPI_) do { if (M <= 8) SLIM_XT(GROUPS_, EPI_, 1); else SLIM_XT(GROUPS_, EPI_, 2); } while (0)
+#define SLIM_ROWS(GROUPS_, EPI_, PAST_) do { if (M <= 8) SLIM_XT(GROUPS_, EPI_, 1, PAST_); else SLIM_XT(GROUPS_, EPI_, 2, PAST_); } while (0)
+#define SLIM(GROUPS_, EPI_) do { if (past) SLIM_ROWS(GROUPS_, EPI_, true); else SLIM_ROWS(GROUPS_, EPI_, false); } while (0)
 #define SLIM_EPI(GROUPS_)                                                                                                                              \
     do {                                                                                                                                               \
         if (epi == EPI_STORE_F32) SLIM(GROUPS_, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM(GROUPS_, EPI_ADD_F32);                               \
@@ -2637,6 +2639,7 @@ static int launch_slim(const void* A, const void* W, void* C, int epi, int M, in
 #undef SLIM_GATED
 #undef SLIM_EPI
 #undef SLIM
+#undef SLIM_ROWS
 #undef SLIM_XT
     GI_CHECK_LAUNCH("gemm_bf16 (slim)");
     return 0;
