@@ -19,7 +19,7 @@
 //           once, activations go through LDS; v_mfma_f32_16x16x32_bf16.  Wide and narrow outputs likewise.
 //   slim    at most 16 rows of A (decode): a workgroup of 8 waves owns 8 to 32 weight rows, its
 //           waves take interleaved steps of k and add their sums through LDS in a fixed order, so
-//           one launch does the whole product and its epilogue.  Strips of so few rows are its too.
+//           one launch does the whole product and its epilogue.
 //
 // The "gated" epilogue serves SwiGLU: the weight is [gate; up] interleaved in groups of 16 rows
 // (16 gate rows, the 16 up rows of the same outputs, and so on), and the output column c of a
@@ -2510,77 +2510,74 @@ static int streamed_from_row(int strips, int K) {
     const double fitted = 12.0 * (2048.0 / K) * (256.0 / strips);
     return fitted < 3 ? 3 : fitted > 12 ? 12 : (int)(fitted + 0.5);
 }
-// Where K is a multiple of 64, from which row on a product counts as strips of columns, which take no norm's pieces beyond a reader's and hand none on: lines drawn between the slim
-// kernel as it was and the strips' ring in LDS.  Since it reads whole cache lines the slim kernel makes most strips of up to 16 rows too (`strips_in_registers` below).
-static int slim_until_row(int strips, int K, bool gated) {
+// Where K is a multiple of 64 the other one is the strips' (the weight-streaming one for some of a short k, `ends_in_strips`).  What decides is how the workgroups of either fill the compute units: strips
+// of 64 columns, one a unit where they are one round or less, two of which a unit runs side by side, against workgroups of at most 32 weight rows in so many more rounds, each with its end; and the
+// activations, which every workgroup of the slim kernel reads and strips share.  Microseconds, slim and strips, in chains of products with weights of their own:
+//   gated                 1 row         8 rows        12 rows       16 rows         stored                1 row         8 rows        12 rows       16 rows
+//   12,288 x 2,048        9.6, 11.5     10.8, 11.9    12.9, 12.0    13.6, 12.0      12,288 x 2,048        9.9, 11.5     10.9, 11.7    12.2, 11.7    13.0, 11.7
+//   16,384 x 2,048        12.4, 14.2    12.3, 14.5    13.1, 14.6    13.9, 14.6      16,384 x 8,192        44.4, 50.6    43.4, 50.9    44.5, 51.2    46.6, 50.5
+//   18,432 x 4,096        26.0, 35.7    29.8, 36.4    33.0, 37.0    35.0, 37.2      18,432 x 4,096        24.4, 35.6    26.3, 36.3    30.3, 36.7    32.2, 37.1
+//   28,672 x 4,096        36.4, 40.8    40.4, 41.3    43.0, 41.0    45.3, 41.5      28,672 x 4,096        36.8, 40.9    37.7, 41.5    41.2, 42.8    43.9, 43.2
+//   36,864 x 3,072        34.1, 45.1    39.2, 46.1    42.2, 46.3    44.9, 46.6      128,256 x 2,048       75.6, 89.8    77.2, 92.1    84.1, 94.1    90.4, 96.0
+//   28,672 x 512          7.7, 7.8      8.1, 8.2      9.1, 8.3      9.5, 8.5        100,352 x 512         21.9, 22.0    23.9, 23.0    27.6, 23.2    29.0, 23.6
+// Of 7,742 products (30 widths to 152,064 columns, 28 k, stored and gated, 1 to 16 rows) the choice is 0.3 % slower than the faster of the two on average, 15 with over 10 % (k of 64, 320 and 704); of 576
+// gated ones that finish a norm 0.8 %.
+static bool slim_beside_strips(int M, int strips, int K, bool gated) {
     const int units = gi_compute_units();
-    const bool three_quarters = strips * 4 <= units * 3, narrow = strips * 5 <= units * 4, second = strips > units && strips * 2 <= units * 3, barely = strips * 4 <= units * 5, whole = K % 2048 == 0;
-    const double filled = (double)strips / ((strips + units - 1) / units * units);
-    if (!gated) {
-        if (K <= 512) return three_quarters ? 12 : 0;
-        const bool third = strips > 2 * units;
-        if (K < 1536) return strips > units && barely ? 10 : third && filled < 0.8 && K > 1024 ? 4 : 0;
-        if (whole) return three_quarters ? 8 : narrow ? 4 : second ? (barely ? 12 : 9) : third && filled < 0.85 ? 10 : filled > 0.9 ? 8 : 7;
-        return three_quarters ? 4 : narrow ? 0 : second ? (barely ? 10 : 6) : third ? (filled < 0.8 ? 6 : filled < 0.9 ? 4 : 3) : strips > units ? 3 : 2;
+    if (K < 256 && strips > units) return false;                      // (most of a workgroup's waves have no k)
+    if (K <= 640) {
+        if (strips * 2 <= units * 3) return gated || K < 512 || strips * 10 > units * 9 || M <= 10;
+        return K > 256 && M <= (gated || strips > 2 * units ? 8 : 4);
     }
-    int until;
-    if (K < 1024) until = narrow && K > 512 ? 8 : strips * 2 <= units * 3 ? 12 : 10;
-    else if (narrow) until = 0;
-    else if (K >= 3072 && filled >= 0.85) until = !whole ? 0 : filled > 0.9 ? 6 : strips <= units ? 3 : 0;
-    else until = K > 2048 ? 6 : whole && strips <= units && filled > 0.9 ? 9 : K > 1024 || strips <= units ? 8 : 10;
-    return strips * 2 > units * 3 ? min(until, streamed_from_row(strips, K)) : until;
+    if (M <= 8) return true;
+    if (strips * 10 <= units * 9) return K < 1536 && M <= 12;
+    if (strips * 5 > units * 8 && strips * 20 <= units * 37) return M <= (gated ? 10 : K < 1536 ? 12 : 16);
+    return true;
 }
 // xielu: the product ends through that activation, which of the kernels only slim has.
 static bool takes_slim(int M, int N, int K, bool gated, bool xielu = false) {
     const int strips = (N + 63) / 64;
     if (M > 16 || gi_gemm_bf16_skinny_splits(N, K) > 0) return M <= 16;
-    if (strips >= 1024) return M < 5;
-    return M < (K % PK != 0 || xielu ? streamed_from_row(strips, K) : slim_until_row(strips, K, gated));
+    if (K % PK != 0 || xielu) return M < (strips >= 1024 ? 5 : streamed_from_row(strips, K));
+    return slim_beside_strips(M, strips, K, gated);
 }
 
-// Workgroups of the slim kernel for an output of N columns that is not gated: the pieces a row's sum of squares comes in.
-// Weight rows per workgroup of the slim kernel.  A round of workgroups, one per compute unit, takes as long as its weights, an eighth to a third of a weight row more for
-// every row of A (all of which every workgroup reads) and two rows' time to begin and end; a round that is not full costs four fifths of one at least.  So an output that
-// 256 workgroups of at most 32 rows cover has one round, and wider ones as few as fill it well.  28 outputs of 640 to 128,256 columns, k of 768 to 14,336, 1 to 16 rows, seven to
-// eight heights each: the choice is 0.3 % slower than the fastest on average, 9.6 % at worst (10,240 x 2,048 at one row).  Microseconds by weight rows a workgroup:
+// Weight rows per workgroup of the slim kernel.  A round of workgroups, one per compute unit, takes as long as its weights, a sixth of a row for each that is missing from a group of 8, a fifth of a row
+// for each row of A (all of which every workgroup reads; half a row from nine on), two rows' time to begin and end, and what finishing a norm takes, about 0.7 us (which gated products alone go by:
+// they have two heights to choose from, and many workgroups); more than 24 rows, with fewer loads in flight, take 5 % longer where k is long, and a round that is not full costs four fifths of one at least.  So an output that
+// 256 workgroups of at most 32 rows cover has one round, and wider ones as few as fill it well.  23 outputs of 512 to 16,384 columns, k of 256 to 8,192, 1 to 16 rows, ten to
+// thirteen heights each: the choice is 1 % slower than the fastest on average, 14 % at worst; of 16 or 32 rows for 18 gated outputs to 65,536 columns 1 %.  Microseconds by weight rows a workgroup:
 //                                      8       12      16      20      24      32
 //   6,144 x 4,096 at 1 row             10.05   10.53   11.21   13.65   9.87    11.47
 //   6,144 x 4,096 at 8 rows            13.09   12.33   13.26   15.56   10.26   12.33
 //   2,048 x 8,192 at 8 rows            9.78    11.93   13.13   15.59   16.82
 //   128,256 x 2,048 at 8 rows          119.1   107.0   90.8    91.0    84.7    80.9
+//   8,192 x 512 added at 8 rows        4.54            3.93    4.58    4.46           (17: 4.76)
 //   28,672 x 4,096 gated, 1 and 12                     37.0, 48.7              42.1, 45.7
-// Gated columns come in pairs of 16 weight rows, half of which or all a workgroup takes; what adds onto rows stays below 32, whose registers it lacks, and where it hands a norm on
-// makes no more pieces of a row's sum of squares than a reader takes.
-static int slim_strip_rows(int M, int N, int epi) {
+//   28,672 x 1,024 gated with a norm, 1 and 8          16.6, 18.7              13.7, 14.5
+// Gated columns come in pairs of 16 weight rows, half of which or all a workgroup takes; what adds onto rows stays below 32, whose registers it lacks, and makes no more pieces of a row's
+// sum of squares than a reader takes where that can be done (else it hands no norm on).
+static int slim_strip_rows(int M, int N, int K, int epi, bool normed) {
     const int units = gi_compute_units();
+    const double ends = 2 + (normed && is_gated(epi) ? 8192.0 / K : 0.0);
     auto cost = [&](int rows) {
         const int groups = (N + rows - 1) / rows, whole = groups / units, rest = groups % units;
         const double share = rest == 0 ? 0.0 : whole == 0 ? 1.0 : rest * 5 < units * 4 ? 0.8 : (double)rest / units;
-        return (whole + share) * (rows + (M <= 8 ? 0.2 : 0.6) * M + 2);
+        return (whole + share) * (rows + (8 - rows % 8) % 8 / 6.0 + (M <= 8 ? 0.2 : 0.5) * M + ends) * (rows > 24 && K > 2048 ? 1.05 : 1.0);
     };
     if (is_gated(epi)) return cost(16) < cost(32) ? 16 : 32;
-    int best = 8;
-    for (int rows = 9; rows <= (epi == EPI_ADD_F32 ? 24 : 32); ++rows)
-        if (cost(rows) < cost(best) || (epi == EPI_ADD_F32 && (N + best - 1) / best > slim_max_parts(M))) best = rows;
+    const int most = epi == EPI_ADD_F32 ? 24 : 32, fit = epi == EPI_ADD_F32 ? (N + slim_max_parts(M) - 1) / slim_max_parts(M) : 8;
+    int best = fit <= 8 || fit > most ? 8 : fit;
+    for (int rows = best + 1; rows <= most; ++rows)
+        if (cost(rows) < cost(best)) best = rows;
     return best;
 }
-// Strips of a few rows of A, which are otherwise made through a ring in LDS, in the slim kernel's workgroups of 16 or 32 weight rows: faster to 14 rows for 18
-// sizes measured, and at 16 by 9 % on average and at most 3 % slower; but stored columns of a short k, whose end weighs most there, from 9 rows on.
-// Microseconds, strips through LDS and in registers:
-//   rows                     4              8              12             16
-//   28,672 x 4,096 gated     46.4, 40.9     46.4, 43.1     46.7, 45.5     46.7, 47.9
-//   24,576 x 2,048 gated     23.2, 17.1     23.6, 17.4     24.2, 18.5     24.4, 19.5
-//   128,256 x 2,048 stored   94.2, 78.3     98.7, 80.9     99.9, 88.6     100.9, 93.1
-//   16,384 x 8,192 stored    66.2, 44.4     65.5, 44.5     65.1, 46.9     65.8, 49.7
-//   65,536 x 512 stored      15.1, 14.9     15.2, 15.2     15.3, 18.0     15.5, 18.3
-static bool strips_in_registers(int M, int K, int epi) { return M <= 8 || (M <= 16 && (is_gated(epi) || K > 512)); }
-
 // How the slim kernel reaches rows so far apart.  It adds a row's place and the one in k behind it in 32 bits: in bytes for more than 24 weight rows a workgroup, in pieces of
 // 16 bytes for fewer, so the end of the last row that a workgroup reads, from its first, has to lie within.  Beyond the former fewer weight rows a workgroup, beyond the latter
 // (68 GB) the variant that reckons in 64 bits, of which there is one for each kind of end.
 struct SlimReach { int rows; bool far; };
-static SlimReach slim_reach(int M, int N, int K, int epi, long lda, long ldw) {
-    int rows = slim_strip_rows(M, N, epi);
+static SlimReach slim_reach(int M, int N, int K, int epi, bool normed, long lda, long ldw) {
+    int rows = slim_strip_rows(M, N, K, epi, normed);
     auto pieces = [&]() {
         const long apart = is_gated(epi) ? 7 : min(rows, N) - 1, w = apart * (ldw / 8), a = (M - 1) * (lda / 8);       // (gated: every group of 8 rows has an address of its own)
         return (w > a ? w : a) + K / 8;
@@ -2591,15 +2588,16 @@ static SlimReach slim_reach(int M, int N, int K, int epi, long lda, long ldw) {
     return {far && rows > fewer ? fewer : rows, far};
 }
 
-static int slim_parts(int M, int N) {
-    const int rows = slim_strip_rows(M, N, EPI_ADD_F32);
+// Workgroups of the slim kernel for an output of N columns that is added onto rows: the pieces a row's sum of squares comes in.
+static int slim_parts(int M, int N, int K) {
+    const int rows = slim_strip_rows(M, N, K, EPI_ADD_F32, false);
     return (N + rows - 1) / rows;
 }
 
 static int launch_slim(const void* A, const void* W, void* C, int epi, int M, int N, int K, long lda, long ldw, long ldc, NormIn norm_in,
                        NormOut norm_out, hipStream_t stream) {
     const bool hand = norm_in.squares != nullptr || (norm_out.scaled != nullptr && epi != EPI_XIELU);
-    const auto [rows, far] = slim_reach(M, N, K, epi, lda, ldw);
+    const auto [rows, far] = slim_reach(M, N, K, epi, norm_in.squares != nullptr, lda, ldw);
     const dim3 grid((N + rows - 1) / rows);
     const int turn = turn_of_steps((K + 63) / 64);
     const bool past = weights_past_caches(N, K);
@@ -2756,11 +2754,7 @@ static int launch_skinny(const void* A, const void* W, void* C, int epi, int M, 
                norm_in.parts, consumer_max_parts(M), M);
     if (splits == 0) {                             // a wide output: every workgroup sees all of k and finishes its columns
         GI_REQUIRE(norm_out.scaled == nullptr && rope == nullptr, "gemm_bf16: a product this wide does not hand a norm on, or its rows to the cache");
-        if (ends_in_strips(M, N, K) && strip_strides(lda, ldw)) {
-            if (strips_in_registers(M, K, epi) && (norm_in.squares == nullptr || norm_in.parts <= slim_max_parts(M)))
-                return launch_slim(A, W, C, epi, M, N, K, lda, ldw, ldc, norm_in, NO_NORM_OUT, stream);
-            return launch_strips(A, W, C, epi, M, N, K, lda, ldw, ldc, nullptr, StripCut{1, 0, 0}, norm_in, stream);
-        }
+        if (ends_in_strips(M, N, K) && strip_strides(lda, ldw)) return launch_strips(A, W, C, epi, M, N, K, lda, ldw, ldc, nullptr, StripCut{1, 0, 0}, norm_in, stream);
         const int k_per_split = K;
         dim3 grid((N + 63) / 64, 1);
         if (epi == EPI_GATED_BF16) SKINNY_MT(EPI_GATED_BF16, false); else if (epi == EPI_GATED_GELU_BF16) SKINNY_MT(EPI_GATED_GELU_BF16, false); else if (epi == EPI_GATED_CLAMP_BF16) SKINNY_MT(EPI_GATED_CLAMP_BF16, false); else if (epi == EPI_STORE_F32) SKINNY_MT(EPI_STORE_F32, false);
@@ -2944,7 +2938,7 @@ static int launch_large(const void* A, const void* W, void* C, int epi, int M, i
 // onto the rows.
 GI_API int gi_gemm_bf16_norm_parts(int M, int N, int K) {
     if (takes_slim(M, N, K, false)) {
-        const int parts = slim_parts(M, N);
+        const int parts = slim_parts(M, N, K);
         return parts <= slim_max_parts(M) ? parts : 0;
     }
     if (takes_slim_tiles(M, N, K, EPI_ADD_F32)) {
@@ -3096,7 +3090,7 @@ GI_API int gi_gemm_bf16_small_kernel(int M, int N, int K, int gated) {
 // How a product of at most 16 rows that the slim kernel makes reaches rows lda and ldw elements apart (`slim_reach`): weight rows a workgroup, and 100 more where it reckons in 64 bits.
 GI_API int gi_gemm_bf16_slim_reach(int M, int N, int K, int gated, int accumulate, long lda, long ldw) {
     if (M <= 0 || M > 16 || N <= 0 || K <= 0) return -1;
-    const SlimReach reach = slim_reach(M, N, K, gated ? EPI_GATED_BF16 : accumulate ? EPI_ADD_F32 : EPI_STORE_F32, lda, ldw);
+    const SlimReach reach = slim_reach(M, N, K, gated ? EPI_GATED_BF16 : accumulate ? EPI_ADD_F32 : EPI_STORE_F32, false, lda, ldw);
     return reach.rows + (reach.far ? 100 : 0);
 }
 

@@ -365,7 +365,7 @@ def test_gemm_bf16_strips_gate_up_to_192_rows(m, gated, limit):
     assert torch.equal(*seen)
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 12320, 64), (20, 16384, 576), (64, 12320, 192), (97, 12320, 576), (128, 16384, 1088)])
+@pytest.mark.parametrize("m,n,k", [(1, 17608, 64), (12, 28680, 384), (20, 16384, 576), (64, 12320, 192), (97, 12320, 576), (128, 16384, 1088)])
 def test_gemm_bf16_strips_of_columns_of_wider_matrices(m, n, k):
     """All of k in a workgroup: rows of A and W further apart than k, in bits as whole matrices."""
     assert ops().gemm_bf16_small_kernel(m, n, k) == "strips"
@@ -494,7 +494,8 @@ def test_gemm_bf16_few_rows_far_apart(m, n, k, lda8, reach):
 
 @pytest.mark.parametrize("m,parts", [(1, 512), (8, 300), (9, 256), (16, 3), (17, 256), (32, 2), (33, 8), (64, 1), (128, 5)])
 def test_gemm_bf16_strips_finish_a_norm(m, parts):
-    n, k = 28672, 3072                                                     # (strips from one row on)
+    n, k = 28672, 3072 if m > 10 else 192
+    assert ops().gemm_bf16_small_kernel(m, n, k, True) == "strips"
     a, w, squares = randn(m, k, dtype=torch.bfloat16, seed=1), randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.1), randn(m, parts, seed=3).abs() * k / parts
     product = (a.double() @ w.double().T) * torch.rsqrt(squares.double().sum(1, keepdim=True) / k + 1e-5)
     gate, up = product.view(m, n // 32, 2, 16).unbind(2)

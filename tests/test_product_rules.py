@@ -37,13 +37,14 @@ def test_strips_where_one_round_of_them_is_faster(m, n, k, kernel):
 
 # m, n, k, gated -> the kernel of up to 128 rows that was the faster one there, by more than 4 % or (on one side of a line) as fast
 FEW_ROWS = [
-    (1, 12288, 2048, True, "strips"), (8, 16384, 2048, True, "slim"), (9, 16384, 2048, True, "strips"), (1, 16384, 3072, True, "strips"), (1, 28672, 4096, True, "strips"), (4, 16384, 4096, True, "slim"),
-    (8, 16384, 4096, True, "strips"), (8, 12288, 256, True, "slim"), (2, 20480, 3072, True, "slim"), (8, 20480, 3072, True, "strips"),
-    (1, 12288, 2048, False, "slim"), (12, 12288, 2048, False, "strips"), (1, 12288, 3072, False, "slim"), (1, 13056, 3072, False, "strips"), (4, 16384, 2048, False, "slim"),
-    (12, 16384, 2048, False, "strips"), (2, 18432, 8192, False, "slim"), (4, 24576, 4096, False, "slim"), (4, 24576, 512, False, "streamed"), (4, 24576, 768, False, "strips"), (1, 32768, 4096, False, "slim"), (8, 32768, 3072, False, "strips"),
-    (4, 33280, 3072, False, "slim"), (8, 33280, 3072, False, "strips"), (3, 33280, 1280, False, "slim"), (4, 40960, 3072, False, "strips"), (3, 40960, 3072, False, "slim"), (8, 33280, 2048, False, "slim"), (3, 28672, 3072, False, "strips"),
-    (16, 16384, 512, False, "streamed"), (16, 16384, 768, False, "strips"), (20, 16384, 512, False, "strips"), (4, 128256, 2048, False, "slim"), (5, 128256, 2048, False, "strips"),
-    (11, 16384, 2056, True, "slim"), (12, 16384, 2056, True, "streamed"), (16, 3072, 2048, False, "slim"), (17, 3072, 2048, False, "slim tiles"), (17, 3072, 2048, True, "strips"),
+    (1, 12288, 2048, True, "slim"), (8, 12288, 2048, True, "slim"), (10, 12288, 2048, True, "strips"), (12, 12288, 1024, True, "slim"), (16, 12288, 1024, True, "strips"), (1, 16384, 3072, True, "slim"),
+    (16, 16384, 2048, True, "slim"), (16, 18432, 4096, True, "slim"), (8, 28672, 4096, True, "slim"), (10, 28672, 4096, True, "slim"), (12, 28672, 4096, True, "strips"), (16, 36864, 3072, True, "slim"),
+    (8, 12288, 256, True, "slim"), (16, 20480, 512, True, "slim"), (1, 33280, 64, True, "strips"), (8, 28672, 384, True, "slim"), (9, 28672, 384, True, "strips"),
+    (1, 12288, 3072, False, "slim"), (8, 12288, 2048, False, "slim"), (12, 12288, 2048, False, "strips"), (12, 13824, 1024, False, "slim"), (16, 13824, 1024, False, "strips"), (16, 16384, 2048, False, "slim"),
+    (16, 20480, 4096, False, "slim"), (16, 28672, 4096, False, "slim"), (12, 28672, 1024, False, "slim"), (16, 28672, 1024, False, "strips"), (16, 33280, 3072, False, "slim"), (5, 128256, 2048, False, "slim"),
+    (16, 128256, 2048, False, "slim"), (1, 152064, 64, False, "strips"), (8, 100352, 256, False, "strips"), (8, 65536, 512, False, "slim"), (9, 65536, 512, False, "strips"), (16, 24576, 512, False, "slim"),
+    (4, 32000, 384, False, "slim"), (9, 32000, 384, False, "strips"), (4, 28672, 512, False, "slim"), (8, 28672, 512, False, "streamed"), (10, 14336, 512, False, "slim"), (14, 14336, 512, False, "streamed"),
+    (20, 16384, 512, False, "strips"), (11, 16384, 2056, True, "slim"), (12, 16384, 2056, True, "streamed"), (16, 3072, 2048, False, "slim"), (17, 3072, 2048, False, "slim tiles"), (17, 3072, 2048, True, "strips"),
     (128, 3072, 2048, False, "strips"), (128, 3072, 2056, False, "streamed"), (129, 3072, 2048, False, None),
 ]
 
@@ -71,6 +72,14 @@ def test_few_rows_far_apart_are_reached(m, n, k, lda8, ldw8, gated, added, reach
     assert far or last * (16 if rows > 24 else 1) < 1 << 32
     if added:
         assert -(-n // rows) == ops.lib().gi_gemm_bf16_norm_parts(m, n, k)
+
+
+# rows, columns, k, added onto, gated -> weight rows a workgroup: what covers the compute units evenly, in whole groups of 8 where that costs less, few enough for a reader of a norm's pieces
+@pytest.mark.parametrize("m,n,k,added,gated,rows", [(1, 2048, 8192, True, False, 8), (8, 2304, 768, False, False, 9), (1, 4096, 4096, True, False, 16), (8, 6144, 4096, False, False, 24), (8, 8192, 512, True, False, 16),
+                                                    (16, 8192, 8192, True, False, 16), (1, 8192, 2048, False, False, 32), (8, 12288, 8192, False, False, 24), (8, 128256, 2048, False, False, 32), (8, 16384, 2048, False, True, 32),
+                                                    (1, 28672, 4096, False, True, 16), (12, 28672, 4096, False, True, 32)])
+def test_weight_rows_of_a_workgroup(m, n, k, added, gated, rows):
+    assert ops.gemm_bf16_slim_reach(m, n, k, k, k, gated, added) == (rows, False)
 
 
 # m, n, k -> tiles of rows and shares of k in strips, or None where the other kernels were the faster ones
