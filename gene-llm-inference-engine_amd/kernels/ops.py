@@ -1595,18 +1595,20 @@ def _single_cut(plan, n_heads, n_kv, hd, seen, target_waves, fused, orders):
     return n_splits, n_waves, ordered, plan.n_decode * n_heads * n_splits * (hd + 2) if n_splits > 1 else 0
 
 
-def _both_splits(plan, n_heads, n_kv, hd, span, tile_splits, most):
+def _both_splits(plan, n_heads, n_kv, hd, seen, tile_splits, most):
     """By how many workgroups each context of a step's single rows is read where they go out in one launch with the tiles; 0: in a launch of their own.
     The tiles' workgroups take about 11 us, half a microsecond for each tile of keys of the longest share and 2.6 for each of a place's even share; one that reads a context
     13.1 (64 channels: 9.8) for every 1,000 positions alone and nearly twice that beside the others.  So as few as keep the longest context within 0.8 of the
     tiles' time: its splits would cost a merge of theirs.  Of 135 drawn steps (1 to 48 single rows at up to 30,000 positions, 256 to 2,048 rows in all) two got
     slower, by 2 and 6 % (many single rows at under 350 positions, 45.6 and 48.3 us), and attention took 0.82 of the two launches' time in the mean: 24 heads of 128 over portions of 1,350 rows behind 1,000 positions and of 674, 24 single rows at up to
     2,990, 110 -> 93 us; 32 heads of 64 over 1,812 rows, 26 at up to 1,643, 53.1 -> 41.7.  Where the single rows' reading is more than four times the tiles' (more
-    than was measured) the places that tiles leave them, two workgroups a unit, are too few."""
-    walks = [-(-c // 64) for c in plan.tile_contexts]
+    than was measured) the places that tiles leave them, two workgroups a unit, are too few.  Tiles and rows count with what a window or
+    chunks leave them (`seen`): a window of 4,096 over 300 rows behind 60,000, a row at 4,096, 8 heads of 128 on two, 64.7 -> 37.0 us; of 512 over 500 rows, 30 at 30,000, 24 on 8, 35.3 -> 24.0."""
+    walks = [-(-seen(c, plan.tile) // 64) for c in plan.tile_contexts]
+    span = seen(plan.max_decode_context, 31)
     even = sum(walks) * n_heads / (lib().gi_compute_units() * (2 if hd == 128 else 3))
     tiles_us = 11 + 0.5 * -(-max(walks) // max(tile_splits, most)) + 2.6 * even
-    if plan.decode_positions * n_kv * hd * 4 > 4 * tiles_us * _DECODE_CHIP_MB_PER_S:
+    if min(plan.decode_positions, plan.n_decode * span) * n_kv * hd * 4 > 4 * tiles_us * _DECODE_CHIP_MB_PER_S:
         return 0
     splits = 1
     while splits < 16 and span >= 128 * (splits + 1) and 3 + span / splits * (0.0131 if hd == 128 else 0.0098) > 0.8 * tiles_us:
@@ -1620,7 +1622,7 @@ def _both_cut(plan, n_heads, n_kv, hd, window, chunk, page_size, seen, tile_spli
         return 0
     key = ("both", n_heads, n_kv, hd, window, chunk, page_size, tile_splits, most)
     if key not in plan.cuts:
-        splits = _both_splits(plan, n_heads, n_kv, hd, seen(plan.max_decode_context, 31), tile_splits, most) if hd in (64, 128) else 0
+        splits = _both_splits(plan, n_heads, n_kv, hd, seen, tile_splits, most) if hd in (64, 128) else 0
         takes = splits and lib().gi_attention_both_takes(plan.n_tiles, plan.tile, 1 if plan.paired else 0, tile_splits, most, plan.n_decode, splits, n_heads, n_kv, hd, page_size)
         plan.cuts[key] = splits if takes else 0
     return plan.cuts[key]

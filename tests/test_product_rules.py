@@ -322,15 +322,18 @@ def test_how_a_step_s_attention_is_cut_is_found_once_for_its_layers(monkeypatch)
     assert splits[0] == splits[1] == splits[2] > 1 and splits[-1] == 1
 
 
-# portions (positions before, rows), single rows at, heads, key heads, channels -> workgroups for each single row's context beside the tiles (0: a launch of their own)
-@pytest.mark.parametrize("portions,singles,heads,kv,hd,splits", [([(1000, 1350), (0, 674)], [380, 3000] * 12, 24, 8, 128, 1), ([(0, 1039)], [1117, 2198], 24, 8, 128, 2), ([(1030, 198), (0, 99)], [2322], 24, 8, 128, 2),
-                                                                 ([(0, 607)], [8452], 24, 8, 128, 9), ([(2073, 670), (0, 334)], [5761], 32, 8, 64, 2), ([(0, 300)], [30000] * 30, 24, 8, 128, 0),
-                                                                 ([(0, 1000)], [500], 24, 8, 96, 0), ([(0, 300)], [500], 32, 8, 64, 0)])
-def test_single_rows_beside_tiles(portions, singles, heads, kv, hd, splits):
+# portions (positions before, rows), single rows at, heads, key heads, channels, window -> workgroups for each single row's context beside the tiles (0: a launch of their own)
+@pytest.mark.parametrize("portions,singles,heads,kv,hd,window,splits", [([(1000, 1350), (0, 674)], [380, 3000] * 12, 24, 8, 128, 0, 1), ([(0, 1039)], [1117, 2198], 24, 8, 128, 0, 2),
+                                                                        ([(1030, 198), (0, 99)], [2322], 24, 8, 128, 0, 2), ([(0, 607)], [8452], 24, 8, 128, 0, 9),
+                                                                        ([(2073, 670), (0, 334)], [5761], 32, 8, 64, 0, 2), ([(0, 300)], [30000] * 30, 24, 8, 128, 0, 0),
+                                                                        ([(0, 1000)], [500], 24, 8, 96, 0, 0), ([(0, 300)], [500], 32, 8, 64, 0, 0),
+                                                                        # windows: tiles far behind walk no longer than those at the start, and rows far behind read no more than the window
+                                                                        ([(60000, 300)], [4096], 8, 2, 128, 4096, 3), ([(4096, 300)], [4096], 8, 2, 128, 4096, 3), ([(0, 300)], [30000] * 30, 24, 8, 128, 512, 1)])
+def test_single_rows_beside_tiles(portions, singles, heads, kv, hd, window, splits):
     segs = [(c - 1, 1) for c in singles] + portions
     plan = ops.AttentionPlan([sum(n for _, n in segs[:i]) for i in range(len(segs))], [n for _, n in segs], [p for p, _ in segs], list(range(len(segs))), "cpu")
-    seen = lambda context, slack: context
-    cut = lambda: (lambda tiles: ops._both_cut(plan, heads, kv, hd, 0, 0, 16, seen, tiles[0], tiles[2]))(ops._prompt_cut(plan, heads, hd, 0, 0, seen, True))
+    seen = lambda context, slack: min(context, window + slack) if window else context
+    cut = lambda: (lambda tiles: ops._both_cut(plan, heads, kv, hd, window, 0, 16, seen, tiles[0], tiles[2]))(ops._prompt_cut(plan, heads, hd, window, 0, seen, True))
     assert cut() == splits and cut() == splits
     plan.decode_positions = None                 # a step still to come
     assert cut() == 0
