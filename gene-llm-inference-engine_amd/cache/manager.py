@@ -224,6 +224,11 @@ class CacheManager:
             self.prefix = PrefixIndex(self.groups[0].pool, self.page_size, [g.pool for g in self.groups[1:]])
         return self.prefix is not None
 
+    @property
+    def pages_in_common(self) -> bool:
+        """Whether open requests hold pages in common, now."""
+        return self.prefix is not None and self.prefix.in_common > 0
+
     # ------------------------------------------------------------------------------ requests
     def open(self, request: Hashable, shared_pages: Sequence[int] = ()) -> int:
         """shared_pages: full pages of an equal prompt prefix, retained for this request by `self.prefix.match`

@@ -27,7 +27,7 @@ whole set.
 from __future__ import annotations
 
 import heapq
-from typing import Dict, List, Optional, Sequence, Tuple
+from typing import Dict, List, Optional, Sequence, Set, Tuple
 
 from .pages import PagePool
 
@@ -49,6 +49,7 @@ class PrefixIndex:
         self._by_page: Dict[int, _Node] = {}
         self._only_mine = 0                                   # named pages whose reference count is 1
         self._idle_leaves: List[Tuple[int, int]] = []         # heap of (stamp, page): leaves nobody else holds, and stale entries
+        self._in_common: Set[int] = set()                     # pages that several requests hold
         self._clock = 0
         self.last_walk = None                # where the last insert ended: (node of the last full page it passed, how many it passed)
         pool.on_change = self._references_changed
@@ -66,6 +67,10 @@ class PrefixIndex:
     # ------------------------------------------------------------------------- bookkeeping
     def _references_changed(self, page: int, count: int) -> None:
         node = self._by_page.get(page)
+        if count > (1 if node is None else 2):
+            self._in_common.add(page)
+        elif self._in_common:
+            self._in_common.discard(page)
         if node is None:
             return
         alone = count == 1
@@ -86,6 +91,11 @@ class PrefixIndex:
 
     def _children_of(self, node: Optional[_Node]) -> Dict[Tuple[int, ...], _Node]:
         return self._first if node is None else node.children
+
+    @property
+    def in_common(self) -> int:
+        """How many pages several requests hold, named or (forgotten since they were shared) not."""
+        return len(self._in_common)
 
     # ----------------------------------------------------------------------------- lookups
     def match(self, tokens: Sequence[int], limit: int) -> List[int]:

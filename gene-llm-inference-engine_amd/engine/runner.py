@@ -68,7 +68,7 @@ class Runner:
                  logits wanted, the same power-of-two bracket of the longest context (at most `max_step_graphs` are kept).
                  Such a step costs the host one copy and one launch instead of some hundred launches; longer steps keep
                  the device busy for longer than the host needs to launch them.  0: none.
-    max_graphs   most captured graphs kept (one per batch size and bracket of the longest context, at least two); the
+    max_graphs   most captured graphs kept (one per batch size, bracket of the longest context and whether requests hold pages in common; at least two); the
                  one used longest ago goes when another is needed.  All graphs take their memory from one pool, so what
                  they hold is what the largest of them needs (a pass's activations and its logits), not the sum.
 
@@ -205,7 +205,7 @@ class Runner:
             meta_dev = meta_dev.view(3, n_rows)
             ctx = StepContext(n_rows=n_rows, dtype=self.model.dtype, device=dev, tokens=meta_dev[0], row_pos=meta_dev[1],
                               row_slot=meta_dev[2], seg_slot=seg_slot, seg_start=seg_start, seg_len=seg_len, seg_pos0=seg_pos0,
-                              upload=self._uploads.put, every_row_wanted=every_row_wanted, pages_in_common=self.cache.prefix is not None)
+                              upload=self._uploads.put, every_row_wanted=every_row_wanted, pages_in_common=self.cache.pages_in_common)
             logits = self._forward(ctx, rows_dev, len(logit_rows))
         self._uploads.end_step()
         for e in entries:
@@ -225,9 +225,10 @@ class Runner:
         if not (self.can_step_from_device and 0 < n_rows <= self.graph_rows):
             return None
         bracket = _context_bracket(max(p + n for p, n in zip(seg_pos0, seg_len)), self.max_positions)
-        key = (tuple(seg_len), n_logit_rows, every_row_wanted, bracket)
-        g, in_common = self._step_graphs.get(key), self.cache.prefix is not None
-        if g is None or g.pages_in_common != in_common:
+        in_common = self.cache.pages_in_common               # (a step's graphs of either kind stay beside each other: requests that share come and go)
+        key = (tuple(seg_len), n_logit_rows, every_row_wanted, bracket, *(("pages in common",) if in_common else ()))
+        g = self._step_graphs.get(key)
+        if g is None:
             if len(self._step_graphs) >= self.max_step_graphs:       # (never during a capture: a graph may not be freed inside one)
                 del self._step_graphs[min(self._step_graphs, key=lambda k: self._step_graphs[k].last_used)]
             if self._graph_pool is None:
@@ -298,15 +299,18 @@ class Runner:
         every replay; nothing else in it depends on the step."""
         batch = meta.shape[1]
         # The attention kernel's cut of the context into pieces is fixed at capture, for the longest context the graph
-        # is to serve well: one graph per batch size and power-of-two bracket of the step's longest context.
+        # is to serve well: one graph per batch size and power-of-two bracket of the step's longest context, and one more where requests
+        # hold pages in common (the kernel then looks which, 0.2 to 0.5 us a layer; a server with the prefix index on and no such requests does without).
         bracket = _context_bracket(max(seg_pos0) + 1, self.max_positions)
-        g, in_common = self._graphs.get((batch, bracket)), self.cache.prefix is not None
-        if g is None or g.pages_in_common != in_common:
+        in_common = self.cache.pages_in_common
+        key = (batch, bracket, *(("pages in common",) if in_common else ()))
+        g = self._graphs.get(key)
+        if g is None:
             if len(self._graphs) >= self.max_graphs:         # (never during a capture: a graph may not be freed inside one)
                 del self._graphs[min(self._graphs, key=lambda k: self._graphs[k].last_used)]
             if self._graph_pool is None:
                 self._graph_pool = torch.cuda.graph_pool_handle()
-            g = self._graphs[(batch, bracket)] = _DecodeGraph(self.model, self._view, bracket, batch, self._graph_pool, self.cache.states, in_common)
+            g = self._graphs[key] = _DecodeGraph(self.model, self._view, bracket, batch, self._graph_pool, self.cache.states, in_common)
         g.last_used = self.steps_run
         self.steps_replayed += 1 if g.calls >= 1 else 0
         return g.run(meta, seg_slot, seg_pos0, tokens_on_device)

@@ -447,6 +447,42 @@ def test_shared_prefixes_over_two_groups_keep_the_books_under_random_use(seed):
     assert m.free_pages() == [14, 14]
 
 
+@pytest.mark.parametrize("seed", [0, 1, 2])
+def test_whether_requests_hold_pages_in_common_is_known_under_random_use(seed):
+    """Against a count of every page's holders after every action, forgotten names among them: requests with the index on that share nothing are told from those that do."""
+    rng = random.Random(seed)
+    m = manager([FULL], n_pages=14, page_size=2, max_requests=4, max_positions=24)
+    assert not m.pages_in_common and m.enable_prefix_sharing() and not m.pages_in_common
+    live, walks, seen = {}, {}, {True: 0, False: 0}
+    for turn in range(600):
+        roll = rng.random()
+        r = rng.choice(list(live)) if live else None
+        if (roll < 0.35 or r is None) and len(live) < 4:
+            live[turn], walks[turn] = [rng.randrange(2) for _ in range(rng.choice([3, 4, 6, 9, 12]))], None
+            m.open(turn, m.prefix.match(live[turn], len(live[turn]) - 1))
+        elif roll < 0.7:
+            n = min(rng.randint(1, 4), len(live[r]) - m.length(r))
+            if n > 0 and m.fits([(r, n)]):
+                m.reserve([(r, n)]); m.advance(r, n)
+                m.index_prefix(r, live[r], m.length(r), after=walks[r])
+                walks[r] = m.prefix.last_walk
+        elif roll < 0.8 and m.length(r) > 0 and m.available_pages()[0] > 0:
+            m.truncate(r, rng.randrange(m.length(r)))
+            walks[r] = None
+        elif roll < 0.83:
+            m.evict(3)
+        elif roll < 0.85:
+            m.prefix.clear()
+            walks = dict.fromkeys(walks)
+        else:
+            m.close(r)
+            del live[r], walks[r]
+        held = [p for r in live for p in m.pages_of(r)]
+        assert m.prefix.in_common == len({p for p in held if held.count(p) > 1}) and m.pages_in_common == (len(set(held)) < len(held))
+        seen[m.pages_in_common and len(m.prefix) > 0] += len(m.prefix) > 0
+    assert min(seen.values()) > 50
+
+
 def test_prefix_sharing_needs_pages_without_window_or_state():
     assert not manager([FULL, WINDOW], n_pages=8, page_size=4, max_requests=2, max_positions=32).enable_prefix_sharing()
     assert not manager([WINDOW], n_pages=8, page_size=4, max_requests=2, max_positions=32).enable_prefix_sharing()
@@ -675,3 +711,37 @@ def test_batch_sizes_of_captured_decode_steps():
     assert all(captured_batch_size(s, 4096) == s for s in sizes)                       # a size of the list serves itself
     assert len(set(sizes[:64])) == 24 and len(set(sizes)) < 60
     assert captured_batch_size(9, 9) == 9 and captured_batch_size(9, 10) == 10         # never beyond the rows a step may hold
+
+
+def test_captured_steps_with_pages_in_common_and_without_stay_beside_each_other(monkeypatch):
+    """The index alone is no reason for the kernels that look, and requests that come to share, or cease to, take no other step's capture (its logits may still be read) away."""
+    from types import SimpleNamespace
+    from geneinfer_amd.engine import runner as engine
+    made = []
+
+    class Graph:
+        def __init__(self, *args):
+            made.append(args[-1])
+            self.graph, self.calls = None, 0
+
+        def run(self, *args):
+            return self
+
+    monkeypatch.setattr(engine, "_DecodeGraph", Graph)
+    monkeypatch.setattr(engine, "_StepGraph", Graph)
+    m = manager([FULL], n_pages=8, page_size=4, max_requests=3, max_positions=32)
+    assert m.enable_prefix_sharing()
+    r = engine.Runner.__new__(engine.Runner)
+    r.__dict__.update(cache=m, model=SimpleNamespace(trace=None), _view=None, _graphs={}, _step_graphs={}, _graph_pool=1, max_graphs=4, max_step_graphs=4, max_positions=32, steps_run=0,
+                      steps_replayed=0, use_graphs=True, graph_rows=64)
+    step = lambda: (r._decode_step(torch.zeros(3, 2, dtype=torch.int32), [0, 1], [9, 9]), r._step_graph_for([5, 1], [0, 9], 2, False))
+    m.open("a")
+    m.reserve([("a", 10)]); m.advance("a", 10)
+    m.prefix.insert(list(range(10)), 10, m.pages_of("a"))
+    apart = step()
+    assert made == [False, False]
+    m.open("b", m.prefix.match(list(range(10)) + [77], 10))
+    shared = step()
+    assert made == [False, False, True, True] and step() == shared
+    m.close("b")
+    assert step() == apart and len(made) == 4 and len(r._graphs) == len(r._step_graphs) == 2
