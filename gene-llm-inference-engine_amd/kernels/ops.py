@@ -1242,7 +1242,7 @@ def latent_queries(q, cos, sin, plain, folded, n_heads, dim, rot, kv_rank, half_
           folded.data_ptr(), _code(folded, "latent_queries: folded"), folded.stride(0), n, n_heads, dim, rot, kv_rank, 1 if half_split else 0, _stream())
 
 
-@lru_cache(maxsize=None)
+@lru_cache(maxsize=8192)
 def _latent_fold_takes(n, n_heads, dim, rot, kv_rank) -> bool:
     return bool(lib().gi_latent_fold_takes(n, n_heads, dim, rot, kv_rank))
 
@@ -1505,7 +1505,7 @@ def _decode_ragged_split(groups, longest, mean, hd, n_waves):
     return best
 
 
-@lru_cache(maxsize=None)
+@lru_cache(maxsize=8192)
 def decode_attention_shape(n_decode, n_heads, n_kv, hd, span, target_waves=4096, fused=False):
     """(splits, waves per workgroup) of the decode kernel: about `target_waves` waves in all and pieces of
     at least 64 positions; a single split (no combine kernel) when a workgroup's waves cover them.

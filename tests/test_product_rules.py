@@ -354,3 +354,9 @@ def test_short_portions_go_row_by_row_over_pages_in_common(rows, apart, monkeypa
         ops.attention_bf16(q, cache, torch.zeros_like(q), plan, at, at, table, 8, 2, 64, memo={}, in_common=in_common)
     told = [a[15:17] for name, a in launched if name == "gi_attention_decode_bf16"]
     assert told == ([(n, 1 - apart), (n, 1)] if plan.n_decode else [])
+
+
+@pytest.mark.parametrize("rule", ["_latent_fold_takes", "decode_attention_shape"])
+def test_answers_kept_for_a_step_s_sizes_are_bounded(rule):
+    """Rows and contexts change from step to step: a process that runs for long keeps no answer for each."""
+    assert getattr(ops, rule).cache_parameters()["maxsize"]
