@@ -1930,17 +1930,20 @@ __global__ __launch_bounds__(256) void skinny_reduce_rope_store_kernel(const flo
 //
 // What bounds it is weights on their way from memory, and behind them the activations, of which every workgroup reads all.  67 MB of weights in a bare read take
 // 12.8 us, 11.4 past the caches (PAST: each line is read once, by one load; with 16 rows' 64 bytes a load, as this kernel read them before, 14.1 and 14.8).  All workgroups
-// starting at the same k would ask the same memory channels first (rows lie a multiple of 4 KB apart): 12.6 us, 11.9 from a place of their own.  Microseconds, before and now, in chains
-// of products with weights of their own:
+// starting at the same k would ask the same memory channels first (rows lie a multiple of 4 KB apart): 12.6 us, 11.9 from a place of their own.  Microseconds, with half lines and all
+// workgroups at the same k and so, in chains of products with weights of their own (400 to 1,050 MB in all; *: 200 MB, which the caches hold; +: made by strips):
 //   rows                        1               8               16
-//   16,384 x 2,048 gated        15.8, 12.2      16.7, 12.4      16.8, 13.9
-//   28,672 x 4,096 gated        45.9, 37.0      46.6, 43.1      46.8, 47.9
-//   2,048 x 8,192 added         8.9, 7.6        11.0, 9.6       13.6, 13.4
-//   2,048 x 2,048 added         3.9, 3.8        4.6, 4.4        5.3, 5.4
-//   4,096 x 14,336 added        25.3, 20.1      26.1, 22.7      32.3, 28.4
-//   6,144 x 4,096 stored        11.3, 9.9       14.1, 10.3      17.1, 12.1
-//   128,256 x 2,048 stored      84.4, 77.7      98.7, 80.9      100.9, 93.1
-//   1,024 x 512 stored          2.2, 2.4        2.5, 2.6        2.7, 2.9
+//   16,384 x 2,048 gated        15.7, 11.7      16.2, 11.7      16.7+, 13.5
+//   28,672 x 4,096 gated        45.7+, 34.6     45.3+, 39.3     46.1+, 40.7+
+//   2,048 x 8,192 added         8.7, 7.4        10.7, 9.5       13.2, 13.1
+//   2,048 x 2,048 added         3.9, 3.7        4.4, 4.3        5.3, 5.4
+//   4,096 x 14,336 added        24.1, 19.0      25.3, 21.9      31.5, 27.7
+//   6,144 x 4,096 stored        10.9, 9.4       14.8, 9.7       16.8, 11.6
+//   128,256 x 2,048 stored      78.7, 74.3      96.9+, 75.2     99.7+, 89.1
+//   4,096 x 768 gated           4.1, 3.4        4.7, 3.6        5.2, 3.9
+//   1,024 x 512 stored          2.4, 2.3        2.6, 2.5        2.8, 2.8
+//   1,024 x 512 stored*         2.2, 2.1        2.4, 2.3        2.6, 2.6
+//   2,048 x 2,048 added*        3.4, 3.7        4.1, 4.4        4.9, 5.3         (`weights_past_caches`)
 // HAND: with the two halves of a norm handed from product to product (`NormIn`, `NormOut` above).
 // Strides come in pieces of 16 bytes, so that all that the first loads need is in the registers that are filled with the launch.  FAR: rows so far apart that 64 bits are needed to
 // reckon with them (`slim_reach`).
@@ -3025,8 +3028,8 @@ GI_API int gi_gemm_bf16_onto_norm(const void* A, const void* W, float* C, int M,
 
 // Whether gi_gemm_bf16_qkv_rope_store takes a q/k/v product of these sizes with heads of hd channels.  17 or 33 to 128 rows: the
 // shapes whose k is shared out over workgroups, whose sums a second kernel adds up anyway.  More rows: the kernels with tiles of
-// 128 x 128 and 256 x 128, whose epilogues lay 128 rows of the tile into LDS and send them off rotated (whole heads must lie inside a tile), or, where they
-// share k out, that second kernel again.
+// 128 x 128, 256 x 128 and 256 x 256, whose epilogues lay 128 rows of the tile into LDS (of 256 columns as two such tiles) and send them off rotated (whole heads must lie
+// inside 128 columns), or, where they share k out, that second kernel again.
 GI_API int gi_gemm_bf16_qkv_rope_store_takes(int M, int N, int K, int hd) {
     if (hd < 8 || hd > 256 || (hd & (hd - 1)) != 0) return 0;
     if (M <= SKINNY_MAX_ROWS)

@@ -141,11 +141,11 @@ def test_gemm_exact_gated_has_the_bits_of_two_kernels(m, n, k, gated):
                                    (12, 12300, 520), (40, 12300, 264), (5, 65600, 72), (16, 12288, 256),
                                    # 17 to 32 rows, narrow outputs, short k: the slim kernel with two tiles of rows
                                    (32, 2048, 2048), (20, 3072, 2048), (31, 130, 136), (17, 16, 8),
-                                   # up to 8 rows and a narrow output: the idle halves of the matrix instructions take a further 32 of k (blocks of 256, cut anywhere)
+                                   # up to 8 rows and a narrow output: 8 weight rows at two places in k to a matrix instruction (steps of 64, cut anywhere)
                                    (8, 2048, 8192), (4, 3072, 2048), (2, 3072, 264), (6, 1000, 1000), (7, 60, 8200), (8, 8, 32), (5, 24, 40),
                                    # ... and 9 to 16 rows, in two groups of 8 that share the weights
                                    (12, 2048, 8192), (9, 100, 136), (16, 3072, 2048), (13, 1000, 1000), (16, 8, 32),
-                                   # strips of 12 or 8 weight rows that fill the compute units evenly, the last strip ragged (up to 16 rows, and 17 to 32)
+                                   # 12 or 8 weight rows a workgroup, which fill the compute units evenly, the last one's fewer (up to 16 rows, and 17 to 32)
                                    (13, 3000, 264), (8, 3071, 264), (3, 3072, 2048), (20, 2000, 264), (32, 2920, 2048)])
 @pytest.mark.parametrize("out_dtype,accumulate", [(torch.float32, False), (torch.float32, True), (torch.bfloat16, False)])
 def test_gemm_bf16(m, n, k, out_dtype, accumulate):
@@ -295,7 +295,7 @@ def test_gated_products_have_one_gate(m, inter, k, few, columns, stride, gated, 
 @pytest.mark.parametrize("m", [1, 17, 33, 64, 65, 97, 128, 129, 160, 161, 192, 193, 225, 256])
 @pytest.mark.parametrize("n,k", [(12320, 64), (12288 + 48, 192), (16384, 576), (200, 1088), (3072, 1536), (2048, 2112)])
 def test_gemm_bf16_strips(m, n, k):
-    """64 columns by all rows, up to 128 of them: on both sides of every height, one to more blocks of k than the ring has stages, a last strip of 8, 32 and 48 columns, k whole and in two to seven shares
+    """64 columns by all rows, 17 to 128 of them (one row: the kernel for few rows): on both sides of every height, one to more blocks of k than the ring has stages, a last strip of 8, 32 and 48 columns, k whole and in two to seven shares
     (uneven ones too), stored, added, in bfloat16 and gated.  With more rows strips make some of these products: two tiles of rows in two shares (3,072 x 1,536), gated ones with all of k."""
     a, w = randn(m, k, dtype=torch.bfloat16, seed=1), randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.1)
     want = a.double() @ w.double().T
@@ -399,7 +399,7 @@ def test_products_that_strips_do_not_make_go_the_way_before(m, n, k, short_of, m
     assert not torch.equal(out[:m, :n], strips)                            # (the sums of other shares)
 
 
-@pytest.mark.parametrize("n", [5, 2300, 4600, 7000])                      # weight rows a workgroup: 8, 9, 18 and 28, the last workgroup's fewer
+@pytest.mark.parametrize("n", [5, 2300, 4600, 7000])                      # weight rows a workgroup: 8, 9, 18 and 28 (15 where added, or of the longest k), the last workgroup's fewer
 @pytest.mark.parametrize("m,k", [(1, 8), (8, 72), (9, 520), (16, 1032), (3, 1536), (8, 2056), (16, 2560), (7, 3080), (12, 4160), (1, 5120)])
 def test_gemm_bf16_few_rows_at_every_height(m, n, k):
     """Workgroups of 8 to 32 weight rows with partly full groups, waves of none to ten steps of 64 k, the last one ragged; operands and outputs within wider ones.  The 32-bit sums' bound: 2e-6."""
@@ -607,8 +607,8 @@ def test_rope_cos_sin_uses_64_bit_angles():
                                             (100, 4096, 14336, 6144, False), (128, 3072, 8192, 16384, True), (33, 1024, 512, 12288, False),
                                             (24, 2048, 2048, 16384, True), (24, 2048, 8192, 3072, False), (14, 2048, 2048, 16384, True), (32, 2048, 2048, 2048, False),
                                             (17, 264, 136, 12288, False), (13, 4096, 4096, 28672, True),
-                                            # strips of 16 weight rows where strips of 8 would make more pieces than the reader takes (9 to 16 rows), and
-                                            # from 4 rows on for the product that hands on with 256 strips or more
+                                            # 12 and 16 weight rows a workgroup, with as many pieces of a row's sum of squares as a reader takes at 9 to 16 rows, and at
+                                            # up to 8
                                             (12, 3072, 8192, 5120, False), (16, 3072, 3072, 16384, True), (8, 4096, 14336, 6144, False), (4, 4096, 4096, 28672, True),
                                             # the rows of prompts: from the tiles of 128 x 128 (or the kernel that adds the shares of k) to the gated
                                             # product on the kernel with tiles of 256 x 256
