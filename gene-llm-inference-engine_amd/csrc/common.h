@@ -76,7 +76,7 @@ __device__ __forceinline__ uint4 load16_once(const bf16_t* p) {
     return uint4{v.x, v.y, v.z, v.w};
 }
 
-// Whether a matrix of weights goes past the caches: from 4,194,304 numbers on.  A product reads every weight once, but the next pass reads it again, and 256 MB behind the L2s hold a small model's
+// Whether a matrix of weights goes past the caches: from 8,388,608 numbers on.  A product reads every weight once, but the next pass reads it again, and 256 MB behind the L2s hold a small model's
 // weights till then.  Microseconds past the caches and through them, at 1 / 8 rows, in chains of products with weights of their own of 800 MB in all, and of 200 MB:
 //   768 x 768, bfloat16          (2.9, 2.9)                  2.8, 2.5 / 3.0, 2.7         2,304 x 768, 32-bit          4.5, 4.5 / 5.3, 5.3         4.7, 4.3 / 5.5, 5.2
 //   2,048 x 2,048                3.7, 3.7 / 4.3, 4.2         3.8, 3.4 / 4.3, 4.1         2,048 x 2,048                6.1, 6.1 / 6.7, 6.7         6.2, 5.6 / 6.8, 6.5
@@ -84,10 +84,8 @@ __device__ __forceinline__ uint4 load16_once(const bf16_t* p) {
 //   5,120 x 2,048                5.4, 5.6 / 5.8, 5.9         5.3, 5.3 / 5.8, 5.5         5,120 x 2,048                10.3, 10.4 / 13.7, 13.7     10.6, 9.6 / 13.5, 13.0
 //   16,384 x 2,048 gated         11.5, 12.4 / 11.7, 12.5     12.0, 12.6 / 12.7, 11.8     16,384 x 2,048               24.4, 25.5 / 26.3, 27.7
 //   16,384 x 3,072 gated         16.5, 18.4 / 17.3, 18.8     17.0, 17.1 / 17.0, 15.7     32,000 x 768                 21.1, 21.7 / 23.6, 24.9     21.5, 19.5 / 23.5, 21.8
-// In chains of one such product all of its weights contend alike.  In a whole model that the caches cannot hold (1.2 billion parameters, one position at a time: 16 layers of 4, 6, 17 and
-// 34 million) what went through them only pushed itself out: from 8,388,608 on a pass takes 731 us in bfloat16 and 1,376 at 3 rows in 32 bits, from 4,194,304 on, as with everything past
-// them, 706 and 1,360.  Models whose matrices are smaller (768 to 1,024 wide) can be held, and theirs go through the caches: 768 x 768 as above, 4,096 x 768 gated 3.6 -> 3.3.
-static inline bool weights_past_caches(int rows, int K) { return (long)rows * K >= 4L << 20; }
+// A model with matrices so large has more of them than the caches hold.
+static inline bool weights_past_caches(int rows, int K) { return (long)rows * K >= 8L << 20; }
 
 // Two loads of 8 rows' 128 bytes each, lane l of either with row l % 8 and the 16 bytes l / 16 + 4 (l / 8 % 2) of it (`low`: rows 0 to 7, `high`: 8 to 15), become operands
 // of two products: lane l with row l % 16 and the 16 bytes l / 16 (`low`) and those 64 bytes further (`high`).  Within 16 lanes the upper half of `low` and the lower half of

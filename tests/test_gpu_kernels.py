@@ -424,10 +424,10 @@ def test_gemm_bf16_few_rows_at_every_height(m, n, k):
 @pytest.mark.parametrize("k", [1000, 4096])
 @pytest.mark.parametrize("m,short_of", [(1, True), (1, False), (8, False), (11, True), (16, False)])
 def test_few_rows_of_as_many_weights_as_go_past_the_caches(m, short_of, k):
-    """4,194,304 weights and a few fewer, in either type: stored, added, gated and handing a norm on."""
+    """8,388,608 weights and a few fewer, in either type: stored, added, gated and handing a norm on."""
     o = ops()
-    n = ((4 << 20) - 1) // k // 32 * 32 + (0 if short_of else 32)
-    assert (n * k < 4 << 20) == short_of
+    n = ((8 << 20) - 1) // k // 32 * 32 + (0 if short_of else 32)
+    assert (n * k < 8 << 20) == short_of
     a, w, x0 = randn(m, k, dtype=torch.bfloat16, seed=1), randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.1), randn(m, n, seed=3)
     want = a.double() @ w.double().T
     out, x, gated, a32, w32 = torch.empty(m, n, device=DEV), x0.clone(), torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV), a.float(), w.float()
