@@ -69,23 +69,16 @@ __device__ __forceinline__ float softplus_f32(float z) { return z > 20.f ? z : l
 __device__ __forceinline__ float xielu(float z, float a, float b) { return z > 0.f ? fmaf(a * z, z, 0.5f * z) : fmaf(b, expm1f(z) - z, 0.5f * z); }
 
 // 16 bytes that a launch reads no second time: they go past the caches, which is faster where the lanes of one load take whole cache lines of 128 bytes
-// (67 MB of weights 12.8 -> 11.4 us in a bare read) and slower where they take half lines (14.1 -> 14.8), and only for bytes that the caches do not hold from before.
-__device__ __forceinline__ uint4 load16_once(const bf16_t* p) {
+// (67 MB of weights 12.8 -> 11.4 us in a bare read) and slower where they take half lines (14.1 -> 14.8).
+// Weights that the next pass reads again go the same way, though 256 MB behind the L2s could hold a small model's till then: in whole models that is worth next to nothing.  Past the caches and through them, us a pass:
+// 768 wide with 200 MB at 1 / 8 rows 298, 298 / 322, 322; 1,024 wide with 213 MB at 4 rows 236, 234; 512 wide with 70 MB 187, 185; 256 wide with 11 MB 136, 131; in 32 bits 462, 466 and 303, 308; two or three
+// models of 200 MB in turn 303, 324 and 238, 251; 1.1 GB, some of whose matrices have 2 million numbers, with these through the caches 1 % slower.  (A chain of one shape of product, 200 MB of weights in all, tells
+// otherwise: 768 x 768 2.5, 2.3.)
+__device__ __forceinline__ uint4 load16_once(const bf16_t* p) {              // of bytes that this launch reads no second time
     typedef uint32_t gi_load4 __attribute__((ext_vector_type(4)));
     const gi_load4 v = __builtin_nontemporal_load(reinterpret_cast<const gi_load4*>(p));
     return uint4{v.x, v.y, v.z, v.w};
 }
-
-// Whether a matrix of weights goes past the caches: from 8,388,608 numbers on.  A product reads every weight once, but the next pass reads it again, and 256 MB behind the L2s hold a small model's
-// weights till then.  Microseconds past the caches and through them, at 1 / 8 rows, in chains of products with weights of their own of 800 MB in all, and of 200 MB:
-//   768 x 768, bfloat16          (2.9, 2.9)                  2.8, 2.5 / 3.0, 2.7         2,304 x 768, 32-bit          4.5, 4.5 / 5.3, 5.3         4.7, 4.3 / 5.5, 5.2
-//   2,048 x 2,048                3.7, 3.7 / 4.3, 4.2         3.8, 3.4 / 4.3, 4.1         2,048 x 2,048                6.1, 6.1 / 6.7, 6.7         6.2, 5.6 / 6.8, 6.5
-//   3,072 x 2,048                4.2, 4.3 / 4.6, 4.6         4.5, 4.0 / 5.1, 4.4         2,048 x 4,096                8.9, 8.9 / 10.2, 10.2       9.2, 7.7 / 10.1, 9.8
-//   5,120 x 2,048                5.4, 5.6 / 5.8, 5.9         5.3, 5.3 / 5.8, 5.5         5,120 x 2,048                10.3, 10.4 / 13.7, 13.7     10.6, 9.6 / 13.5, 13.0
-//   16,384 x 2,048 gated         11.5, 12.4 / 11.7, 12.5     12.0, 12.6 / 12.7, 11.8     16,384 x 2,048               24.4, 25.5 / 26.3, 27.7
-//   16,384 x 3,072 gated         16.5, 18.4 / 17.3, 18.8     17.0, 17.1 / 17.0, 15.7     32,000 x 768                 21.1, 21.7 / 23.6, 24.9     21.5, 19.5 / 23.5, 21.8
-// A model with matrices so large has more of them than the caches hold.
-static inline bool weights_past_caches(int rows, int K) { return (long)rows * K >= 8L << 20; }
 
 // Two loads of 8 rows' 128 bytes each, lane l of either with row l % 8 and the 16 bytes l / 16 + 4 (l / 8 % 2) of it (`low`: rows 0 to 7, `high`: 8 to 15), become operands
 // of two products: lane l with row l % 16 and the 16 bytes l / 16 (`low`) and those 64 bytes further (`high`).  Within 16 lanes the upper half of `low` and the lower half of

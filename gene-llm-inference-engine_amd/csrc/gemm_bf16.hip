@@ -1929,9 +1929,9 @@ __global__ __launch_bounds__(256) void skinny_reduce_rope_store_kernel(const flo
 // Loads run DEPTH steps ahead of the products.  The waves' sums meet in LDS and are added in the order of the waves, the lower halves before the upper.
 //
 // What bounds it is weights on their way from memory, and behind them the activations, of which every workgroup reads all.  67 MB of weights in a bare read take
-// 12.8 us, 11.4 past the caches (PAST: each line is read once, by one load; with 16 rows' 64 bytes a load, as this kernel read them before, 14.1 and 14.8).  All workgroups
+// 12.8 us, 11.4 past the caches (each line is read once, by one load; with 16 rows' 64 bytes a load, as this kernel read them before, 14.1 and 14.8).  All workgroups
 // starting at the same k would ask the same memory channels first (rows lie a multiple of 4 KB apart): 12.6 us, 11.9 from a place of their own.  Microseconds, with half lines and all
-// workgroups at the same k and so, in chains of products with weights of their own (400 to 1,050 MB in all; *: 200 MB, which the caches hold; +: made by strips):
+// workgroups at the same k and so, in chains of products with weights of their own (400 to 1,050 MB in all; +: made by strips):
 //   rows                        1               8               16
 //   16,384 x 2,048 gated        15.7, 11.7      16.2, 11.7      16.7+, 13.5
 //   28,672 x 4,096 gated        45.7+, 34.6     45.3+, 39.3     46.1+, 40.7+
@@ -1940,16 +1940,14 @@ __global__ __launch_bounds__(256) void skinny_reduce_rope_store_kernel(const flo
 //   4,096 x 14,336 added        24.1, 19.0      25.3, 21.9      31.5, 27.7
 //   6,144 x 4,096 stored        10.9, 9.4       14.8, 9.7       16.8, 11.6
 //   128,256 x 2,048 stored      78.7, 74.3      96.9+, 75.2     99.7+, 89.1
-//   4,096 x 768 gated           4.1, 3.4        4.7, 3.6        5.2, 3.9
-//   1,024 x 512 stored          2.4, 2.3        2.6, 2.5        2.8, 2.8
-//   1,024 x 512 stored*         2.2, 2.1        2.4, 2.3        2.6, 2.6
-//   2,048 x 2,048 added*        3.4, 3.7        4.1, 4.4        4.9, 5.3         (`weights_past_caches`)
+//   4,096 x 768 gated           4.2, 3.5        4.7, 3.6        5.2, 4.0         (200 MB of such weights, which the caches could hold: 3.7, 3.5; 4.2, 3.6; 4.7, 3.9)
+//   1,024 x 512 stored          2.4, 2.4        2.6, 2.5        2.8, 2.8         (2.2, 2.4; 2.4, 2.6; 2.6, 2.8)
 // HAND: with the two halves of a norm handed from product to product (`NormIn`, `NormOut` above).
 // Strides come in pieces of 16 bytes, so that all that the first loads need is in the registers that are filled with the launch.  FAR: rows so far apart that 64 bits are needed to
 // reckon with them (`slim_reach`).
 template <bool FAR> struct SlimPlaces { typedef int Stride; typedef unsigned At; };
 template <> struct SlimPlaces<true> { typedef long Stride; typedef size_t At; };
-template <int GROUPS, int EPI, bool HAND, int XT, bool PAST, bool FAR = false>
+template <int GROUPS, int EPI, bool HAND, int XT, bool FAR = false>
 __global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, typename SlimPlaces<FAR>::Stride lda8,
                                                                 typename SlimPlaces<FAR>::Stride ldw8, int M, int N, int K, int rows, int turn,
                                                                 void* __restrict__ C, long ldc, NormIn norm_in, NormOut norm_out) {
@@ -1994,7 +1992,7 @@ __global__ __launch_bounds__(512, 4) void gemm_bf16_slim_kernel(const bf16_t* __
 #pragma unroll
         for (int t = 0; t < XT; ++t) x[t] = load16(whereof(A, x_at[t] + at));
 #pragma unroll
-        for (int g = 0; g < GROUPS; ++g) w[g] = PAST ? load16_once(whereof(w_base[g], w_at[g] + at)) : load16(whereof(w_base[g], w_at[g] + at));
+        for (int g = 0; g < GROUPS; ++g) w[g] = load16_once(whereof(w_base[g], w_at[g] + at));
     };
     floatx4 acc[XT][GROUPS];
 #pragma unroll
@@ -2603,9 +2601,8 @@ static int launch_slim(const void* A, const void* W, void* C, int epi, int M, in
     const auto [rows, far] = slim_reach(M, N, K, epi, norm_in.squares != nullptr, lda, ldw);
     const dim3 grid((N + rows - 1) / rows);
     const int turn = turn_of_steps((K + 63) / 64);
-    const bool past = weights_past_caches(N, K);
     if (far) {
-#define SLIM_FAR(GROUPS_, EPI_) gemm_bf16_slim_kernel<GROUPS_, EPI_, true, 2, false, true><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, lda / 8, ldw / 8, M, N, K, rows, turn, C, ldc, norm_in, norm_out)
+#define SLIM_FAR(GROUPS_, EPI_) gemm_bf16_slim_kernel<GROUPS_, EPI_, true, 2, true><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, lda / 8, ldw / 8, M, N, K, rows, turn, C, ldc, norm_in, norm_out)
         if (epi == EPI_GATED_BF16) SLIM_FAR(2, EPI_GATED_BF16); else if (epi == EPI_GATED_GELU_BF16) SLIM_FAR(2, EPI_GATED_GELU_BF16); else if (is_gated(epi)) SLIM_FAR(2, EPI_GATED_CLAMP_BF16);
         else if (epi == EPI_STORE_F32) SLIM_FAR(3, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM_FAR(3, EPI_ADD_F32);
         else if (epi == EPI_XIELU) SLIM_FAR(3, EPI_XIELU); else SLIM_FAR(3, EPI_STORE_BF16);
@@ -2613,13 +2610,12 @@ static int launch_slim(const void* A, const void* W, void* C, int epi, int M, in
         GI_CHECK_LAUNCH("gemm_bf16 (slim, far)");
         return 0;
     }
-#define SLIM_XT(GROUPS_, EPI_, XT_, PAST_)                                                                                                             \
+#define SLIM_XT(GROUPS_, EPI_, XT_)                                                                                                                    \
     do {                                                                                                                                               \
-        if (hand) gemm_bf16_slim_kernel<GROUPS_, EPI_, true, XT_, PAST_><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, (int)(lda / 8), (int)(ldw / 8), M, N, K, rows, turn, C, ldc, norm_in, norm_out); \
-        else gemm_bf16_slim_kernel<GROUPS_, EPI_, false, XT_, PAST_><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, (int)(lda / 8), (int)(ldw / 8), M, N, K, rows, turn, C, ldc, norm_in, norm_out);     \
+        if (hand) gemm_bf16_slim_kernel<GROUPS_, EPI_, true, XT_><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, (int)(lda / 8), (int)(ldw / 8), M, N, K, rows, turn, C, ldc, norm_in, norm_out); \
+        else gemm_bf16_slim_kernel<GROUPS_, EPI_, false, XT_><<<grid, 512, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, (int)(lda / 8), (int)(ldw / 8), M, N, K, rows, turn, C, ldc, norm_in, norm_out);     \
     } while (0)
-#define SLIM_ROWS(GROUPS_, EPI_, PAST_) do { if (M <= 8) SLIM_XT(GROUPS_, EPI_, 1, PAST_); else SLIM_XT(GROUPS_, EPI_, 2, PAST_); } while (0)
-#define SLIM(GROUPS_, EPI_) do { if (past) SLIM_ROWS(GROUPS_, EPI_, true); else SLIM_ROWS(GROUPS_, EPI_, false); } while (0)
+#define SLIM(GROUPS_, EPI_) do { if (M <= 8) SLIM_XT(GROUPS_, EPI_, 1); else SLIM_XT(GROUPS_, EPI_, 2); } while (0)
 #define SLIM_EPI(GROUPS_)                                                                                                                              \
     do {                                                                                                                                               \
         if (epi == EPI_STORE_F32) SLIM(GROUPS_, EPI_STORE_F32); else if (epi == EPI_ADD_F32) SLIM(GROUPS_, EPI_ADD_F32);                               \
@@ -2640,7 +2636,6 @@ static int launch_slim(const void* A, const void* W, void* C, int epi, int M, in
 #undef SLIM_GATED
 #undef SLIM_EPI
 #undef SLIM
-#undef SLIM_ROWS
 #undef SLIM_XT
     GI_CHECK_LAUNCH("gemm_bf16 (slim)");
     return 0;

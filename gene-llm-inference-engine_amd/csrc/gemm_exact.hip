@@ -319,7 +319,7 @@ __global__ __launch_bounds__(256) void gemm_exact_add_parts_kernel(const float* 
 // range of k (strips of 16 rows, 8 waves) or two (strips of 8 rows and at most 8 rows of activations, 4 waves: the idle half of
 // every matrix instruction takes the second range, weight rows 8..15 and activation rows 8..15 of the instruction standing for the
 // same rows at the other range's k; twice the workgroups for the same waves, which is what narrow outputs lack).  The operands go
-// from memory straight into the matrix instructions' registers: 32-bit weights a whole cache line of 8 rows a load, past the caches where they are many (PAST), four pairs of blocks of 16 k
+// from memory straight into the matrix instructions' registers: 32-bit weights a whole cache line of 8 rows a load, past the caches, four pairs of blocks of 16 k
 // in flight behind the products (with 16 rows' 64 bytes a load, eight blocks asked for at once and all awaited: the figures before); bfloat16 weights AHEAD blocks at once.
 // The ranges' sums meet in LDS and are added there.  At 3 rows, before and now, in chains of products with weights of their own: 16,384 x 2,048 gated 28.4, 26.6 us (5.0 TB/s), 2,048 x 8,192
 // added 17.4, 15.4 (4.35; a bare read of these places 13.0), 2,048 x 2,048 added 7.4, 6.2, 3,072 x 2,048 8.8, 8.4, 128,256 x 2,048 184, 178 (5.9); what is added onto is
@@ -345,7 +345,7 @@ struct Turn {
     int page_size, n_heads, n_kv, hd;
 };
 
-__device__ __forceinline__ f32x4 load4_once(const float* p) { return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p)); }      // (`load16_once`)
+__device__ __forceinline__ f32x4 load4_once(const float* p) { return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p)); }      // of bytes that this launch reads no second time
 // Lane l of either load holds row l % 8 and the 4 k from 4 (l / 16) + 16 (l / 8 % 2) on (`low`: rows 0 to 7, `high`: 8 to 15); afterwards row l % 16 and the 4 k from 4 (l / 16)
 // on (`low`) and those 16 further (`high`): within 16 lanes the upper half of `low` and the lower half of `high` change places.
 __device__ __forceinline__ void rows_of_halves(f32x4& low, f32x4& high) {
@@ -357,7 +357,7 @@ __device__ __forceinline__ void rows_of_halves(f32x4& low, f32x4& high) {
     }
 }
 
-template <int STRIP, typename TA, typename TW, typename TC, bool ACCUMULATE, typename End, bool PAST>
+template <int STRIP, typename TA, typename TW, typename TC, bool ACCUMULATE, typename End>
 __global__ __launch_bounds__(STRIP == 16 ? 512 : 256) void gemm_exact_few_rows_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C,
                                                                                       int M, int N, int K, long lda, long ldw, long ldc, End end) {
     constexpr bool GATED = End::KIND == 1, TURNED = End::KIND == 2;
@@ -405,7 +405,7 @@ __global__ __launch_bounds__(STRIP == 16 ? 512 : 256) void gemm_exact_few_rows_k
     f32x4 acc[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
     int whole;
     if constexpr (sizeof(TW) == 4) {
-        // 32-bit weights: a load brings 32 k of 8 rows, a whole cache line of each; two of them hold two blocks of 16 rows' (or 8 rows' in both
+        // 32-bit weights: a load brings 32 k of 8 rows, a whole cache line of each, past the caches; two of them hold two blocks of 16 rows' (or 8 rows' in both
         // ranges) operands, whose halves then change places.  DEPTH such pairs are in flight.
         constexpr int DEPTH = 4;
         const int w_k = 4 * (g + 4 * (r >> 3)), low_row = __shfl(first_row, r & 7, 64), high_row = STRIP == 16 ? __shfl(first_row, 8 + (r & 7), 64) : low_row;
@@ -414,8 +414,8 @@ __global__ __launch_bounds__(STRIP == 16 ? 512 : 256) void gemm_exact_few_rows_k
         whole = 2 * pairs;
         f32x4 w[DEPTH][2], a[DEPTH][2];
         auto fetch = [&](int i, int d) __attribute__((always_inline)) {
-            w[d][0] = PAST ? load4_once(w_low + 32 * i) : load4(w_low + 32 * i);
-            w[d][1] = PAST ? load4_once(w_high + 32 * i) : load4(w_high + 32 * i);
+            w[d][0] = load4_once(w_low + 32 * i);
+            w[d][1] = load4_once(w_high + 32 * i);
             a[d][0] = load4(a_row + base + 32 * i);
             a[d][1] = load4(a_row + base + 32 * i + 16);
         };
@@ -567,18 +567,6 @@ Cut cut_for(int M, int N, int K) {
     return c;
 }
 
-template <int STRIP, typename TA, typename TW, typename TC, bool ACC, typename End>
-void launch_few_rows(const TA* A, const TW* W, TC* C, int M, int N, int K, long lda, long ldw, long ldc, End end, hipStream_t stream) {
-    const dim3 grid((N + STRIP - 1) / STRIP), threads(STRIP == 16 ? 512 : 256);
-    if constexpr (sizeof(TW) == 4) {
-        if (weights_past_caches(N, K)) {
-            gemm_exact_few_rows_kernel<STRIP, TA, TW, TC, ACC, End, true><<<grid, threads, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, end);
-            return;
-        }
-    }
-    gemm_exact_few_rows_kernel<STRIP, TA, TW, TC, ACC, End, false><<<grid, threads, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, end);
-}
-
 template <typename TA, typename TW, typename TC, bool ACC>
 int launch(const TA* A, const TW* W, TC* C, float* part, long part_floats, int M, int N, int K, long lda, long ldw, long ldc, hipStream_t stream) {
     const auto by4 = [](const void* p, size_t elem) { return ((uintptr_t)p & (4 * elem - 1)) == 0; };
@@ -586,9 +574,9 @@ int launch(const TA* A, const TW* W, TC* C, float* part, long part_floats, int M
     if (vector && few_rows(M, N, K)) {
         // strips of 8 where strips of 16 would give fewer than two workgroups a compute unit
         if (M <= 8 && N < 32 * gi_compute_units())
-            launch_few_rows<8, TA, TW, TC, ACC>(A, W, C, M, N, K, lda, ldw, ldc, Plain{}, stream);
+            gemm_exact_few_rows_kernel<8, TA, TW, TC, ACC, Plain><<<(N + 7) / 8, 256, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, Plain{});
         else
-            launch_few_rows<16, TA, TW, TC, ACC>(A, W, C, M, N, K, lda, ldw, ldc, Plain{}, stream);
+            gemm_exact_few_rows_kernel<16, TA, TW, TC, ACC, Plain><<<(N + 15) / 16, 512, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, Plain{});
         return 0;
     }
     Cut c = cut_for(M, N, K);
@@ -665,7 +653,7 @@ GI_API int gi_gemm_exact_gated(const float* A, const float* W, float* C, int act
     GI_REQUIRE(act >= 0 && act < GI_N_ACTIVATIONS && gi_gemm_exact_gated_takes(M, N, K), "gemm_exact (gated): sizes M %d, N %d, K %d or activation %d are not taken", M, N, K, act);
     GI_REQUIRE(lda >= K && ldw >= K && ldc >= N / 2 && lda % 4 == 0 && ldw % 4 == 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0,
                "gemm_exact (gated): rows must be 16-byte aligned (strides %ld, %ld, %ld)", lda, ldw, ldc);
-    launch_few_rows<16, float, float, float, false>(A, W, C, M, N, K, lda, ldw, ldc, Gate{act, limit}, stream);          // (N is even: a strip of 16 rows is 8 columns)
+    gemm_exact_few_rows_kernel<16, float, float, float, false, Gate><<<(N / 2 + 7) / 8, 512, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, Gate{act, limit});
     GI_CHECK_LAUNCH("gemm_exact (gated)");
     return 0;
 }
@@ -688,7 +676,7 @@ GI_API int gi_gemm_exact_qkv_rope_store(const float* A, const float* W, int M, i
                    page_stride >= 2L * n_kv * page_size * hd && page_stride % 4 == 0,
                "gemm_exact (q/k/v): positions, slots, a table, q_out, both tables of the rotation or none, and a cache with a page stride of at least 2*n_kv*page_size*hd are needed");
     const Turn turn = {cos_t, sin_t, pos, slot, table, table_stride, q_out, cache, page_stride, page_size, n_heads, n_kv, hd};
-    launch_few_rows<8, float, float, float, false>(A, W, (float*)nullptr, M, N, K, lda, ldw, 0L, turn, stream);
+    gemm_exact_few_rows_kernel<8, float, float, float, false, Turn><<<N / 8, 256, 0, stream>>>(A, W, nullptr, M, N, K, lda, ldw, 0L, turn);
     GI_CHECK_LAUNCH("gemm_exact (q/k/v)");
     return 0;
 }

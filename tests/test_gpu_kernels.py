@@ -421,34 +421,6 @@ def test_gemm_bf16_few_rows_at_every_height(m, n, k):
         assert bool((gated[m:] == 3.0).all()) and bool((gated[:, cols:] == 3.0).all())
 
 
-@pytest.mark.parametrize("k", [1000, 4096])
-@pytest.mark.parametrize("m,short_of", [(1, True), (1, False), (8, False), (11, True), (16, False)])
-def test_few_rows_of_as_many_weights_as_go_past_the_caches(m, short_of, k):
-    """8,388,608 weights and a few fewer, in either type: stored, added, gated and handing a norm on."""
-    o = ops()
-    n = ((8 << 20) - 1) // k // 32 * 32 + (0 if short_of else 32)
-    assert (n * k < 8 << 20) == short_of
-    a, w, x0 = randn(m, k, dtype=torch.bfloat16, seed=1), randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.1), randn(m, n, seed=3)
-    want = a.double() @ w.double().T
-    out, x, gated, a32, w32 = torch.empty(m, n, device=DEV), x0.clone(), torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV), a.float(), w.float()
-    o.gemm_bf16(a, w, out)
-    o.gemm_bf16(a, w, x, accumulate=True)
-    o.gemm_bf16(a, w, gated, gated=True)
-    gate, up = want.reshape(m, n // 32, 2, 16).unbind(2)
-    assert rel(out, want) < 2e-6 and rel(x, x0.double() + want) < 2e-6 and rel(gated, (torch.nn.functional.silu(gate) * up).reshape(m, n // 2)) < 4.1e-3
-    if o.gemm_bf16_norm_parts(m, n, k):
-        squares, g, y, scaled = torch.rand(m, 5, device=DEV) * k, torch.rand(n, device=DEV), x0.clone(), torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
-        pieces = torch.empty(m, o.gemm_bf16_norm_parts(m, n, k), device=DEV)
-        o.gemm_bf16(a, w, y, accumulate=True, norm_in=(squares, 1e-5), norm_out=(g, scaled, pieces))
-        new = x0.double() + want * torch.rsqrt(squares.double().sum(1, keepdim=True) / k + 1e-5)
-        assert rel(y, new) < 2e-6 and rel(scaled, g.double() * new) < 4.1e-3 and rel(pieces.double().sum(1), (new ** 2).sum(1)) < 2e-6
-    exact, added, tiles = torch.empty(m, n, device=DEV), x0.clone(), torch.empty(40, n, device=DEV)
-    o.gemm_exact(a32, w32, exact)
-    o.gemm_exact(a32, w32, added, accumulate=True)
-    o.gemm_exact(torch.cat([a32, torch.zeros(40 - m, k, device=DEV)]), w32, tiles)
-    assert torch.equal(exact, tiles[:m]) and rel(exact, want) < 2e-6 and torch.equal(added, x0 + exact)
-
-
 @pytest.mark.parametrize("m,n,k,lda8,reach", [(16, 8192, 256, ((1 << 28) - 32) // 15, (32, False)), (16, 8192, 256, ((1 << 28) - 32) // 15 + 1, (24, False)), (16, 8192, 264, ((1 << 32) - 33) // 15, (24, False)),
                                               (16, 6144, 264, ((1 << 32) - 33) // 15 + 1, (24, True)), (16, 300, 56, ((1 << 32) - 7) // 15 + 1, (8, True))])
 def test_gemm_bf16_few_rows_far_apart(m, n, k, lda8, reach):
